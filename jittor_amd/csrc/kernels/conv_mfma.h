@@ -304,7 +304,9 @@ extern "C" __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu
             grp = grp < GROUPS ? grp : GROUPS - 1;
             voff = (live ? x_lane_off : 0x80000000u) + (unsigned)grp * 16;
         }
-        asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen" : "=v"(dst) : "v"(voff), "s"(x_desc), "s"(soff) : "memory");
+        // (five wait states: the scalar offset may come out of a vector register one instruction earlier, and in front of a
+        // spelled-out load the compiler does not keep the distance that the hardware asks for between the two)
+        asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %0, %1, %2, %3 offen" : "=v"(dst) : "v"(voff), "s"(x_desc), "s"(soff) : "memory");
     };
     auto commit_stage = [&](auto sc, bool live, mjt_u32x4v& d, int r0, int lrows, int buf, int item, int limit) {
         constexpr int stg = decltype(sc)::v;

@@ -208,7 +208,7 @@ extern "C" __global__ __launch_bounds__(512) void ENTRY(Params p) {
         for (int w = 0; w < 8; w++) {
             int n = 0;
             for (int q = 0; q < (NA + 7) / 8; q++) n += q * 8 + w < NA ? 1 : 0;
-            for (int q = 0; q < (NB + 7) / 8; q++) n += (q * 8 + w < NB ? 1 : 0) + (q * 8 + ((w + 6) & 7) < NB ? 1 : 0);
+            for (int q = 0; q < (NB + 7) / 8; q++) n += (q * 8 + w < NB ? 1 : 0) + (!WHOLE_ROW && q * 8 + ((w + 6) & 7) < NB ? 1 : 0);
             best = n < best ? n : best;
         }
         return best;

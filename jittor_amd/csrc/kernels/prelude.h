@@ -95,11 +95,14 @@ __device__ __forceinline__ void mjt_store(T* p, const mjt_pack<T, N>& src) {
 // Streaming store: non-temporal and system scope (sc0 sc1 nt), for results that are written once and not read back by the
 // kernel.  On MI355X this is the fastest policy for large outputs (a fill of 231 MB: 6.9 TB/s against 6.6 for plain
 // non-temporal stores and 6.5 for ordinary ones).  Spelled out because the non-temporal builtin sets nt only.
+// The hardware reads a 16-byte store's data late: two wait states have to pass before an instruction overwrites those
+// registers, and behind a spelled-out store the compiler does not count them (a group with four outputs whose next
+// address was worked out in the registers just stored wrote wrong values).
 template <class T, int N>
 __device__ __forceinline__ void mjt_store_nt(T* p, const mjt_pack<T, N>& src) {
     constexpr int BYTES = (int)(sizeof(T) * N);
     if constexpr (BYTES == 16) {
-        asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1 nt" : : "v"(p), "v"(*reinterpret_cast<const mjt_u32x4*>(&src)) : "memory");
+        asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1 nt\n\ts_nop 1" : : "v"(p), "v"(*reinterpret_cast<const mjt_u32x4*>(&src)) : "memory");
     } else if constexpr (BYTES == 8) {
         typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
         asm volatile("global_store_dwordx2 %0, %1, off sc0 sc1 nt" : : "v"(p), "v"(*reinterpret_cast<const u32x2*>(&src)) : "memory");
