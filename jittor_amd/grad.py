@@ -18,6 +18,25 @@ from .core import (Var, UnaryOp, BinaryOp, TernaryOp, BroadcastOp, ReduceOp, Rei
 from . import _lib
 
 
+def _is_one(v):
+    """Is v a constant 1, spread and cast (the gradient that arrives below a sum of the loss)?"""
+    while v._op is not None:
+        if v._buf is not None or not (isinstance(v._op, BroadcastOp) or isinstance(v._op, UnaryOp) and v._op.op == "cast" and v.is_float()):
+            return False
+        v = v._op.inputs[0]
+    return v._host is not None and v.num == 1 and v.dtype in ("float32", "float64", "float16") and v._host.reshape(-1)[0] == 1 \
+        or v.dtype == "bfloat16" and v._host is not None and v.num == 1 and v._host.reshape(-1)[0] == 0x3f80
+
+
+def _times(factor, dout):
+    """factor * dout, which is `factor` itself where dout is a constant 1: the product would be a pass over memory that changes
+    nothing (the gradient of a 32 x 128 x 56 x 56 float32 result under (y * g).sum(): 19 us).  A factor that is spread or gathered
+    stays a product: it is how the operands of convolutions and matrix products appear, which are recognised by it."""
+    if _is_one(dout) and not isinstance(factor._op, (BroadcastOp, ReindexOp)) and dt.binary_dtype_infer("multiply", factor.dtype, dout.dtype, factor.is_scalar, dout.is_scalar) == factor.dtype:
+        return factor
+    return binary(factor, dout, "multiply")
+
+
 def _unary_grad(op, x, y, dout):
     """ops/unary_op.cc:891-1019 (y is the op's output)."""
     ns = op.op
@@ -81,7 +100,7 @@ def _binary_grad(op, x, y, z, dout, index):
     if ns == "subtract":
         return dout if index == 0 else unary(dout, "negative")
     if ns == "multiply":
-        return binary(y if index == 0 else x, dout, "multiply")
+        return _times(y if index == 0 else x, dout)
     if ns == "divide":
         if index == 0:
             return binary(dout, y, "divide")
@@ -209,5 +228,7 @@ def grad(loss, targets, retain_graph=True):
     out = []
     for t in targets:
         g = grads.get(t.id)
+        if g is not None and g.id in nodes:                     # a var of the caller's own: the gradient is a var of its own
+            g = core.unary_clone(g)
         out.append(g if g is not None else make_number(0.0, t))
     return out[0] if single else out
