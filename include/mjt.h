@@ -331,6 +331,14 @@ int mjt_conv2d_meta_grouped(const mjt_tensor* x, const mjt_tensor* w, const mjt_
 int mjt_conv2d_meta_dgrad(const mjt_tensor* dy, const mjt_tensor* w, const mjt_tensor* dx,
                           const mjt_conv_params* p);
 
+/* The same for a depthwise convolution with as many output as input channels
+ * (w [groups,1,R,S], dx and dy with `groups` channels; python/jittor/nn.py:1272-1294):
+ * one launch that reads dy and w as they lie.  Other groupings, more than 49
+ * taps, padding beyond the taps' reach and windows too large for LDS return
+ * MJT_ERR_UNSUPPORTED. */
+int mjt_conv2d_meta_dgrad_depthwise(const mjt_tensor* dy, const mjt_tensor* w, const mjt_tensor* dx,
+                                    const mjt_conv_params* p, int groups);
+
 /* Weight gradient of the same convolution (the pattern
  * reindex(x) * broadcast(dy) -> reduce.add over (n, oh, ow) that jt.grad builds;
  * opt/tuner/conv_tuner.cc:375-397 relays it to a backward-w library op,

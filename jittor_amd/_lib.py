@@ -91,7 +91,7 @@ EXPORTS = ["mjt_init", "mjt_shutdown", "mjt_last_error", "mjt_get_device_info",
            "mjt_alloc", "mjt_free", "mjt_h2d", "mjt_d2h", "mjt_d2d", "mjt_fill_u32",
            "mjt_sync", "mjt_event_create", "mjt_event_record", "mjt_event_elapsed_ms",
            "mjt_event_destroy", "mjt_reduce", "mjt_reduce_static", "mjt_reindex", "mjt_reindex_reduce",
-           "mjt_fused_elementwise", "mjt_fused_reduce", "mjt_conv2d_meta", "mjt_conv2d_meta_pack", "mjt_conv2d_meta_packed", "mjt_conv2d_meta_grouped", "mjt_conv2d_meta_dgrad", "mjt_conv2d_meta_wgrad", "mjt_conv2d_meta_wgrad_grouped",
+           "mjt_fused_elementwise", "mjt_fused_reduce", "mjt_conv2d_meta", "mjt_conv2d_meta_pack", "mjt_conv2d_meta_packed", "mjt_conv2d_meta_grouped", "mjt_conv2d_meta_dgrad", "mjt_conv2d_meta_dgrad_depthwise", "mjt_conv2d_meta_wgrad", "mjt_conv2d_meta_wgrad_grouped",
            "mjt_reindex_then_reduce", "mjt_fused_reindex_reduce", "mjt_matmul", "mjt_matmul_available",
            "mjt_expr_affine", "mjt_where_count", "mjt_where",
            "mjt_jit_stats", "mjt_last_kernel"]
@@ -149,6 +149,7 @@ def load():
                                             ctypes.POINTER(ConvParams), ctypes.c_int]
     lib.mjt_conv2d_meta_dgrad.argtypes = [ctypes.POINTER(Tensor), ctypes.POINTER(Tensor), ctypes.POINTER(Tensor),
                                           ctypes.POINTER(ConvParams)]
+    lib.mjt_conv2d_meta_dgrad_depthwise.argtypes = lib.mjt_conv2d_meta_grouped.argtypes
     lib.mjt_conv2d_meta_wgrad.argtypes = [ctypes.POINTER(Tensor), ctypes.POINTER(Tensor), ctypes.POINTER(Tensor),
                                           ctypes.POINTER(ConvParams)]
     lib.mjt_conv2d_meta_wgrad_grouped.argtypes = [ctypes.POINTER(Tensor), ctypes.POINTER(Tensor), ctypes.POINTER(Tensor),

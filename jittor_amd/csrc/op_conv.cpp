@@ -74,6 +74,92 @@ void gemm_launch(int in_dtype, int out_dtype, const void* A, const void* B, void
                  int64_t lda, int64_t ldb, int64_t ldc, int64_t sa, int64_t sb, int64_t sc, int64_t batch, bool a_kcont,
                  bool b_kcont, int tile_m = 0, int tile_n = 0, bool allow_direct = true);
 
+// ---- depthwise convolution (kernels/conv_depthwise.h) ----------------------------------
+namespace {
+struct DepthwiseShape {                       // see the kernel's header: staged planes H x W, strips in planes of OH x OW
+    int64_t H, W, OH, OW, R, S, SH, SW, PH, PW, DH, DW, UH, UW, K, mult;
+    bool flip;
+};
+struct DepthwisePlan {
+    int64_t TH, NTILE, PPW, VEC, STVEC;
+};
+constexpr int kDwCW = 4, kDwRS = 4;           // a lane's strip: 4 columns (16 bytes of float32) x 4 rows
+
+// Tile and vector widths, or false when the shape does not fit: at most 49 taps (they live in registers) and a window of
+// strip rows that fits LDS.  A workgroup stages whole planes while one is at most 40 KB (four workgroups or more then share a
+// compute unit and one loads while another computes), else rows of one plane; small planes together, as many as give every
+// lane a strip, as long as 512 workgroups are left.
+bool depthwise_plan(const DepthwiseShape& g, int in_size, int strip_size, const void* x, const void* strips, int64_t planes, int64_t most_ppw, DepthwisePlan* out) {
+    if (g.R * g.S > 49 || g.PH < 0 || g.PW < 0 || g.H * g.W >= (int64_t(1) << 31) || g.OH * g.OW >= (int64_t(1) << 31)) return false;
+    const int64_t ncg = (g.OW + kDwCW - 1) / kDwCW;
+    const int64_t nv = ((kDwCW - 1) * g.SW + (g.S - 1) * g.DW + 1 + 3) / 4;
+    const int64_t lc = ((ncg - 1) * kDwCW * g.SW + nv * 4 + 3) / 4 * 4;
+    if (nv > 8) return false;
+    auto bytes = [&](int64_t th) { return (((th + kDwRS - 1) / kDwRS * kDwRS - 1) * g.SH + (g.R - 1) * g.DH + 1) * lc * 4; };
+    int64_t th = g.OH;
+    while (th > kDwRS && bytes(th) > 40 * 1024) th = ((th + 1) / 2 + kDwRS - 1) / kDwRS * kDwRS;
+    if (bytes(th) > 60 * 1024) return false;
+    out->TH = th;
+    out->NTILE = (g.OH + th - 1) / th;
+    int64_t ppw = 1;
+    if (out->NTILE == 1) {
+        ppw = 256 / (((th + kDwRS - 1) / kDwRS) * ncg);
+        if (ppw > 40 * 1024 / bytes(th)) ppw = 40 * 1024 / bytes(th);
+        if (ppw > planes / 512) ppw = planes / 512;
+        if (ppw > most_ppw) ppw = most_ppw;
+        if (ppw < 1) ppw = 1;
+    }
+    out->PPW = ppw;
+    int64_t vec = 16 / in_size;
+    while (vec > 1 && (g.W % vec || (uintptr_t)x % (size_t)(vec * in_size))) vec /= 2;
+    out->VEC = vec;
+    int64_t sv = kDwCW;
+    while (sv > 1 && (g.OW % sv || (uintptr_t)strips % (size_t)(sv * strip_size))) sv /= 2;
+    out->STVEC = sv;
+    return true;
+}
+
+JitKernel* depthwise_kernel(int mode, const DepthwiseShape& g, const DepthwisePlan& q, int tin, int tout) {
+    std::ostringstream key;
+    key << "dw|" << mode << "|" << tin << "|" << tout << "|" << g.H << "|" << g.W << "|" << g.OH << "|" << g.OW << "|" << g.R << "|" << g.S << "|" << g.SH << "|" << g.SW
+        << "|" << g.PH << "|" << g.PW << "|" << g.DH << "|" << g.DW << "|" << g.UH << "|" << g.UW << "|" << g.K << "|" << g.mult << "|" << g.flip << "|" << q.TH << "|"
+        << q.PPW << "|" << q.VEC << "|" << q.STVEC;
+    JitKernel* k = cached(key.str());
+    if (k) return k;
+    std::ostringstream name;
+    name << (mode ? "mjt_conv_wgrad_direct_" : "mjt_conv_direct_") << mjt_dtype_name(tin);
+    if (!mode) name << "_" << mjt_dtype_name(tout);
+    name << "_depthwise_" << g.H << "x" << g.W << "_r" << g.R << "x" << g.S << "_s" << g.SH << "x" << g.SW << "_p" << g.PH << "x" << g.PW << "_d" << g.DH
+         << "x" << g.DW << "_u" << g.UH << "x" << g.UW << (g.flip ? "_flip" : "") << (g.mult > 1 ? "_m" + std::to_string(g.mult) : std::string()) << "_g" << g.K / g.mult;
+    std::ostringstream src;
+    src << "#define ENTRY " << name.str() << "\n#define MODE " << mode << "\n#define TIN " << dtype_cname(tin) << "\n#define TOUT " << dtype_cname(tout) << "\n#define H_ " << g.H
+        << "\n#define W_ " << g.W << "\n#define OH_ " << g.OH << "\n#define OW_ " << g.OW << "\n#define R_ " << g.R << "\n#define S_ " << g.S << "\n#define SH " << g.SH
+        << "\n#define SW " << g.SW << "\n#define PH " << g.PH << "\n#define PW " << g.PW << "\n#define DH " << g.DH << "\n#define DW " << g.DW << "\n#define UH " << g.UH
+        << "\n#define UW " << g.UW << "\n#define MULT " << g.mult << "\n#define K_ " << g.K << "\n#define FLIP " << (g.flip ? 1 : 0) << "\n#define TH " << q.TH
+        << "\n#define NTILE " << q.NTILE << "\n#define PPW " << q.PPW << "\n#define VEC " << q.VEC << "\n#define CW " << kDwCW << "\n#define RS " << kDwRS
+        << "\n#define STVEC " << q.STVEC << "\n";
+    src << embedded_source("prelude.h") << "\n" << embedded_source("conv_depthwise.h") << "\n";
+    k = jit_get(src.str(), name.str());
+    remember(key.str(), k);
+    return k;
+}
+
+// y[planes of OH x OW] = convolution of x[planes of H x W] (or, with flip, the input gradient); false: not covered
+bool depthwise_run(const DepthwiseShape& g, const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y) {
+    const int64_t planes = y->shape[0] * y->shape[1];
+    DepthwisePlan q;
+    if (getenv("MJT_NO_FASTPATH") ||
+        !depthwise_plan(g, dtype_size(x->dtype), dtype_size(y->dtype), x->ptr, y->ptr, planes, g.mult == 1 ? planes : 1, &q))
+        return false;
+    const int64_t blocks = (planes + q.PPW - 1) / q.PPW * q.NTILE;
+    if (blocks >= (int64_t(1) << 31)) return false;
+    JitKernel* k = depthwise_kernel(0, g, q, x->dtype, y->dtype);
+    std::vector<uint64_t> a{bits_of_ptr(x->ptr), bits_of_ptr(w->ptr), bits_of_ptr(y->ptr), (uint64_t)planes, 0, 0};
+    jit_launch(k, (unsigned)blocks, 1, 256, 0, a);
+    return true;
+}
+}  // namespace
+
 // free_extent: y's rows and columns are taken as they are instead of checked against the extents that stride, padding and
 // taps give (output (oh, ow) reads x around (oh*sh - ph, ow*sw - pw) whatever oh and ow; outside the image x is 0): what the
 // stride phases of an input gradient need, whose zero margins differ between the two ends of an axis.
@@ -476,6 +562,12 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
         return;
     }
 
+    // ---- depthwise: one input channel per group -----------------------------------------
+    if (G > 1 && C == 1 && !free_extent) {
+        const DepthwiseShape g{H, W, OH, OW, R, S, p->stride_h, p->stride_w, p->pad_h, p->pad_w, p->dil_h, p->dil_w, 1, 1, K, K / G, false};
+        if (depthwise_run(g, x, w, y)) return;
+    }
+
     // ---- direct path ----------------------------------------------------------------
     const bool idx32 = numel(x) < (int64_t(1) << 31) && numel(y) < (int64_t(1) << 31) - 256 && numel(w) < (int64_t(1) << 31);
     std::ostringstream key;
@@ -548,6 +640,29 @@ static void conv_wgrad_direct(const mjt_tensor* x, const mjt_tensor* dy, const m
     if (N == 0 || OH * OW == 0) {                                // a sum over nothing: zeros, written by the reduce kernel
         fold_wgrad_slices(wgrad_partials(4), 0, dw);
         return;
+    }
+    if (C == 1 && G > 1 && !getenv("MJT_NO_FASTPATH")) {           // depthwise: planes through LDS
+        const int64_t cus = ctx().dry_run || ctx().prop.multiProcessorCount <= 0 ? 256 : ctx().prop.multiProcessorCount;
+        // slices of images: about four workgroups per compute unit, each of which has the planes of its next images on their way
+        // while it sums; every slice ends in a fold of its lanes' sums and a row of partial results (us with the fold, float32, 3x3,
+        // 2 / 4 / 8 / 16 workgroups a unit: 32 x 128 x 56 x 56 34.6 / 26.5 / 30.6 / 32.7; 64 x 256 x 14 x 14 - / 12.4 / 15.8 / 18.5)
+        int64_t slices = (4 * cus + K - 1) / K;
+        if (slices > N) slices = N;
+        const int64_t ips = (N + slices - 1) / slices;
+        slices = (N + ips - 1) / ips;
+        const DepthwiseShape g{H, W, OH, OW, R, S, p->stride_h, p->stride_w, p->pad_h, p->pad_w, p->dil_h, p->dil_w, 1, 1, K, K / G, false};
+        DepthwisePlan q;
+        if (slices * K < (int64_t(1) << 31) &&
+            depthwise_plan(g, dtype_size(x->dtype), dtype_size(dy->dtype), x->ptr, dy->ptr, int64_t(1) << 40, ips, &q)) {
+            JitKernel* k = depthwise_kernel(1, g, q, x->dtype, x->dtype);
+            const bool in_place = slices == 1 && dw->dtype == MJT_FLOAT32;
+            void* part = in_place ? dw->ptr : wgrad_partials((size_t)slices * (size_t)numel(dw) * 4);
+            std::vector<uint64_t> a{bits_of_ptr(x->ptr), bits_of_ptr(dy->ptr), bits_of_ptr(part), (uint64_t)N, (uint64_t)ips, 0};
+            jit_launch(k, (unsigned)(slices * K), 1, 256, 0, a);
+            if (!in_place) fold_wgrad_slices(part, slices, dw);
+            set_last_kernel(k->name.c_str());
+            return;
+        }
     }
     const int64_t taps = R * S;
     const int64_t TCH = taps <= 49 ? taps : 32;
@@ -836,6 +951,37 @@ void conv_dgrad_impl(const mjt_tensor* dy, const mjt_tensor* w, const mjt_tensor
     conv_impl(&tz, &tw, dx, &q, 1);
 }
 }  // namespace mjt
+
+namespace mjt {
+// Input gradient of a depthwise convolution with as many output as input channels: one launch on the forward kernel, which
+// reads the taps from the last to the first and keeps the rows and columns of a strided dy apart.
+void conv_dgrad_depthwise(const mjt_tensor* dy, const mjt_tensor* w, const mjt_tensor* dx, const mjt_conv_params* p, int64_t G) {
+    require_init();
+    check_tensor(dy, "conv dgrad dy");
+    check_tensor(w, "conv dgrad w");
+    check_tensor(dx, "conv dgrad dx");
+    MJT_CHECK(p, "conv dgrad: null parameters");
+    MJT_CHECK(dy->ndim == 4 && w->ndim == 4 && dx->ndim == 4, "conv dgrad: dy, w and dx must have rank 4");
+    MJT_CHECK(dy->dtype == w->dtype && (dy->dtype == MJT_BFLOAT16 || dy->dtype == MJT_FLOAT16 || dy->dtype == MJT_FLOAT32),
+              "conv dgrad: dy and w must both be bfloat16, float16 or float32");
+    MJT_CHECK(dx->dtype == MJT_FLOAT32 || dx->dtype == dy->dtype, "conv dgrad: dx must be float32 or the operands' dtype");
+    MJT_CHECK(p->stride_h >= 1 && p->stride_w >= 1 && p->dil_h >= 1 && p->dil_w >= 1 && p->pad_h >= 0 && p->pad_w >= 0,
+              "conv dgrad: bad stride / padding / dilation");
+    const int64_t C = dx->shape[1], H = dx->shape[2], W = dx->shape[3], R = w->shape[2], S = w->shape[3];
+    const int64_t OH = (H + 2 * p->pad_h - p->dil_h * (R - 1) - 1) / p->stride_h + 1, OW = (W + 2 * p->pad_w - p->dil_w * (S - 1) - 1) / p->stride_w + 1;
+    MJT_CHECK(G >= 1 && C % G == 0 && w->shape[0] % G == 0, "conv dgrad: channels do not split into " << G << " groups");
+    MJT_CHECK(dy->shape[0] == dx->shape[0] && dy->shape[1] == w->shape[0] && dy->shape[2] == OH && dy->shape[3] == OW,
+              "conv dgrad: dy shape " << shape_str(dy) << " does not follow from dx " << shape_str(dx) << " and w " << shape_str(w));
+    if (G < 2 || C != G || w->shape[0] != G || w->shape[1] != 1) MJT_FAIL(MJT_ERR_UNSUPPORTED, "conv dgrad: only depthwise convolutions with as many output as input channels");
+    if (numel(dx) == 0) return;
+    const DepthwiseShape g{OH, OW, H, W, R, S, 1, 1, p->dil_h * (R - 1) - p->pad_h, p->dil_w * (S - 1) - p->pad_w, p->dil_h, p->dil_w, p->stride_h, p->stride_w, C, 1, true};
+    if (numel(dy) == 0 || !depthwise_run(g, dy, w, dx)) MJT_FAIL(MJT_ERR_UNSUPPORTED, "conv dgrad: this shape takes another route");
+}
+}  // namespace mjt
+
+extern "C" int mjt_conv2d_meta_dgrad_depthwise(const mjt_tensor* dy, const mjt_tensor* w, const mjt_tensor* dx, const mjt_conv_params* p, int groups) {
+    return mjt::guarded([&] { mjt::conv_dgrad_depthwise(dy, w, dx, p, groups); });
+}
 
 extern "C" int mjt_conv2d_meta_dgrad(const mjt_tensor* dy, const mjt_tensor* w, const mjt_tensor* dx, const mjt_conv_params* p) {
     return mjt::guarded([&] { mjt::conv_dgrad_impl(dy, w, dx, p); });

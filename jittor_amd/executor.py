@@ -1093,6 +1093,15 @@ def _run_single(op):
             p = _lib.ConvParams(sh, sw, ph, pw, dh, dw)
             _lib.check(lib.mjt_conv2d_meta_dgrad(ctypes.byref(td), ctypes.byref(tw), ctypes.byref(tx), ctypes.byref(p)))
             return
+        if G == K == C * G:                                    # depthwise: one launch (rc: shapes it hands back)
+            td, tw = _tensor_of(dy), _tensor_of(w)
+            tx = _tensor(_alloc_out(out), out.dtype, out.shape)
+            p = _lib.ConvParams(sh, sw, ph, pw, dh, dw)
+            rc = lib.mjt_conv2d_meta_dgrad_depthwise(ctypes.byref(td), ctypes.byref(tw), ctypes.byref(tx), ctypes.byref(p), G)
+            if rc == 0:
+                return
+            if rc != _lib.ERR_UNSUPPORTED:
+                _lib.check(rc)
         with core.no_grad():
             if G > 1:
                 # w [G*Kg, Cg, R, S] -> [G*Cg, Kg, R, S]: transposed within each group, taps flipped

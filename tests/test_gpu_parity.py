@@ -1717,3 +1717,63 @@ def test_scatter_with_element_wise_prologue(gpu):
         assert np.allclose(got, want, rtol=1e-4, atol=1e-5), kernel
     # a gathered var is refused where it has no meaning
     assert lib.mjt_fused_elementwise(ctypes.byref(d)) < 0 and "role" in lib.mjt_last_error().decode()
+
+
+@pytest.mark.parametrize("case", [
+    dict(dt="float32", n=2, c=3, hw=(9, 8), rs=(3, 3), p=(1, 1, 1, 1, 1, 1)),                # rows of whole vectors, one strip short of rows
+    dict(dt="float32", n=1, c=2, hw=(1, 1), rs=(1, 1), p=(1, 1, 0, 0, 1, 1)),                # the smallest plane
+    dict(dt="bfloat16", n=3, c=5, hw=(7, 7), rs=(5, 5), p=(2, 2, 2, 2, 1, 1), out="bfloat16"),   # several odd planes staged together, strided
+    dict(dt="float16", n=2, c=4, hw=(10, 13), rs=(3, 2), p=(3, 2, 1, 0, 2, 3), out="float16"),   # strides and dilations that differ
+    dict(dt="float32", n=2, c=2, hw=(130, 100), rs=(3, 3), p=(1, 1, 1, 1, 1, 1)),            # a plane in several tiles of rows
+    dict(dt="float32", n=1, c=2, hw=(200, 60), rs=(7, 7), p=(2, 2, 3, 3, 1, 1)),             # the most taps; tiles of rows of a strided dy
+    dict(dt="float32", n=3, c=4, hw=(6, 12), rs=(3, 3), p=(1, 1, 1, 1, 1, 1), mult=2),       # two output channels per input channel
+    dict(dt="bfloat16", n=520, c=3, hw=(5, 6), rs=(3, 3), p=(1, 1, 1, 1, 1, 1)),             # small planes in groups, a short last group
+])
+def test_depthwise_conv_and_gradients(gpu, case):
+    """The depthwise kernels (planes staged in LDS) against float64 shift-and-add over the taps: forward, input gradient (as many
+    output as input channels) and weight gradient.  Products of 16-bit values are exact in float32 and sums run in float32: the
+    error is at most (terms) * 2^-24 of the sum of the terms' magnitudes, plus one narrowing of a 16-bit result (2^-7, 2^-10)."""
+    rng = np.random.default_rng(41)
+    dt, N, C, (H, W), (R, S), m = case["dt"], case["n"], case["c"], case["hw"], case["rs"], case.get("mult", 1)
+    sh, sw, ph, pw, dh, dw_ = case["p"]
+    out = case.get("out", "float32")
+    OH, OW = (H + 2 * ph - dh * (R - 1) - 1) // sh + 1, (W + 2 * pw - dw_ * (S - 1) - 1) // sw + 1
+    narrow = {"float32": lambda a: a.astype(np.float32), "bfloat16": _bf16, "float16": lambda a: a.astype(np.float16)}[dt]
+    widen = {"float32": lambda a: a, "bfloat16": lambda a: O.BF16(a).to_f32(), "float16": lambda a: a.astype(np.float32)}
+    xb, wb, db = (narrow(rng.standard_normal(s)) for s in ((N, C, H, W), (C * m, 1, R, S), (N, C * m, OH, OW)))
+    xf, wf, df = (widen[dt](a).astype(np.float64) for a in (xb, wb, db))
+    p = L.ConvParams(*case["p"])
+    lib = L.load()
+
+    def tensor(raw=None, shape=None, dtype=dt):
+        v = jt.from_storage(raw, dtype) if raw is not None else jt.zeros(shape, dtype) + 7.0
+        jt.sync([v], True)
+        return v, L.tensor(v.raw_ptr(), dtype, v.shape)
+
+    (vx, tx), (vw, tw), (vd, td) = tensor(xb), tensor(wb), tensor(db)
+    (vy, ty), (vdx, tdx), (vdw, tdw) = tensor(shape=df.shape, dtype=out), tensor(shape=xf.shape, dtype=out), tensor(shape=wf.shape, dtype=out)
+    L.check(lib.mjt_conv2d_meta_grouped(ctypes.byref(tx), ctypes.byref(tw), ctypes.byref(ty), ctypes.byref(p), C))
+    assert "_depthwise" in L.last_kernel()
+    L.check(lib.mjt_conv2d_meta_wgrad_grouped(ctypes.byref(tx), ctypes.byref(td), ctypes.byref(tdw), ctypes.byref(p), C))
+    assert "_depthwise" in L.last_kernel()
+    rc = lib.mjt_conv2d_meta_dgrad_depthwise(ctypes.byref(td), ctypes.byref(tw), ctypes.byref(tdx), ctypes.byref(p), C)
+    assert rc == (0 if m == 1 else L.ERR_UNSUPPORTED)
+    xp = np.pad(xf, ((0, 0), (0, 0), (ph, ph), (pw, pw))).repeat(m, axis=1)
+    want = {k: np.zeros(s) for k, s in (("y", df.shape), ("x", (N, C * m) + xp.shape[2:]), ("w", wf.shape))}
+    size = {k: np.zeros(s.shape) for k, s in want.items()}
+    for r in range(R):
+        for s in range(S):
+            at = np.s_[:, :, r * dh:r * dh + (OH - 1) * sh + 1:sh, s * dw_:s * dw_ + (OW - 1) * sw + 1:sw]
+            tap = wf[:, 0, r, s][None, :, None, None]
+            for acc, f in ((want, lambda a: a), (size, np.abs)):
+                acc["y"] += f(xp[at] * tap)
+                acc["x"][at] += f(df * tap)
+                acc["w"][:, 0, r, s] = f(df * xp[at]).sum((0, 2, 3))
+    inner = np.s_[:, :, ph:ph + H, pw:pw + W]
+    eps = {"float32": 0.0, "bfloat16": 2.0 ** -7, "float16": 2.0 ** -10}[out]
+    checks = [("y", vy, want["y"], size["y"], R * S), ("w", vdw, want["w"], size["w"], N * OH * OW)]
+    if m == 1:
+        checks.append(("x", vdx, want["x"][inner], size["x"][inner], R * S))
+    for name, v, ref, mag, terms in checks:
+        got = widen[out](L.d2h(v.raw_ptr(), v.shape, L.NP_STORAGE[out]))
+        assert np.all(np.abs(got - ref) <= terms * 2.0 ** -24 * mag + eps * np.abs(ref) + 2.0 ** -24 * (out == "float16")), name
