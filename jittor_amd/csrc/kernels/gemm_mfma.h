@@ -38,6 +38,14 @@
 // y[image][k][oh][ow].
 // Geometry comes as C_, H_, W_, K_, R_, S_, OH_, OW_, SH, SW, PH, PW, DH, DW; N = images * OH_ * OW_.
 //
+// CONV = 2 makes it the weight gradient of that convolution (opt/tuner/conv_tuner.cc:375-397):
+//   dw[k][(c, r, s)] = sum over q = (image, oh, ow) of dy[image][k][oh][ow] * x[image][c][oh*SH-PH+r*DH][ow*SW-PW+s*DW]
+// A = dy with rows k, B' = the shifted planes of x with columns (c, r, s), both with the summed index q innermost, gathered on their
+// way to LDS: a lane owns one chunk of EPC pixels per stage and works out their image, row and column once for all rows and
+// columns it loads; a chunk of dy is one 16-byte load where a plane is whole chunks, x is loaded by elements.  The sum over q is cut into slices of a[9] stages; the slices' float32 partial
+// results are added up by a reduce launch.  Before, the shifted planes were written to memory, multiplied image by image
+// and the images' results added (float32 32 x 3 x 224 x 224, 7x7 stride 2 -> 64: 110 + 337 + 9 us; 116 here).
+//
 // Rows of A' and columns of B' beyond M and N are read from the last valid row (their
 // results are not stored); k beyond K is zeroed in both operands.  Leading dimensions are
 // multiples of 16 bytes and the operand pointers 16-byte aligned (the host sends
@@ -215,7 +223,7 @@ template <int ROWS, bool KCONT> struct mjt_stager {
     }
 };
 
-#if CONV
+#if CONV == 1
 // The B tile of a stage of the implicit-GEMM convolution.  Same blocks as mjt_stager<TN, false>: EPC lanes hold EPC
 // k-rows x EPC columns (4 x 4 float32 values, 8 x 8 16-bit ones), lane tid % EPC the k-row.  What depends on a column
 // alone (its image and pixel) is worked out once per workgroup (mjt_conv_cols): base = element offset of
@@ -292,11 +300,139 @@ struct mjt_conv_stager {
 };
 #endif
 
+#if CONV == 2
+constexpr int P_ = OH_ * OW_;
+constexpr int ESZ = (int)sizeof(TIN);
+#define MJT_NONE 0x80000000u         // an offset beyond every buffer (they are smaller than 2 GB): the load delivers zeros
+// The pixels of the lane's chunk of a stage (chunk tid % KC), the same for all rows and columns that it loads.  All loads go
+// through buffer descriptors, unconditionally: what lies outside the image or past the sum gets an offset past the buffer's
+// end and reads zero, so nothing has to be looked at before it is written to LDS.
+struct mjt_wg_chunk {
+    static constexpr int NDY = P_ % EPC == 0 ? 1 : EPC;
+    unsigned dy[NDY];                // byte offset of dy[image][0][pixel], or MJT_NONE
+    unsigned x[EPC];                 // byte offset of x[image][0][oh*SH-PH][ow*SW-PW] (may wrap below zero)
+    unsigned hw[EPC];                // that row and column, both biased by 0x4000; 0 for a pixel past the sum
+    __device__ __forceinline__ void at(int k0, int K, int tid) {
+        const int q = k0 + (tid % KC) * EPC;
+        mjt_static_for<0, EPC>([&](auto ec) {
+            constexpr int e = decltype(ec)::v;
+            constexpr bool decode = OW_ % EPC != 0 || e == 0;          // a row of outputs is whole chunks: neighbours of the first
+            if constexpr (decode || (NDY > 1 && e < NDY)) {
+                const int qe = q + e;
+                const int img = qe / P_, px = qe - img * P_;
+                if constexpr (e < NDY) dy[e] = qe < K ? (unsigned)(img * (K_ * P_) + px) * ESZ : MJT_NONE;
+                const int oh = px / OW_, ow = px - oh * OW_;
+                const int ih = oh * SH - PH, iw = ow * SW - PW;
+                x[e] = (unsigned)((img * C_ * H_ + ih) * W_ + iw) * ESZ;
+                hw[e] = qe < K ? ((unsigned)(ih + 0x4000) << 16) | (unsigned)(iw + 0x4000) : 0u;
+            } else {
+                x[e] = x[0] + e * SW * ESZ;
+                hw[e] = hw[0] + e * SW;                                // (0 + e * SW stays far below the bias)
+            }
+        });
+    }
+};
+__device__ __forceinline__ mjt_u32x4v mjt_wg_pack(const unsigned (&v)[EPC]) {
+    mjt_u32x4v r;
+#if IN == 2
+    r[0] = v[0]; r[1] = v[1]; r[2] = v[2]; r[3] = v[3];
+#else
+    r[0] = v[0] | (v[1] << 16); r[1] = v[2] | (v[3] << 16); r[2] = v[4] | (v[5] << 16); r[3] = v[6] | (v[7] << 16);
+#endif
+    return r;
+}
+__device__ __forceinline__ unsigned mjt_wg_load(__amdgpu_buffer_rsrc_t d, unsigned off) {
+#if IN == 2
+    return __builtin_amdgcn_raw_buffer_load_b32(d, (int)off, 0, 0);
+#else
+    return (unsigned short)__builtin_amdgcn_raw_buffer_load_b16(d, (int)off, 0, 0);
+#endif
+}
+struct mjt_wg_dy {
+    static constexpr int PER = TM * KC / NTHR;
+    mjt_u32x4v reg[PER];
+    unsigned row[PER];               // byte offset of the lane's rows inside an image of dy
+    __device__ __forceinline__ void init(int m0, int M, int tid) {
+        mjt_static_for<0, PER>([&](auto ic) {
+            const int r = m0 + tid / KC + decltype(ic)::v * (NTHR / KC);
+            row[decltype(ic)::v] = (unsigned)((r < M ? r : M - 1) * P_) * ESZ;
+        });
+    }
+    __device__ __forceinline__ void fetch(__amdgpu_buffer_rsrc_t d, const mjt_wg_chunk& ch) {
+        mjt_static_for<0, PER>([&](auto ic) {
+            constexpr int i = decltype(ic)::v;
+            if constexpr (mjt_wg_chunk::NDY == 1) {
+                reg[i] = __builtin_amdgcn_raw_buffer_load_b128(d, (int)((ch.dy[0] + row[i]) | (ch.dy[0] & MJT_NONE)), 0, 0);
+            } else {
+                unsigned v[EPC];
+                mjt_static_for<0, EPC>([&](auto ec) { constexpr int e = decltype(ec)::v; v[e] = mjt_wg_load(d, (ch.dy[e] + row[i]) | (ch.dy[e] & MJT_NONE)); });
+                reg[i] = mjt_wg_pack(v);
+            }
+        });
+    }
+    __device__ __forceinline__ void commit(unsigned char* lds, int tid) const {
+        mjt_static_for<0, PER>([&](auto ic) {
+            constexpr int i = decltype(ic)::v;
+            *(mjt_u32x4v*)(lds + (tid / KC + i * (NTHR / KC)) * ROWB + (tid % KC) * 16) = reg[i];
+        });
+    }
+};
+struct mjt_wg_x {
+    static constexpr int PER = TN * KC / NTHR;
+    unsigned v[PER][EPC];
+    unsigned koff[PER], dhw[PER];    // of the lane's columns (c, r, s): byte offset inside an image, row and column shift
+    __device__ __forceinline__ void init(int n0, int N, int tid) {
+        mjt_static_for<0, PER>([&](auto ic) {
+            constexpr int i = decltype(ic)::v;
+            int k = n0 + tid / KC + i * (NTHR / KC);
+            k = k < N ? k : N - 1;
+            const int c = k / (R_ * S_), rs = k - c * (R_ * S_), r = rs / S_, t = rs - r * S_;
+            koff[i] = (unsigned)((c * H_ + r * DH) * W_ + t * DW) * ESZ;
+            dhw[i] = ((unsigned)(r * DH) << 16) | (unsigned)(t * DW);
+        });
+    }
+    __device__ __forceinline__ void fetch(__amdgpu_buffer_rsrc_t d, const mjt_wg_chunk& ch) {
+        mjt_static_for<0, PER>([&](auto ic) {
+            constexpr int i = decltype(ic)::v;
+            mjt_static_for<0, EPC>([&](auto ec) {
+                constexpr int e = decltype(ec)::v;
+                const unsigned h = ch.hw[e] + dhw[i];
+                const bool in = (h >> 16) - 0x4000u < (unsigned)H_ && (h & 0xffffu) - 0x4000u < (unsigned)W_;
+                v[i][e] = mjt_wg_load(d, in ? ch.x[e] + koff[i] : MJT_NONE);
+            });
+        });
+    }
+    __device__ __forceinline__ void commit(unsigned char* lds, int tid) const {
+        mjt_static_for<0, PER>([&](auto ic) {
+            constexpr int i = decltype(ic)::v;
+            *(mjt_u32x4v*)(lds + (tid / KC + i * (NTHR / KC)) * ROWB + (tid % KC) * 16) = mjt_wg_pack(v[i]);
+        });
+    }
+};
+#endif
+
 extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
     const int M = (int)(long long)p.a[3], N = (int)(long long)p.a[4], K = (int)(long long)p.a[5];
     const long long lda = (long long)p.a[6], ldb = (long long)p.a[7], ldc = (long long)p.a[8];
+#if CONV == 2
+    const TIN* __restrict__ A = (const TIN*)p.a[0];
+    const TIN* __restrict__ B = (const TIN*)p.a[1];
+    const __amdgpu_buffer_rsrc_t dy_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, (int)(K * K_) * ESZ, 0x00020000);
+    const __amdgpu_buffer_rsrc_t x_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, (int)(long long)p.a[10], 0x00020000);   // a[10]: bytes of x
+    // Workgroups go round-robin over the 8 XCDs: every XCD takes a run of neighbouring (slice, tile) pairs, so that the tiles
+    // of one slice, which read the same dy and x, run next to each other and share an L2 (64 x 64 x 56 x 56, 3x3 -> 64: 269 us
+    // with the tiles dealt out one by one, 162 with runs).
+    const int slice_tiles = (M + TM - 1) / TM * ((N + TN - 1) / TN);
+    const int per_slice = (int)(long long)p.a[9];
+    const int pairs = ((K + KS - 1) / KS + per_slice - 1) / per_slice * slice_tiles, run = (pairs + 7) / 8;
+    const int pair = (int)(blockIdx.x & 7) * run + (int)(blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= run || pair >= pairs) return;
+    const int slice = pair / slice_tiles;
+    const int first_stage = slice * per_slice;
+#else
     const TIN* __restrict__ A = (const TIN*)p.a[0] + (long long)blockIdx.y * (long long)p.a[9];
     const TIN* __restrict__ B = (const TIN*)p.a[1] + (long long)blockIdx.y * (long long)p.a[10];
+#endif
     // NBUF 1: the host promises K <= KS, a single stage -- one staging buffer, so twice as many workgroups fit a compute unit
     __shared__ __attribute__((aligned(16))) unsigned char lds[NBUF][(TM + TN) * ROWB];
 
@@ -306,11 +442,15 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
     const int tiles_m = (M + TM - 1) / TM, tiles_n = (N + TN - 1) / TN;
     const int tiles = tiles_m * tiles_n;
     int L = blockIdx.x;
+#if CONV == 2
+    L = pair - slice * slice_tiles;
+#else
     {
         const int per_xcd = (tiles + 7) / 8;
         L = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
         if (L >= tiles || (blockIdx.x >> 3) >= per_xcd) return;
     }
+#endif
     int tm, tn;
     {
         const int panel = L / (4 * tiles_n);
@@ -327,7 +467,27 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
     // is shorter than a trip to memory, so those keep two stages in registers (2048^3 bfloat16: 31.7 -> 30.6 us; tiles
     // of 64 x 64: 40.8 -> 38.6 us).  Larger tiles have no registers to spare, and float32 stages are long enough (two
     // sets: 153 -> 159 us for 2048^3).
-    constexpr int NSET = (NBUF > 1 && MI * NI <= 4 && IN != 2 && !CONV) ? 2 : 1;
+        constexpr int NSET = (NBUF > 1 && MI * NI <= 4 && IN != 2 && !CONV) ? 2 : 1;
+#if CONV == 2
+    const int all_stages = (K + KS - 1) / KS;
+    const int nstages = all_stages - first_stage < per_slice ? all_stages - first_stage : per_slice;
+    mjt_wg_dy sa[NSET];
+    mjt_wg_x sb[NSET];
+    mjt_static_for<0, NSET>([&](auto tc) { sa[decltype(tc)::v].init(m0, M, tid); sb[decltype(tc)::v].init(n0, N, tid); });
+    auto fetch = [&](auto setc, int stage) {
+        constexpr int SET = decltype(setc)::v;
+        mjt_wg_chunk ch;
+        ch.at((first_stage + stage) * KS, K, tid);
+        sa[SET].fetch(dy_rsrc, ch);
+        sb[SET].fetch(x_rsrc, ch);
+    };
+    auto commit = [&](auto setc, int stage) {
+        constexpr int SET = decltype(setc)::v;
+        unsigned char* buf = &lds[stage & (NBUF - 1)][0];
+        sa[SET].commit(buf, tid);
+        sb[SET].commit(buf + TM * ROWB, tid);
+    };
+#else
     const int nstages = NBUF == 1 ? 1 : (K + KS - 1) / KS;
     mjt_stager<TM, A_KCONT> sa[NSET];
     const int arows = M, brows = N;
@@ -357,6 +517,7 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
         sb[SET].commit(buf + TM * ROWB, stage * KS, K, tid);
 #endif
     };
+#endif
     mjt_static_for<0, NSET>([&](auto tc) {
         if (decltype(tc)::v < nstages) fetch(tc, decltype(tc)::v);
     });
@@ -425,7 +586,11 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
 
     // D of a 32x32 tile: lane holds column lane % 32, rows 8 * (e / 4) + 4 * (lane / 32) + e % 4
 #if OUT == 2
+#if CONV == 2
+    float* __restrict__ C = (float*)p.a[2] + (long long)slice * (long long)p.a[11];
+#else
     float* __restrict__ C = (float*)p.a[2] + (long long)blockIdx.y * (long long)p.a[11];
+#endif
 #else
     unsigned short* __restrict__ C = (unsigned short*)p.a[2] + (long long)blockIdx.y * (long long)p.a[11];
 #endif
@@ -434,7 +599,7 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
 #pragma unroll
         for (int j = 0; j < NI; j++) {
             const int col = n0 + wn * 32 * NI + j * 32 + (lane & 31);
-#if CONV
+#if CONV == 1
             const int img = col / (OH_ * OW_), px = col - img * (OH_ * OW_);      // y[img][row][px]
 #endif
 #pragma unroll
@@ -442,7 +607,7 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
                 const int row = m0 + wm * 32 * MI + i * 32 + 8 * (e / 4) + 4 * (lane >> 5) + (e & 3);
                 if (row < M && col < N) {
                     const float v = acc[i][j][e];
-#if CONV
+#if CONV == 1
                     const long long at = ((long long)img * K_ + row) * (OH_ * OW_) + px;
 #else
                     const long long at = (long long)row * ldc + col;

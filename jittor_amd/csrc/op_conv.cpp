@@ -3,6 +3,7 @@
 // python/jittor/src/opt/tuner/conv_tuner.cc:312-356).
 #include "common.h"
 #include <array>
+#include <cmath>
 #include <mutex>
 #include <unordered_map>
 
@@ -708,6 +709,70 @@ static void conv_wgrad_direct(const mjt_tensor* x, const mjt_tensor* dy, const m
     set_last_kernel(k->name.c_str());
 }
 
+// Weight gradient as an implicit product (kernels/gemm_mfma.h with CONV 2): both operands are gathered on their way to LDS and
+// the sum over images and pixels is cut into slices.  False: not covered.
+static bool conv_wgrad_product(const mjt_tensor* x, const mjt_tensor* dy, const mjt_tensor* dw, const mjt_conv_params* p) {
+    const int64_t N = x->shape[0], C = x->shape[1], H = x->shape[2], W = x->shape[3];
+    const int64_t K = dy->shape[1], OH = dy->shape[2], OW = dy->shape[3], R = dw->shape[2], S = dw->shape[3];
+    const int64_t P = OH * OW, CRS = C * R * S, Q = N * P;
+    if (x->dtype != MJT_FLOAT32 || dy->dtype != x->dtype || dw->dtype != MJT_FLOAT32 || getenv("MJT_NO_FASTPATH") || getenv("MJT_CONV_NO_IGEMM")) return false;
+    // (offsets inside x and dy are 32-bit elements, rows and columns 14-bit; a few million multiply-adds are worth the set-up)
+    if ((double)Q * K * CRS < (double)(1 << 22) || Q >= (int64_t(1) << 31) - 64 ||
+        numel(x) * 4 >= (int64_t(1) << 31) || numel(dy) * 4 >= (int64_t(1) << 31) || H >= 16384 || W >= 16384 || (R - 1) * p->dil_h >= 16384 || (S - 1) * p->dil_w >= 16384 || p->pad_h >= 16384 || p->pad_w >= 16384 ||
+        OH * p->stride_h >= 16384 || OW * p->stride_w >= 16384 || (uintptr_t)dy->ptr % 16)
+        return false;
+    const int64_t cus = ctx().dry_run || ctx().prop.multiProcessorCount <= 0 ? 256 : ctx().prop.multiProcessorCount;
+    const int in = 2, KS = 32;
+    // 128 x 128 tiles gather half as much per multiply-add and hold two workgroups a compute unit, 64 x 64 tiles waste less on
+    // the edges and hold four (us at 3x3, 64 / 128: 64 x 64 x 56 x 56 -> 64: 162 / 447; 64 x 128 x 28 x 28 -> 128: 161 / 155;
+    // 64 x 256 x 14 x 14 -> 256: 180 / 150; 64 x 512 x 7 x 7 -> 512: 195 / 176)
+    auto tiles_of = [&](int64_t t) { return ((K + t - 1) / t) * ((CRS + t - 1) / t); };
+    const int MI = tiles_of(128) * 4 * 0.85 <= (double)tiles_of(64) ? 2 : 1, NI = MI;
+    const int64_t tiles = tiles_of(64 * MI);
+    // slices of the sum: one, two or three full rounds of workgroups, whichever leaves fewest places empty, of at least 8 stages
+    // each (one workgroup more than a round costs a round: 64 x 256 x 14 x 14 -> 256 in 14 slices 150, in 15 slices 212)
+    const int64_t stages = (Q + KS - 1) / KS, places = cus * (MI == 1 ? 4 : 2);
+    int64_t slices = 1;
+    double best = 0.0;
+    for (int64_t r = 1; r <= 3; r++) {
+        int64_t n = r * places / tiles;
+        if (n > stages / 8) n = stages / 8;
+        if (n < 1) n = 1;
+        const double wgs = (double)(n * tiles), full = wgs / (std::ceil(wgs / places) * places);
+        if (full > best + 0.05) { best = full; slices = n; }
+    }
+    if (slices * numel(dw) * 4 > (int64_t(1) << 30)) return false;
+    const int64_t per = (stages + slices - 1) / slices;
+    slices = (stages + per - 1) / per;
+    std::ostringstream key;
+    key << "wgprod|" << C << "|" << H << "|" << W << "|" << K << "|" << R << "|" << S << "|" << OH << "|" << OW << "|" << p->stride_h << "|" << p->stride_w << "|" << p->pad_h << "|" << p->pad_w
+        << "|" << p->dil_h << "|" << p->dil_w << "|" << MI << NI << in;
+    JitKernel* k = cached(key.str());
+    if (!k) {
+        std::ostringstream name;
+        name << "mjt_conv_wgrad_igemm_" << mjt_dtype_name(x->dtype) << "_c" << C << "_k" << K << "_" << H << "x" << W << "_r" << R << "x" << S << "_s" << p->stride_h << "x" << p->stride_w << "_p"
+             << p->pad_h << "x" << p->pad_w << "_d" << p->dil_h << "x" << p->dil_w << "_" << 64 * MI << "x" << 64 * NI;
+        std::ostringstream src;
+        src << "#define ENTRY " << name.str() << "\n#define CONV 2\n#define IN " << in << "\n#define OUT 2\n#define MI " << MI << "\n#define NI " << NI << "\n#define A_KCONT 1\n#define B_KCONT 1"
+            << "\n#define C_ " << C << "\n#define H_ " << H << "\n#define W_ " << W << "\n#define K_ " << K << "\n#define R_ " << R << "\n#define S_ " << S << "\n#define OH_ " << OH
+            << "\n#define OW_ " << OW << "\n#define SH " << p->stride_h << "\n#define SW " << p->stride_w << "\n#define PH " << p->pad_h << "\n#define PW " << p->pad_w << "\n#define DH " << p->dil_h
+            << "\n#define DW " << p->dil_w << "\n";
+        src << embedded_source("gemm_mfma.h") << "\n";
+        k = jit_get(src.str(), name.str());
+        remember(key.str(), k);
+    }
+    const bool in_place = slices == 1 && dw->dtype == MJT_FLOAT32;
+    void* part = in_place ? dw->ptr : wgrad_partials((size_t)slices * (size_t)numel(dw) * 4);
+    std::vector<uint64_t> a{bits_of_ptr(dy->ptr), bits_of_ptr(x->ptr), bits_of_ptr(part), (uint64_t)K, (uint64_t)CRS, (uint64_t)Q, 0, 0, (uint64_t)CRS, (uint64_t)per,
+                            (uint64_t)(numel(x) * 4), (uint64_t)(K * CRS)};
+    const int64_t grid = (slices * tiles + 7) / 8 * 8;
+    MJT_CHECK(grid < (int64_t(1) << 31), "conv wgrad: launch too large");
+    jit_launch(k, (unsigned)grid, 1, 256, 0, a);
+    if (!in_place) fold_wgrad_slices(part, slices, dw);
+    set_last_kernel(k->name.c_str());
+    return true;
+}
+
 // Weight gradient: dw[k,c,r,s] = sum_{n,oh,ow} dy[n,k,oh,ow] * x[n,c,oh*sh-ph+r*dh,ow*sw-pw+s*dw].
 // With `any_shape` (the grouped entry point) what the MFMA kernel does not cover runs on the direct kernel instead of
 // being handed back; G > 1: x has G groups of dw->shape[1] channels, dy G groups of K / G (python/jittor/nn.py:1272-1294).
@@ -742,6 +807,7 @@ void conv_wgrad_impl(const mjt_tensor* x, const mjt_tensor* dy, const mjt_tensor
                     W % 2 == 0 && N >= 1 && numel(x) * 2 < (int64_t(1) << 31) && numel(dy) * 2 < (int64_t(1) << 31) &&
                     (uintptr_t)x->ptr % 4 == 0 && (uintptr_t)dy->ptr % 16 == 0 &&
                     !getenv("MJT_NO_FASTPATH");
+    if (!ok && G == 1 && N >= 1 && conv_wgrad_product(x, dy, dw, p)) return;
     if (!ok && any_shape) {
         conv_wgrad_direct(x, dy, dw, p, G);
         return;

@@ -1140,14 +1140,16 @@ def _run_single(op):
         # (the kernel walks rows in chunks of 32 output columns: a width that fills less than 0.6 of its chunks and is no
         # multiple of 8 is better off as a product, 64 x 256 x 14 x 14 3x3: 68 us on the kernel, 59 as the product below)
         narrow = OW % 8 != 0 and OW < 0.6 * 32 * -(-OW // 32)
-        if x.dtype in ("bfloat16", "float16") and flags["enable_conv_wgrad_kernel"] and not narrow:
-            # the MFMA kernel; shapes it does not cover come back as unsupported and take the paths below
+        half = x.dtype in ("bfloat16", "float16")
+        if (half and not narrow or x.dtype == "float32") and flags["enable_conv_wgrad_kernel"]:
+            # 16-bit: the MFMA kernel; float32: the product that gathers its operands; shapes they do not cover come back as
+            # unsupported and take the paths below
             tx, td = _tensor_of(x), _tensor_of(dy)
             tw = _tensor(_alloc_out(out), out.dtype, out.shape)
             p = _lib.ConvParams(sh, sw, ph, pw, dh, dw)
             rc = lib.mjt_conv2d_meta_wgrad(ctypes.byref(tx), ctypes.byref(td), ctypes.byref(tw), ctypes.byref(p))
             if rc == 0:
-                stats["wgrad_kernel"] += 1
+                stats["wgrad_kernel"] += half
                 return
             if rc != _lib.ERR_UNSUPPORTED:
                 _lib.check(rc)

@@ -441,3 +441,40 @@ def test_small_cnn_step_with_and_without_the_executor_rewrites(gpu):
         assert a.shape == b.shape
         close(a, b, rtol=2e-4, atol=2e-5)
     assert np.isfinite(fast[0]).all() and float(fast[0][0]) > 0
+
+
+@pytest.mark.parametrize("xs,k,rs,stride,pad,dil", [
+    ((4, 16, 32, 32), 64, (3, 3), 1, 1, 1),             # rows of whole chunks, one tile of output channels
+    ((3, 20, 31, 29), 65, (3, 3), 1, 1, 1),             # planes that are no whole chunks, one channel and a few columns past a tile
+    ((2, 3, 65, 64), 64, (7, 7), 2, 3, 1),              # an image stem: two columns of tiles, the second part empty
+    ((5, 40, 15, 13), 130, (5, 3), 2, 2, 1),            # 128 x 128 tiles with a second row of tiles; windows that are not square
+    ((2, 64, 14, 14), 129, (3, 3), 1, 2, 2),            # dilated taps
+    ((40, 64, 3, 3), 128, (3, 3), 1, 1, 1),             # planes smaller than two chunks: a chunk spans images
+    ((256, 128, 1, 1), 256, (1, 1), 1, 0, 1),           # planes of one pixel: a product
+])
+def test_grad_conv_weight_float32_gathered_product(gpu, xs, k, rs, stride, pad, dil):
+    """Weight gradient of float32 convolutions as a product that gathers dy and x (kernels/gemm_mfma.h, CONV 2) against the float64
+    gradient: a sum of n float32 products taken in any order is off by at most n * 2^-24 of the sum of their magnitudes."""
+    rng = np.random.default_rng(19)
+    x = rng.standard_normal(xs).astype(np.float32)
+    N, C, H, W = xs
+    R, S = rs
+    OH, OW = (H + 2 * pad - dil * (R - 1) - 1) // stride + 1, (W + 2 * pad - dil * (S - 1) - 1) // stride + 1
+    dy = rng.standard_normal((N, k, OH, OW)).astype(np.float32)
+    vx, vd, vw = jt.array(x), jt.array(dy), jt.zeros([k, C, R, S]) + 7.0
+    jt.sync([vx, vd, vw], True)
+    import ctypes
+    from jittor_amd import _lib as L
+    tx, td, tw = (L.tensor(v.raw_ptr(), "float32", v.shape) for v in (vx, vd, vw))
+    p = L.ConvParams(stride, stride, pad, pad, dil, dil)
+    L.check(L.load().mjt_conv2d_meta_wgrad(ctypes.byref(tx), ctypes.byref(td), ctypes.byref(tw), ctypes.byref(p)))
+    assert L.last_kernel().startswith("mjt_conv_wgrad_igemm_float32")
+    got = vw.numpy()
+    xp = np.pad(x.astype(np.float64), ((0, 0), (0, 0), (pad, pad), (pad, pad)))
+    d2 = dy.astype(np.float64).transpose(1, 0, 2, 3).reshape(k, -1)
+    for r in range(R):
+        for s in range(S):
+            patch = xp[:, :, r * dil:r * dil + (OH - 1) * stride + 1:stride, s * dil:s * dil + (OW - 1) * stride + 1:stride]
+            p2 = patch.transpose(0, 2, 3, 1).reshape(-1, C)
+            bound = N * OH * OW * 2.0 ** -24 * (np.abs(d2) @ np.abs(p2))
+            assert np.all(np.abs(got[:, :, r, s] - d2 @ p2) <= bound), (r, s)
