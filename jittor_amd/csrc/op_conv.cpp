@@ -74,6 +74,7 @@ bool matmul_available();
 void gemm_launch(int in_dtype, int out_dtype, const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K,
                  int64_t lda, int64_t ldb, int64_t ldc, int64_t sa, int64_t sb, int64_t sc, int64_t batch, bool a_kcont,
                  bool b_kcont, int tile_m = 0, int tile_n = 0, bool allow_direct = true);
+bool gemm_pixels(int in_dtype, int out_dtype, const void* A, const void* x, void* y, int64_t M, int64_t K, int64_t P, int64_t images, bool a_kcont);
 
 // ---- depthwise convolution (kernels/conv_depthwise.h) ----------------------------------
 namespace {
@@ -195,6 +196,14 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
     MJT_CHECK(numel(x) < (int64_t(1) << 40) && numel(y) < (int64_t(1) << 40), "conv: too large");
     Context& c = ctx();
 
+    // a 1x1 convolution on large enough planes of an even number of pixels: one product for the batch, x read as it lies
+    if (G == 1 && R == 1 && S == 1 && p->stride_h == 1 && p->stride_w == 1 && p->pad_h == 0 && p->pad_w == 0 && OH == H && OW == W && pack_mode == 0 &&
+        !getenv("MJT_NO_FASTPATH") && !getenv("MJT_CONV_NO_GEMM") && !getenv("MJT_CONV_FLAT") && (double)N * K * C * H * W >= (double)(1 << 22) &&
+        gemm_pixels(x->dtype, y->dtype, w->ptr, x->ptr, y->ptr, K, C, H * W, N, true)) {
+        set_last_kernel("conv_as_gemm");
+        return;
+    }
+
     std::ostringstream geo;
     geo << "#define C_ " << C << "\n#define H_ " << H << "\n#define W_ " << W << "\n#define K_ " << K << "\n#define R_ " << R
         << "\n#define S_ " << S << "\n#define OH_ " << OH << "\n#define OW_ " << OW << "\n#define SH " << p->stride_h
@@ -285,7 +294,7 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
                          // measured (64 x 512 x 28 x 28 -> 128 channels: 22 us against 42; 64 x 256 x 56 x 56 -> 64: 31 against
                          // 73; 64 x 1024 x 16 x 16 -> 2048: 82 against 387; closest 64 x 512 x 28 x 28 -> 512: 74 against 74),
                          // this kernel walking one-step channel blocks.  With other plane sizes the product kernel gathers x
-                         // (its CONV mode), which wins with more than 64 output channels and enough 128 x 64 tiles for the chip
+                         // (its CONV mode; long sums have gone to the product over pieces above), which wins with more than 64 output channels and enough 128 x 64 tiles for the chip
                          // (64 x 512 x 14 x 14 -> 512: 36 against 61; 64 x 1024 x 14 x 14 -> 512: 63 against 100; -> 256: 37
                          // against 142) and with many more input than output channels and few output channels or a small map
                          !(R * S == 1 && G == 1 && p->stride_h == 1 && p->stride_w == 1 && matmul_available() && !getenv("MJT_CONV_NO_GEMM") &&
@@ -1002,6 +1011,12 @@ void conv_dgrad_impl(const mjt_tensor* dy, const mjt_tensor* w, const mjt_tensor
         mjt_tensor tp = view(part, dx->dtype, {sh * sw, N, C, Hs, Ws});
         reindex(tp, *dx, {"i2%" + str(sh) + "*" + str(sw) + "+i3%" + str(sw), "i0", "i1", "i2/" + str(sh), "i3/" + str(sw)}, {});
         set_last_kernel(("conv_dgrad_phases:" + kernels).c_str());
+        return;
+    }
+    // a 1x1 convolution: the product takes the weights as they lie
+    if (R == 1 && S == 1 && sh == 1 && sw == 1 && ph == 0 && pw == 0 && !getenv("MJT_NO_FASTPATH") && !getenv("MJT_CONV_NO_GEMM") &&
+        (double)N * K * C * H * W >= (double)(1 << 22) && gemm_pixels(dy->dtype, dx->dtype, w->ptr, dy->ptr, dx->ptr, C, K, H * W, N, false)) {
+        set_last_kernel("conv_as_gemm");
         return;
     }
     mjt_tensor tw = view(wbuf, w->dtype, {C, K, R, S});

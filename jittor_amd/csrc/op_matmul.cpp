@@ -187,6 +187,49 @@ void gemm_launch(int in_dtype, int out_dtype, const void* A, const void* B, void
                                     nullptr, config));
 }
 
+// 1x1 convolution of stride 1 over a batch of planes that need not be 16-byte multiples (kernels/gemm_dma.h with IMG):
+// y[image][m][p] = sum over k of A'[m][k] * x[image][k][p], 16-bit operands, an even number of pixels.  a_kcont: A' = A [M][K], else
+// A [K][M] (the input gradient takes the weights as they lie).  False: not covered.
+bool gemm_pixels(int in_dtype, int out_dtype, const void* A, const void* x, void* y, int64_t M, int64_t K, int64_t P, int64_t images, bool a_kcont) {
+    Context& c = ctx();
+    const int64_t lda = a_kcont ? K : M, pieces = (P + 7) / 8, N = images * pieces * 8;
+    if ((in_dtype != MJT_BFLOAT16 && in_dtype != MJT_FLOAT16) || !(out_dtype == MJT_FLOAT32 || out_dtype == in_dtype) || K % 64 || P % 2 || K < 64 ||
+        lda % 8 || (uintptr_t)A % 16 || (uintptr_t)x % 4 || images * K * P * 2 >= (int64_t(1) << 31) || N >= (int64_t(1) << 31) || M * P >= (int64_t(1) << 31) ||
+        (a_kcont ? lda * 2 * 256 : lda * 2 * K) >= (int64_t(1) << 31) || getenv("MJT_GEMM_NO_DMA"))
+        return false;
+    const int64_t cus = c.dry_run || c.prop.multiProcessorCount <= 0 ? 256 : c.prop.multiProcessorCount;
+    // 128 x 128 tiles, also where they are few: the alternatives gather x by elements or run image by image (us at 64 images,
+    // forward, before / tiles of 128 / of 256: 1024 x 14 x 14 -> 256: 37.9 / 14.1 / 31.2; 256 x 14 x 14 -> 1024: 40.2 / 18.7 / 20.8;
+    // 512 x 28 x 28 -> 128: 20.0 / 15.4 / 24.8; 256 x 28 x 28 -> 512: 36.7 / 31.5 / 35.2; 8 images of 1024 x 14 x 14 -> 256: 24.7 / 11.5 /
+    // 29.3).  Not for a half-empty tile of output channels where the plain product per image takes the planes (256 x 56 x 56 -> 64:
+    // 37.8 / 40.6), nor, in the forward direction, for short sums and a handful of tiles of odd-sized planes, where little is to be
+    // had (64 x 14 x 14 -> 64: 9.0 / 6.1; 128 x 28 x 28 -> 128: 10.9 / 9.5) and the convolution kernels stay; an input gradient also
+    // saves the transposed copy of the weights (the same two: 11.9 / 5.9, 15.1 / 9.7).
+    const int tile = 128;
+    const int64_t tm = (M + tile - 1) / tile, tn = (N + tile - 1) / tile;
+    if (P % 8 == 0 ? (double)M < 0.7 * (double)(tm * tile) && tm * tn > cus : a_kcont && (K < 256 || tm * tn < 16)) return false;
+    const int in = in_dtype == MJT_BFLOAT16 ? 0 : 1, out = out_dtype == MJT_BFLOAT16 ? 0 : out_dtype == MJT_FLOAT16 ? 1 : 2;
+    const int nbuf = tm * tn > cus ? 2 : 4, wpe = nbuf == 2 ? 2 : 1;      // as for the plain product: two workgroups a unit, or a deeper ring
+    std::ostringstream key;
+    key << "gemmpx|" << in << out << a_kcont << tile << nbuf << "|" << P;
+    JitKernel* k = cached(key.str());
+    if (!k) {
+        std::ostringstream name;
+        name << "mjt_gemm_mfma_" << mjt_dtype_name(in_dtype) << "_" << mjt_dtype_name(out_dtype) << "_" << tile << "x" << tile << (a_kcont ? "_n" : "_t") << "_pixels" << P << (wpe == 2 ? "_direct2" : "_direct");
+        std::ostringstream src;
+        src << "#define ENTRY " << name.str() << "\n#define IN " << in << "\n#define OUT " << out << "\n#define A_KCONT " << (a_kcont ? 1 : 0) << "\n#define B_KCONT 0\n#define IMG " << P
+            << "\n#define TILE " << tile << "\n#define NBUF " << nbuf << "\n#define WPE " << wpe << "\n";
+        src << embedded_source("gemm_dma.h") << "\n";
+        k = jit_get(src.str(), name.str());
+        remember(key.str(), k);
+    }
+    if (k->spilled != 0 || k->agprs < 0 || k->agprs > tile * tile / 256) return false;     // (see gemm_launch)
+    std::vector<uint64_t> args{bits_of_ptr(A), bits_of_ptr(x), bits_of_ptr(y), (uint64_t)M, (uint64_t)N, (uint64_t)K, (uint64_t)lda, (uint64_t)(K * P), (uint64_t)(M * P), 0,
+                               (uint64_t)(images * K * P * 2), 0};
+    jit_launch(k, (unsigned)((tm * tn + 7) / 8 * 8), 1, 256, 0, args);
+    return true;
+}
+
 // With `share_a` every matrix of the batch is multiplied by the first matrix of a (batch stride 0: the weights of a
 // convolution against the column matrices of a chunk of images).
 void matmul_impl(const mjt_tensor* a, const mjt_tensor* b, const mjt_tensor* c, int trans_a, int trans_b, bool share_a) {

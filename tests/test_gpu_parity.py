@@ -1052,6 +1052,42 @@ def test_conv_as_reindex_and_gemm(gpu, case, monkeypatch):
     assert np.abs(widen[out](got2) - ref).max() <= tol * np.abs(ref).max()
 
 
+@pytest.mark.parametrize("dt,out,n,c,k,hw", [
+    ("bfloat16", "bfloat16", 64, 256, 130, (2, 7)),      # 14 pixels: the second piece of a plane holds six; two tiles of channels
+    ("float16", "float16", 41, 320, 64, (14, 14)),       # the last piece of the last plane ends past the tensor
+    ("bfloat16", "float32", 33, 256, 192, (10, 25)),     # 250 pixels, more tiles of pixels than a multiple of eight
+    ("bfloat16", "bfloat16", 70, 64, 256, (16, 16)),     # planes of whole pieces, more tiles than compute units
+])
+def test_conv_1x1_on_pieces_of_planes(gpu, dt, out, n, c, k, hw):
+    """A 1x1 convolution and its input gradient as products over the 16-byte pieces of a batch's planes against float64: exact
+    products, float32 sums (at most terms * 2^-24 of the terms' magnitudes) and one narrowing of the result (2^-7, 2^-10)."""
+    rng = np.random.default_rng(43)
+    narrow = {"bfloat16": _bf16, "float16": lambda a: a.astype(np.float16)}[dt]
+    widen = {"float32": lambda a: a, "bfloat16": lambda a: O.BF16(a).to_f32(), "float16": lambda a: a.astype(np.float32)}
+    xb, wb, db = (narrow(rng.standard_normal(s)) for s in ((n, c) + hw, (k, c, 1, 1), (n, k) + hw))
+    xf, wf, df = (widen[dt](a).astype(np.float64) for a in (xb, wb, db))
+    p = L.ConvParams(1, 1, 0, 0, 1, 1)
+    lib = L.load()
+
+    def tensor(raw=None, shape=None, dtype=dt):
+        v = jt.from_storage(raw, dtype) if raw is not None else jt.zeros(shape, dtype) + 7.0
+        jt.sync([v], True)
+        return v, L.tensor(v.raw_ptr(), dtype, v.shape)
+
+    (vx, tx), (vw, tw), (vd, td) = tensor(xb), tensor(wb), tensor(db)
+    (vy, ty), (vdx, tdx) = tensor(shape=df.shape, dtype=out), tensor(shape=xf.shape, dtype=out)
+    L.check(lib.mjt_conv2d_meta(ctypes.byref(tx), ctypes.byref(tw), ctypes.byref(ty), ctypes.byref(p)))
+    assert L.last_kernel() == "conv_as_gemm"
+    L.check(lib.mjt_conv2d_meta_dgrad(ctypes.byref(td), ctypes.byref(tw), ctypes.byref(tdx), ctypes.byref(p)))
+    assert k % 64 or L.last_kernel() == "conv_as_gemm"
+    eps = {"float32": 0.0, "bfloat16": 2.0 ** -7, "float16": 2.0 ** -10}[out]
+    m = wf[:, :, 0, 0]
+    for v, a, b, terms in ((vy, m, xf, c), (vdx, m.T, df, k)):
+        want, mag = (np.matmul(f(a), f(b).reshape(n, terms, -1)) for f in (lambda t: t, np.abs))
+        got = widen[out](L.d2h(v.raw_ptr(), v.shape, L.NP_STORAGE[out])).reshape(want.shape)
+        assert np.all(np.abs(got - want) <= terms * 2.0 ** -24 * mag + eps * np.abs(want) + 2.0 ** -24 * (out == "float16"))
+
+
 def test_conv_1x1_runs_as_a_product(gpu, monkeypatch):
     """A 1x1 convolution of stride 1 is handed to the matrix-product kernel although the MFMA convolution kernel would
     take it: always when a plane's rows are 16-byte multiples (the product then reads x as it lies, with tiles picked for
