@@ -392,6 +392,26 @@ int mjt_matmul_available(void);
 int mjt_expr_affine(const char* expr, const mjt_tensor* x, const mjt_tensor* y,
                     int64_t* c0, int64_t coef[MJT_MAX_DIM]);
 
+/* ---- recorded launches --------------------------------------------------
+ * A program that issues the same calls again and again on other buffers can
+ * keep what they launch.  Between mjt_record_begin and mjt_record_end the
+ * calls of this thread note their kernels and parameter words instead of
+ * launching them.  Two recordings of the same calls, made with stand-in
+ * addresses (base1 / base2, slots `span` bytes apart, 256-byte aligned) and
+ * stand-in scalars, show which words come from which buffer or scalar:
+ * mjt_record_relocate works that out and makes `first` replayable (`second`
+ * is only read).  mjt_record_launch then launches it on real buffers in one
+ * call.  MJT_ERR_UNSUPPORTED: a call that cannot be recorded, a word of other
+ * origin, a buffer that is not 256-byte aligned, or a recording that is out of
+ * date because the library's own scratch memory moved or it was shut down;
+ * nothing has been launched then and the calls themselves are the way. */
+int  mjt_record_begin(void);
+int  mjt_record_end(void** rec);                 /* rec == NULL: drop it */
+int  mjt_record_relocate(void* first, void* second, int n_slots, const uint64_t* base1, const uint64_t* base2, uint64_t span,
+                         int n_scalars, const int64_t* scalar1, const int64_t* scalar2);
+int  mjt_record_launch(void* rec, int n_slots, const uint64_t* bases, int n_scalars, const double* fvalues, const int64_t* ivalues);
+void mjt_record_free(void* rec);
+
 /* Number of kernels specialised at run time so far, and how many launches
  * reused one (the role of jit_ops / jit_fused_ops, op.cc:30, fused_op.cc:18). */
 int mjt_jit_stats(int64_t* compiled, int64_t* cache_hits);

@@ -94,6 +94,7 @@ EXPORTS = ["mjt_init", "mjt_shutdown", "mjt_last_error", "mjt_get_device_info",
            "mjt_fused_elementwise", "mjt_fused_reduce", "mjt_conv2d_meta", "mjt_conv2d_meta_pack", "mjt_conv2d_meta_packed", "mjt_conv2d_meta_grouped", "mjt_conv2d_meta_dgrad", "mjt_conv2d_meta_dgrad_depthwise", "mjt_conv2d_meta_wgrad", "mjt_conv2d_meta_wgrad_grouped",
            "mjt_reindex_then_reduce", "mjt_fused_reindex_reduce", "mjt_matmul", "mjt_matmul_available",
            "mjt_expr_affine", "mjt_where_count", "mjt_where",
+           "mjt_record_begin", "mjt_record_end", "mjt_record_relocate", "mjt_record_launch", "mjt_record_free",
            "mjt_jit_stats", "mjt_last_kernel"]
 
 _lib = None
@@ -160,6 +161,12 @@ def load():
     lib.mjt_where.argtypes = [ctypes.POINTER(Tensor), ctypes.c_int64, ctypes.POINTER(Tensor)]
     lib.mjt_expr_affine.argtypes = [ctypes.c_char_p, ctypes.POINTER(Tensor), ctypes.POINTER(Tensor),
                                     ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_int64)]
+    u64s, i64s = ctypes.POINTER(ctypes.c_uint64), ctypes.POINTER(ctypes.c_int64)
+    lib.mjt_record_end.argtypes = [ctypes.POINTER(ctypes.c_void_p)]
+    lib.mjt_record_relocate.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, u64s, u64s, ctypes.c_uint64, ctypes.c_int, i64s, i64s]
+    lib.mjt_record_launch.argtypes = [ctypes.c_void_p, ctypes.c_int, u64s, ctypes.c_int, ctypes.POINTER(ctypes.c_double), i64s]
+    lib.mjt_record_free.argtypes = [ctypes.c_void_p]
+    lib.mjt_record_free.restype = None
     lib.mjt_jit_stats.argtypes = [ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_int64)]
     _lib = lib
     return lib

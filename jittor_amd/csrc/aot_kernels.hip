@@ -39,7 +39,9 @@ __global__ __launch_bounds__(256) void mjt_fill_pattern_kernel(T* __restrict__ d
 // (identity values of the scatter op).
 void launch_fill_pattern(void* dst, uint64_t pattern, int elem_size, size_t n) {
     Context& c = ctx();
-    if (c.dry_run || n == 0) return;
+    if (n == 0) return;
+    refuse_recording("a fill");
+    if (c.dry_run) return;
     size_t blocks = (n + 256 * 8 - 1) / (256 * 8);
     if (blocks > (size_t)1 << 20) blocks = (size_t)1 << 20;
     set_last_kernel("mjt_fill_pattern_kernel");
@@ -55,6 +57,7 @@ void launch_fill_pattern(void* dst, uint64_t pattern, int elem_size, size_t n) {
 
 void launch_copy(void* dst, const void* src, size_t bytes) {
     Context& c = ctx();
+    refuse_recording("a copy");
     if (c.dry_run) return;
     bool aligned = ((uintptr_t)dst % 16 == 0) && ((uintptr_t)src % 16 == 0);
     size_t n16 = aligned ? bytes / 16 : 0;
@@ -76,6 +79,7 @@ void launch_copy(void* dst, const void* src, size_t bytes) {
 
 void launch_fill_u32(void* dst, uint32_t pattern, size_t n_words) {
     Context& c = ctx();
+    refuse_recording("a fill");
     if (c.dry_run) return;
     size_t blocks = (n_words + 256 * 8 - 1) / (256 * 8);
     if (blocks > (size_t)1 << 20) blocks = (size_t)1 << 20;

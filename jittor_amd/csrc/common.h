@@ -109,7 +109,14 @@ JitKernel* jit_lookup(const std::string& source);
 void reduce_static_setup(int device);
 // Launch with a parameter block of 8-byte words.
 void jit_launch(JitKernel* k, unsigned grid_x, unsigned grid_y, unsigned block, unsigned shmem,
-                const std::vector<uint64_t>& args);
+                const std::vector<uint64_t>& args, unsigned grid_z = 1);
+
+// ---- recorded launches (runtime.cpp) ----------------------------------------
+// While this thread records, jit_launch notes its kernel and parameter words instead of launching.  Whatever acts on the device in
+// another way, or keeps state between calls, calls this first: it throws, and the recording is given up.
+void refuse_recording(const char* what);
+// A buffer that the library keeps between calls has moved (or goes away): recordings made so far may hold its old address.
+void kept_buffer_moved();
 
 // embedded kernel sources (generated from csrc/kernels/)
 const char* embedded_source(const char* name);

@@ -56,6 +56,7 @@ void* conv_scratch(int which, size_t bytes) {
     Context& c = ctx();
     if (c.dry_run) return (void*)(uintptr_t)0x1000;
     if (bytes > g_conv_scratch_bytes[which]) {
+        kept_buffer_moved();
         if (g_conv_scratch[which]) {
             HIP_CHECK(hipStreamSynchronize(c.stream));
             HIP_CHECK(hipFree(g_conv_scratch[which]));
@@ -387,6 +388,7 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
             size_t wbytes = (size_t)numel(w) * 2;
             if (pack_mode) MJT_CHECK(packed && (uintptr_t)packed % 16 == 0, "conv: packed weights must be a 16-byte aligned device buffer");
             if (!pack_mode && !c.dry_run && wbytes > g_wpack_bytes) {
+                kept_buffer_moved();
                 if (g_wpack) {
                     HIP_CHECK(hipStreamSynchronize(c.stream));
                     HIP_CHECK(hipFree(g_wpack));
@@ -610,6 +612,7 @@ static void* wgrad_partials(size_t bytes) {
     Context& c = ctx();
     if (c.dry_run) return (void*)(uintptr_t)0x1000;
     if (bytes > g_wgrad_bytes) {
+        kept_buffer_moved();
         if (g_wgrad_part) {
             HIP_CHECK(hipStreamSynchronize(c.stream));
             HIP_CHECK(hipFree(g_wgrad_part));

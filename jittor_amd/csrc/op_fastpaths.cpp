@@ -434,6 +434,7 @@ bool try_scatter_1d(const mjt_tensor* y, const mjt_tensor* x, int op, const mjt_
                             bits_of_ptr(base + off_counts), bits_of_ptr(base + off_lists), bits_of_ptr(base + off_pmain),
                             owner->state[0] & 1, bits_of_ptr(base + off_hotof), bits_of_ptr(base + off_ovf),
                             bits_of_ptr(base + off_novf), bits_of_ptr(base + off_dbg), 0, 0};
+    refuse_recording("a scatter that keeps tallies between calls");
     if (!owner->state[1]) jit_launch(ks[2], 1, 1, (unsigned)nthreads, 0, a);
     owner->state[1] = 0;                                      // until the tail pass of this call is under way
     if (!fill_in_main) launch_fill_pattern(x->ptr, ident, 4, (size_t)bins);

@@ -179,12 +179,7 @@ void gemm_launch(int in_dtype, int out_dtype, const void* A, const void* B, void
         remember(key.str(), k);
     }
     MJT_CHECK(batch < 65536 && (M + 63) / 64 < 65536, "matmul: launch too large");
-    set_last_kernel(k->name.c_str());
-    if (c.dry_run) return;
-    size_t size = args.size() * sizeof(uint64_t);
-    void* config[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, (void*)args.data(), HIP_LAUNCH_PARAM_BUFFER_SIZE, &size, HIP_LAUNCH_PARAM_END};
-    HIP_CHECK(hipModuleLaunchKernel(k->fn, (unsigned)((N + 63) / 64), (unsigned)((M + 63) / 64), (unsigned)batch, 256, 1, 1, 0, c.stream,
-                                    nullptr, config));
+    jit_launch(k, (unsigned)((N + 63) / 64), (unsigned)((M + 63) / 64), 256, 0, args, (unsigned)batch);
 }
 
 // 1x1 convolution of stride 1 over a batch of planes that need not be 16-byte multiples (kernels/gemm_dma.h with IMG):

@@ -22,6 +22,33 @@ static std::mutex g_jit_mutex;
 static std::unordered_map<std::string, JitKernel*> g_jit_cache;
 static int64_t g_jit_compiled = 0, g_jit_hits = 0;
 
+// ---- recorded launches ---------------------------------------------------------
+namespace {
+struct Launch {
+    JitKernel* kernel;
+    unsigned gx, gy, gz, block, shmem;
+    std::vector<uint64_t> words;
+};
+struct Patch {
+    int launch, word, slot;
+    int kind;                     // 0: words = base of the slot + add; 1: the scalar's double bits; 2: the scalar's integer
+    uint64_t add;
+};
+}  // namespace
+struct Recording {
+    std::vector<Launch> launches;
+    std::vector<Patch> patches;
+    uint64_t generation = 0;
+    bool ready = false;           // mjt_record_relocate has found every word's origin
+};
+static thread_local Recording* t_recording = nullptr;
+static uint64_t g_generation = 1;         // guarded by the library's lock
+
+void refuse_recording(const char* what) {
+    if (t_recording) MJT_FAIL(MJT_ERR_UNSUPPORTED, what << " cannot be part of a recording");
+}
+void kept_buffer_moved() { g_generation++; }
+
 std::recursive_mutex& api_mutex() {
     static std::recursive_mutex m;
     return m;
@@ -53,6 +80,7 @@ void* scratch(size_t bytes) {
     Context& c = ctx();
     if (c.dry_run) return (void*)(uintptr_t)0x1000;
     if (bytes > c.scratch_bytes) {
+        kept_buffer_moved();
         if (c.scratch) {
             HIP_CHECK(hipStreamSynchronize(c.stream));
             HIP_CHECK(hipFree(c.scratch));
@@ -291,13 +319,17 @@ JitKernel* jit_lookup(const std::string& source) {
 }
 
 void jit_launch(JitKernel* k, unsigned grid_x, unsigned grid_y, unsigned block, unsigned shmem,
-                const std::vector<uint64_t>& args) {
+                const std::vector<uint64_t>& args, unsigned grid_z) {
+    if (t_recording) {
+        t_recording->launches.push_back(Launch{k, grid_x, grid_y, grid_z, block, shmem, args});
+        return;
+    }
     size_t size = args.size() * sizeof(uint64_t);
     void* config[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, (void*)args.data(), HIP_LAUNCH_PARAM_BUFFER_SIZE, &size,
                       HIP_LAUNCH_PARAM_END};
     set_last_kernel(k->name.c_str());
     if (ctx().dry_run) return;
-    HIP_CHECK(hipModuleLaunchKernel(k->fn, grid_x, grid_y, 1, block, 1, 1, shmem, ctx().stream, nullptr, config));
+    HIP_CHECK(hipModuleLaunchKernel(k->fn, grid_x, grid_y, grid_z, block, 1, 1, shmem, ctx().stream, nullptr, config));
 }
 
 // defined in aot_kernels.hip
@@ -342,6 +374,7 @@ int mjt_init(int device) {
 void mjt_shutdown(void) {
     Context& c = ctx();
     if (!c.ready) return;
+    kept_buffer_moved();
     if (!c.dry_run) (void)hipStreamSynchronize(c.stream);
     for (auto fn : shutdown_hooks()) fn();
     {
@@ -478,6 +511,76 @@ int mjt_event_destroy(void* ev) {
     return guarded([&] {
         require_device();
         HIP_CHECK(hipEventDestroy((hipEvent_t)ev));
+    });
+}
+
+int mjt_record_begin(void) {
+    return guarded([&] {
+        require_init();
+        MJT_CHECK(!t_recording, "mjt_record_begin: this thread is recording already");
+        t_recording = new Recording();
+        t_recording->generation = g_generation;
+    });
+}
+int mjt_record_end(void** out) {
+    return guarded([&] {
+        MJT_CHECK(t_recording, "mjt_record_end without mjt_record_begin");
+        Recording* r = t_recording;
+        t_recording = nullptr;
+        if (out) *out = r;
+        else delete r;
+    });
+}
+void mjt_record_free(void* rec) { delete (Recording*)rec; }
+
+int mjt_record_relocate(void* first, void* second, int n_slots, const uint64_t* base1, const uint64_t* base2, uint64_t span,
+                        int n_scalars, const int64_t* scalar1, const int64_t* scalar2) {
+    return guarded([&] {
+        Recording *a = (Recording*)first, *b = (Recording*)second;
+        MJT_CHECK(a && b && !a->ready && n_slots >= 0 && n_scalars >= 0, "mjt_record_relocate: bad arguments");
+        auto differ = [](const char* what) { MJT_FAIL(MJT_ERR_UNSUPPORTED, "mjt_record_relocate: the recordings differ in " << what); };
+        if (a->generation != g_generation || b->generation != g_generation || a->launches.size() != b->launches.size()) differ("their launches");
+        for (size_t l = 0; l < a->launches.size(); l++) {
+            const Launch &p = a->launches[l], &q = b->launches[l];
+            if (p.kernel != q.kernel || p.gx != q.gx || p.gy != q.gy || p.gz != q.gz || p.block != q.block || p.shmem != q.shmem ||
+                p.words.size() != q.words.size())
+                differ("a kernel or its grid");
+            for (size_t w = 0; w < p.words.size(); w++) {
+                const uint64_t u = p.words[w], v = q.words[w];
+                if (u == v) continue;
+                Patch patch{(int)l, (int)w, -1, 0, 0};
+                for (int k = 0; k < n_slots && patch.slot < 0; k++)
+                    if (u - base1[k] < span && u - base1[k] == v - base2[k]) patch.slot = k, patch.add = u - base1[k];
+                for (int k = 0; k < n_scalars && patch.slot < 0; k++) {
+                    if (u == bits_of((double)scalar1[k]) && v == bits_of((double)scalar2[k])) patch.slot = k, patch.kind = 1;
+                    else if (u == (uint64_t)scalar1[k] && v == (uint64_t)scalar2[k]) patch.slot = k, patch.kind = 2;
+                }
+                if (patch.slot < 0) differ("a word that is neither a slot's address nor a scalar");
+                a->patches.push_back(patch);
+            }
+        }
+        a->ready = true;
+    });
+}
+
+int mjt_record_launch(void* rec, int n_slots, const uint64_t* bases, int n_scalars, const double* fvalues, const int64_t* ivalues) {
+    return guarded([&] {
+        Recording* r = (Recording*)rec;
+        MJT_CHECK(r && r->ready, "mjt_record_launch: not a finished recording");
+        if (r->generation != g_generation) MJT_FAIL(MJT_ERR_UNSUPPORTED, "mjt_record_launch: the recording is out of date");
+        refuse_recording("mjt_record_launch");
+        for (const Patch& p : r->patches) {
+            MJT_CHECK(p.slot < (p.kind == 0 ? n_slots : n_scalars), "mjt_record_launch: too few slots or scalars");
+            uint64_t word;
+            if (p.kind == 0) {
+                // routes were chosen for addresses aligned like those of whole allocations
+                if (bases[p.slot] == 0 || bases[p.slot] % 256) MJT_FAIL(MJT_ERR_UNSUPPORTED, "mjt_record_launch: unaligned buffer");
+                word = bases[p.slot] + p.add;
+            } else
+                word = p.kind == 1 ? bits_of(fvalues[p.slot]) : (uint64_t)ivalues[p.slot];
+            r->launches[(size_t)p.launch].words[(size_t)p.word] = word;
+        }
+        for (const Launch& l : r->launches) jit_launch(l.kernel, l.gx, l.gy, l.block, l.shmem, l.words, l.gz);
     });
 }
 

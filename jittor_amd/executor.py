@@ -20,7 +20,7 @@ from . import profiler as _profiler
 from .flags import flags
 
 stats = {"launches": 0, "fused_groups": 0, "fused_reduces": 0, "conv_matches": 0, "syncs": 0, "sunk_ops": 0, "matmul_matches": 0,
-         "wgrad_kernel": 0, "wgrad_chunked": 0, "gather_reduces": 0, "fused_scatters": 0, "plans": 0, "replays": 0}
+         "wgrad_kernel": 0, "wgrad_chunked": 0, "gather_reduces": 0, "fused_scatters": 0, "plans": 0, "replays": 0, "recorded_launches": 0}
 
 
 class ConvUnit:
@@ -488,8 +488,24 @@ class _Capture:
         return call
 
 
+class _Recording:
+    """What a plan's calls launch, held by the library (mjt_record_*): freed with the plan."""
+    __slots__ = ("rec", "n", "ns", "bases", "fvalues", "ivalues")
+
+    def __init__(self, rec, n, ns):
+        self.rec, self.n, self.ns = rec, n, ns
+        self.bases, self.fvalues, self.ivalues = ctypes.c_uint64 * n, ctypes.c_double * max(1, ns), ctypes.c_int64 * max(1, ns)
+
+    def __del__(self):
+        try:
+            _lib.load().mjt_record_free(self.rec)
+        except Exception:
+            pass
+
+
 class _Plan:
-    __slots__ = ("slots", "needs_ptr", "produce", "ptrs", "scalars", "calls", "stats", "cleared")
+    # native: None until the plan has been replayed by its calls, then its _Recording, or False where the calls cannot be recorded
+    __slots__ = ("slots", "needs_ptr", "produce", "ptrs", "scalars", "calls", "stats", "cleared", "seen", "native")
 
 
 _cap = None
@@ -615,12 +631,85 @@ def _capture(ops, target_ids, sig):
             produce.append((k, src))
             needs_ptr.add(src)
     plan.slots, plan.needs_ptr, plan.produce, plan.calls = slots, needs_ptr, produce, cap.calls
+    plan.seen, plan.native = 0, None
     plan.stats = [(key, stats[key] - before[key]) for key in stats if stats[key] != before[key]]
     plan.cleared = [(i, had_inputs[i] and not op.inputs) for i, op in enumerate(ops) if op.out is not None and op.out._op is None]
     if len(_plans) >= _PLAN_LIMIT:
         _plans.clear()
     _plans[sig] = plan
     stats["plans"] += 1
+
+
+_SPAN = 1 << 36                  # stand-in addresses: one buffer each, far apart
+
+
+def _fill_in(plan, base, scalars):
+    for obj, idx, k, off in plan.ptrs:
+        if idx is None:
+            obj.ptr = base[k] + off
+        else:
+            obj[idx].ptr = base[k] + off
+    for (arr, idx, _), (fvalue, ivalue) in zip(plan.scalars, scalars):
+        fv = arr[idx]
+        fv.fvalue, fv.ivalue = fvalue, ivalue
+
+
+def _record(plan):
+    """The plan's calls as recorded launches: made twice with stand-in addresses and scalars, which launches nothing and tells the
+    library where each parameter word comes from.  False where a call cannot be recorded."""
+    lib = _lib.ensure_init()
+    n, ns = len(plan.slots), len(plan.scalars)
+    recs, sets = [], []
+    try:
+        for run in (1, 2):
+            base = [(run << 45) + _SPAN * (k if run == 1 else n - k) for k in range(n)]
+            vals = [run * 1000003 + k for k in range(ns)]
+            _fill_in(plan, base, [(float(v), v) for v in vals])
+            _lib.check(lib.mjt_record_begin())
+            rec, rc = ctypes.c_void_p(), 0
+            try:
+                for fn, args in plan.calls:
+                    rc = fn(*args)
+                    if rc:
+                        break
+            finally:
+                lib.mjt_record_end(ctypes.byref(rec))
+            recs.append(rec)
+            sets.append(((ctypes.c_uint64 * n)(*base), (ctypes.c_int64 * max(1, ns))(*vals)))
+            if rc:
+                return False
+        (b1, s1), (b2, s2) = sets
+        if lib.mjt_record_relocate(recs[0], recs[1], n, b1, b2, _SPAN, ns, s1, s2):
+            return False
+        return _Recording(recs.pop(0), n, ns)
+    finally:
+        for rec in recs:
+            lib.mjt_record_free(rec)
+
+
+def _launch(plan, base, scalars):
+    """The plan's calls on these buffers and scalars.  The calls look their kernels up and lay out parameters anew each time
+    (3 us a call); from the third execution of a graph on the launches themselves are issued, all by one call."""
+    if plan.native is None:
+        if plan.seen:
+            plan.native = _record(plan)
+        plan.seen += 1
+    r = plan.native
+    if r:
+        rc = _lib.load().mjt_record_launch(r.rec, r.n, r.bases(*base), r.ns, r.fvalues(*[f for f, _ in scalars]),
+                                           r.ivalues(*[i for _, i in scalars]))
+        if rc == 0:
+            stats["recorded_launches"] += 1
+            return
+        if rc != _lib.ERR_UNSUPPORTED:
+            _lib.check(rc)
+        plan.native = None                                     # out of date (scratch memory of the library has moved): made again next time
+    _fill_in(plan, base, scalars)
+    check = _lib.check
+    for fn, args in plan.calls:
+        rc = fn(*args)
+        if rc:
+            check(rc)
 
 
 def _replay(plan, ops):
@@ -648,19 +737,7 @@ def _replay(plan, ops):
             v._buf = Buffer(max(v.nbytes, 1))
         buf[k] = v._buf
         base[k] = v._buf.ptr
-    for obj, idx, k, off in plan.ptrs:
-        if idx is None:
-            obj.ptr = base[k] + off
-        else:
-            obj[idx].ptr = base[k] + off
-    for arr, idx, k in plan.scalars:
-        fv = arr[idx]
-        fv.fvalue, fv.ivalue = _scalar_value(var[k])
-    check = _lib.check
-    for fn, args in plan.calls:
-        rc = fn(*args)
-        if rc:
-            check(rc)
+    _launch(plan, base, [_scalar_value(var[k]) for _, _, k in plan.scalars])
     for key, d in plan.stats:
         stats[key] += d
     for i, clear_inputs in plan.cleared:

@@ -146,3 +146,27 @@ def test_replay_keeps_the_graph_bookkeeping(gpu):
         assert np.array_equal(b.numpy(), np.full(64, 64 * (2.0 * (s + 1) + 1.0), np.float32))
         c = (b + 1.0).numpy()                                  # a later graph on a replayed result
         assert np.array_equal(c, b.numpy() + 1.0)
+
+
+def test_recorded_launches_equal_fresh_ones(gpu):
+    """From the third execution on one call issues all launches: scalars and buffers of the step at hand, an input that shares
+    another's buffer, and scratch memory that moved in between (a longer reduction needs more of it)."""
+    def step(seed):
+        rng = np.random.default_rng(300 + seed)
+        x = jt.array(rng.standard_normal((40, 96)).astype(np.float32))
+        w = jt.array(rng.standard_normal((72, 96)).astype(np.float32))
+        jt.sync([x, w])
+        other = jt.reshape(x, [96, 40]) if seed % 2 else jt.array(rng.standard_normal((96, 40)).astype(np.float32))
+        jt.sync([other])
+        y = jt.nn.linear(x, w) * jt.array(np.float32(0.5 + seed))
+        loss = (y * y).sum() + other.sum()
+        gx, gw = jt.grad(loss, [x, w])
+        jt.sync([loss, gx, gw])
+        if seed == 3:
+            big = jt.array(np.ones((4096, 8192), np.float32))
+            jt.sync([big.sum([0])])
+        return [loss.numpy(), gx.numpy(), gw.numpy()]
+    before = executor.stats["recorded_launches"]
+    fresh, again, replays = _both_ways(step, 8)
+    _same(fresh, again)
+    assert executor.stats["recorded_launches"] > before

@@ -764,3 +764,61 @@ def test_executor_replays_a_graph_it_has_seen(compile_only, monkeypatch):
     monkeypatch.setitem(executor.flags, "enable_replay", False)
     d = step(0.5)[0]
     assert d["plans"] == 0 and d["replays"] == 0
+
+
+def test_recorded_launches(compile_only, monkeypatch):
+    """From its third execution on a graph's launches are issued by one call; what cannot be recorded (a scatter that keeps
+    tallies) stays with its calls, a recording older than a shutdown is refused and made again, two recordings of different
+    work are not matched."""
+    from jittor_amd import core, executor
+    nxt = [0x10000000]
+
+    def fake_alloc(nbytes):
+        size = core._Pool._round(nbytes)
+        nxt[0] += size
+        return nxt[0] - size, size
+
+    monkeypatch.setattr(core.pool, "alloc", fake_alloc)
+    monkeypatch.setattr(core.pool, "free", lambda ptr, size: None)
+    monkeypatch.setattr(L, "h2d", lambda ptr, arr: None)
+    monkeypatch.setitem(executor.flags, "enable_replay", True)
+    executor._plans.clear()
+
+    def norm(scale):
+        x = jt.array(np.ones((64, 48), np.float32))
+        d = x - x.mean([1], keepdims=True)
+        jt.sync([d * jt.array(np.float32(scale)), (d * d).sum([0])])
+
+    def scatter(_):
+        v, i = jt.array(np.ones(1 << 20, np.float32)), jt.array(np.zeros(1 << 20, np.int32))
+        jt.sync([v.reindex_reduce("add", [1 << 18], ["@e0(i0)"], extras=[i])])
+
+    def recorded(step, n):
+        before = executor.stats["recorded_launches"]
+        for k in range(n):
+            step(1.0 + k)
+        return executor.stats["recorded_launches"] - before
+
+    assert recorded(norm, 2) == 0 and recorded(norm, 3) == 3
+    plan = next(iter(executor._plans.values()))
+    assert plan.native and all((o if i is None else o[i]).ptr is not None for o, i, _, _ in plan.ptrs)
+    assert recorded(scatter, 4) == 0
+    L.load().mjt_shutdown()
+    L.check(L.load().mjt_init(-1))
+    assert recorded(norm, 2) == 1                                # refused once, recorded anew
+    lib = L.load()
+    recs = []
+    for shape in ([64, 48], [64, 40]):
+        x, y = L.tensor(1 << 45, "float32", shape), L.tensor(1 << 46, "float32", [64])
+        L.check(lib.mjt_record_begin())
+        assert lib.mjt_record_begin() < 0                        # one at a time
+        L.check(lib.mjt_reduce(ctypes.byref(x), ctypes.byref(y), L.OP_CODE["add"], 2))
+        rec = ctypes.c_void_p()
+        L.check(lib.mjt_record_end(ctypes.byref(rec)))
+        recs.append(rec)
+    b = (ctypes.c_uint64 * 2)(1 << 45, 1 << 46)
+    none = (ctypes.c_int64 * 1)()
+    assert lib.mjt_record_relocate(recs[0], recs[1], 2, b, b, 1 << 36, 0, none, none) == L.ERR_UNSUPPORTED
+    assert lib.mjt_record_launch(recs[0], 2, b, 0, None, none) < 0
+    for rec in recs:
+        lib.mjt_record_free(rec)
