@@ -22,8 +22,12 @@
 // The other kind (m or n innermost) is transposed on the way in registers: 8 lanes load
 // 16 bytes of 8 consecutive k rows, exchange among themselves with three butterfly steps
 // (4 lanes and two steps for float32) until each owns one column for the 8 (4) k, and
-// write 16 bytes.  The loads of the next stage are in flight during the MFMAs of the
-// current one and are written to the other LDS buffer after them: one barrier per stage.
+// write 16 bytes.  A stage's tiles are loaded into registers one or two stages ahead and move to the other LDS buffer piece by
+// piece between the MFMAs of the current stage; its barrier and the first fragment reads of the next stage stand in front
+// of the last MFMAs.  (With these one after the other at the end of each stage the matrix cores stood still for 570 of the
+// 1700 cycles of a 64 x 64 float32 stage.  us before / now: float32 a b^T 2048 x 1024 x 1024 49.9 / 42, 2048^3 152 / 127,
+// a^T b 1024 x 1024 x 2048 69 / 55; bfloat16 2048 x 2048 x 2048 32.5 / 23, 12544 x 256 x 1024 18.8 / 14.)
+// The float32 MFMAs alone, 140 TFLOP/s measured, bound the large products.
 // float32 uses v_mfma_f32_32x32x2: a lane's 16-byte read holds 4 k of its row, which feed
 // four MFMAs (lanes 32..63 read the next chunk, so that an MFMA sums k and k + 4 of a
 // chunk pair; any pairing is right as long as both operands use the same one).
@@ -66,6 +70,9 @@ typedef unsigned short TIN;
 #define NTHR 256
 #ifndef CONV
 #define CONV 0
+#endif
+#ifndef SLICED
+#define SLICED 0                 // 1: workgroup (tile, slice) sums stages slice * a[9] .. of K into its own float32 C, a[11] apart
 #endif
 #ifndef NBUF
 #define NBUF 2                   // staging buffers: 2, or 1 for a product of a single stage (K <= KS)
@@ -128,18 +135,6 @@ __device__ __forceinline__ mjt_u32x4v mjt_transpose4x4_b32(mjt_u32x4v v, int lan
     return y;
 }
 
-// Fragment reads and the waits for them are written out, so that the order below is what runs: the compiler
-// would otherwise move every read next to its first use and wait for it there.
-template <int OFF> __device__ __forceinline__ void mjt_ds_read(mjt_u32x4v& dst, unsigned addr) {
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst) : "v"(addr), "n"(OFF) : "memory");
-}
-// wait until at most N LDS operations are outstanding (LDS returns in order); names the registers that are
-// ready then, so that no use of them is scheduled in front of the wait
-template <int N, int CNT> __device__ __forceinline__ void mjt_frag_wait(mjt_u32x4v (&f)[CNT]) {
-    if constexpr (CNT == 1) asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(f[0]) : "n"(N));
-    else if constexpr (CNT == 2) asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(f[0]), "+v"(f[1]) : "n"(N));
-    else asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(f[0]), "+v"(f[1]), "+v"(f[2]), "+v"(f[3]) : "n"(N));
-}
 template <int I, int N, class F> __device__ __forceinline__ void mjt_static_for(F&& f) {
     if constexpr (I < N) {
         f(mjt_ic<I>());
@@ -150,78 +145,89 @@ template <int I, int N, class F> __device__ __forceinline__ void mjt_static_for(
 // One operand tile of a stage on its way from memory to LDS.  ROWS = tile rows (m or n), KCONT = memory has k
 // innermost.  p = first element of the operand (of this batch), ld = leading dimension in elements, r0 = first
 // tile row, rmax = rows of the operand, k0 = first k of the stage, K = total k.
-// fetch() only issues the loads (unconditional: nothing in it looks at a loaded value, so no wait is needed
-// before the MFMAs that follow); commit() zeroes what lies beyond K, transposes and writes to LDS.
+// A tile moves in PER pieces, one 16-byte move per thread each.  fetch() only issues piece I's load (unconditional: nothing in it
+// looks at a loaded value, so no wait is needed before the MFMAs that follow); commit() zeroes what lies beyond K, transposes
+// and writes to LDS.  FULL: the stage does not reach beyond K.
 template <int ROWS, bool KCONT> struct mjt_stager {
     static constexpr int PER = ROWS * KC / NTHR;          // 16-byte moves per thread
     mjt_u32x4v reg[PER];
 
-    __device__ __forceinline__ void fetch(const TIN* __restrict__ p, long long ld, int r0, int rmax, int k0, int K, int tid) {
-#pragma unroll
-        for (int i = 0; i < PER; i++) {
-            if constexpr (KCONT) {
-                // chunk c = tid + i * NTHR: row c / KC, k-chunk c % KC (8 consecutive lanes read one 128-byte line)
-                const int c = tid + i * NTHR;
-                int row = r0 + c / KC;
-                row = row < rmax ? row : rmax - 1;
-                const int k = k0 + (c % KC) * EPC;
-                const int kk = k < K ? k : 0;             // a chunk past the end reads chunk 0 and is zeroed in commit
-                reg[i] = *(const mjt_u32x4v*)(p + (long long)row * ld + kk);
-            } else {
-                // blocks of EPC k-rows x EPC columns: EPC lanes each load 16 bytes (EPC columns) of one k-row.
-                // Block b = tid / EPC + i * (NTHR / EPC): column group b % (ROWS / EPC), k-chunk b / (ROWS / EPC);
-                // the blocks of a wave are neighbouring column groups, so a k-row's loads of a wave are contiguous.
-                const int b = tid / EPC + i * (NTHR / EPC);
-                const int cg = b % (ROWS / EPC), kc = b / (ROWS / EPC);
-                int col = r0 + cg * EPC;
-                col = col < rmax ? col : ((rmax - 1) / EPC) * EPC;      // a group outside the operand reads the last one (ld is a multiple of EPC: a group never leaves its row)
-                const int k = k0 + kc * EPC + tid % EPC;
-                const int kk = k < K ? k : 0;
-                reg[i] = *(const mjt_u32x4v*)(p + (long long)kk * ld + col);
-            }
+    template <int I, bool FULL> __device__ __forceinline__ void fetch(const TIN* __restrict__ p, long long ld, int r0, int rmax, int k0, int K, int tid) {
+        if constexpr (KCONT) {
+            // chunk c = tid + I * NTHR: row c / KC, k-chunk c % KC (8 consecutive lanes read one 128-byte line)
+            const int c = tid + I * NTHR;
+            int row = r0 + c / KC;
+            row = row < rmax ? row : rmax - 1;
+            const int k = k0 + (c % KC) * EPC;
+            const int kk = FULL || k < K ? k : 0;         // a chunk past the end reads chunk 0 and is zeroed in commit
+            reg[I] = *(const mjt_u32x4v*)(p + (long long)row * ld + kk);
+        } else {
+            // blocks of EPC k-rows x EPC columns: EPC lanes each load 16 bytes (EPC columns) of one k-row.
+            // Block b = tid / EPC + I * (NTHR / EPC): column group b % (ROWS / EPC), k-chunk b / (ROWS / EPC);
+            // the blocks of a wave are neighbouring column groups, so a k-row's loads of a wave are contiguous.
+            const int b = tid / EPC + I * (NTHR / EPC);
+            const int cg = b % (ROWS / EPC), kc = b / (ROWS / EPC);
+            int col = r0 + cg * EPC;
+            col = col < rmax ? col : ((rmax - 1) / EPC) * EPC;      // a group outside the operand reads the last one (ld is a multiple of EPC: a group never leaves its row)
+            const int k = k0 + kc * EPC + tid % EPC;
+            const int kk = FULL || k < K ? k : 0;
+            reg[I] = *(const mjt_u32x4v*)(p + (long long)kk * ld + col);
         }
     }
-    // TAIL: the stage reaches beyond K
-    template <bool TAIL> __device__ __forceinline__ void commit_as(unsigned char* lds, int k0, int K, int tid) const {
-#pragma unroll
-        for (int i = 0; i < PER; i++) {
-            mjt_u32x4v v = reg[i];
-            int row, kc;
-            if constexpr (KCONT) {
-                const int c = tid + i * NTHR;
-                row = c / KC;
-                kc = c % KC;
-                if constexpr (TAIL) {
-                    const int valid = K - (k0 + kc * EPC);    // elements of this chunk that exist
+    template <int I, bool FULL> __device__ __forceinline__ void commit(unsigned char* lds, int k0, int K, int tid) const {
+        mjt_u32x4v v = reg[I];
+        int row, kc;
+        if constexpr (KCONT) {
+            const int c = tid + I * NTHR;
+            row = c / KC;
+            kc = c % KC;
+            if constexpr (!FULL) {
+                const int valid = K - (k0 + kc * EPC);    // elements of this chunk that exist
 #if IN == 2
 #pragma unroll
-                    for (int e = 0; e < 4; e++) v[e] = e < valid ? v[e] : 0u;
+                for (int e = 0; e < 4; e++) v[e] = e < valid ? v[e] : 0u;
 #else
 #pragma unroll
-                    for (int e = 0; e < 4; e++) v[e] = 2 * e + 1 < valid ? v[e] : 2 * e < valid ? (v[e] & 0xffffu) : 0u;
-#endif
-                }
-            } else {
-                const int b = tid / EPC + i * (NTHR / EPC);
-                row = (b % (ROWS / EPC)) * EPC + tid % EPC;
-                kc = b / (ROWS / EPC);
-                if constexpr (TAIL) {
-                    if (k0 + kc * EPC + tid % EPC >= K) v = (mjt_u32x4v)(0u);
-                }
-#if IN == 2
-                v = mjt_transpose4x4_b32(v, tid);
-#else
-                v = mjt_transpose8x8_b16(v, tid);
+                for (int e = 0; e < 4; e++) v[e] = 2 * e + 1 < valid ? v[e] : 2 * e < valid ? (v[e] & 0xffffu) : 0u;
 #endif
             }
-            *(mjt_u32x4v*)(lds + row * ROWB + kc * 16) = v;
+        } else {
+            const int b = tid / EPC + I * (NTHR / EPC);
+            row = (b % (ROWS / EPC)) * EPC + tid % EPC;
+            kc = b / (ROWS / EPC);
+            if constexpr (!FULL) {
+                if (k0 + kc * EPC + tid % EPC >= K) v = (mjt_u32x4v)(0u);
+            }
+#if IN == 2
+            v = mjt_transpose4x4_b32(v, tid);
+#else
+            v = mjt_transpose8x8_b16(v, tid);
+#endif
         }
-    }
-    __device__ __forceinline__ void commit(unsigned char* lds, int k0, int K, int tid) const {
-        if (k0 + KS > K) commit_as<true>(lds, k0, K, tid);    // uniform
-        else commit_as<false>(lds, k0, K, tid);
+        *(mjt_u32x4v*)(lds + row * ROWB + kc * 16) = v;
     }
 };
+
+#if CONV
+constexpr int ESZ = (int)sizeof(TIN);
+#define MJT_NONE 0x80000000u         // an offset beyond every buffer (they are smaller than 2 GB): the load delivers zeros
+__device__ __forceinline__ unsigned mjt_wg_load(__amdgpu_buffer_rsrc_t d, unsigned off) {
+#if IN == 2
+    return __builtin_amdgcn_raw_buffer_load_b32(d, (int)off, 0, 0);
+#else
+    return (unsigned short)__builtin_amdgcn_raw_buffer_load_b16(d, (int)off, 0, 0);
+#endif
+}
+__device__ __forceinline__ mjt_u32x4v mjt_wg_pack(const unsigned (&v)[EPC]) {
+    mjt_u32x4v r;
+#if IN == 2
+    r[0] = v[0]; r[1] = v[1]; r[2] = v[2]; r[3] = v[3];
+#else
+    r[0] = v[0] | (v[1] << 16); r[1] = v[2] | (v[3] << 16); r[2] = v[4] | (v[5] << 16); r[3] = v[6] | (v[7] << 16);
+#endif
+    return r;
+}
+#endif
 
 #if CONV == 1
 // The B tile of a stage of the implicit-GEMM convolution.  Same blocks as mjt_stager<TN, false>: EPC lanes hold EPC
@@ -235,7 +241,7 @@ struct mjt_conv_cols {
     unsigned hw[PER][EPC];
     // (compile-time loop indices throughout: with run-time ones the compiler keeps these arrays in scratch memory
     // once the loops are too long for it to unroll them itself)
-    __device__ __forceinline__ void init(int n0, int N, int tid) {
+    __device__ __forceinline__ void init(int n0, int N, int img0, int tid) {
         mjt_static_for<0, PER * EPC>([&](auto ic) {
             constexpr int i = decltype(ic)::v / EPC, e = decltype(ic)::v % EPC;
             const int b = tid / EPC + i * (NTHR / EPC);
@@ -243,67 +249,58 @@ struct mjt_conv_cols {
             const int img = j / (OH_ * OW_), px = j - img * (OH_ * OW_);
             const int oh = px / OW_, ow = px - oh * OW_;
             const int ih = oh * SH - PH, iw = ow * SW - PW;
-            base[i][e] = j < N ? (img * C_ * H_ + ih) * W_ + iw : 0;
+            base[i][e] = j < N ? ((img - img0) * C_ * H_ + ih) * W_ + iw : 0;
             hw[i][e] = j < N ? ((unsigned)(ih + 0x4000) << 16) | (unsigned)(iw + 0x4000) : 0u;
         });
     }
 };
+// XBUF 1: x is read through a buffer descriptor that begins at the tile's first image (the host promises that a tile's images
+// are less than 2 GB), unconditionally: a tap outside the image gets an offset past the buffer's end and reads zero, so nothing
+// has to be looked at before the value is written to LDS.  XBUF 0: plain loads, zeroed afterwards, which wait for them.
 struct mjt_conv_stager {
     static constexpr int PER = TN * KC / NTHR;
     static constexpr int RS = R_ * S_, CRS = C_ * R_ * S_;
-    mjt_u32x4v reg[PER];
+    unsigned v[PER][EPC];
 
-    __device__ __forceinline__ void fetch(const TIN* __restrict__ x, const mjt_conv_cols& cols, int k0, int tid) {
-        mjt_static_for<0, PER>([&](auto ic) {
-            constexpr int i = decltype(ic)::v;
-            const int b = tid / EPC + i * (NTHR / EPC);
-            const int k = k0 + (b / (TN / EPC)) * EPC + tid % EPC;
-            const bool kvalid = k < CRS;
-            const int kk = kvalid ? k : 0;
-            const int c = kk / RS, rs = kk - c * RS;
-            const int r = rs / S_, t = rs - r * S_;
-            const int koff = (c * H_ + r * DH) * W_ + t * DW;
-            const unsigned dhw = ((unsigned)(r * DH) << 16) | (unsigned)(t * DW);
-            unsigned v[EPC];
-            mjt_static_for<0, EPC>([&](auto ec) {
-                constexpr int e = decltype(ec)::v;
-                const unsigned q = cols.hw[i][e] + dhw;
-                const bool ok = kvalid && (q >> 16) - 0x4000u < (unsigned)H_ && (q & 0xffffu) - 0x4000u < (unsigned)W_;
-                // an unconditional load from a valid address, zeroed afterwards: a load under a condition is a branch per
-                // element
-#if IN == 2
-                const unsigned ld = __float_as_uint(x[ok ? cols.base[i][e] + koff : 0]);
+    template <int I> __device__ __forceinline__ void fetch(const TIN* __restrict__ x, __amdgpu_buffer_rsrc_t d, const mjt_conv_cols& cols, int k0, int tid) {
+        const int b = tid / EPC + I * (NTHR / EPC);
+        const int k = k0 + (b / (TN / EPC)) * EPC + tid % EPC;
+        const bool kvalid = k < CRS;
+        const int kk = kvalid ? k : 0;
+        const int c = kk / RS, rs = kk - c * RS;
+        const int r = rs / S_, t = rs - r * S_;
+        const int koff = (c * H_ + r * DH) * W_ + t * DW;
+        const unsigned dhw = ((unsigned)(r * DH) << 16) | (unsigned)(t * DW);
+        mjt_static_for<0, EPC>([&](auto ec) {
+            constexpr int e = decltype(ec)::v;
+            const unsigned q = cols.hw[I][e] + dhw;
+            const bool ok = kvalid && (q >> 16) - 0x4000u < (unsigned)H_ && (q & 0xffffu) - 0x4000u < (unsigned)W_;
+#if XBUF
+            v[I][e] = mjt_wg_load(d, ok ? (unsigned)(cols.base[I][e] + koff) * ESZ : MJT_NONE);
 #else
-                const unsigned ld = x[ok ? cols.base[i][e] + koff : 0];
+#if IN == 2
+            const unsigned ld = __float_as_uint(x[ok ? cols.base[I][e] + koff : 0]);
+#else
+            const unsigned ld = x[ok ? cols.base[I][e] + koff : 0];
 #endif
-                v[e] = ok ? ld : 0u;
-            });
-#if IN == 2
-            reg[i][0] = v[0]; reg[i][1] = v[1]; reg[i][2] = v[2]; reg[i][3] = v[3];
-#else
-            reg[i][0] = v[0] | (v[1] << 16); reg[i][1] = v[2] | (v[3] << 16); reg[i][2] = v[4] | (v[5] << 16); reg[i][3] = v[6] | (v[7] << 16);
+            v[I][e] = ok ? ld : 0u;
 #endif
         });
     }
-    __device__ __forceinline__ void commit(unsigned char* lds, int tid) const {
-        mjt_static_for<0, PER>([&](auto ic) {
-            constexpr int i = decltype(ic)::v;
-            const int b = tid / EPC + i * (NTHR / EPC);
-            const int row = (b % (TN / EPC)) * EPC + tid % EPC, kc = b / (TN / EPC);
+    template <int I> __device__ __forceinline__ void commit(unsigned char* lds, int tid) const {
+        const int b = tid / EPC + I * (NTHR / EPC);
+        const int row = (b % (TN / EPC)) * EPC + tid % EPC, kc = b / (TN / EPC);
 #if IN == 2
-            *(mjt_u32x4v*)(lds + row * ROWB + kc * 16) = mjt_transpose4x4_b32(reg[i], tid);
+        *(mjt_u32x4v*)(lds + row * ROWB + kc * 16) = mjt_transpose4x4_b32(mjt_wg_pack(v[I]), tid);
 #else
-            *(mjt_u32x4v*)(lds + row * ROWB + kc * 16) = mjt_transpose8x8_b16(reg[i], tid);
+        *(mjt_u32x4v*)(lds + row * ROWB + kc * 16) = mjt_transpose8x8_b16(mjt_wg_pack(v[I]), tid);
 #endif
-        });
     }
 };
 #endif
 
 #if CONV == 2
 constexpr int P_ = OH_ * OW_;
-constexpr int ESZ = (int)sizeof(TIN);
-#define MJT_NONE 0x80000000u         // an offset beyond every buffer (they are smaller than 2 GB): the load delivers zeros
 // The pixels of the lane's chunk of a stage (chunk tid % KC), the same for all rows and columns that it loads.  All loads go
 // through buffer descriptors, unconditionally: what lies outside the image or past the sum gets an offset past the buffer's
 // end and reads zero, so nothing has to be looked at before it is written to LDS.
@@ -332,22 +329,6 @@ struct mjt_wg_chunk {
         });
     }
 };
-__device__ __forceinline__ mjt_u32x4v mjt_wg_pack(const unsigned (&v)[EPC]) {
-    mjt_u32x4v r;
-#if IN == 2
-    r[0] = v[0]; r[1] = v[1]; r[2] = v[2]; r[3] = v[3];
-#else
-    r[0] = v[0] | (v[1] << 16); r[1] = v[2] | (v[3] << 16); r[2] = v[4] | (v[5] << 16); r[3] = v[6] | (v[7] << 16);
-#endif
-    return r;
-}
-__device__ __forceinline__ unsigned mjt_wg_load(__amdgpu_buffer_rsrc_t d, unsigned off) {
-#if IN == 2
-    return __builtin_amdgcn_raw_buffer_load_b32(d, (int)off, 0, 0);
-#else
-    return (unsigned short)__builtin_amdgcn_raw_buffer_load_b16(d, (int)off, 0, 0);
-#endif
-}
 struct mjt_wg_dy {
     static constexpr int PER = TM * KC / NTHR;
     mjt_u32x4v reg[PER];
@@ -358,23 +339,17 @@ struct mjt_wg_dy {
             row[decltype(ic)::v] = (unsigned)((r < M ? r : M - 1) * P_) * ESZ;
         });
     }
-    __device__ __forceinline__ void fetch(__amdgpu_buffer_rsrc_t d, const mjt_wg_chunk& ch) {
-        mjt_static_for<0, PER>([&](auto ic) {
-            constexpr int i = decltype(ic)::v;
-            if constexpr (mjt_wg_chunk::NDY == 1) {
-                reg[i] = __builtin_amdgcn_raw_buffer_load_b128(d, (int)((ch.dy[0] + row[i]) | (ch.dy[0] & MJT_NONE)), 0, 0);
-            } else {
-                unsigned v[EPC];
-                mjt_static_for<0, EPC>([&](auto ec) { constexpr int e = decltype(ec)::v; v[e] = mjt_wg_load(d, (ch.dy[e] + row[i]) | (ch.dy[e] & MJT_NONE)); });
-                reg[i] = mjt_wg_pack(v);
-            }
-        });
+    template <int I> __device__ __forceinline__ void fetch(__amdgpu_buffer_rsrc_t d, const mjt_wg_chunk& ch) {
+        if constexpr (mjt_wg_chunk::NDY == 1) {
+            reg[I] = __builtin_amdgcn_raw_buffer_load_b128(d, (int)((ch.dy[0] + row[I]) | (ch.dy[0] & MJT_NONE)), 0, 0);
+        } else {
+            unsigned v[EPC];
+            mjt_static_for<0, EPC>([&](auto ec) { constexpr int e = decltype(ec)::v; v[e] = mjt_wg_load(d, (ch.dy[e] + row[I]) | (ch.dy[e] & MJT_NONE)); });
+            reg[I] = mjt_wg_pack(v);
+        }
     }
-    __device__ __forceinline__ void commit(unsigned char* lds, int tid) const {
-        mjt_static_for<0, PER>([&](auto ic) {
-            constexpr int i = decltype(ic)::v;
-            *(mjt_u32x4v*)(lds + (tid / KC + i * (NTHR / KC)) * ROWB + (tid % KC) * 16) = reg[i];
-        });
+    template <int I> __device__ __forceinline__ void commit(unsigned char* lds, int tid) const {
+        *(mjt_u32x4v*)(lds + (tid / KC + I * (NTHR / KC)) * ROWB + (tid % KC) * 16) = reg[I];
     }
 };
 struct mjt_wg_x {
@@ -391,22 +366,16 @@ struct mjt_wg_x {
             dhw[i] = ((unsigned)(r * DH) << 16) | (unsigned)(t * DW);
         });
     }
-    __device__ __forceinline__ void fetch(__amdgpu_buffer_rsrc_t d, const mjt_wg_chunk& ch) {
-        mjt_static_for<0, PER>([&](auto ic) {
-            constexpr int i = decltype(ic)::v;
-            mjt_static_for<0, EPC>([&](auto ec) {
-                constexpr int e = decltype(ec)::v;
-                const unsigned h = ch.hw[e] + dhw[i];
-                const bool in = (h >> 16) - 0x4000u < (unsigned)H_ && (h & 0xffffu) - 0x4000u < (unsigned)W_;
-                v[i][e] = mjt_wg_load(d, in ? ch.x[e] + koff[i] : MJT_NONE);
-            });
+    template <int I> __device__ __forceinline__ void fetch(__amdgpu_buffer_rsrc_t d, const mjt_wg_chunk& ch) {
+        mjt_static_for<0, EPC>([&](auto ec) {
+            constexpr int e = decltype(ec)::v;
+            const unsigned h = ch.hw[e] + dhw[I];
+            const bool in = (h >> 16) - 0x4000u < (unsigned)H_ && (h & 0xffffu) - 0x4000u < (unsigned)W_;
+            v[I][e] = mjt_wg_load(d, in ? ch.x[e] + koff[I] : MJT_NONE);
         });
     }
-    __device__ __forceinline__ void commit(unsigned char* lds, int tid) const {
-        mjt_static_for<0, PER>([&](auto ic) {
-            constexpr int i = decltype(ic)::v;
-            *(mjt_u32x4v*)(lds + (tid / KC + i * (NTHR / KC)) * ROWB + (tid % KC) * 16) = mjt_wg_pack(v[i]);
-        });
+    template <int I> __device__ __forceinline__ void commit(unsigned char* lds, int tid) const {
+        *(mjt_u32x4v*)(lds + (tid / KC + I * (NTHR / KC)) * ROWB + (tid % KC) * 16) = mjt_wg_pack(v[I]);
     }
 };
 #endif
@@ -430,8 +399,14 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
     const int slice = pair / slice_tiles;
     const int first_stage = slice * per_slice;
 #else
+#if SLICED
+    const TIN* __restrict__ A = (const TIN*)p.a[0];
+    const TIN* __restrict__ B = (const TIN*)p.a[1];
+    const int per_slice = (int)(long long)p.a[9], slice = blockIdx.y, first_stage = slice * per_slice;
+#else
     const TIN* __restrict__ A = (const TIN*)p.a[0] + (long long)blockIdx.y * (long long)p.a[9];
     const TIN* __restrict__ B = (const TIN*)p.a[1] + (long long)blockIdx.y * (long long)p.a[10];
+#endif
 #endif
     // NBUF 1: the host promises K <= KS, a single stage -- one staging buffer, so twice as many workgroups fit a compute unit
     __shared__ __attribute__((aligned(16))) unsigned char lds[NBUF][(TM + TN) * ROWB];
@@ -463,63 +438,78 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
 
-    // The operand tiles of a stage are asked for NSET stages ahead: one stage of 16-bit MFMAs on tiles up to 128 x 128
-    // is shorter than a trip to memory, so those keep two stages in registers (2048^3 bfloat16: 31.7 -> 30.6 us; tiles
-    // of 64 x 64: 40.8 -> 38.6 us).  Larger tiles have no registers to spare, and float32 stages are long enough (two
-    // sets: 153 -> 159 us for 2048^3).
-        constexpr int NSET = (NBUF > 1 && MI * NI <= 4 && IN != 2 && !CONV) ? 2 : 1;
+    // The operand tiles of a stage are asked for NSET stages ahead: one stage of MFMAs is shorter than a trip to memory on tiles
+    // up to 128 x 128 of 16-bit and on all float32 tiles that are run (us with one set / two / three, float32: 1024 x 1024 x 2048
+    // on 64 x 64 57.7 / 55.4 / 57.1, 2048^3 on 128 x 128 133 / 127 / -).  Larger tiles have no registers to spare.
+    // The gathering operands hold more registers: two sets on 64 x 64 tiles only (64 x 512 x 7 x 7 3x3 -> 512 247 / 218;
+    // 64 x 128 x 28 x 28 3x3 -> 128 on 128 x 128 186 / 194).
+    constexpr int NSET = NBUF > 1 && MI * NI <= (CONV ? 1 : 4) ? 2 : 1;
 #if CONV == 2
     const int all_stages = (K + KS - 1) / KS;
     const int nstages = all_stages - first_stage < per_slice ? all_stages - first_stage : per_slice;
     mjt_wg_dy sa[NSET];
     mjt_wg_x sb[NSET];
     mjt_static_for<0, NSET>([&](auto tc) { sa[decltype(tc)::v].init(m0, M, tid); sb[decltype(tc)::v].init(n0, N, tid); });
-    auto fetch = [&](auto setc, int stage) {
-        constexpr int SET = decltype(setc)::v;
-        mjt_wg_chunk ch;
-        ch.at((first_stage + stage) * KS, K, tid);
-        sa[SET].fetch(dy_rsrc, ch);
-        sb[SET].fetch(x_rsrc, ch);
+    mjt_wg_chunk ch;
+    constexpr int PA = mjt_wg_dy::PER, PIECES = PA + mjt_wg_x::PER;
+    auto fetch = [&](auto ic, auto setc, auto, int stage) {
+        constexpr int I = decltype(ic)::v, SET = decltype(setc)::v;
+        if constexpr (I == 0) ch.at((first_stage + stage) * KS, K, tid);
+        if constexpr (I < PA) sa[SET].template fetch<I>(dy_rsrc, ch);
+        else sb[SET].template fetch<I - PA>(x_rsrc, ch);
     };
-    auto commit = [&](auto setc, int stage) {
-        constexpr int SET = decltype(setc)::v;
+    auto commit = [&](auto ic, auto setc, auto, int stage) {
+        constexpr int I = decltype(ic)::v, SET = decltype(setc)::v;
         unsigned char* buf = &lds[stage & (NBUF - 1)][0];
-        sa[SET].commit(buf, tid);
-        sb[SET].commit(buf + TM * ROWB, tid);
+        if constexpr (I < PA) sa[SET].template commit<I>(buf, tid);
+        else sb[SET].template commit<I - PA>(buf + TM * ROWB, tid);
     };
 #else
+#if SLICED
+    const int all_stages = (K + KS - 1) / KS;
+    const int nstages = all_stages - first_stage < per_slice ? all_stages - first_stage : per_slice;
+#else
+    constexpr int first_stage = 0;
     const int nstages = NBUF == 1 ? 1 : (K + KS - 1) / KS;
+#endif
     mjt_stager<TM, A_KCONT> sa[NSET];
     const int arows = M, brows = N;
 #if CONV
+    const int img0 = n0 / (OH_ * OW_);
     mjt_conv_cols cols;
-    cols.init(n0, N, tid);
+    cols.init(n0, N, XBUF ? img0 : 0, tid);
     mjt_conv_stager sb[NSET];
+    const long long x_bytes = ((long long)(N / (OH_ * OW_)) - img0) * (C_ * H_) * W_ * ESZ;
+    const __amdgpu_buffer_rsrc_t x_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(B + (long long)img0 * (C_ * H_) * W_), 0,
+                                                                            (int)(x_bytes < 0x7fffffffll ? x_bytes : 0x7fffffffll), 0x00020000);
 #else
     mjt_stager<TN, B_KCONT> sb[NSET];
 #endif
-    auto fetch = [&](auto setc, int stage) {
-        constexpr int SET = decltype(setc)::v;
-        sa[SET].fetch(A, lda, m0, arows, stage * KS, K, tid);
+    constexpr int PA = TM * KC / NTHR, PIECES = PA + TN * KC / NTHR;
+    auto fetch = [&](auto ic, auto setc, auto fullc, int stage) {
+        constexpr int I = decltype(ic)::v, SET = decltype(setc)::v;
+        constexpr bool FULL = decltype(fullc)::v != 0;
+        if constexpr (I < PA) sa[SET].template fetch<I, FULL>(A, lda, m0, arows, (first_stage + stage) * KS, K, tid);
 #if CONV
-        sb[SET].fetch(B, cols, stage * KS, tid);
+        else sb[SET].template fetch<I - PA>(B, x_rsrc, cols, (first_stage + stage) * KS, tid);
 #else
-        sb[SET].fetch(B, ldb, n0, brows, stage * KS, K, tid);
+        else sb[SET].template fetch<I - PA, FULL>(B, ldb, n0, brows, (first_stage + stage) * KS, K, tid);
 #endif
     };
-    auto commit = [&](auto setc, int stage) {
-        constexpr int SET = decltype(setc)::v;
+    auto commit = [&](auto ic, auto setc, auto fullc, int stage) {
+        constexpr int I = decltype(ic)::v, SET = decltype(setc)::v;
+        constexpr bool FULL = decltype(fullc)::v != 0;
         unsigned char* buf = &lds[stage & (NBUF - 1)][0];
-        sa[SET].commit(buf, stage * KS, K, tid);
+        if constexpr (I < PA) sa[SET].template commit<I, FULL>(buf, (first_stage + stage) * KS, K, tid);
 #if CONV
-        sb[SET].commit(buf + TM * ROWB, tid);
+        else sb[SET].template commit<I - PA>(buf + TM * ROWB, tid);
 #else
-        sb[SET].commit(buf + TM * ROWB, stage * KS, K, tid);
+        else sb[SET].template commit<I - PA, FULL>(buf + TM * ROWB, (first_stage + stage) * KS, K, tid);
 #endif
     };
 #endif
     mjt_static_for<0, NSET>([&](auto tc) {
-        if (decltype(tc)::v < nstages) fetch(tc, decltype(tc)::v);
+        if (decltype(tc)::v < nstages) mjt_static_for<0, PIECES>([&](auto ic) { fetch(ic, tc, mjt_ic<0>(), decltype(tc)::v); });
     });
 
     mjt_f32x16 acc[MI][NI];
@@ -530,63 +520,84 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
 #pragma unroll
             for (int e = 0; e < 16; e++) acc[i][j][e] = 0.0f;
 
-    commit(mjt_ic<0>(), 0);
+    mjt_static_for<0, PIECES>([&](auto ic) { commit(ic, mjt_ic<0>(), mjt_ic<0>(), 0); });
+    if (NSET < nstages) mjt_static_for<0, PIECES>([&](auto ic) { fetch(ic, mjt_ic<0>(), mjt_ic<0>(), NSET); });
     __syncthreads();
 
     // fragment addresses of this lane: row lane % 32 of its wave's tile rows, chunk lane / 32
     const int frow = lane & 31, fhalf = lane >> 5;
-    // stage s: its tiles sit in LDS buffer s % NBUF; the registers of set s % NSET are free (committed before the
-    // stage began) and take stage s + NSET; at the end stage s + 1 goes from set (s + 1) % NSET to the other buffer
-    auto run_stage = [&](auto parc, const int s) {
-        constexpr int PAR = decltype(parc)::v;
-        const unsigned char* la = &lds[s & (NBUF - 1)][0] + (wm * 32 * MI + frow) * ROWB + fhalf * 16;
-        const unsigned char* lb = &lds[s & (NBUF - 1)][TM * ROWB] + (wn * 32 * NI + frow) * ROWB + fhalf * 16;
-        if (s + NSET < nstages) fetch(parc, s + NSET);
-        // a pair of chunks per step; the fragments of the next step are requested before the MFMAs of this one
-        mjt_u32x4v fa[2][MI], fb[2][NI];
-        const unsigned la_addr = (unsigned)(unsigned long long)(__attribute__((address_space(3))) const unsigned char*)la;
-        const unsigned lb_addr = (unsigned)(unsigned long long)(__attribute__((address_space(3))) const unsigned char*)lb;
-        auto request = [&](auto ksc, auto setc) {
-            constexpr int KSX = decltype(ksc)::v, SET = decltype(setc)::v;
-            mjt_static_for<0, MI>([&](auto ic) { mjt_ds_read<decltype(ic)::v * 32 * ROWB + KSX * 32>(fa[SET][decltype(ic)::v], la_addr); });
-            mjt_static_for<0, NI>([&](auto jc) { mjt_ds_read<decltype(jc)::v * 32 * ROWB + KSX * 32>(fb[SET][decltype(jc)::v], lb_addr); });
-        };
-        request(mjt_ic<0>(), mjt_ic<0>());
+    const unsigned char* const la = &lds[0][0] + (wm * 32 * MI + frow) * ROWB + fhalf * 16;
+    const unsigned char* const lb = &lds[0][TM * ROWB] + (wn * 32 * NI + frow) * ROWB + fhalf * 16;
+    // a pair of chunks per step; the fragments of the next step, across the end of a stage too, are requested before the MFMAs of
+    // this one (the scheduling barriers keep them there: the compiler would move every read next to its first use)
+    mjt_u32x4v fa[2][MI], fb[2][NI];
+    auto request = [&](auto ksc, auto setc, const int s) {
+        constexpr int KSX = decltype(ksc)::v, SET = decltype(setc)::v;
+        const int off = (s & (NBUF - 1)) * ((TM + TN) * ROWB) + KSX * 32;
+        mjt_static_for<0, MI>([&](auto ic) { fa[SET][decltype(ic)::v] = *(const mjt_u32x4v*)(la + off + decltype(ic)::v * 32 * ROWB); });
+        mjt_static_for<0, NI>([&](auto jc) { fb[SET][decltype(jc)::v] = *(const mjt_u32x4v*)(lb + off + decltype(jc)::v * 32 * ROWB); });
+    };
+    request(mjt_ic<0>(), mjt_ic<0>(), 0);
+    // Stage s: its tiles sit in LDS buffer s % NBUF, its first fragments are on their way, and the register sets hold the stages
+    // s + 1 .. s + NSET.  Piece by piece between the MFMAs of all steps but the last, stage s + 1 goes to the other buffer, which
+    // nobody has read since the barrier of stage s - 1, and its registers take stage s + 1 + NSET.  The barrier stands in front
+    // of the last step's MFMAs: every wave has then read the last fragments of this stage and written the next one, whose first
+    // fragments arrive during these MFMAs.
+    // FULL: stages s + 1 and s + 1 + NSET exist and do not reach beyond K -- no branches, so that the pieces' instructions can
+    // stand between MFMAs.
+    auto run_stage = [&](auto parc, auto fullc, const int s) {
+        constexpr int PAR = decltype(parc)::v, SET = (PAR + 1) % NSET;
+        constexpr bool FULL = decltype(fullc)::v != 0;
         mjt_static_for<0, KC / 2>([&](auto ksc) {
             constexpr int ks = decltype(ksc)::v, cur = ks & 1, nxt = cur ^ 1;
-            constexpr bool more = ks + 1 < KC / 2;
-            if constexpr (more) request(mjt_ic<ks + 1>(), mjt_ic<nxt>());
-            mjt_frag_wait<(more ? MI + NI : 0), MI>(fa[cur]);
-            mjt_frag_wait<(more ? MI + NI : 0), NI>(fb[cur]);
+            if constexpr (ks + 1 < KC / 2) {
+                request(mjt_ic<ks + 1>(), mjt_ic<nxt>(), s);
+            } else if (FULL || s + 1 < nstages) {
+                __syncthreads();
+                request(mjt_ic<0>(), mjt_ic<nxt>(), s + 1);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            constexpr int EK = IN == 2 ? 4 : 1, PER_STEP = EK * MI * NI, SLOTS = PER_STEP * (KC / 2 - 1) - PER_STEP / 2;
+            mjt_static_for<0, PER_STEP>([&](auto mc) {
+                constexpr int m = decltype(mc)::v, e = m / (MI * NI), i = m / NI % MI, j = m % NI, slot = ks * PER_STEP + m;
 #if IN == 2
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-#pragma unroll
-                for (int i = 0; i < MI; i++)
-#pragma unroll
-                    for (int j = 0; j < NI; j++)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(fa[cur][i][e]), __uint_as_float(fb[cur][j][e]), acc[i][j], 0, 0, 0);
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(fa[cur][i][e]), __uint_as_float(fb[cur][j][e]), acc[i][j], 0, 0, 0);
 #else
-#pragma unroll
-            for (int i = 0; i < MI; i++)
-#pragma unroll
-                for (int j = 0; j < NI; j++)
-                    acc[i][j] = MJT_MFMA16(__builtin_bit_cast(mjt_h8, fa[cur][i]), __builtin_bit_cast(mjt_h8, fb[cur][j]), acc[i][j]);
+                acc[i][j] = MJT_MFMA16(__builtin_bit_cast(mjt_h8, fa[cur][i]), __builtin_bit_cast(mjt_h8, fb[cur][j]), acc[i][j]);
 #endif
+                if constexpr (NBUF > 1 && ks + 1 < KC / 2) {
+                    constexpr int first = slot < SLOTS ? PIECES * slot / SLOTS : PIECES, last = slot + 1 < SLOTS ? PIECES * (slot + 1) / SLOTS : PIECES;
+                    if constexpr (FULL && last > first) {
+                        __builtin_amdgcn_sched_barrier(0);
+                        mjt_static_for<first, last>([&](auto ic) {
+                            commit(ic, mjt_ic<SET>(), mjt_ic<1>(), s + 1);
+                            fetch(ic, mjt_ic<SET>(), mjt_ic<1>(), s + 1 + NSET);
+                        });
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+            });
+            if constexpr (!FULL && NBUF > 1 && ks == KC / 2 - 2) {
+                if (s + 1 < nstages) {
+                    mjt_static_for<0, PIECES>([&](auto ic) { commit(ic, mjt_ic<SET>(), mjt_ic<0>(), s + 1); });
+                    if (s + 1 + NSET < nstages) mjt_static_for<0, PIECES>([&](auto ic) { fetch(ic, mjt_ic<SET>(), mjt_ic<0>(), s + 1 + NSET); });
+                }
+            }
         });
-        if (s + 1 < nstages) {
-            commit(mjt_ic<(PAR + 1) % NSET>(), s + 1);           // the other buffer: nobody reads it now
-            __syncthreads();
-        }
     };
-    for (int s0 = 0; s0 < nstages; s0 += NSET)
+    const int nstages_full = CONV == 2 ? nstages : K / KS - first_stage < nstages ? K / KS - first_stage : nstages;     // (the weight gradient's operands read zeros beyond K by themselves)
+    int s0 = 0;
+    if constexpr (NBUF > 1)
+        for (; s0 + 2 * NSET < nstages_full; s0 += NSET)
+            mjt_static_for<0, NSET>([&](auto parc) { run_stage(parc, mjt_ic<1>(), s0 + decltype(parc)::v); });
+    for (; s0 < nstages; s0 += NSET)
         mjt_static_for<0, NSET>([&](auto parc) {
-            if (s0 + decltype(parc)::v < nstages) run_stage(parc, s0 + decltype(parc)::v);
+            if (s0 + decltype(parc)::v < nstages) run_stage(parc, mjt_ic<0>(), s0 + decltype(parc)::v);
         });
 
     // D of a 32x32 tile: lane holds column lane % 32, rows 8 * (e / 4) + 4 * (lane / 32) + e % 4
 #if OUT == 2
-#if CONV == 2
+#if CONV == 2 || SLICED
     float* __restrict__ C = (float*)p.a[2] + (long long)slice * (long long)p.a[11];
 #else
     float* __restrict__ C = (float*)p.a[2] + (long long)blockIdx.y * (long long)p.a[11];

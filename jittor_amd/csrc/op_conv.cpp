@@ -500,7 +500,8 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
             const int in = x->dtype == MJT_BFLOAT16 ? 0 : x->dtype == MJT_FLOAT16 ? 1 : 2;
             const int out = y->dtype == MJT_BFLOAT16 ? 0 : y->dtype == MJT_FLOAT16 ? 1 : 2;
             std::ostringstream key;
-            key << "igemm|" << geo.str() << MI << NI << in << out;
+            const bool xbuf = (64 * NI / P + 2) * C * H * W * esz < (int64_t(1) << 31);      // a tile's images through one buffer descriptor
+            key << "igemm|" << geo.str() << MI << NI << in << out << xbuf;
             JitKernel* k = cached(key.str());
             if (!k) {
                 std::ostringstream name;
@@ -508,7 +509,7 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
                      << p->stride_w << "_p" << p->pad_h << "x" << p->pad_w << "_d" << p->dil_h << "x" << p->dil_w << "_" << 64 * MI << "x" << 64 * NI;
                 std::ostringstream src;
                 src << "#define ENTRY " << name.str() << "\n#define CONV 1\n#define IN " << in << "\n#define OUT " << out << "\n#define MI " << MI << "\n#define NI " << NI
-                    << "\n#define A_KCONT 1\n#define B_KCONT 0\n" << geo.str();
+                    << "\n#define A_KCONT 1\n#define B_KCONT 0\n#define XBUF " << (xbuf ? 1 : 0) << "\n" << geo.str();
                 src << embedded_source("gemm_mfma.h") << "\n";
                 k = jit_get(src.str(), name.str());
                 remember(key.str(), k);

@@ -139,19 +139,40 @@ void gemm_launch(int in_dtype, int out_dtype, const void* A, const void* B, void
         // the caller's tile, if it names one (tile_m x tile_n of 64, 128 or 256)
         if (tile_m == 64 || tile_m == 128 || tile_m == 256) best_mi = tile_m / 64;
         if (tile_n == 64 || tile_n == 128 || tile_n == 256) best_ni = tile_n / 64;
+        // Few tiles and a long sum: the sum is cut into slices, whose float32 results a reduce launch adds up.  A stage of a
+        // 64 x 64 tile takes about 0.75 us in float32 and 0.5 in 16 bits with a compute unit to itself, 1.75 / 2.6 / 3.4 times that
+        // with two / three / four workgroups a unit; the reduce launch 5 us and its traffic.  At most 16 slices: their reduce is
+        // a single launch, which leaves the scratch memory alone.  (us whole / in slices; a^T b: 512 x 512 x 8192 float32
+        // 183 / 50, bfloat16 64.5 / 22.7; 64 x 64 x 4096 float32 94 / 13.5; 1024 x 512 x 4096 float32 96 / 50; a b^T:
+        // 256 x 1024 x 1024 float32 20.1 / 12.4; 1024 x 1024 x 2048 a^T b, 256 tiles, 50.4 / 50.6, stays whole.)
+        const int64_t ks = esz == 2 ? 64 : 32, stages = (K + ks - 1) / ks;
+        int64_t slices = 1, per = stages;
+        if (batch == 1 && !tile_m && !tile_n && ldc == N) {
+            const double st = esz == 2 ? 0.5 : 0.75;
+            auto crowd = [&](double wgs) { const double r = std::ceil(wgs / cus); return 1.0 + 0.8 * (r - 1.0); };
+            const double tiles64 = (double)((M + 63) / 64) * ((N + 63) / 64);
+            const double whole = (double)stages * st * crowd(tiles64) * (best_mi * best_ni > 1 ? 0.95 : 1.0);
+            double least = 0.9 * whole;
+            for (int64_t n = 2; n <= 16 && n <= stages / 4; n++) {
+                const int64_t pn = (stages + n - 1) / n, nn = (stages + pn - 1) / pn;
+                const double t = (double)pn * st * crowd(tiles64 * nn) + 5.0 + (double)nn * M * N * 8 / 3e6;
+                if (t < least && nn * M * N * 4 <= (int64_t(256) << 20)) { least = t; slices = nn; per = pn; }
+            }
+        }
+        if (slices > 1) best_mi = best_ni = 1;
         const int MI = best_mi, NI = best_ni;
         const int in = in_dtype == MJT_BFLOAT16 ? 0 : in_dtype == MJT_FLOAT16 ? 1 : 2;
-        const int out = out_dtype == MJT_BFLOAT16 ? 0 : out_dtype == MJT_FLOAT16 ? 1 : 2;
-        const bool one_stage = K <= (esz == 2 ? 64 : 32) && !getenv("MJT_GEMM_TWO_BUFFERS");       // a single stage of the kernel's k loop
+        const int out = slices > 1 || out_dtype == MJT_FLOAT32 ? 2 : out_dtype == MJT_BFLOAT16 ? 0 : 1;
+        const bool one_stage = stages == 1 && !getenv("MJT_GEMM_TWO_BUFFERS");       // a single stage of the kernel's k loop
         std::ostringstream key;
-        key << "gemm|" << in << out << MI << NI << a_kcont << b_kcont << one_stage;
+        key << "gemm|" << in << out << MI << NI << a_kcont << b_kcont << one_stage << (slices > 1);
         JitKernel* k = cached(key.str());
         if (!k) {
             std::ostringstream name;
-            name << "mjt_gemm_mfma_" << mjt_dtype_name(in_dtype) << "_" << mjt_dtype_name(out_dtype) << "_" << 64 * MI << "x" << 64 * NI
-                 << (a_kcont ? "_n" : "_t") << (b_kcont ? "t" : "n") << (one_stage ? "_k1" : "");
+            name << "mjt_gemm_mfma_" << mjt_dtype_name(in_dtype) << "_" << (out == 2 ? "float32" : mjt_dtype_name(out_dtype)) << "_" << 64 * MI << "x" << 64 * NI
+                 << (a_kcont ? "_n" : "_t") << (b_kcont ? "t" : "n") << (one_stage ? "_k1" : "") << (slices > 1 ? "_slices" : "");
             std::ostringstream src;
-            src << "#define NBUF " << (one_stage ? 1 : 2) << "\n";
+            src << "#define NBUF " << (one_stage ? 1 : 2) << "\n#define SLICED " << (slices > 1 ? 1 : 0) << "\n";
             src << "#define ENTRY " << name.str() << "\n#define IN " << in << "\n#define OUT " << out << "\n#define MI " << MI
                 << "\n#define NI " << NI << "\n#define A_KCONT " << (a_kcont ? 1 : 0) << "\n#define B_KCONT " << (b_kcont ? 1 : 0) << "\n";
             src << embedded_source("gemm_mfma.h") << "\n";
@@ -161,7 +182,26 @@ void gemm_launch(int in_dtype, int out_dtype, const void* A, const void* B, void
         const int64_t tiles = ((M + 64 * MI - 1) / (64 * MI)) * ((N + 64 * NI - 1) / (64 * NI));
         const int64_t grid = (tiles + 7) / 8 * 8;
         MJT_CHECK(grid < (int64_t(1) << 31), "matmul: launch too large");
-        jit_launch(k, (unsigned)grid, (unsigned)batch, 256, 0, args);
+        if (slices == 1) {
+            jit_launch(k, (unsigned)grid, (unsigned)batch, 256, 0, args);
+            return;
+        }
+        mjt_tensor part{}, whole{};
+        part.ptr = scratch((size_t)(slices * M * N * 4));
+        part.dtype = MJT_FLOAT32;
+        part.ndim = 2;
+        part.shape[0] = slices;
+        part.shape[1] = M * N;
+        whole.ptr = C;
+        whole.dtype = out_dtype;
+        whole.ndim = 1;
+        whole.shape[0] = M * N;
+        args[2] = bits_of_ptr(part.ptr);
+        args[9] = (uint64_t)per;
+        args[11] = (uint64_t)(M * N);
+        jit_launch(k, (unsigned)grid, (unsigned)slices, 256, 0, args);
+        if (mjt_reduce(&part, &whole, MJT_OP_ADD, 0b01) != MJT_OK) MJT_FAIL(MJT_ERR_DEVICE, "matmul: adding up the slices failed: " << mjt_last_error());
+        set_last_kernel(k->name.c_str());
         return;
     }
     std::ostringstream key;

@@ -240,3 +240,27 @@ def test_gemm_full_size_4096_bf16_properties(gpu):
     finally:
         for p in (pa, pb, pc):
             L.free(p)
+
+
+@pytest.mark.parametrize("dt", ["bfloat16", "float32"])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_gemm_stage_pipeline_lengths(gpu, dt, ta, tb):
+    """Sums of one stage up to several (64 elements of 16 bits, 32 of float32), whole and with a remainder: fewer stages than are
+    in flight, the last whole ones, a last one that ends inside a chunk; tiles of 64 and more, over both edges."""
+    lib = L.load()
+    ks = 32 if dt == "float32" else 64
+    for stages in range(1, 9):
+        for rest in (0, 8):
+            _run(lib, dt, "float32", 72, ks * stages + rest, 136, ta, tb, seed=stages)
+    _run(lib, dt, dt, 1032, 7 * ks + 8, 1160, ta, tb, seed=9)
+    _run(lib, dt, dt, 72, 3 * ks + 8, 72, ta, tb, seed=10, batch=(5,))
+
+
+@pytest.mark.parametrize("dt", ["bfloat16", "float16", "float32"])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_gemm_slices_of_a_long_sum(gpu, dt, ta, tb):
+    """Few tiles and a long sum: slices of the sum, added up by a reduce; the last slice shorter and ending inside a stage."""
+    lib = L.load()
+    for M, K, N in ((64, 4104, 72), (8, 2000, 520), (264, 8200, 200)):
+        assert _run(lib, dt, dt, M, K, N, ta, tb, seed=K).endswith("_slices")
+        assert _run(lib, dt, "float32", M, K, N, ta, tb, seed=K + 1).endswith("_slices")
