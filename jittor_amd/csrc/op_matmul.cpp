@@ -21,9 +21,16 @@ void launch_fill_pattern(void* dst, uint64_t pattern, int elem_size, size_t n);
 namespace {
 std::mutex g_mu;
 std::unordered_map<std::string, JitKernel*> g_kernels;
+void* g_rows[2] = {nullptr, nullptr};      // operands with rows padded to 16 bytes (guarded by the library's lock, as the scratch memory)
+size_t g_rows_bytes[2] = {0, 0};
 void forget() {   // the kernels belong to the run-time compiler's cache, which mjt_shutdown empties
     std::lock_guard<std::mutex> lock(g_mu);
     g_kernels.clear();
+    for (int i = 0; i < 2; i++) {
+        if (g_rows[i] && !ctx().dry_run) (void)hipFree(g_rows[i]);
+        g_rows[i] = nullptr;
+        g_rows_bytes[i] = 0;
+    }
 }
 const bool g_registered = (at_shutdown(&forget), true);
 
@@ -39,6 +46,34 @@ void remember(const std::string& key, JitKernel* k) {
 int env_int(const char* name, int dflt) {
     const char* v = getenv(name);
     return v && *v ? atoi(v) : dflt;
+}
+
+// [rows, ld] copied into rows of `ldp` elements (zeros behind each), into the buffer of operand `which`.
+const void* padded_rows(int which, const void* src, int dtype, int64_t rows, int64_t ld, int64_t ldp) {
+    Context& c = ctx();
+    const size_t bytes = (size_t)(rows * ldp * dtype_size(dtype));
+    if (!c.dry_run && bytes > g_rows_bytes[which]) {
+        kept_buffer_moved();
+        if (g_rows[which]) {
+            HIP_CHECK(hipStreamSynchronize(c.stream));
+            HIP_CHECK(hipFree(g_rows[which]));
+            g_rows[which] = nullptr;
+            g_rows_bytes[which] = 0;
+        }
+        HIP_CHECK(hipMalloc(&g_rows[which], bytes));
+        g_rows_bytes[which] = bytes;
+    }
+    mjt_tensor t{}, d{};
+    t.ptr = (void*)src;
+    d.ptr = c.dry_run ? (void*)(uintptr_t)0x1000 : g_rows[which];
+    t.dtype = d.dtype = dtype;
+    t.ndim = d.ndim = 2;
+    t.shape[0] = d.shape[0] = rows;
+    t.shape[1] = ld;
+    d.shape[1] = ldp;
+    const char* idx[2] = {"i0", "i1"};                          // columns past ld lie outside the source: overflow value 0
+    if (mjt_reindex(&t, &d, 2, idx, 0.0, 0, nullptr, 0, nullptr) != MJT_OK) MJT_FAIL(MJT_ERR_DEVICE, "matmul: padding the rows failed: " << mjt_last_error());
+    return d.ptr;
 }
 }  // namespace
 
@@ -301,6 +336,26 @@ void matmul_impl(const mjt_tensor* a, const mjt_tensor* b, const mjt_tensor* c, 
     }
     // c[n,k] = a'[n,m] * b'[m,k]: rows n, columns k, sum over m
     const int64_t lda = a->shape[nd - 1], ldb = b->shape[nd - 1];
+    // Rows that are no 16-byte multiples, or operands that do not begin at one, are what only the kernel without MFMAs takes as
+    // they lie, 0.14 us for every element of the sum however few tiles there are.  From a few million multiply-adds on, or one
+    // million and a sum of some length, they are copied into padded rows first, 6 to 9 us with the launches (us as they lie /
+    // copied: bfloat16 a b^T 1000 x 500 x 900 111 / 15.8, a b 300 x 300 x 700 86.5 / 14.2, a b^T 100 x 1000 x 300 38.3 / 11.7;
+    // float32 a b^T 130 x 100 x 333 45.3 / 14.7).
+    {
+        const int esz = dtype_size(a->dtype);
+        const int64_t ra = batch * a->shape[nd - 2], rb = batch * b->shape[nd - 2], epc = 16 / esz;
+        const int64_t lap = (lda + epc - 1) / epc * epc, lbp = (ldb + epc - 1) / epc * epc;
+        const bool pad_a = lda != lap || (uintptr_t)a->ptr % 16, pad_b = ldb != lbp || (uintptr_t)b->ptr % 16;
+        const int64_t most = int64_t(1) << 30;
+        if ((pad_a || pad_b) && a->dtype != MJT_FLOAT64 && !share_a && batch < 65536 && !getenv("MJT_GEMM_PLAIN") && !getenv("MJT_NO_FASTPATH") &&
+            (double)batch * n * k * m >= (double)(1 << (m >= 96 ? 20 : 22)) && (!pad_a || ra * lap * esz <= most) && (!pad_b || rb * lbp * esz <= most)) {
+            const void* pa = pad_a ? padded_rows(0, a->ptr, a->dtype, ra, lda, lap) : a->ptr;
+            const void* pb = pad_b ? padded_rows(1, b->ptr, b->dtype, rb, ldb, lbp) : b->ptr;
+            const int64_t la = pad_a ? lap : lda, lb = pad_b ? lbp : ldb;
+            gemm_launch(a->dtype, c->dtype, pa, pb, c->ptr, n, k, m, la, lb, k, a->shape[nd - 2] * la, b->shape[nd - 2] * lb, n * k, batch, !trans_a, trans_b != 0, 0, 0, k % 8 == 0);
+            return;
+        }
+    }
     const int64_t per_launch = 65535;                         // the batch rides on a grid axis
     for (int64_t b0 = 0; b0 < batch; b0 += per_launch) {
         const int64_t nb = batch - b0 < per_launch ? batch - b0 : per_launch;

@@ -264,3 +264,13 @@ def test_gemm_slices_of_a_long_sum(gpu, dt, ta, tb):
     for M, K, N in ((64, 4104, 72), (8, 2000, 520), (264, 8200, 200)):
         assert _run(lib, dt, dt, M, K, N, ta, tb, seed=K).endswith("_slices")
         assert _run(lib, dt, "float32", M, K, N, ta, tb, seed=K + 1).endswith("_slices")
+
+
+@pytest.mark.parametrize("dt", ["bfloat16", "float16", "float32"])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_gemm_unaligned_rows_are_copied(gpu, dt, ta, tb):
+    """Rows that are no 16-byte multiples, from a few million multiply-adds on: one operand copied, both, batches."""
+    lib = L.load()
+    for i, (M, K, N) in enumerate([(301, 203, 129), (304, 201, 136), (129, 336, 201), (1001, 1001, 67), (257, 4099, 65)]):
+        assert _run(lib, dt, dt, M, K, N, ta, tb, seed=i).startswith("mjt_gemm_mfma_"), (M, K, N)
+    assert _run(lib, dt, dt, 61, 203, 129, ta, tb, seed=7, batch=(5,)).startswith("mjt_gemm_mfma_")
