@@ -8,6 +8,8 @@ ops/reindex_op.cc:20-91, ops/reindex_reduce_op.cc:26-73, ops/array_op.cc:54-80).
 Nothing executes until a Var is synchronised (lazy_execution,
 var_holder.cc:25-33); execution is in executor.py.
 """
+import functools
+import itertools
 import math
 import numbers
 import weakref
@@ -19,8 +21,8 @@ from . import dtypes as dt
 from ._lib import MjtError
 from .flags import flags as _flags
 
-_next_id = [0]
 _grad_enabled = [True]
+_flag_value = dict.__getitem__
 
 
 class no_grad:
@@ -36,9 +38,8 @@ class no_grad:
         return False
 
 
-def _new_id():
-    _next_id[0] += 1
-    return _next_id[0]
+_new_id = itertools.count(1).__next__
+_ref = weakref.ref
 
 
 # --------------------------------------------------------------------------
@@ -130,11 +131,13 @@ class Buffer:
 class Op:
     kind = "op"
     fusable = False        # element / broadcast type (executor.cc:555)
+    _out_ref = None
 
     def __init__(self, inputs):
-        self.inputs = list(inputs)
-        me = weakref.ref(self)
-        for v in self.inputs:              # who reads a Var (weakly): Var.assign moves them to the old value
+        """Takes the list over."""
+        self.inputs = inputs
+        me = _ref(self)
+        for v in inputs:                   # who reads a Var (weakly): Var.assign moves them to the old value
             lst = v._consumers
             if lst is None:
                 v._consumers = [me]
@@ -143,7 +146,6 @@ class Op:
                 if len(lst) > 64 and len(lst) & (len(lst) - 1) == 0:     # a long-lived var (a weight): drop the dead readers now and then
                     lst[:] = [r for r in lst if r() is not None]
         self.id = _new_id()
-        self._out_ref = None
         self.amp = dt.amp_reg & 63          # the register at creation; its gradient is built under it (op.cc:38, grad.cc:48-55)
 
     # The result is held weakly: a Var owns its producing op (and through it the inputs), never the other way round, so
@@ -156,7 +158,11 @@ class Op:
 
     @out.setter
     def out(self, v):
-        self._out_ref = weakref.ref(v) if v is not None else None
+        self._out_ref = _ref(v) if v is not None else None
+
+    def sig(self):
+        """What the execution depends on besides the operands and the result (None: not known)."""
+        return None
 
     def __repr__(self):
         return "%s#%d" % (self.kind, self.id)
@@ -167,8 +173,11 @@ class UnaryOp(Op):
     fusable = True
 
     def __init__(self, x, op):
-        super().__init__([x])
+        Op.__init__(self, [x])
         self.op = op
+
+    def sig(self):
+        return ("unary", self.op)
 
 
 class BinaryOp(Op):
@@ -176,8 +185,11 @@ class BinaryOp(Op):
     fusable = True
 
     def __init__(self, x, y, op):
-        super().__init__([x, y])
+        Op.__init__(self, [x, y])
         self.op = op
+
+    def sig(self):
+        return ("binary", self.op)
 
 
 class TernaryOp(Op):
@@ -185,7 +197,10 @@ class TernaryOp(Op):
     fusable = True
 
     def __init__(self, c, x, y):
-        super().__init__([c, x, y])
+        Op.__init__(self, [c, x, y])
+
+    def sig(self):
+        return ("ternary",)
 
 
 class BroadcastOp(Op):
@@ -193,39 +208,52 @@ class BroadcastOp(Op):
     fusable = True
 
     def __init__(self, x, bcast_mask, keepdims_mask):
-        super().__init__([x])
+        Op.__init__(self, [x])
         self.bcast_mask = bcast_mask
         self.keepdims_mask = keepdims_mask
+
+    def sig(self):
+        return ("broadcast", self.bcast_mask, self.keepdims_mask)
 
 
 class ReduceOp(Op):
     kind = "reduce"
 
     def __init__(self, x, op, reduce_mask, keepdims_mask):
-        super().__init__([x])
+        Op.__init__(self, [x])
         self.op = op
         self.reduce_mask = reduce_mask
         self.keepdims_mask = keepdims_mask
 
+    def sig(self):
+        return ("reduce", self.op, self.reduce_mask, self.keepdims_mask)
+
 
 class ReindexOp(Op):
     kind = "reindex"
+    same_memory = False    # a row-major reinterpretation of the input
 
     def __init__(self, x, indexes, overflow_value, overflow_conditions, extras):
-        super().__init__([x] + list(extras))
+        Op.__init__(self, [x] + list(extras))
         self.indexes = list(indexes)
         self.overflow_value = float(overflow_value)
         self.overflow_conditions = list(overflow_conditions)
+
+    def sig(self):
+        return ("reindex", tuple(self.indexes), self.overflow_value, tuple(self.overflow_conditions), self.same_memory)
 
 
 class ReindexReduceOp(Op):
     kind = "reindex_reduce"
 
     def __init__(self, y, op, indexes, overflow_conditions, extras):
-        super().__init__([y] + list(extras))
+        Op.__init__(self, [y] + list(extras))
         self.op = op
         self.indexes = list(indexes)
         self.overflow_conditions = list(overflow_conditions)
+
+    def sig(self):
+        return ("reindex_reduce", self.op, tuple(self.indexes), tuple(self.overflow_conditions))
 
 
 # --------------------------------------------------------------------------
@@ -237,42 +265,47 @@ class Var:
 
     __array_priority__ = 100
 
-    def __init__(self, shape, dtype, op=None):
-        shape = [int(s) for s in shape]
-        if len(shape) == 0:
-            shape = [1]
-        if len(shape) > _lib.MAX_DIM:
-            raise ValueError("at most %d dims are supported" % _lib.MAX_DIM)
-        n = 1
-        for e in shape:
-            if e < 0:
-                raise ValueError("Shape should greater than 0: %r" % (shape,))
-            n *= e
+    # what most Vars never change (set on the instance where it is)
+    _buf = None              # Buffer once materialised
+    _host = None             # host copy for array leaves (and fused scalars)
+    is_scalar = False        # NodeFlags::_is_scalar
+    _name = None
+    _consumers = None        # ops that take this Var as an input (weakly)
+    _compile_options = None
+    _stop_fuse = False
+
+    def __init__(self, shape, dtype, op=None, num=None):
+        """With `num` given, `shape` is a list of the caller's making with that many elements and is taken over."""
+        if num is None:
+            shape = [int(s) for s in shape]
+            if len(shape) == 0:
+                shape = [1]
+            if len(shape) > _lib.MAX_DIM:
+                raise ValueError("at most %d dims are supported" % _lib.MAX_DIM)
+            num = 1
+            for e in shape:
+                if e < 0:
+                    raise ValueError("Shape should greater than 0: %r" % (shape,))
+                num *= e
         self.shape = shape
-        self._num = n
+        self.num = num
         self.dtype = dtype
         self._op = op
-        if op is not None:
-            op.out = self
         # history for grad(): the producing op and its inputs outlive materialisation (the executor
         # clears _op / op.inputs of computed vars), like the reference's backward liveness
         # (python/jittor/src/node.h).  Cleared by stop_grad() and under no_grad().
-        self._history = (op, tuple(op.inputs)) if op is not None and _grad_enabled[0] else None
-        self._buf = None         # Buffer once materialised
-        self._host = None        # host copy for array leaves (and fused scalars)
-        self.is_scalar = False   # NodeFlags::_is_scalar
+        if op is not None:
+            op._out_ref = _ref(self)
+            self._history = (op, tuple(op.inputs)) if _grad_enabled[0] else None
+        else:
+            self._history = None
         self.id = _new_id()
-        self._name = None
-        self._consumers = None   # ops that take this Var as an input (weakly)
         # compile options: the flag's value at creation (var.cc:75)
-        co = dict.__getitem__(_flags, "compile_options")
-        self._compile_options = dict(co) if co else None
+        co = _flag_value(_flags, "compile_options")
+        if co:
+            self._compile_options = dict(co)
 
     # ---- properties ----
-    @property
-    def num(self):
-        return self._num
-
     @property
     def ndim(self):
         return len(self.shape)
@@ -370,7 +403,8 @@ class Var:
         return self.numpy()
 
     def raw_ptr(self):
-        self.sync()
+        if self._buf is None:
+            self.sync()
         return self._device_ptr()
 
     # ---- op sugar ----
@@ -463,6 +497,7 @@ class Var:
             self._split_off_value()
         name = self._name
         src = other._split_off_value()                 # `other` stays valid: it now reads this Var (and has a new id)
+        self.__dict__.clear()
         self.__dict__.update(src.__dict__)             # with the id of the value taken over
         self._name = name
         if self._op is not None:
@@ -620,21 +655,26 @@ def _as_var(v):
 # --------------------------------------------------------------------------
 # constructors
 # --------------------------------------------------------------------------
+_DTYPE_SET, _UNARY_SET, _BINARY_SET = frozenset(_lib.DTYPES), frozenset(_lib.UNARY_OPS), frozenset(_lib.BINARY_OPS)
+
+
 def unary(x, op, force_dtype=None, allow_forward=True):
     """ops/unary_op.cc:860-889.  `op` is a unary op name or a dtype name."""
-    x = _as_var(x)
-    if op in _lib.DTYPES and op != "void":
+    if not isinstance(x, Var):
+        x = _as_var(x)
+    if op in _DTYPE_SET and op != "void":
         if op == x.dtype and allow_forward:
             return x                      # forward(x), unary_op.cc:867-870
         dtype, op = op, "cast"
     elif op == "cast" and force_dtype is not None:
         dtype = force_dtype
     else:
-        if op not in _lib.UNARY_OPS:
+        if op not in _UNARY_SET:
             raise ValueError("unknown unary op %r" % (op,))
         dtype = dt.unary_dtype_infer(op, x.dtype)
-    y = Var(x.shape, dtype, UnaryOp(x, op))
-    y.is_scalar = x.is_scalar
+    y = Var(x.shape[:], dtype, UnaryOp(x, op), x.num)
+    if x.is_scalar:
+        y.is_scalar = True
     return y
 
 
@@ -650,7 +690,13 @@ def _need_broadcast(xshape, shape):
 
 def _broadcast_shape(xshape, yshape, bmask, kmask):
     """infer_shape of ops/broadcast_to_op.cc:119-168.  Returns
-    (zshape, bcast_mask, keepdims_mask) with the implicit broadcasts added."""
+    (zshape, bcast_mask, keepdims_mask, elements of zshape) with the implicit broadcasts added; the list is the caller's."""
+    zz, bmask, kmask, num = _broadcast_rule(tuple(xshape), tuple(yshape), bmask, kmask)
+    return list(zz), bmask, kmask, num
+
+
+@functools.lru_cache(maxsize=4096)           # (a pure function of extents and masks)
+def _broadcast_rule(xshape, yshape, bmask, kmask):
     xdim, ydim = len(xshape), len(yshape)
     cnt = bin(bmask & ~kmask).count("1")
     zdim = max(xdim, ydim - cnt) + cnt
@@ -674,12 +720,17 @@ def _broadcast_shape(xshape, yshape, bmask, kmask):
             zs = xs * ys
         else:
             if xs != ys:
-                raise ValueError("Shape not match %r %r" % (xshape, yshape))
+                raise ValueError("Shape not match %r %r" % (list(xshape), list(yshape)))
             zs = xs
         zz[i] = zs
         xi -= 1
         yi -= 1
-    return zz, bmask, kmask
+    if zdim > _lib.MAX_DIM:
+        raise ValueError("at most %d dims are supported" % _lib.MAX_DIM)
+    for e in zz:
+        if e < 0:
+            raise ValueError("Shape should greater than 0: %r" % (zz,))
+    return tuple(zz), bmask, kmask, math.prod(zz)
 
 
 def broadcast(x, shape, dims=()):
@@ -708,9 +759,10 @@ def broadcast(x, shape, dims=()):
         if not (0 <= d < ydim):
             raise ValueError("Wrong dims number: %r" % (dims,))
         bmask |= 1 << d
-    zshape, bmask, kmask = _broadcast_shape(x.shape, shape, bmask, 0)
-    z = Var(zshape, x.dtype, BroadcastOp(x, bmask, kmask))
-    z.is_scalar = x.is_scalar
+    zshape, bmask, kmask, num = _broadcast_shape(x.shape, shape, bmask, 0)
+    z = Var(zshape, x.dtype, BroadcastOp(x, bmask, kmask), num)
+    if x.is_scalar:
+        z.is_scalar = True
     return z
 
 
@@ -720,20 +772,27 @@ def broadcast_var(x, y, dims=()):
 
 def _broadcast_mask(x, shape, bmask, kmask):
     """make_broadcast_to(x, shape, dims_mask, keepdims_mask), used by grads."""
-    if not bin(bmask).count("1"):
+    if not bmask:
         return x
-    zshape, bmask, kmask = _broadcast_shape(x.shape, list(shape), bmask, kmask)
-    z = Var(zshape, x.dtype, BroadcastOp(x, bmask, kmask))
-    z.is_scalar = x.is_scalar
+    zshape, bmask, kmask, num = _broadcast_shape(x.shape, shape, bmask, kmask)
+    z = Var(zshape, x.dtype, BroadcastOp(x, bmask, kmask), num)
+    if x.is_scalar:
+        z.is_scalar = True
     return z
 
 
 def binary(x, y, op):
     """ops/binary_op.cc:421-474: broadcasts are inserted when ranks differ or
     an extent is 1 on one side only; other mismatches are errors."""
-    x, y = _as_var(x), _as_var(y)
-    if op not in _lib.BINARY_OPS:
+    if not isinstance(x, Var):
+        x = _as_var(x)
+    if not isinstance(y, Var):
+        y = _as_var(y)
+    if op not in _BINARY_SET:
         raise ValueError("unknown binary op %r" % (op,))
+    if x.shape == y.shape:
+        dtype = dt.binary_dtype_infer(op, x.dtype, y.dtype, x.is_scalar, y.is_scalar)
+        return Var(x.shape[:], dtype, BinaryOp(x, y, op), x.num)
     need = x.ndim != y.ndim
     for i in range(1, min(x.ndim, y.ndim) + 1):
         xs, ys = x.shape[-i], y.shape[-i]
@@ -753,6 +812,9 @@ def binary(x, y, op):
 def ternary(cond, x, y):
     """ops/ternary_op.cc:21-47."""
     cond, x, y = _as_var(cond), _as_var(x), _as_var(y)
+    if cond.shape == x.shape == y.shape:
+        dtype = x.dtype if x.dtype == y.dtype else dt.dtype_infer(x.dtype, y.dtype, x.is_scalar, y.is_scalar)
+        return Var(x.shape[:], dtype, TernaryOp(cond, x, y), x.num)
     bx = cond.ndim > x.ndim or cond.num > x.num
     by = cond.ndim > y.ndim or cond.num > y.num
     bx2 = cond.ndim < x.ndim or cond.num < x.num
@@ -885,5 +947,15 @@ def reindex_reduce(y, op, shape, indexes, overflow_conditions=(), extras=()):
 
 def make_number(value, like):
     """ops/op_utils.cc:19-36: a [1] array of like's dtype broadcast to like."""
-    v = array(value, like.dtype)
+    if like.shape == [1]:                        # nothing to spread: the caller's own Var
+        return array(value, like.dtype)
+    tv = type(value)
+    if tv is not float and tv is not int:
+        return broadcast(array(value, like.dtype), like.shape)
+    key = (tv, value, math.copysign(1.0, value), like.dtype)
+    v = _scalar_vars.get(key)
+    if v is None:
+        if len(_scalar_vars) >= 4096:
+            _scalar_vars.clear()
+        v = _scalar_vars[key] = array(value, like.dtype)
     return broadcast(v, like.shape)

@@ -82,8 +82,21 @@ def dtype_infer(x, y, xscalar=False, yscalar=False):
     return int_dtype(d)
 
 
+_binary_dtypes = {}      # what the rules below give, by their arguments and the register (a few hundred entries at most)
+
+
 def binary_dtype_infer(op, x, y, xscalar=False, yscalar=False):
     """nano_string.h:238-254."""
+    key = (op, x, y, xscalar, yscalar, amp_reg)
+    got = _binary_dtypes.get(key)
+    if got is None:
+        if len(_binary_dtypes) >= 4096:
+            _binary_dtypes.clear()
+        got = _binary_dtypes[key] = _binary_dtype(op, x, y, xscalar, yscalar)
+    return got
+
+
+def _binary_dtype(op, x, y, xscalar, yscalar):
     if op in BOOL_OPS:
         return "bool"
     d = max(dsize_(x), dsize_(y))

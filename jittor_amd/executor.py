@@ -221,23 +221,24 @@ def _match_conv_bwd(op):
 def _pending_ops(targets):
     """Pending producers behind `targets`, in topological order."""
     order, seen = [], set()
-    stack = [(v, False) for v in targets]
+    stack = [v._op for v in targets if v._buf is None and v._op is not None]
     while stack:
-        v, done = stack.pop()
-        if v.materialised:
-            continue
-        op = v._op
-        if done:
+        op = stack.pop()
+        if op is None:                                          # the op below it: everything it reads has been visited
+            op = stack.pop()
             if op.id not in seen:
                 seen.add(op.id)
                 order.append(op)
             continue
         if op.id in seen:
             continue
-        stack.append((v, True))
+        stack.append(op)
+        stack.append(None)
         for u in op.inputs:
-            if not u.materialised and u._op.id not in seen:
-                stack.append((u, False))
+            if u._buf is None:
+                p = u._op
+                if p is not None and p.id not in seen:
+                    stack.append(p)
     return order
 
 
@@ -517,47 +518,32 @@ def _libh():
     return _cap if _cap is not None else _lib.ensure_init()
 
 
-def _op_sig(op):
-    if isinstance(op, (UnaryOp, BinaryOp)):
-        return (op.kind, op.op)
-    if isinstance(op, TernaryOp):
-        return (op.kind,)
-    if isinstance(op, BroadcastOp):
-        return (op.kind, op.bcast_mask, op.keepdims_mask)
-    if isinstance(op, ReduceOp):
-        return (op.kind, op.op, op.reduce_mask, op.keepdims_mask)
-    if isinstance(op, ReindexOp):
-        return (op.kind, tuple(op.indexes), op.overflow_value, tuple(op.overflow_conditions), getattr(op, "same_memory", False))
-    if isinstance(op, ReindexReduceOp):
-        return (op.kind, op.op, tuple(op.indexes), tuple(op.overflow_conditions))
-    return None
-
-
 def _signature(ops, target_ids):
     """Hashable description of everything the execution of `ops` depends on besides the data, or None."""
     pos, leaf, parts = {}, {}, []
     for i, op in enumerate(ops):
-        sig = _op_sig(op)
+        sig = op.sig()
         out = op.out
         if sig is None or out is None:
             return None
         ins = []
         for u in op.inputs:
-            k = pos.get(u.id)
+            uid = u.id
+            k = pos.get(uid)
             if k is not None:
                 ins.append(k)
                 continue
-            l = leaf.get(u.id)
+            l = leaf.get(uid)
             if l is None:
-                l = leaf[u.id] = len(leaf)
-                ins.append((l, tuple(u.shape), u.dtype, u._op is None, u._buf is None, u._host is not None,
-                            getattr(u, "_stop_fuse", False)))
+                l = leaf[uid] = len(leaf)
+                ins.append((l, tuple(u.shape), u.dtype, u._op is None, u._buf is None, u._host is not None, u._stop_fuse))
             else:
                 ins.append(-1 - l)
-        pos[out.id] = i
-        parts.append((sig, tuple(out.shape), out.dtype, out.id in target_ids, out._buf is None, getattr(out, "_stop_fuse", False),
-                      tuple(ins)))
-    return (tuple(parts), tuple(sorted((k, str(v)) for k, v in flags.items())), dt_amp())
+        uid = out.id
+        pos[uid] = i
+        parts.append((sig, tuple(out.shape), out.dtype, uid in target_ids, out._buf is None, out._stop_fuse, tuple(ins)))
+    # (the flags are entered once and keep their order)
+    return (tuple(parts), tuple(map(str, flags.values())), dt_amp())
 
 
 def dt_amp():

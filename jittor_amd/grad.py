@@ -191,17 +191,23 @@ def grad(loss, targets, retain_graph=True):
         if v.id in nodes:
             continue
         nodes[v.id] = v
-        if v._history is not None:
-            stack.extend(v._history[1])
+        h = v._history
+        if h is not None:
+            for u in h[1]:
+                if u.id not in nodes:
+                    stack.append(u)
     # of those, the ones that depend on a target (ids grow from inputs to outputs)
     target_ids = {t.id for t in targets}
-    order = sorted(nodes.values(), key=lambda v: v.id)
+    order = [nodes[k] for k in sorted(nodes)]
     dep = set()
     for v in order:
         if v.id in target_ids:
             dep.add(v.id)
-        elif v._history is not None and any(u.id in dep for u in v._history[1]):
-            dep.add(v.id)
+        elif v._history is not None:
+            for u in v._history[1]:
+                if u.id in dep:
+                    dep.add(v.id)
+                    break
 
     grads = {}
     if loss.id in dep:
@@ -215,11 +221,15 @@ def grad(loss, targets, retain_graph=True):
             if u.id not in dep or not u.is_float():
                 continue
             saved = dt.amp_reg                                  # an op's gradient is built under the register
-            dt.amp_reg |= getattr(op, "amp", 0)                 # the op was created with (grad.cc:48-55)
-            try:
+            amp = saved | getattr(op, "amp", 0)                 # the op was created with (grad.cc:48-55)
+            if amp == saved:
                 du = _op_grad(op, inputs, v, g, i)
-            finally:
-                dt.amp_reg = saved
+            else:
+                dt.amp_reg = amp
+                try:
+                    du = _op_grad(op, inputs, v, g, i)
+                finally:
+                    dt.amp_reg = saved
             if du is None:
                 continue
             if du.shape != u.shape:
