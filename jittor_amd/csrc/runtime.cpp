@@ -39,10 +39,22 @@ struct Recording {
     std::vector<Launch> launches;
     std::vector<Patch> patches;
     uint64_t generation = 0;
+    uint64_t environment = 0;     // of the MJT_ variables, which choose routes, when it was made
     bool ready = false;           // mjt_record_relocate has found every word's origin
 };
 static thread_local Recording* t_recording = nullptr;
 static uint64_t g_generation = 1;         // guarded by the library's lock
+
+static uint64_t environment_now() {
+    uint64_t h = 1469598103934665603ull;
+    for (char** e = environ; e && *e; e++)
+        if (!strncmp(*e, "MJT_", 4))
+            for (const char* c = *e;; c++) {           // with the terminator: entries stay apart
+                h = (h ^ (unsigned char)*c) * 1099511628211ull;
+                if (!*c) break;
+            }
+    return h;
+}
 
 void refuse_recording(const char* what) {
     if (t_recording) MJT_FAIL(MJT_ERR_UNSUPPORTED, what << " cannot be part of a recording");
@@ -520,6 +532,7 @@ int mjt_record_begin(void) {
         MJT_CHECK(!t_recording, "mjt_record_begin: this thread is recording already");
         t_recording = new Recording();
         t_recording->generation = g_generation;
+        t_recording->environment = environment_now();
     });
 }
 int mjt_record_end(void** out) {
@@ -539,7 +552,7 @@ int mjt_record_relocate(void* first, void* second, int n_slots, const uint64_t* 
         Recording *a = (Recording*)first, *b = (Recording*)second;
         MJT_CHECK(a && b && !a->ready && n_slots >= 0 && n_scalars >= 0, "mjt_record_relocate: bad arguments");
         auto differ = [](const char* what) { MJT_FAIL(MJT_ERR_UNSUPPORTED, "mjt_record_relocate: the recordings differ in " << what); };
-        if (a->generation != g_generation || b->generation != g_generation || a->launches.size() != b->launches.size()) differ("their launches");
+        if (a->generation != g_generation || b->generation != g_generation || a->environment != b->environment || a->launches.size() != b->launches.size()) differ("their launches");
         for (size_t l = 0; l < a->launches.size(); l++) {
             const Launch &p = a->launches[l], &q = b->launches[l];
             if (p.kernel != q.kernel || p.gx != q.gx || p.gy != q.gy || p.gz != q.gz || p.block != q.block || p.shmem != q.shmem ||
@@ -567,7 +580,7 @@ int mjt_record_launch(void* rec, int n_slots, const uint64_t* bases, int n_scala
     return guarded([&] {
         Recording* r = (Recording*)rec;
         MJT_CHECK(r && r->ready, "mjt_record_launch: not a finished recording");
-        if (r->generation != g_generation) MJT_FAIL(MJT_ERR_UNSUPPORTED, "mjt_record_launch: the recording is out of date");
+        if (r->generation != g_generation || r->environment != environment_now()) MJT_FAIL(MJT_ERR_UNSUPPORTED, "mjt_record_launch: the recording is out of date");
         refuse_recording("mjt_record_launch");
         for (const Patch& p : r->patches) {
             MJT_CHECK(p.slot < (p.kind == 0 ? n_slots : n_scalars), "mjt_record_launch: too few slots or scalars");
