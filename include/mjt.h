@@ -344,12 +344,14 @@ int mjt_conv2d_meta_dgrad_depthwise(const mjt_tensor* dy, const mjt_tensor* w, c
  * opt/tuner/conv_tuner.cc:375-397 relays it to a backward-w library op,
  * extern/cuda/cudnn/ops/cudnn_conv_backward_w_op.cc):
  *   dw[k,c,r,s] = sum_{n,oh,ow} dy[n,k,oh,ow] * x[n,c,oh*sh-ph+r*dh,ow*sw-pw+s*dw]
- * x [N,C,H,W] and dy [N,K,OH,OW] bfloat16 or float16, dw [K,C,R,S] float32 or their dtype
- * (float32 accumulation, rounded once).  One MFMA kernel plus a reduce over
- * slices of images; shapes it does not cover (horizontal stride > 1, more
- * than 9 taps, left padding > 2, K % 64 != 0, an odd OW or W, a geometry whose
- * kernel would need more registers than a wave has, ...) return MJT_ERR_UNSUPPORTED
- * and are the caller's to run through mjt_matmul or mjt_conv2d_meta. */
+ * x [N,C,H,W] and dy [N,K,OH,OW] bfloat16, float16 or float32, dw [K,C,R,S] float32 or their
+ * dtype (float32 accumulation, rounded once).  16-bit operands run on an MFMA kernel of their
+ * own plus a reduce over slices of images, or as float32 ones on the product kernel, which
+ * gathers both operands, plus such a reduce (1x1 taps, narrow maps, and what the former does
+ * not cover: horizontal stride > 1, more than 9 taps, left padding > 2, K % 64 != 0, an
+ * odd OW or W, ...).  Fewer than 2^22 multiply-adds there, tensors of 2 GB and unaligned
+ * pointers return MJT_ERR_UNSUPPORTED and are the caller's to run through mjt_matmul
+ * or mjt_conv2d_meta. */
 int mjt_conv2d_meta_wgrad(const mjt_tensor* x, const mjt_tensor* dy, const mjt_tensor* dw,
                           const mjt_conv_params* p);
 

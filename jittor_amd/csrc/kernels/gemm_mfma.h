@@ -46,7 +46,8 @@
 //   dw[k][(c, r, s)] = sum over q = (image, oh, ow) of dy[image][k][oh][ow] * x[image][c][oh*SH-PH+r*DH][ow*SW-PW+s*DW]
 // A = dy with rows k, B' = the shifted planes of x with columns (c, r, s), both with the summed index q innermost, gathered on their
 // way to LDS: a lane owns one chunk of EPC pixels per stage and works out their image, row and column once for all rows and
-// columns it loads; a chunk of dy is one 16-byte load where a plane is whole chunks, x is loaded by elements.  The sum over q is cut into slices of a[9] stages; the slices' float32 partial
+// columns it loads; dy is loaded in the widest pieces that a plane consists of, as is x
+// for taps of 1 x 1 without stride and padding; otherwise x is loaded by elements.  The sum over q is cut into slices of a[9] stages; the slices' float32 partial
 // results are added up by a reduce launch.  Before, the shifted planes were written to memory, multiplied image by image
 // and the images' results added (float32 32 x 3 x 224 x 224, 7x7 stride 2 -> 64: 110 + 337 + 9 us; 116 here).
 //
@@ -304,54 +305,78 @@ constexpr int P_ = OH_ * OW_;
 // The pixels of the lane's chunk of a stage (chunk tid % KC), the same for all rows and columns that it loads.  All loads go
 // through buffer descriptors, unconditionally: what lies outside the image or past the sum gets an offset past the buffer's
 // end and reads zero, so nothing has to be looked at before it is written to LDS.
+constexpr int PU = P_ % EPC == 0 ? EPC : P_ % 4 == 0 ? 4 : P_ % 2 == 0 ? 2 : 1;     // pixels of a plane that one load takes
+constexpr int NL = EPC / PU;
+#define XPLANE (R_ * S_ == 1 && SH == 1 && SW == 1 && PH == 0 && PW == 0)             /* x is read in planes, as dy is */
 struct mjt_wg_chunk {
-    static constexpr int NDY = P_ % EPC == 0 ? 1 : EPC;
-    unsigned dy[NDY];                // byte offset of dy[image][0][pixel], or MJT_NONE
-    unsigned x[EPC];                 // byte offset of x[image][0][oh*SH-PH][ow*SW-PW] (may wrap below zero)
+    unsigned dy[NL];                 // byte offsets of dy[image][0][pixel], or MJT_NONE
+    unsigned x[EPC];                 // byte offset of x[image][0][oh*SH-PH][ow*SW-PW] (may wrap below zero); XPLANE: as dy
     unsigned hw[EPC];                // that row and column, both biased by 0x4000; 0 for a pixel past the sum
     __device__ __forceinline__ void at(int k0, int K, int tid) {
         const int q = k0 + (tid % KC) * EPC;
         mjt_static_for<0, EPC>([&](auto ec) {
             constexpr int e = decltype(ec)::v;
             constexpr bool decode = OW_ % EPC != 0 || e == 0;          // a row of outputs is whole chunks: neighbours of the first
-            if constexpr (decode || (NDY > 1 && e < NDY)) {
+            if constexpr (e % PU == 0) {
+                const int qe = q + e, img = qe / P_, px = qe - img * P_;
+                dy[e / PU] = qe < K ? (unsigned)(img * (K_ * P_) + px) * ESZ : MJT_NONE;
+                if constexpr (XPLANE) x[e / PU] = qe < K ? (unsigned)(img * (C_ * P_) + px) * ESZ : MJT_NONE;
+            }
+            if constexpr (!XPLANE && decode) {
                 const int qe = q + e;
                 const int img = qe / P_, px = qe - img * P_;
-                if constexpr (e < NDY) dy[e] = qe < K ? (unsigned)(img * (K_ * P_) + px) * ESZ : MJT_NONE;
                 const int oh = px / OW_, ow = px - oh * OW_;
                 const int ih = oh * SH - PH, iw = ow * SW - PW;
                 x[e] = (unsigned)((img * C_ * H_ + ih) * W_ + iw) * ESZ;
                 hw[e] = qe < K ? ((unsigned)(ih + 0x4000) << 16) | (unsigned)(iw + 0x4000) : 0u;
-            } else {
+            } else if constexpr (!XPLANE) {
                 x[e] = x[0] + e * SW * ESZ;
                 hw[e] = hw[0] + e * SW;                                // (0 + e * SW stays far below the bias)
             }
         });
     }
 };
-struct mjt_wg_dy {
-    static constexpr int PER = TM * KC / NTHR;
+// An operand read in planes: the lane's chunk of PER channels, NL loads of PU pixels each.  A load's pixels lie in one plane (PU
+// divides the planes) at an address that is a multiple of its size.
+template <int ROWS> struct mjt_wg_plane {
+    static constexpr int PER = ROWS * KC / NTHR;
     mjt_u32x4v reg[PER];
-    unsigned row[PER];               // byte offset of the lane's rows inside an image of dy
-    __device__ __forceinline__ void init(int m0, int M, int tid) {
+    unsigned row[PER];               // byte offset of the lane's channels inside an image
+    __device__ __forceinline__ void init(int r0, int rmax, int tid) {
         mjt_static_for<0, PER>([&](auto ic) {
-            const int r = m0 + tid / KC + decltype(ic)::v * (NTHR / KC);
-            row[decltype(ic)::v] = (unsigned)((r < M ? r : M - 1) * P_) * ESZ;
+            const int r = r0 + tid / KC + decltype(ic)::v * (NTHR / KC);
+            row[decltype(ic)::v] = (unsigned)((r < rmax ? r : rmax - 1) * P_) * ESZ;
         });
     }
-    template <int I> __device__ __forceinline__ void fetch(__amdgpu_buffer_rsrc_t d, const mjt_wg_chunk& ch) {
-        if constexpr (mjt_wg_chunk::NDY == 1) {
-            reg[I] = __builtin_amdgcn_raw_buffer_load_b128(d, (int)((ch.dy[0] + row[I]) | (ch.dy[0] & MJT_NONE)), 0, 0);
-        } else {
+    template <int I> __device__ __forceinline__ void fetch(__amdgpu_buffer_rsrc_t d, const unsigned* at) {
+        if constexpr (PU * ESZ == 2) {
             unsigned v[EPC];
-            mjt_static_for<0, EPC>([&](auto ec) { constexpr int e = decltype(ec)::v; v[e] = mjt_wg_load(d, (ch.dy[e] + row[I]) | (ch.dy[e] & MJT_NONE)); });
+            mjt_static_for<0, EPC>([&](auto ec) { constexpr int e = decltype(ec)::v; v[e] = mjt_wg_load(d, (at[e] + row[I]) | (at[e] & MJT_NONE)); });
             reg[I] = mjt_wg_pack(v);
+        } else {
+            mjt_static_for<0, NL>([&](auto gc) {
+                constexpr int g = decltype(gc)::v;
+                const int off = (int)((at[g] + row[I]) | (at[g] & MJT_NONE));
+                if constexpr (PU * ESZ == 16) {
+                    reg[I] = __builtin_amdgcn_raw_buffer_load_b128(d, off, 0, 0);
+                } else if constexpr (PU * ESZ == 8) {
+                    const auto two = __builtin_amdgcn_raw_buffer_load_b64(d, off, 0, 0);
+                    reg[I][2 * g] = two[0];
+                    reg[I][2 * g + 1] = two[1];
+                } else {
+                    reg[I][g] = __builtin_amdgcn_raw_buffer_load_b32(d, off, 0, 0);
+                }
+            });
         }
     }
     template <int I> __device__ __forceinline__ void commit(unsigned char* lds, int tid) const {
         *(mjt_u32x4v*)(lds + (tid / KC + I * (NTHR / KC)) * ROWB + (tid % KC) * 16) = reg[I];
     }
 };
+typedef mjt_wg_plane<TM> mjt_wg_dy;
+#if XPLANE
+typedef mjt_wg_plane<TN> mjt_wg_x;
+#else
 struct mjt_wg_x {
     static constexpr int PER = TN * KC / NTHR;
     unsigned v[PER][EPC];
@@ -378,6 +403,7 @@ struct mjt_wg_x {
         *(mjt_u32x4v*)(lds + (tid / KC + I * (NTHR / KC)) * ROWB + (tid % KC) * 16) = mjt_wg_pack(v[I]);
     }
 };
+#endif
 #endif
 
 extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
@@ -455,8 +481,12 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
     auto fetch = [&](auto ic, auto setc, auto, int stage) {
         constexpr int I = decltype(ic)::v, SET = decltype(setc)::v;
         if constexpr (I == 0) ch.at((first_stage + stage) * KS, K, tid);
-        if constexpr (I < PA) sa[SET].template fetch<I>(dy_rsrc, ch);
+        if constexpr (I < PA) sa[SET].template fetch<I>(dy_rsrc, ch.dy);
+#if XPLANE
+        else sb[SET].template fetch<I - PA>(x_rsrc, ch.x);
+#else
         else sb[SET].template fetch<I - PA>(x_rsrc, ch);
+#endif
     };
     auto commit = [&](auto ic, auto setc, auto, int stage) {
         constexpr int I = decltype(ic)::v, SET = decltype(setc)::v;

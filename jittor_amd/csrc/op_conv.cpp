@@ -728,32 +728,55 @@ static bool conv_wgrad_product(const mjt_tensor* x, const mjt_tensor* dy, const 
     const int64_t N = x->shape[0], C = x->shape[1], H = x->shape[2], W = x->shape[3];
     const int64_t K = dy->shape[1], OH = dy->shape[2], OW = dy->shape[3], R = dw->shape[2], S = dw->shape[3];
     const int64_t P = OH * OW, CRS = C * R * S, Q = N * P;
-    if (x->dtype != MJT_FLOAT32 || dy->dtype != x->dtype || dw->dtype != MJT_FLOAT32 || getenv("MJT_NO_FASTPATH") || getenv("MJT_CONV_NO_IGEMM")) return false;
-    // (offsets inside x and dy are 32-bit elements, rows and columns 14-bit; a few million multiply-adds are worth the set-up)
+    const bool half = x->dtype == MJT_FLOAT16 || x->dtype == MJT_BFLOAT16;
+    if (!(x->dtype == MJT_FLOAT32 || half) || dy->dtype != x->dtype || !(dw->dtype == MJT_FLOAT32 || dw->dtype == x->dtype) || getenv("MJT_NO_FASTPATH") || getenv("MJT_CONV_NO_IGEMM")) return false;
+    const int64_t esz = dtype_size(x->dtype);
+    // (offsets inside x and dy are 31-bit bytes, rows and columns 14-bit; a few million multiply-adds are worth the set-up)
     if ((double)Q * K * CRS < (double)(1 << 22) || Q >= (int64_t(1) << 31) - 64 ||
-        numel(x) * 4 >= (int64_t(1) << 31) || numel(dy) * 4 >= (int64_t(1) << 31) || H >= 16384 || W >= 16384 || (R - 1) * p->dil_h >= 16384 || (S - 1) * p->dil_w >= 16384 || p->pad_h >= 16384 || p->pad_w >= 16384 ||
-        OH * p->stride_h >= 16384 || OW * p->stride_w >= 16384 || (uintptr_t)dy->ptr % 16)
+        numel(x) * esz >= (int64_t(1) << 31) || numel(dy) * esz >= (int64_t(1) << 31) || H >= 16384 || W >= 16384 || (R - 1) * p->dil_h >= 16384 || (S - 1) * p->dil_w >= 16384 || p->pad_h >= 16384 || p->pad_w >= 16384 ||
+        OH * p->stride_h >= 16384 || OW * p->stride_w >= 16384 || (uintptr_t)dy->ptr % 16 || (uintptr_t)x->ptr % 16)
         return false;
     const int64_t cus = ctx().dry_run || ctx().prop.multiProcessorCount <= 0 ? 256 : ctx().prop.multiProcessorCount;
-    const int in = 2, KS = 32;
+    const int in = x->dtype == MJT_BFLOAT16 ? 0 : half ? 1 : 2;
+    const int64_t KS = half ? 64 : 32;
     // 128 x 128 tiles gather half as much per multiply-add and hold two workgroups a compute unit, 64 x 64 tiles waste less on
     // the edges and hold four (us at 3x3, 64 / 128: 64 x 64 x 56 x 56 -> 64: 162 / 447; 64 x 128 x 28 x 28 -> 128: 161 / 155;
     // 64 x 256 x 14 x 14 -> 256: 180 / 150; 64 x 512 x 7 x 7 -> 512: 195 / 176)
     auto tiles_of = [&](int64_t t) { return ((K + t - 1) / t) * ((CRS + t - 1) / t); };
-    const int MI = tiles_of(128) * 4 * 0.85 <= (double)tiles_of(64) ? 2 : 1, NI = MI;
-    const int64_t tiles = tiles_of(64 * MI);
-    // slices of the sum: one, two or three full rounds of workgroups, whichever leaves fewest places empty, of at least 8 stages
-    // each (one workgroup more than a round costs a round: 64 x 256 x 14 x 14 -> 256 in 14 slices 150, in 15 slices 212)
-    const int64_t stages = (Q + KS - 1) / KS, places = cus * (MI == 1 ? 4 : 2);
+    int MI = tiles_of(128) * 4 * 0.85 <= (double)tiles_of(64) ? 2 : 1;
+    // slices of the sum, float32: one, two or three full rounds of workgroups, whichever leaves fewest places empty, of at least 8
+    // stages each (one workgroup more than a round costs a round: 64 x 256 x 14 x 14 -> 256 in 14 slices 150, in 15 slices 212)
+    const int64_t stages = (Q + KS - 1) / KS;
     int64_t slices = 1;
-    double best = 0.0;
-    for (int64_t r = 1; r <= 3; r++) {
-        int64_t n = r * places / tiles;
-        if (n > stages / 8) n = stages / 8;
-        if (n < 1) n = 1;
-        const double wgs = (double)(n * tiles), full = wgs / (std::ceil(wgs / places) * places);
-        if (full > best + 0.05) { best = full; slices = n; }
+    if (!half) {
+        const int64_t places = cus * (MI == 1 ? 4 : 2);
+        double best = 0.0;
+        for (int64_t r = 1; r <= 3; r++) {
+            int64_t n = r * places / tiles_of(64 * MI);
+            if (n > stages / 8) n = stages / 8;
+            if (n < 1) n = 1;
+            const double wgs = (double)(n * tiles_of(64 * MI)), full = wgs / (std::ceil(wgs / places) * places);
+            if (full > best + 0.05) { best = full; slices = n; }
+        }
+    } else {
+        // 16 bits: the loads bound a stage, 0.045 us for each that a thread issues on 128 x 128 tiles (four chunks of each operand)
+        // and 0.05 on 64 x 64 (two), 0.7 and 0.37 at least; a further workgroup on a compute unit adds 0.7 of that time, folding the
+        // slices 5 us and their traffic.  us at 64 images, tile / slices as found here, and others: 1024 x 14 x 14 1x1 -> 256
+        // 128 / 16 21.7 (64 / 4 24.8, 128 / 8 26.7, 128 / 48 32.1); 256 x 14 x 14 3x3 -> 256 128 / 14 60.7 (128 / 4 90.5, 64 / 12
+        // 96.5); 256 x 28 x 28 1x1 -> 128 64 / 32 16.5 (128 / 64 20.3).
+        const bool planes = R * S == 1 && p->stride_h == 1 && p->stride_w == 1 && p->pad_h == 0 && p->pad_w == 0;
+        const int nl = P % 8 == 0 ? 1 : P % 4 == 0 ? 2 : P % 2 == 0 ? 4 : 8, loads = nl + (planes ? nl : 8);
+        double least = 1e30;
+        for (int mi = 1; mi <= 2; mi++)
+            for (int64_t n = 1; n <= 64 && (n == 1 || n <= stages / 4); n++) {
+                const int64_t pn = (stages + n - 1) / n, nn = (stages + pn - 1) / pn;
+                const double st = mi == 2 ? std::max(0.7, 0.045 * 4 * loads) : std::max(0.37, 0.05 * 2 * loads);
+                const double t = (double)pn * st * (1.0 + 0.7 * (std::ceil((double)(nn * tiles_of(64 * mi)) / cus) - 1.0)) + 5.0 + (double)nn * numel(dw) * 8 / 5e6;
+                if (t < least) { least = t; MI = mi; slices = nn; }
+            }
     }
+    const int NI = MI;
+    const int64_t tiles = tiles_of(64 * MI);
     if (slices * numel(dw) * 4 > (int64_t(1) << 30)) return false;
     const int64_t per = (stages + slices - 1) / slices;
     slices = (stages + per - 1) / per;
@@ -777,7 +800,7 @@ static bool conv_wgrad_product(const mjt_tensor* x, const mjt_tensor* dy, const 
     const bool in_place = slices == 1 && dw->dtype == MJT_FLOAT32;
     void* part = in_place ? dw->ptr : wgrad_partials((size_t)slices * (size_t)numel(dw) * 4);
     std::vector<uint64_t> a{bits_of_ptr(dy->ptr), bits_of_ptr(x->ptr), bits_of_ptr(part), (uint64_t)K, (uint64_t)CRS, (uint64_t)Q, 0, 0, (uint64_t)CRS, (uint64_t)per,
-                            (uint64_t)(numel(x) * 4), (uint64_t)(K * CRS)};
+                            (uint64_t)(numel(x) * esz), (uint64_t)(K * CRS)};
     const int64_t grid = (slices * tiles + 7) / 8 * 8;
     MJT_CHECK(grid < (int64_t(1) << 31), "conv wgrad: launch too large");
     jit_launch(k, (unsigned)grid, 1, 256, 0, a);
@@ -820,7 +843,14 @@ void conv_wgrad_impl(const mjt_tensor* x, const mjt_tensor* dy, const mjt_tensor
                     W % 2 == 0 && N >= 1 && numel(x) * 2 < (int64_t(1) << 31) && numel(dy) * 2 < (int64_t(1) << 31) &&
                     (uintptr_t)x->ptr % 4 == 0 && (uintptr_t)dy->ptr % 16 == 0 &&
                     !getenv("MJT_NO_FASTPATH");
-    if (!ok && G == 1 && N >= 1 && conv_wgrad_product(x, dy, dw, p)) return;
+    // 16-bit operands: the product instead of the MFMA kernel for 1x1 taps without stride and padding, whose operands it reads as they
+    // lie, and for maps that fill less than 0.6 of the kernel's chunks of 32 columns (us at 64 images, kernel / product:
+    // 1024 x 14 x 14 1x1 -> 256 65.9 / 21.7; 256 x 28 x 28 1x1 -> 128 25.5 / 16.5; 256 x 14 x 14 3x3 -> 256 70.6 / 60.7;
+    // 128 x 28 x 28 3x3 -> 128 54.8 / 62.0 stays), from 2^27 multiply-adds on: below, either is a few us.
+    const bool narrow = OW % 8 != 0 && (double)OW < 0.6 * 32 * (double)((OW + 31) / 32);
+    const bool planes = R * S == 1 && p->stride_h == 1 && p->stride_w == 1 && p->pad_h == 0 && p->pad_w == 0;
+    const bool large = (double)N * OH * OW * K * C * R * S >= (double)(1 << 27);
+    if ((!ok || (OH * OW % 2 == 0 && (planes || narrow) && large)) && G == 1 && N >= 1 && conv_wgrad_product(x, dy, dw, p)) return;
     if (!ok && any_shape) {
         conv_wgrad_direct(x, dy, dw, p, G);
         return;

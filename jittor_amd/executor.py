@@ -1200,12 +1200,13 @@ def _run_single(op):
         N, C, H, W = x.shape
         _, K, OH, OW = dy.shape
         R, S = out.shape[2], out.shape[3]
-        # (the kernel walks rows in chunks of 32 output columns: a width that fills less than 0.6 of its chunks and is no
-        # multiple of 8 is better off as a product, 64 x 256 x 14 x 14 3x3: 68 us on the kernel, 59 as the product below)
-        narrow = OW % 8 != 0 and OW < 0.6 * 32 * -(-OW // 32)
+        # 16-bit maps of an odd number of pixels, narrower than 0.6 of the kernel's chunks of 32 columns, are better off as the product
+        # over chunks of images below where the images make chunks (64 x 512 x 7 x 7 3x3: 61 us, 88 as the product that gathers
+        # its operands by elements); those of an even number go to the latter (64 x 256 x 14 x 14 3x3: 63 and 61, 1x1: 60 and 22)
         half = x.dtype in ("bfloat16", "float16")
-        if (half and not narrow or x.dtype == "float32") and flags["enable_conv_wgrad_kernel"]:
-            # 16-bit: the MFMA kernel; float32: the product that gathers its operands; shapes they do not cover come back as
+        chunked = half and OH * OW % 2 == 1 and N % 8 == 0 and OW < 0.6 * 32 * -(-OW // 32)
+        if (half or x.dtype == "float32") and not chunked and flags["enable_conv_wgrad_kernel"]:
+            # the MFMA kernel (16 bits) or the product that gathers its operands; shapes they do not cover come back as
             # unsupported and take the paths below
             tx, td = _tensor_of(x), _tensor_of(dy)
             tw = _tensor(_alloc_out(out), out.dtype, out.shape)

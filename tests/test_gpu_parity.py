@@ -1813,3 +1813,51 @@ def test_depthwise_conv_and_gradients(gpu, case):
     for name, v, ref, mag, terms in checks:
         got = widen[out](L.d2h(v.raw_ptr(), v.shape, L.NP_STORAGE[out]))
         assert np.all(np.abs(got - ref) <= terms * 2.0 ** -24 * mag + eps * np.abs(ref) + 2.0 ** -24 * (out == "float16")), name
+
+
+@pytest.mark.parametrize("case", [
+    dict(x=(8, 64, 14, 14), k=96, rs=(1, 1), p=(1, 1, 0, 0, 1, 1)),        # planes of 196 pixels: pieces of four, chunks that span images
+    dict(x=(14, 72, 6, 7), k=136, rs=(1, 1), p=(1, 1, 0, 0, 1, 1)),         # 42 pixels: pairs
+    dict(x=(15, 64, 9, 7), k=80, rs=(1, 1), p=(1, 1, 0, 0, 1, 1)),         # 63 pixels: single ones
+    dict(x=(5, 40, 16, 16), k=200, rs=(1, 1), p=(1, 1, 0, 0, 1, 1)),       # whole chunks
+    dict(x=(7, 40, 15, 13), k=72, rs=(3, 3), p=(2, 2, 1, 1, 1, 1)),        # stride 2, 8 x 7 maps
+    dict(x=(6, 33, 12, 10), k=70, rs=(3, 2), p=(1, 1, 1, 0, 1, 2)),        # dilation, ragged channels
+    dict(x=(4, 24, 31, 17), k=66, rs=(5, 5), p=(2, 1, 2, 2, 1, 1)),
+])
+@pytest.mark.parametrize("dt", ["bfloat16", "float16"])
+def test_conv_wgrad_product_16_bit(gpu, dt, case):
+    """The weight gradient of 16-bit operands as a product that gathers its operands.  Products are exact and sums float32: 1e-4 of
+    the sums of magnitudes, and one rounding (or truncation) for a result of 16 bits."""
+    rng = np.random.default_rng(91)
+    N, C, H, W = case["x"]
+    K, (R, S) = case["k"], case["rs"]
+    sh, sw, ph, pw, dh, dw_ = case["p"]
+    OH, OW = (H + 2 * ph - dh * (R - 1) - 1) // sh + 1, (W + 2 * pw - dw_ * (S - 1) - 1) // sw + 1
+
+    def operand(shape):
+        v = rng.standard_normal(shape).astype(np.float32)
+        if dt == "float16":
+            h = v.astype(np.float16)
+            return jt.from_storage(h, dt), h.astype(np.float64)
+        bits = (v.view(np.uint32) >> 16).astype(np.uint16)
+        return jt.from_storage(bits, dt), (bits.astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+
+    x, xf = operand((N, C, H, W))
+    dy, df = operand((N, K, OH, OW))
+    xp = np.pad(xf, ((0, 0), (0, 0), (ph, ph), (pw, pw)))
+    want, mag = np.zeros((K, C, R, S)), np.zeros((K, C, R, S))
+    for r in range(R):
+        for s in range(S):
+            patch = xp[:, :, r * dh:r * dh + (OH - 1) * sh + 1:sh, s * dw_:s * dw_ + (OW - 1) * sw + 1:sw]
+            want[:, :, r, s] = np.einsum("nkhw,nchw->kc", df, patch)
+            mag[:, :, r, s] = np.einsum("nkhw,nchw->kc", np.abs(df), np.abs(patch))
+    for odt in ("float32", dt):
+        out = jt.from_storage(np.zeros((K, C, R, S), L.NP_STORAGE[odt]), odt)
+        p = L.ConvParams(*case["p"])
+        tx, td, tw = (L.tensor(v.raw_ptr(), v.dtype, v.shape) for v in (x, dy, out))
+        rc = L.load().mjt_conv2d_meta_wgrad(ctypes.byref(tx), ctypes.byref(td), ctypes.byref(tw), ctypes.byref(p))
+        assert rc == 0 and L.last_kernel().startswith("mjt_conv_wgrad_igemm_"), L.last_kernel()
+        got = L.d2h(out.raw_ptr(), out.shape, L.NP_STORAGE[odt])
+        got = (got.astype(np.uint32) << 16).view(np.float32).astype(np.float64) if odt == "bfloat16" else got.astype(np.float64)
+        bound = 1e-4 * mag + (np.abs(want) * 2.0 ** -7 if odt == "bfloat16" else np.abs(want) * 2.0 ** -10 if odt == "float16" else 0)
+        assert (np.abs(got - want) <= bound).all(), float(np.abs(got - want).max())
