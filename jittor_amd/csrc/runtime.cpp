@@ -551,6 +551,8 @@ int mjt_record_relocate(void* first, void* second, int n_slots, const uint64_t* 
     return guarded([&] {
         Recording *a = (Recording*)first, *b = (Recording*)second;
         MJT_CHECK(a && b && !a->ready && n_slots >= 0 && n_scalars >= 0, "mjt_record_relocate: bad arguments");
+        for (int k = 0; k < n_slots; k++)                     // a slot whose address is the same in both would be taken for a constant
+            MJT_CHECK(base1[k] != base2[k], "mjt_record_relocate: slot " << k << " has one address in both recordings");
         auto differ = [](const char* what) { MJT_FAIL(MJT_ERR_UNSUPPORTED, "mjt_record_relocate: the recordings differ in " << what); };
         if (a->generation != g_generation || b->generation != g_generation || a->environment != b->environment || a->launches.size() != b->launches.size()) differ("their launches");
         for (size_t l = 0; l < a->launches.size(); l++) {

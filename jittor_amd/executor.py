@@ -648,7 +648,9 @@ def _record(plan):
     recs, sets = [], []
     try:
         for run in (1, 2):
-            base = [(run << 45) + _SPAN * (k if run == 1 else n - k) for k in range(n)]
+            # the second set lies behind the whole first one (no slot has one address in both, however many there are) and runs the
+            # other way round (an address worked out past a slot's end is not taken for its neighbour's)
+            base = [(1 << 45) + _SPAN * (k if run == 1 else 2 * n - k) for k in range(n)]
             vals = [run * 1000003 + k for k in range(ns)]
             _fill_in(plan, base, [(float(v), v) for v in vals])
             _lib.check(lib.mjt_record_begin())

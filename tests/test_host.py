@@ -816,9 +816,47 @@ def test_recorded_launches(compile_only, monkeypatch):
         rec = ctypes.c_void_p()
         L.check(lib.mjt_record_end(ctypes.byref(rec)))
         recs.append(rec)
-    b = (ctypes.c_uint64 * 2)(1 << 45, 1 << 46)
+    b, b2 = (ctypes.c_uint64 * 2)(1 << 45, 1 << 46), (ctypes.c_uint64 * 2)(1 << 47, 1 << 48)
     none = (ctypes.c_int64 * 1)()
-    assert lib.mjt_record_relocate(recs[0], recs[1], 2, b, b, 1 << 36, 0, none, none) == L.ERR_UNSUPPORTED
+    assert lib.mjt_record_relocate(recs[0], recs[1], 2, b, b, 1 << 36, 0, none, none) not in (0, L.ERR_UNSUPPORTED)   # one address in both
+    assert lib.mjt_record_relocate(recs[0], recs[1], 2, b, b2, 1 << 36, 0, none, none) == L.ERR_UNSUPPORTED
     assert lib.mjt_record_launch(recs[0], 2, b, 0, None, none) < 0
     for rec in recs:
         lib.mjt_record_free(rec)
+
+
+@pytest.mark.parametrize("pairs", [1, 170, 171, 172, 400])
+def test_recorded_launches_tell_all_buffers_apart(compile_only, monkeypatch, pairs):
+    """The two sets of stand-in addresses share none, also where a graph has more buffers (3 per pair) than fit between two
+    powers of two: a buffer with one address in both would be recorded as a constant."""
+    from jittor_amd import core, executor
+    nxt = [0x10000000]
+
+    def fake_alloc(nbytes):
+        size = core._Pool._round(nbytes)
+        nxt[0] += size
+        return nxt[0] - size, size
+
+    monkeypatch.setattr(core.pool, "alloc", fake_alloc)
+    monkeypatch.setattr(core.pool, "free", lambda ptr, size: None)
+    monkeypatch.setattr(L, "h2d", lambda ptr, arr: None)
+    monkeypatch.setitem(executor.flags, "enable_replay", True)
+    executor._plans.clear()
+    lib, sets = L.ensure_init(), []
+
+    class Library:
+        def __getattr__(self, name):
+            return getattr(lib, name)
+
+        def mjt_record_relocate(self, first, second, n, b1, b2, *rest):
+            sets.append((list(b1), list(b2)))
+            return lib.mjt_record_relocate(first, second, n, b1, b2, *rest)
+
+    monkeypatch.setattr(L, "ensure_init", lambda: Library())
+    before = executor.stats["recorded_launches"]
+    for _ in range(3):
+        keep = [(jt.array(np.ones((4, 4 + k % 2), np.float32)), jt.array(np.ones((4, 4 + k % 2), np.float32))) for k in range(pairs)]
+        jt.sync([(a * b).sum([1]) for a, b in keep])
+    assert executor.stats["recorded_launches"] == before + 1
+    (b1, b2), = sets
+    assert len(b1) >= 3 * pairs and len(set(b1 + b2)) == 2 * len(b1)
