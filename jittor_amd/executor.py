@@ -1202,11 +1202,13 @@ def _run_single(op):
         N, C, H, W = x.shape
         _, K, OH, OW = dy.shape
         R, S = out.shape[2], out.shape[3]
-        # 16-bit maps of an odd number of pixels, narrower than 0.6 of the kernel's chunks of 32 columns, are better off as the product
-        # over chunks of images below where the images make chunks (64 x 512 x 7 x 7 3x3: 61 us, 88 as the product that gathers
-        # its operands by elements); those of an even number go to the latter (64 x 256 x 14 x 14 3x3: 63 and 61, 1x1: 60 and 22)
+        # 16-bit maps narrower than 0.6 of the kernel's chunks of 32 columns: the product over chunks of images below for an odd number
+        # of pixels where the images make chunks (64 x 512 x 7 x 7 3x3: 61 us, 88 as the product that gathers its operands by elements)
+        # and below 2^27 multiply-adds, where either takes a few us; the gathering product for the others (64 x 256 x 14 x 14
+        # 3x3: 63 and 61, 1x1: 60 and 22)
         half = x.dtype in ("bfloat16", "float16")
-        chunked = half and OH * OW % 2 == 1 and N % 8 == 0 and OW < 0.6 * 32 * -(-OW // 32)
+        narrow = OW % 8 != 0 and OW < 0.6 * 32 * -(-OW // 32)
+        chunked = half and narrow and (OH * OW % 2 == 1 and N % 8 == 0 or N * OH * OW * K * C * R * S < 1 << 27)
         if (half or x.dtype == "float32") and not chunked and flags["enable_conv_wgrad_kernel"]:
             # the MFMA kernel (16 bits) or the product that gathers its operands; shapes they do not cover come back as
             # unsupported and take the paths below
@@ -1215,7 +1217,7 @@ def _run_single(op):
             p = _lib.ConvParams(sh, sw, ph, pw, dh, dw)
             rc = lib.mjt_conv2d_meta_wgrad(ctypes.byref(tx), ctypes.byref(td), ctypes.byref(tw), ctypes.byref(p))
             if rc == 0:
-                stats["wgrad_kernel"] += half
+                stats["wgrad_kernel"] += _lib.last_kernel().startswith("mjt_conv_wgrad_mfma")
                 return
             if rc != _lib.ERR_UNSUPPORTED:
                 _lib.check(rc)
