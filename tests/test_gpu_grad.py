@@ -478,3 +478,36 @@ def test_grad_conv_weight_float32_gathered_product(gpu, xs, k, rs, stride, pad, 
             p2 = patch.transpose(0, 2, 3, 1).reshape(-1, C)
             bound = N * OH * OW * 2.0 ** -24 * (np.abs(d2) @ np.abs(p2))
             assert np.all(np.abs(got[:, :, r, s] - d2 @ p2) <= bound), (r, s)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("k,s,p,hw", [
+    ((3, 3), (2, 2), (1, 1), (12, 16)),                                # several elements a lane, windows shared by two of them
+    ((3, 3), (1, 1), (1, 1), (5, 8)),                                  # every window reaches three elements of a lane
+    ((2, 2), (3, 3), (0, 0), (9, 12)),                                 # elements that no window reaches
+    ((2, 7), (1, 2), (1, 3), (4, 24)),                                 # windows wider than a lane's elements
+    ((3, 2), (2, 3), (1, 0), (7, 9)),                                  # rows that are no whole vectors
+    ((3, 3), (2, 2), (1, 1), (3, 4)),                                  # one vector a row
+])
+def test_max_pooling_gradient_of_windows_shared_by_a_lane(gpu, k, s, p, hw, dtype):
+    """The windows that reach a lane's elements, of every overlap and at every edge, against numpy.  Whole numbers up to 8 in x and
+    dy: sums of at most 21 of them are exact in float32 and in bfloat16."""
+    rng = np.random.default_rng(71)
+    (kh, kw), (sh, sw), (ph, pw), (H, W) = k, s, p, hw
+    OH, OW = (H + 2 * ph - kh) // sh + 1, (W + 2 * pw - kw) // sw + 1
+    x = rng.integers(1, 9, (2, 3, H, W)).astype(np.float32)
+    dy = rng.integers(1, 5, (2, 3, OH, OW)).astype(np.float32)
+    xp, dp = np.pad(x, ((0, 0), (0, 0), (ph, ph), (pw, pw))), np.zeros((2, 3, H + 2 * ph, W + 2 * pw), np.float32)
+    for i in range(OH):
+        for j in range(OW):
+            win = xp[:, :, i * sh:i * sh + kh, j * sw:j * sw + kw]
+            top = win == win.max((2, 3), keepdims=True)                # equal elements all receive the gradient
+            dp[:, :, i * sh:i * sh + kh, j * sw:j * sw + kw] += top * dy[:, :, i:i + 1, j:j + 1]
+    want = dp[:, :, ph:ph + H, pw:pw + W]
+    vx, vd = (jt.array(a).cast(dtype) for a in (x, dy))
+    y = jt.pool(vx, k, "maximum", p, s)
+    g = jt.grad((y * vd).sum(), vx)
+    before = jt.executor_stats["fused_scatters"]
+    jt.sync([y, g])
+    assert jt.executor_stats["fused_scatters"] == before + 1
+    assert np.array_equal(g.cast("float32").numpy(), want)
