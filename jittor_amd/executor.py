@@ -10,6 +10,7 @@ once.  Everything runs on the device; there is no host path.
 """
 import ctypes
 import math
+import threading
 
 from . import _lib
 from . import core
@@ -736,23 +737,29 @@ def _replay(plan, ops):
     stats["replays"] += 1
 
 
+# Plans are shared by all threads: their descriptors are filled in for one execution at a time (and with stand-in addresses while
+# they are recorded), and a graph that is being captured notes every call made.
+_running = threading.RLock()
+
+
 def run_sync(targets, device_sync=False):
     targets = [t for t in targets if isinstance(t, Var)]
-    stats["syncs"] += 1
     _lib.ensure_init()
-    ops = _pending_ops(targets)
-    if ops:
-        target_ids = {t.id for t in targets}
-        sig = _signature(ops, target_ids) if flags["enable_replay"] and _cap is None and _profiler.active() is None else None
-        plan = _plans.get(sig) if sig is not None else False
-        if plan is None:
-            _capture(ops, target_ids, sig)
-        elif plan is False:
-            _execute(ops, target_ids)
-        else:
-            _replay(plan, ops)
-    for t in targets:
-        t._device_ptr()
+    with _running:
+        stats["syncs"] += 1
+        ops = _pending_ops(targets)
+        if ops:
+            target_ids = {t.id for t in targets}
+            sig = _signature(ops, target_ids) if flags["enable_replay"] and _cap is None and _profiler.active() is None else None
+            plan = _plans.get(sig) if sig is not None else False
+            if plan is None:
+                _capture(ops, target_ids, sig)
+            elif plan is False:
+                _execute(ops, target_ids)
+            else:
+                _replay(plan, ops)
+        for t in targets:
+            t._device_ptr()
     if device_sync:
         _lib.sync()
 

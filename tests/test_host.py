@@ -860,3 +860,50 @@ def test_recorded_launches_tell_all_buffers_apart(compile_only, monkeypatch, pai
     assert executor.stats["recorded_launches"] == before + 1
     (b1, b2), = sets
     assert len(b1) >= 3 * pairs and len(set(b1 + b2)) == 2 * len(b1)
+
+
+def test_one_thread_at_a_time_executes_a_plan(compile_only, monkeypatch):
+    """A plan's descriptors, which hold stand-in addresses while its launches are recorded, belong to one execution at a time."""
+    import threading
+    import time
+    from jittor_amd import core, executor
+    nxt = [0x10000000]
+
+    def fake_alloc(nbytes):
+        size = core._Pool._round(nbytes)
+        nxt[0] += size
+        return nxt[0] - size, size
+
+    monkeypatch.setattr(core.pool, "alloc", fake_alloc)
+    monkeypatch.setattr(core.pool, "free", lambda ptr, size: None)
+    monkeypatch.setattr(L, "h2d", lambda ptr, arr: None)
+    monkeypatch.setitem(executor.flags, "enable_replay", True)
+    executor._plans.clear()
+    inside, met, failed = [], [], []
+    for name in ("_launch", "_record"):
+        def watched(*args, _f=getattr(executor, name)):
+            me = threading.get_ident()
+            met.extend(t for t in inside if t != me)
+            inside.append(me)
+            time.sleep(0.001)                                          # lets the others run
+            try:
+                return _f(*args)
+            finally:
+                inside.remove(me)
+        monkeypatch.setattr(executor, name, watched)
+
+    def work():
+        try:
+            for _ in range(5):
+                x = jt.array(np.ones((32, 24), np.float32))
+                jt.sync([(x * x).sum([1])])
+        except Exception as e:                                         # shown by the assertion below
+            failed.append(e)
+
+    work()                                                             # the plan is there
+    threads = [threading.Thread(target=work) for _ in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed and not met
