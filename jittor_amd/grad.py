@@ -18,32 +18,31 @@ from .core import (Var, UnaryOp, BinaryOp, TernaryOp, BroadcastOp, ReduceOp, Rei
 from . import _lib
 
 
-def _is_one(v):
-    """Is v a constant 1, spread and cast (the gradient that arrives below a sum of the loss)?"""
-    while v._op is not None:
-        if v._buf is not None or not (isinstance(v._op, BroadcastOp) or isinstance(v._op, UnaryOp) and v._op.op == "cast" and v.is_float()):
-            return False
-        v = v._op.inputs[0]
-    return v._host is not None and v.num == 1 and v.dtype in ("float32", "float64", "float16") and v._host.reshape(-1)[0] == 1 \
-        or v.dtype == "bfloat16" and v._host is not None and v.num == 1 and v._host.reshape(-1)[0] == 0x3f80
-
-
-def _times(factor, dout):
-    """factor * dout, which is `factor` itself where dout is a constant 1: the product would be a pass over memory that changes
-    nothing (the gradient of a 32 x 128 x 56 x 56 float32 result under (y * g).sum(): 19 us).  A factor that is spread or gathered
-    stays a product: it is how the operands of convolutions and matrix products appear, which are recognised by it."""
-    if _is_one(dout) and not isinstance(factor._op, (BroadcastOp, ReindexOp)) and dt.binary_dtype_infer("multiply", factor.dtype, dout.dtype, factor.is_scalar, dout.is_scalar) == factor.dtype:
+def _times(factor, dout, ones):
+    """factor * dout, which is `factor` itself where dout is the seed of this call, spread or cast: the product would be a pass over
+    memory that changes nothing (the gradient of a 32 x 128 x 56 x 56 float32 result under (y * g).sum(): 19 us).  `ones` holds the
+    ids of those Vars; a Var of the program's own that happens to hold a 1 is not among them, whatever its value, since a second
+    derivative may ask for it.  A factor that is spread or gathered stays a product: it is how the operands of convolutions and
+    matrix products appear, which are recognised by it."""
+    if dout.id in ones and not isinstance(factor._op, (BroadcastOp, ReindexOp)) and dt.binary_dtype_infer("multiply", factor.dtype, dout.dtype, factor.is_scalar, dout.is_scalar) == factor.dtype:
         return factor
     return binary(factor, dout, "multiply")
 
 
-def _unary_grad(op, x, y, dout):
+def _still_one(v, dout, ones):
+    """v is dout, spread or cast."""
+    if dout.id in ones:
+        ones.add(v.id)
+    return v
+
+
+def _unary_grad(op, x, y, dout, ones):
     """ops/unary_op.cc:891-1019 (y is the op's output)."""
     ns = op.op
     if not x.is_float():
         return None
     if ns in _lib.DTYPES or ns == "cast":
-        return unary(dout, x.dtype)
+        return _still_one(unary(dout, x.dtype), dout, ones)
     one = lambda: make_number(1, x)
     if ns == "negative":
         return unary(dout, "negative")
@@ -92,7 +91,7 @@ def _unary_grad(op, x, y, dout):
     return None      # round / floor / ceil / logical ops: no gradient
 
 
-def _binary_grad(op, x, y, z, dout, index):
+def _binary_grad(op, x, y, z, dout, index, ones):
     """ops/binary_op.cc:491-561 (z is the op's output)."""
     ns = op.op
     if ns == "add":
@@ -100,7 +99,7 @@ def _binary_grad(op, x, y, z, dout, index):
     if ns == "subtract":
         return dout if index == 0 else unary(dout, "negative")
     if ns == "multiply":
-        return _times(y if index == 0 else x, dout)
+        return _times(y if index == 0 else x, dout, ones)
     if ns == "divide":
         if index == 0:
             return binary(dout, y, "divide")
@@ -122,12 +121,12 @@ def _binary_grad(op, x, y, z, dout, index):
     return None      # comparisons, logical and bitwise ops, floor_divide
 
 
-def _op_grad(op, inputs, out, dout, index):
+def _op_grad(op, inputs, out, dout, index, ones):
     x = inputs[index]
     if isinstance(op, UnaryOp):
-        return _unary_grad(op, inputs[0], out, dout)
+        return _unary_grad(op, inputs[0], out, dout, ones)
     if isinstance(op, BinaryOp):
-        return _binary_grad(op, inputs[0], inputs[1], out, dout, index)
+        return _binary_grad(op, inputs[0], inputs[1], out, dout, index, ones)
     if isinstance(op, TernaryOp):                       # ops/ternary_op.cc:49-56
         if index == 0:
             return None
@@ -140,7 +139,7 @@ def _op_grad(op, inputs, out, dout, index):
     if isinstance(op, ReduceOp):                        # ops/reduce_op.cc:339-362
         bc = lambda v: core._broadcast_mask(v, x.shape, op.reduce_mask, op.keepdims_mask)
         if op.op == "add":
-            return bc(dout)
+            return _still_one(bc(dout), dout, ones)
         if op.op == "multiply":
             return binary(bc(binary(dout, out, "multiply")), x, "divide")
         if op.op == "mean":
@@ -170,6 +169,42 @@ def _op_grad(op, inputs, out, dout, index):
             return ternary(cond, back(dout), make_number(0, x))
         return None
     return None
+
+
+def _backward(loss, order, dep, ones):
+    """The gradients of the Vars in `dep` by id.  `ones` takes the ids of the seed and of what is only it, spread or cast, so that
+    products with it are left out; None: no product is."""
+    grads = {}
+    if loss.id in dep:
+        grads[loss.id] = make_number(1.0, loss)
+        if ones is None:
+            ones = frozenset()
+        else:
+            ones.add(grads[loss.id].id)
+    for v in reversed(order):
+        g = grads.get(v.id)
+        if g is None or v._history is None:
+            continue
+        op, inputs = v._history
+        for i, u in enumerate(inputs):
+            if u.id not in dep or not u.is_float():
+                continue
+            saved = dt.amp_reg                                  # an op's gradient is built under the register
+            amp = saved | getattr(op, "amp", 0)                 # the op was created with (grad.cc:48-55)
+            if amp == saved:
+                du = _op_grad(op, inputs, v, g, i, ones)
+            else:
+                dt.amp_reg = amp
+                try:
+                    du = _op_grad(op, inputs, v, g, i, ones)
+                finally:
+                    dt.amp_reg = saved
+            if du is None:
+                continue
+            if du.shape != u.shape:
+                raise RuntimeError("gradient of %r has shape %r, expected %r" % (op, du.shape, u.shape))
+            grads[u.id] = du if u.id not in grads else binary(grads[u.id], du, "add")
+    return grads
 
 
 def grad(loss, targets, retain_graph=True):
@@ -209,32 +244,11 @@ def grad(loss, targets, retain_graph=True):
                     dep.add(v.id)
                     break
 
-    grads = {}
-    if loss.id in dep:
-        grads[loss.id] = make_number(1.0, loss)
-    for v in reversed(order):
-        g = grads.get(v.id)
-        if g is None or v._history is None or v.id in target_ids and v._history is None:
-            continue
-        op, inputs = v._history
-        for i, u in enumerate(inputs):
-            if u.id not in dep or not u.is_float():
-                continue
-            saved = dt.amp_reg                                  # an op's gradient is built under the register
-            amp = saved | getattr(op, "amp", 0)                 # the op was created with (grad.cc:48-55)
-            if amp == saved:
-                du = _op_grad(op, inputs, v, g, i)
-            else:
-                dt.amp_reg = amp
-                try:
-                    du = _op_grad(op, inputs, v, g, i)
-                finally:
-                    dt.amp_reg = saved
-            if du is None:
-                continue
-            if du.shape != u.shape:
-                raise RuntimeError("gradient of %r has shape %r, expected %r" % (op, du.shape, u.shape))
-            grads[u.id] = du if u.id not in grads else binary(grads[u.id], du, "add")
+    ones = set()
+    grads = _backward(loss, order, dep, ones)
+    if any(t.id in grads and grads[t.id].id in ones for t in targets):
+        # the caller gets hold of the seed (or of it spread or cast) and may ask for derivatives by it: nothing is left out then
+        grads = _backward(loss, order, dep, None)
     out = []
     for t in targets:
         g = grads.get(t.id)

@@ -907,3 +907,51 @@ def test_one_thread_at_a_time_executes_a_plan(compile_only, monkeypatch):
     for t in threads:
         t.join()
     assert not failed and not met
+
+
+def _graph_of(v):
+    """What v is computed from: its ops in the order of their results, with their inputs by number; leaves by their shape."""
+    seen, stack = {}, [v]
+    while stack:
+        u = stack.pop()
+        if u.id not in seen:
+            seen[u.id] = u
+            stack.extend(u._history[1] if u._history is not None else ())
+    order = [seen[k] for k in sorted(seen)]
+    number = {u.id: i for i, u in enumerate(order)}
+    return [(u._history[0].sig(),) + tuple(number[w.id] for w in u._history[1]) if u._history is not None else tuple(u.shape) for u in order], seen
+
+
+@pytest.mark.parametrize("scale", [
+    lambda x, s: (x * x).sum() * s,                                    # the factor is a leaf of one element
+    lambda x, s: ((x * x) * s).sum(),                                  # ... spread inside the graph
+    lambda x, s: ((x * x) * s.cast("float64").cast("float32")).sum(),  # ... cast
+])
+@pytest.mark.parametrize("dtype", ["float32", "float16", "bfloat16"])
+def test_second_derivative_by_a_scale_whatever_its_value(scale, dtype):
+    """A gradient leaves out the products with its own seed only: a parameter that holds a 1 stays in the graph like any other."""
+    graphs = []
+    for value in (1.0, 1.5):
+        x = jt.array(np.arange(1, 5, dtype=np.float32), dtype)
+        s = jt.array(np.array([value], np.float32), dtype)
+        dx = jt.grad(scale(x, s), x)
+        graph, seen = _graph_of(dx)
+        assert s.id in seen
+        ds, seen = _graph_of(jt.grad(dx.sum(), s))
+        assert x.id in seen
+        graphs.append((graph, ds))
+    assert graphs[0] == graphs[1]
+
+
+def test_products_with_the_seed_are_left_out_unless_the_caller_holds_it():
+    x, w = jt.array(np.ones((3, 4), np.float32)), jt.array(np.ones((3, 4), np.float32))
+    y = x * w
+    gx = jt.grad(y.sum(), x)
+    assert gx.id != w.id and _graph_of(gx)[0] == [(3, 4), (("unary", "cast"), 0)]           # w, as a Var of its own
+    gx, gy = jt.grad(y.sum(), [x, y])                                    # gy is the seed, spread
+    assert gy.id in _graph_of(gx)[1]
+    assert w.id in _graph_of(jt.grad(gx.sum(), gy))[1]
+    one = jt.grad(x.sum(), x)                                            # a seed of an earlier call is a Var like any other
+    a = jt.array(np.ones((3, 4), np.float32))
+    da = jt.grad(((a * x) * one).sum(), a)
+    assert one.id in _graph_of(da)[1]
