@@ -8,10 +8,12 @@ ops/reindex_op.cc:20-91, ops/reindex_reduce_op.cc:26-73, ops/array_op.cc:54-80).
 Nothing executes until a Var is synchronised (lazy_execution,
 var_holder.cc:25-33); execution is in executor.py.
 """
+import collections
 import functools
 import itertools
 import math
 import numbers
+import threading
 import weakref
 
 import numpy as np
@@ -52,10 +54,17 @@ _ref = weakref.ref
 # few larger layers: 2540 us a call, 21 us with room in the pool).
 # --------------------------------------------------------------------------
 class _Pool:
+    """Buffers are made and dropped by any thread, and a collection may drop some in the middle of the bookkeeping below: one lock
+    around it, blocks that come back while it is under way on the same thread wait in `_late` until it is done, and the driver,
+    which other threads may enter meanwhile, is called outside it on blocks that are in no list."""
+
     def __init__(self):
-        self.free_blocks = {}          # size -> free blocks of it, the size used last at the end
+        self.free_blocks = {}          # size -> free blocks of it (one at least), the size used last at the end
         self.cached_bytes = 0
         self.limit = 8 << 30
+        self._lock = threading.RLock()
+        self._inside = False
+        self._late = collections.deque()
 
     @staticmethod
     def _round(n):
@@ -66,13 +75,14 @@ class _Pool:
 
     def alloc(self, nbytes):
         size = self._round(nbytes)
-        lst = self.free_blocks.get(size)
-        if lst:
-            self.cached_bytes -= size
-            ptr = lst.pop()
-            if not lst:
-                del self.free_blocks[size]
-            return ptr, size
+        with self._lock:                                   # (nothing in here starts a collection)
+            lst = self.free_blocks.get(size)
+            if lst is not None and not self._inside:
+                ptr = lst.pop()
+                if not lst:
+                    del self.free_blocks[size]
+                self.cached_bytes -= size
+                return ptr, size
         try:
             return _lib.alloc(size), size
         except MjtError:
@@ -82,31 +92,65 @@ class _Pool:
     def free(self, ptr, size):
         if _lib.device() is None:
             return
-        lst = self.free_blocks.pop(size, None)
+        surplus = None
+        with self._lock:
+            if self._inside:
+                self._late.append((ptr, size))
+                return
+            self._inside = True
+            try:
+                cached = self.cached_bytes + size
+                if cached <= self.limit:
+                    lst = self.free_blocks.pop(size, None)
+                    if lst is None:
+                        lst = [ptr]
+                    else:
+                        lst.append(ptr)
+                    self.free_blocks[size] = lst
+                    self.cached_bytes = cached
+                else:
+                    surplus = self._make_room(size)
+                    if self.cached_bytes + size <= self.limit:
+                        self.free_blocks.setdefault(size, []).append(ptr)
+                        self.cached_bytes += size
+                    else:
+                        surplus.append(ptr)
+            finally:
+                self._inside = False
+        if surplus is not None:
+            for old in surplus:
+                _lib.free(old)
+        while self._late:
+            try:
+                ptr, size = self._late.popleft()
+            except IndexError:                             # another thread was faster
+                return
+            self.free(ptr, size)
+
+    def _make_room(self, size):
+        """Takes blocks out until `size` bytes fit in, those of that size last and not at all."""
+        same = self.free_blocks.pop(size, None)
+        gone = []
         while self.cached_bytes + size > self.limit and self.free_blocks:
             old = next(iter(self.free_blocks))
-            stale = self.free_blocks[old]
-            _lib.free(stale.pop())
-            self.cached_bytes -= old
-            if not stale:
+            lst = self.free_blocks[old]
+            gone.append(lst.pop())
+            if not lst:
                 del self.free_blocks[old]
-        if self.cached_bytes + size > self.limit:          # nothing left but blocks of this size
-            if lst:
-                self.free_blocks[size] = lst
-            _lib.free(ptr)
-            return
-        if lst is None:
-            lst = []
-        lst.append(ptr)
-        self.free_blocks[size] = lst
-        self.cached_bytes += size
+            self.cached_bytes -= old
+        if same:
+            self.free_blocks[size] = same
+        return gone
 
     def release_all(self):
-        for lst in self.free_blocks.values():
+        blocks = {}
+        with self._lock:
+            if not self._inside:
+                blocks, self.free_blocks = self.free_blocks, blocks
+                self.cached_bytes = 0
+        for lst in blocks.values():
             for p in lst:
                 _lib.free(p)
-        self.free_blocks.clear()
-        self.cached_bytes = 0
 
 
 pool = _Pool()

@@ -955,3 +955,91 @@ def test_products_with_the_seed_are_left_out_unless_the_caller_holds_it():
     a = jt.array(np.ones((3, 4), np.float32))
     da = jt.grad(((a * x) * one).sum(), a)
     assert one.id in _graph_of(da)[1]
+
+
+class _FakeDriver:
+    """Allocations that are only counted; a call lets other threads run, as the driver does."""
+
+    def __init__(self, monkeypatch):
+        self.live, self.made, self.on_free = {}, 0, None
+        monkeypatch.setattr(L, "alloc", self.alloc)
+        monkeypatch.setattr(L, "free", self.free)
+        monkeypatch.setattr(L, "device", lambda: 0)
+
+    def alloc(self, size):
+        import time
+        time.sleep(0)
+        self.made += 1
+        ptr = object()
+        self.live[id(ptr)] = (ptr, size)
+        return ptr
+
+    def free(self, ptr):
+        import time
+        time.sleep(0)
+        del self.live[id(ptr)]
+
+
+@pytest.mark.parametrize("limit", [1 << 40, 5000])
+def test_pool_keeps_count_of_its_blocks_between_threads(monkeypatch, limit):
+    """Threads that take and give back blocks of a few sizes, with a pool that has room and with one that is always full: no
+    error, every block is in the pool or with the driver, and the pool's count is that of its lists."""
+    import sys
+    import threading
+    from jittor_amd import core
+    driver, pool, failed = _FakeDriver(monkeypatch), core._Pool(), []
+    pool.limit = limit
+    every = sys.getswitchinterval()
+    sys.setswitchinterval(1e-6)
+
+    def work(seed):
+        rng = np.random.default_rng(seed)
+        held = []
+        try:
+            for size in rng.choice([256, 512, 1024, 4096], 8000):
+                held.append(pool.alloc(int(size)))
+                if len(held) > 3:
+                    pool.free(*held.pop(0))
+            for block in held:
+                pool.free(*block)
+        except Exception as e:                                         # shown by the assertion below
+            failed.append(repr(e))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    try:
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+    finally:
+        sys.setswitchinterval(every)
+    assert not failed, failed[:3]
+    cached = [(id(p), size) for size, lst in pool.free_blocks.items() for p in lst]
+    assert len(set(cached)) == len(cached) and sorted(cached) == sorted((k, size) for k, (_, size) in driver.live.items())
+    assert pool.cached_bytes == sum(size for _, size in cached) <= limit
+    assert all(pool.free_blocks.values())
+    pool.release_all()
+    assert not driver.live and pool.cached_bytes == 0
+
+
+@pytest.mark.parametrize("first,second", [(256, 256), (256, 512), (512, 256)])
+def test_pool_takes_blocks_back_from_a_finaliser_inside_its_own_bookkeeping(monkeypatch, first, second):
+    """A collection may start while a block is taken in and drop another one: both are kept, and counted."""
+    from jittor_amd import core
+    driver, pool = _FakeDriver(monkeypatch), core._Pool()
+    blocks, late = [pool.alloc(first), pool.alloc(first)], [pool.alloc(second)]
+
+    class Collecting(dict):
+        def pop(self, *args):
+            got = dict.pop(self, *args)
+            if late and not armed:
+                pool.free(*late.pop())                                 # between two steps of the call under way
+            return got
+
+    armed = [1]
+    pool.free(*blocks[0])
+    pool.free_blocks = Collecting(pool.free_blocks)
+    armed.clear()
+    pool.free(*blocks[1])
+    sizes = sorted(size for size, lst in pool.free_blocks.items() for _ in lst)
+    assert sizes == sorted([first, first, second]) and pool.cached_bytes == sum(sizes) and len(driver.live) == 3
