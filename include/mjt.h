@@ -403,10 +403,13 @@ int mjt_expr_affine(const char* expr, const mjt_tensor* x, const mjt_tensor* y,
  * stand-in scalars, show which words come from which buffer or scalar:
  * mjt_record_relocate works that out and makes `first` replayable (`second`
  * is only read).  mjt_record_launch then launches it on real buffers in one
- * call.  MJT_ERR_UNSUPPORTED: a call that cannot be recorded, a word of other
- * origin, a buffer that is not 256-byte aligned, or a recording that is out of
- * date because the library's own scratch memory moved or it was shut down;
- * nothing has been launched then and the calls themselves are the way. */
+ * call.  MJT_ERR_UNSUPPORTED: a call that cannot be recorded (copies to and
+ * from host memory, fills, device copies, events, mjt_where and its count, a
+ * scatter that keeps tallies: they act the moment they are made), a word of
+ * other origin, a buffer that is not 256-byte aligned, or a recording that is
+ * out of date because the library's own scratch memory moved, it was shut down
+ * or an MJT_ environment variable has changed; nothing has been launched then
+ * and the calls themselves are the way. */
 int  mjt_record_begin(void);
 int  mjt_record_end(void** rec);                 /* rec == NULL: drop it */
 int  mjt_record_relocate(void* first, void* second, int n_slots, const uint64_t* base1, const uint64_t* base2, uint64_t span,

@@ -166,7 +166,9 @@ void where_count_impl(const mjt_tensor* cond, int64_t* count) {
     const size_t n = (size_t)numel(cond);
     *count = 0;
     Context& c = ctx();
-    if (n == 0 || c.dry_run) return;
+    if (n == 0) return;
+    refuse_recording("a count that the host waits for");
+    if (c.dry_run) return;
     const size_t nblocks = (n + kTile - 1) / kTile;
     MJT_CHECK(nblocks < (size_t(1) << 31), "where: tensor too large");
     unsigned long long* offsets = count_and_scan(cond, n, nblocks);
@@ -200,7 +202,9 @@ void where_impl(const mjt_tensor* cond, int64_t count, const mjt_tensor* outs) {
     }
     const size_t n = (size_t)numel(cond);
     Context& c = ctx();
-    if (n == 0 || count == 0 || c.dry_run) return;
+    if (n == 0 || count == 0) return;
+    refuse_recording("where");
+    if (c.dry_run) return;
     const size_t nblocks = (n + kTile - 1) / kTile;
     MJT_CHECK(nblocks < (size_t(1) << 31), "where: tensor too large");
     unsigned long long* offsets = count_and_scan(cond, n, nblocks);

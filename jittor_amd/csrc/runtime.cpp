@@ -463,6 +463,7 @@ int mjt_free(void* p) {
 }
 int mjt_h2d(void* dst, const void* src, size_t bytes) {
     return guarded([&] {
+        if (bytes) refuse_recording("a copy from host memory");
         require_device();
         if (!bytes) return;
         HIP_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx().stream));
@@ -471,6 +472,7 @@ int mjt_h2d(void* dst, const void* src, size_t bytes) {
 }
 int mjt_d2h(void* dst, const void* src, size_t bytes) {
     return guarded([&] {
+        if (bytes) refuse_recording("a copy to host memory");
         require_device();
         if (!bytes) return;
         HIP_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx().stream));
@@ -508,6 +510,7 @@ int mjt_event_create(void** ev) {
 }
 int mjt_event_record(void* ev) {
     return guarded([&] {
+        refuse_recording("an event");
         require_device();
         HIP_CHECK(hipEventRecord((hipEvent_t)ev, ctx().stream));
     });

@@ -825,6 +825,28 @@ def test_recorded_launches(compile_only, monkeypatch):
         lib.mjt_record_free(rec)
 
 
+def test_recording_refuses_what_is_no_launch_of_its_own(compile_only):
+    """Copies to and from host memory, events and the two calls of where act on the device, or on the host, the moment they are
+    made: between begin and end, where addresses may be stand-ins, they are refused.  Nothing to do is nothing to refuse."""
+    lib = L.load()
+    count, host = ctypes.c_int64(), ctypes.create_string_buffer(64)
+    cond, empty, out = L.tensor(1 << 45, "float32", [64]), L.tensor(1 << 45, "float32", [0]), (L.Tensor * 1)(L.tensor(1 << 46, "int32", [64]))
+    none = (L.Tensor * 1)(L.tensor(1 << 46, "int32", [0]))
+    dev = ctypes.c_void_p(1 << 45)
+    L.check(lib.mjt_record_begin())
+    try:
+        for name, rc in (("where_count", lib.mjt_where_count(ctypes.byref(cond), ctypes.byref(count))),
+                         ("where", lib.mjt_where(ctypes.byref(cond), 64, out)),
+                         ("h2d", lib.mjt_h2d(dev, host, 64)), ("d2h", lib.mjt_d2h(host, dev, 64)), ("event", lib.mjt_event_record(None))):
+            assert rc == L.ERR_UNSUPPORTED and "recording" in lib.mjt_last_error().decode(), name
+        assert lib.mjt_where_count(ctypes.byref(empty), ctypes.byref(count)) == 0 and count.value == 0
+        assert lib.mjt_where(ctypes.byref(empty), 0, none) == 0
+    finally:
+        L.check(lib.mjt_record_end(None))
+    assert lib.mjt_where_count(ctypes.byref(cond), ctypes.byref(count)) == 0
+    assert lib.mjt_where(ctypes.byref(cond), 64, out) == 0
+
+
 @pytest.mark.parametrize("pairs", [1, 170, 171, 172, 400])
 def test_recorded_launches_tell_all_buffers_apart(compile_only, monkeypatch, pairs):
     """The two sets of stand-in addresses share none, also where a graph has more buffers (3 per pair) than fit between two
