@@ -73,6 +73,13 @@ Context& ctx();
 void require_init();
 void require_device();
 void* scratch(size_t bytes);      // grows the scratch arena when needed
+// A buffer that the library keeps between calls, grown to `bytes`.  False, with nothing left in it, where the device has no room.
+bool grow_kept(void** buffer, size_t* have, size_t bytes);
+// Memory that a call would like for speed only: false where the route that needs it is not to be taken, because it is more than
+// MJT_MOST_WORKSPACE bytes.  A route that gets true and then no memory goes back to the one without, too.
+bool workspace_allowed(size_t bytes);
+// scratch() for such a route: null instead of an error
+void* scratch_if_any(size_t bytes);
 // mjt_shutdown runs these first, while the stream and the kernel modules still exist: whatever a file keeps
 // beyond a call (kernel look-up tables, device buffers, library handles) is dropped there
 void at_shutdown(void (*fn)());

@@ -610,19 +610,8 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
 
 // The buffer of per-slice partial weight gradients, grown to `bytes`.
 static void* wgrad_partials(size_t bytes) {
-    Context& c = ctx();
-    if (c.dry_run) return (void*)(uintptr_t)0x1000;
-    if (bytes > g_wgrad_bytes) {
-        kept_buffer_moved();
-        if (g_wgrad_part) {
-            HIP_CHECK(hipStreamSynchronize(c.stream));
-            HIP_CHECK(hipFree(g_wgrad_part));
-            g_wgrad_part = nullptr;
-            g_wgrad_bytes = 0;
-        }
-        HIP_CHECK(hipMalloc(&g_wgrad_part, bytes));
-        g_wgrad_bytes = bytes;
-    }
+    if (ctx().dry_run) return (void*)(uintptr_t)0x1000;
+    if (!grow_kept(&g_wgrad_part, &g_wgrad_bytes, bytes)) MJT_FAIL(MJT_ERR_DEVICE, "conv wgrad: no device memory for " << bytes << " bytes of partial sums");
     return g_wgrad_part;
 }
 
@@ -780,6 +769,9 @@ static bool conv_wgrad_product(const mjt_tensor* x, const mjt_tensor* dy, const 
     if (slices * numel(dw) * 4 > (int64_t(1) << 30)) return false;
     const int64_t per = (stages + slices - 1) / slices;
     slices = (stages + per - 1) / per;
+    const bool in_place = slices == 1 && dw->dtype == MJT_FLOAT32;
+    const size_t part_bytes = (size_t)slices * (size_t)numel(dw) * 4;
+    if (!in_place && !(workspace_allowed(part_bytes) && (ctx().dry_run || grow_kept(&g_wgrad_part, &g_wgrad_bytes, part_bytes)))) return false;
     std::ostringstream key;
     key << "wgprod|" << C << "|" << H << "|" << W << "|" << K << "|" << R << "|" << S << "|" << OH << "|" << OW << "|" << p->stride_h << "|" << p->stride_w << "|" << p->pad_h << "|" << p->pad_w
         << "|" << p->dil_h << "|" << p->dil_w << "|" << MI << NI << in;
@@ -797,8 +789,7 @@ static bool conv_wgrad_product(const mjt_tensor* x, const mjt_tensor* dy, const 
         k = jit_get(src.str(), name.str());
         remember(key.str(), k);
     }
-    const bool in_place = slices == 1 && dw->dtype == MJT_FLOAT32;
-    void* part = in_place ? dw->ptr : wgrad_partials((size_t)slices * (size_t)numel(dw) * 4);
+    void* part = in_place ? dw->ptr : wgrad_partials(part_bytes);
     std::vector<uint64_t> a{bits_of_ptr(dy->ptr), bits_of_ptr(x->ptr), bits_of_ptr(part), (uint64_t)K, (uint64_t)CRS, (uint64_t)Q, 0, 0, (uint64_t)CRS, (uint64_t)per,
                             (uint64_t)(numel(x) * esz), (uint64_t)(K * CRS)};
     const int64_t grid = (slices * tiles + 7) / 8 * 8;

@@ -48,21 +48,12 @@ int env_int(const char* name, int dflt) {
     return v && *v ? atoi(v) : dflt;
 }
 
-// [rows, ld] copied into rows of `ldp` elements (zeros behind each), into the buffer of operand `which`.
+// [rows, ld] copied into rows of `ldp` elements (zeros behind each), into the buffer of operand `which`; null where there is no
+// memory for it.
 const void* padded_rows(int which, const void* src, int dtype, int64_t rows, int64_t ld, int64_t ldp) {
     Context& c = ctx();
     const size_t bytes = (size_t)(rows * ldp * dtype_size(dtype));
-    if (!c.dry_run && bytes > g_rows_bytes[which]) {
-        kept_buffer_moved();
-        if (g_rows[which]) {
-            HIP_CHECK(hipStreamSynchronize(c.stream));
-            HIP_CHECK(hipFree(g_rows[which]));
-            g_rows[which] = nullptr;
-            g_rows_bytes[which] = 0;
-        }
-        HIP_CHECK(hipMalloc(&g_rows[which], bytes));
-        g_rows_bytes[which] = bytes;
-    }
+    if (!workspace_allowed(bytes) || !(c.dry_run || grow_kept(&g_rows[which], &g_rows_bytes[which], bytes))) return nullptr;
     mjt_tensor t{}, d{};
     t.ptr = (void*)src;
     d.ptr = c.dry_run ? (void*)(uintptr_t)0x1000 : g_rows[which];
@@ -194,6 +185,8 @@ void gemm_launch(int in_dtype, int out_dtype, const void* A, const void* B, void
                 if (t < least && nn * M * N * 4 <= (int64_t(256) << 20)) { least = t; slices = nn; per = pn; }
             }
         }
+        void* part_mem = slices > 1 ? scratch_if_any((size_t)(slices * M * N * 4)) : nullptr;
+        if (!part_mem) slices = 1;
         if (slices > 1) best_mi = best_ni = 1;
         const int MI = best_mi, NI = best_ni;
         const int in = in_dtype == MJT_BFLOAT16 ? 0 : in_dtype == MJT_FLOAT16 ? 1 : 2;
@@ -222,7 +215,7 @@ void gemm_launch(int in_dtype, int out_dtype, const void* A, const void* B, void
             return;
         }
         mjt_tensor part{}, whole{};
-        part.ptr = scratch((size_t)(slices * M * N * 4));
+        part.ptr = part_mem;
         part.dtype = MJT_FLOAT32;
         part.ndim = 2;
         part.shape[0] = slices;
@@ -350,10 +343,12 @@ void matmul_impl(const mjt_tensor* a, const mjt_tensor* b, const mjt_tensor* c, 
         if ((pad_a || pad_b) && a->dtype != MJT_FLOAT64 && !share_a && batch < 65536 && !getenv("MJT_GEMM_PLAIN") && !getenv("MJT_NO_FASTPATH") &&
             (double)batch * n * k * m >= (double)(1 << (m >= 96 ? 20 : 22)) && (!pad_a || ra * lap * esz <= most) && (!pad_b || rb * lbp * esz <= most)) {
             const void* pa = pad_a ? padded_rows(0, a->ptr, a->dtype, ra, lda, lap) : a->ptr;
-            const void* pb = pad_b ? padded_rows(1, b->ptr, b->dtype, rb, ldb, lbp) : b->ptr;
+            const void* pb = !pad_b ? b->ptr : pa ? padded_rows(1, b->ptr, b->dtype, rb, ldb, lbp) : nullptr;
             const int64_t la = pad_a ? lap : lda, lb = pad_b ? lbp : ldb;
-            gemm_launch(a->dtype, c->dtype, pa, pb, c->ptr, n, k, m, la, lb, k, a->shape[nd - 2] * la, b->shape[nd - 2] * lb, n * k, batch, !trans_a, trans_b != 0, 0, 0, k % 8 == 0);
-            return;
+            if (pa && pb) {
+                gemm_launch(a->dtype, c->dtype, pa, pb, c->ptr, n, k, m, la, lb, k, a->shape[nd - 2] * la, b->shape[nd - 2] * lb, n * k, batch, !trans_a, trans_b != 0, 0, 0, k % 8 == 0);
+                return;
+            }
         }
     }
     const int64_t per_launch = 65535;                         // the batch rides on a grid axis

@@ -88,23 +88,39 @@ static std::vector<void (*)()>& shutdown_hooks() {
 }
 void at_shutdown(void (*fn)()) { shutdown_hooks().push_back(fn); }
 
-void* scratch(size_t bytes) {
+bool grow_kept(void** buffer, size_t* have, size_t bytes) {
+    if (bytes <= *have) return true;
+    kept_buffer_moved();
+    if (*buffer) {
+        HIP_CHECK(hipStreamSynchronize(ctx().stream));
+        HIP_CHECK(hipFree(*buffer));
+        *buffer = nullptr;
+        *have = 0;
+    }
+    if (hipMalloc(buffer, bytes) != hipSuccess) {
+        (void)hipGetLastError();                              // the next launch is not to find this error
+        *buffer = nullptr;
+        return false;
+    }
+    *have = bytes;
+    return true;
+}
+bool workspace_allowed(size_t bytes) {
+    const char* most = getenv("MJT_MOST_WORKSPACE");
+    return !most || !*most || bytes <= (size_t)strtoull(most, nullptr, 10);
+}
+static void* scratch_or_null(size_t bytes) {
     Context& c = ctx();
     if (c.dry_run) return (void*)(uintptr_t)0x1000;
-    if (bytes > c.scratch_bytes) {
-        kept_buffer_moved();
-        if (c.scratch) {
-            HIP_CHECK(hipStreamSynchronize(c.stream));
-            HIP_CHECK(hipFree(c.scratch));
-            c.scratch = nullptr;
-            c.scratch_bytes = 0;
-        }
-        size_t want = bytes < (size_t(8) << 20) ? (size_t(8) << 20) : bytes;
-        HIP_CHECK(hipMalloc(&c.scratch, want));
-        c.scratch_bytes = want;
-    }
-    return c.scratch;
+    const size_t least = size_t(8) << 20;
+    return grow_kept(&c.scratch, &c.scratch_bytes, bytes < least ? least : bytes) ? c.scratch : nullptr;
 }
+void* scratch(size_t bytes) {
+    void* p = scratch_or_null(bytes);
+    if (!p) MJT_FAIL(MJT_ERR_DEVICE, "no device memory for " << bytes << " bytes of scratch");
+    return p;
+}
+void* scratch_if_any(size_t bytes) { return workspace_allowed(bytes) ? scratch_or_null(bytes) : nullptr; }
 
 // ---- dtype tables ------------------------------------------------------------
 static const char* k_dtype_names[MJT_DTYPE_COUNT] = {

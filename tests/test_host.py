@@ -1065,3 +1065,39 @@ def test_pool_takes_blocks_back_from_a_finaliser_inside_its_own_bookkeeping(monk
     pool.free(*blocks[1])
     sizes = sorted(size for size, lst in pool.free_blocks.items() for _ in lst)
     assert sizes == sorted([first, first, second]) and pool.cached_bytes == sum(sizes) and len(driver.live) == 3
+
+
+def test_routes_that_want_workspace_have_one_without(compile_only, monkeypatch):
+    """Padded copies of unaligned rows, slices of long sums and slices of a weight gradient are for speed: without the memory for
+    them (here: a limit on it) the call runs as it lies, or is handed back to the caller who has another way."""
+    lib = compile_only.load()
+    p = L.ConvParams(1, 1, 1, 1, 1, 1)
+
+    def product(m, k, n, dt, ta, tb):
+        a, b = (L.tensor(P, dt, s) for s in ([k, m] if ta else [m, k], [n, k] if tb else [k, n]))
+        c = L.tensor(P, dt, [m, n])
+        L.check(lib.mjt_matmul(ctypes.byref(a), ctypes.byref(b), ctypes.byref(c), ta, tb))
+        return L.last_kernel()
+
+    def wgrad(dt):
+        x, dy, dw = L.tensor(P, dt, [64, 40, 15, 13]), L.tensor(P, dt, [64, 72, 15, 13]), L.tensor(P, "float32", [72, 40, 3, 3])
+        rc = lib.mjt_conv2d_meta_wgrad(ctypes.byref(x), ctypes.byref(dy), ctypes.byref(dw), ctypes.byref(p))
+        return rc, L.last_kernel()
+
+    monkeypatch.delenv("MJT_MOST_WORKSPACE", raising=False)
+    assert product(301, 203, 129, "bfloat16", 0, 0).startswith("mjt_gemm_mfma_")
+    assert product(64, 4096, 64, "float32", 1, 0).endswith("_slices")
+    for dt in ("float32", "bfloat16"):
+        rc, kernel = wgrad(dt)
+        assert rc == 0 and kernel.startswith("mjt_conv_wgrad_igemm_")
+    monkeypatch.setenv("MJT_MOST_WORKSPACE", "4096")
+    for ta in (0, 1):
+        for tb in (0, 1):
+            assert product(301, 203, 129, "bfloat16", ta, tb).startswith("mjt_gemm_plain_")
+    assert product(301, 208, 129, "bfloat16", 0, 0).startswith("mjt_gemm_plain_")          # one operand of the two
+    kernel = product(64, 4096, 64, "float32", 1, 0)
+    assert kernel.startswith("mjt_gemm_mfma_") and not kernel.endswith("_slices")
+    for dt in ("float32", "bfloat16"):
+        assert wgrad(dt)[0] == L.ERR_UNSUPPORTED
+    monkeypatch.setenv("MJT_MOST_WORKSPACE", str(1 << 30))
+    assert product(301, 203, 129, "bfloat16", 0, 0).startswith("mjt_gemm_mfma_")
