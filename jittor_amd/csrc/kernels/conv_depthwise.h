@@ -179,16 +179,25 @@ extern "C" __global__ __launch_bounds__(256) void ENTRY(Params p) {
                     for (int k = 0; k < STVEC; k++) dy[ro][j + k] = in ? (float)v.v[k] : 0.0f;
                 }
             }
+            // A strip may reach past the map's last row and column, over pixels that exist: those positions are no term of the sum, and
+            // a product with their zero would be one (0 times an infinity).  Columns are taken out of x once per row, rows are skipped.
+            constexpr bool PART_ROWS = OH_ % RS != 0 || OH_ % TH != 0, PART_COLS = OW_ % CW != 0;
+            const int rows = OH_ - oh0 < TH ? OH_ - oh0 - strip * RS : TH - strip * RS;
             mjt_dw_rows(pl, strip, cg, [&](int lr, const float* x) {
+                float xv[S_][CW];
+#pragma unroll
+                for (int s = 0; s < S_; s++)
+#pragma unroll
+                    for (int j = 0; j < CW; j++) xv[s][j] = !PART_COLS || cg * CW + j < OW_ ? x[j * SW + s * DW] : 0.0f;
 #pragma unroll
                 for (int ro = 0; ro < RS; ro++)
 #pragma unroll
                     for (int r = 0; r < R_; r++)
-                        if (ro * SH + r * DH == lr) {
+                        if (ro * SH + r * DH == lr && (!PART_ROWS || ro < rows)) {
 #pragma unroll
                             for (int s = 0; s < S_; s++)
 #pragma unroll
-                                for (int j = 0; j < CW; j++) acc[r * S_ + s] = acc[r * S_ + s] + dy[ro][j] * x[j * SW + s * DW];
+                                for (int j = 0; j < CW; j++) acc[r * S_ + s] = acc[r * S_ + s] + dy[ro][j] * xv[s][j];
                         }
             });
         }

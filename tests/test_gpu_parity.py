@@ -1815,6 +1815,44 @@ def test_depthwise_conv_and_gradients(gpu, case):
         assert np.all(np.abs(got - ref) <= terms * 2.0 ** -24 * mag + eps * np.abs(ref) + 2.0 ** -24 * (out == "float16")), name
 
 
+@pytest.mark.parametrize("dt", ["float32", "bfloat16"])
+@pytest.mark.parametrize("hw,p", [
+    ((7, 7), (1, 1, 1, 1, 1, 1)),              # the last strip is one row and three columns short
+    ((7, 7), (1, 1, 0, 0, 1, 1)),              # 5 x 5 positions on real pixels
+    ((14, 14), (2, 2, 1, 1, 1, 1)),            # stride 2: the positions past the map lie over the last pixels
+    ((8, 6), (1, 1, 1, 1, 1, 1)),              # whole rows, columns short
+    ((6, 8), (1, 1, 1, 1, 1, 1)),              # whole columns, rows short
+    ((130, 100), (1, 1, 1, 1, 1, 1)),          # tiles of rows, the last one short
+])
+def test_depthwise_weight_gradient_leaves_an_infinity_where_it_belongs(gpu, hw, p, dt):
+    """Infinite pixels in the last rows and columns reach the taps whose sums contain them and no other: positions past the map are
+    no terms of a sum.  Against float64; float32 sums of n products are off by n * 2^-24 of their magnitudes."""
+    rng = np.random.default_rng(47)
+    N, C, (H, W), R = 3, 4, hw, 3
+    sh, sw, ph, pw, dh, dw_ = p
+    OH, OW = (H + 2 * ph - dh * (R - 1) - 1) // sh + 1, (W + 2 * pw - dw_ * (R - 1) - 1) // sw + 1
+    for at in ((H - 1, W - 1), (0, W - 1), (H - 1, 0), (H // 2, W - 2)):
+        x = rng.integers(1, 9, (N, C, H, W)).astype(np.float32)
+        dy = rng.integers(1, 9, (N, C, OH, OW)).astype(np.float32)              # exact in both types, no sum cancels
+        x[1, 2][at] = np.inf
+        vx, vd = (jt.from_storage(a if dt == "float32" else _bf16(a), dt) for a in (x, dy))
+        vw = jt.zeros([C, 1, R, R]) + 7.0
+        jt.sync([vx, vd, vw], True)
+        tx, td, tw = (L.tensor(v.raw_ptr(), v.dtype, v.shape) for v in (vx, vd, vw))
+        cp = L.ConvParams(*p)
+        L.check(L.load().mjt_conv2d_meta_wgrad_grouped(ctypes.byref(tx), ctypes.byref(td), ctypes.byref(tw), ctypes.byref(cp), C))
+        assert "_depthwise" in L.last_kernel()
+        got = vw.numpy()[:, 0]
+        xp, want = np.pad(x.astype(np.float64), ((0, 0), (0, 0), (ph, ph), (pw, pw))), np.zeros((C, R, R))
+        for r in range(R):
+            for s in range(R):
+                want[:, r, s] = (dy * xp[:, :, r * dh:r * dh + (OH - 1) * sh + 1:sh, s * dw_:s * dw_ + (OW - 1) * sw + 1:sw]).sum((0, 2, 3))
+        assert np.isfinite(want).any() and not np.isnan(want).any()
+        fin = np.isfinite(want)
+        assert np.array_equal(np.isfinite(got), fin), (at, got[2], want[2])
+        assert np.all(got[~fin] == np.inf) and np.all(np.abs(got[fin] - want[fin]) <= N * OH * OW * 2.0 ** -24 * want[fin])
+
+
 @pytest.mark.parametrize("case", [
     dict(x=(8, 64, 14, 14), k=96, rs=(1, 1), p=(1, 1, 0, 0, 1, 1)),        # planes of 196 pixels: pieces of four, chunks that span images
     dict(x=(14, 72, 6, 7), k=136, rs=(1, 1), p=(1, 1, 0, 0, 1, 1)),         # 42 pixels: pairs
