@@ -145,7 +145,8 @@ extern "C" __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu
     // scalar offset.  An operand with m (or n) innermost is staged as it lies in memory, [64 k][256 columns], 512-byte
     // rows of sixteen 32-byte units: lane i of instruction j fills k-row 2 j + i / 32, 16-byte piece i % 32, and unit u of
     // k-row r sits at position u ^ (r % 4).  Its descriptor starts at the tile's first column and ends with the operand,
-    // so whatever lies past the matrix reads as zero; a stage adds 64 rows through the scalar offset.
+    // so whatever lies past the matrix reads as zero; a stage adds 64 rows through the scalar offset.  The range is checked by the
+    // dword: an odd number of columns ends with the element behind it, which the leading dimension, a multiple of 8, holds.
     const int last_a = M - 1 - m0, last_b = N - 1 - n0;             // last valid row of the tile
     unsigned voff_a[CPW], voff_b[CPW];
 #pragma unroll
@@ -173,7 +174,7 @@ extern "C" __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu
     const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(A + (long long)m0 * lda), 0, 0x7fffffff, 0x00020000);
     const int a_step = KS * 2;
 #else
-    const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(A + m0), 0, (int)(((long long)(K - 1) * lda + (M - m0)) * 2), 0x00020000);
+    const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(A + m0), 0, (int)(((long long)(K - 1) * lda + ((M - m0 + 1) & ~1)) * 2), 0x00020000);
     const int a_step = (int)(KS * lda * 2);
 #endif
 #if IMG
@@ -183,7 +184,7 @@ extern "C" __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu
     const __amdgpu_buffer_rsrc_t b_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(B + (long long)n0 * ldb), 0, 0x7fffffff, 0x00020000);
     const int b_step = KS * 2;
 #else
-    const __amdgpu_buffer_rsrc_t b_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(B + n0), 0, (int)(((long long)(K - 1) * ldb + (N - n0)) * 2), 0x00020000);
+    const __amdgpu_buffer_rsrc_t b_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(B + n0), 0, (int)(((long long)(K - 1) * ldb + ((N - n0 + 1) & ~1)) * 2), 0x00020000);
     const int b_step = (int)(KS * ldb * 2);
 #endif
     // instruction q (0 .. 15: eight of A, eight of B) of this wave's share of stage s; s and slot uniform

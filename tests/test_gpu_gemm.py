@@ -274,3 +274,12 @@ def test_gemm_unaligned_rows_are_copied(gpu, dt, ta, tb):
     for i, (M, K, N) in enumerate([(301, 203, 129), (304, 201, 136), (129, 336, 201), (1001, 1001, 67), (257, 4099, 65)]):
         assert _run(lib, dt, dt, M, K, N, ta, tb, seed=i).startswith("mjt_gemm_mfma_"), (M, K, N)
     assert _run(lib, dt, dt, 61, 203, 129, ta, tb, seed=7, batch=(5,)).startswith("mjt_gemm_mfma_")
+
+
+@pytest.mark.parametrize("dt", ["bfloat16", "float16"])
+@pytest.mark.parametrize("tb", [0, 1])
+@pytest.mark.parametrize("M,K,N", [(1001, 128, 1024), (1001, 1024, 1024), (1151, 192, 1016)])
+def test_gemm_odd_rows_of_a_transposed_operand(gpu, dt, tb, M, K, N):
+    """a^T b with an odd number of result rows on the kernel that copies its operands into LDS: the last element of a, half of the
+    last dword in range, belongs to the last row's sum."""
+    assert "_direct" in _run(L.load(), dt, "float32", M, K, N, 1, tb, seed=M + K)
