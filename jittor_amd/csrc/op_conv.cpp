@@ -728,34 +728,40 @@ static bool conv_wgrad_product(const mjt_tensor* x, const mjt_tensor* dy, const 
     const int64_t cus = ctx().dry_run || ctx().prop.multiProcessorCount <= 0 ? 256 : ctx().prop.multiProcessorCount;
     const int in = x->dtype == MJT_BFLOAT16 ? 0 : half ? 1 : 2;
     const int64_t KS = half ? 64 : 32;
-    // 128 x 128 tiles gather half as much per multiply-add and hold two workgroups a compute unit, 64 x 64 tiles waste less on
-    // the edges and hold four (us at 3x3, 64 / 128: 64 x 64 x 56 x 56 -> 64: 162 / 447; 64 x 128 x 28 x 28 -> 128: 161 / 155;
-    // 64 x 256 x 14 x 14 -> 256: 180 / 150; 64 x 512 x 7 x 7 -> 512: 195 / 176)
+    // Tile and slices of the sum by what they are estimated to take.  Slices end in a fold: 5 us, 8 with more than 16 of them (the
+    // reduce is then two launches), and its traffic.
     auto tiles_of = [&](int64_t t) { return ((K + t - 1) / t) * ((CRS + t - 1) / t); };
-    int MI = tiles_of(128) * 4 * 0.85 <= (double)tiles_of(64) ? 2 : 1;
-    // slices of the sum, float32: one, two or three full rounds of workgroups, whichever leaves fewest places empty, of at least 8
-    // stages each (one workgroup more than a round costs a round: 64 x 256 x 14 x 14 -> 256 in 14 slices 150, in 15 slices 212)
     const int64_t stages = (Q + KS - 1) / KS;
     int64_t slices = 1;
+    int MI = 1;
+    double least = 1e30;
     if (!half) {
-        const int64_t places = cus * (MI == 1 ? 4 : 2);
-        double best = 0.0;
-        for (int64_t r = 1; r <= 3; r++) {
-            int64_t n = r * places / tiles_of(64 * MI);
-            if (n > stages / 8) n = stages / 8;
-            if (n < 1) n = 1;
-            const double wgs = (double)(n * tiles_of(64 * MI)), full = wgs / (std::ceil(wgs / places) * places);
-            if (full > best + 0.05) { best = full; slices = n; }
-        }
+        // float32: a stage of a 64 x 64 tile takes 0.78 us with a compute unit to itself and 0.9 of that more for each further
+        // workgroup there (four fit), one of a 128 x 128 tile 2.55 us and 1.85 times that with two, which is all that fit; its
+        // first operands and its results 5 us more.  Slices that give every compute unit one, two, four or eight workgroups (128: one,
+        // two or four), down to a single stage each; more 64 x 64 tiles than compute units share less and take 1.25 times that.
+        // us, 64 x 64 / 128 x 128 tiles at their best slices: 64 x 64 x 7 x 7 1x1 -> 64 11.8 / 16.9 (one slice 84);
+        // 16 x 100 x 9 x 9 3x3 stride 2 -> 70 9.6 / 14.9; 16 x 256 x 14 x 14 1x1 -> 256 13.1 / 21.0; 64 x 64 x 28 x 28 3x3 -> 64
+        // 52.4 / 90; 64 x 128 x 28 x 28 3x3 -> 128 155 / 148; 64 x 256 x 14 x 14 3x3 -> 256 173 / 145; 64 x 512 x 7 x 7 3x3 -> 512
+        // 187 / 170.
+        for (int mi = 1; mi <= 2; mi++)
+            for (int64_t r = 1; r <= (mi == 1 ? 8 : 4); r *= 2) {
+                int64_t n = r * cus / tiles_of(64 * mi);
+                n = n < 1 ? 1 : n > stages ? stages : n;
+                const int64_t pn = (stages + n - 1) / n, nn = (stages + pn - 1) / pn;
+                const double wgs = std::ceil((double)(nn * tiles_of(64 * mi)) / cus);
+                const double st = mi == 1 ? 0.78 * (1.0 + 0.9 * (wgs - 1.0)) : 2.55 * (1.85 * std::floor(wgs / 2) + std::fmod(wgs, 2.0));
+                const double t = (double)pn * st * (mi == 1 && tiles_of(64) > cus ? 1.25 : 1.0) + (mi == 2 ? 5.0 : 0.0) +
+                                 (nn > 1 ? (nn > 16 ? 8.0 : 5.0) + (double)nn * numel(dw) * 8 / 5e6 : 0.0);
+                if (t < least) { least = t; MI = mi; slices = nn; }
+            }
     } else {
         // 16 bits: the loads bound a stage, 0.045 us for each that a thread issues on 128 x 128 tiles (four chunks of each operand)
-        // and 0.05 on 64 x 64 (two), 0.7 and 0.37 at least; a further workgroup on a compute unit adds 0.7 of that time, folding the
-        // slices 5 us and their traffic.  us at 64 images, tile / slices as found here, and others: 1024 x 14 x 14 1x1 -> 256
-        // 128 / 16 21.7 (64 / 4 24.8, 128 / 8 26.7, 128 / 48 32.1); 256 x 14 x 14 3x3 -> 256 128 / 14 60.7 (128 / 4 90.5, 64 / 12
+        // and 0.05 on 64 x 64 (two), 0.7 and 0.37 at least; a further workgroup on a compute unit adds 0.7 of that time.
+        // us at 64 images, tile / slices as found here, and others: 1024 x 14 x 14 1x1 -> 256 128 / 16 21.7 (64 / 4 24.8, 128 / 8 26.7, 128 / 48 32.1); 256 x 14 x 14 3x3 -> 256 128 / 14 60.7 (128 / 4 90.5, 64 / 12
         // 96.5); 256 x 28 x 28 1x1 -> 128 64 / 32 16.5 (128 / 64 20.3).
         const bool planes = R * S == 1 && p->stride_h == 1 && p->stride_w == 1 && p->pad_h == 0 && p->pad_w == 0;
         const int nl = P % 8 == 0 ? 1 : P % 4 == 0 ? 2 : P % 2 == 0 ? 4 : 8, loads = nl + (planes ? nl : 8);
-        double least = 1e30;
         for (int mi = 1; mi <= 2; mi++)
             for (int64_t n = 1; n <= 64 && (n == 1 || n <= stages / 4); n++) {
                 const int64_t pn = (stages + n - 1) / n, nn = (stages + pn - 1) / pn;

@@ -1101,3 +1101,19 @@ def test_routes_that_want_workspace_have_one_without(compile_only, monkeypatch):
         assert wgrad(dt)[0] == L.ERR_UNSUPPORTED
     monkeypatch.setenv("MJT_MOST_WORKSPACE", str(1 << 30))
     assert product(301, 203, 129, "bfloat16", 0, 0).startswith("mjt_gemm_mfma_")
+
+
+def test_float32_weight_gradient_of_a_few_tiles_is_cut_into_slices(compile_only, monkeypatch):
+    """One to thirty tiles and a sum of ten to a hundred stages: small tiles, and as many slices as there are compute units to run
+    them (they need workspace, so that a limit on it hands the call back), not one workgroup for the whole sum."""
+    lib = compile_only.load()
+    for n, c, h, k, r, s in ((64, 64, 7, 64, 1, 1), (16, 100, 9, 70, 3, 2), (4, 64, 14, 64, 3, 1), (18, 48, 14, 82, 1, 1), (16, 256, 14, 256, 1, 1)):
+        pad = r // 2
+        o = (h + 2 * pad - r) // s + 1
+        x, dy, dw = L.tensor(P, "float32", [n, c, h, h]), L.tensor(P, "float32", [n, k, o, o]), L.tensor(P, "float32", [k, c, r, r])
+        p = L.ConvParams(s, s, pad, pad, 1, 1)
+        monkeypatch.delenv("MJT_MOST_WORKSPACE", raising=False)
+        L.check(lib.mjt_conv2d_meta_wgrad(ctypes.byref(x), ctypes.byref(dy), ctypes.byref(dw), ctypes.byref(p)))
+        assert L.last_kernel().startswith("mjt_conv_wgrad_igemm_float32") and L.last_kernel().endswith("_64x64")
+        monkeypatch.setenv("MJT_MOST_WORKSPACE", "0")
+        assert lib.mjt_conv2d_meta_wgrad(ctypes.byref(x), ctypes.byref(dy), ctypes.byref(dw), ctypes.byref(p)) == L.ERR_UNSUPPORTED
