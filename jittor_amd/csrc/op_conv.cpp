@@ -84,9 +84,9 @@ struct DepthwiseShape {                       // see the kernel's header: staged
     bool flip;
 };
 struct DepthwisePlan {
-    int64_t TH, NTILE, PPW, VEC, STVEC;
+    int64_t TH, NTILE, PPW, VEC, STVEC, RS;
 };
-constexpr int kDwCW = 4, kDwRS = 4;           // a lane's strip: 4 columns (16 bytes of float32) x 4 rows
+constexpr int kDwCW = 4, kDwRS = 4;           // a lane's strip: 4 columns (16 bytes of float32) x at most 4 rows
 
 // Tile and vector widths, or false when the shape does not fit: at most 49 taps (they live in registers) and a window of
 // strip rows that fits LDS.  A workgroup stages whole planes while one is at most 40 KB (four workgroups or more then share a
@@ -102,6 +102,8 @@ bool depthwise_plan(const DepthwiseShape& g, int in_size, int strip_size, const 
     int64_t th = g.OH;
     while (th > kDwRS && bytes(th) > 40 * 1024) th = ((th + 1) / 2 + kDwRS - 1) / kDwRS * kDwRS;
     if (bytes(th) > 60 * 1024) return false;
+    // a plane or so a call: rows of it for as many workgroups (forward float32, 1 x 32 x 56 x 56 3x3: 3.4 / 2.9 us)
+    while (th > 8 && planes * ((g.OH + th - 1) / th) < 128) th = ((th + 1) / 2 + kDwRS - 1) / kDwRS * kDwRS;
     out->TH = th;
     out->NTILE = (g.OH + th - 1) / th;
     int64_t ppw = 1;
@@ -113,6 +115,10 @@ bool depthwise_plan(const DepthwiseShape& g, int in_size, int strip_size, const 
         if (ppw < 1) ppw = 1;
     }
     out->PPW = ppw;
+    // Few small planes leave most lanes without a strip of 4 rows, and each of those with all the work: shorter strips then (forward
+    // float32, us with 4 rows / as chosen: 16 x 128 x 7 x 7 5x5 4.1 / 2.9; 4 x 512 x 14 x 14 3x3 stride 2 3.4 / 3.2)
+    out->RS = kDwRS;
+    while (out->RS > 1 && ppw * ((th + out->RS - 1) / out->RS) * ncg < 48) out->RS /= 2;
     int64_t vec = 16 / in_size;
     while (vec > 1 && (g.W % vec || (uintptr_t)x % (size_t)(vec * in_size))) vec /= 2;
     out->VEC = vec;
@@ -125,7 +131,7 @@ bool depthwise_plan(const DepthwiseShape& g, int in_size, int strip_size, const 
 JitKernel* depthwise_kernel(int mode, const DepthwiseShape& g, const DepthwisePlan& q, int tin, int tout) {
     std::ostringstream key;
     key << "dw|" << mode << "|" << tin << "|" << tout << "|" << g.H << "|" << g.W << "|" << g.OH << "|" << g.OW << "|" << g.R << "|" << g.S << "|" << g.SH << "|" << g.SW
-        << "|" << g.PH << "|" << g.PW << "|" << g.DH << "|" << g.DW << "|" << g.UH << "|" << g.UW << "|" << g.K << "|" << g.mult << "|" << g.flip << "|" << q.TH << "|"
+        << "|" << g.PH << "|" << g.PW << "|" << g.DH << "|" << g.DW << "|" << g.UH << "|" << g.UW << "|" << g.K << "|" << g.mult << "|" << g.flip << "|" << q.TH << "|" << q.RS << "|"
         << q.PPW << "|" << q.VEC << "|" << q.STVEC;
     JitKernel* k = cached(key.str());
     if (k) return k;
@@ -139,7 +145,7 @@ JitKernel* depthwise_kernel(int mode, const DepthwiseShape& g, const DepthwisePl
         << "\n#define W_ " << g.W << "\n#define OH_ " << g.OH << "\n#define OW_ " << g.OW << "\n#define R_ " << g.R << "\n#define S_ " << g.S << "\n#define SH " << g.SH
         << "\n#define SW " << g.SW << "\n#define PH " << g.PH << "\n#define PW " << g.PW << "\n#define DH " << g.DH << "\n#define DW " << g.DW << "\n#define UH " << g.UH
         << "\n#define UW " << g.UW << "\n#define MULT " << g.mult << "\n#define K_ " << g.K << "\n#define FLIP " << (g.flip ? 1 : 0) << "\n#define TH " << q.TH
-        << "\n#define NTILE " << q.NTILE << "\n#define PPW " << q.PPW << "\n#define VEC " << q.VEC << "\n#define CW " << kDwCW << "\n#define RS " << kDwRS
+        << "\n#define NTILE " << q.NTILE << "\n#define PPW " << q.PPW << "\n#define VEC " << q.VEC << "\n#define CW " << kDwCW << "\n#define RS " << q.RS
         << "\n#define STVEC " << q.STVEC << "\n";
     src << embedded_source("prelude.h") << "\n" << embedded_source("conv_depthwise.h") << "\n";
     k = jit_get(src.str(), name.str());
@@ -648,9 +654,12 @@ static void conv_wgrad_direct(const mjt_tensor* x, const mjt_tensor* dy, const m
         const int64_t cus = ctx().dry_run || ctx().prop.multiProcessorCount <= 0 ? 256 : ctx().prop.multiProcessorCount;
         // slices of images: about four workgroups per compute unit, each of which has the planes of its next images on their way
         // while it sums; every slice ends in a fold of its lanes' sums and a row of partial results (us with the fold, float32, 3x3,
-        // 2 / 4 / 8 / 16 workgroups a unit: 32 x 128 x 56 x 56 34.6 / 26.5 / 30.6 / 32.7; 64 x 256 x 14 x 14 - / 12.4 / 15.8 / 18.5)
+        // 2 / 4 / 8 / 16 workgroups a unit: 32 x 128 x 56 x 56 34.6 / 26.5 / 30.6 / 32.7; 64 x 256 x 14 x 14 - / 12.4 / 15.8 / 18.5).
+        // Below 2048 positions a channel one slice, whose sums are the result of a float32 gradient (in slices / in one, 3x3:
+        // 4 x 512 x 7 x 7 8.4 / 4.9, 16 x 128 x 7 x 7 8.3 / 5.0, 64 x 256 x 7 x 7 stride 2 8.8 / 5.6).
         int64_t slices = (4 * cus + K - 1) / K;
         if (slices > N) slices = N;
+        if (N * OH * OW < 2048) slices = 1;
         const int64_t ips = (N + slices - 1) / slices;
         slices = (N + ips - 1) / ips;
         const DepthwiseShape g{H, W, OH, OW, R, S, p->stride_h, p->stride_w, p->pad_h, p->pad_w, p->dil_h, p->dil_w, 1, 1, K, K / G, false};

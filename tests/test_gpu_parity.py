@@ -1815,6 +1815,42 @@ def test_depthwise_conv_and_gradients(gpu, case):
         assert np.all(np.abs(got - ref) <= terms * 2.0 ** -24 * mag + eps * np.abs(ref) + 2.0 ** -24 * (out == "float16")), name
 
 
+@pytest.mark.parametrize("n,c,hw,rs,p", [
+    (5, 3, (7, 7), (3, 3), (1, 1, 1, 1, 1, 1)),          # strips of one row, a plane a workgroup
+    (2, 4, (10, 18), (5, 5), (1, 1, 2, 2, 1, 1)),        # strips of two rows
+    (3, 2, (9, 50), (3, 3), (1, 1, 1, 1, 1, 1)),         # tiles of rows of a small plane, the last one short
+    (1, 3, (57, 45), (5, 5), (2, 2, 2, 2, 1, 1)),        # ... strided, whose planes of the input gradient are tiled too
+    (1, 130, (12, 12), (3, 3), (1, 1, 1, 1, 1, 1)),      # just enough planes for whole ones
+    (700, 3, (2, 3), (3, 3), (1, 1, 1, 1, 1, 1)),        # planes of a strip or two, several a workgroup
+])
+def test_depthwise_strips_and_tiles_of_few_planes(gpu, n, c, hw, rs, p):
+    """Few or small planes: shorter strips, and rows of a plane as workgroups of their own.  Whole numbers whose sums are exact in
+    float32, so that the three directions equal float64 bit for bit."""
+    rng = np.random.default_rng(53)
+    (H, W), (R, S), (sh, sw, ph, pw, dh, dw_) = hw, rs, p
+    OH, OW = (H + 2 * ph - dh * (R - 1) - 1) // sh + 1, (W + 2 * pw - dw_ * (S - 1) - 1) // sw + 1
+    x, w, dy = (rng.integers(-4, 5, s).astype(np.float32) for s in ((n, c, H, W), (c, 1, R, S), (n, c, OH, OW)))
+    lib, cp = L.load(), L.ConvParams(*p)
+    vs = [jt.array(a) for a in (x, w, dy)] + [jt.zeros(s) + 7.0 for s in (dy.shape, x.shape, w.shape)]
+    jt.sync(vs, True)
+    tx, tw, td, ty, tdx, tdw = (L.tensor(v.raw_ptr(), "float32", v.shape) for v in vs)
+    L.check(lib.mjt_conv2d_meta_grouped(ctypes.byref(tx), ctypes.byref(tw), ctypes.byref(ty), ctypes.byref(cp), c))
+    assert "_depthwise" in L.last_kernel()
+    L.check(lib.mjt_conv2d_meta_dgrad_depthwise(ctypes.byref(td), ctypes.byref(tw), ctypes.byref(tdx), ctypes.byref(cp), c))
+    L.check(lib.mjt_conv2d_meta_wgrad_grouped(ctypes.byref(tx), ctypes.byref(td), ctypes.byref(tdw), ctypes.byref(cp), c))
+    xp = np.pad(x.astype(np.float64), ((0, 0), (0, 0), (ph, ph), (pw, pw)))
+    wy, wx, ww = np.zeros(dy.shape), np.zeros(xp.shape), np.zeros(w.shape)
+    for r in range(R):
+        for s in range(S):
+            at = np.s_[:, :, r * dh:r * dh + (OH - 1) * sh + 1:sh, s * dw_:s * dw_ + (OW - 1) * sw + 1:sw]
+            tap = w[:, 0, r, s][None, :, None, None]
+            wy += xp[at] * tap
+            wx[at] += dy * tap
+            ww[:, 0, r, s] = (dy * xp[at]).sum((0, 2, 3))
+    for v, want in zip(vs[3:], (wy, wx[:, :, ph:ph + H, pw:pw + W], ww)):
+        assert np.array_equal(v.numpy(), want)
+
+
 @pytest.mark.parametrize("dt", ["float32", "bfloat16"])
 @pytest.mark.parametrize("hw,p", [
     ((7, 7), (1, 1, 1, 1, 1, 1)),              # the last strip is one row and three columns short
