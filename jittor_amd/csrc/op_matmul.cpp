@@ -271,6 +271,10 @@ bool gemm_pixels(int in_dtype, int out_dtype, const void* A, const void* x, void
     const int tile = 128;
     const int64_t tm = (M + tile - 1) / tile, tn = (N + tile - 1) / tile;
     if (P % 8 == 0 ? (double)M < 0.7 * (double)(tm * tile) && tm * tn > cus : a_kcont && (K < 256 || tm * tn < 16)) return false;
+    // nor, forward on planes that the plain product takes too, for a sum of one stage, or one of less than eight on few tiles (us
+    // plain / this: 8 x 64 x 28 x 28 -> 64 3.7 / 6.3, 32 x 64 x 28 x 28 -> 384 10.0 / 12.5; 4 x 128 x 16 x 16 -> 512 4.8 / 6.4, 8 x 256 x 28 x 28
+    // -> 256 7.3 / 7.7, but 32 x 256 x 28 x 28 -> 256 12.3 / 11.2 and 8 x 512 x 16 x 16 -> 128 8.7 / 8.3).
+    if (P % 8 == 0 && a_kcont && (K < 128 || (K < 512 && tm * tn <= cus / 2))) return false;
     const int in = in_dtype == MJT_BFLOAT16 ? 0 : 1, out = out_dtype == MJT_BFLOAT16 ? 0 : out_dtype == MJT_FLOAT16 ? 1 : 2;
     const int nbuf = tm * tn > cus ? 2 : 4, wpe = nbuf == 2 ? 2 : 1;      // as for the plain product: two workgroups a unit, or a deeper ring
     std::ostringstream key;

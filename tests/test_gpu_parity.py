@@ -1088,6 +1088,27 @@ def test_conv_1x1_on_pieces_of_planes(gpu, dt, out, n, c, k, hw):
         assert np.all(np.abs(got - want) <= terms * 2.0 ** -24 * mag + eps * np.abs(want) + 2.0 ** -24 * (out == "float16"))
 
 
+@pytest.mark.parametrize("n,c,k,hw", [
+    (8, 64, 64, 16),         # a sum of one stage: the plain product
+    (5, 256, 136, 8),        # few tiles
+    (5, 448, 136, 8),        # just below eight stages
+    (3, 512, 136, 8),        # eight stages: the product over the planes' pieces
+    (70, 256, 136, 16),      # more tiles than compute units
+])
+def test_conv_1x1_on_whole_pieces_either_side_of_the_rule(gpu, n, c, k, hw):
+    """Planes that both products take: the plain one for short sums, the one over pieces for the others.  Whole numbers: exact in
+    bfloat16 operands and float32 sums."""
+    rng = np.random.default_rng(59)
+    x, w = rng.integers(-3, 4, (n, c, hw, hw)).astype(np.float32), rng.integers(-3, 4, (k, c, 1, 1)).astype(np.float32)
+    vx, vw, vy = jt.from_storage(_bf16(x), "bfloat16"), jt.from_storage(_bf16(w), "bfloat16"), jt.zeros([n, k, hw, hw]) + 7.0
+    jt.sync([vx, vw, vy], True)
+    tx, tw, ty = (L.tensor(v.raw_ptr(), v.dtype, v.shape) for v in (vx, vw, vy))
+    p = L.ConvParams(1, 1, 0, 0, 1, 1)
+    L.check(L.load().mjt_conv2d_meta(ctypes.byref(tx), ctypes.byref(tw), ctypes.byref(ty), ctypes.byref(p)))
+    assert L.last_kernel() == "conv_as_gemm"
+    assert np.array_equal(vy.numpy().reshape(n, k, -1), np.matmul(w[:, :, 0, 0].astype(np.float64), x.reshape(n, c, -1).astype(np.float64)))
+
+
 def test_conv_1x1_runs_as_a_product(gpu, monkeypatch):
     """A 1x1 convolution of stride 1 is handed to the matrix-product kernel although the MFMA convolution kernel would
     take it: always when a plane's rows are 16-byte multiples (the product then reads x as it lies, with tiles picked for
