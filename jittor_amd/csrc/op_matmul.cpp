@@ -334,18 +334,22 @@ void matmul_impl(const mjt_tensor* a, const mjt_tensor* b, const mjt_tensor* c, 
     // c[n,k] = a'[n,m] * b'[m,k]: rows n, columns k, sum over m
     const int64_t lda = a->shape[nd - 1], ldb = b->shape[nd - 1];
     // Rows that are no 16-byte multiples, or operands that do not begin at one, are what only the kernel without MFMAs takes as
-    // they lie, 0.14 us for every element of the sum however few tiles there are.  From a few million multiply-adds on, or one
-    // million and a sum of some length, they are copied into padded rows first, 6 to 9 us with the launches (us as they lie /
+    // they lie, 0.14 us for every element of the sum however few tiles there are.  They are copied into padded rows first, 6 to 9 us
+    // with the launches, where that is less: from a million multiply-adds on with a sum of 96 and more; from four million with one
+    // of 40 (one operand copied) or 48 (both); with a shorter one, down to 16, from 33 million or 67 million (us as they lie /
     // copied: bfloat16 a b^T 1000 x 500 x 900 111 / 15.8, a b 300 x 300 x 700 86.5 / 14.2, a b^T 100 x 1000 x 300 38.3 / 11.7;
-    // float32 a b^T 130 x 100 x 333 45.3 / 14.7).
+    // float32 a b^T 130 x 100 x 333 45.3 / 14.7, 4097 x 49 x 513 17.2 / 14.7; on the other side bfloat16 a^T b 1025 x 5 x 1025 5.6 / 10.3,
+    // a b^T 4097 x 17 x 65 6.4 / 9.5, a b 1025 x 33 x 1025 9.7 / 10.6; again worth it: a b 4097 x 33 x 513 12.0 / 11.1, with one copy
+    // 1001 x 33 x 2000 10.7 / 8.1).
     {
         const int esz = dtype_size(a->dtype);
         const int64_t ra = batch * a->shape[nd - 2], rb = batch * b->shape[nd - 2], epc = 16 / esz;
         const int64_t lap = (lda + epc - 1) / epc * epc, lbp = (ldb + epc - 1) / epc * epc;
         const bool pad_a = lda != lap || (uintptr_t)a->ptr % 16, pad_b = ldb != lbp || (uintptr_t)b->ptr % 16;
-        const int64_t most = int64_t(1) << 30;
+        const int64_t most = int64_t(1) << 30, copies = (pad_a ? 1 : 0) + (pad_b ? 1 : 0);
+        auto worth = [&](double macs) { return macs >= (double)(1 << (m >= 96 ? 20 : m >= 32 + 8 * copies ? 22 : 24 + copies)) && m >= 16; };
         if ((pad_a || pad_b) && a->dtype != MJT_FLOAT64 && !share_a && batch < 65536 && !getenv("MJT_GEMM_PLAIN") && !getenv("MJT_NO_FASTPATH") &&
-            (double)batch * n * k * m >= (double)(1 << (m >= 96 ? 20 : 22)) && (!pad_a || ra * lap * esz <= most) && (!pad_b || rb * lbp * esz <= most)) {
+            worth((double)batch * n * k * m) && (!pad_a || ra * lap * esz <= most) && (!pad_b || rb * lbp * esz <= most)) {
             const void* pa = pad_a ? padded_rows(0, a->ptr, a->dtype, ra, lda, lap) : a->ptr;
             const void* pb = !pad_b ? b->ptr : pa ? padded_rows(1, b->ptr, b->dtype, rb, ldb, lbp) : nullptr;
             const int64_t la = pad_a ? lap : lda, lb = pad_b ? lbp : ldb;

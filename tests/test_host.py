@@ -1117,3 +1117,23 @@ def test_float32_weight_gradient_of_a_few_tiles_is_cut_into_slices(compile_only,
         assert L.last_kernel().startswith("mjt_conv_wgrad_igemm_float32") and L.last_kernel().endswith("_64x64")
         monkeypatch.setenv("MJT_MOST_WORKSPACE", "0")
         assert lib.mjt_conv2d_meta_wgrad(ctypes.byref(x), ctypes.byref(dy), ctypes.byref(dw), ctypes.byref(p)) == L.ERR_UNSUPPORTED
+
+
+def test_products_of_unaligned_rows_are_copied_where_that_pays(compile_only):
+    """Short sums run as they lie, unless there is much of them: copying operands into padded rows costs more than such a sum."""
+    lib = compile_only.load()
+
+    def kernel(m, k, n, dt, ta, tb):
+        a, b = (L.tensor(P, dt, s) for s in ([k, m] if ta else [m, k], [n, k] if tb else [k, n]))
+        c = L.tensor(P, dt, [m, n])
+        L.check(lib.mjt_matmul(ctypes.byref(a), ctypes.byref(b), ctypes.byref(c), ta, tb))
+        return "plain" if L.last_kernel().startswith("mjt_gemm_plain_") else "copied" if L.last_kernel().startswith("mjt_gemm_mfma_") else L.last_kernel()
+
+    for dt in ("float32", "bfloat16", "float16"):
+        assert [kernel(m, k, n, dt, 0, 0) for m, k, n in (
+            (4097, 17, 65), (1025, 33, 1025), (1025, 47, 257), (20001, 15, 513)           # short sums; below 16 however many
+        )] == ["plain"] * 4
+        assert [kernel(m, k, n, dt, 0, 0) for m, k, n in (
+            (1025, 49, 1025), (4097, 33, 513), (4097, 17, 1025), (101, 97, 129), (129, 4097, 65)
+        )] == ["copied"] * 5
+        assert kernel(1001, 41, 504, dt, 0, 0) == "copied" and kernel(1001, 41, 505, dt, 0, 0) == "plain"      # one operand copied, both
