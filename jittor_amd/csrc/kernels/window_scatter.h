@@ -5,10 +5,11 @@
 // elements of y meet in the same element of x and atomic updates queue up behind each other.  Every element of x knows
 // which windows reach it, so one lane per element of x folds them itself: no atomics, no identity fill, one coalesced
 // store.  Row h is reached from output row oh through tap kh when oh*SH + kh*DH + CH == h; the candidates are the NCH
-// output rows at and below (h - CH) / SH (NCH = (KH-1)*DH / SH + 1), likewise for columns.
+// output rows at and below (h - CH) / SH (NCH = (KH-1)*DH / SH + 1), likewise for columns, where a lane looks at the NCU that
+// reach any of its elements (NCU = (VEC-1 + (KW-1)*DW) / SW + 1).
 //
 // Constants and fragments supplied by the host:
-//   TX, TACC, index_t, VEC, NPARAM, NB (batch axes), KH, KW, SH, SW, DH, DW, CH, CW, NCH, NCW
+//   TX, TACC, index_t, VEC, NPARAM, NB (batch axes), KH, KW, SH, SW, DH, DW, CH, CW, NCH, NCU
 //   MJT_RX_SETUP    xshapeK, yshapeK and strides (the names the index language uses)
 //   MJT_WS_BATCH    coordinates i0 .. i{NB-1} of plane number plane_
 //   I_OH, I_OW, I_KH, I_KW   the names of the four window coordinates (i{NB} .. i{NB+3})
@@ -20,6 +21,7 @@
 // the loads of a lane.
 
 struct Params { void* a[NPARAM]; };
+static_assert(NCH * NCU * VEC <= 40, "bodies that a lane unrolls");
 
 extern "C" __global__ __launch_bounds__(256) void ENTRY(Params p) {
     TX* __restrict__ xp = (TX*)p.a[0];
@@ -46,7 +48,6 @@ extern "C" __global__ __launch_bounds__(256) void ENTRY(Params p) {
     // windows in the same order, rows and columns falling.  (Elements outside, every element loaded its windows' values for
     // itself, 32 scattered loads a lane against 12: gradient of a 3x3 stride-2 maximum pooling of 32 x 64 x 112 x 112 float32
     // 111 -> 63 us, 4.1 TB/s of what it cannot do without.)
-    constexpr int NCU = (VEC - 1 + (KW - 1) * DW) / SW + 1;
     const index_t tw0_ = w0_ - (CW), tw1_ = tw0_ + (VEC - 1);
     const index_t ow_hi = tw1_ >= 0 ? tw1_ / SW : (index_t)-1;
     TACC acc_[VEC];

@@ -352,7 +352,11 @@ bool try_window_scatter(Plan* plan, int op, const mjt_tensor* x, const mjt_tenso
     // elements of a row of x per lane: one 16-byte store when the rows and the pointer allow it
     int wvec = std::min(8, 16 / dtype_size(x->dtype));
     while (wvec > 1 && (x->shape[XD - 1] % wvec != 0 || (uintptr_t)x->ptr % (size_t)(wvec * dtype_size(x->dtype)) != 0)) wvec /= 2;
-    while (wvec > 1 && NCH * NCW * wvec > 32) wvec /= 2;                  // at most 32 candidate windows per lane
+    // At most 40 bodies a lane: NCH x NCU windows for each of its elements (gradient of maximum / mean pooling in bfloat16, us at 8 / 4
+    // elements: 2x2 stride 2 of [64,128,64,64] 57.3 / 60.6, 17.9 / 22.6 (40 bodies at 8); 3x3 stride 2 of [32,64,112,112] 83.8 / 79.5,
+    // 27.6 / 27.0 (80); 4x4 stride 2 of [16,64,64,64] 25.7 / 23.4, 7.9 / 7.7 (96); 2x2 stride 1 of the same 37.8 / 32.9, 10.7 / 8.5 (144))
+    auto columns = [&](int v) { return (v - 1 + (KW - 1) * DW) / SW + 1; };      // of windows that reach v neighbouring elements
+    while (wvec > 1 && NCH * columns(wvec) * wvec > 40) wvec /= 2;
     // without a prologue the candidates are loads from y itself, far apart for neighbouring elements of x: more of them
     // per lane coalesce worse (3x3 stride-2 windows into [64,64,112,112]: 230 us with four elements per lane, 175 with one)
     if (!sp) wvec = 1;
@@ -394,7 +398,7 @@ bool try_window_scatter(Plan* plan, int op, const mjt_tensor* x, const mjt_tenso
         frag << "#define TX " << dtype_cname(x->dtype) << "\n#define TACC " << dtype_cname(ta) << "\n#define index_t " << IT << "\n#define VEC " << wvec
              << "\n#define NPARAM " << args.size() << "\n#define NB " << nb << "\n#define KH " << KH << "\n#define KW " << KW << "\n#define SH " << SH << "\n#define SW " << SW
              << "\n#define DH " << DH << "\n#define DW " << DW << "\n#define CH " << CH << "\n#define CW " << CW << "\n#define NCH " << NCH
-             << "\n#define NCW " << NCW << "\n";
+             << "\n#define NCU " << columns(wvec) << "\n";
         // extents as literals: the lane's coordinates come from divisions by them
         frag << "#define xshape_h " << x->shape[nb] << "\n#define xshape_w " << x->shape[nb + 1] << "\n#define yshape_oh " << y->shape[a_oh]
              << "\n#define yshape_ow " << y->shape[a_ow] << "\n";

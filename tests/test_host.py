@@ -1137,3 +1137,27 @@ def test_products_of_unaligned_rows_are_copied_where_that_pays(compile_only):
             (1025, 49, 1025), (4097, 33, 513), (4097, 17, 1025), (101, 97, 129), (129, 4097, 65)
         )] == ["copied"] * 5
         assert kernel(1001, 41, 504, dt, 0, 0) == "copied" and kernel(1001, 41, 505, dt, 0, 0) == "plain"      # one operand copied, both
+
+
+@pytest.mark.parametrize("k,s,p,dtype", [(2, 2, 0, "bfloat16"), (3, 2, 1, "bfloat16"), (3, 1, 1, "float32"), (4, 1, 0, "float32"),
+                                         (2, 1, 0, "float16"), (4, 2, 1, "bfloat16"), (5, 2, 2, "float32")])
+def test_window_gradients_bound_what_a_lane_unrolls(compile_only, monkeypatch, k, s, p, dtype):
+    """The windows that reach any of a lane's elements, for each of them: the kernel does not compile with more than 40 bodies."""
+    from jittor_amd import core, executor
+    nxt = [0x10000000]
+
+    def fake_alloc(nbytes):
+        size = core._Pool._round(nbytes)
+        nxt[0] += size
+        return nxt[0] - size, size
+
+    monkeypatch.setattr(core.pool, "alloc", fake_alloc)
+    monkeypatch.setattr(core.pool, "free", lambda ptr, size: None)
+    monkeypatch.setattr(L, "h2d", lambda ptr, arr: None)
+    x = jt.array(np.ones((2, 3, 32, 32), np.float32), dtype)
+    y = jt.pool(x, k, "maximum", p, s)
+    g = jt.array(np.ones(y.shape, np.float32), dtype)
+    jt.sync([x, y, g])
+    before = executor.stats["fused_scatters"]
+    jt.sync([jt.grad((jt.pool(x, k, "maximum", p, s) * g).sum(), x)])
+    assert executor.stats["fused_scatters"] == before + 1
