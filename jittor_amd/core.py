@@ -317,6 +317,7 @@ class Var:
     _consumers = None        # ops that take this Var as an input (weakly)
     _compile_options = None
     _stop_fuse = False
+    _SELDOM = ("_buf", "_host", "is_scalar", "_name", "_consumers", "_compile_options", "_stop_fuse")
 
     def __init__(self, shape, dtype, op=None, num=None):
         """With `num` given, `shape` is a list of the caller's making with that many elements and is taken over."""
@@ -541,7 +542,8 @@ class Var:
             self._split_off_value()
         name = self._name
         src = other._split_off_value()                 # `other` stays valid: it now reads this Var (and has a new id)
-        self.__dict__.clear()
+        for k in Var._SELDOM:                          # what the old value had and the new one may not; a program's own attributes stay
+            self.__dict__.pop(k, None)
         self.__dict__.update(src.__dict__)             # with the id of the value taken over
         self._name = name
         if self._op is not None:

@@ -1161,3 +1161,16 @@ def test_window_gradients_bound_what_a_lane_unrolls(compile_only, monkeypatch, k
     before = executor.stats["fused_scatters"]
     jt.sync([jt.grad((jt.pool(x, k, "maximum", p, s) * g).sum(), x)])
     assert executor.stats["fused_scatters"] == before + 1
+
+
+def test_assign_keeps_what_a_program_hung_on_the_var():
+    """assign() rebinds the value; attributes that are the program's own stay, and nothing of the old value lingers."""
+    w = jt.array(np.float32(3.0)).stop_fuse().name("w")
+    w.decay = 0.1
+    assert w.is_scalar
+    w.assign(jt.array(np.ones((2, 3), np.float32)))
+    assert w.decay == 0.1 and w.name() == "w" and w.shape == [2, 3] and not w.is_scalar and not w._stop_fuse
+    w.assign(w * 2.0)
+    assert w.decay == 0.1 and w.name() == "w" and w._host is None
+    w.assign(1.5)
+    assert w.decay == 0.1 and w.is_scalar and w.item() == 1.5
