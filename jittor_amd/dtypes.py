@@ -51,12 +51,14 @@ def is_int(name):
     return name in ("int8", "int16", "int32", "int64", "uint8", "uint16", "uint32", "uint64")
 
 
-def float_dtype(d, has_scalar=False, has_bf16=False):
-    """nano_string.h:205-215."""
+def float_dtype(d, has_scalar=False, has_bf16=False, reg=None):
+    """nano_string.h:205-215; `reg`: the register, if not as it is now."""
     if not has_scalar:
-        if amp_reg & AMP_PREFER32:
+        if reg is None:
+            reg = amp_reg
+        if reg & AMP_PREFER32:
             return "float32"
-        if amp_reg & AMP_PREFER16:
+        if reg & AMP_PREFER16:
             return "bfloat16" if has_bf16 else "float16"
     if d == 3:
         return "float64"
@@ -92,11 +94,11 @@ def binary_dtype_infer(op, x, y, xscalar=False, yscalar=False):
     if got is None:
         if len(_binary_dtypes) >= 4096:
             _binary_dtypes.clear()
-        got = _binary_dtypes[key] = _binary_dtype(op, x, y, xscalar, yscalar)
+        got = _binary_dtypes[key] = _binary_dtype(*key)
     return got
 
 
-def _binary_dtype(op, x, y, xscalar, yscalar):
+def _binary_dtype(op, x, y, xscalar, yscalar, reg):
     if op in BOOL_OPS:
         return "bool"
     d = max(dsize_(x), dsize_(y))
@@ -106,9 +108,9 @@ def _binary_dtype(op, x, y, xscalar, yscalar):
         d = dsize_(x)
     fl = op not in INT_OPS and (is_float(x) or is_float(y) or op in FLOAT_OPS)
     if fl:
-        if op in WHITE_OPS and not amp_reg & AMP_KEEP_WHITE:
+        if op in WHITE_OPS and not reg & AMP_KEEP_WHITE:
             return "float64" if d == 3 else "float32"
-        return float_dtype(d, xscalar or yscalar, "bfloat16" in (x, y))
+        return float_dtype(d, xscalar or yscalar, "bfloat16" in (x, y), reg)
     if x == "bool" and y == "bool":
         return "bool"
     return int_dtype(d)

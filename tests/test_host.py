@@ -1174,3 +1174,24 @@ def test_assign_keeps_what_a_program_hung_on_the_var():
     assert w.decay == 0.1 and w.name() == "w" and w._host is None
     w.assign(1.5)
     assert w.decay == 0.1 and w.is_scalar and w.item() == 1.5
+
+
+def test_dtype_rules_kept_are_those_of_one_register(monkeypatch):
+    """Another thread may set the register (a gradient does, op by op) while a rule is worked out: what is kept for a register is
+    what that register gives."""
+    from jittor_amd import dtypes as dt
+    monkeypatch.setattr(dt, "amp_reg", 0)
+    monkeypatch.setattr(dt, "_binary_dtypes", {})
+    size = dt.dsize_
+
+    def meanwhile(name):
+        dt.amp_reg = dt.AMP_PREFER16
+        return size(name)
+
+    monkeypatch.setattr(dt, "dsize_", meanwhile)
+    assert dt.binary_dtype_infer("add", "float32", "float32") == "float32"
+    monkeypatch.setattr(dt, "dsize_", size)
+    dt.amp_reg = 0
+    assert dt.binary_dtype_infer("add", "float32", "float32") == "float32"
+    dt.amp_reg = dt.AMP_PREFER16
+    assert dt.binary_dtype_infer("add", "float32", "float32") == "float16"
