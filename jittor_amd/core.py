@@ -62,20 +62,24 @@ class _Pool:
         self.free_blocks = {}          # size -> free blocks of it (one at least), the size used last at the end
         self.cached_bytes = 0
         self.limit = 8 << 30
-        self._lock = threading.RLock()
+        lock = threading.RLock()
+        self._enter, self._leave = lock.acquire, lock.release
         self._inside = False
         self._late = collections.deque()
 
     @staticmethod
     def _round(n):
-        n = max(int(n), 256)
-        if n <= (1 << 20):
+        if n <= 256:
+            return 256
+        n = int(n)
+        if n <= 1 << 20:
             return 1 << (n - 1).bit_length()
         return (n + (1 << 20) - 1) >> 20 << 20
 
     def alloc(self, nbytes):
         size = self._round(nbytes)
-        with self._lock:                                   # (nothing in here starts a collection)
+        self._enter()
+        try:                                               # (nothing in here starts a collection)
             lst = self.free_blocks.get(size)
             if lst is not None and not self._inside:
                 ptr = lst.pop()
@@ -83,6 +87,8 @@ class _Pool:
                     del self.free_blocks[size]
                 self.cached_bytes -= size
                 return ptr, size
+        finally:
+            self._leave()
         try:
             return _lib.alloc(size), size
         except MjtError:
@@ -92,34 +98,34 @@ class _Pool:
     def free(self, ptr, size):
         if _lib.device() is None:
             return
-        surplus = None
-        with self._lock:
-            if self._inside:
-                self._late.append((ptr, size))
-                return
-            self._inside = True
-            try:
+        self._enter()
+        if self._inside:
+            self._late.append((ptr, size))
+            self._leave()
+            return
+        self._inside = True
+        surplus = ()
+        try:
+            blocks = self.free_blocks
+            cached = self.cached_bytes + size
+            if cached > self.limit:
+                surplus = self._make_room(size)
                 cached = self.cached_bytes + size
-                if cached <= self.limit:
-                    lst = self.free_blocks.pop(size, None)
-                    if lst is None:
-                        lst = [ptr]
-                    else:
-                        lst.append(ptr)
-                    self.free_blocks[size] = lst
-                    self.cached_bytes = cached
+            if cached > self.limit:                        # nothing left but blocks of this size
+                surplus.append(ptr)
+            else:
+                if size in blocks:
+                    lst = blocks.pop(size)
+                    lst.append(ptr)
                 else:
-                    surplus = self._make_room(size)
-                    if self.cached_bytes + size <= self.limit:
-                        self.free_blocks.setdefault(size, []).append(ptr)
-                        self.cached_bytes += size
-                    else:
-                        surplus.append(ptr)
-            finally:
-                self._inside = False
-        if surplus is not None:
-            for old in surplus:
-                _lib.free(old)
+                    lst = [ptr]
+                blocks[size] = lst
+                self.cached_bytes = cached
+        finally:
+            self._inside = False
+            self._leave()
+        for old in surplus:
+            _lib.free(old)
         while self._late:
             try:
                 ptr, size = self._late.popleft()
@@ -143,14 +149,17 @@ class _Pool:
         return gone
 
     def release_all(self):
-        blocks = {}
-        with self._lock:
+        gone = []
+        self._enter()
+        try:
             if not self._inside:
-                blocks, self.free_blocks = self.free_blocks, blocks
+                while self.free_blocks:
+                    gone.extend(self.free_blocks.popitem()[1])
                 self.cached_bytes = 0
-        for lst in blocks.values():
-            for p in lst:
-                _lib.free(p)
+        finally:
+            self._leave()
+        for p in gone:
+            _lib.free(p)
 
 
 pool = _Pool()
