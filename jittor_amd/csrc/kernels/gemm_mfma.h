@@ -25,8 +25,8 @@
 // write 16 bytes.  A stage's tiles are loaded into registers one or two stages ahead and move to the other LDS buffer piece by
 // piece between the MFMAs of the current stage; its barrier and the first fragment reads of the next stage stand in front
 // of the last MFMAs.  (With these one after the other at the end of each stage the matrix cores stood still for 570 of the
-// 1700 cycles of a 64 x 64 float32 stage.  us before / now: float32 a b^T 2048 x 1024 x 1024 49.9 / 42, 2048^3 152 / 127,
-// a^T b 1024 x 1024 x 2048 69 / 55; bfloat16 2048 x 2048 x 2048 32.5 / 23, 12544 x 256 x 1024 18.8 / 14.)
+// 1700 cycles of a 64 x 64 float32 stage.  us before / now, in turn: float32 a b^T 2048 x 1024 x 1024 51 / 43,
+// 2048^3 163 / 143, a^T b 1024 x 1024 x 2048 72 / 58; bfloat16 2048 x 2048 x 2048 32.5 / 23, 12544 x 256 x 1024 18.8 / 14.)
 // The float32 MFMAs alone, 140 TFLOP/s measured, bound the large products.
 // float32 uses v_mfma_f32_32x32x2: a lane's 16-byte read holds 4 k of its row, which feed
 // four MFMAs (lanes 32..63 read the next chunk, so that an MFMA sums k and k + 4 of a

@@ -852,7 +852,9 @@ void conv_wgrad_impl(const mjt_tensor* x, const mjt_tensor* dy, const mjt_tensor
     // 16-bit operands: the product instead of the MFMA kernel for 1x1 taps without stride and padding, whose operands it reads as they
     // lie, and for maps that fill less than 0.6 of the kernel's chunks of 32 columns (us at 64 images, kernel / product:
     // 1024 x 14 x 14 1x1 -> 256 65.9 / 21.7; 256 x 28 x 28 1x1 -> 128 25.5 / 16.5; 256 x 14 x 14 3x3 -> 256 70.6 / 60.7;
-    // 128 x 28 x 28 3x3 -> 128 54.8 / 62.0 stays), from 2^27 multiply-adds on: below, either is a few us.
+    // 128 x 28 x 28 3x3 -> 128 54.8 / 62.0 stays), from 2^27 multiply-adds on.  Smaller layers stay on the kernel they had (16 x 64 x
+    // 14 x 14 3x3 -> 64 20.5 / 12.0, 8 x 256 x 14 x 14 1x1 -> 256 14.1 / 8.3, 4 x 64 x 6 x 6 3x3 -> 64 12.8 / 8.7); the front end sends the
+    // narrow ones of them to the product over chunks of images instead of here.
     const bool narrow = OW % 8 != 0 && (double)OW < 0.6 * 32 * (double)((OW + 31) / 32);
     const bool planes = R * S == 1 && p->stride_h == 1 && p->stride_w == 1 && p->pad_h == 0 && p->pad_w == 0;
     const bool large = (double)N * OH * OW * K * C * R * S >= (double)(1 << 27);

@@ -1210,9 +1210,11 @@ def _run_single(op):
         _, K, OH, OW = dy.shape
         R, S = out.shape[2], out.shape[3]
         # 16-bit maps narrower than 0.6 of the kernel's chunks of 32 columns: the product over chunks of images below for an odd number
-        # of pixels where the images make chunks (64 x 512 x 7 x 7 3x3: 61 us, 88 as the product that gathers its operands by elements)
-        # and below 2^27 multiply-adds, where either takes a few us; the gathering product for the others (64 x 256 x 14 x 14
-        # 3x3: 63 and 61, 1x1: 60 and 22)
+        # of pixels where the images make chunks, and below 2^27 multiply-adds; the product that gathers its operands (in the library,
+        # which chooses between it and the MFMA kernel for the others) otherwise.  us, chunks / gathering: 64 x 512 x 7 x 7 3x3 61 / 88,
+        # 64 x 256 x 15 x 15 3x3 97 / 114, 64 x 256 x 13 x 13 77 / 85, but 64 x 64 x 13 x 13 57 / 22; 64 x 256 x 14 x 14 3x3 63 / 61,
+        # 1x1 60 / 22.  The line at 2^27 keeps small layers on the route they had, 13 to 30 us where the gathering product takes
+        # 10 to 18 (8 x 32 x 14 x 14 3x3 -> 64 17.8 / 11.0, 8 x 128 x 7 x 7 3x3 13.7 / 16.3).
         half = x.dtype in ("bfloat16", "float16")
         narrow = OW % 8 != 0 and OW < 0.6 * 32 * -(-OW // 32)
         chunked = half and narrow and (OH * OW % 2 == 1 and N % 8 == 0 or N * OH * OW * K * C * R * S < 1 << 27)
