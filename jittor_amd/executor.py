@@ -718,15 +718,21 @@ def _replay(plan, ops):
         else:
             b = buf[k] = Buffer(d[1])
             base[k] = b.ptr
-    for k, src in plan.produce:
-        v = var[k]
-        if src >= 0:
-            v._buf = buf[src]
-        elif v._buf is None:
-            v._buf = Buffer(max(v.nbytes, 1))
-        buf[k] = v._buf
-        base[k] = v._buf.ptr
-    _launch(plan, base, [_scalar_value(var[k]) for _, _, k in plan.scalars])
+    try:
+        for k, src in plan.produce:
+            v = var[k]
+            if src >= 0:
+                v._buf = buf[src]
+            elif v._buf is None:
+                v._buf = Buffer(max(v.nbytes, 1))
+            buf[k] = v._buf
+            base[k] = v._buf.ptr
+        _launch(plan, base, [_scalar_value(var[k]) for _, _, k in plan.scalars])
+    except BaseException:
+        for k, _ in plan.produce:                              # none is computed, and a buffer would say that it is
+            if var[k]._op is not None:
+                var[k]._buf = None
+        raise
     for key, d in plan.stats:
         stats[key] += d
     for i, clear_inputs in plan.cleared:
@@ -757,7 +763,15 @@ def run_sync(targets, device_sync=False):
             elif plan is False:
                 _execute(ops, target_ids)
             else:
-                _replay(plan, ops)
+                try:
+                    _replay(plan, ops)
+                except _lib.MjtError as e:
+                    if e.code != _lib.ERR_UNSUPPORTED:
+                        raise
+                    # a call that is handed back now was not when the plan was made (no workspace left, another MJT_ variable):
+                    # the graph is worked out anew
+                    _plans.pop(sig, None)
+                    _capture(ops, target_ids, sig)
         for t in targets:
             t._device_ptr()
     if device_sync:

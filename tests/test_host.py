@@ -1195,3 +1195,69 @@ def test_dtype_rules_kept_are_those_of_one_register(monkeypatch):
     assert dt.binary_dtype_infer("add", "float32", "float32") == "float32"
     dt.amp_reg = dt.AMP_PREFER16
     assert dt.binary_dtype_infer("add", "float32", "float32") == "float16"
+
+
+@pytest.fixture
+def fake_buffers(compile_only, monkeypatch):
+    """The front end on made-up device addresses, nothing launched; no plans from before."""
+    from jittor_amd import core, executor
+    nxt = [0x10000000]
+
+    def fake_alloc(nbytes):
+        size = core._Pool._round(nbytes)
+        nxt[0] += size
+        return nxt[0] - size, size
+
+    monkeypatch.setattr(core.pool, "alloc", fake_alloc)
+    monkeypatch.setattr(core.pool, "free", lambda ptr, size: None)
+    monkeypatch.setattr(L, "h2d", lambda ptr, arr: None)
+    monkeypatch.setitem(executor.flags, "enable_replay", True)
+    executor._plans.clear()
+    return executor
+
+
+@pytest.mark.parametrize("groups,by,variable", [(1, "w", "MJT_NO_FASTPATH"), (1, "w", "MJT_MOST_WORKSPACE"), (32, "x", "MJT_NO_FASTPATH")])
+def test_replayed_graph_whose_call_is_handed_back_is_worked_out_anew(fake_buffers, monkeypatch, groups, by, variable):
+    """A route that was there when the plan was made and is not any more: the graph takes the route without it, as on a first
+    execution, replayed by its calls or by recorded launches."""
+    stats = fake_buffers.stats
+
+    def step():
+        v = {"x": jt.array(np.ones((64, 32, 15, 13), np.float32)), "w": jt.array(np.ones((32, 32 // groups, 3, 3), np.float32))}
+        g = jt.array(np.ones((64, 32, 15, 13), np.float32))
+        y = jt.nn.conv2d(v["x"], v["w"], padding=1, groups=groups)
+        out = jt.grad((y * g).sum(), v[by])
+        jt.sync([out])
+        return out
+
+    for warm in (2, 4):
+        for _ in range(warm):
+            step()
+        before = dict(stats)
+        monkeypatch.setenv(variable, "1")
+        assert step()._buf is not None
+        assert stats["plans"] == before["plans"] + 1 and stats["replays"] == before["replays"]
+        step()
+        assert stats["replays"] == before["replays"] + 1
+        monkeypatch.delenv(variable)
+        fake_buffers._plans.clear()
+
+
+def test_replay_that_fails_leaves_its_results_uncomputed(fake_buffers):
+    """An error in the middle of a replay: the results have no buffer that would pass for computed, and the next attempt computes them."""
+    def graph():
+        x = jt.array(np.ones((64, 48), np.float32))
+        return [x.sum([0]), (x * x).sum([1])]
+
+    for _ in range(2):
+        jt.sync(graph())
+    plan = next(iter(fake_buffers._plans.values()))
+    outs = graph()
+    plan.calls.append((lambda: L.ERR_UNSUPPORTED - 1, ()))             # some other error
+    plan.native = False
+    with pytest.raises(L.MjtError):
+        jt.sync(outs)
+    assert all(v._buf is None and v._op is not None for v in outs)
+    plan.calls.pop()
+    jt.sync(outs)
+    assert all(v._buf is not None and v._op is None for v in outs)
