@@ -521,7 +521,7 @@ def _libh():
 
 def _signature(ops, target_ids):
     """Hashable description of everything the execution of `ops` depends on besides the data, or None."""
-    pos, leaf, parts = {}, {}, []
+    pos, leaf, bufs, parts = {}, {}, {}, []
     for i, op in enumerate(ops):
         sig = op.sig()
         out = op.out
@@ -537,7 +537,10 @@ def _signature(ops, target_ids):
             l = leaf.get(uid)
             if l is None:
                 l = leaf[uid] = len(leaf)
-                ins.append((l, tuple(u.shape), u.dtype, u._op is None, u._buf is None, u._host is not None, u._stop_fuse))
+                b = u._buf
+                # (inputs that share a buffer, as a reshape does, are told apart from others: a plan knows a result that is an
+                # input's own memory by the buffer)
+                ins.append((l, tuple(u.shape), u.dtype, u._op is None, b if b is None else bufs.setdefault(id(b), l), u._host is not None, u._stop_fuse))
             else:
                 ins.append(-1 - l)
         uid = out.id

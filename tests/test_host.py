@@ -1261,3 +1261,22 @@ def test_replay_that_fails_leaves_its_results_uncomputed(fake_buffers):
     plan.calls.pop()
     jt.sync(outs)
     assert all(v._buf is not None and v._op is None for v in outs)
+
+
+@pytest.mark.parametrize("shared_first", [True, False])
+def test_replayed_result_is_the_memory_of_its_own_input(fake_buffers, shared_first):
+    """A reshape of one input, replayed after an execution in which the two inputs were one buffer (and the other way round): the
+    result is that input's memory, not the other's."""
+    def step(shared):
+        a = jt.array(np.ones((8, 4), np.float32)) + 1.0
+        b = a.reshape([32]) if shared else jt.array(np.ones(32, np.float32)) + 2.0
+        jt.sync([a])
+        jt.sync([b])
+        assert (b._buf is a._buf) == shared
+        y, z = b.reshape([4, 8]), a * 2.0
+        jt.sync([y, z])
+        return b, y
+
+    for shared in (shared_first, shared_first, not shared_first, not shared_first, shared_first):
+        b, y = step(shared)
+        assert y._buf is b._buf
