@@ -521,7 +521,7 @@ def _libh():
 
 def _signature(ops, target_ids):
     """Hashable description of everything the execution of `ops` depends on besides the data, or None."""
-    pos, leaf, bufs, parts = {}, {}, {}, []
+    pos, leaf, parts = {}, {}, []
     for i, op in enumerate(ops):
         sig = op.sig()
         out = op.out
@@ -537,10 +537,7 @@ def _signature(ops, target_ids):
             l = leaf.get(uid)
             if l is None:
                 l = leaf[uid] = len(leaf)
-                b = u._buf
-                # (inputs that share a buffer, as a reshape does, are told apart from others: a plan knows a result that is an
-                # input's own memory by the buffer)
-                ins.append((l, tuple(u.shape), u.dtype, u._op is None, b if b is None else bufs.setdefault(id(b), l), u._host is not None, u._stop_fuse))
+                ins.append((l, tuple(u.shape), u.dtype, u._op is None, u._buf is None, u._host is not None, u._stop_fuse))
             else:
                 ins.append(-1 - l)
         uid = out.id
@@ -571,6 +568,7 @@ def _capture(ops, target_ids, sig):
         slots.append(("out", i))
         held.append(op.out)
     had_inputs = [bool(op.inputs) for op in ops]
+    first_input = [op.inputs[0] if op.inputs else None for op in ops]
     before = dict(stats)
     cap = _cap = _Capture(_lib.ensure_init())
     try:
@@ -602,11 +600,13 @@ def _capture(ops, target_ids, sig):
             _plans[sig] = False
             return
         plan.scalars.append((arr, idx, k))
-    # who owns which buffer: inputs first, then the vars made on the way, then the results in the order of the ops
-    owner, produce = {}, []
+    # who owns which buffer: inputs first, then the vars made on the way, then the results in the order of the ops.  Inputs that are
+    # one buffer now may be two the next time: a result that is its op's input's own memory, a reshape's, belongs to that input
+    owner, produce, several = {}, [], set()
     for k, d in enumerate(slots):
         if d[0] != "out" and held[k]._buf is not None:
-            owner.setdefault(id(held[k]._buf), k)
+            if owner.setdefault(id(held[k]._buf), k) != k and d[0] == "in":
+                several.add(id(held[k]._buf))
     for k, d in enumerate(slots):
         if d[0] != "out":
             continue
@@ -614,6 +614,12 @@ def _capture(ops, target_ids, sig):
         if buf is None:
             continue
         src = owner.get(id(buf))
+        if id(buf) in several:
+            own = first_input[d[1]]
+            if own is None or own._buf is not buf:             # (whose memory it is cannot be told)
+                _plans[sig] = False
+                return
+            src = slot_of[id(own)]
         if src is None:
             owner[id(buf)] = k
             produce.append((k, -1))

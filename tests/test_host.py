@@ -1264,7 +1264,8 @@ def test_replay_that_fails_leaves_its_results_uncomputed(fake_buffers):
 
 
 @pytest.mark.parametrize("shared_first", [True, False])
-def test_replayed_result_is_the_memory_of_its_own_input(fake_buffers, shared_first):
+@pytest.mark.parametrize("twice", [False, True])
+def test_replayed_result_is_the_memory_of_its_own_input(fake_buffers, shared_first, twice):
     """A reshape of one input, replayed after an execution in which the two inputs were one buffer (and the other way round): the
     result is that input's memory, not the other's."""
     def step(shared):
@@ -1274,9 +1275,13 @@ def test_replayed_result_is_the_memory_of_its_own_input(fake_buffers, shared_fir
         jt.sync([b])
         assert (b._buf is a._buf) == shared
         y, z = b.reshape([4, 8]), a * 2.0
+        if twice:
+            y = y.reshape([2, 16])
         jt.sync([y, z])
         return b, y
 
     for shared in (shared_first, shared_first, not shared_first, not shared_first, shared_first):
+        replays = fake_buffers.stats["replays"]
         b, y = step(shared)
         assert y._buf is b._buf
+    assert fake_buffers.stats["replays"] > replays + 1
