@@ -622,9 +622,9 @@ def _capture(ops, target_ids, sig):
             src = slot_of[id(own)]
         if src is None:
             owner[id(buf)] = k
-            produce.append((k, -1))
+            produce.append((k, -1, max(held[k].nbytes, 1)))
         else:
-            produce.append((k, src))
+            produce.append((k, src, 0))
             needs_ptr.add(src)
     plan.slots, plan.needs_ptr, plan.produce, plan.calls = slots, needs_ptr, produce, cap.calls
     plan.seen, plan.native = 0, None
@@ -728,17 +728,16 @@ def _replay(plan, ops):
             b = buf[k] = Buffer(d[1])
             base[k] = b.ptr
     try:
-        for k, src in plan.produce:
+        for k, src, nbytes in plan.produce:
             v = var[k]
-            if src >= 0:
-                v._buf = buf[src]
-            elif v._buf is None:
-                v._buf = Buffer(max(v.nbytes, 1))
-            buf[k] = v._buf
-            base[k] = v._buf.ptr
+            b = buf[src] if src >= 0 else v._buf
+            if b is None:
+                b = Buffer(nbytes)
+            v._buf = buf[k] = b
+            base[k] = b.ptr
         _launch(plan, base, [_scalar_value(var[k]) for _, _, k in plan.scalars])
     except BaseException:
-        for k, _ in plan.produce:                              # none is computed, and a buffer would say that it is
+        for k, _, _ in plan.produce:                           # none is computed, and a buffer would say that it is
             if var[k]._op is not None:
                 var[k]._buf = None
         raise
