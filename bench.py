@@ -5,10 +5,10 @@
 
 A step is one pass of one workload's hot path (one C-ABI call = one kernel, or
 the launches of the scatter) over synthetic input that is already resident in
-HBM.  The headline line is BASELINE.json's configs[1] (C2, the im2col reindex);
+HBM.  The headline line is C2, the im2col reindex (32 x 64 x 56 x 56, 3x3);
 every configuration is reported inside the same JSON line under "workloads",
 and its fraction of the roofline beside the headline under "fractions" with
-the number of configurations that meet north_star's targets ("targets_met").
+the number of configurations that meet their targets ("targets_met").
 Each workload rotates over buffer sets whose inputs alone exceed the 256 MB
 memory-side cache, so the rates are HBM rates.  A block of exactly --steps
 launches is timed between two HIP events; blocks are repeated until 0.2 s of
@@ -721,7 +721,7 @@ def main():
             results[name] = {"error": str(err)}
         print("[bench] %s: %s" % (name, json.dumps(results[name])), file=sys.stderr, flush=True)
     head = results.get("C2") or next(iter(results.values()))
-    # every configuration's fraction of its roofline beside the headline, against north_star's targets
+    # every configuration's fraction of its roofline beside the headline, against its target
     # (0.70 of peak HBM bandwidth for C1-C4, 0.50 of peak MFMA throughput for C5)
     targets = {"C1": 0.70, "C2": 0.70, "C3add": 0.70, "C3max": 0.70, "C4": 0.70, "C5": 0.50}
     fractions = {k: results[k]["roofline"]["frac"] for k in targets if k in results and "roofline" in results[k]}

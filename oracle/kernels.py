@@ -1,6 +1,6 @@
 """ctypes loader for oracle/_build/liboracle_kernels.so.  TEST INFRASTRUCTURE
 ONLY (see oracle_kernels.cc): the C++ restatement of the reference's CPU
-kernels for the benchmark configurations, used as checker and as the timed CPU
+kernels for the benchmark configurations, used as oracle and as the timed CPU
 baseline."""
 import ctypes
 import os
