@@ -75,8 +75,18 @@ typedef unsigned short TIN;
 #ifndef SLICED
 #define SLICED 0                 // 1: workgroup (tile, slice) sums stages slice * a[9] .. of K into its own float32 C, a[11] apart
 #endif
+// A convolution's sum is known here, and images have few channels: a single stage takes one buffer, so that eight workgroups share a
+// compute unit instead of four, two stages one register set, and the loop of whole stages is left out where it would not be entered.
+// (us with the general form / this: bfloat16 32 x 3 x 224 x 224 3x3 stride 2 -> 32 43.3 / 30.5, 32 x 3 x 112 x 112 7x7 stride 2 -> 64
+// 28.9 / 23.7; float16 43 x 1 x 56 x 56 5x5 -> 16 16.8 / 13.6, 12 x 31 x 14 x 14 2x2 -> 224 10.7 / 10.2, 16 x 100 x 9 x 9 3x3 stride 2 -> 70
+// 25.8 / 21.3; float32 32 x 3 x 64 x 64 3x3 -> 96 27.0 / 23.6, 64 x 64 x 56 x 56 3x3 -> 64 177 / 174.)
+#if CONV == 1
+#define STAGES ((C_ * R_ * S_ + KS - 1) / KS)
+#else
+#define STAGES 0
+#endif
 #ifndef NBUF
-#define NBUF 2                   // staging buffers: 2, or 1 for a product of a single stage (K <= KS)
+#define NBUF (CONV == 1 && STAGES == 1 ? 1 : 2)      // staging buffers: 2, or 1 for a product of a single stage (K <= KS)
 #endif
 
 typedef float mjt_f32x16 __attribute__((ext_vector_type(16)));
@@ -407,7 +417,12 @@ struct mjt_wg_x {
 #endif
 
 extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
-    const int M = (int)(long long)p.a[3], N = (int)(long long)p.a[4], K = (int)(long long)p.a[5];
+    const int M = (int)(long long)p.a[3], N = (int)(long long)p.a[4];
+#if CONV == 1
+    constexpr int K = C_ * R_ * S_;
+#else
+    const int K = (int)(long long)p.a[5];
+#endif
     const long long lda = (long long)p.a[6], ldb = (long long)p.a[7], ldc = (long long)p.a[8];
 #if CONV == 2
     const TIN* __restrict__ A = (const TIN*)p.a[0];
@@ -469,7 +484,7 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
     // on 64 x 64 57.7 / 55.4 / 57.1, 2048^3 on 128 x 128 133 / 127 / -).  Larger tiles have no registers to spare.
     // The gathering operands hold more registers: two sets on 64 x 64 tiles only (64 x 512 x 7 x 7 3x3 -> 512 247 / 218;
     // 64 x 128 x 28 x 28 3x3 -> 128 on 128 x 128 186 / 194).
-    constexpr int NSET = NBUF > 1 && MI * NI <= (CONV ? 1 : 4) ? 2 : 1;
+    constexpr int NSET = NBUF > 1 && STAGES != 2 && MI * NI <= (CONV ? 1 : 4) ? 2 : 1;
 #if CONV == 2
     const int all_stages = (K + KS - 1) / KS;
     const int nstages = all_stages - first_stage < per_slice ? all_stages - first_stage : per_slice;
@@ -617,9 +632,16 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
     };
     const int nstages_full = CONV == 2 ? nstages : K / KS - first_stage < nstages ? K / KS - first_stage : nstages;     // (the weight gradient's operands read zeros beyond K by themselves)
     int s0 = 0;
-    if constexpr (NBUF > 1)
+#if CONV == 1
+    constexpr bool LONG = K / KS > 2 * NSET;
+#else
+    constexpr bool LONG = NBUF > 1;
+#endif
+    if constexpr (LONG)
+#pragma unroll 1
         for (; s0 + 2 * NSET < nstages_full; s0 += NSET)
             mjt_static_for<0, NSET>([&](auto parc) { run_stage(parc, mjt_ic<1>(), s0 + decltype(parc)::v); });
+#pragma unroll 1
     for (; s0 < nstages; s0 += NSET)
         mjt_static_for<0, NSET>([&](auto parc) {
             if (s0 + decltype(parc)::v < nstages) run_stage(parc, mjt_ic<0>(), s0 + decltype(parc)::v);

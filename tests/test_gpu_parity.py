@@ -1088,6 +1088,21 @@ def test_conv_1x1_on_pieces_of_planes(gpu, dt, out, n, c, k, hw):
         assert np.all(np.abs(got - want) <= terms * 2.0 ** -24 * mag + eps * np.abs(want) + 2.0 ** -24 * (out == "float16"))
 
 
+@pytest.mark.parametrize("dt", ["float32", "bfloat16", "float16"])
+@pytest.mark.parametrize("n,k,tile", [(6, 70, {"64x64"}), (17, 130, {"128x64", "128x128"})])
+def test_conv_whose_sum_is_a_few_stages(gpu, dt, n, k, tile):
+    """The gathering product at the edges of its stages of 32 (float32) or 64 elements: one stage, which has a single buffer, two, and
+    the first sums that enter the loop of whole stages.  Whole numbers whose sums are exact in float32."""
+    rng = np.random.default_rng(61)
+    for c in (15, 16, 17, 31, 32, 33, 48, 49, 63, 64, 65, 96, 97, 129, 200):
+        x, w = rng.integers(-3, 4, (n, c, 29, 37)).astype(np.float32), rng.integers(-3, 4, (k, c, 1, 2)).astype(np.float32)
+        narrow = (lambda a: a) if dt == "float32" else _bf16 if dt == "bfloat16" else (lambda a: a.astype(np.float16))
+        got, kern = _conv_call(narrow(x), narrow(w), (1, 1, 0, 0, 1, 1), in_dtype=dt)
+        assert kern.startswith("mjt_conv_igemm_" + dt) and kern.split("_")[-1] in tile, kern
+        want = sum(np.matmul(w[:, :, 0, s].astype(np.float64), x[:, :, :, s:36 + s].astype(np.float64).reshape(n, c, -1)) for s in (0, 1))
+        assert np.array_equal(got.reshape(n, k, -1), want), (c, kern)
+
+
 @pytest.mark.parametrize("n,c,k,hw", [
     (8, 64, 64, 16),         # a sum of one stage: the plain product
     (5, 256, 136, 8),        # few tiles
