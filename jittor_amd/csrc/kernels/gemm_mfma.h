@@ -454,7 +454,10 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
 
     // Tile order: panels of 4 tile rows, inside a panel column by column.  Workgroups go round-robin over the
     // 8 XCDs, so workgroup id takes tile (id % 8) * per_xcd + id / 8: every XCD works on a compact run of
-    // tiles and finds the operand rows and columns it shares in its own L2.
+    // tiles and finds the operand rows and columns it shares in its own L2.  The next matrix of a batch, or slice of a sum, starts
+    // one XCD further on unless its tiles spread evenly: with fewer than eight, all would otherwise run on the same few (us, a b^T,
+    // before / so: float32 256 x 64 x 64 x 64 20.4 / 10.6, 512 x 32 x 128 x 64 66 / 31, 100 x 200 x 200 x 128 a b 107 / 52.5; bfloat16 the
+    // same 8.7 / 7.2, 18.1 / 10.2, 44.3 / 21.6).
     const int tiles_m = (M + TM - 1) / TM, tiles_n = (N + TN - 1) / TN;
     const int tiles = tiles_m * tiles_n;
     int L = blockIdx.x;
@@ -463,7 +466,8 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
 #else
     {
         const int per_xcd = (tiles + 7) / 8;
-        L = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+        const unsigned turn = tiles % 8 ? blockIdx.y : 0;
+        L = ((blockIdx.x + turn) & 7) * per_xcd + (blockIdx.x >> 3);
         if (L >= tiles || (blockIdx.x >> 3) >= per_xcd) return;
     }
 #endif

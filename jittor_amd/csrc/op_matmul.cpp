@@ -10,6 +10,7 @@
 // (everything else, float64 included).  Float accumulation for every input
 // type (double for float64).
 #include "common.h"
+#include <algorithm>
 #include <cmath>
 #include <mutex>
 #include <unordered_map>
@@ -348,8 +349,17 @@ void matmul_impl(const mjt_tensor* a, const mjt_tensor* b, const mjt_tensor* c, 
         const bool pad_a = lda != lap || (uintptr_t)a->ptr % 16, pad_b = ldb != lbp || (uintptr_t)b->ptr % 16;
         const int64_t most = int64_t(1) << 30, copies = (pad_a ? 1 : 0) + (pad_b ? 1 : 0);
         auto worth = [&](double macs) { return macs >= (double)(1 << (m >= 96 ? 20 : m >= 32 + 8 * copies ? 22 : 24 + copies)) && m >= 16; };
+        // Nor in a batch of small matrices, whose many rows share little work: a copied element takes 4e-6 us (16 bits 2.2e-6),
+        // every element of the sum gives back 0.09 us for each round of 64 x 64 tiles, of which the launches take 3.5 to 5 us (us as
+        // they lie / copied, a b^T: float32 256 x 50 x 50 x 63 11.1 / 18.0, x 111 18.5 / 26.1; 17 x 816 x 48 x 63 10.9 / 13.9, x 131
+        // 22.2 / 21.5; 8 x 512 x 512 x 41 12.4 / 14.6; bfloat16 256 x 50 x 50 x 63 9.6 / 13.7, x 131 18.9 / 16.9; 17 x 816 x 48 x 71
+        // 11.1 / 12.8, x 97 14.9 / 13.6).
+        const int64_t units = ctxt.dry_run || ctxt.prop.multiProcessorCount <= 0 ? 256 : ctxt.prop.multiProcessorCount;
+        const double rounds = std::max(1.0, 0.5 + (double)(batch * ((n + 63) / 64) * ((k + 63) / 64)) / (double)(2 * units));
+        const double copied = (double)((pad_a ? ra * lap : 0) + (pad_b ? rb * lbp : 0)) * (esz == 2 ? 2.2e-6 : 4e-6);
+        const bool pays = batch == 1 || ((m >= 48 || copies == 1) && copied <= 0.09 * (double)m * rounds - (esz == 2 ? 5.0 : 3.5) + (copies == 1 ? 2.5 : 0.0));
         if ((pad_a || pad_b) && a->dtype != MJT_FLOAT64 && !share_a && batch < 65536 && !getenv("MJT_GEMM_PLAIN") && !getenv("MJT_NO_FASTPATH") &&
-            worth((double)batch * n * k * m) && (!pad_a || ra * lap * esz <= most) && (!pad_b || rb * lbp * esz <= most)) {
+            worth((double)batch * n * k * m) && pays && (!pad_a || ra * lap * esz <= most) && (!pad_b || rb * lbp * esz <= most)) {
             const void* pa = pad_a ? padded_rows(0, a->ptr, a->dtype, ra, lda, lap) : a->ptr;
             const void* pb = !pad_b ? b->ptr : pa ? padded_rows(1, b->ptr, b->dtype, rb, ldb, lbp) : nullptr;
             const int64_t la = pad_a ? lap : lda, lb = pad_b ? lbp : ldb;

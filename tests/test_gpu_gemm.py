@@ -283,3 +283,17 @@ def test_gemm_odd_rows_of_a_transposed_operand(gpu, dt, tb, M, K, N):
     """a^T b with an odd number of result rows on the kernel that copies its operands into LDS: the last element of a, half of the
     last dword in range, belongs to the last row's sum."""
     assert "_direct" in _run(L.load(), dt, "float32", M, K, N, 1, tb, seed=M + K)
+
+
+@pytest.mark.parametrize("dt", ["float32", "bfloat16", "float16"])
+@pytest.mark.parametrize("batch,M,N,K", [(1, 40, 40, 64), (3, 64, 128, 96), (8, 65, 64, 64), (17, 200, 70, 128), (21, 130, 257, 192), (9, 640, 640, 64), (300, 24, 40, 72)])
+@pytest.mark.parametrize("ta,tb", [(0, 1), (1, 0)])
+def test_gemm_batches_of_few_tiles(gpu, dt, batch, M, N, K, ta, tb):
+    """The tiles of a batch's matrices begin one XCD further on with each: every tile of every matrix is made, with less than eight
+    tiles a matrix, with eight and with more, on the general kernel and on the one that copies its operands into LDS."""
+    M, N = (M, N) if dt == "float32" else ((M + 7) // 8 * 8, (N + 7) // 8 * 8)
+    _run(L.load(), dt, dt, M, K, N, ta, tb, batch=(batch,), seed=M + K)
+    if dt != "float32" and K % 64 == 0:
+        with pytest.MonkeyPatch.context() as m:
+            m.setenv("MJT_GEMM_DMA", "128")
+            assert "_direct" in _run(L.load(), dt, dt, M, K, N, ta, tb, batch=(batch,), seed=M + K)

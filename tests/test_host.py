@@ -1139,6 +1139,22 @@ def test_products_of_unaligned_rows_are_copied_where_that_pays(compile_only):
         assert kernel(1001, 41, 504, dt, 0, 0) == "copied" and kernel(1001, 41, 505, dt, 0, 0) == "plain"      # one operand copied, both
 
 
+def test_batches_of_small_unaligned_products_run_as_they_lie(compile_only):
+    """Many rows that share little work: copying them into padded rows costs more than the matrix cores save."""
+    lib = compile_only.load()
+
+    def copied(batch, m, k, n, dt):
+        a, b, c = (L.tensor(P, dt, s) for s in ([batch, m, k], [batch, n, k], [batch, m, n]))
+        L.check(lib.mjt_matmul(ctypes.byref(a), ctypes.byref(b), ctypes.byref(c), 0, 1))
+        return not L.last_kernel().startswith("mjt_gemm_plain_")
+
+    for dt in ("float32", "bfloat16", "float16"):
+        for shape in ((256, 50, 63, 50), (256, 50, 97, 50), (17, 816, 63, 48), (64, 100, 49, 100)):
+            assert not copied(*shape, dt), (shape, dt)
+        for shape in ((17, 816, 201, 48), (64, 100, 131, 100), (8, 512, 71, 512), (1, 816, 63, 816)):
+            assert copied(*shape, dt), (shape, dt)
+
+
 @pytest.mark.parametrize("k,s,p,dtype", [(2, 2, 0, "bfloat16"), (3, 2, 1, "bfloat16"), (3, 1, 1, "float32"), (4, 1, 0, "float32"),
                                          (2, 1, 0, "float16"), (4, 2, 1, "bfloat16"), (5, 2, 2, "float32")])
 def test_window_gradients_bound_what_a_lane_unrolls(compile_only, monkeypatch, k, s, p, dtype):
