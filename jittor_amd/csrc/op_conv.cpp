@@ -499,7 +499,7 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
             // 16-bit: the gather bounds the kernel and every 64 rows of output channels repeat it, so 128 x 64 when
             // such tiles fill the chip (us, 64x64 / 128x64 / 256x64 / column matrices: 64x1024x14x14 1x1 -> 256: 51 / 37 /
             // 36 / 68; 64x256x13x13 3x3 -> 384: 116 / 76 / 139 / 103; 64x64x27x27 3x3 stride 2 -> 128: 20 / 18 / 23 / 29;
-            // 64x48x28x28 3x3 -> 96: 40 / 35 / 67 / 69; 64x3x224x224 7x7 stride 2 -> 64: 136 / - / - / 285).
+            // 64x48x28x28 3x3 -> 96: 40 / 35 / 67 / 69; 64x3x224x224 7x7 stride 2 -> 64: 114 / - / - / 285).
             const bool big = !ig16 && K > 64 && ((K + 127) / 128) * ((NP + 127) / 128) >= cus;
             const bool tall = ig16 && K > 64 && ((K + 127) / 128) * ((NP + 63) / 64) >= cus;
             const int MI = big || tall ? 2 : 1, NI = big ? 2 : 1;
