@@ -139,4 +139,7 @@ std::string fused_emit_ops(const mjt_fused_desc* d, bool store_outputs);
 inline uint64_t bits_of(double v) { uint64_t u; memcpy(&u, &v, 8); return u; }
 inline uint64_t bits_of_ptr(const void* p) { return (uint64_t)(uintptr_t)p; }
 
+// Threads of a workgroup of kernels/gemm_mfma.h, with float32 operands in parts or as they are.
+inline unsigned product_threads(bool split) { return split ? 512 : 256; }
+
 }  // namespace mjt

@@ -11,7 +11,7 @@
 // truncation, 1 float16 rounded to nearest even, 2 float32), MI, NI (32x32 accumulator
 // tiles per wave along m and n), A_KCONT, B_KCONT (the operand's memory has k innermost).
 //
-// Mapping.  A workgroup of four waves (2 x 2) owns a TM x TN = 64 MI x 64 NI tile of C and
+// Mapping.  A workgroup of four waves (2 x 2; SPLIT: eight) owns a TM x TN = 64 MI x 64 NI tile of C and
 // walks K in stages of KS elements (eight 16-byte chunks per row: 64 for 16-bit operands,
 // 32 for float32).  Both operand tiles of a stage sit in LDS with k innermost,
 // [row][8 chunks + one chunk of padding] (144 bytes per row: 16-byte fragment reads of
@@ -27,7 +27,19 @@
 // of the last MFMAs.  (With these one after the other at the end of each stage the matrix cores stood still for 570 of the
 // 1700 cycles of a 64 x 64 float32 stage.  us before / now, in turn: float32 a b^T 2048 x 1024 x 1024 51 / 43,
 // 2048^3 163 / 143, a^T b 1024 x 1024 x 2048 72 / 58; bfloat16 2048 x 2048 x 2048 32.5 / 23, 12544 x 256 x 1024 18.8 / 14.)
-// The float32 MFMAs alone, 140 TFLOP/s measured, bound the large products.
+// SPLIT = 1 (float32): the float32 MFMAs, 140 TFLOP/s measured, bound the large products, and the bfloat16 ones run at 16 times their
+// rate.  On its way to LDS every value becomes three bfloat16 parts, x = h + m + l, each the rest so far rounded to nearest: 24 bits,
+// all of x.  Six of the nine products of two such values are summed, l h + h l + m m + m h + h m into one accumulator and h h into
+// another; what is left out, m l + l m + l l, is below 2^-26 of the product.  A bfloat16 MFMA rounds once per 16 products where
+// the float32 one rounds per product, so the result is closer to 64 bits than before (relative error, normal operands, K = 64 / 1024 /
+// 4096: 1.4e-7 / 5.7e-7 / 1.15e-6 before, 5e-8 / 1.9e-7 / 4.0e-7 so; also for positive operands and for ones over 9 decades).
+// The parts hold where nothing overflows and nothing falls below the normal range, which the bfloat16 MFMAs take for zero: a
+// workgroup whose operands' smallest magnitudes (zeros apart) are below 2^-100, alone or multiplied, or whose sums are not
+// all finite (an infinity's other parts are NaN), throws its sums away and runs the float32 loop.  Eight waves share a tile,
+// two to a SIMD: one splits while the other's MFMAs run (a b^T 2048 x 1024 x 1024 on 128 x 64 tiles 36.1 us with four waves, 31.0 with
+// eight; 4096 x 4096 x 2048 on 128 x 128 415 / 375).  What bounds it: splitting, 11 vector instructions for two values, takes as
+// long as the MFMAs on 128 x 64 tiles, LDS carries 6 bytes for each value (without the writes 28.5 us, without the loads 24.8, with
+// one MFMA of six 21); a third buffer changes nothing (33), nor does splitting by truncation (30.4) or by v_dot2 (31.2).
 // float32 uses v_mfma_f32_32x32x2: a lane's 16-byte read holds 4 k of its row, which feed
 // four MFMAs (lanes 32..63 read the next chunk, so that an MFMA sums k and k + 4 of a
 // chunk pair; any pairing is right as long as both operands use the same one).
@@ -68,7 +80,22 @@ typedef unsigned short TIN;
 #define TM (64 * MI)
 #define TN (64 * NI)
 #define ROWB 144                 // bytes per LDS row: 8 chunks + 1 of padding
-#define NTHR 256
+#ifndef SPLIT
+#define SPLIT 0                  // 1: float32 products from bfloat16 parts (below)
+#endif
+// Waves: WM x WN, of FI x FJ accumulator tiles each.
+#if SPLIT
+#define SPLIT_ROWB 208           // of a float32 row as three rows of bfloat16: 3 x 64 bytes + 16 of padding
+#define WM (MI >= NI ? 4 : 2)
+#define WN (8 / WM)
+#else
+#define SPLIT_ROWB ROWB
+#define WM 2
+#define WN 2
+#endif
+#define NTHR (64 * WM * WN)
+#define FI (TM / 32 / WM)
+#define FJ (TN / 32 / WN)
 #ifndef CONV
 #define CONV 0
 #endif
@@ -101,7 +128,7 @@ typedef _Float16 mjt_h8 __attribute__((ext_vector_type(8)));
 
 template <int V> struct mjt_ic { static constexpr int v = V; };
 struct Params { void* a[12]; };
-// a[0] A  a[1] B  a[2] C  a[3] M  a[4] N  a[5] K  a[6] lda  a[7] ldb  a[8] ldc (elements)
+// a[0] A  a[1] B  a[2] C  a[3] M (upper half: matrices of the batch)  a[4] N  a[5] K  a[6] lda  a[7] ldb  a[8] ldc (elements)
 // a[9] batch stride of A  a[10] of B  a[11] of C (elements)
 
 __device__ __forceinline__ unsigned mjt_dpp_xor1(unsigned v) { return (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xf, 0xf, true); }
@@ -146,6 +173,56 @@ __device__ __forceinline__ mjt_u32x4v mjt_transpose4x4_b32(mjt_u32x4v v, int lan
     return y;
 }
 
+#if SPLIT
+typedef __bf16 mjt_h8 __attribute__((ext_vector_type(8)));
+typedef unsigned mjt_u32x2v __attribute__((ext_vector_type(2)));
+typedef float mjt_f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 mjt_b16x2 __attribute__((ext_vector_type(2)));
+#define MJT_MFMA16(a, b, c) __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0)
+__device__ __forceinline__ unsigned mjt_bf16_pair(float x, float y) {      // both rounded to nearest even
+    return __builtin_bit_cast(unsigned, __builtin_convertvector((mjt_f32x2){x, y}, mjt_b16x2));
+}
+#define MJT_KEY(e) ((unsigned)(127 + (e)) << 24)
+template <int CTRL, int ROWS> __device__ __forceinline__ unsigned mjt_min_dpp(unsigned v) {
+    return min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, CTRL, ROWS, 0xf, false));
+}
+__device__ __forceinline__ unsigned mjt_wave_min(unsigned v) {             // of all 64 lanes, in every lane
+    v = mjt_min_dpp<0x111, 0xf>(v);                                        // from the lane 1, 2, 4, 8 below, inside rows of 16
+    v = mjt_min_dpp<0x112, 0xf>(v);
+    v = mjt_min_dpp<0x114, 0xf>(v);
+    v = mjt_min_dpp<0x118, 0xf>(v);
+    v = mjt_min_dpp<0x142, 0xa>(v);                                        // a row's last lane to the next row; lane 31 to the upper half
+    v = mjt_min_dpp<0x143, 0xc>(v);
+    return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+__device__ __forceinline__ float mjt_low(unsigned p) { return __uint_as_float(p << 16); }
+__device__ __forceinline__ float mjt_high(unsigned p) { return __uint_as_float(p & 0xffff0000u); }
+#endif
+// One 16-byte chunk on its way to LDS.  SP: as its three bfloat16 parts, each the rest of the ones before it rounded to nearest;
+// `least` keeps the smallest 2 |value| - 1 of the bits as integers (zeros wrap round to the largest).
+template <bool SP> __device__ __forceinline__ void mjt_put(unsigned char* lds, int row, int kc, mjt_u32x4v v, unsigned& least) {
+#if SPLIT
+    if constexpr (SP) {
+        unsigned char* const at = lds + row * SPLIT_ROWB + kc * 8;
+        mjt_u32x2v h, m, l;
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+            const float x = __uint_as_float(v[2 * p]), y = __uint_as_float(v[2 * p + 1]);
+            h[p] = mjt_bf16_pair(x, y);
+            const float x1 = x - mjt_low(h[p]), y1 = y - mjt_high(h[p]);
+            m[p] = mjt_bf16_pair(x1, y1);
+            l[p] = mjt_bf16_pair(x1 - mjt_low(m[p]), y1 - mjt_high(m[p]));
+            least = min(least, min((v[2 * p] << 1) - 1u, (v[2 * p + 1] << 1) - 1u));
+        }
+        *(mjt_u32x2v*)at = h;
+        *(mjt_u32x2v*)(at + 64) = m;
+        *(mjt_u32x2v*)(at + 128) = l;
+        return;
+    }
+#endif
+    *(mjt_u32x4v*)(lds + row * ROWB + kc * 16) = v;
+}
+
 template <int I, int N, class F> __device__ __forceinline__ void mjt_static_for(F&& f) {
     if constexpr (I < N) {
         f(mjt_ic<I>());
@@ -185,7 +262,7 @@ template <int ROWS, bool KCONT> struct mjt_stager {
             reg[I] = *(const mjt_u32x4v*)(p + (long long)kk * ld + col);
         }
     }
-    template <int I, bool FULL> __device__ __forceinline__ void commit(unsigned char* lds, int k0, int K, int tid) const {
+    template <int I, bool FULL, bool SP> __device__ __forceinline__ void commit(unsigned char* lds, int k0, int K, int tid, unsigned& least) const {
         mjt_u32x4v v = reg[I];
         int row, kc;
         if constexpr (KCONT) {
@@ -215,7 +292,7 @@ template <int ROWS, bool KCONT> struct mjt_stager {
             v = mjt_transpose8x8_b16(v, tid);
 #endif
         }
-        *(mjt_u32x4v*)(lds + row * ROWB + kc * 16) = v;
+        mjt_put<SP>(lds, row, kc, v, least);
     }
 };
 
@@ -298,13 +375,13 @@ struct mjt_conv_stager {
 #endif
         });
     }
-    template <int I> __device__ __forceinline__ void commit(unsigned char* lds, int tid) const {
+    template <int I, bool SP> __device__ __forceinline__ void commit(unsigned char* lds, int tid, unsigned& least) const {
         const int b = tid / EPC + I * (NTHR / EPC);
         const int row = (b % (TN / EPC)) * EPC + tid % EPC, kc = b / (TN / EPC);
 #if IN == 2
-        *(mjt_u32x4v*)(lds + row * ROWB + kc * 16) = mjt_transpose4x4_b32(mjt_wg_pack(v[I]), tid);
+        mjt_put<SP>(lds, row, kc, mjt_transpose4x4_b32(mjt_wg_pack(v[I]), tid), least);
 #else
-        *(mjt_u32x4v*)(lds + row * ROWB + kc * 16) = mjt_transpose8x8_b16(mjt_wg_pack(v[I]), tid);
+        mjt_put<SP>(lds, row, kc, mjt_transpose8x8_b16(mjt_wg_pack(v[I]), tid), least);
 #endif
     }
 };
@@ -379,8 +456,8 @@ template <int ROWS> struct mjt_wg_plane {
             });
         }
     }
-    template <int I> __device__ __forceinline__ void commit(unsigned char* lds, int tid) const {
-        *(mjt_u32x4v*)(lds + (tid / KC + I * (NTHR / KC)) * ROWB + (tid % KC) * 16) = reg[I];
+    template <int I, bool SP> __device__ __forceinline__ void commit(unsigned char* lds, int tid, unsigned& least) const {
+        mjt_put<SP>(lds, tid / KC + I * (NTHR / KC), tid % KC, reg[I], least);
     }
 };
 typedef mjt_wg_plane<TM> mjt_wg_dy;
@@ -409,8 +486,8 @@ struct mjt_wg_x {
             v[I][e] = mjt_wg_load(d, in ? ch.x[e] + koff[I] : MJT_NONE);
         });
     }
-    template <int I> __device__ __forceinline__ void commit(unsigned char* lds, int tid) const {
-        *(mjt_u32x4v*)(lds + (tid / KC + I * (NTHR / KC)) * ROWB + (tid % KC) * 16) = mjt_wg_pack(v[I]);
+    template <int I, bool SP> __device__ __forceinline__ void commit(unsigned char* lds, int tid, unsigned& least) const {
+        mjt_put<SP>(lds, tid / KC + I * (NTHR / KC), tid % KC, mjt_wg_pack(v[I]), least);
     }
 };
 #endif
@@ -429,48 +506,48 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
     const TIN* __restrict__ B = (const TIN*)p.a[1];
     const __amdgpu_buffer_rsrc_t dy_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, (int)(K * K_) * ESZ, 0x00020000);
     const __amdgpu_buffer_rsrc_t x_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, (int)(long long)p.a[10], 0x00020000);   // a[10]: bytes of x
-    // Workgroups go round-robin over the 8 XCDs: every XCD takes a run of neighbouring (slice, tile) pairs, so that the tiles
-    // of one slice, which read the same dy and x, run next to each other and share an L2 (64 x 64 x 56 x 56, 3x3 -> 64: 269 us
-    // with the tiles dealt out one by one, 162 with runs).
-    const int slice_tiles = (M + TM - 1) / TM * ((N + TN - 1) / TN);
-    const int per_slice = (int)(long long)p.a[9];
-    const int pairs = ((K + KS - 1) / KS + per_slice - 1) / per_slice * slice_tiles, run = (pairs + 7) / 8;
-    const int pair = (int)(blockIdx.x & 7) * run + (int)(blockIdx.x >> 3);
-    if ((int)(blockIdx.x >> 3) >= run || pair >= pairs) return;
-    const int slice = pair / slice_tiles;
-    const int first_stage = slice * per_slice;
+#endif
+    // Workgroups go round-robin over the 8 XCDs: every XCD takes a run of neighbouring (matrix of the batch or slice of the sum, tile)
+    // pairs, so that the tiles that read the same operands run next to each other and share an L2 (weight gradient 64 x 64 x 56 x 56,
+    // 3x3 -> 64: 269 us with the tiles dealt out one by one, 162 with runs), and all XCDs have work however few tiles a matrix has
+    // (us, a b^T, each matrix on the same first XCDs / so: float32 256 x 64 x 64 x 64 20.4 / 10.6, 512 x 32 x 128 x 64 66 / 31;
+    // bfloat16 the same 8.7 / 7.2, 18.1 / 10.2).  (Before, each matrix had a row of the
+    // grid to itself, rounded up to eight workgroups, and which compute units the empty ones kept from work was chance: float32
+    // 64 x 256 x 196 x 1024 on 128 x 128 tiles, four a matrix, 92 / 56; 256 x 64 x 64 x 64 9.2 / 5.2; bfloat16 the same 7.1 / 4.0,
+    // 100 x 200 x 200 x 128 22.2 / 12.2.)
+    const int tiles_m = (M + TM - 1) / TM, tiles_n = (N + TN - 1) / TN, tiles = tiles_m * tiles_n;
+#if CONV == 2 || SLICED
+    const int per_slice = (int)(long long)p.a[9], pairs = ((K + KS - 1) / KS + per_slice - 1) / per_slice * tiles;
 #else
+    const int pairs = (CONV ? 1 : (int)((long long)p.a[3] >> 32)) * tiles;
+#endif
+    const int run = (pairs + 7) / 8, pair = (int)(blockIdx.x & 7) * run + (int)(blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= run || pair >= pairs) return;
+    const int outer = pair / tiles, L = pair - outer * tiles;        // slice or matrix; tile
+#if CONV == 2 || SLICED
+    const int first_stage = outer * per_slice;
+#endif
+#if CONV != 2
 #if SLICED
     const TIN* __restrict__ A = (const TIN*)p.a[0];
     const TIN* __restrict__ B = (const TIN*)p.a[1];
-    const int per_slice = (int)(long long)p.a[9], slice = blockIdx.y, first_stage = slice * per_slice;
 #else
-    const TIN* __restrict__ A = (const TIN*)p.a[0] + (long long)blockIdx.y * (long long)p.a[9];
-    const TIN* __restrict__ B = (const TIN*)p.a[1] + (long long)blockIdx.y * (long long)p.a[10];
+    const TIN* __restrict__ A = (const TIN*)p.a[0] + (long long)outer * (long long)p.a[9];
+    const TIN* __restrict__ B = (const TIN*)p.a[1] + (long long)outer * (long long)p.a[10];
 #endif
 #endif
     // NBUF 1: the host promises K <= KS, a single stage -- one staging buffer, so twice as many workgroups fit a compute unit
-    __shared__ __attribute__((aligned(16))) unsigned char lds[NBUF][(TM + TN) * ROWB];
-
-    // Tile order: panels of 4 tile rows, inside a panel column by column.  Workgroups go round-robin over the
-    // 8 XCDs, so workgroup id takes tile (id % 8) * per_xcd + id / 8: every XCD works on a compact run of
-    // tiles and finds the operand rows and columns it shares in its own L2.  The next matrix of a batch, or slice of a sum, starts
-    // one XCD further on unless its tiles spread evenly: with fewer than eight, all would otherwise run on the same few (us, a b^T,
-    // before / so: float32 256 x 64 x 64 x 64 20.4 / 10.6, 512 x 32 x 128 x 64 66 / 31, 100 x 200 x 200 x 128 a b 107 / 52.5; bfloat16 the
-    // same 8.7 / 7.2, 18.1 / 10.2, 44.3 / 21.6).
-    const int tiles_m = (M + TM - 1) / TM, tiles_n = (N + TN - 1) / TN;
-    const int tiles = tiles_m * tiles_n;
-    int L = blockIdx.x;
-#if CONV == 2
-    L = pair - slice * slice_tiles;
-#else
-    {
-        const int per_xcd = (tiles + 7) / 8;
-        const unsigned turn = tiles % 8 ? blockIdx.y : 0;
-        L = ((blockIdx.x + turn) & 7) * per_xcd + (blockIdx.x >> 3);
-        if (L >= tiles || (blockIdx.x >> 3) >= per_xcd) return;
-    }
+    __shared__ __attribute__((aligned(16))) unsigned char lds[NBUF][(TM + TN) * SPLIT_ROWB];
+#if SPLIT
+    __shared__ int in_float32;
+    __shared__ unsigned least[2];
+    if (threadIdx.x == 0) in_float32 = 0;
+    if (threadIdx.x < 2) least[threadIdx.x] = ~0u;
+    __syncthreads();
 #endif
+
+    // Tile order inside a matrix: panels of 4 tile rows, inside a panel column by column, so that a run of tiles is compact and
+    // finds the operand rows and columns it shares in its XCD's L2.
     int tm, tn;
     {
         const int panel = L / (4 * tiles_n);
@@ -481,13 +558,17 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
     }
     const int m0 = tm * TM, n0 = tn * TN;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
+    const int wm = wave / WN, wn = wave % WN;
 
     // The operand tiles of a stage are asked for NSET stages ahead: one stage of MFMAs is shorter than a trip to memory on tiles
     // up to 128 x 128 of 16-bit and on all float32 tiles that are run (us with one set / two / three, float32: 1024 x 1024 x 2048
     // on 64 x 64 57.7 / 55.4 / 57.1, 2048^3 on 128 x 128 133 / 127 / -).  Larger tiles have no registers to spare.
     // The gathering operands hold more registers: two sets on 64 x 64 tiles only (64 x 512 x 7 x 7 3x3 -> 512 247 / 218;
     // 64 x 128 x 28 x 28 3x3 -> 128 on 128 x 128 186 / 194).
+    auto multiply = [&](auto spc) -> bool {
+    constexpr bool SP = decltype(spc)::v != 0;
+    constexpr int RB = SP ? SPLIT_ROWB : ROWB, BUFB = (TM + TN) * RB;
+    unsigned least_a = ~0u, least_b = ~0u;
     constexpr int NSET = NBUF > 1 && STAGES != 2 && MI * NI <= (CONV ? 1 : 4) ? 2 : 1;
 #if CONV == 2
     const int all_stages = (K + KS - 1) / KS;
@@ -509,9 +590,9 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
     };
     auto commit = [&](auto ic, auto setc, auto, int stage) {
         constexpr int I = decltype(ic)::v, SET = decltype(setc)::v;
-        unsigned char* buf = &lds[stage & (NBUF - 1)][0];
-        if constexpr (I < PA) sa[SET].template commit<I>(buf, tid);
-        else sb[SET].template commit<I - PA>(buf + TM * ROWB, tid);
+        unsigned char* buf = &lds[0][0] + (stage & (NBUF - 1)) * BUFB;
+        if constexpr (I < PA) sa[SET].template commit<I, SP>(buf, tid, least_a);
+        else sb[SET].template commit<I - PA, SP>(buf + TM * RB, tid, least_b);
     };
 #else
 #if SLICED
@@ -548,12 +629,12 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
     auto commit = [&](auto ic, auto setc, auto fullc, int stage) {
         constexpr int I = decltype(ic)::v, SET = decltype(setc)::v;
         constexpr bool FULL = decltype(fullc)::v != 0;
-        unsigned char* buf = &lds[stage & (NBUF - 1)][0];
-        if constexpr (I < PA) sa[SET].template commit<I, FULL>(buf, (first_stage + stage) * KS, K, tid);
+        unsigned char* buf = &lds[0][0] + (stage & (NBUF - 1)) * BUFB;
+        if constexpr (I < PA) sa[SET].template commit<I, FULL, SP>(buf, (first_stage + stage) * KS, K, tid, least_a);
 #if CONV
-        else sb[SET].template commit<I - PA>(buf + TM * ROWB, tid);
+        else sb[SET].template commit<I - PA, SP>(buf + TM * RB, tid, least_b);
 #else
-        else sb[SET].template commit<I - PA, FULL>(buf + TM * ROWB, (first_stage + stage) * KS, K, tid);
+        else sb[SET].template commit<I - PA, FULL, SP>(buf + TM * RB, (first_stage + stage) * KS, K, tid, least_b);
 #endif
     };
 #endif
@@ -561,61 +642,85 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
         if (decltype(tc)::v < nstages) mjt_static_for<0, PIECES>([&](auto ic) { fetch(ic, tc, mjt_ic<0>(), decltype(tc)::v); });
     });
 
-    mjt_f32x16 acc[MI][NI];
+    mjt_f32x16 acc[FI][FJ], low[SP ? FI : 1][SP ? FJ : 1];
 #pragma unroll
-    for (int i = 0; i < MI; i++)
+    for (int i = 0; i < FI; i++)
 #pragma unroll
-        for (int j = 0; j < NI; j++)
+        for (int j = 0; j < FJ; j++)
 #pragma unroll
-            for (int e = 0; e < 16; e++) acc[i][j][e] = 0.0f;
+            for (int e = 0; e < 16; e++) {
+                acc[i][j][e] = 0.0f;
+                if constexpr (SP) low[i][j][e] = 0.0f;
+            }
 
     mjt_static_for<0, PIECES>([&](auto ic) { commit(ic, mjt_ic<0>(), mjt_ic<0>(), 0); });
+#if SPLIT
+    if constexpr (SP)
+        if (min(least_a, least_b) < MJT_KEY(-100)) in_float32 = 1;
+#endif
     if (NSET < nstages) mjt_static_for<0, PIECES>([&](auto ic) { fetch(ic, mjt_ic<0>(), mjt_ic<0>(), NSET); });
     __syncthreads();
+#if SPLIT
+    if constexpr (SP)
+        if (in_float32) return false;                          // (usually seen here, where little is lost)
+#endif
 
     // fragment addresses of this lane: row lane % 32 of its wave's tile rows, chunk lane / 32
     const int frow = lane & 31, fhalf = lane >> 5;
-    const unsigned char* const la = &lds[0][0] + (wm * 32 * MI + frow) * ROWB + fhalf * 16;
-    const unsigned char* const lb = &lds[0][TM * ROWB] + (wn * 32 * NI + frow) * ROWB + fhalf * 16;
+    const unsigned char* const la = &lds[0][0] + (wm * 32 * FI + frow) * RB + fhalf * 16;
+    const unsigned char* const lb = &lds[0][0] + (TM + wn * 32 * FJ + frow) * RB + fhalf * 16;
     // a pair of chunks per step; the fragments of the next step, across the end of a stage too, are requested before the MFMAs of
     // this one (the scheduling barriers keep them there: the compiler would move every read next to its first use)
-    mjt_u32x4v fa[2][MI], fb[2][NI];
+    constexpr int PARTS = SP ? 3 : 1, STEPS = SP ? KS / 16 : KC / 2;
+    mjt_u32x4v fa[2][FI][PARTS], fb[2][FJ][PARTS];
     auto request = [&](auto ksc, auto setc, const int s) {
         constexpr int KSX = decltype(ksc)::v, SET = decltype(setc)::v;
-        const int off = (s & (NBUF - 1)) * ((TM + TN) * ROWB) + KSX * 32;
-        mjt_static_for<0, MI>([&](auto ic) { fa[SET][decltype(ic)::v] = *(const mjt_u32x4v*)(la + off + decltype(ic)::v * 32 * ROWB); });
-        mjt_static_for<0, NI>([&](auto jc) { fb[SET][decltype(jc)::v] = *(const mjt_u32x4v*)(lb + off + decltype(jc)::v * 32 * ROWB); });
+        const int off = (s & (NBUF - 1)) * BUFB + KSX * 32;
+        mjt_static_for<0, PARTS>([&](auto pc) {
+            constexpr int part = decltype(pc)::v;
+            mjt_static_for<0, FI>([&](auto ic) { fa[SET][decltype(ic)::v][part] = *(const mjt_u32x4v*)(la + off + part * 64 + decltype(ic)::v * 32 * RB); });
+            mjt_static_for<0, FJ>([&](auto jc) { fb[SET][decltype(jc)::v][part] = *(const mjt_u32x4v*)(lb + off + part * 64 + decltype(jc)::v * 32 * RB); });
+        });
     };
     request(mjt_ic<0>(), mjt_ic<0>(), 0);
     // Stage s: its tiles sit in LDS buffer s % NBUF, its first fragments are on their way, and the register sets hold the stages
     // s + 1 .. s + NSET.  Piece by piece between the MFMAs of all steps but the last, stage s + 1 goes to the other buffer, which
     // nobody has read since the barrier of stage s - 1, and its registers take stage s + 1 + NSET.  The barrier stands in front
-    // of the last step's MFMAs: every wave has then read the last fragments of this stage and written the next one, whose first
-    // fragments arrive during these MFMAs.
+    // of the last step's MFMAs (SP, two long steps: of the last half of them): every wave has then read the last fragments of this
+    // stage and written the next one, whose first fragments arrive during these MFMAs.
     // FULL: stages s + 1 and s + 1 + NSET exist and do not reach beyond K -- no branches, so that the pieces' instructions can
     // stand between MFMAs.
     auto run_stage = [&](auto parc, auto fullc, const int s) {
         constexpr int PAR = decltype(parc)::v, SET = (PAR + 1) % NSET;
         constexpr bool FULL = decltype(fullc)::v != 0;
-        mjt_static_for<0, KC / 2>([&](auto ksc) {
+        mjt_static_for<0, STEPS>([&](auto ksc) {
             constexpr int ks = decltype(ksc)::v, cur = ks & 1, nxt = cur ^ 1;
-            if constexpr (ks + 1 < KC / 2) {
-                request(mjt_ic<ks + 1>(), mjt_ic<nxt>(), s);
-            } else if (FULL || s + 1 < nstages) {
-                __syncthreads();
-                request(mjt_ic<0>(), mjt_ic<nxt>(), s + 1);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            constexpr int EK = IN == 2 ? 4 : 1, PER_STEP = EK * MI * NI, SLOTS = PER_STEP * (KC / 2 - 1) - PER_STEP / 2;
+            constexpr int EK = SP ? 6 : IN == 2 ? 4 : 1, PER_STEP = EK * FI * FJ;
+            constexpr int BARRIER = SP ? PER_STEP * STEPS - PER_STEP / 2 : PER_STEP * (STEPS - 1), SLOTS = SP ? BARRIER * 3 / 4 : BARRIER - PER_STEP / 2;
+            if constexpr (ks + 1 < STEPS) request(mjt_ic<ks + 1>(), mjt_ic<nxt>(), s);
             mjt_static_for<0, PER_STEP>([&](auto mc) {
-                constexpr int m = decltype(mc)::v, e = m / (MI * NI), i = m / NI % MI, j = m % NI, slot = ks * PER_STEP + m;
+                constexpr int m = decltype(mc)::v, e = m / (FI * FJ), i = m / FJ % FI, j = m % FJ, slot = ks * PER_STEP + m;
+                if constexpr (slot == BARRIER) {
+                    if (FULL || s + 1 < nstages) {
+                        __syncthreads();
+                        request(mjt_ic<0>(), mjt_ic<nxt>(), s + 1);
+                    }
+                }
+                if constexpr (m == 0 || slot == BARRIER) __builtin_amdgcn_sched_barrier(0);
 #if IN == 2
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(fa[cur][i][e]), __uint_as_float(fb[cur][j][e]), acc[i][j], 0, 0, 0);
-#else
-                acc[i][j] = MJT_MFMA16(__builtin_bit_cast(mjt_h8, fa[cur][i]), __builtin_bit_cast(mjt_h8, fb[cur][j]), acc[i][j]);
+#if SPLIT
+                if constexpr (SP) {
+                    constexpr int pa = e == 0 ? 2 : e == 2 || e == 3 ? 1 : 0, pb = e == 1 ? 2 : e == 2 || e == 4 ? 1 : 0;
+                    mjt_f32x16& sum = e == 5 ? acc[i][j] : low[i][j];
+                    sum = MJT_MFMA16(__builtin_bit_cast(mjt_h8, fa[cur][i][pa]), __builtin_bit_cast(mjt_h8, fb[cur][j][pb]), sum);
+                } else
 #endif
-                if constexpr (NBUF > 1 && ks + 1 < KC / 2) {
-                    constexpr int first = slot < SLOTS ? PIECES * slot / SLOTS : PIECES, last = slot + 1 < SLOTS ? PIECES * (slot + 1) / SLOTS : PIECES;
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(fa[cur][i][0][e & 3]), __uint_as_float(fb[cur][j][0][e & 3]), acc[i][j], 0, 0, 0);
+#else
+                acc[i][j] = MJT_MFMA16(__builtin_bit_cast(mjt_h8, fa[cur][i][0]), __builtin_bit_cast(mjt_h8, fb[cur][j][0]), acc[i][j]);
+#endif
+                if constexpr (NBUF > 1 && slot < SLOTS) {
+                    constexpr int first = PIECES * slot / SLOTS, last = PIECES * (slot + 1) / SLOTS;
                     if constexpr (FULL && last > first) {
                         __builtin_amdgcn_sched_barrier(0);
                         mjt_static_for<first, last>([&](auto ic) {
@@ -626,7 +731,7 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
                     }
                 }
             });
-            if constexpr (!FULL && NBUF > 1 && ks == KC / 2 - 2) {
+            if constexpr (!FULL && NBUF > 1 && ks == STEPS - 2) {
                 if (s + 1 < nstages) {
                     mjt_static_for<0, PIECES>([&](auto ic) { commit(ic, mjt_ic<SET>(), mjt_ic<0>(), s + 1); });
                     if (s + 1 + NSET < nstages) mjt_static_for<0, PIECES>([&](auto ic) { fetch(ic, mjt_ic<SET>(), mjt_ic<0>(), s + 1 + NSET); });
@@ -651,27 +756,51 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
             if (s0 + decltype(parc)::v < nstages) run_stage(parc, mjt_ic<0>(), s0 + decltype(parc)::v);
         });
 
+#if SPLIT
+    if constexpr (SP) {
+        float z = 0.0f;                                        // not zero if any sum is not finite
+#pragma unroll
+        for (int i = 0; i < FI; i++)
+#pragma unroll
+            for (int j = 0; j < FJ; j++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) {
+                    acc[i][j][e] += low[i][j][e];
+                    z = __builtin_fmaf(acc[i][j][e], 0.0f, z);
+                }
+        const unsigned wave_a = mjt_wave_min(least_a), wave_b = mjt_wave_min(least_b);
+        if (lane == 0) {
+            atomicMin(&least[0], wave_a);
+            atomicMin(&least[1], wave_b);
+        }
+        if (z != 0.0f) in_float32 = 1;
+        __syncthreads();
+        const unsigned all_a = least[0], all_b = least[1];
+        if (in_float32 || all_a < MJT_KEY(-100) || all_b < MJT_KEY(-100) || (all_a >> 24) + (all_b >> 24) < 2 * 127 - 100) return false;
+    }
+#endif
+
     // D of a 32x32 tile: lane holds column lane % 32, rows 8 * (e / 4) + 4 * (lane / 32) + e % 4
 #if OUT == 2
 #if CONV == 2 || SLICED
-    float* __restrict__ C = (float*)p.a[2] + (long long)slice * (long long)p.a[11];
+    float* __restrict__ C = (float*)p.a[2] + (long long)outer * (long long)p.a[11];
 #else
-    float* __restrict__ C = (float*)p.a[2] + (long long)blockIdx.y * (long long)p.a[11];
+    float* __restrict__ C = (float*)p.a[2] + (long long)outer * (long long)p.a[11];
 #endif
 #else
-    unsigned short* __restrict__ C = (unsigned short*)p.a[2] + (long long)blockIdx.y * (long long)p.a[11];
+    unsigned short* __restrict__ C = (unsigned short*)p.a[2] + (long long)outer * (long long)p.a[11];
 #endif
 #pragma unroll
-    for (int i = 0; i < MI; i++)
+    for (int i = 0; i < FI; i++)
 #pragma unroll
-        for (int j = 0; j < NI; j++) {
-            const int col = n0 + wn * 32 * NI + j * 32 + (lane & 31);
+        for (int j = 0; j < FJ; j++) {
+            const int col = n0 + wn * 32 * FJ + j * 32 + (lane & 31);
 #if CONV == 1
             const int img = col / (OH_ * OW_), px = col - img * (OH_ * OW_);      // y[img][row][px]
 #endif
 #pragma unroll
             for (int e = 0; e < 16; e++) {
-                const int row = m0 + wm * 32 * MI + i * 32 + 8 * (e / 4) + 4 * (lane >> 5) + (e & 3);
+                const int row = m0 + wm * 32 * FI + i * 32 + 8 * (e / 4) + 4 * (lane >> 5) + (e & 3);
                 if (row < M && col < N) {
                     const float v = acc[i][j][e];
 #if CONV == 1
@@ -690,4 +819,11 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
                 }
             }
         }
+    return true;
+    };
+#if SPLIT
+    if (multiply(mjt_ic<1>())) return;
+    __syncthreads();
+#endif
+    multiply(mjt_ic<0>());
 }

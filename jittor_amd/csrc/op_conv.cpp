@@ -490,31 +490,45 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
             numel(x) < (int64_t(1) << 31) && numel(y) < (int64_t(1) << 31) && H < 16384 && W < 16384 &&
             (R - 1) * p->dil_h < 16384 && (S - 1) * p->dil_w < 16384 && p->pad_h < 16384 && p->pad_w < 16384 &&
             OH * p->stride_h < 16384 && OW * p->stride_w < 16384) {
-            // Tile, float32: 64 output channels x 64 pixels, or 128 x 128 when there are more than 64 output channels and
-            // enough tiles of that size for every compute unit.  Measured (us, tiles 64x64 / 64x128 / 128x64 / 128x128):
-            // 64x64x56x56 3x3 -> 64: 202 / 244 / 381 / 365; 64x3x224x224 7x7 stride 2 -> 64: 228 / 254 / 426 / 379;
-            // 64x128x28x28 3x3 -> 128: 208 / 246 / 214 / 192; 64x512x7x7 3x3 -> 512: 272 / 335 / 273 / 469.  Small tiles
-            // win because four workgroups then share a compute unit: the gather's address arithmetic of one overlaps the
-            // MFMAs of another.
+            // Tile, float32, sums of less than four stages (32 elements): 64 output channels x 64 pixels, or 128 x 128 when there
+            // are more than 64 output channels and enough tiles of that size for every compute unit.  Longer sums: float32
+            // MFMAs on 64 x 64 tiles, of which four workgroups share a compute unit, so that the gather's address arithmetic of one
+            // overlaps the MFMAs of another, or products of bfloat16 parts on 128 x 64 or 128 x 128 tiles, by what they are
+            // estimated to take: 0.92, 1.05 or 1.85 us a stage and 3, 4 or 5 for each round's first loads and results, four 64 x 64
+            // workgroups running at once on a unit (us, 64x64 / 64x128 / 128x64 / 128x128:
+            // 64x64x56x56 3x3 -> 64: 178 / 190 / 286 / 261; 64x3x224x224 7x7 stride 2 -> 64: 229 / 278 / 434 / 361; 64x128x28x28 3x3 ->
+            // 128: 213 / 199 / 172 / 137; 64x256x14x14 3x3 -> 256: 214 / 192 / 166 / 151; 64x512x7x7 3x3 -> 512: 220 / 186 / 163 / 255;
+            // 32x64x56x56 3x3 stride 2 -> 128: 62 / 57 / 50 / 43; 16x256x14x14 3x3 -> 256: 66 / 83 / 71 / 124).
             // 16-bit: the gather bounds the kernel and every 64 rows of output channels repeat it, so 128 x 64 when
             // such tiles fill the chip (us, 64x64 / 128x64 / 256x64 / column matrices: 64x1024x14x14 1x1 -> 256: 51 / 37 /
             // 36 / 68; 64x256x13x13 3x3 -> 384: 116 / 76 / 139 / 103; 64x64x27x27 3x3 stride 2 -> 128: 20 / 18 / 23 / 29;
             // 64x48x28x28 3x3 -> 96: 40 / 35 / 67 / 69; 64x3x224x224 7x7 stride 2 -> 64: 114 / - / - / 285).
             const bool big = !ig16 && K > 64 && ((K + 127) / 128) * ((NP + 127) / 128) >= cus;
             const bool tall = ig16 && K > 64 && ((K + 127) / 128) * ((NP + 63) / 64) >= cus;
-            const int MI = big || tall ? 2 : 1, NI = big ? 2 : 1;
+            int MI = big || tall ? 2 : 1, NI = big ? 2 : 1;
+            bool split = false;
+            if (!ig16 && CRS >= 128) {
+                const int64_t stages = (CRS + 31) / 32;
+                double least = 1e30;
+                for (int t = big ? 1 : 0; t < 3; t++) {
+                    const int mi = t ? 2 : 1, ni = t == 2 ? 2 : 1;
+                    const double rounds = std::ceil((double)(((K + 64 * mi - 1) / (64 * mi)) * ((NP + 64 * ni - 1) / (64 * ni))) / cus);
+                    const double us = t == 0 ? (0.92 * stages + 3.0) * (0.25 + 0.75 * rounds) : t == 1 ? (1.05 * stages + 4.0) * rounds : (1.85 * stages + 5.0) * rounds;
+                    if (us < least) { least = us; MI = mi; NI = ni; split = t > 0; }
+                }
+            }
             const int in = x->dtype == MJT_BFLOAT16 ? 0 : x->dtype == MJT_FLOAT16 ? 1 : 2;
             const int out = y->dtype == MJT_BFLOAT16 ? 0 : y->dtype == MJT_FLOAT16 ? 1 : 2;
             std::ostringstream key;
             const bool xbuf = (64 * NI / P + 2) * C * H * W * esz < (int64_t(1) << 31);      // a tile's images through one buffer descriptor
-            key << "igemm|" << geo.str() << MI << NI << in << out << xbuf;
+            key << "igemm|" << geo.str() << MI << NI << in << out << xbuf << split;
             JitKernel* k = cached(key.str());
             if (!k) {
                 std::ostringstream name;
                 name << "mjt_conv_igemm_" << mjt_dtype_name(x->dtype) << (y->dtype != x->dtype ? "_of32" : "") << "_c" << C << "_k" << K << "_" << H << "x" << W << "_r" << R << "x" << S << "_s" << p->stride_h << "x"
-                     << p->stride_w << "_p" << p->pad_h << "x" << p->pad_w << "_d" << p->dil_h << "x" << p->dil_w << "_" << 64 * MI << "x" << 64 * NI;
+                     << p->stride_w << "_p" << p->pad_h << "x" << p->pad_w << "_d" << p->dil_h << "x" << p->dil_w << (split ? "_parts_" : "_") << 64 * MI << "x" << 64 * NI;
                 std::ostringstream src;
-                src << "#define ENTRY " << name.str() << "\n#define CONV 1\n#define IN " << in << "\n#define OUT " << out << "\n#define MI " << MI << "\n#define NI " << NI
+                src << "#define ENTRY " << name.str() << "\n#define SPLIT " << (split ? 1 : 0) << "\n#define CONV 1\n#define IN " << in << "\n#define OUT " << out << "\n#define MI " << MI << "\n#define NI " << NI
                     << "\n#define A_KCONT 1\n#define B_KCONT 0\n#define XBUF " << (xbuf ? 1 : 0) << "\n" << geo.str();
                 src << embedded_source("gemm_mfma.h") << "\n";
                 k = jit_get(src.str(), name.str());
@@ -525,7 +539,7 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
             MJT_CHECK(grid < (int64_t(1) << 31), "conv: launch too large");
             std::vector<uint64_t> a{bits_of_ptr(wmat), bits_of_ptr(x->ptr), bits_of_ptr(y->ptr), (uint64_t)K, (uint64_t)NP, (uint64_t)CRS,
                                     (uint64_t)lda, 0, 0, 0, 0, 0};
-            jit_launch(k, (unsigned)grid, 1, 256, 0, a);
+            jit_launch(k, (unsigned)grid, 1, product_threads(split), 0, a);
             return;
         }
         int64_t chunk = (int64_t(1) << 30) / (CRS * Ppad * esz);
@@ -746,21 +760,20 @@ static bool conv_wgrad_product(const mjt_tensor* x, const mjt_tensor* dy, const 
     double least = 1e30;
     if (!half) {
         // float32: a stage of a 64 x 64 tile takes 0.78 us with a compute unit to itself and 0.9 of that more for each further
-        // workgroup there (four fit), one of a 128 x 128 tile 2.55 us and 1.85 times that with two, which is all that fit; its
+        // workgroup there (four fit), one of a 128 x 128 tile, which multiplies bfloat16 parts, 1.75 us, one workgroup at a time; its
         // first operands and its results 5 us more.  Slices that give every compute unit one, two, four or eight workgroups (128: one,
         // two or four), down to a single stage each; more 64 x 64 tiles than compute units share less and take 1.25 times that.
-        // us, 64 x 64 / 128 x 128 tiles at their best slices: 64 x 64 x 7 x 7 1x1 -> 64 11.8 / 16.9 (one slice 84);
-        // 16 x 100 x 9 x 9 3x3 stride 2 -> 70 9.6 / 14.9; 16 x 256 x 14 x 14 1x1 -> 256 13.1 / 21.0; 64 x 64 x 28 x 28 3x3 -> 64
-        // 52.4 / 90; 64 x 128 x 28 x 28 3x3 -> 128 155 / 148; 64 x 256 x 14 x 14 3x3 -> 256 173 / 145; 64 x 512 x 7 x 7 3x3 -> 512
-        // 187 / 170.
+        // us, 64 x 64 / 128 x 128 tiles at their best slices: 16 x 100 x 9 x 9 3x3 stride 2 -> 70 9.1 / 12.0; 8 x 64 x 28 x 28 3x3 -> 64 15.8 /
+        // 19.5; 64 x 64 x 56 x 56 3x3 -> 64 152 / 221; 32 x 64 x 56 x 56 3x3 stride 2 -> 128 59 / 40; 64 x 128 x 28 x 28 3x3 -> 128 168 / 101;
+        // 64 x 256 x 14 x 14 3x3 -> 256 189 / 108; 64 x 512 x 7 x 7 3x3 -> 512 216 / 131 (128 x 128 with float32 MFMAs 140, 141, 156).
         for (int mi = 1; mi <= 2; mi++)
             for (int64_t r = 1; r <= (mi == 1 ? 8 : 4); r *= 2) {
                 int64_t n = r * cus / tiles_of(64 * mi);
                 n = n < 1 ? 1 : n > stages ? stages : n;
                 const int64_t pn = (stages + n - 1) / n, nn = (stages + pn - 1) / pn;
                 const double wgs = std::ceil((double)(nn * tiles_of(64 * mi)) / cus);
-                const double st = mi == 1 ? 0.78 * (1.0 + 0.9 * (wgs - 1.0)) : 2.55 * (1.85 * std::floor(wgs / 2) + std::fmod(wgs, 2.0));
-                const double t = (double)pn * st * (mi == 1 && tiles_of(64) > cus ? 1.25 : 1.0) + (mi == 2 ? 5.0 : 0.0) +
+                const double st = mi == 1 ? 0.78 * (1.0 + 0.9 * (wgs - 1.0)) : 1.75 * wgs;
+                const double t = (double)pn * st * (mi == 1 && tiles_of(64) > cus ? 1.25 : 1.0) + (mi == 2 ? 5.0 * wgs : 0.0) +
                                  (nn > 1 ? (nn > 16 ? 8.0 : 5.0) + (double)nn * numel(dw) * 8 / 5e6 : 0.0);
                 if (t < least) { least = t; MI = mi; slices = nn; }
             }
@@ -780,6 +793,7 @@ static bool conv_wgrad_product(const mjt_tensor* x, const mjt_tensor* dy, const 
             }
     }
     const int NI = MI;
+    const bool split = !half && MI == 2;
     const int64_t tiles = tiles_of(64 * MI);
     if (slices * numel(dw) * 4 > (int64_t(1) << 30)) return false;
     const int64_t per = (stages + slices - 1) / slices;
@@ -794,9 +808,9 @@ static bool conv_wgrad_product(const mjt_tensor* x, const mjt_tensor* dy, const 
     if (!k) {
         std::ostringstream name;
         name << "mjt_conv_wgrad_igemm_" << mjt_dtype_name(x->dtype) << "_c" << C << "_k" << K << "_" << H << "x" << W << "_r" << R << "x" << S << "_s" << p->stride_h << "x" << p->stride_w << "_p"
-             << p->pad_h << "x" << p->pad_w << "_d" << p->dil_h << "x" << p->dil_w << "_" << 64 * MI << "x" << 64 * NI;
+             << p->pad_h << "x" << p->pad_w << "_d" << p->dil_h << "x" << p->dil_w << (split ? "_parts_" : "_") << 64 * MI << "x" << 64 * NI;
         std::ostringstream src;
-        src << "#define ENTRY " << name.str() << "\n#define CONV 2\n#define IN " << in << "\n#define OUT 2\n#define MI " << MI << "\n#define NI " << NI << "\n#define A_KCONT 1\n#define B_KCONT 1"
+        src << "#define ENTRY " << name.str() << "\n#define SPLIT " << (split ? 1 : 0) << "\n#define CONV 2\n#define IN " << in << "\n#define OUT 2\n#define MI " << MI << "\n#define NI " << NI << "\n#define A_KCONT 1\n#define B_KCONT 1"
             << "\n#define C_ " << C << "\n#define H_ " << H << "\n#define W_ " << W << "\n#define K_ " << K << "\n#define R_ " << R << "\n#define S_ " << S << "\n#define OH_ " << OH
             << "\n#define OW_ " << OW << "\n#define SH " << p->stride_h << "\n#define SW " << p->stride_w << "\n#define PH " << p->pad_h << "\n#define PW " << p->pad_w << "\n#define DH " << p->dil_h
             << "\n#define DW " << p->dil_w << "\n";
@@ -809,7 +823,7 @@ static bool conv_wgrad_product(const mjt_tensor* x, const mjt_tensor* dy, const 
                             (uint64_t)(numel(x) * esz), (uint64_t)(K * CRS)};
     const int64_t grid = (slices * tiles + 7) / 8 * 8;
     MJT_CHECK(grid < (int64_t(1) << 31), "conv wgrad: launch too large");
-    jit_launch(k, (unsigned)grid, 1, 256, 0, a);
+    jit_launch(k, (unsigned)grid, 1, product_threads(split), 0, a);
     if (!in_place) fold_wgrad_slices(part, slices, dw);
     set_last_kernel(k->name.c_str());
     return true;

@@ -166,42 +166,59 @@ void gemm_launch(int in_dtype, int out_dtype, const void* A, const void* B, void
         // the caller's tile, if it names one (tile_m x tile_n of 64, 128 or 256)
         if (tile_m == 64 || tile_m == 128 || tile_m == 256) best_mi = tile_m / 64;
         if (tile_n == 64 || tile_n == 128 || tile_n == 256) best_ni = tile_n / 64;
-        // Few tiles and a long sum: the sum is cut into slices, whose float32 results a reduce launch adds up.  A stage of a
-        // 64 x 64 tile takes about 0.75 us in float32 and 0.5 in 16 bits with a compute unit to itself, 1.75 / 2.6 / 3.4 times that
+        // Few tiles and a long sum: the sum is cut into slices, whose float32 results a reduce launch adds up.  A stage (32 float32 or 64
+        // 16-bit elements of the sum) of a 64 x 64 tile takes about 0.75 us in float32 and 0.5 in 16 bits with a compute unit to itself, 1.75 / 2.6 / 3.4 times that
         // with two / three / four workgroups a unit; the reduce launch 5 us and its traffic.  At most 16 slices: their reduce is
         // a single launch, which leaves the scratch memory alone.  (us whole / in slices; a^T b: 512 x 512 x 8192 float32
         // 183 / 50, bfloat16 64.5 / 22.7; 64 x 64 x 4096 float32 94 / 13.5; 1024 x 512 x 4096 float32 96 / 50; a b^T:
         // 256 x 1024 x 1024 float32 20.1 / 12.4; 1024 x 1024 x 2048 a^T b, 256 tiles, 50.4 / 50.6, stays whole.)
         const int64_t ks = esz == 2 ? 64 : 32, stages = (K + ks - 1) / ks;
         int64_t slices = 1, per = stages;
-        if (batch == 1 && !tile_m && !tile_n && ldc == N) {
-            const double st = esz == 2 ? 0.5 : 0.75;
-            auto crowd = [&](double wgs) { const double r = std::ceil(wgs / cus); return 1.0 + 0.8 * (r - 1.0); };
-            const double tiles64 = (double)((M + 63) / 64) * ((N + 63) / 64);
-            const double whole = (double)stages * st * crowd(tiles64) * (best_mi * best_ni > 1 ? 0.95 : 1.0);
-            double least = 0.9 * whole;
-            for (int64_t n = 2; n <= 16 && n <= stages / 4; n++) {
+        bool split = false;
+        const bool sliceable = batch == 1 && !tile_m && !tile_n && ldc == N;
+        const double tiles64 = (double)((M + 63) / 64) * ((N + 63) / 64) * batch;
+        auto crowd = [&](double wgs) { const double r = std::ceil(wgs / cus); return 1.0 + 0.8 * (r - 1.0); };
+        const double st = esz == 2 ? 0.5 : 0.75;
+        double least = (double)stages * st * crowd(tiles64) * (best_mi * best_ni > 1 ? 0.95 : 1.0);
+        // float32 sums of four stages and more go as products of bfloat16 parts (kernels/gemm_mfma.h) on 128 x 64, 64 x 128 or
+        // 128 x 128 tiles, whole or in slices, where that is estimated to take less.  A stage takes 0.92 us on 128 x 64 tiles and 1.45
+        // on 128 x 128, a little more where an operand is transposed on the way; a round of workgroups adds a first load and a
+        // store that nothing overlaps.  64 x 64 tiles stay with the float32 MFMAs: their stage is bound by the splitting (46 to
+        // 56 us / 52 to 57 for a^T b 1024 x 1024 x 2048, 17.1 / 15.7 for a b^T 8192 x 64 x 1024).
+        // us, float32 MFMAs on the tiles chosen before / so: a b^T 2048 x 1024 x 1024 42 / 32.7 (128 x 64), a b 45.6 / 35.7, a^T b 1024 x
+        // 1024 x 2048 54 / 40.5 (128 x 128, 4 slices), a b^T 2048^3 127 / 94 (128 x 128), 4096^3 966 / 709, 512 x 512 x 8192 a^T b
+        // 55 / 39, 64 x 512 x 512 x 256 143 / 65.5, 12 x 384 x 384 x 384 35.5 / 17.2.
+        const bool parts = in_dtype == MJT_FLOAT32 && stages >= 4;
+        for (int t = 0; t < (parts ? 4 : 1); t++) {
+            const int mi = t == 1 || t == 3 ? 2 : 1, ni = t >= 2 ? 2 : 1;
+            const double tiles = (double)((M + 64 * mi - 1) / (64 * mi)) * ((N + 64 * ni - 1) / (64 * ni)) * batch;
+            for (int64_t n = t ? 1 : 2; n == 1 || (sliceable && n <= 16 && n <= stages / 4); n++) {
                 const int64_t pn = (stages + n - 1) / n, nn = (stages + pn - 1) / pn;
-                const double t = (double)pn * st * crowd(tiles64 * nn) + 5.0 + (double)nn * M * N * 8 / 3e6;
-                if (t < least && nn * M * N * 4 <= (int64_t(256) << 20)) { least = t; slices = nn; per = pn; }
+                const double rounds = std::ceil(tiles * nn / cus);
+                double us = t ? (nn > 1 ? 4.0 + (double)nn * M * N * 8 / 4.5e6 : -2.0) : nn > 1 ? 5.0 + (double)nn * M * N * 8 / 3e6 : 0.0;
+                if (t == 0) us = (us + (double)pn * st * crowd(tiles * nn)) / 0.9;
+                else if (t == 3) us += rounds * ((double)pn * (a_kcont && b_kcont ? 1.45 : 1.55) + 6.5);
+                else us += rounds * ((double)pn * (a_kcont && b_kcont ? 0.92 : 1.05) * (rounds > 1 ? 0.9 : 1.0) * (t == 2 ? 1.06 : 1.0) + 3.5);
+                if (us < least && (nn == 1 || nn * M * N * 4 <= (int64_t(256) << 20))) {
+                    least = us; slices = nn; per = pn; split = t > 0; best_mi = mi; best_ni = ni;
+                }
             }
         }
         void* part_mem = slices > 1 ? scratch_if_any((size_t)(slices * M * N * 4)) : nullptr;
         if (!part_mem) slices = 1;
-        if (slices > 1) best_mi = best_ni = 1;
         const int MI = best_mi, NI = best_ni;
         const int in = in_dtype == MJT_BFLOAT16 ? 0 : in_dtype == MJT_FLOAT16 ? 1 : 2;
         const int out = slices > 1 || out_dtype == MJT_FLOAT32 ? 2 : out_dtype == MJT_BFLOAT16 ? 0 : 1;
         const bool one_stage = stages == 1 && !getenv("MJT_GEMM_TWO_BUFFERS");       // a single stage of the kernel's k loop
         std::ostringstream key;
-        key << "gemm|" << in << out << MI << NI << a_kcont << b_kcont << one_stage << (slices > 1);
+        key << "gemm|" << in << out << MI << NI << a_kcont << b_kcont << one_stage << (slices > 1) << split;
         JitKernel* k = cached(key.str());
         if (!k) {
             std::ostringstream name;
             name << "mjt_gemm_mfma_" << mjt_dtype_name(in_dtype) << "_" << (out == 2 ? "float32" : mjt_dtype_name(out_dtype)) << "_" << 64 * MI << "x" << 64 * NI
-                 << (a_kcont ? "_n" : "_t") << (b_kcont ? "t" : "n") << (one_stage ? "_k1" : "") << (slices > 1 ? "_slices" : "");
+                 << (a_kcont ? "_n" : "_t") << (b_kcont ? "t" : "n") << (one_stage ? "_k1" : "") << (split ? "_parts" : "") << (slices > 1 ? "_slices" : "");
             std::ostringstream src;
-            src << "#define NBUF " << (one_stage ? 1 : 2) << "\n#define SLICED " << (slices > 1 ? 1 : 0) << "\n";
+            src << "#define NBUF " << (one_stage ? 1 : 2) << "\n#define SLICED " << (slices > 1 ? 1 : 0) << "\n#define SPLIT " << (split ? 1 : 0) << "\n";
             src << "#define ENTRY " << name.str() << "\n#define IN " << in << "\n#define OUT " << out << "\n#define MI " << MI
                 << "\n#define NI " << NI << "\n#define A_KCONT " << (a_kcont ? 1 : 0) << "\n#define B_KCONT " << (b_kcont ? 1 : 0) << "\n";
             src << embedded_source("gemm_mfma.h") << "\n";
@@ -209,10 +226,11 @@ void gemm_launch(int in_dtype, int out_dtype, const void* A, const void* B, void
             remember(key.str(), k);
         }
         const int64_t tiles = ((M + 64 * MI - 1) / (64 * MI)) * ((N + 64 * NI - 1) / (64 * NI));
-        const int64_t grid = (tiles + 7) / 8 * 8;
+        const int64_t grid = (tiles * (slices > 1 ? slices : batch) + 7) / 8 * 8;
         MJT_CHECK(grid < (int64_t(1) << 31), "matmul: launch too large");
         if (slices == 1) {
-            jit_launch(k, (unsigned)grid, (unsigned)batch, 256, 0, args);
+            args[3] |= (uint64_t)batch << 32;
+            jit_launch(k, (unsigned)grid, 1, product_threads(split), 0, args);
             return;
         }
         mjt_tensor part{}, whole{};
@@ -228,7 +246,7 @@ void gemm_launch(int in_dtype, int out_dtype, const void* A, const void* B, void
         args[2] = bits_of_ptr(part.ptr);
         args[9] = (uint64_t)per;
         args[11] = (uint64_t)(M * N);
-        jit_launch(k, (unsigned)grid, (unsigned)slices, 256, 0, args);
+        jit_launch(k, (unsigned)grid, 1, product_threads(split), 0, args);
         if (mjt_reduce(&part, &whole, MJT_OP_ADD, 0b01) != MJT_OK) MJT_FAIL(MJT_ERR_DEVICE, "matmul: adding up the slices failed: " << mjt_last_error());
         set_last_kernel(k->name.c_str());
         return;

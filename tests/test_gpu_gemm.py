@@ -297,3 +297,130 @@ def test_gemm_batches_of_few_tiles(gpu, dt, batch, M, N, K, ta, tb):
         with pytest.MonkeyPatch.context() as m:
             m.setenv("MJT_GEMM_DMA", "128")
             assert "_direct" in _run(L.load(), dt, dt, M, K, N, ta, tb, batch=(batch,), seed=M + K)
+
+
+# ---- float32 products of bfloat16 parts: a value is h + m + l, six of nine products are summed, an MFMA rounds once per 16 of them ----
+def _parts_bound(A, B, K):
+    """Two sums of K / 16 MFMAs of up to three products each and one addition, every rounding at most 2^-23 (the MFMA may truncate) of
+    the sum of magnitudes; what is left out of a product is below 2^-25 of it."""
+    with np.errstate(all="ignore"):
+        return (K / 16 * 4 + 8) * 2.0 ** -23 * (np.abs(A) @ np.abs(B))
+
+
+def _parts_product(lib, A, B, ta, tb, batch=()):
+    pa, pb = _to_dev(A), _to_dev(B)
+    M, K = A.shape[-1 if ta else -2], A.shape[-2 if ta else -1]
+    N = B.shape[-2 if tb else -1]
+    pc = L.alloc(int(np.prod(batch, dtype=np.int64)) * M * N * 4)
+    try:
+        t = [L.tensor(pa, "float32", A.shape), L.tensor(pb, "float32", B.shape), L.tensor(pc, "float32", tuple(batch) + (M, N))]
+        L.check(lib.mjt_matmul(*[ctypes.byref(q) for q in t], ta, tb))
+        return L.d2h(pc, tuple(batch) + (M, N), np.float32).astype(np.float64), L.last_kernel()
+    finally:
+        for p in (pa, pb, pc):
+            L.free(p)
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,K,N,batch,tile", [(2044, 1020, 1000, (), "128x64"), (1916, 260, 2100, (), "128x128"), (1020, 2052, 1012, (), "slices"),
+                                              (384, 380, 364, (12,), "parts"), (100, 2500, 4100, (), "parts")])
+def test_gemm_float32_parts(gpu, M, K, N, batch, tile, ta, tb):
+    """Tiles that hang over both edges, a sum that ends inside a stage and inside a chunk, slices, a batch; operands over nine decades with
+    zeros among them."""
+    rng = np.random.default_rng(M + K)
+    scale = lambda shape: 10.0 ** rng.integers(-4, 5, shape) * (rng.random(shape) > 0.1)
+    A = (rng.standard_normal(batch + ((K, M) if ta else (M, K)))).astype(np.float32)
+    B = (rng.standard_normal(batch + ((N, K) if tb else (K, N)))).astype(np.float32)
+    A = (A * scale(A.shape)).astype(np.float32)
+    got, kern = _parts_product(L.load(), A, B, ta, tb, batch)
+    assert "_parts" in kern and (tile in kern), kern
+    a64 = np.swapaxes(A, -1, -2).astype(np.float64) if ta else A.astype(np.float64)
+    b64 = np.swapaxes(B, -1, -2).astype(np.float64) if tb else B.astype(np.float64)
+    assert (np.abs(got - a64 @ b64) <= _parts_bound(a64, b64, K)).all(), kern
+
+
+@pytest.mark.parametrize("what", ["inf", "nan", "rounds to inf", "denormal", "tiny", "small products", "overflow", "zeros"])
+def test_gemm_float32_parts_hand_over(gpu, what):
+    """Operands whose parts leave bfloat16's range or whose sums are not finite: the tiles concerned run on the float32 MFMAs, results are
+    what float32 gives; the other tiles stay."""
+    rng = np.random.default_rng(5)
+    M, K, N = 2048, 1024, 1024
+    A, B = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((N, K)).astype(np.float32)
+    if what == "inf":
+        A[5, 7], A[700, 1000], B[1000, 3] = np.inf, -np.inf, np.inf
+    elif what == "nan":
+        A[1500, 1023], B[64, 0] = np.nan, np.nan
+    elif what == "rounds to inf":                                      # finite, but the first part is not
+        A[9, 11], A[1400, 900] = 3.4e38, -3.4028e38
+        B *= 1e-3
+    elif what == "denormal":
+        A[130], A[1999, ::2] = 1e-40, 1.1e-39
+        B[:, :] *= np.float32(1e25)
+    elif what == "tiny":                                               # the second and third parts are below the normal range
+        A *= np.float32(1e-35)
+        B *= np.float32(1e33)
+    elif what == "small products":
+        A *= np.float32(1e-17)
+        B *= np.float32(1e-19)
+    elif what == "overflow":
+        A[77] *= np.float32(1e30)
+        B[900] *= np.float32(1e12)
+    else:
+        A[:200], B[:, 100:300] = 0.0, 0.0
+    got, kern = _parts_product(L.load(), A, B, 0, 1)
+    assert "_parts" in kern, kern
+    a, b = A.astype(np.float64), B.astype(np.float64).T
+    with np.errstate(all="ignore"):
+        want, bound = a @ b, _parts_bound(a, b, K)
+        f32 = want.astype(np.float32)
+    if what == "overflow":                                             # partial sums may pass the largest float before the total does
+        sure = (np.abs(a) @ np.abs(b) < 3e38) | (np.abs(want) > 1e39)
+        assert np.array_equal(np.isfinite(got)[sure], np.isfinite(f32)[sure]) and (~np.isfinite(f32)).any()
+    else:
+        assert np.array_equal(np.isnan(got), np.isnan(f32))
+        assert np.array_equal(got[np.isinf(f32)], f32[np.isinf(f32)].astype(np.float64))
+    ok = np.isfinite(f32) & np.isfinite(got)
+    # (a sum below the normal range may be taken for zero)
+    assert (np.abs(got[ok] - want[ok]) <= bound[ok] + K * 2.0 ** -126).all(), np.abs(got[ok] - want[ok]).max()
+
+
+def _columns(x, R, stride, pad):
+    n, c, h, w = x.shape
+    xp = np.pad(x, ((0, 0), (0, 0), (pad, pad), (pad, pad)))
+    v = np.lib.stride_tricks.sliding_window_view(xp, (R, R), axis=(2, 3))[:, :, ::stride, ::stride]       # n c oh ow r s
+    return np.ascontiguousarray(v.transpose(0, 2, 3, 1, 4, 5)).reshape(n * v.shape[2] * v.shape[3], c * R * R), v.shape[2]
+
+
+@pytest.mark.parametrize("xs,k,R,stride,tiny", [((16, 40, 27, 27), 200, 3, 1, False), ((16, 39, 27, 27), 100, 3, 1, False), ((32, 64, 56, 56), 128, 3, 2, False),
+                                                ((16, 40, 27, 27), 200, 3, 1, True), ((32, 64, 56, 56), 128, 3, 2, True)])
+def test_conv_float32_parts(gpu, xs, k, R, stride, tiny):
+    """The gathering forward and weight-gradient products on bfloat16 parts; with operands whose parts leave the range too."""
+    lib = L.load()
+    rng = np.random.default_rng(k)
+    x, w = rng.standard_normal(xs).astype(np.float32), rng.standard_normal((k, xs[1], R, R)).astype(np.float32)
+    if tiny:
+        x[3, 5] *= np.float32(1e-34)
+        x[4, 6, 2, 2] = np.inf
+    cols, o = _columns(x.astype(np.float64), R, stride, R // 2)
+    dy = rng.standard_normal((xs[0], k, o, o)).astype(np.float32)
+    px, pw, pdy, py, pdw = _to_dev(x), _to_dev(w), _to_dev(dy), L.alloc(dy.nbytes), L.alloc(w.nbytes)
+    try:
+        tx, tw, tdy, ty, tdw = L.tensor(px, "float32", xs), L.tensor(pw, "float32", w.shape), L.tensor(pdy, "float32", dy.shape), L.tensor(py, "float32", dy.shape), L.tensor(pdw, "float32", w.shape)
+        p = L.ConvParams(stride, stride, R // 2, R // 2, 1, 1)
+        L.check(lib.mjt_conv2d_meta(ctypes.byref(tx), ctypes.byref(tw), ctypes.byref(ty), ctypes.byref(p)))
+        assert L.last_kernel().startswith("mjt_conv_igemm_float32") and "_parts_" in L.last_kernel(), L.last_kernel()
+        y = L.d2h(py, dy.shape, np.float32).astype(np.float64).transpose(0, 2, 3, 1).reshape(-1, k)
+        L.check(lib.mjt_conv2d_meta_wgrad_grouped(ctypes.byref(tx), ctypes.byref(tdy), ctypes.byref(tdw), ctypes.byref(p), 1))
+        split = "_parts_" in L.last_kernel()
+        dw = L.d2h(pdw, w.shape, np.float32).astype(np.float64).reshape(k, -1)
+    finally:
+        for q in (px, pw, pdy, py, pdw):
+            L.free(q)
+    assert split or stride == 1
+    w2, d2 = w.astype(np.float64).reshape(k, -1), dy.astype(np.float64).transpose(0, 2, 3, 1).reshape(-1, k).T
+    with np.errstate(all="ignore"):
+        for got, a, b in ((y, cols, w2.T), (dw, d2, cols)):
+            want, bound = a @ b, _parts_bound(a, b, a.shape[1])
+            assert np.array_equal(np.isfinite(got), np.isfinite(want))
+            ok = np.isfinite(want)
+            assert (np.abs(got[ok] - want[ok]) <= bound[ok]).all()
