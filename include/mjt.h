@@ -244,6 +244,23 @@ int mjt_fused_elementwise(const mjt_fused_desc* desc);
  * mjt_reduce. */
 int mjt_fused_reduce(const mjt_fused_desc* desc, const mjt_tensor* y, int op, uint32_t reduce_mask);
 
+/* Fused groups and the reductions between them in one kernel: a normalisation
+ * or softmax, forward and backward (executor.cc:555: element, broadcast and
+ * reduce ops share a group; the reference runs such a graph as one group per
+ * reduce).  `desc` is a group over the shape whose last n_row_axes axes are the
+ * rows' elements; beside the kinds above it has
+ *   MJT_FOP_ROW_REDUCE  op = add, mean, maximum or minimum over a row;
+ *   MJT_FOP_COLUMN_SUM  sum over the other axes, into an output var that no op reads.
+ * An input var is full, one value per row (bcast_mask = exactly the axes of
+ * extent > 1 among the last n_row_axes), one per column (exactly the others) or
+ * a single element; `reserved` of the other vars: MJT_SPACE_* | MJT_ROUNDED (the value takes its dtype although
+ * it is not stored).  Accumulation as in mjt_reduce.  MJT_ERR_UNSUPPORTED for what
+ * the kernel does not take (rows of more than 16384 elements, reductions in
+ * other types than float32 and the 16-bit floats): the parts run one by one. */
+typedef enum { MJT_FOP_ROW_REDUCE = 4, MJT_FOP_COLUMN_SUM = 5 } mjt_rows_kind;
+typedef enum { MJT_SPACE_FULL = 0, MJT_SPACE_ROW = 1, MJT_SPACE_COLUMN = 2, MJT_ROUNDED = 256 } mjt_rows_space;
+int mjt_fused_rows(const mjt_fused_desc* desc, int n_row_axes);
+
 /* A fused group that ends in a ReindexReduceOp (element, broadcast, reindex and
  * reduce-type ops share a group in the reference, executor.cc:555; this is the
  * gradient of pooling, python/jittor/pool.py:200-208 differentiated): `desc`

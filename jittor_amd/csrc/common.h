@@ -132,6 +132,7 @@ const char* embedded_source(const char* name);
 int64_t fused_validate(const mjt_fused_desc* d, std::vector<int>* inputs, bool outputs_need_data,
                        bool allow_gathered = false);   // returns the element count
 std::string fused_emit_ops(const mjt_fused_desc* d, bool store_outputs);
+std::string fused_op_expr(const mjt_fused_desc* d, const mjt_fused_op& o);
 
 // plan cache: per entry point, a string key maps to a prepared plan object
 // (parsed expressions, chosen kernel); see op_*.cpp

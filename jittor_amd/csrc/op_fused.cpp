@@ -85,6 +85,25 @@ int64_t fused_validate(const mjt_fused_desc* d, std::vector<int>* inputs_out, bo
     return total;
 }
 
+// One op as a C expression over its inputs' `vI`.
+std::string fused_op_expr(const mjt_fused_desc* d, const mjt_fused_op& o) {
+    const mjt_fused_var& ov = d->vars[o.out];
+    const char* Tz = dtype_cname(ov.dtype);
+    std::string expr;
+    if (o.kind == MJT_FOP_BROADCAST) {
+        expr = vname(o.in[0]);
+    } else if (o.kind == MJT_FOP_UNARY) {
+        expr = std::string("mjt_") + mjt_op_name(o.op) + "<" + Tz + ">(" + vname(o.in[0]) + ")";
+    } else if (o.kind == MJT_FOP_BINARY) {
+        expr = std::string("mjt_") + mjt_op_name(o.op) + "<" + Tz + ">(" + vname(o.in[0]) + ", " + vname(o.in[1]) + ")";
+    } else {
+        expr = std::string("(") + vname(o.in[0]) + " ? (" + Tz + ")(" + vname(o.in[1]) + ") : (" + Tz + ")(" +
+               vname(o.in[2]) + "))";
+    }
+    // bool results are wrapped in (bool)(...) (type/common_op_type.cc:161)
+    return ov.dtype == MJT_BOOL ? "(bool)(" + expr + ")" : expr;
+}
+
 // The op chain for one element as C statements: every var i becomes `vI`; intermediates keep the natural
 // type of their expression, outputs take their dtype (and are also written to `outI.v[k]` when
 // store_outputs is set).
@@ -94,20 +113,7 @@ std::string fused_emit_ops(const mjt_fused_desc* d, bool store_outputs) {
         const mjt_fused_op& o = d->ops[k];
         const mjt_fused_var& ov = d->vars[o.out];
         const char* Tz = dtype_cname(ov.dtype);
-        std::string expr;
-        if (o.kind == MJT_FOP_BROADCAST) {
-            expr = vname(o.in[0]);
-        } else if (o.kind == MJT_FOP_UNARY) {
-            expr = std::string("mjt_") + mjt_op_name(o.op) + "<" + Tz + ">(" + vname(o.in[0]) + ")";
-        } else if (o.kind == MJT_FOP_BINARY) {
-            expr = std::string("mjt_") + mjt_op_name(o.op) + "<" + Tz + ">(" + vname(o.in[0]) + ", " + vname(o.in[1]) + ")";
-        } else {
-            expr = std::string("(") + vname(o.in[0]) + " ? (" + Tz + ")(" + vname(o.in[1]) + ") : (" + Tz + ")(" +
-                   vname(o.in[2]) + "))";
-        }
-        // bool results are wrapped in (bool)(...) (type/common_op_type.cc:161); outputs take the
-        // declared dtype, intermediates keep the natural type of the expression
-        if (ov.dtype == MJT_BOOL) expr = "(bool)(" + expr + ")";
+        const std::string expr = fused_op_expr(d, o);
         if (ov.role == MJT_VAR_OUTPUT) {
             body << "const " << Tz << " " << vname(o.out) << " = (" << Tz << ")(" << expr << "); ";
             if (store_outputs) body << "out" << o.out << ".v[k] = " << vname(o.out) << "; ";

@@ -10,10 +10,12 @@ once.  Everything runs on the device; there is no host path.
 """
 import ctypes
 import math
+import sys
 import threading
 
 from . import _lib
 from . import core
+from . import rowfuse
 from .core import (Var, Buffer, UnaryOp, BinaryOp, TernaryOp, BroadcastOp,
                    ReduceOp, ReindexOp, ReindexReduceOp)
 from ._lib import MjtError
@@ -21,7 +23,7 @@ from . import profiler as _profiler
 from .flags import flags
 
 stats = {"launches": 0, "fused_groups": 0, "fused_reduces": 0, "conv_matches": 0, "syncs": 0, "sunk_ops": 0, "matmul_matches": 0,
-         "wgrad_kernel": 0, "wgrad_chunked": 0, "gather_reduces": 0, "fused_scatters": 0, "plans": 0, "replays": 0, "recorded_launches": 0}
+         "wgrad_kernel": 0, "wgrad_chunked": 0, "gather_reduces": 0, "fused_scatters": 0, "fused_rows": 0, "plans": 0, "replays": 0, "recorded_launches": 0}
 
 
 class ConvUnit:
@@ -1048,28 +1050,52 @@ def _execute(ops, target_ids):
         rec = _profiler.active()
         return call() if rec is None else rec.run(call, kind, *io())
 
+    def run_members(members):
+        timed(lambda: _run_group(members, consumers, target_ids, pre=pre), "fused", lambda: group_io(members))
+
+    def run_node(op):
+        sc = scatter_of.get(op.id)
+        if sc is not None:
+            if timed(lambda: _run_group(sc[0], consumers, target_ids, scatter=op, gathered=sc[1], pre=pre), "fused+scatter",
+                     lambda: group_io(sc[0], op.out)):
+                return
+            for p in sc[1].values():                           # not taken in that form: the plain sequence
+                timed(lambda: _run_single(p), p.kind, lambda: (sum(u.nbytes for u in p.inputs), p.out.nbytes))
+            run_members(sc[0])
+        members = prologue_of.get(op.id)
+        if members is not None:
+            if timed(lambda: _run_group(members, consumers, target_ids, reduce=op, pre=pre), "fused+reduce",
+                     lambda: group_io(members, op.out)):
+                return
+            run_members(members)
+        timed(lambda: _run_single(op), op.kind, lambda: (sum(u.nbytes for u in op.inputs), op.out.nbytes))
+
+    def reads_of(members):
+        made = {op.out.id for op in members}
+        return {u.id for op in members for u in ins(op)} - made
+
+    tasks = []
     for s in range(nstage):
         for members in by_stage_groups[s]:
             if id(members) not in absorbed_groups:
-                timed(lambda: _run_group(members, consumers, target_ids, pre=pre), "fused", lambda: group_io(members))
+                tasks.append(rowfuse.Task(lambda members=members: run_members(members), reads_of(members), {op.out.id for op in members}, members))
         for op in by_stage_other[s]:
             if op.id in absorbed_nodes:
                 continue
-            sc = scatter_of.get(op.id)
-            if sc is not None:
-                if timed(lambda: _run_group(sc[0], consumers, target_ids, scatter=op, gathered=sc[1], pre=pre), "fused+scatter",
-                         lambda: group_io(sc[0], op.out)):
-                    continue
-                for p in sc[1].values():                       # not taken in that form: the plain sequence
-                    timed(lambda: _run_single(p), p.kind, lambda: (sum(u.nbytes for u in p.inputs), p.out.nbytes))
-                timed(lambda: _run_group(sc[0], consumers, target_ids, pre=pre), "fused", lambda: group_io(sc[0]))
-            members = prologue_of.get(op.id)
-            if members is not None:
-                if timed(lambda: _run_group(members, consumers, target_ids, reduce=op, pre=pre), "fused+reduce",
-                         lambda: group_io(members, op.out)):
-                    continue
-                timed(lambda: _run_group(members, consumers, target_ids, pre=pre), "fused", lambda: group_io(members))
-            timed(lambda: _run_single(op), op.kind, lambda: (sum(u.nbytes for u in op.inputs), op.out.nbytes))
+            members, reads = prologue_of.get(op.id, ()), {u.id for u in op.inputs}
+            if op.id in scatter_of:
+                sc = scatter_of[op.id]
+                reads = (reads | reads_of(sc[0])) - {q.out.id for q in sc[0]} | {u.id for p in sc[1].values() for u in p.inputs}
+                reads -= set(sc[1])
+            elif members:
+                reads = reads_of(members)
+            plain = isinstance(op, ReduceOp)
+            tasks.append(rowfuse.Task(lambda op=op: run_node(op), reads, {op.out.id}, members if plain else (), op if plain else None))
+    # chains of groups and row reduces over one shape run as one kernel each (while a profile is taken the parts are timed as they are)
+    if flags["enable_row_fusion"] and _profiler.active() is None:
+        tasks = rowfuse.merge(tasks, ins, pre, consumers, target_ids, sys.modules[__name__]) or tasks
+    for t in tasks:
+        t.run()
     # materialised vars become leaves: the graph behind them can be dropped
     for op in sched:
         if op.out._buf is not None:

@@ -1301,3 +1301,23 @@ def test_replayed_result_is_the_memory_of_its_own_input(fake_buffers, shared_fir
         b, y = step(shared)
         assert y._buf is b._buf
     assert fake_buffers.stats["replays"] > replays + 1
+
+
+def test_fused_rows_descriptor_is_checked(compile_only):
+    """mjt_fused_rows: what it hands back runs part by part, what makes no sense is an error; nothing is launched."""
+    L, lib = compile_only, compile_only.load()
+    f32, P = L.DTYPE_CODE["float32"], 0x1000
+
+    def call(shape, n_row, mask=0, reduce_op="add", dtype=f32, in_space=1, second_in=1):
+        fv = [L.FusedVar(L.VAR_INPUT, dtype, P, 0, 0, 0, 0), L.FusedVar(L.VAR_INTERMEDIATE, dtype, None, 0, 0, 0, in_space),
+              L.FusedVar(L.VAR_INPUT, dtype, P, 0, 0, mask, 0), L.FusedVar(L.VAR_OUTPUT, dtype, P, 0, 0, 0, 0)]
+        fo = [L.FusedOp(L.FOP_ROW_REDUCE, L.OP_CODE[reduce_op], (0, 0, 0), 1), L.FusedOp(L.FOP_BINARY, L.OP_CODE["divide"], (2, second_in, 0), 3)]
+        d = L.FusedDesc(len(shape), tuple(shape), 4, (L.FusedVar * 4)(*fv), 2, (L.FusedOp * 2)(*fo))
+        return lib.mjt_fused_rows(ctypes.byref(d), n_row)
+    assert call((100, 512), 1) == 0 and call((7, 9, 30, 20), 2) == 0 and call((5, 16384), 1, reduce_op="maximum") == 0
+    assert call((100, 512), 1, mask=0b10) == 0 and call((100, 512), 1, mask=0b01) == 0 and call((100, 512), 1, mask=0b11) == 0
+    assert call((7, 9, 30, 20), 2, mask=0b1000) == L.ERR_UNSUPPORTED                   # along part of the rows
+    assert call((5, 16385), 1) == L.ERR_UNSUPPORTED and call((0, 64), 1) == L.ERR_UNSUPPORTED and call((64, 0), 1) == L.ERR_UNSUPPORTED
+    assert call((100, 512), 1, reduce_op="multiply") == L.ERR_UNSUPPORTED and call((100, 512), 1, dtype=L.DTYPE_CODE["int32"]) == L.ERR_UNSUPPORTED
+    assert call((100, 512), 0) == L.ERR_INVALID and call((100, 512), 2) == L.ERR_INVALID
+    assert call((100, 512), 1, in_space=0) == L.ERR_INVALID and call((100, 512), 1, second_in=9) == L.ERR_INVALID
