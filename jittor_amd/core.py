@@ -9,9 +9,6 @@ Nothing executes until a Var is synchronised (lazy_execution,
 var_holder.cc:25-33); execution is in executor.py.
 """
 import collections
-import functools
-import itertools
-import math
 import numbers
 import threading
 import weakref
@@ -19,6 +16,8 @@ import weakref
 import numpy as np
 
 from . import _lib
+_lib.load()              # says what to build where nothing is
+from . import _graph
 from . import dtypes as dt
 from ._lib import MjtError
 from .flags import flags as _flags
@@ -40,7 +39,7 @@ class no_grad:
         return False
 
 
-_new_id = itertools.count(1).__next__
+_new_id = _graph.new_id
 _ref = weakref.ref
 
 
@@ -687,21 +686,10 @@ def unary_clone(x):
     return unary(x, "cast", force_dtype=x.dtype, allow_forward=False)
 
 
-_scalar_vars = {}        # (type, value, sign) -> the host Var of a Python number: `x * 2.0` builds no new array each time
+_scalar_vars = {}        # (type, value, sign[, dtype]) -> the host Var of a Python number: `x * 2.0` builds no new array each time
 
 
-def _as_var(v):
-    if isinstance(v, Var):
-        return v
-    tv = type(v)
-    if tv is float or tv is int or tv is bool:
-        key = (tv, v, math.copysign(1.0, v) if tv is float else 0)
-        got = _scalar_vars.get(key)
-        if got is None:
-            if len(_scalar_vars) >= 4096:
-                _scalar_vars.clear()
-            got = _scalar_vars[key] = array(v)
-        return got
+def _array_like(v):
     if isinstance(v, (numbers.Number, np.generic, list, tuple, np.ndarray, bool)):
         return array(v)
     raise TypeError("cannot convert %r to a Var" % type(v))
@@ -710,235 +698,17 @@ def _as_var(v):
 # --------------------------------------------------------------------------
 # constructors
 # --------------------------------------------------------------------------
-_DTYPE_SET, _UNARY_SET, _BINARY_SET = frozenset(_lib.DTYPES), frozenset(_lib.UNARY_OPS), frozenset(_lib.BINARY_OPS)
+_DTYPE_SET, _UNARY_SET, _BINARY_SET, _REDUCE_SET = (frozenset(names) for names in (_lib.DTYPES, _lib.UNARY_OPS, _lib.BINARY_OPS, dt.REDUCE_OPS))
+_MAX_DIM = _lib.MAX_DIM
 
-
-def unary(x, op, force_dtype=None, allow_forward=True):
-    """ops/unary_op.cc:860-889.  `op` is a unary op name or a dtype name."""
-    if not isinstance(x, Var):
-        x = _as_var(x)
-    if op in _DTYPE_SET and op != "void":
-        if op == x.dtype and allow_forward:
-            return x                      # forward(x), unary_op.cc:867-870
-        dtype, op = op, "cast"
-    elif op == "cast" and force_dtype is not None:
-        dtype = force_dtype
-    else:
-        if op not in _UNARY_SET:
-            raise ValueError("unknown unary op %r" % (op,))
-        dtype = dt.unary_dtype_infer(op, x.dtype)
-    y = Var(x.shape[:], dtype, UnaryOp(x, op), x.num)
-    if x.is_scalar:
-        y.is_scalar = True
-    return y
-
-
-def _need_broadcast(xshape, shape):
-    """ops/broadcast_to_op.cc:98-103."""
-    if len(xshape) < len(shape):
-        return True
-    for i in range(1, len(shape) + 1):
-        if xshape[-i] != shape[-i] and shape[-i] != 1:
-            return True
-    return False
-
-
-def _broadcast_shape(xshape, yshape, bmask, kmask):
-    """infer_shape of ops/broadcast_to_op.cc:119-168.  Returns
-    (zshape, bcast_mask, keepdims_mask, elements of zshape) with the implicit broadcasts added; the list is the caller's."""
-    zz, bmask, kmask, num = _broadcast_rule(tuple(xshape), tuple(yshape), bmask, kmask)
-    return list(zz), bmask, kmask, num
-
-
-@functools.lru_cache(maxsize=4096)           # (a pure function of extents and masks)
-def _broadcast_rule(xshape, yshape, bmask, kmask):
-    xdim, ydim = len(xshape), len(yshape)
-    cnt = bin(bmask & ~kmask).count("1")
-    zdim = max(xdim, ydim - cnt) + cnt
-    zz = [0] * zdim
-    xi, yi = xdim - 1, ydim - 1
-    for i in range(zdim - 1, -1, -1):
-        bx, by = xi >= 0, yi >= 0
-        xs = xshape[xi] if bx else 1
-        ys = yshape[yi] if by else 1
-        if bmask >> i & 1:
-            yi -= 1
-            if kmask >> i & 1:
-                xi -= 1
-            zz[i] = ys
-            continue
-        m = int(xs == 1 and (ys != 1 or not bx)) << i
-        bmask |= m
-        if bx:
-            kmask |= m
-        if (xs == 1 or ys == 1) and xs != ys:
-            zs = xs * ys
-        else:
-            if xs != ys:
-                raise ValueError("Shape not match %r %r" % (list(xshape), list(yshape)))
-            zs = xs
-        zz[i] = zs
-        xi -= 1
-        yi -= 1
-    if zdim > _lib.MAX_DIM:
-        raise ValueError("at most %d dims are supported" % _lib.MAX_DIM)
-    for e in zz:
-        if e < 0:
-            raise ValueError("Shape should greater than 0: %r" % (zz,))
-    return tuple(zz), bmask, kmask, math.prod(zz)
-
-
-def broadcast(x, shape, dims=()):
-    """broadcast(x, shape, dims) / broadcast(x, y, dims): `dims` name the new
-    axes of the output, the other axes align right to left
-    (ops/broadcast_to_op.cc:23-96)."""
-    x = _as_var(x)
-    if isinstance(shape, Var):
-        shape = shape.shape
-    shape = [int(s) for s in shape]
-    if isinstance(dims, numbers.Integral):
-        dims = (dims,)
-    dims = list(dims)
-    if not dims and not _need_broadcast(x.shape, shape):
-        return x                           # forward(x)
-    if len(shape) == 0:
-        raise ValueError("Number of shape should greater than 0.")
-    for s in shape:
-        if s < 0:
-            raise ValueError("Shape should greater than 0.")
-    ydim = max(x.ndim, len(shape) - len(dims)) + len(dims)
-    bmask = 0
-    for d in dims:
-        if d < 0:
-            d += ydim
-        if not (0 <= d < ydim):
-            raise ValueError("Wrong dims number: %r" % (dims,))
-        bmask |= 1 << d
-    zshape, bmask, kmask, num = _broadcast_shape(x.shape, shape, bmask, 0)
-    z = Var(zshape, x.dtype, BroadcastOp(x, bmask, kmask), num)
-    if x.is_scalar:
-        z.is_scalar = True
-    return z
+# made natively (csrc/py/graph.cpp): a step builds hundreds of these
+_graph.setup(globals())
+unary, binary, ternary, broadcast, reduce, make_number = _graph.unary, _graph.binary, _graph.ternary, _graph.broadcast, _graph.reduce, _graph.make_number
+_as_var, _broadcast_mask, _reduce_mask = _graph.as_var, _graph.broadcast_mask, _graph.reduce_mask
 
 
 def broadcast_var(x, y, dims=()):
     return broadcast(x, _as_var(y).shape, dims)
-
-
-def _broadcast_mask(x, shape, bmask, kmask):
-    """make_broadcast_to(x, shape, dims_mask, keepdims_mask), used by grads."""
-    if not bmask:
-        return x
-    zshape, bmask, kmask, num = _broadcast_shape(x.shape, shape, bmask, kmask)
-    z = Var(zshape, x.dtype, BroadcastOp(x, bmask, kmask), num)
-    if x.is_scalar:
-        z.is_scalar = True
-    return z
-
-
-def binary(x, y, op):
-    """ops/binary_op.cc:421-474: broadcasts are inserted when ranks differ or
-    an extent is 1 on one side only; other mismatches are errors."""
-    if not isinstance(x, Var):
-        x = _as_var(x)
-    if not isinstance(y, Var):
-        y = _as_var(y)
-    if op not in _BINARY_SET:
-        raise ValueError("unknown binary op %r" % (op,))
-    if x.shape == y.shape:
-        dtype = dt.binary_dtype_infer(op, x.dtype, y.dtype, x.is_scalar, y.is_scalar)
-        return Var(x.shape[:], dtype, BinaryOp(x, y, op), x.num)
-    need = x.ndim != y.ndim
-    for i in range(1, min(x.ndim, y.ndim) + 1):
-        xs, ys = x.shape[-i], y.shape[-i]
-        if (xs == 1 or ys == 1) and xs != ys:
-            need = True
-            continue
-        if xs != ys:
-            raise ValueError("Shape not match, x:%r y:%r" % (x.shape, y.shape))
-    if need:
-        xp = broadcast(x, y.shape)
-        yp = broadcast(y, x.shape)
-        return binary(xp, yp, op)
-    dtype = dt.binary_dtype_infer(op, x.dtype, y.dtype, x.is_scalar, y.is_scalar)
-    return Var(x.shape, dtype, BinaryOp(x, y, op))
-
-
-def ternary(cond, x, y):
-    """ops/ternary_op.cc:21-47."""
-    cond, x, y = _as_var(cond), _as_var(x), _as_var(y)
-    if cond.shape == x.shape == y.shape:
-        dtype = x.dtype if x.dtype == y.dtype else dt.dtype_infer(x.dtype, y.dtype, x.is_scalar, y.is_scalar)
-        return Var(x.shape[:], dtype, TernaryOp(cond, x, y), x.num)
-    bx = cond.ndim > x.ndim or cond.num > x.num
-    by = cond.ndim > y.ndim or cond.num > y.num
-    bx2 = cond.ndim < x.ndim or cond.num < x.num
-    by2 = cond.ndim < y.ndim or cond.num < y.num
-    if bx or by or bx2 or by2:
-        if bx2:
-            cond = broadcast(cond, x.shape)
-        if by2:
-            cond = broadcast(cond, y.shape)
-        bx = cond.ndim > x.ndim or cond.num > x.num
-        by = cond.ndim > y.ndim or cond.num > y.num
-        if bx:
-            x = broadcast(x, cond.shape)
-        if by:
-            y = broadcast(y, cond.shape)
-        return ternary(cond, x, y)
-    if not (x.ndim == y.ndim == cond.ndim):
-        raise ValueError("Number of dims should be the same.")
-    for a, b, c in zip(x.shape, y.shape, cond.shape):
-        if not (a == b == c):
-            raise ValueError("Shape not match %r %r %r" % (x.shape, y.shape, cond.shape))
-    dtype = x.dtype if x.dtype == y.dtype else dt.dtype_infer(x.dtype, y.dtype, x.is_scalar, y.is_scalar)
-    return Var(x.shape, dtype, TernaryOp(cond, x, y))
-
-
-def reduce(x, op, dims=(), keepdims=False):
-    """ops/reduce_op.cc:257-337."""
-    x = _as_var(x)
-    if op not in _lib.BINARY_OPS:
-        raise ValueError("unknown reduce op %r" % (op,))
-    if op not in dt.REDUCE_OPS:
-        raise ValueError("reduce op %r is not associative; not supported on the device" % (op,))
-    if isinstance(dims, numbers.Integral):
-        dims = (dims,)
-    dims = list(dims)
-    xdim = x.ndim
-    if not dims:
-        rmask = (1 << xdim) - 1
-    else:
-        rmask = 0
-        for d in dims:
-            if d < 0:
-                d += xdim
-            if not (0 <= d < xdim):
-                raise ValueError("Wrong dims number: %r" % (dims,))
-            rmask |= 1 << d
-    kmask = (1 << 30) - 1 if keepdims else 0
-    return _reduce_mask(x, op, rmask, kmask)
-
-
-def _reduce_mask(x, op, rmask, kmask):
-    if not dt.amp_reg & dt.AMP_REDUCE16_DIRECT and x.dtype in ("float16", "bfloat16") and op in ("mean", "add"):
-        # improve 16-bit float precision: cast -> reduce -> cast (reduce_op.cc:259-266, 295-302)
-        return unary(_reduce_mask(unary(x, "float32"), op, rmask, kmask), x.dtype)
-    ys = []
-    for i in range(x.ndim):
-        if rmask >> i & 1:
-            if kmask >> i & 1:
-                ys.append(1)
-        else:
-            ys.append(x.shape[i])
-    if not ys:
-        ys = [1]
-        kmask |= 1
-    dtype = dt.reduce_dtype_infer(op, x.dtype)
-    y = Var(ys, dtype, ReduceOp(x, op, rmask, kmask))
-    if len(ys) == 1 and y.num == 1:
-        y.is_scalar = True
-    return y
 
 
 def reindex(x, shape, indexes=None, overflow_value=0, overflow_conditions=(), extras=()):
@@ -998,19 +768,3 @@ def reindex_reduce(y, op, shape, indexes, overflow_conditions=(), extras=()):
             raise ValueError("Shape should greater than 0.")
     extras = [_as_var(e) for e in extras]
     return Var(shape, y.dtype, ReindexReduceOp(y, op, indexes, [str(s) for s in overflow_conditions], extras))
-
-
-def make_number(value, like):
-    """ops/op_utils.cc:19-36: a [1] array of like's dtype broadcast to like."""
-    if like.shape == [1]:                        # nothing to spread: the caller's own Var
-        return array(value, like.dtype)
-    tv = type(value)
-    if tv is not float and tv is not int:
-        return broadcast(array(value, like.dtype), like.shape)
-    key = (tv, value, math.copysign(1.0, value), like.dtype)
-    v = _scalar_vars.get(key)
-    if v is None:
-        if len(_scalar_vars) >= 4096:
-            _scalar_vars.clear()
-        v = _scalar_vars[key] = array(value, like.dtype)
-    return broadcast(v, like.shape)

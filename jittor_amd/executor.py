@@ -13,6 +13,7 @@ import math
 import sys
 import threading
 
+from . import _graph
 from . import _lib
 from . import core
 from . import rowfuse
@@ -221,28 +222,7 @@ def _match_conv_bwd(op):
     return None
 
 
-def _pending_ops(targets):
-    """Pending producers behind `targets`, in topological order."""
-    order, seen = [], set()
-    stack = [v._op for v in targets if v._buf is None and v._op is not None]
-    while stack:
-        op = stack.pop()
-        if op is None:                                          # the op below it: everything it reads has been visited
-            op = stack.pop()
-            if op.id not in seen:
-                seen.add(op.id)
-                order.append(op)
-            continue
-        if op.id in seen:
-            continue
-        stack.append(op)
-        stack.append(None)
-        for u in op.inputs:
-            if u._buf is None:
-                p = u._op
-                if p is not None and p.id not in seen:
-                    stack.append(p)
-    return order
+_pending_ops = _graph.pending_ops            # of a list of targets, in topological order
 
 
 def _affine(expr, xshape, yshape):
@@ -521,39 +501,6 @@ def _libh():
     return _cap if _cap is not None else _lib.ensure_init()
 
 
-def _signature(ops, target_ids):
-    """Hashable description of everything the execution of `ops` depends on besides the data, or None."""
-    pos, leaf, parts = {}, {}, []
-    for i, op in enumerate(ops):
-        sig = op.sig()
-        out = op.out
-        if sig is None or out is None:
-            return None
-        ins = []
-        for u in op.inputs:
-            uid = u.id
-            k = pos.get(uid)
-            if k is not None:
-                ins.append(k)
-                continue
-            l = leaf.get(uid)
-            if l is None:
-                l = leaf[uid] = len(leaf)
-                ins.append((l, tuple(u.shape), u.dtype, u._op is None, u._buf is None, u._host is not None, u._stop_fuse))
-            else:
-                ins.append(-1 - l)
-        uid = out.id
-        pos[uid] = i
-        parts.append((sig, tuple(out.shape), out.dtype, uid in target_ids, out._buf is None, out._stop_fuse, tuple(ins)))
-    # (the flags are entered once and keep their order)
-    return (tuple(parts), tuple(map(str, flags.values())), dt_amp())
-
-
-def dt_amp():
-    from . import dtypes
-    return dtypes.amp_reg
-
-
 def _capture(ops, target_ids, sig):
     """Executes `ops` and records the execution as a plan under `sig` (or marks the signature as not replayable)."""
     global _cap
@@ -766,7 +713,7 @@ def run_sync(targets, device_sync=False):
         ops = _pending_ops(targets)
         if ops:
             target_ids = {t.id for t in targets}
-            sig = _signature(ops, target_ids) if flags["enable_replay"] and _cap is None and _profiler.active() is None else None
+            sig = _graph.signature(ops, targets, flags) if flags["enable_replay"] and _cap is None and _profiler.active() is None else None
             plan = _plans.get(sig) if sig is not None else False
             if plan is None:
                 _capture(ops, target_ids, sig)

@@ -1321,3 +1321,70 @@ def test_fused_rows_descriptor_is_checked(compile_only):
     assert call((100, 512), 1, reduce_op="multiply") == L.ERR_UNSUPPORTED and call((100, 512), 1, dtype=L.DTYPE_CODE["int32"]) == L.ERR_UNSUPPORTED
     assert call((100, 512), 0) == L.ERR_INVALID and call((100, 512), 2) == L.ERR_INVALID
     assert call((100, 512), 1, in_space=0) == L.ERR_INVALID and call((100, 512), 1, second_in=9) == L.ERR_INVALID
+
+
+def test_native_constructors_take_what_they_took():
+    """unary, binary, ternary, broadcast and reduce (csrc/py/graph.cpp): keyword arguments, numbers and arrays as operands, numpy integers and
+    negative axes, what is refused and how; a Var's readers, ids and history are kept as the classes' own constructors keep them."""
+    import gc
+    from jittor_amd import core
+    x = jt.array(np.ones((2, 3), np.float32))
+    assert jt.binary(x=x, y=2, op="add").shape == [2, 3] and jt.unary(op="sqrt", x=4.0).dtype == "float32" and jt.ternary(cond=x > 0, x=x, y=1.0).shape == [2, 3]
+    assert jt.reduce(x, "add", dims=np.int64(-1)).shape == [2] and jt.reduce(x, op="mean", dims=(0, 1), keepdims=True).shape == [1, 1] and x.sum([]).shape == [1]
+    assert jt.broadcast(x, (np.int32(4), 2, 3), [0]).shape == [4, 2, 3] and jt.broadcast(x, [2, 3]) is x and jt.broadcast(jt.array([1.0]), shape=x).shape == [2, 3]
+    assert jt.binary(np.arange(3), x, "multiply").shape == [2, 3] and (x + True).shape == [2, 3] and jt.unary(x, "float32") is x and jt.unary(x, "float64").dtype == "float64"
+    for call, error, text in ((lambda: jt.binary(x, 1, "nope"), ValueError, "unknown binary op 'nope'"), (lambda: jt.unary(x, "nope"), ValueError, "unknown unary op 'nope'"),
+                              (lambda: jt.binary(x, jt.array(np.ones((2, 4), np.float32)), "add"), ValueError, r"Shape not match, x:\[2, 3\] y:\[2, 4\]"),
+                              (lambda: jt.reduce(x, "add", 2), ValueError, "Wrong dims number"), (lambda: jt.reduce(x, "less"), ValueError, "not associative|unknown"),
+                              (lambda: jt.broadcast(x, [4, 2, 3], [5]), ValueError, "Wrong dims number"), (lambda: jt.broadcast(x, [-1, 2, 3]), ValueError, "greater than 0|not match"),
+                              (lambda: jt.binary(x, object(), "add"), TypeError, "cannot convert"), (lambda: jt.binary(x, 1), TypeError, "missing"),
+                              (lambda: jt.binary(x, 1, "add", 3), TypeError, "at most"), (lambda: jt.binary(x, 1, op="add", z=2), TypeError, "unexpected"),
+                              (lambda: jt.broadcast(x, [1] * 12), ValueError, "dims are supported|not match")):
+        with pytest.raises(error, match=text):
+            call()
+    y = x * x
+    assert [r() for r in x._consumers][-2:] == [y._op, y._op] and y._history == (y._op, (x, x)) and y._op.out is y and y._op.id < y.id and y._op.amp == 0
+    with jt.no_grad():
+        assert (x * 2.0)._history is None
+    for _ in range(600):
+        x + 1.0                                                # dead readers of a long-lived var are dropped now and then
+    assert len(x._consumers) < 300
+    gc.collect()
+    ref = core._ref(y._op)
+    del y
+    assert ref() is None                                       # no cycle keeps a graph alive
+    with jt.flag_scope(compile_options={"k": 3}):
+        assert (x + 1.0).compile_options == {"k": 3}
+
+
+def test_graph_keys_tell_graphs_apart():
+    """What a key depends on: ops, attributes, shapes, types, wiring, which results are asked for, what is computed already, flags, the
+    register; the same graph built again has the same key."""
+    from jittor_amd import _graph, executor
+
+    def key(build, targets=-1):
+        vs = build()
+        ts = [vs[targets]] if isinstance(targets, int) else [vs[i] for i in targets]
+        return _graph.signature(_graph.pending_ops(ts), ts, executor.flags), vs
+
+    def base(shape=(4, 6), dt="float32", op="add", k=2.0, dims=(1,), swap=False, twice=False, idx="i0"):
+        a, b = jt.array(np.ones(shape, np.float32)).cast(dt) if dt != "float32" else jt.array(np.ones(shape, np.float32)), jt.array(np.ones(shape, np.float32))
+        c = jt.binary(*((b, a) if swap else (a, a if twice else b)), op)
+        d = c * k
+        return [a, b, c, d, d.sum(list(dims), keepdims=True), d.reindex([shape[0]], [idx, "0"])]
+
+    seen = {}
+    for name, kw, targets in (("base", {}, 4), ("shape", {"shape": (4, 7)}, 4), ("dtype", {"dt": "float64"}, 4), ("op", {"op": "subtract"}, 4), ("dims", {"dims": (0,)}, 4),
+                              ("twice", {"twice": True}, 4), ("targets", {}, (3, 4)), ("reindex", {}, 5), ("index", {"idx": "3-i0"}, 5), ("other", {}, 3)):
+        k, _ = key(lambda: base(**kw), targets)
+        assert k is not None and k not in seen.values(), name
+        seen[name] = k
+        assert key(lambda: base(**kw), targets)[0] == k
+    assert key(lambda: base(k=3.0), 4)[0] == seen["base"]       # a number's value is data
+    k0, vs = key(lambda: base(), 4)
+    with jt.flag_scope(enable_reduce_fusion=False):
+        assert _graph.signature(_graph.pending_ops([vs[4]]), [vs[4]], executor.flags) != k0
+    with jt.flag_scope(amp_reg=32):
+        assert _graph.signature(_graph.pending_ops([vs[4]]), [vs[4]], executor.flags) != k0
+    vs[2].stop_fuse()
+    assert _graph.signature(_graph.pending_ops([vs[4]]), [vs[4]], executor.flags) != k0
