@@ -734,6 +734,91 @@ static void conv_wgrad_direct(const mjt_tensor* x, const mjt_tensor* dy, const m
     set_last_kernel(k->name.c_str());
 }
 
+// Weight gradient from windows in LDS (kernels/conv_wgrad_window.h): 16-bit operands, 2 to 9 taps, horizontal strides 1 and 2.
+// False: not covered, or estimated to take longer than `other` us.
+static bool conv_wgrad_window(const mjt_tensor* x, const mjt_tensor* dy, const mjt_tensor* dw, const mjt_conv_params* p, double other) {
+    const int64_t N = x->shape[0], C = x->shape[1], H = x->shape[2], W = x->shape[3];
+    const int64_t K = dy->shape[1], OH = dy->shape[2], OW = dy->shape[3], R = dw->shape[2], S = dw->shape[3];
+    const int64_t SH = p->stride_h, SW = p->stride_w, PW = p->pad_w, DH = p->dil_h, DW = p->dil_w, taps = R * S, npw = (OW + 7) / 8;
+    const bool half = x->dtype == MJT_FLOAT16;
+    if (!(half || x->dtype == MJT_BFLOAT16) || dy->dtype != x->dtype || !(dw->dtype == MJT_FLOAT32 || dw->dtype == x->dtype) || getenv("MJT_NO_FASTPATH") || getenv("MJT_CONV_NO_IGEMM")) return false;
+    if (taps < 2 || taps > 9 || SW > 2 || PW > 8 || (S - 1) * DW > 8 || !(npw == 1 || npw == 2 || npw % 4 == 0) || H > 1024 || W > 256 || numel(x) * 2 >= (int64_t(1) << 31) ||
+        numel(dy) * 2 >= (int64_t(1) << 31) || (uintptr_t)x->ptr % 16 || (uintptr_t)dy->ptr % 16)
+        return false;
+    // The kernel's layout for `rb` output rows and `ib` images a stage: its bytes of LDS, and the dwords a thread holds on their way there.
+    auto floor_div = [](int64_t a, int64_t b) { return a >= 0 ? a / b : -((b - 1 - a) / b); };
+    int64_t lo = 0, hi = 3;
+    for (int64_t s = 0; s < S; s++) {
+        const int64_t shift = floor_div(s * DW - PW, SW);
+        lo = std::min(lo, floor_div(shift, 2));
+        hi = std::max(hi, floor_div(shift, 2) + 3 + (shift & 1));
+    }
+    const int64_t lp = std::max<int64_t>(8, (-2 * lo + 7) / 8 * 8), rw = (lp + std::max((W + SW - 1) / SW, npw * 8 - 8 + 2 * hi + 2 - lp) + 7) / 8 * 8, xrow = SW * rw * 2;
+    auto unit = [](int64_t n) { return n % 8 == 0 ? 8 : n % 4 == 0 ? 4 : n % 2 == 0 ? 2 : 1; };
+    auto lds_bytes = [&](int64_t rb, int64_t ib) {
+        const int64_t xr = (rb - 1) * SH + (R - 1) * DH + 1, steps = (rb * npw + 3) / 4;
+        const int64_t xcb = ((xr * xrow + lp * 2) / 16 | 1) * 16, dcb = (steps * 4 | 1) * 16;
+        const bool checked = OH % rb != 0 || rb * npw % 4 != 0 || ib > 1;
+        return std::max(2 * ib * 64 * (xcb + dcb) + (checked ? lp * 2 + xrow + hi * 4 + 16 : 0), 64 * (64 * taps + 8) * 4);
+    };
+    auto dwords = [&](int64_t rb, int64_t ib) {
+        const bool whole = rb == OH;
+        const int64_t xr = (rb - 1) * SH + (R - 1) * DH + 1, gx = unit(whole ? H * W : W), gd = unit(whole ? OH * OW : OW);
+        const int64_t nx = ((whole ? H : xr) * W / gx + 7) / 8, nd = (rb * OW / gd + 7) / 8;
+        return ib * (nx * std::max<int64_t>(1, gx / 2) + nd * std::max<int64_t>(1, gd / 2));
+    };
+    const int64_t blocks = ((K + 63) / 64) * ((C + 63) / 64), cus = ctx().dry_run || ctx().prop.multiProcessorCount <= 0 ? 256 : ctx().prop.multiProcessorCount;
+    // Rows, images and slices by what they are estimated to take: 0.8 us and 0.04 for each row of 32 x 32 products of a wave a stage, 11.5 for
+    // the launches, the first loads and the meeting of the groups, the slices' results written (3 TB/s: all compute units at once) and read by
+    // the fold, 4 more for a fold in two launches.  us, estimated / measured: 64 x 256 x 14 x 14 -> 256 41.8 / 39.4, 64 x 512 x 7 x 7 -> 512 46.4 / 42.9,
+    // 64 x 256 x 28 x 28 stride 2 -> 256 52.8 / 50.9, 4 x 256 x 16 x 16 -> 256 20.2 / 18.5.  (Twenty-eight dwords on their way are what a thread
+    // has registers for beside nine accumulators.)
+    int64_t RB = 0, IB = 1, slices = 1;
+    double least = 1e30;
+    for (int64_t rb = 1; rb <= OH; rb++)
+        for (int64_t ib = 1; ib <= (rb == OH ? 4 : 1); ib++) {
+            if (lds_bytes(rb, ib) > 160 * 1024 || dwords(rb, ib) > 28) continue;
+            const int64_t stages = rb == OH ? (N + ib - 1) / ib : N * ((OH + rb - 1) / rb);
+            const double stage = 0.8 + 0.04 * (double)(ib * ((rb * npw + 3) / 4) * taps);
+            const int64_t most = std::min(stages, std::max<int64_t>(1, cus / blocks));
+            for (int64_t n = 1; n <= most; n++) {
+                const int64_t per = (stages + n - 1) / n, nn = (stages + per - 1) / per;
+                const double t = 11.5 + std::ceil((double)(nn * blocks) / cus) * (double)per * stage + (double)nn * numel(dw) * 4 * (C * taps % 4 ? 0.7e-6 : 0.45e-6) + (nn > 16 ? 4.0 : 0.0);
+                if (t < least) { least = t; RB = rb; IB = ib; slices = nn; }
+            }
+        }
+    if (RB == 0 || least >= other) return false;
+    const int64_t stages = RB == OH ? (N + IB - 1) / IB : N * ((OH + RB - 1) / RB), per = (stages + slices - 1) / slices;
+    slices = (stages + per - 1) / per;
+    if (slices * numel(dw) * 4 > (int64_t(1) << 30) || slices * blocks > (1 << 28)) return false;
+    const bool in_place = slices == 1 && dw->dtype == MJT_FLOAT32 && (uintptr_t)dw->ptr % 16 == 0;
+    const size_t part_bytes = (size_t)slices * (size_t)numel(dw) * 4;
+    if (!in_place && !(workspace_allowed(part_bytes) && (ctx().dry_run || grow_kept(&g_wgrad_part, &g_wgrad_bytes, part_bytes)))) return false;
+    std::ostringstream key;
+    key << "wgwin|" << C << "|" << H << "|" << W << "|" << K << "|" << R << "|" << S << "|" << OH << "|" << OW << "|" << SH << "|" << SW << "|" << p->pad_h << "|" << PW
+        << "|" << DH << "|" << DW << "|" << half << "|" << RB << "|" << IB;
+    JitKernel* k = cached(key.str());
+    if (!k) {
+        std::ostringstream name;
+        name << "mjt_conv_wgrad_mfma_" << (half ? "f16" : "bf16") << "_window_c" << C << "_k" << K << "_" << H << "x" << W << "_r" << R << "x" << S << "_s" << SH << "x" << SW << "_p"
+             << p->pad_h << "x" << PW << "_d" << DH << "x" << DW << "_rows" << RB << "_images" << IB;
+        std::ostringstream src;
+        src << "#define ENTRY " << name.str() << "\n#define IN_F16 " << half << "\n#define RB " << RB << "\n#define IB " << IB
+            << "\n#define C_ " << C << "\n#define H_ " << H << "\n#define W_ " << W << "\n#define K_ " << K << "\n#define R_ " << R << "\n#define S_ " << S << "\n#define OH_ " << OH
+            << "\n#define OW_ " << OW << "\n#define SH " << SH << "\n#define SW " << SW << "\n#define PH " << p->pad_h << "\n#define PW " << PW << "\n#define DH " << DH << "\n#define DW " << DW << "\n";
+        src << embedded_source("conv_wgrad_window.h") << "\n";
+        k = jit_get(src.str(), name.str());
+        remember(key.str(), k);
+    }
+    if (k->spilled != 0) return false;
+    void* part = in_place ? dw->ptr : wgrad_partials(part_bytes);
+    std::vector<uint64_t> a{bits_of_ptr(x->ptr), bits_of_ptr(dy->ptr), bits_of_ptr(part), (uint64_t)N, (uint64_t)stages, (uint64_t)per, (uint64_t)(numel(x) * 2), (uint64_t)(numel(dy) * 2)};
+    jit_launch(k, (unsigned)((slices * blocks + 7) / 8 * 8), 1, 512, 0, a);
+    if (!in_place) fold_wgrad_slices(part, slices, dw);
+    set_last_kernel(k->name.c_str());
+    return true;
+}
+
 // Weight gradient as an implicit product (kernels/gemm_mfma.h with CONV 2): both operands are gathered on their way to LDS and
 // the sum over images and pixels is cut into slices.  False: not covered.
 static bool conv_wgrad_product(const mjt_tensor* x, const mjt_tensor* dy, const mjt_tensor* dw, const mjt_conv_params* p) {
@@ -792,6 +877,9 @@ static bool conv_wgrad_product(const mjt_tensor* x, const mjt_tensor* dy, const 
                 if (t < least) { least = t; MI = mi; slices = nn; }
             }
     }
+    // us at 16 bits, this / the windows: 64 x 256 x 14 x 14 3x3 -> 256 59.9 / 39.4; 64 x 512 x 7 x 7 -> 512 91.8 / 42.9; 64 x 256 x 28 x 28 stride 2 ->
+    // 256 63.9 / 50.9; 16 x 512 x 14 x 14 -> 512 64.2 / 38.9; 4 x 128 x 12 x 12 -> 256 11.9 / 15.6, 64 x 64 x 14 x 14 -> 64 18.2 / 25.0 stay.
+    if (half && R * S > 1 && conv_wgrad_window(x, dy, dw, p, least)) return true;
     const int NI = MI;
     const bool split = !half && MI == 2;
     const int64_t tiles = tiles_of(64 * MI);
@@ -873,6 +961,11 @@ void conv_wgrad_impl(const mjt_tensor* x, const mjt_tensor* dy, const mjt_tensor
     const bool planes = R * S == 1 && p->stride_h == 1 && p->stride_w == 1 && p->pad_h == 0 && p->pad_w == 0;
     const bool large = (double)N * OH * OW * K * C * R * S >= (double)(1 << 27);
     if ((!ok || (OH * OW % 2 == 0 && (planes || narrow) && large)) && G == 1 && N >= 1 && conv_wgrad_product(x, dy, dw, p)) return;
+    // What is left for the MFMA kernel, on maps whose rows the windows take (us, kernel / windows: 64 x 128 x 28 x 28 3x3 -> 128 55.0 / 41.7;
+    // 64 x 512 x 8 x 8 -> 512 93.9 / 37.0; 64 x 64 x 28 x 28 -> 64 39.1 / 30.3; 1 x 128 x 8 x 8 -> 64 15.0 / 13.2; a few images of few
+    // channels stay: 1 x 64 x 14 x 14 -> 64 12.0 / 13.3, 1 x 64 x 28 x 28 -> 64 13.0 / 13.7).
+    // (MJT_WGRAD_IPS, MJT_WGRAD_RPS: that kernel's slices, for experiments)
+    if (ok && R * S > 1 && !getenv("MJT_WGRAD_IPS") && !getenv("MJT_WGRAD_RPS") && (K * C >= 8192 || (double)N * OH * OW * K * C * R * S >= (double)(1 << 25)) && conv_wgrad_window(x, dy, dw, p, 1e30)) return;
     if (!ok && any_shape) {
         conv_wgrad_direct(x, dy, dw, p, G);
         return;

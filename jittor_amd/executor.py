@@ -1212,7 +1212,9 @@ def _run_single(op):
         # 10 to 18 (8 x 32 x 14 x 14 3x3 -> 64 17.8 / 11.0, 8 x 128 x 7 x 7 3x3 13.7 / 16.3).
         half = x.dtype in ("bfloat16", "float16")
         narrow = OW % 8 != 0 and OW < 0.6 * 32 * -(-OW // 32)
-        chunked = half and narrow and (OH * OW % 2 == 1 and N % 8 == 0 or N * OH * OW * K * C * R * S < 1 << 27)
+        # Rows of at most 8 pixels with 2 to 9 taps stay with the library: 64 x 512 x 7 x 7 3x3 43 from windows in LDS.
+        windows = OW <= 8 and 2 <= R * S <= 9 and sw <= 2
+        chunked = half and narrow and (OH * OW % 2 == 1 and N % 8 == 0 and not windows or N * OH * OW * K * C * R * S < 1 << 27)
         if (half or x.dtype == "float32") and not chunked and flags["enable_conv_wgrad_kernel"]:
             # the MFMA kernel (16 bits) or the product that gathers its operands; shapes they do not cover come back as
             # unsupported and take the paths below
