@@ -1036,8 +1036,86 @@ extern "C" int mjt_conv2d_meta_wgrad_grouped(const mjt_tensor* x, const mjt_tens
 }
 
 namespace mjt {
+// All stride phases of an input gradient in one launch behind the weights' packing (kernels/conv_dgrad_phases.h): 16-bit operands, strides 1 and 2, any
+// padding and dilation; no shape of these that was timed is slower than before.  False: not covered.
+static bool conv_dgrad_all_phases(const mjt_tensor* dy, const mjt_tensor* w, const mjt_tensor* dx, const mjt_conv_params* p) {
+    const int64_t N = dx->shape[0], C = dx->shape[1], H = dx->shape[2], W = dx->shape[3];
+    const int64_t K = dy->shape[1], OH = dy->shape[2], OW = dy->shape[3], R = w->shape[2], S = w->shape[3], taps = R * S;
+    const int64_t SH = p->stride_h, SW = p->stride_w, PH = p->pad_h, PW = p->pad_w, DH = p->dil_h, DW = p->dil_w;
+    const bool half = dy->dtype == MJT_FLOAT16, narrow = dx->dtype == dy->dtype;
+    if (!(half || dy->dtype == MJT_BFLOAT16) || SH > 2 || SW > 2 || SH * SW == 1 || taps < 1 || taps > 25 || getenv("MJT_NO_FASTPATH") || getenv("MJT_CONV_DGRAD_NO_PHASES")) return false;
+    if (numel(dy) < 1 || numel(dy) * 2 >= (int64_t(1) << 31) || numel(dx) >= (int64_t(1) << 31) || H > 4096 || W > 4096 || (R - 1) * DH > 64 || (S - 1) * DW > 64 ||
+        (uintptr_t)dy->ptr % 4 || (uintptr_t)dx->ptr % 8)
+        return false;
+    // the kernel's layout: margins that the taps' shifts reach, and the positions between the first and the last that a tile reads
+    auto phase = [](int64_t t, int64_t stride) { return (t % stride + stride) % stride; };
+    int64_t rlo = 0, rhi = 0, clo = 0, chi = 0;
+    for (int64_t r = 0; r < R; r++) {
+        const int64_t d = (phase(r * DH - PH, SH) + PH - r * DH) / SH;
+        rlo = std::min(rlo, d);
+        rhi = std::max(rhi, d);
+    }
+    for (int64_t s = 0; s < S; s++) {
+        const int64_t d = (phase(s * DW - PW, SW) + PW - s * DW) / SW;
+        clo = std::min(clo, d);
+        chi = std::max(chi, d);
+    }
+    const int64_t unit = OW % 2 == 0 ? 2 : 1, HB = (H + SH - 1) / SH, WB = (W + SW - 1) / SW, lpc = (-clo + unit - 1) / unit * unit;
+    const int64_t PR = HB + rhi - rlo, PC = (lpc + WB + chi + unit - 1) / unit * unit, total = N * HB * WB, CT = (C + 63) / 64;
+    if (N * PR * PC >= (int64_t(1) << 30)) return false;
+    auto pos = [&](int64_t f) { return (f / (HB * WB) * PR + f % (HB * WB) / WB - rlo) * PC + f % WB + lpc; };
+    auto span_of = [&](int64_t tile) {
+        int64_t most = 0;
+        for (int64_t t = 0; t < (total + tile - 1) / tile && t < HB * WB; t++)       // (tiles begin at the same places of an image again after that)
+            most = std::max(most, pos(t * tile + tile - 1) + rhi * PC + chi + 1 - (pos(t * tile) + rlo * PC + clo) / unit * unit);
+        return (most + unit - 1) / unit * unit;
+    };
+    const int64_t cus = ctx().dry_run || ctx().prop.multiProcessorCount <= 0 ? 256 : ctx().prop.multiProcessorCount;
+    const int64_t PT = (total + 127) / 128 * CT >= cus ? 2 : 1, span = span_of(64 * PT), tiles = (total + 64 * PT - 1) / (64 * PT) * CT;
+    // A stage of 6 to 9 taps is 16 channels of dy, of fewer taps more, so that its MFMAs take longer than its barrier.  Where every workgroup has
+    // a compute unit to itself nothing hides a stage's latency: twice as many (us, 16 / 32 channels: 1 x 512 x 7 x 7 -> 512 29.0 / 26.4, 8 x 256 x 28 x 28 -> 256 17.8 / 16.7).
+    auto fits = [&](int64_t ku) { return 2 * ku * (taps * 2048 + span * 32) <= 160 * 1024 && span / unit * 2 * ku <= 4 * 256; };
+    int64_t KU = taps >= 6 ? 1 : taps >= 3 ? 2 : 4;
+    if (tiles <= cus && KU * 16 < K && fits(2 * KU)) KU *= 2;
+    const int64_t stages = (K + 16 * KU - 1) / (16 * KU), packed = CT * stages * KU * taps * 2048;
+    if (!fits(KU) || packed >= (int64_t(1) << 31) || tiles >= (1 << 28)) return false;
+    std::ostringstream key;
+    key << "dgphases|" << C << "|" << H << "|" << W << "|" << K << "|" << R << "|" << S << "|" << OH << "|" << OW << "|" << SH << "|" << SW << "|" << PH << "|" << PW << "|" << DH << "|" << DW
+        << "|" << half << narrow << "|" << PT << "|" << KU << "|" << span;
+    JitKernel* k = cached(key.str());
+    if (!k) {
+        std::ostringstream name;
+        name << "mjt_conv_mfma_" << (half ? "f16" : "bf16") << "_dgrad_c" << C << "_k" << K << "_" << H << "x" << W << "_r" << R << "x" << S << "_s" << SH << "x" << SW << "_p" << PH << "x" << PW
+             << "_d" << DH << "x" << DW << "_o" << (narrow ? (half ? "f16" : "bf16") : "f32") << "_t" << 64 * PT << "_ku" << KU;
+        std::ostringstream src;
+        src << "#define ENTRY " << name.str() << "\n#define IN_F16 " << half << "\n#define Y_16 " << narrow << "\n#define KU " << KU << "\n#define PT " << PT << "\n#define SPAN " << span
+            << "\n#define C_ " << C << "\n#define H_ " << H << "\n#define W_ " << W << "\n#define K_ " << K << "\n#define R_ " << R << "\n#define S_ " << S << "\n#define OH_ " << OH
+            << "\n#define OW_ " << OW << "\n#define SH " << SH << "\n#define SW " << SW << "\n#define PH " << PH << "\n#define PW " << PW << "\n#define DH " << DH << "\n#define DW " << DW << "\n";
+        src << embedded_source("conv_dgrad_phases.h") << "\n";
+        k = jit_get(src.str(), name.str());
+        remember(key.str(), k);
+    }
+    if (k->spilled != 0) return false;
+    void* wbuf = conv_scratch(2, (size_t)packed);
+    mjt_tensor tw;
+    memset(&tw, 0, sizeof(tw));
+    tw.ptr = wbuf;
+    tw.dtype = w->dtype;
+    for (int64_t e : {CT, stages, KU, taps, int64_t(64), int64_t(16)}) tw.shape[tw.ndim++] = e;
+    const std::string ks = "i1*" + std::to_string(16 * KU) + "+i2*16+i5", cs = "i0*64+i4", rs = "i3/" + std::to_string(S), ss = "i3%" + std::to_string(S);
+    const std::string over_k = ks + ">=" + std::to_string(K), over_c = cs + ">=" + std::to_string(C);
+    const char* idx[4] = {ks.c_str(), cs.c_str(), rs.c_str(), ss.c_str()};
+    const char* over[2] = {over_k.c_str(), over_c.c_str()};
+    if (mjt_reindex(w, &tw, 4, idx, 0.0, 2, over, 0, nullptr) != MJT_OK) MJT_FAIL(MJT_ERR_DEVICE, "conv dgrad: a rearrangement failed: " << mjt_last_error());
+    std::vector<uint64_t> a{bits_of_ptr(wbuf), bits_of_ptr(dy->ptr), bits_of_ptr(dx->ptr), (uint64_t)N, (uint64_t)(numel(dy) * 2), (uint64_t)packed};
+    jit_launch(k, (unsigned)((tiles + 7) / 8 * 8), 1, 256, 0, a);
+    set_last_kernel(((H % SH == 0 && W % SW == 0 && DH == 1 && DW == 1 ? "conv_dgrad_phases:" : "") + k->name).c_str());
+    return true;
+}
+
 // Input gradient of the convolution y = conv(x, w): dx[n,c,h,w] = sum over (k, r, s) of dy[n,k,oh,ow] * w[k,c,r,s] with
 // h = oh*sh - ph + r*dh, w = ow*sw - pw + s*dw.  It is itself a convolution of dy, run on the forward kernels:
+//   * 16-bit operands at strides 1 and 2 other than 1 x 1: one launch for all phases (above);
 //   * stride 1: with the weights transposed and their taps flipped, padding d*(R-1) - p;
 //   * a stride without dilation, H and W multiples of it: one stride-1 convolution per stride phase.  The rows
 //     h = sh*i + a of dx see only the taps r = r_a + sh*u (r_a = (a + ph) % sh, u = 0 .. U_a - 1) and
@@ -1065,6 +1143,7 @@ void conv_dgrad_impl(const mjt_tensor* dy, const mjt_tensor* w, const mjt_tensor
               "conv dgrad: dy shape " << shape_str(dy) << " != [" << N << "," << K << "," << OH << "," << OW << "]");
     MJT_CHECK(dh * (R - 1) >= ph && dw * (S - 1) >= pw, "conv dgrad: padding beyond the taps' reach is not supported");
     if (N == 0 || C == 0) return;
+    if (conv_dgrad_all_phases(dy, w, dx, p)) return;
     const int64_t esz = dtype_size(w->dtype);
     auto view = [](void* ptr, int dtype, std::initializer_list<int64_t> shape) {
         mjt_tensor t;

@@ -1154,7 +1154,7 @@ def _run_single(op):
         K, C, R, S = w.shape
         G = op.groups
         if G == 1:
-            # the library's own entry: transposed, flipped weights for stride 1, one convolution per stride phase otherwise
+            # the library's own entry: transposed, flipped weights for stride 1, the stride phases (at once or one by one) otherwise
             td, tw = _tensor_of(dy), _tensor_of(w)
             tx = _tensor(_alloc_out(out), out.dtype, out.shape)
             p = _lib.ConvParams(sh, sw, ph, pw, dh, dw)
