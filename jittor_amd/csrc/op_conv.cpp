@@ -169,6 +169,64 @@ bool depthwise_run(const DepthwiseShape& g, const mjt_tensor* x, const mjt_tenso
 }
 }  // namespace
 
+// The first layer of a network, few channels and long rows of taps at horizontal stride 2, from windows in LDS (kernels/conv_stem.h).  False: not covered.
+static bool conv_stem(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, const mjt_conv_params* p) {
+    const int64_t N = x->shape[0], C = x->shape[1], H = x->shape[2], W = x->shape[3];
+    const int64_t K = w->shape[0], R = w->shape[2], S = w->shape[3], OH = y->shape[2], OW = y->shape[3], SH = p->stride_h, PH = p->pad_h, PW = p->pad_w, DH = p->dil_h;
+    const int in = x->dtype == MJT_BFLOAT16 ? 0 : x->dtype == MJT_FLOAT16 ? 1 : 2;
+    const int64_t esz = dtype_size(x->dtype), shift = PW & 1, steps = (C * R + 1) / 2, parts = in == 2 ? 3 : 1;
+    const bool narrow = y->dtype != MJT_FLOAT32;
+    if (p->stride_w != 2 || (p->dil_w != 1 && S > 1) || S + shift > 8 || steps * parts > 36 || getenv("MJT_CONV_NO_IGEMM")) return false;
+    // (a row of taps is 8 places of the sum whatever S is: half of them at least are to be taps)
+    if (2 * C * R * S < 16 * steps || numel(x) * esz >= (int64_t(1) << 31) || H > 8192 || W > 4096 || PH > 64 || PW > 64 || SH > 8 || (R - 1) * DH > 64 || (uintptr_t)x->ptr % 16) return false;
+    const int64_t cus = ctx().dry_run || ctx().prop.multiProcessorCount <= 0 ? 256 : ctx().prop.multiProcessorCount;
+    // float32 and more than 32 channels: a workgroup's way to its weights costs a few tiles more than it gives (us, gather / this: 1 x 224 x 224 -> 64 10.4 /
+    // 14.6, 4 x 96 x 96 -> 48 10.7 / 12.7, 2 x 224 x 224 -> 64 15.4 / 15.7, 3 x 224 x 224 19.9 / 19.2, 4 x 224 x 224 24.3 / 19.7; up to 32 channels 4 x 160 x 160 -> 16
+    // 14.4 / 11.5, 3 x 48 x 48 -> 17 10.2 / 9.0; bfloat16 1 x 224 x 224 -> 64 9.6 / 8.8, 4 x 128 x 128 -> 32 9.1 / 5.8).
+    if (in == 2 && K > 32 && (N * OH * OW + 63) / 64 * ((K + 63) / 64) < 2 * cus) return false;
+    const int64_t KH = K > 32 ? 2 : 1, kblocks = (K + 32 * KH - 1) / (32 * KH), waves = 4 / KH, unit = W % 4 == 0 ? 4 : W % 2 == 0 ? 2 : 1;
+    const int64_t lp = (PW + shift + 3) / 4 * 4, pitch = (std::max(lp + W, lp - PW - shift + 2 * OW + 6) + 3) / 4 * 4;
+    // Rows of a tile and tiles of a workgroup by what they are estimated to take, in cycles: a wave's 32 pixels their MFMAs and 300, a tile
+    // its values' way to LDS and 1000, a workgroup 6000 for the weights; two workgroups share a compute unit in 1.6 times the time of one.
+    int64_t TR = 0, per = 1;
+    double best = 1e300;
+    for (int64_t tr = 1; tr <= 8 && tr <= OH; tr++) {
+        const int64_t xr = (tr - 1) * SH + (R - 1) * DH + 1, units = C * xr * (W / unit), ni = (units + 255) / 256;
+        const int64_t lds = std::max(parts * C * xr * pitch * 2, 32 * KH * (C * R * S | 1) * 4);
+        if (lds > 78 * 1024 || ni * std::max<int64_t>(1, unit * esz / 4) > 40) continue;
+        const int64_t pts = (tr * OW + 31) / 32, tiles = N * ((OH + tr - 1) / tr);
+        const double tile = (double)((pts + waves - 1) / waves) * (double)(steps * (in == 2 ? 6 : 1) * 32 + 300) + 1000.0 + (double)(ni * unit) * (in == 2 ? 40.0 : 15.0);
+        for (int64_t n = 1; n <= 16 && n <= tiles; n++) {
+            const int64_t wgs = (tiles + n - 1) / n * kblocks;
+            const double t = wgs <= cus ? 6000.0 + (double)n * tile : std::ceil((double)wgs / (2 * cus)) * 1.6 * (6000.0 + (double)n * tile);
+            if (t < best) { best = t; TR = tr; per = n; }
+        }
+    }
+    if (TR == 0) return false;
+    const int64_t tiles = N * ((OH + TR - 1) / TR), grid = (tiles + per - 1) / per * kblocks;
+    if (tiles >= (1 << 28) || grid >= (1 << 28)) return false;
+    std::ostringstream key;
+    key << "stem|" << C << "|" << H << "|" << W << "|" << K << "|" << R << "|" << S << "|" << OH << "|" << OW << "|" << SH << "|" << PH << "|" << PW << "|" << DH << "|" << in << narrow << "|" << TR;
+    JitKernel* k = cached(key.str());
+    if (!k) {
+        std::ostringstream name;
+        name << "mjt_conv_igemm_" << mjt_dtype_name(x->dtype) << (y->dtype != x->dtype ? "_of32" : "") << "_stem_c" << C << "_k" << K << "_r" << R << "x" << S << "_s" << SH << "x2_p" << PH << "x" << PW << "_d"
+             << DH << "x1_rows" << TR << "_" << H << "x" << W;
+        std::ostringstream src;
+        src << "#define ENTRY " << name.str() << "\n#define IN " << in << "\n#define Y_16 " << narrow << "\n#define TR " << TR << "\n#define C_ " << C << "\n#define H_ " << H << "\n#define W_ " << W
+            << "\n#define K_ " << K << "\n#define R_ " << R << "\n#define S_ " << S << "\n#define OH_ " << OH << "\n#define OW_ " << OW << "\n#define SH " << SH << "\n#define PH " << PH
+            << "\n#define PW " << PW << "\n#define DH " << DH << "\n";
+        src << embedded_source("conv_stem.h") << "\n";
+        k = jit_get(src.str(), name.str());
+        remember(key.str(), k);
+    }
+    if (k->spilled != 0) return false;
+    std::vector<uint64_t> a{bits_of_ptr(x->ptr), bits_of_ptr(w->ptr), bits_of_ptr(y->ptr), (uint64_t)N, (uint64_t)per, (uint64_t)(numel(x) * esz)};
+    jit_launch(k, (unsigned)grid, 1, 256, 0, a);
+    set_last_kernel(k->name.c_str());
+    return true;
+}
+
 // free_extent: y's rows and columns are taken as they are instead of checked against the extents that stride, padding and
 // taps give (output (oh, ow) reads x around (oh*sh - ph, ow*sw - pw) whatever oh and ow; outside the image x is 0): what the
 // stride phases of an input gradient need, whose zero margins differ between the two ends of an axis.
@@ -434,6 +492,7 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
     const int64_t P = OH * OW, CRS = C * R * S;
     if (G == 1 && !getenv("MJT_NO_FASTPATH") && !getenv("MJT_CONV_NO_GEMM") && (double)N * K * P * CRS >= (double)(1 << 22) &&
         P < (int64_t(1) << 31) && CRS < (int64_t(1) << 31) && matmul_available()) {
+        if (!flat_forced && conv_stem(x, w, y, p)) return;
         const int64_t esz = dtype_size(x->dtype);
         const int64_t Ppad = (P * esz + 15) / 16 * 16 / esz;
         const bool plain = R == 1 && S == 1 && p->stride_h == 1 && p->stride_w == 1 && p->pad_h == 0 && p->pad_w == 0 && Ppad == P && OH == H && OW == W;
