@@ -878,6 +878,63 @@ static bool conv_wgrad_window(const mjt_tensor* x, const mjt_tensor* dy, const m
     return true;
 }
 
+// Weight gradient of the first layer of a network, float32, few channels at horizontal stride 2, from windows in LDS (kernels/conv_stem_wgrad.h).
+// False: not covered, or estimated to take longer than `other` us.
+static bool conv_wgrad_stem(const mjt_tensor* x, const mjt_tensor* dy, const mjt_tensor* dw, const mjt_conv_params* p, double other) {
+    const int64_t N = x->shape[0], C = x->shape[1], H = x->shape[2], W = x->shape[3];
+    const int64_t K = dy->shape[1], OH = dy->shape[2], OW = dy->shape[3], R = dw->shape[2], S = dw->shape[3], CRS = C * R * S, NT = (CRS + 31) / 32;
+    const int64_t SH = p->stride_h, PH = p->pad_h, PW = p->pad_w, DH = p->dil_h;
+    if (x->dtype != MJT_FLOAT32 || dw->dtype != MJT_FLOAT32 || p->stride_w != 2 || (p->dil_w != 1 && S > 1) || NT < 3 || NT > 5 || H > 8192 || W > 4096 || PH > 64 || PW > 64 || SH > 8 || (R - 1) * DH > 64 ||
+        (uintptr_t)x->ptr % 16 || (uintptr_t)dy->ptr % 16 || numel(x) * 4 >= (int64_t(1) << 31) || numel(dy) * 4 >= (int64_t(1) << 31))
+        return false;
+    const int64_t cus = ctx().dry_run || ctx().prop.multiProcessorCount <= 0 ? 256 : ctx().prop.multiProcessorCount;
+    const int64_t KH = K > 32 ? 2 : 1, kblocks = (K + 32 * KH - 1) / (32 * KH), groups = 4 / KH, unit = W % 4 == 0 ? 4 : W % 2 == 0 ? 2 : 1, steps = (OW + 15) / 16;
+    const int64_t lp = (PW + 3) / 4 * 4, halfw = std::max((lp + W + 1) / 2, steps * 16 + (S - 1 - PW + lp) / 2 + 2), dwords = (halfw + 1) / 2 | 1;
+    // Rows of a tile and tiles of a workgroup by what they are estimated to take, in us: terms as for the forward kernel, the slices' fold as for the
+    // gathering product, whose estimate `other` is.  us, gather / this: 32 x 3 x 224 x 224 7x7 -> 64 107.5 / 68.0, -> 16 103 / 41; 8 x 3 x 224 x 224 -> 64 38.0 / 31.4;
+    // 32 x 3 x 125 x 125 -> 64 53.7 / 43.1; on the other side 1 x 3 x 224 x 224 -> 64 14.8 / 19.9, 4 x 3 x 96 x 96 -> 48 13.8 / 18.3.  (Up to 64 columns, such as 3 x 3 taps
+    // of 3 channels, the waves have few MFMAs to a step: 16 x 3 x 128 x 128 3x3 -> 64 16.6 / 16.6, 64 x 3 x 32 x 32 -> 16 11.1 / 13.6.)
+    int64_t TR = 0, per = 1;
+    double best = other;
+    for (int64_t tr = 1; tr <= 8 && tr <= OH; tr++) {
+        const int64_t xr = (tr - 1) * SH + (R - 1) * DH + 1, ni = (C * xr * (W / unit) + 255) / 256;
+        if (std::max(3 * C * xr * dwords * 8, 32 * KH * NT * 128) > 78 * 1024 || ni * unit > 36) continue;
+        const int64_t tiles = N * ((OH + tr - 1) / tr);
+        const double tile = (double)((tr * steps + groups - 1) / groups) * (double)(NT * 6 * 32 + 200) + 1000.0 + (double)(ni * unit) * 40.0;
+        for (int64_t n = 1; n <= 64 && n <= tiles; n++) {
+            const int64_t nn = (tiles + n - 1) / n, wgs = nn * kblocks;
+            const double cycles = wgs <= cus ? 3000.0 + (double)n * tile : std::ceil((double)wgs / (2 * cus)) * 1.6 * (3000.0 + (double)n * tile);
+            const double t = cycles / 2200.0 + 3.0 + (nn > 1 ? (nn > 16 ? 8.0 : 5.0) + (double)nn * numel(dw) * 8 / 5e6 : 0.0);
+            if (t < best) { best = t; TR = tr; per = n; }
+        }
+    }
+    if (TR == 0) return false;
+    const int64_t tiles = N * ((OH + TR - 1) / TR), slices = (tiles + per - 1) / per;
+    if (tiles >= (1 << 28) || slices * kblocks >= (1 << 28) || slices * numel(dw) * 4 > (int64_t(1) << 30)) return false;
+    const size_t part_bytes = (size_t)slices * (size_t)numel(dw) * 4;
+    if (slices > 1 && !(workspace_allowed(part_bytes) && (ctx().dry_run || grow_kept(&g_wgrad_part, &g_wgrad_bytes, part_bytes)))) return false;
+    std::ostringstream key;
+    key << "wgstem|" << C << "|" << H << "|" << W << "|" << K << "|" << R << "|" << S << "|" << OH << "|" << OW << "|" << SH << "|" << PH << "|" << PW << "|" << DH << "|" << TR;
+    JitKernel* k = cached(key.str());
+    if (!k) {
+        std::ostringstream name;
+        name << "mjt_conv_wgrad_igemm_float32_stem_c" << C << "_k" << K << "_r" << R << "x" << S << "_s" << SH << "x2_p" << PH << "x" << PW << "_d" << DH << "x1_rows" << TR << "_" << H << "x" << W;
+        std::ostringstream src;
+        src << "#define ENTRY " << name.str() << "\n#define TR " << TR << "\n#define C_ " << C << "\n#define H_ " << H << "\n#define W_ " << W << "\n#define K_ " << K << "\n#define R_ " << R
+            << "\n#define S_ " << S << "\n#define OH_ " << OH << "\n#define OW_ " << OW << "\n#define SH " << SH << "\n#define PH " << PH << "\n#define PW " << PW << "\n#define DH " << DH << "\n";
+        src << embedded_source("conv_stem_wgrad.h") << "\n";
+        k = jit_get(src.str(), name.str());
+        remember(key.str(), k);
+    }
+    if (k->spilled != 0) return false;
+    void* part = slices == 1 ? dw->ptr : wgrad_partials(part_bytes);
+    std::vector<uint64_t> a{bits_of_ptr(x->ptr), bits_of_ptr(dy->ptr), bits_of_ptr(part), (uint64_t)N, (uint64_t)per, (uint64_t)(numel(x) * 4), (uint64_t)(numel(dy) * 4)};
+    jit_launch(k, (unsigned)(slices * kblocks), 1, 256, 0, a);
+    if (slices > 1) fold_wgrad_slices(part, slices, dw);
+    set_last_kernel(k->name.c_str());
+    return true;
+}
+
 // Weight gradient as an implicit product (kernels/gemm_mfma.h with CONV 2): both operands are gathered on their way to LDS and
 // the sum over images and pixels is cut into slices.  False: not covered.
 static bool conv_wgrad_product(const mjt_tensor* x, const mjt_tensor* dy, const mjt_tensor* dw, const mjt_conv_params* p) {
@@ -939,6 +996,7 @@ static bool conv_wgrad_product(const mjt_tensor* x, const mjt_tensor* dy, const 
     // us at 16 bits, this / the windows: 64 x 256 x 14 x 14 3x3 -> 256 59.9 / 39.4; 64 x 512 x 7 x 7 -> 512 91.8 / 42.9; 64 x 256 x 28 x 28 stride 2 ->
     // 256 63.9 / 50.9; 16 x 512 x 14 x 14 -> 512 64.2 / 38.9; 4 x 128 x 12 x 12 -> 256 11.9 / 15.6, 64 x 64 x 14 x 14 -> 64 18.2 / 25.0 stay.
     if (half && R * S > 1 && conv_wgrad_window(x, dy, dw, p, least)) return true;
+    if (!half && conv_wgrad_stem(x, dy, dw, p, least)) return true;
     const int NI = MI;
     const bool split = !half && MI == 2;
     const int64_t tiles = tiles_of(64 * MI);
