@@ -340,7 +340,8 @@ int mjt_conv2d_meta_grouped(const mjt_tensor* x, const mjt_tensor* w, const mjt_
  *   dx[n,c,h,w] = sum over (k,r,s) with h = oh*sh-ph+r*dh, w = ow*sw-pw+s*dw of dy[n,k,oh,ow] * w[k,c,r,s]
  * dy [N,K,OH,OW] and w [K,C,R,S] bfloat16, float16 or float32 (same dtype), dx
  * [N,C,H,W] float32 or their dtype; p is the forward convolution's.  Runs on
- * the forward kernels: with transposed, flipped weights for stride 1; for a
+ * the forward kernels: with transposed, flipped weights for stride 1; 16-bit
+ * operands at strides 1 and 2 in one kernel for all stride phases; for another
  * stride (no dilation, H and W multiples of it) as one stride-1 convolution
  * per stride phase on that phase's taps, so that no product has a zero
  * factor; otherwise on dy spread out with zeros.  Padding beyond the taps'
