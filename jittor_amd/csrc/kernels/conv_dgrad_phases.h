@@ -10,16 +10,17 @@
 // time more and was ten launches.  Here a workgroup takes 64 channels and 64 * PT base positions (n, i, j) with the accumulators of all
 // phases, so dy comes in once and phases that share a row leave as pairs.
 //
-// Layout.  A stage is KU * 16 channels of dy.  dy lies in LDS as [16 channels of KU][position][channel], positions being those of dy with
+// Layout.  A stage is KU * 16 channels of dy.  dy lies in LDS as [8 channels of 2 KU][position][channel], positions being those of dy with
 // the margins that the taps' shifts reach (zeros), SPAN of them from the tile's first on: a shift is a constant distance.  A thread makes 8
 // channels' pieces of one position from single values, or of two from dwords where rows are even.  Weights come packed as
-// [64 channels][stage][16 channels of KU][tap][channel of dx][channel of dy].  Both are rows of 32 bytes, which 32 lanes read as one run.
+// [64 channels][stage][16 channels of KU][tap][8 channels of dy][channel of dx][channel of dy].  Both are runs of 16 bytes that neighbouring lanes read side by
+// side (rows of 32 bytes, the halves side by side, met in the banks: 64 x 512 x 14 x 14 3x3 -> 512 43.1 us so, 40.4 now).
 // v_mfma_f32_32x32x16, weights the first operand: a lane ends up with one position and 16 channels.  Four waves, 2 halves of the channels x
 // 2 of the positions; two LDS buffers, the next stage is loaded into registers ahead of a stage's MFMAs and written behind them; two
 // workgroups on a compute unit hide one another's barriers.
-// us a call, packing included, phase by phase / this: 64 x 256 x 28 x 28 3x3 -> 256 96 / 32.7; 64 x 128 x 56 x 56 -> 128 82 / 34.4; 64 x 512 x 14 x 14 -> 512 134 /
-// 43.2; 1 x 256 x 28 x 28 -> 256 76 / 17; 32 x 64 x 32 x 32 5x5 -> 128 66 / 17.2; 64 x 256 x 28 x 28 1x1 -> 512 49 / 20.4; odd maps, with dy spread out / this: 64 x 64 x
-// 31 x 31 3x3 -> 64 47 / 11.3; closest 1 x 512 x 7 x 7 -> 512 26.9 / 26.4.  What bounds it there: the 16 stages of a workgroup, 0.9 us each of which the
+// us a call, packing included, phase by phase / this: 64 x 256 x 28 x 28 3x3 -> 256 96 / 32.0; 64 x 128 x 56 x 56 -> 128 82 / 33.4; 64 x 512 x 14 x 14 -> 512 134 /
+// 40.4; 1 x 256 x 28 x 28 -> 256 76 / 15.1; 32 x 64 x 32 x 32 5x5 -> 128 66 / 16.9; 64 x 256 x 28 x 28 1x1 -> 512 49 / 18.8; odd maps, with dy spread out / this: 64 x 64 x
+// 31 x 31 3x3 -> 64 47 / 11.1; closest 1 x 512 x 7 x 7 -> 512 26.9 / 25.2.  What bounds the first of these: the 16 stages of a workgroup, 0.9 us each of which the
 // MFMAs are half, on 392 of 512 places; the packing takes 5.
 //
 // Supplied by the host: C_, H_, W_, K_, R_, S_, OH_, OW_, SH, SW, PH, PW, DH, DW, IN_F16, Y_16 (result in the operands' type, else float32), KU, PT, SPAN.
@@ -142,7 +143,7 @@ extern "C" __global__ __launch_bounds__(256, 2) void ENTRY(Params p) {
             constexpr int i = decltype(ic)::v;
             const int it = tid + i * 256, h = it / UNITS, u = it - h * UNITS;
             if (i * 256 + 255 < ITEMS || it < ITEMS) {
-                unsigned char* const to = buf + AB + ((h >> 1) * SPAN + u * UNIT) * 32 + (h & 1) * 16;
+                unsigned char* const to = buf + AB + (h * SPAN + u * UNIT) * 16;
                 mjt_u32x4v lo, hi;
                 mjt_static_for<0, 4>([&](auto ec) {
                     constexpr int e = decltype(ec)::v;
@@ -150,7 +151,7 @@ extern "C" __global__ __launch_bounds__(256, 2) void ENTRY(Params p) {
                     hi[e] = __builtin_amdgcn_perm(dv[i][2 * e + 1], dv[i][2 * e], 0x07060302u);
                 });
                 *(mjt_u32x4v*)to = lo;
-                if constexpr (UNIT == 2) *(mjt_u32x4v*)(to + 32) = hi;
+                if constexpr (UNIT == 2) *(mjt_u32x4v*)(to + 16) = hi;
             }
         });
         mjt_static_for<0, NA>([&](auto ic) {
@@ -159,11 +160,11 @@ extern "C" __global__ __launch_bounds__(256, 2) void ENTRY(Params p) {
         });
     };
 
-    const unsigned char* const al = lds + (wc * 32 + l32) * 32 + half * 16;
+    const unsigned char* const al = lds + half * 1024 + (wc * 32 + l32) * 16;
     const unsigned char* bl[PT];
     mjt_static_for<0, PT>([&](auto tc) {
         constexpr int t = decltype(tc)::v;
-        bl[t] = lds + AB + (pos_of(f0 + (wp * PT + t) * 32 + l32) - q0) * 32 + half * 16;
+        bl[t] = lds + AB + (half * SPAN + pos_of(f0 + (wp * PT + t) * 32 + l32) - q0) * 16;
     });
     mjt_f32x16 acc[PHASES][PT];
     mjt_static_for<0, PHASES * PT>([&](auto ic) { acc[decltype(ic)::v / PT][decltype(ic)::v % PT] = (mjt_f32x16)(0.0f); });
@@ -179,7 +180,7 @@ extern "C" __global__ __launch_bounds__(256, 2) void ENTRY(Params p) {
             constexpr int s = decltype(sc)::v, ku = s / (NRS * NCS), dr = s / NCS % NRS + RLO, dc = s % NCS + CLO;
             if constexpr (shift_used(dr, dc)) {
                 mjt_u32x4v b[PT];
-                mjt_static_for<0, PT>([&](auto tc) { b[decltype(tc)::v] = *(const mjt_u32x4v*)(bl[decltype(tc)::v] + buf + (ku * SPAN + dr * PC + dc) * 32); });
+                mjt_static_for<0, PT>([&](auto tc) { b[decltype(tc)::v] = *(const mjt_u32x4v*)(bl[decltype(tc)::v] + buf + (2 * ku * SPAN + dr * PC + dc) * 16); });
                 mjt_static_for<0, TAPS>([&](auto tapc) {
                     constexpr int tap = decltype(tapc)::v, r = tap / S_, c = tap % S_;
                     if constexpr (row_shift(r) == dr && col_shift(c) == dc) {

@@ -1218,8 +1218,8 @@ static bool conv_dgrad_all_phases(const mjt_tensor* dy, const mjt_tensor* w, con
     memset(&tw, 0, sizeof(tw));
     tw.ptr = wbuf;
     tw.dtype = w->dtype;
-    for (int64_t e : {CT, stages, KU, taps, int64_t(64), int64_t(16)}) tw.shape[tw.ndim++] = e;
-    const std::string ks = "i1*" + std::to_string(16 * KU) + "+i2*16+i5", cs = "i0*64+i4", rs = "i3/" + std::to_string(S), ss = "i3%" + std::to_string(S);
+    for (int64_t e : {CT, stages, KU, taps, int64_t(2), int64_t(64), int64_t(8)}) tw.shape[tw.ndim++] = e;
+    const std::string ks = "i1*" + std::to_string(16 * KU) + "+i2*16+i4*8+i6", cs = "i0*64+i5", rs = "i3/" + std::to_string(S), ss = "i3%" + std::to_string(S);
     const std::string over_k = ks + ">=" + std::to_string(K), over_c = cs + ">=" + std::to_string(C);
     const char* idx[4] = {ks.c_str(), cs.c_str(), rs.c_str(), ss.c_str()};
     const char* over[2] = {over_k.c_str(), over_c.c_str()};
