@@ -227,6 +227,100 @@ static bool conv_stem(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor
     return true;
 }
 
+// Convolutions of 16-bit operands with horizontal stride 2 from windows in LDS (kernels/conv_strided.h), for shapes that the row kernel takes too.  False: not
+// covered, or the row kernel is the faster one: more than one tap on maps of less than 100 pixels, whose tiles hold mostly margins, or on more tiles than
+// compute units.  us, row kernel / this: 32 x 256 x 14 x 14 3x3 -> 256 20.7 / 22.3, 32 x 128 x 14 x 14 5x5 -> 128 17.9 / 21.4, 64 x 512 x 14 x 14 3x3 -> 512 45.0 / 56.4, 64 x 128 x
+// 56 x 56 3x3 -> 128 34.5 / 36.8; on this side 1 x 64 x 32 x 32 3x3 -> 128 18.0 / 9.5, 2 x 512 x 28 x 28 3x3 -> 128 72.3 / 35.6, 64 x 32 x 28 x 28 5x5 -> 128 16.6 / 12.8; single
+// taps 64 x 256 x 28 x 28 -> 512 32.1 / 18.9, 64 x 512 x 14 x 14 -> 512 24.7 / 17.6, 64 x 64 x 32 x 32 -> 128 16.2 / 14.1.
+// `packed`, `pack_mode`: as below; the packed weights are as many bytes as w.
+static bool conv_strided(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, const mjt_conv_params* p, void* packed, int pack_mode) {
+    const int64_t N = x->shape[0], C = x->shape[1], H = x->shape[2], W = x->shape[3];
+    const int64_t K = w->shape[0], R = w->shape[2], S = w->shape[3], OH = y->shape[2], OW = y->shape[3], taps = R * S;
+    const int64_t SH = p->stride_h, PH = p->pad_h, PW = p->pad_w, DH = p->dil_h, DW = p->dil_w;
+    const bool half = x->dtype == MJT_FLOAT16, narrow = y->dtype == x->dtype;
+    if (!(half || x->dtype == MJT_BFLOAT16) || p->stride_w != 2 || SH > 2 || taps < 1 || taps > 25) return false;
+    if (numel(x) < 1 || numel(x) * 2 >= (int64_t(1) << 31) || numel(y) >= (int64_t(1) << 31) || H > 4096 || W > 4096 || PH > 64 || PW > 64 || (R - 1) * DH > 64 || (S - 1) * DW > 64 || (uintptr_t)x->ptr % 4 || W % 2 || C % 32 || (taps > 1 && OH * OW < 100))
+        return false;
+    // the kernel's layout: margins that the taps' shifts reach, row phases of x that are read, and the positions between the first and the last that a tile reads
+    auto floor_of = [](int64_t a, int64_t b) { return a >= 0 ? a / b : -((b - 1 - a) / b); };
+    int64_t rlo = 0, rhi = 0, clo = 0, chi = 0;
+    bool phase[2] = {false, false};
+    for (int64_t r = 0; r < R; r++) {
+        const int64_t d = floor_of(r * DH - PH, SH);
+        phase[r * DH - PH - SH * d] = true;
+        rlo = std::min(rlo, d);
+        rhi = std::max(rhi, d);
+    }
+    for (int64_t s = 0; s < S; s++) {
+        const int64_t d = floor_of(s * DW - PW, 2);
+        clo = std::min(clo, d);
+        chi = std::max(chi, d);
+    }
+    const int64_t PR = OH + rhi - rlo, PC = OW + chi - clo, P = OH * OW, total = N * P, nrp = phase[0] && phase[1] ? 2 : 1;
+    if (N * PR * PC >= (int64_t(1) << 30)) return false;
+    auto pos = [&](int64_t f) { return (f / P * PR + f % P / OW - rlo) * PC + f % OW - clo; };
+    auto span_of = [&](int64_t tile) {
+        int64_t most = 0;
+        for (int64_t t = 0; t < (total + tile - 1) / tile && t < P; t++)       // (tiles begin at the same places of an image again after that)
+            most = std::max(most, pos(t * tile + tile - 1) + rhi * PC + chi + 1 - (pos(t * tile) + rlo * PC + clo));
+        return most;
+    };
+    const int64_t cus = ctx().dry_run || ctx().prop.multiProcessorCount <= 0 ? 256 : ctx().prop.multiProcessorCount;
+    const int64_t KU = taps >= 6 ? 1 : taps >= 3 || C % 64 ? 2 : 4, stages = C / (16 * KU);      // (C is a multiple of 32)
+    // Channels and positions of a workgroup by what a stage is estimated to take: its operands' way out of LDS and the next stage's way in, at 128
+    // bytes a cycle, and 400 cycles for its barrier and what nothing hides.
+    int64_t WK = 0, PT = 0, span = 0;
+    double best = 1e300;
+    for (int64_t wk = K % 64 ? 1 : 2; wk <= 4 && K % (32 * wk) == 0; wk *= 2)
+        for (int64_t pt = 1; pt <= 2; pt++) {
+            const int64_t sp = span_of(64 * pt), stage_bytes = KU * (taps * wk * 1024 + nrp * 2 * sp * 32);
+            if (2 * stage_bytes > 160 * 1024 || (sp * nrp * 2 * KU + 128 * wk - 1) / (128 * wk) > 6) continue;
+            const int64_t wgs = (total + 64 * pt - 1) / (64 * pt) * (K / (32 * wk));
+            const double t = std::ceil((double)wgs / cus) * ((double)(2 * wk * KU * taps * (1 + pt) * 1024 + stage_bytes) / 128 + 400.0);
+            if (t < best) { best = t; WK = wk; PT = pt; span = sp; }
+        }
+    if (WK == 0) return false;
+    const int64_t KB = K / (32 * WK), bytes = numel(w) * 2, tiles = (total + 64 * PT - 1) / (64 * PT) * KB;
+    if (bytes >= (int64_t(1) << 31) || tiles >= (1 << 28) || (taps > 1 && tiles > cus)) return false;
+    std::ostringstream key;
+    key << "strided|" << C << "|" << H << "|" << W << "|" << K << "|" << R << "|" << S << "|" << OH << "|" << OW << "|" << SH << "|" << PH << "|" << PW << "|" << DH << "|" << DW << "|" << half << narrow << "|"
+        << PT << "|" << WK << "|" << span;
+    JitKernel* k = cached(key.str());
+    if (!k) {
+        std::ostringstream name;
+        name << "mjt_conv_mfma_" << (half ? "f16" : "bf16") << "_strided_c" << C << "_k" << K << "_" << H << "x" << W << "_r" << R << "x" << S << "_s" << SH << "x2_p" << PH << "x" << PW << "_d" << DH << "x" << DW
+             << "_o" << (narrow ? (half ? "f16" : "bf16") : "f32") << "_t" << 32 * WK << "x" << 64 * PT;
+        std::ostringstream src;
+        src << "#define ENTRY " << name.str() << "\n#define IN_F16 " << half << "\n#define Y_16 " << narrow << "\n#define KU " << KU << "\n#define PT " << PT << "\n#define WK " << WK << "\n#define SPAN " << span
+            << "\n#define C_ " << C << "\n#define H_ " << H << "\n#define W_ " << W << "\n#define K_ " << K << "\n#define R_ " << R << "\n#define S_ " << S << "\n#define OH_ " << OH
+            << "\n#define OW_ " << OW << "\n#define SH " << SH << "\n#define PH " << PH << "\n#define PW " << PW << "\n#define DH " << DH << "\n#define DW " << DW << "\n";
+        src << embedded_source("conv_strided.h") << "\n";
+        k = jit_get(src.str(), name.str());
+        remember(key.str(), k);
+    }
+    if (k->spilled != 0) return false;
+    if (pack_mode) MJT_CHECK(packed && (uintptr_t)packed % 16 == 0, "conv: packed weights must be a 16-byte aligned device buffer");
+    void* wbuf = pack_mode ? packed : conv_scratch(2, (size_t)bytes);
+    if (pack_mode != 2) {
+        mjt_tensor tw;
+        memset(&tw, 0, sizeof(tw));
+        tw.ptr = wbuf;
+        tw.dtype = w->dtype;
+        for (int64_t e : {KB, stages, KU, taps, int64_t(2), 32 * WK, int64_t(8)}) tw.shape[tw.ndim++] = e;
+        const std::string ks = "i0*" + std::to_string(32 * WK) + "+i5", cs = "i1*" + std::to_string(16 * KU) + "+i2*16+i4*8+i6", rs = "i3/" + std::to_string(S), ss = "i3%" + std::to_string(S);
+        const char* idx[4] = {ks.c_str(), cs.c_str(), rs.c_str(), ss.c_str()};
+        if (mjt_reindex(w, &tw, 4, idx, 0.0, 0, nullptr, 0, nullptr) != MJT_OK) MJT_FAIL(MJT_ERR_DEVICE, "conv: packing the weights failed: " << mjt_last_error());
+    }
+    if (pack_mode == 1) {
+        set_last_kernel((k->name + "_pack").c_str());
+        return true;
+    }
+    std::vector<uint64_t> a{bits_of_ptr(wbuf), bits_of_ptr(x->ptr), bits_of_ptr(y->ptr), (uint64_t)N, (uint64_t)(numel(x) * 2), (uint64_t)bytes};
+    jit_launch(k, (unsigned)((tiles + 7) / 8 * 8), 1, (unsigned)(128 * WK), 0, a);
+    set_last_kernel(k->name.c_str());
+    return true;
+}
+
 // free_extent: y's rows and columns are taken as they are instead of checked against the extents that stride, padding and
 // taps give (output (oh, ow) reads x around (oh*sh - ph, ow*sw - pw) whatever oh and ow; outside the image x is 0): what the
 // stride phases of an input gradient need, whose zero margins differ between the two ends of an axis.
@@ -366,6 +460,7 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
                            ((p->pad_h == 0 && p->pad_w == 0 && OH == H && OW == W && (OH * OW * 2) % 16 == 0 && (uintptr_t)w->ptr % 16 == 0) ||
                             (C >= 4 * K && (K <= 64 || OH * OW <= 256)) ||
                             (K > 64 && !getenv("MJT_CONV_NO_IGEMM") && ((K + 127) / 128) * ((N * OH * OW + 63) / 64) >= 256)));
+    if (mfma_ok && G == 1 && !free_extent && !getenv("MJT_ABLATE_CONV") && !getenv("MJT_CONV_RPW") && conv_strided(x, w, y, p, packed, pack_mode)) return;
     if (mfma_ok) {
         // Rows per workgroup: a workgroup walks RPW output rows as NFULL tiles of TR rows plus one
         // shorter tile.  Pick the RPW that minimises (rounds of workgroups over the compute units) x
