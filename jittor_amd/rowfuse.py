@@ -56,8 +56,10 @@ class _Chooser:
     def __init__(self, tasks, ins, pre):
         self.tasks, self.ins, self.pre = tasks, ins, pre
 
-    def place_of(self, t, full, first):
-        """FULL (an element group or a row reduce over `full`), ROW (a group of one value per row), COLUMN (a sum over the rows), or None."""
+    def place_of(self, t, full, first, row_values):
+        """FULL (an element group or a row reduce over `full`), ROW (a group of one value per row), COLUMN (a sum over the rows), or None.
+        `row_values`: the vars that tasks ahead of this one make as one value per row.  Where there are as many rows as columns a
+        broadcast can read them per column too: that takes other rows' values, which are complete when the kernel ends."""
         members, red = t.members, t.reduce
         if not members and red is None:
             return None
@@ -91,6 +93,8 @@ class _Chooser:
                         continue
                     sp = _space(mask, shape, min(first, len(shape)))
                     if sp == OTHER or (rowwise and sp not in (FULL, SINGLE)):
+                        return None
+                    if sp != (FULL if rowwise else ROW) and any(u.id in row_values for u in reads):
                         return None
                 else:
                     for u in op.inputs:
@@ -128,14 +132,23 @@ class _Chooser:
         for k in full:
             num *= k
         writer = {v: i for i, t in enumerate(self.tasks) for v in t.writes}
-        behind, inside, place = set(), set(), {}
+        # vars that some group over the full shape reads as one value per column
+        by_column = {u.id for t in self.tasks for op in t.members if isinstance(op, BroadcastOp) and list(op.out.shape) == full
+                     and _space(op.bcast_mask & ((1 << len(full)) - 1), full, first) == COLUMN for u in self.ins(op)}
+        behind, inside, place, row_values = set(), set(), {}, set()
         for i, t in enumerate(self.tasks):
             deps = {writer[v] for v in t.reads if v in writer and writer[v] != i}
-            place[i] = None if deps & behind else self.place_of(t, full, first)
+            place[i] = None if deps & behind else self.place_of(t, full, first, row_values)
+            if place[i] == ROW and not deps & inside and by_column & t.writes:
+                place[i] = None                                # as many rows as columns: it runs ahead, for all its readers
             if place[i] is not None:
                 inside.add(i)
                 if place[i] == COLUMN:                         # complete when the kernel ends
                     behind.add(i)
+                elif place[i] == ROW:
+                    row_values |= t.writes
+                elif t.reduce is not None:
+                    row_values.add(t.reduce.out.id)
             elif deps & (inside | behind):
                 behind.add(i)
         # connected parts

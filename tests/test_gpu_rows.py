@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 import jittor_amd as jt
+import rows_graphs
 from jittor_amd import executor as E
 
 pytestmark = pytest.mark.gpu
@@ -187,3 +188,17 @@ def test_random_graphs_over_rows(gpu):
             scale = max(1.0, float(np.abs(want).max()))
             assert list(g.shape) == list(want.shape) and np.allclose(g, want, rtol=2e-4, atol=2e-5 * scale), (case, float(np.abs(g - want).max()), scale)
     assert E.stats["fused_rows"] - before >= 15
+
+
+@pytest.mark.parametrize("n", [182, 256])
+@pytest.mark.parametrize("graph", rows_graphs.GRAPHS + [None])
+def test_square_matrices(gpu, graph, n):
+    """As many rows as columns, without keepdims: values per row that are read per column.  Terms are of size 0.5 to 1.5, sums of up to n of
+    them; a handful of roundings of each, the sums' chains included."""
+    rng = np.random.default_rng(n)
+    X, e = (rng.uniform(0.5, 1.5, (n, n) if graph else (14, 16, 14, 16)).astype(np.float32), rng.uniform(0.5, 1.5, n).astype(np.float32))
+    x, v = jt.array(X), jt.array(e)
+    for _ in range(3):                                                 # executed, replayed, as recorded launches
+        outs = graph(x, X.astype(np.float64), v, e.astype(np.float64)) if graph else rows_graphs.several_axes(x, X.astype(np.float64))
+        for got, (_, want) in zip(jt.fetch_sync([q for q, _ in outs]), outs):
+            assert np.abs(got - want).max() <= 64 * EPS * max(n, np.abs(want).max())

@@ -11,6 +11,7 @@ import numpy as np
 import pytest
 
 import jittor_amd as jt
+import rows_graphs
 from jittor_amd import _lib as L
 
 G = json.load(open(os.path.join(os.path.dirname(__file__), "golden", "vectors.json")))
@@ -1321,6 +1322,77 @@ def test_fused_rows_descriptor_is_checked(compile_only):
     assert call((100, 512), 1, reduce_op="multiply") == L.ERR_UNSUPPORTED and call((100, 512), 1, dtype=L.DTYPE_CODE["int32"]) == L.ERR_UNSUPPORTED
     assert call((100, 512), 0) == L.ERR_INVALID and call((100, 512), 2) == L.ERR_INVALID
     assert call((100, 512), 1, in_space=0) == L.ERR_INVALID and call((100, 512), 1, second_in=9) == L.ERR_INVALID
+
+
+class _Rows:
+    """mjt_fused_rows worked out in numpy from its descriptor; `at` has the arrays in memory by address."""
+
+    def __init__(self):
+        self.at, self.calls = {}, 0
+
+    def __call__(self, desc, n_row_axes):
+        d = desc._obj
+        shape = [d.shape[a] for a in range(d.ndim)]
+        rows = int(np.prod(shape[:d.ndim - n_row_axes]))
+        cols = int(np.prod(shape)) // rows
+        name = {v: k for k, v in L.OP_CODE.items()}
+        val, declared = {}, {}
+        for i in range(d.n_vars):
+            v = d.vars[i]
+            declared[i] = v.reserved & 3
+            if v.role == L.VAR_SCALAR:
+                val[i] = np.float64(v.fvalue)
+            elif v.role == L.VAR_INPUT:
+                a = self.at[int(v.ptr)]
+                val[i] = np.broadcast_to(a.reshape([1 if v.bcast_mask >> q & 1 else shape[q] for q in range(d.ndim)]), shape).reshape(rows, cols)
+        for k in range(d.n_ops):
+            o = d.ops[k]
+            a = [val[o.inp[j]] for j in range(2 if o.kind == L.FOP_BINARY else 1)]
+            if o.kind == L.FOP_ROW_REDUCE:
+                r = {"add": np.sum, "mean": np.mean, "maximum": np.max}[name[o.op]](a[0], axis=1, keepdims=True)
+            elif o.kind == L.FOP_COLUMN_SUM:
+                r = a[0].sum(0, keepdims=True)
+            elif o.kind == L.FOP_BROADCAST:
+                r = a[0]
+            elif o.kind == L.FOP_UNARY:
+                r = {"sqrt": np.sqrt, "exp": np.exp}[name[o.op]](a[0])
+            else:
+                r = {"add": np.add, "subtract": np.subtract, "multiply": np.multiply, "divide": np.divide}[name[o.op]](*a)
+            if o.kind not in (L.FOP_ROW_REDUCE, L.FOP_COLUMN_SUM):
+                r = np.broadcast_to(r, [rows, 1] if declared[o.out] == 1 else [rows, cols]) if declared[o.out] == 0 or np.ndim(r) < 2 else r[:, :1]
+            val[o.out] = r
+            if d.vars[o.out].role == L.VAR_OUTPUT:
+                self.at[int(d.vars[o.out].ptr)] = r
+        self.calls += 1
+        return 0
+
+
+@pytest.mark.parametrize("graph,fused", list(zip(rows_graphs.GRAPHS, [0, 0, 0, 0, 1, 1, 1, 1])) + [(None, 1)])
+def test_rows_of_square_matrices_are_told_from_their_columns(fake_buffers, monkeypatch, graph, fused):
+    """What runs as one kernel over rows where there are as many rows as columns: a value per row that is read per column is read from
+    memory, behind the kernel that makes it.  The descriptors are worked out in numpy."""
+    rows = _Rows()
+    monkeypatch.setitem(fake_buffers.flags, "enable_replay", False)
+    rng = np.random.default_rng(3)
+    X, E = rng.uniform(0.5, 1.5, (256, 256) if graph else (16, 12, 16, 12)), rng.uniform(0.5, 1.5, 256)
+    x, e = jt.array(X.astype(np.float32)), jt.array(E.astype(np.float32))
+    jt.sync([x, e])
+    outs = graph(x, X, e, E) if graph else rows_graphs.several_axes(x, X)
+
+    def call(desc, n):
+        for v, want in [(x, X), (e, E)] + outs:                # what lies in memory when the kernel runs
+            if v._buf is not None:
+                rows.at.setdefault(v._buf.ptr, want)
+        return rows(desc, n)
+    monkeypatch.setattr(L.load(), "mjt_fused_rows", call)
+    jt.sync([v for v, _ in outs])
+    checked = 0
+    for v, want in outs:
+        got = rows.at.get(v._buf.ptr)
+        if got is not None and got is not want:
+            checked += 1
+            assert np.allclose(got.reshape(want.shape), want, rtol=1e-9)
+    assert rows.calls == fused and (checked > 0) == (fused > 0)
 
 
 def test_native_constructors_take_what_they_took():
