@@ -47,7 +47,7 @@ static void rows_impl(const mjt_fused_desc* d, int n_row_axes) {
         MJT_CHECK(d->shape[a] >= 0, "rows: negative extent");
         (a < first ? rows : cols) *= d->shape[a];
     }
-    if (rows == 0 || cols == 0 || cols > 16384 || rows >= (int64_t(1) << 31) - 65536) MJT_FAIL(MJT_ERR_UNSUPPORTED, "rows: " << rows << " x " << cols << " is not covered");
+    if (rows == 0 || cols == 0 || cols > 16384 || rows >= (int64_t(1) << 31)) MJT_FAIL(MJT_ERR_UNSUPPORTED, "rows: " << rows << " x " << cols << " is not covered");
 
     // ---- where every var lives; how many reductions lie in front of it -----------------------
     std::vector<int> space(nv, -1), level(nv, 0), maker(nv, -1);
@@ -149,13 +149,15 @@ static void rows_impl(const mjt_fused_desc* d, int n_row_axes) {
     if ((n_full + n_cols + n_sums) * nvp * vec > 160) MJT_FAIL(MJT_ERR_UNSUPPORTED, "rows: " << n_full + n_cols << " inputs of " << nvp * vec << " elements a lane");
     const int block = g > 256 ? (int)g : 256;
     const int64_t rpb = block / g, passes = (rows + rpb - 1) / rpb;
-    int64_t blocks = passes;
+    int64_t blocks = std::min(passes, int64_t(1) << 20);       // (they walk over the rest: a launch is less than 2^32 lanes)
     if (n_sums) {
         // the partial sums are written and read once more, so a workgroup takes four rows at least; and one for every compute unit at
         // least, four of 256 lanes at most (4096 x 2048 float32, rows a workgroup 16 / 8 / 4: 48 / 34 / 30.5)
         const int64_t cus = ctx().dry_run || ctx().prop.multiProcessorCount <= 0 ? 256 : ctx().prop.multiProcessorCount;
         blocks = std::min(passes, std::max(cus, std::min((1024 / block) * cus, rows / 4)));
     }
+    // a workgroup counts rows in 32 bits, up to one step past the last
+    if (rows + blocks * rpb >= int64_t(1) << 31) MJT_FAIL(MJT_ERR_UNSUPPORTED, "rows: " << rows << " rows are not covered");
     const bool streams = rows * cols * maxsize >= (int64_t(32) << 20);
 
     // ---- parameters -----------------------------------------------------------------------------

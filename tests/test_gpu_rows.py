@@ -202,3 +202,22 @@ def test_square_matrices(gpu, graph, n):
         outs = graph(x, X.astype(np.float64), v, e.astype(np.float64)) if graph else rows_graphs.several_axes(x, X.astype(np.float64))
         for got, (_, want) in zip(jt.fetch_sync([q for q, _ in outs]), outs):
             assert np.abs(got - want).max() <= 64 * EPS * max(n, np.abs(want).max())
+
+
+def test_more_rows_than_a_launch_takes_at_once(gpu):
+    """2^28 + 1024 rows: the workgroups walk on to the rows past the first 2^20 * 256.  Sums of two elements are the same part by part."""
+    rng = np.random.default_rng(4)
+    a, b = (jt.array(rng.uniform(0.5, 1.5, s).astype(np.float32)).bfloat16() for s in ((1, 1024, 2), (2 ** 18 + 1, 1, 1)))
+    x = (a * b).reshape([(2 ** 18 + 1) * 1024, 2])
+    jt.sync([x])
+    got = {}
+    for on in (True, False):
+        jt.flags["enable_row_fusion"] = on
+        try:
+            before = E.stats["fused_rows"]
+            got[on] = x - x.max([1], keepdims=True)
+            jt.sync([got[on]])
+            assert (E.stats["fused_rows"] > before) == on
+        finally:
+            jt.flags["enable_row_fusion"] = True
+    assert float((got[True] - got[False]).abs().max().data[0]) == 0.0 and float(got[True].min().data[0]) < 0.0

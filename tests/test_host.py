@@ -1324,6 +1324,25 @@ def test_fused_rows_descriptor_is_checked(compile_only):
     assert call((100, 512), 1, in_space=0) == L.ERR_INVALID and call((100, 512), 1, second_in=9) == L.ERR_INVALID
 
 
+@pytest.mark.parametrize("column_sum", [False, True])
+def test_fused_rows_counts_rows_in_32_bits(compile_only, column_sum):
+    """The kernel's row counter goes one step past the last row: 2^20 workgroups of 256 rows, or with column sums the 1024 that 256 compute units
+    are given.  Nothing is launched."""
+    L, lib = compile_only, compile_only.load()
+    f32, P = L.DTYPE_CODE["float32"], 0x1000
+
+    def call(rows):
+        fv = [L.FusedVar(L.VAR_INPUT, f32, P), L.FusedVar(L.VAR_INTERMEDIATE, f32, None, 0, 0, 0, 1), L.FusedVar(L.VAR_OUTPUT, f32, P, 0, 0, 0, 0), L.FusedVar(L.VAR_OUTPUT, f32, P, 0, 0, 0, 2)]
+        fo = [L.FusedOp(L.FOP_ROW_REDUCE, L.OP_CODE["maximum"], (0, 0, 0), 1), L.FusedOp(L.FOP_BINARY, L.OP_CODE["subtract"], (0, 1, 0), 2), L.FusedOp(L.FOP_COLUMN_SUM, L.OP_CODE["add"], (2, 0, 0), 3)]
+        n = 4 if column_sum else 3
+        d = L.FusedDesc(2, (rows, 4), n, (L.FusedVar * n)(*fv[:n]), n - 1, (L.FusedOp * (n - 1))(*fo[:n - 1]))
+        return lib.mjt_fused_rows(ctypes.byref(d), 1)
+    step = 1024 * 256 if column_sum else 2 ** 20 * 256
+    assert call(1100000000) == 0 and call(2 ** 31 - step - 1) == 0
+    for rows in (2 ** 31 - step, 2 ** 31 - 70000, 2 ** 31, 2 ** 33):
+        assert call(rows) == L.ERR_UNSUPPORTED
+
+
 class _Rows:
     """mjt_fused_rows worked out in numpy from its descriptor; `at` has the arrays in memory by address."""
 
