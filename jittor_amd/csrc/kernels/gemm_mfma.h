@@ -539,10 +539,11 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
     // NBUF 1: the host promises K <= KS, a single stage -- one staging buffer, so twice as many workgroups fit a compute unit
     __shared__ __attribute__((aligned(16))) unsigned char lds[NBUF][(TM + TN) * SPLIT_ROWB];
 #if SPLIT
-    __shared__ int in_float32;
+    // [0]: seen with the first stage, [1]: with the sums.  (Two: with a single stage no barrier keeps a wave that sets the second from
+    // one that has yet to read the first.)
+    __shared__ int in_float32[2];
     __shared__ unsigned least[2];
-    if (threadIdx.x == 0) in_float32 = 0;
-    if (threadIdx.x < 2) least[threadIdx.x] = ~0u;
+    if (threadIdx.x < 2) in_float32[threadIdx.x] = 0, least[threadIdx.x] = ~0u;
     __syncthreads();
 #endif
 
@@ -656,13 +657,13 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
     mjt_static_for<0, PIECES>([&](auto ic) { commit(ic, mjt_ic<0>(), mjt_ic<0>(), 0); });
 #if SPLIT
     if constexpr (SP)
-        if (min(least_a, least_b) < MJT_KEY(-100)) in_float32 = 1;
+        if (min(least_a, least_b) < MJT_KEY(-100)) in_float32[0] = 1;
 #endif
     if (NSET < nstages) mjt_static_for<0, PIECES>([&](auto ic) { fetch(ic, mjt_ic<0>(), mjt_ic<0>(), NSET); });
     __syncthreads();
 #if SPLIT
     if constexpr (SP)
-        if (in_float32) return false;                          // (usually seen here, where little is lost)
+        if (in_float32[0]) return false;                       // (usually seen here, where little is lost)
 #endif
 
     // fragment addresses of this lane: row lane % 32 of its wave's tile rows, chunk lane / 32
@@ -773,10 +774,10 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
             atomicMin(&least[0], wave_a);
             atomicMin(&least[1], wave_b);
         }
-        if (z != 0.0f) in_float32 = 1;
+        if (z != 0.0f) in_float32[1] = 1;
         __syncthreads();
         const unsigned all_a = least[0], all_b = least[1];
-        if (in_float32 || all_a < MJT_KEY(-100) || all_b < MJT_KEY(-100) || (all_a >> 24) + (all_b >> 24) < 2 * 127 - 100) return false;
+        if (in_float32[1] || all_a < MJT_KEY(-100) || all_b < MJT_KEY(-100) || (all_a >> 24) + (all_b >> 24) < 2 * 127 - 100) return false;
     }
 #endif
 

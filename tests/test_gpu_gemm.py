@@ -384,6 +384,27 @@ def test_gemm_float32_parts_hand_over(gpu, what):
     assert (np.abs(got[ok] - want[ok]) <= bound[ok] + K * 2.0 ** -126).all(), np.abs(got[ok] - want[ok]).max()
 
 
+@pytest.mark.parametrize("what", ["inf", "nan", "rounds to inf"])
+def test_gemm_float32_parts_of_a_single_stage(gpu, what):
+    """43 stages in slices of 6: the last slice is one stage, whose workgroups have no barrier between their first operands and their sums.
+    Sums that are not finite there, in every other tile, run on the float32 MFMAs."""
+    rng = np.random.default_rng(6)
+    M, K, N = 512, 1376, 512
+    A, B = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((N, K)).astype(np.float32)
+    A[3::256, 1350 + (what == "nan")] = {"inf": np.inf, "nan": np.nan, "rounds to inf": 3.4e38}[what]
+    if what == "rounds to inf":
+        B *= np.float32(1e-3)
+    for _ in range(3):
+        got, kern = _parts_product(L.load(), A, B, 0, 1)
+        assert "_parts_slices" in kern and "128x64" in kern, kern
+        a, b = A.astype(np.float64), B.astype(np.float64).T
+        with np.errstate(all="ignore"):
+            want, bound = a @ b, _parts_bound(a, b, K)
+        ok = np.isfinite(want)
+        assert np.array_equal(np.isfinite(got), ok) and np.array_equal(np.isnan(got), np.isnan(want))
+        assert (np.abs(got[ok] - want[ok]) <= bound[ok]).all()
+
+
 def _columns(x, R, stride, pad):
     n, c, h, w = x.shape
     xp = np.pad(x, ((0, 0), (0, 0), (pad, pad), (pad, pad)))
