@@ -1,7 +1,7 @@
 // Convolution of images with few channels, the first layer of a network, from windows that lie in LDS:
 //   y[n][k][oh][ow] = sum_{c,r,s} w[k][c][r][s] * x[n][c][oh*SH-PH+r*DH][ow*2-PW+s]
 // (python/jittor/nn.py:1251-1262, recognised by opt/tuner/conv_tuner.cc:218-411) with horizontal stride 2 and rows of up to 8 taps.  bfloat16 and
-// float16 operands as they are, float32 ones as three bfloat16 parts each (gemm_mfma.h, SPLIT, has the reasoning and the error), float32 sums.
+// float16 operands as they are, float32 ones as three bfloat16 parts each (split.h has the reasoning and the error), float32 sums.
 //
 // What it replaces, the product that gathers x (gemm_mfma.h, CONV 1), loads every element of x once for each tap that sees it, works out
 // where it lies and multiplies float32 with float32 MFMAs.  Here a row of taps is 8 consecutive values of a row of x, taps beyond S zero, so
@@ -13,17 +13,14 @@
 // 102 / 37; 32 x 3 x 190 x 190 -> 51 float32 80.9 / 50.2; 32 x 3 x 125 x 125 -> 64 bfloat16 24.2 / 16.5.  What bounds it: float32 the MFMAs, 54 GFLOP of parts and padding (43 at
 // the rate of a large bfloat16 product); bfloat16 the stores, 51 MB.
 //
-// float32: sums whose operands leave the range of the parts (smallest magnitudes, zeros apart, below 2^-100, alone or multiplied) or that are
-// not finite are thrown away, and the wave's 32 x 32 results come from float32 MFMAs over memory.
+// float32: sums that are not finite are thrown away, and the wave's 32 x 32 results come from float32 MFMAs over memory.
 //
 // Supplied by the host: IN (0 bfloat16, 1 float16, 2 float32), Y_16 (result in the operands' 16-bit type, else float32), C_, H_, W_, K_, R_, S_, OH_, OW_,
 // SH, PH, PW, DH, TR (output rows of a tile).
 
 typedef float mjt_f32x16 __attribute__((ext_vector_type(16)));
-typedef float mjt_f32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned mjt_u32x4v __attribute__((ext_vector_type(4)));
 typedef unsigned mjt_u32x2v __attribute__((ext_vector_type(2)));
-typedef __bf16 mjt_b16x2 __attribute__((ext_vector_type(2)));
 #if IN == 1
 typedef _Float16 mjt_h8 __attribute__((ext_vector_type(8)));
 #define MJT_MFMA(a, b, c) __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(mjt_h8, a), __builtin_bit_cast(mjt_h8, b), c, 0, 0, 0)
@@ -32,7 +29,6 @@ typedef __bf16 mjt_h8 __attribute__((ext_vector_type(8)));
 #define MJT_MFMA(a, b, c) __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(mjt_h8, a), __builtin_bit_cast(mjt_h8, b), c, 0, 0, 0)
 #endif
 #define MJT_NONE 0x80000000u         // an offset beyond every buffer (they are smaller than 2 GB): the load delivers zeros
-#define MJT_KEY(e) ((unsigned)(127 + (e)) << 24)
 
 template <int V> struct mjt_ic { static constexpr int v = V; };
 template <int I, int N, class F> __device__ __forceinline__ void mjt_static_for(F&& f) {
@@ -62,27 +58,12 @@ constexpr int row_at(int row) { return (row / R_ * XR + row % R_ * DH) * PITCH *
 constexpr unsigned mask_of(int d) {                                    // values of dword d of a window that are taps
     return (2 * d >= SHIFT && 2 * d < SHIFT + S_ ? 0xffffu : 0u) | (2 * d + 1 >= SHIFT && 2 * d + 1 < SHIFT + S_ ? 0xffff0000u : 0u);
 }
-__device__ __forceinline__ unsigned mjt_bf16_pair(float x, float y) {  // both rounded to nearest even
-    return __builtin_bit_cast(unsigned, __builtin_convertvector((mjt_f32x2){x, y}, mjt_b16x2));
-}
-__device__ __forceinline__ float mjt_low(unsigned p) { return __uint_as_float(p << 16); }
-__device__ __forceinline__ float mjt_high(unsigned p) { return __uint_as_float(p & 0xffff0000u); }
-// two values as three parts, each the rest of the ones before it; `least`: the smallest 2 |value| - 1 of the bits (zeros wrap round)
-__device__ __forceinline__ void mjt_split(unsigned a, unsigned b, unsigned* to, unsigned& least) {
-    const float x = __uint_as_float(a), y = __uint_as_float(b);
-    to[0] = mjt_bf16_pair(x, y);
-    const float x1 = x - mjt_low(to[0]), y1 = y - mjt_high(to[0]);
-    to[1] = mjt_bf16_pair(x1, y1);
-    to[2] = mjt_bf16_pair(x1 - mjt_low(to[1]), y1 - mjt_high(to[1]));
-    least = min(least, min((a << 1) - 1u, (b << 1) - 1u));
-}
 
 extern "C" __global__ __launch_bounds__(256, 2) void ENTRY(Params p) {
     const int N = (int)(long long)p.a[3], per = (int)(long long)p.a[4], tiles = N * TPI;
     const int kb = blockIdx.x % KBLOCKS, first = blockIdx.x / KBLOCKS * per, last = first + per < tiles ? first + per : tiles;
     if (first >= tiles) return;
     __shared__ __attribute__((aligned(16))) unsigned char lds[LDSB];
-    __shared__ unsigned least_w, in_float32[2];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, half = lane >> 5, wk = wave % KH, wp = wave / KH;
     const int k0 = (kb * KH + wk) * 32;
     const __amdgpu_buffer_rsrc_t x_rsrc = __builtin_amdgcn_make_buffer_rsrc(p.a[0], 0, (int)(long long)p.a[5], 0x00020000);
@@ -110,8 +91,7 @@ extern "C" __global__ __launch_bounds__(256, 2) void ENTRY(Params p) {
             }
         });
     };
-    auto commit = [&]() -> unsigned {                  // to LDS; float32: the smallest magnitude's key
-        unsigned least = ~0u;
+    auto commit = [&]() {                              // to LDS
         unsigned t = tid;
         asm volatile("" : "+v"(t));
         mjt_static_for<0, NI>([&](auto ic) {
@@ -121,8 +101,8 @@ extern "C" __global__ __launch_bounds__(256, 2) void ENTRY(Params p) {
                 unsigned char* const to = lds + (row * PITCH + LP + q * G) * 2;
 #if IN == 2
                 unsigned a[2][3];
-                mjt_split(xv[i][0], G > 1 ? xv[i][G > 1 ? 1 : 0] : 0u, a[0], least);
-                if constexpr (G == 4) mjt_split(xv[i][GD - 2], xv[i][GD - 1], a[1], least);
+                mjt_split(xv[i][0], G > 1 ? xv[i][G > 1 ? 1 : 0] : 0u, a[0][0], a[0][1], a[0][2]);
+                if constexpr (G == 4) mjt_split(xv[i][GD - 2], xv[i][GD - 1], a[1][0], a[1][1], a[1][2]);
                 mjt_static_for<0, 3>([&](auto pc) {
                     constexpr int part = decltype(pc)::v;
                     if constexpr (G == 4) *(mjt_u32x2v*)(to + part * PARTB) = (mjt_u32x2v){a[0][part], a[1][part]};
@@ -136,13 +116,11 @@ extern "C" __global__ __launch_bounds__(256, 2) void ENTRY(Params p) {
 #endif
             }
         });
-        return least;
     };
 
     // the weights of the wave's channels, by way of LDS: lane (l32, half) holds channel l32 and row 2 * step + half of taps
     fetch(first);
     mjt_u32x4v wf[STEPS][PARTS];
-    if (tid == 0) { least_w = ~0u; in_float32[0] = in_float32[1] = 0; }
     for (int i = tid; i < 32 * KH * CRS; i += 256) {
         const int k = i / CRS, e = i - k * CRS, ko = kb * KH * 32 + k;
 #if IN == 2
@@ -153,7 +131,6 @@ extern "C" __global__ __launch_bounds__(256, 2) void ENTRY(Params p) {
     }
     __syncthreads();
     {
-        unsigned least = ~0u;
         const unsigned* const from = (const unsigned*)lds + (wk * 32 + l32) * WPITCH;
         mjt_static_for<0, STEPS>([&](auto sc) {
             constexpr int step = decltype(sc)::v;
@@ -169,29 +146,24 @@ extern "C" __global__ __launch_bounds__(256, 2) void ENTRY(Params p) {
                 constexpr int d = decltype(dc)::v;
 #if IN == 2
                 unsigned a[3];
-                mjt_split(v[2 * d], v[2 * d + 1], a, least);
+                mjt_split(v[2 * d], v[2 * d + 1], a[0], a[1], a[2]);
                 mjt_static_for<0, 3>([&](auto pc) { wf[step][decltype(pc)::v][d] = a[decltype(pc)::v]; });
 #else
                 wf[step][0][d] = v[2 * d] | v[2 * d + 1] << 16;
 #endif
             });
         });
-        if (IN == 2) atomicMin(&least_w, least);
     }
     __syncthreads();
-    const unsigned low_w = least_w;
     for (int i = tid * 16; i < LDSB / 16 * 16; i += 256 * 16) *(mjt_u32x4v*)(lds + i) = (mjt_u32x4v)(0u);      // (margins stay zero)
     for (int i = LDSB / 16 * 16 + tid; i < LDSB; i += 256) lds[i] = 0;
 
 #pragma unroll 1
     for (int tile = first; tile < last; tile++) {
         __syncthreads();
-        const unsigned low = commit();
-        if (IN == 2 && (low < MJT_KEY(-100) || low_w < MJT_KEY(-100) || (low >> 24) + (low_w >> 24) < 2 * 127 - 100)) in_float32[tile & 1] = 1;
-        if (tid == 0) in_float32[(tile + 1) & 1] = 0;  // (read before the barrier above, set after the one below)
+        commit();
         __syncthreads();
         if (tile + 1 < last) fetch(tile + 1);
-        const bool wide = IN == 2 && in_float32[tile & 1] != 0;
         const int n = tile / TPI, oh0 = (tile - n * TPI) * TR;
 #pragma unroll 1
         for (int pt = wp; pt < PT; pt += PW_) {
@@ -200,49 +172,45 @@ extern "C" __global__ __launch_bounds__(256, 2) void ENTRY(Params p) {
             const int row = q / OW_, col = q - row * OW_;
             const unsigned char* const from = lds + (row * SH * PITCH + FIRST + 2 * col) * 2;
             mjt_f32x16 acc = (mjt_f32x16)(0.0f), acc2 = (mjt_f32x16)(0.0f);
-            bool again = wide;
-            if (!again) {
-                // operand f: part 2, 1 or 0 (16 bits: the only one) of step f / PARTS, asked for three operands ahead of its MFMAs
-                mjt_u32x4v ring[4];
-                auto request = [&](auto fc) {
-                    constexpr int f = decltype(fc)::v, step = f / PARTS, part = PARTS - 1 - f % PARTS, r0 = 2 * step, r1 = 2 * step + 1 < ROWS ? 2 * step + 1 : 2 * step;
-                    const unsigned char* const at = from + (half ? row_at(r1) : row_at(r0)) + part * PARTB;
-                    mjt_static_for<0, 4>([&](auto dc) { ring[f % 4][decltype(dc)::v] = *(const unsigned*)(at + decltype(dc)::v * 4); });
-                };
-                mjt_static_for<0, (STEPS * PARTS < 3 ? STEPS * PARTS : 3)>(request);
-                mjt_static_for<0, STEPS * PARTS>([&](auto fc) {
-                    constexpr int f = decltype(fc)::v, step = f / PARTS, part = PARTS - 1 - f % PARTS;
-                    __builtin_amdgcn_sched_barrier(0);     // (left to itself the compiler asks for an operand where it is needed)
-                    if constexpr (f + 3 < STEPS * PARTS) request(mjt_ic<f + 3>());
-                    mjt_u32x4v b = ring[f % 4];
-                    if constexpr (IN != 2)                 // (what is no tap may be infinite; float32 sums are looked at)
-                        mjt_static_for<0, 4>([&](auto dc) {
-                            constexpr int d = decltype(dc)::v;
-                            if constexpr (mask_of(d) != ~0u) b[d] &= mask_of(d);
-                            if constexpr (2 * step + 1 >= ROWS) b[d] = half ? 0u : b[d];
-                        });
-                    if constexpr (PARTS == 1) {
-                        acc = MJT_MFMA(wf[step][0], b, acc);
-                    } else if constexpr (part == 2) {
-                        acc2 = MJT_MFMA(wf[step][0], b, acc2);
-                    } else if constexpr (part == 1) {
-                        acc2 = MJT_MFMA(wf[step][1 % PARTS], b, acc2);
-                        acc2 = MJT_MFMA(wf[step][0], b, acc2);
-                    } else {
-                        acc2 = MJT_MFMA(wf[step][2 % PARTS], b, acc2);
-                        acc = MJT_MFMA(wf[step][0], b, acc);
-                        acc2 = MJT_MFMA(wf[step][1 % PARTS], b, acc2);
-                    }
-                });
-#if IN == 2
-                acc += acc2;
-                float z = 0.0f;                        // not zero if any sum is not finite
-                mjt_static_for<0, 16>([&](auto ec) { z += acc[decltype(ec)::v] * 0.0f; });
-                again = __any(!(z == 0.0f));
-#endif
-            }
+            // operand f: part 2, 1 or 0 (16 bits: the only one) of step f / PARTS, asked for three operands ahead of its MFMAs
+            mjt_u32x4v ring[4];
+            auto request = [&](auto fc) {
+                constexpr int f = decltype(fc)::v, step = f / PARTS, part = PARTS - 1 - f % PARTS, r0 = 2 * step, r1 = 2 * step + 1 < ROWS ? 2 * step + 1 : 2 * step;
+                const unsigned char* const at = from + (half ? row_at(r1) : row_at(r0)) + part * PARTB;
+                mjt_static_for<0, 4>([&](auto dc) { ring[f % 4][decltype(dc)::v] = *(const unsigned*)(at + decltype(dc)::v * 4); });
+            };
+            mjt_static_for<0, (STEPS * PARTS < 3 ? STEPS * PARTS : 3)>(request);
+            mjt_static_for<0, STEPS * PARTS>([&](auto fc) {
+                constexpr int f = decltype(fc)::v, step = f / PARTS, part = PARTS - 1 - f % PARTS;
+                __builtin_amdgcn_sched_barrier(0);     // (left to itself the compiler asks for an operand where it is needed)
+                if constexpr (f + 3 < STEPS * PARTS) request(mjt_ic<f + 3>());
+                mjt_u32x4v b = ring[f % 4];
+                if constexpr (IN != 2)                 // (what is no tap may be infinite; float32 sums are looked at)
+                    mjt_static_for<0, 4>([&](auto dc) {
+                        constexpr int d = decltype(dc)::v;
+                        if constexpr (mask_of(d) != ~0u) b[d] &= mask_of(d);
+                        if constexpr (2 * step + 1 >= ROWS) b[d] = half ? 0u : b[d];
+                    });
+                if constexpr (PARTS == 1) {
+                    acc = MJT_MFMA(wf[step][0], b, acc);
+                } else if constexpr (part == 2) {
+                    acc2 = MJT_MFMA(wf[step][0], b, acc2);
+                } else if constexpr (part == 1) {
+                    acc2 = MJT_MFMA(wf[step][1 % PARTS], b, acc2);
+                    acc2 = MJT_MFMA(wf[step][0], b, acc2);
+                } else {
+                    acc2 = MJT_MFMA(wf[step][2 % PARTS], b, acc2);
+                    acc = MJT_MFMA(wf[step][0], b, acc);
+                    acc2 = MJT_MFMA(wf[step][1 % PARTS], b, acc2);
+                }
+            });
             const int oh = oh0 + row;
 #if IN == 2
+            acc += acc2;
+            float z = 0.0f;                        // not zero if any sum is not finite
+            mjt_static_for<0, 16>([&](auto ec) { z += acc[decltype(ec)::v] * 0.0f; });
+            const bool again = __any(!(z == 0.0f));
+            acc *= MJT_SPLIT_DOWN;
             if (again) {
                 acc = (mjt_f32x16)(0.0f);
                 const int ih0 = oh * SH - PH, iw0 = col * 2 - PW, ko = k0 + l32 < K_ ? k0 + l32 : K_ - 1;

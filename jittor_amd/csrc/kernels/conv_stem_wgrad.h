@@ -1,7 +1,7 @@
 // Weight gradient of a float32 convolution of images with few channels, the first layer of a network, from windows that lie in LDS:
 //   dw[k][c][r][s] = sum_{n,oh,ow} dy[n][k][oh][ow] * x[n][c][oh*SH-PH+r*DH][ow*2-PW+s]
 // (python/jittor/nn.py:1251-1262 differentiated by ops/reduce_op.cc:339-362; opt/tuner/conv_tuner.cc:375-397 relays it) with horizontal stride 2.  Every
-// value becomes three bfloat16 parts, six of whose nine products are summed (gemm_mfma.h, SPLIT, has the reasoning), in float32.
+// value becomes three bfloat16 parts, six of whose nine products are summed (split.h has the reasoning), in float32.
 //
 // What it replaces, the product that gathers both operands (gemm_mfma.h, CONV 2), loads x once for each tap that sees it and multiplies with
 // float32 MFMAs.  Here the rows of x under TR output rows lie in LDS, split, even and odd columns apart: a column (c, r, s) of the product
@@ -14,19 +14,15 @@
 // 2.4e-7 / 1.8e-7 at 1 x 3 x 224 x 224.  What bounds it: 49 GFLOP of parts and padding on the MFMAs (39 at the rate of a large bfloat16 product) beside 5 dwords of LDS
 // and 4 shifts for every operand of 8 pixels; the fold takes 10.
 //
-// Sums whose operands leave the range of the parts (smallest magnitudes, zeros apart, below 2^-100, alone or multiplied) or that are not finite
-// are thrown away, and the workgroup's slice comes from float32 MFMAs over memory.
+// Sums that are not finite are thrown away, and the workgroup's slice comes from float32 MFMAs over memory.
 //
 // Supplied by the host: C_, H_, W_, K_, R_, S_, OH_, OW_, SH, PH, PW, DH, TR (output rows of a tile).
 
 typedef float mjt_f32x16 __attribute__((ext_vector_type(16)));
-typedef float mjt_f32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned mjt_u32x4v __attribute__((ext_vector_type(4)));
-typedef __bf16 mjt_b16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 mjt_h8 __attribute__((ext_vector_type(8)));
 #define MJT_MFMA(a, b, c) __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(mjt_h8, a), __builtin_bit_cast(mjt_h8, b), c, 0, 0, 0)
 #define MJT_NONE 0x80000000u         // an offset beyond every buffer (they are smaller than 2 GB): the load delivers zeros
-#define MJT_KEY(e) ((unsigned)(127 + (e)) << 24)
 
 template <int V> struct mjt_ic { static constexpr int v = V; };
 template <int I, int N, class F> __device__ __forceinline__ void mjt_static_for(F&& f) {
@@ -50,20 +46,6 @@ constexpr int G = W_ % 4 == 0 ? 4 : W_ % 2 == 0 ? 2 : 1, XU = C_ * XR * (W_ / G)
 constexpr int GY = OW_ % 4 == 0 ? 4 : OW_ % 2 == 0 ? 2 : 1;            // values of a load of x, of dy
 static_assert(LDSB <= 160 * 1024, "LDS");
 
-__device__ __forceinline__ unsigned mjt_bf16_pair(float x, float y) {  // both rounded to nearest even
-    return __builtin_bit_cast(unsigned, __builtin_convertvector((mjt_f32x2){x, y}, mjt_b16x2));
-}
-__device__ __forceinline__ float mjt_low(unsigned p) { return __uint_as_float(p << 16); }
-__device__ __forceinline__ float mjt_high(unsigned p) { return __uint_as_float(p & 0xffff0000u); }
-// two values as three parts, each the rest of the ones before it; `least`: the smallest 2 |value| - 1 of the bits (zeros wrap round)
-__device__ __forceinline__ void mjt_split(unsigned a, unsigned b, unsigned& h, unsigned& m, unsigned& l, unsigned& least) {
-    const float x = __uint_as_float(a), y = __uint_as_float(b);
-    h = mjt_bf16_pair(x, y);
-    const float x1 = x - mjt_low(h), y1 = y - mjt_high(h);
-    m = mjt_bf16_pair(x1, y1);
-    l = mjt_bf16_pair(x1 - mjt_low(m), y1 - mjt_high(m));
-    least = min(least, min((a << 1) - 1u, (b << 1) - 1u));
-}
 // G values from byte `off` on
 template <int N> __device__ __forceinline__ void mjt_load(__amdgpu_buffer_rsrc_t r, unsigned off, unsigned* to) {
     if constexpr (N == 4) {
@@ -82,7 +64,7 @@ extern "C" __global__ __launch_bounds__(256, 2) void ENTRY(Params p) {
     const int kb = blockIdx.x % KBLOCKS, slice = blockIdx.x / KBLOCKS, first = slice * per, last = first + per < tiles ? first + per : tiles;
     if (first >= tiles) return;
     __shared__ __attribute__((aligned(16))) unsigned char lds[LDSB];
-    __shared__ unsigned least_x, least_d, unsound;
+    __shared__ unsigned unsound;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, half = lane >> 5, wk = wave % KH, group = wave / KH;
     const int k = (kb * KH + wk) * 32 + l32;
     const __amdgpu_buffer_rsrc_t x_rsrc = __builtin_amdgcn_make_buffer_rsrc(p.a[0], 0, (int)(long long)p.a[5], 0x00020000);
@@ -100,7 +82,6 @@ extern "C" __global__ __launch_bounds__(256, 2) void ENTRY(Params p) {
             mjt_load<G>(x_rsrc, in ? (unsigned)(((n * C_ + c) * H_ + ih) * W_ + q * G) * 4u : MJT_NONE, xv[i]);
         });
     };
-    unsigned low_x = ~0u, low_d = ~0u;
     auto commit = [&]() {                              // to LDS, as parts: [part][c][row][even, odd columns][column / 2]
         unsigned t = tid;
         asm volatile("" : "+v"(t));
@@ -111,15 +92,15 @@ extern "C" __global__ __launch_bounds__(256, 2) void ENTRY(Params p) {
                 unsigned e[3], o[3];                   // even columns and odd ones, two each (or one)
                 unsigned char* const to = lds + (row * 2 * PL + (col >> 1)) * 2;
                 if constexpr (G == 4) {
-                    mjt_split(xv[i][0], xv[i][G / 2], e[0], e[1], e[2], low_x);
-                    mjt_split(xv[i][G / 4], xv[i][G - 1], o[0], o[1], o[2], low_x);
+                    mjt_split(xv[i][0], xv[i][G / 2], e[0], e[1], e[2]);
+                    mjt_split(xv[i][G / 4], xv[i][G - 1], o[0], o[1], o[2]);
                     mjt_static_for<0, 3>([&](auto pc) {
                         constexpr int part = decltype(pc)::v;
                         *(unsigned*)(to + part * PARTB) = e[part];
                         *(unsigned*)(to + part * PARTB + PL * 2) = o[part];
                     });
                 } else {
-                    mjt_split(xv[i][0], xv[i][G - 1], e[0], e[1], e[2], low_x);
+                    mjt_split(xv[i][0], xv[i][G - 1], e[0], e[1], e[2]);
                     mjt_static_for<0, 3>([&](auto pc) {
                         constexpr int part = decltype(pc)::v;
                         if constexpr (G == 2) {
@@ -157,7 +138,7 @@ extern "C" __global__ __launch_bounds__(256, 2) void ENTRY(Params p) {
     mjt_static_for<0, NT>([&](auto tc) { acc[decltype(tc)::v] = (mjt_f32x16)(0.0f); });
 
     fetch(first);
-    if (tid == 0) { least_x = least_d = ~0u; unsound = 0; }
+    if (tid == 0) unsound = 0;
     for (int i = tid * 16; i < LDSB / 16 * 16; i += 256 * 16) *(mjt_u32x4v*)(lds + i) = (mjt_u32x4v)(0u);      // (margins stay zero)
 #pragma unroll 1
     for (int tile = first; tile < last; tile++) {
@@ -173,7 +154,7 @@ extern "C" __global__ __launch_bounds__(256, 2) void ENTRY(Params p) {
             unsigned a[3][4];
             mjt_static_for<0, 4>([&](auto ec) {
                 constexpr int e = decltype(ec)::v;
-                mjt_split(dv[2 * e], dv[2 * e + 1], a[0][e], a[1][e], a[2][e], low_d);
+                mjt_split(dv[2 * e], dv[2 * e + 1], a[0][e], a[1][e], a[2][e]);
             });
             fetch_dy(n, oh0, u + GROUPS, dv);
             const mjt_u32x4v ah = {a[0][0], a[0][1], a[0][2], a[0][3]}, am = {a[1][0], a[1][1], a[1][2], a[1][3]}, al = {a[2][0], a[2][1], a[2][2], a[2][3]};
@@ -205,11 +186,10 @@ extern "C" __global__ __launch_bounds__(256, 2) void ENTRY(Params p) {
         float z = 0.0f;                                // not zero if any sum is not finite
         mjt_static_for<0, NT * 16>([&](auto ec) { z += acc[decltype(ec)::v / 16][decltype(ec)::v % 16] * 0.0f; });
         if (!(z == 0.0f)) unsound = 1;
-        atomicMin(&least_x, low_x);
-        atomicMin(&least_d, low_d);
+        mjt_static_for<0, NT>([&](auto tc) { acc[decltype(tc)::v] *= MJT_SPLIT_DOWN; });
     }
     __syncthreads();
-    if (unsound || least_x < MJT_KEY(-100) || least_d < MJT_KEY(-100) || (least_x >> 24) + (least_d >> 24) < 2 * 127 - 100) {
+    if (unsound) {
         mjt_static_for<0, NT>([&](auto tc) { acc[decltype(tc)::v] = (mjt_f32x16)(0.0f); });
 #pragma unroll 1
         for (int tile = first; tile < last; tile++) {

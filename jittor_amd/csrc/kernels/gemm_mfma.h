@@ -28,16 +28,10 @@
 // 1700 cycles of a 64 x 64 float32 stage.  us before / now, in turn: float32 a b^T 2048 x 1024 x 1024 51 / 43,
 // 2048^3 163 / 143, a^T b 1024 x 1024 x 2048 72 / 58; bfloat16 2048 x 2048 x 2048 32.5 / 23, 12544 x 256 x 1024 18.8 / 14.)
 // SPLIT = 1 (float32): the float32 MFMAs, 140 TFLOP/s measured, bound the large products, and the bfloat16 ones run at 16 times their
-// rate.  On its way to LDS every value becomes three bfloat16 parts, x = h + m + l, each the rest so far rounded to nearest: 24 bits,
-// all of x.  Six of the nine products of two such values are summed, l h + h l + m m + m h + h m into one accumulator and h h into
-// another; what is left out, m l + l m + l l, is below 2^-26 of the product.  A bfloat16 MFMA rounds once per 16 products where
-// the float32 one rounds per product, so the result is closer to 64 bits than before (relative error, normal operands, K = 64 / 1024 /
-// 4096: 1.4e-7 / 5.7e-7 / 1.15e-6 before, 5e-8 / 1.9e-7 / 4.0e-7 so; also for positive operands and for ones over 9 decades).
-// The parts hold where nothing overflows and nothing falls below the normal range, which the bfloat16 MFMAs take for zero: a
-// workgroup whose operands' smallest magnitudes (zeros apart) are below 2^-100, alone or multiplied, or whose sums are not
-// all finite (an infinity's other parts are NaN), throws its sums away and runs the float32 loop.  Eight waves share a tile,
+// rate.  On its way to LDS every value becomes three bfloat16 parts (split.h, which has the reasoning and the error).  A
+// workgroup whose sums are not all finite throws them away and runs the float32 loop.  Eight waves share a tile,
 // two to a SIMD: one splits while the other's MFMAs run (a b^T 2048 x 1024 x 1024 on 128 x 64 tiles 36.1 us with four waves, 31.0 with
-// eight; 4096 x 4096 x 2048 on 128 x 128 415 / 375).  What bounds it: splitting, 11 vector instructions for two values, takes as
+// eight; 4096 x 4096 x 2048 on 128 x 128 415 / 375).  What bounds it: splitting, 13 vector instructions for two values, takes as
 // long as the MFMAs on 128 x 64 tiles, LDS carries 6 bytes for each value (without the writes 28.5 us, without the loads 24.8, with
 // one MFMA of six 21); a third buffer changes nothing (33), nor does splitting by truncation (30.4) or by v_dot2 (31.2).
 // float32 uses v_mfma_f32_32x32x2: a lane's 16-byte read holds 4 k of its row, which feed
@@ -176,47 +170,19 @@ __device__ __forceinline__ mjt_u32x4v mjt_transpose4x4_b32(mjt_u32x4v v, int lan
 #if SPLIT
 typedef __bf16 mjt_h8 __attribute__((ext_vector_type(8)));
 typedef unsigned mjt_u32x2v __attribute__((ext_vector_type(2)));
-typedef float mjt_f32x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 mjt_b16x2 __attribute__((ext_vector_type(2)));
 #define MJT_MFMA16(a, b, c) __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0)
-__device__ __forceinline__ unsigned mjt_bf16_pair(float x, float y) {      // both rounded to nearest even
-    return __builtin_bit_cast(unsigned, __builtin_convertvector((mjt_f32x2){x, y}, mjt_b16x2));
-}
-#define MJT_KEY(e) ((unsigned)(127 + (e)) << 24)
-template <int CTRL, int ROWS> __device__ __forceinline__ unsigned mjt_min_dpp(unsigned v) {
-    return min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, CTRL, ROWS, 0xf, false));
-}
-__device__ __forceinline__ unsigned mjt_wave_min(unsigned v) {             // of all 64 lanes, in every lane
-    v = mjt_min_dpp<0x111, 0xf>(v);                                        // from the lane 1, 2, 4, 8 below, inside rows of 16
-    v = mjt_min_dpp<0x112, 0xf>(v);
-    v = mjt_min_dpp<0x114, 0xf>(v);
-    v = mjt_min_dpp<0x118, 0xf>(v);
-    v = mjt_min_dpp<0x142, 0xa>(v);                                        // a row's last lane to the next row; lane 31 to the upper half
-    v = mjt_min_dpp<0x143, 0xc>(v);
-    return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
-}
-__device__ __forceinline__ float mjt_low(unsigned p) { return __uint_as_float(p << 16); }
-__device__ __forceinline__ float mjt_high(unsigned p) { return __uint_as_float(p & 0xffff0000u); }
 #endif
-// One 16-byte chunk on its way to LDS.  SP: as its three bfloat16 parts, each the rest of the ones before it rounded to nearest;
-// `least` keeps the smallest 2 |value| - 1 of the bits as integers (zeros wrap round to the largest).
-template <bool SP> __device__ __forceinline__ void mjt_put(unsigned char* lds, int row, int kc, mjt_u32x4v v, unsigned& least) {
+// One 16-byte chunk on its way to LDS.  SP: as its three bfloat16 parts.
+template <bool SP> __device__ __forceinline__ void mjt_put(unsigned char* lds, int row, int kc, mjt_u32x4v v) {
 #if SPLIT
     if constexpr (SP) {
         unsigned char* const at = lds + row * SPLIT_ROWB + kc * 8;
-        mjt_u32x2v h, m, l;
-#pragma unroll
-        for (int p = 0; p < 2; p++) {
-            const float x = __uint_as_float(v[2 * p]), y = __uint_as_float(v[2 * p + 1]);
-            h[p] = mjt_bf16_pair(x, y);
-            const float x1 = x - mjt_low(h[p]), y1 = y - mjt_high(h[p]);
-            m[p] = mjt_bf16_pair(x1, y1);
-            l[p] = mjt_bf16_pair(x1 - mjt_low(m[p]), y1 - mjt_high(m[p]));
-            least = min(least, min((v[2 * p] << 1) - 1u, (v[2 * p + 1] << 1) - 1u));
-        }
-        *(mjt_u32x2v*)at = h;
-        *(mjt_u32x2v*)(at + 64) = m;
-        *(mjt_u32x2v*)(at + 128) = l;
+        unsigned h[2], m[2], l[2];
+        mjt_split(v[0], v[1], h[0], m[0], l[0]);
+        mjt_split(v[2], v[3], h[1], m[1], l[1]);
+        *(mjt_u32x2v*)at = (mjt_u32x2v){h[0], h[1]};
+        *(mjt_u32x2v*)(at + 64) = (mjt_u32x2v){m[0], m[1]};
+        *(mjt_u32x2v*)(at + 128) = (mjt_u32x2v){l[0], l[1]};
         return;
     }
 #endif
@@ -262,7 +228,7 @@ template <int ROWS, bool KCONT> struct mjt_stager {
             reg[I] = *(const mjt_u32x4v*)(p + (long long)kk * ld + col);
         }
     }
-    template <int I, bool FULL, bool SP> __device__ __forceinline__ void commit(unsigned char* lds, int k0, int K, int tid, unsigned& least) const {
+    template <int I, bool FULL, bool SP> __device__ __forceinline__ void commit(unsigned char* lds, int k0, int K, int tid) const {
         mjt_u32x4v v = reg[I];
         int row, kc;
         if constexpr (KCONT) {
@@ -292,7 +258,7 @@ template <int ROWS, bool KCONT> struct mjt_stager {
             v = mjt_transpose8x8_b16(v, tid);
 #endif
         }
-        mjt_put<SP>(lds, row, kc, v, least);
+        mjt_put<SP>(lds, row, kc, v);
     }
 };
 
@@ -375,13 +341,13 @@ struct mjt_conv_stager {
 #endif
         });
     }
-    template <int I, bool SP> __device__ __forceinline__ void commit(unsigned char* lds, int tid, unsigned& least) const {
+    template <int I, bool SP> __device__ __forceinline__ void commit(unsigned char* lds, int tid) const {
         const int b = tid / EPC + I * (NTHR / EPC);
         const int row = (b % (TN / EPC)) * EPC + tid % EPC, kc = b / (TN / EPC);
 #if IN == 2
-        mjt_put<SP>(lds, row, kc, mjt_transpose4x4_b32(mjt_wg_pack(v[I]), tid), least);
+        mjt_put<SP>(lds, row, kc, mjt_transpose4x4_b32(mjt_wg_pack(v[I]), tid));
 #else
-        mjt_put<SP>(lds, row, kc, mjt_transpose8x8_b16(mjt_wg_pack(v[I]), tid), least);
+        mjt_put<SP>(lds, row, kc, mjt_transpose8x8_b16(mjt_wg_pack(v[I]), tid));
 #endif
     }
 };
@@ -456,8 +422,8 @@ template <int ROWS> struct mjt_wg_plane {
             });
         }
     }
-    template <int I, bool SP> __device__ __forceinline__ void commit(unsigned char* lds, int tid, unsigned& least) const {
-        mjt_put<SP>(lds, tid / KC + I * (NTHR / KC), tid % KC, reg[I], least);
+    template <int I, bool SP> __device__ __forceinline__ void commit(unsigned char* lds, int tid) const {
+        mjt_put<SP>(lds, tid / KC + I * (NTHR / KC), tid % KC, reg[I]);
     }
 };
 typedef mjt_wg_plane<TM> mjt_wg_dy;
@@ -486,8 +452,8 @@ struct mjt_wg_x {
             v[I][e] = mjt_wg_load(d, in ? ch.x[e] + koff[I] : MJT_NONE);
         });
     }
-    template <int I, bool SP> __device__ __forceinline__ void commit(unsigned char* lds, int tid, unsigned& least) const {
-        mjt_put<SP>(lds, tid / KC + I * (NTHR / KC), tid % KC, mjt_wg_pack(v[I]), least);
+    template <int I, bool SP> __device__ __forceinline__ void commit(unsigned char* lds, int tid) const {
+        mjt_put<SP>(lds, tid / KC + I * (NTHR / KC), tid % KC, mjt_wg_pack(v[I]));
     }
 };
 #endif
@@ -539,11 +505,8 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
     // NBUF 1: the host promises K <= KS, a single stage -- one staging buffer, so twice as many workgroups fit a compute unit
     __shared__ __attribute__((aligned(16))) unsigned char lds[NBUF][(TM + TN) * SPLIT_ROWB];
 #if SPLIT
-    // [0]: seen with the first stage, [1]: with the sums.  (Two: with a single stage no barrier keeps a wave that sets the second from
-    // one that has yet to read the first.)
-    __shared__ int in_float32[2];
-    __shared__ unsigned least[2];
-    if (threadIdx.x < 2) in_float32[threadIdx.x] = 0, least[threadIdx.x] = ~0u;
+    __shared__ int in_float32;                                 // some sum is not finite
+    if (threadIdx.x == 0) in_float32 = 0;
     __syncthreads();
 #endif
 
@@ -569,7 +532,6 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
     auto multiply = [&](auto spc) -> bool {
     constexpr bool SP = decltype(spc)::v != 0;
     constexpr int RB = SP ? SPLIT_ROWB : ROWB, BUFB = (TM + TN) * RB;
-    unsigned least_a = ~0u, least_b = ~0u;
     constexpr int NSET = NBUF > 1 && STAGES != 2 && MI * NI <= (CONV ? 1 : 4) ? 2 : 1;
 #if CONV == 2
     const int all_stages = (K + KS - 1) / KS;
@@ -592,8 +554,8 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
     auto commit = [&](auto ic, auto setc, auto, int stage) {
         constexpr int I = decltype(ic)::v, SET = decltype(setc)::v;
         unsigned char* buf = &lds[0][0] + (stage & (NBUF - 1)) * BUFB;
-        if constexpr (I < PA) sa[SET].template commit<I, SP>(buf, tid, least_a);
-        else sb[SET].template commit<I - PA, SP>(buf + TM * RB, tid, least_b);
+        if constexpr (I < PA) sa[SET].template commit<I, SP>(buf, tid);
+        else sb[SET].template commit<I - PA, SP>(buf + TM * RB, tid);
     };
 #else
 #if SLICED
@@ -631,11 +593,11 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
         constexpr int I = decltype(ic)::v, SET = decltype(setc)::v;
         constexpr bool FULL = decltype(fullc)::v != 0;
         unsigned char* buf = &lds[0][0] + (stage & (NBUF - 1)) * BUFB;
-        if constexpr (I < PA) sa[SET].template commit<I, FULL, SP>(buf, (first_stage + stage) * KS, K, tid, least_a);
+        if constexpr (I < PA) sa[SET].template commit<I, FULL, SP>(buf, (first_stage + stage) * KS, K, tid);
 #if CONV
-        else sb[SET].template commit<I - PA, SP>(buf + TM * RB, tid, least_b);
+        else sb[SET].template commit<I - PA, SP>(buf + TM * RB, tid);
 #else
-        else sb[SET].template commit<I - PA, FULL, SP>(buf + TM * RB, (first_stage + stage) * KS, K, tid, least_b);
+        else sb[SET].template commit<I - PA, FULL, SP>(buf + TM * RB, (first_stage + stage) * KS, K, tid);
 #endif
     };
 #endif
@@ -655,16 +617,8 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
             }
 
     mjt_static_for<0, PIECES>([&](auto ic) { commit(ic, mjt_ic<0>(), mjt_ic<0>(), 0); });
-#if SPLIT
-    if constexpr (SP)
-        if (min(least_a, least_b) < MJT_KEY(-100)) in_float32[0] = 1;
-#endif
     if (NSET < nstages) mjt_static_for<0, PIECES>([&](auto ic) { fetch(ic, mjt_ic<0>(), mjt_ic<0>(), NSET); });
     __syncthreads();
-#if SPLIT
-    if constexpr (SP)
-        if (in_float32[0]) return false;                       // (usually seen here, where little is lost)
-#endif
 
     // fragment addresses of this lane: row lane % 32 of its wave's tile rows, chunk lane / 32
     const int frow = lane & 31, fhalf = lane >> 5;
@@ -768,16 +722,11 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
                 for (int e = 0; e < 16; e++) {
                     acc[i][j][e] += low[i][j][e];
                     z = __builtin_fmaf(acc[i][j][e], 0.0f, z);
+                    acc[i][j][e] *= MJT_SPLIT_DOWN;
                 }
-        const unsigned wave_a = mjt_wave_min(least_a), wave_b = mjt_wave_min(least_b);
-        if (lane == 0) {
-            atomicMin(&least[0], wave_a);
-            atomicMin(&least[1], wave_b);
-        }
-        if (z != 0.0f) in_float32[1] = 1;
+        if (z != 0.0f) in_float32 = 1;
         __syncthreads();
-        const unsigned all_a = least[0], all_b = least[1];
-        if (in_float32[1] || all_a < MJT_KEY(-100) || all_b < MJT_KEY(-100) || (all_a >> 24) + (all_b >> 24) < 2 * 127 - 100) return false;
+        if (in_float32) return false;
     }
 #endif
 

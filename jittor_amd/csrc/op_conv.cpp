@@ -216,7 +216,7 @@ static bool conv_stem(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor
         src << "#define ENTRY " << name.str() << "\n#define IN " << in << "\n#define Y_16 " << narrow << "\n#define TR " << TR << "\n#define C_ " << C << "\n#define H_ " << H << "\n#define W_ " << W
             << "\n#define K_ " << K << "\n#define R_ " << R << "\n#define S_ " << S << "\n#define OH_ " << OH << "\n#define OW_ " << OW << "\n#define SH " << SH << "\n#define PH " << PH
             << "\n#define PW " << PW << "\n#define DH " << DH << "\n";
-        src << embedded_source("conv_stem.h") << "\n";
+        src << embedded_source("split.h") << "\n" << embedded_source("conv_stem.h") << "\n";
         k = jit_get(src.str(), name.str());
         remember(key.str(), k);
     }
@@ -684,6 +684,7 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
                 std::ostringstream src;
                 src << "#define ENTRY " << name.str() << "\n#define SPLIT " << (split ? 1 : 0) << "\n#define CONV 1\n#define IN " << in << "\n#define OUT " << out << "\n#define MI " << MI << "\n#define NI " << NI
                     << "\n#define A_KCONT 1\n#define B_KCONT 0\n#define XBUF " << (xbuf ? 1 : 0) << "\n" << geo.str();
+                if (split) src << embedded_source("split.h") << "\n";
                 src << embedded_source("gemm_mfma.h") << "\n";
                 k = jit_get(src.str(), name.str());
                 remember(key.str(), k);
@@ -1017,7 +1018,7 @@ static bool conv_wgrad_stem(const mjt_tensor* x, const mjt_tensor* dy, const mjt
         std::ostringstream src;
         src << "#define ENTRY " << name.str() << "\n#define TR " << TR << "\n#define C_ " << C << "\n#define H_ " << H << "\n#define W_ " << W << "\n#define K_ " << K << "\n#define R_ " << R
             << "\n#define S_ " << S << "\n#define OH_ " << OH << "\n#define OW_ " << OW << "\n#define SH " << SH << "\n#define PH " << PH << "\n#define PW " << PW << "\n#define DH " << DH << "\n";
-        src << embedded_source("conv_stem_wgrad.h") << "\n";
+        src << embedded_source("split.h") << "\n" << embedded_source("conv_stem_wgrad.h") << "\n";
         k = jit_get(src.str(), name.str());
         remember(key.str(), k);
     }
@@ -1114,6 +1115,7 @@ static bool conv_wgrad_product(const mjt_tensor* x, const mjt_tensor* dy, const 
             << "\n#define C_ " << C << "\n#define H_ " << H << "\n#define W_ " << W << "\n#define K_ " << K << "\n#define R_ " << R << "\n#define S_ " << S << "\n#define OH_ " << OH
             << "\n#define OW_ " << OW << "\n#define SH " << p->stride_h << "\n#define SW " << p->stride_w << "\n#define PH " << p->pad_h << "\n#define PW " << p->pad_w << "\n#define DH " << p->dil_h
             << "\n#define DW " << p->dil_w << "\n";
+        if (split) src << embedded_source("split.h") << "\n";
         src << embedded_source("gemm_mfma.h") << "\n";
         k = jit_get(src.str(), name.str());
         remember(key.str(), k);

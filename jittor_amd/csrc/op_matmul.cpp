@@ -221,6 +221,7 @@ void gemm_launch(int in_dtype, int out_dtype, const void* A, const void* B, void
             src << "#define NBUF " << (one_stage ? 1 : 2) << "\n#define SLICED " << (slices > 1 ? 1 : 0) << "\n#define SPLIT " << (split ? 1 : 0) << "\n";
             src << "#define ENTRY " << name.str() << "\n#define IN " << in << "\n#define OUT " << out << "\n#define MI " << MI
                 << "\n#define NI " << NI << "\n#define A_KCONT " << (a_kcont ? 1 : 0) << "\n#define B_KCONT " << (b_kcont ? 1 : 0) << "\n";
+            if (split) src << embedded_source("split.h") << "\n";
             src << embedded_source("gemm_mfma.h") << "\n";
             k = jit_get(src.str(), name.str());
             remember(key.str(), k);

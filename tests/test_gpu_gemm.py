@@ -341,8 +341,8 @@ def test_gemm_float32_parts(gpu, M, K, N, batch, tile, ta, tb):
 
 @pytest.mark.parametrize("what", ["inf", "nan", "rounds to inf", "denormal", "tiny", "small products", "overflow", "zeros"])
 def test_gemm_float32_parts_hand_over(gpu, what):
-    """Operands whose parts leave bfloat16's range or whose sums are not finite: the tiles concerned run on the float32 MFMAs, results are
-    what float32 gives; the other tiles stay."""
+    """Operands at the ends of float32's range and sums that are not finite, 2^48 times as large as they come: the tiles of the latter run
+    on the float32 MFMAs, results are what float32 gives; the other tiles stay."""
     rng = np.random.default_rng(5)
     M, K, N = 2048, 1024, 1024
     A, B = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((N, K)).astype(np.float32)
@@ -356,7 +356,7 @@ def test_gemm_float32_parts_hand_over(gpu, what):
     elif what == "denormal":
         A[130], A[1999, ::2] = 1e-40, 1.1e-39
         B[:, :] *= np.float32(1e25)
-    elif what == "tiny":                                               # the second and third parts are below the normal range
+    elif what == "tiny":                                               # the second and third parts of the value itself are below the normal range
         A *= np.float32(1e-35)
         B *= np.float32(1e33)
     elif what == "small products":
@@ -405,6 +405,46 @@ def test_gemm_float32_parts_of_a_single_stage(gpu, what):
         assert (np.abs(got[ok] - want[ok]) <= bound[ok]).all()
 
 
+def _scaled_runs(call, inputs, out_shape):
+    """Results of call(*tensors, out) with the first input times 2^-105, 1 and 2^40, taken back, with the kernel's name."""
+    po, got = L.alloc(int(np.prod(out_shape)) * 4), []
+    try:
+        for e in (-105, 0, 40):
+            ps = [_to_dev(inputs[0] * np.float32(2.0 ** e))] + [_to_dev(a) for a in inputs[1:]]
+            try:
+                call(*[L.tensor(q, "float32", a.shape) for q, a in zip(ps, inputs)], L.tensor(po, "float32", out_shape))
+                got.append((L.d2h(po, out_shape, np.float32) * np.float32(2.0 ** -e), L.last_kernel()))
+            finally:
+                for q in ps:
+                    L.free(q)
+    finally:
+        L.free(po)
+    return got
+
+
+@pytest.mark.parametrize("what", ["128x64", "128x128", "slices", "conv", "conv wgrad", "stem", "stem wgrad"])
+def test_float32_parts_take_powers_of_two_out(gpu, what):
+    """Operands of any size run on their parts and no bit depends on their common power of two.  (The float32 MFMAs, to which tiles with values
+    below 2^-100 went, round more often.)"""
+    lib, rng, ref = L.load(), np.random.default_rng(9), ctypes.byref
+    draw = lambda *s: rng.standard_normal(s).astype(np.float32)
+    if what in ("128x64", "128x128", "slices"):
+        M, K, N = {"128x64": (2048, 1024, 1024), "128x128": (1916, 256, 2100), "slices": (512, 1376, 512)}[what]
+        got = _scaled_runs(lambda a, b, c: L.check(lib.mjt_matmul(ref(a), ref(b), ref(c), 0, 1)), [draw(M, K), draw(N, K)], (M, N))
+    else:
+        xs, k, R, p, o = ((2, 3, 224, 224), 32, 7, L.ConvParams(2, 2, 3, 3, 1, 1), 112) if "stem" in what else ((32, 64, 56, 56), 128, 3, L.ConvParams(2, 2, 1, 1, 1, 1), 28)
+        if what == "stem wgrad":
+            xs = (8,) + xs[1:]
+        x, w, dy = draw(*xs), draw(k, xs[1], R, R), draw(xs[0], k, o, o)
+        if "wgrad" in what:
+            got = _scaled_runs(lambda a, b, c: L.check(lib.mjt_conv2d_meta_wgrad(ref(a), ref(b), ref(c), ref(p))), [x, dy], w.shape)
+        else:
+            got = _scaled_runs(lambda a, b, c: L.check(lib.mjt_conv2d_meta(ref(a), ref(b), ref(c), ref(p))), [x, w], dy.shape)
+    for g, kern in got:
+        assert ("_stem_" if "stem" in what else what if "128" in what else "_parts") in kern, kern
+        assert np.array_equal(g, got[1][0]), (what, np.abs(g - got[1][0]).max())
+
+
 def _columns(x, R, stride, pad):
     n, c, h, w = x.shape
     xp = np.pad(x, ((0, 0), (0, 0), (pad, pad), (pad, pad)))
@@ -415,7 +455,7 @@ def _columns(x, R, stride, pad):
 @pytest.mark.parametrize("xs,k,R,stride,tiny", [((16, 40, 27, 27), 200, 3, 1, False), ((16, 39, 27, 27), 100, 3, 1, False), ((32, 64, 56, 56), 128, 3, 2, False),
                                                 ((16, 40, 27, 27), 200, 3, 1, True), ((32, 64, 56, 56), 128, 3, 2, True)])
 def test_conv_float32_parts(gpu, xs, k, R, stride, tiny):
-    """The gathering forward and weight-gradient products on bfloat16 parts; with operands whose parts leave the range too."""
+    """The gathering forward and weight-gradient products on bfloat16 parts; with tiny values and an infinity among the operands too."""
     lib = L.load()
     rng = np.random.default_rng(k)
     x, w = rng.standard_normal(xs).astype(np.float32), rng.standard_normal((k, xs[1], R, R)).astype(np.float32)

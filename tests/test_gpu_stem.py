@@ -1,5 +1,5 @@
 """The convolution of images with few channels from windows in LDS (csrc/kernels/conv_stem.h): rows of 4, 2 and 1 values a load, paddings of
-either parity, remainders of channels, rows and pixels, and float32 operands that the bfloat16 parts do not hold."""
+either parity, remainders of channels, rows and pixels, and float32 operands at the ends of the range."""
 import ctypes
 
 import numpy as np
@@ -100,8 +100,8 @@ def test_stem_convolution_keeps_infinities_in_their_windows(gpu, case, dt):
 
 @pytest.mark.parametrize("xscale,wscale", [(1e-33, 1e-2), (1e-20, 1e-20), (1e18, 1e18), (1e-2, 1e-33), (1e38, 1e-30)])
 def test_stem_convolution_beyond_the_range_of_the_parts(gpu, xscale, wscale):
-    """Operands whose parts would fall below the normal range take the float32 MFMAs, which keep 2^-24 of every product (147 roundings: 1e-5 of
-    the sum of magnitudes) down to results at the edge of the range."""
+    """Operands and results at both ends of float32's range: small ones on the parts of 2^24 their value, those above 2^104 and sums above 2^80 on
+    the float32 MFMAs, which keep 2^-24 of every product (147 roundings: 1e-5 of the sum of magnitudes)."""
     rng = np.random.default_rng(33)
     case = CASES[1]
     ys = _shape(case)

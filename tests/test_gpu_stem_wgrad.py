@@ -1,5 +1,5 @@
 """The weight gradient of float32 convolutions of images with few channels from windows in LDS (csrc/kernels/conv_stem_wgrad.h): loads of 4, 2
-and 1 values of either operand, remainders of channels, columns, rows and pixels, and operands that the bfloat16 parts do not hold."""
+and 1 values of either operand, remainders of channels, columns, rows and pixels, and operands at the ends of the range."""
 import ctypes
 
 import numpy as np
@@ -78,7 +78,8 @@ def test_stem_weight_gradient_keeps_infinities_in_their_taps(gpu, case):
 
 @pytest.mark.parametrize("xscale,dscale", [(1e-33, 1e-2), (1e-20, 1e-19), (1e16, 1e17), (1e-2, 1e-33)])
 def test_stem_weight_gradient_beyond_the_range_of_the_parts(gpu, xscale, dscale):
-    """Operands whose parts would fall below the normal range take the float32 MFMAs (every product 2^-24, a rounding for each of at most 52272 of them)."""
+    """Operands and results at both ends of float32's range: small ones on the parts of 2^24 their value, sums above 2^80 on the float32 MFMAs (every
+    product 2^-24, a rounding for each of at most 52272 of them)."""
     rng = np.random.default_rng(43)
     case = CASES[1]
     x, dy = (rng.uniform(0.5, 1, case["x"]) * xscale).astype(np.float32), (rng.uniform(-1, -0.5, _extents(case)) * dscale).astype(np.float32)
