@@ -4,6 +4,7 @@
 #include "common.h"
 #include <array>
 #include <cmath>
+#include <map>
 #include <mutex>
 #include <unordered_map>
 
@@ -227,6 +228,34 @@ static bool conv_stem(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor
     return true;
 }
 
+// The layout that kernels/conv_strided.h and conv_dgrad_phases.h keep in LDS: outputs or base positions of images of P in rows of W, in planes of PR x PC with
+// the margins that the taps' shifts reach (rlo .. rhi, clo .. chi; `left` columns ahead of a row), loaded `unit` positions at a time.
+struct MarginPlanes {
+    int64_t total, P, W, PR, PC, rlo, rhi, clo, chi, left, unit;
+    // The most positions between the first and the last that a tile of `tile` outputs reads.  Tiles begin at the same places of an image again after P of
+    // them, which a call would have to walk over (us of host time a call: 64 x 32 x 224 x 224 stride 2 256 forward, 98 input gradient), so what was
+    // found is kept.
+    int64_t span(int64_t tile) const {
+        static std::mutex mu;
+        static std::map<std::array<int64_t, 12>, int64_t> kept;
+        const int64_t tiles = std::min((total + tile - 1) / tile, P);
+        const std::array<int64_t, 12> key{tile, tiles, P, W, PR, PC, rlo, rhi, clo, chi, left, unit};
+        {
+            std::lock_guard<std::mutex> lock(mu);
+            auto it = kept.find(key);
+            if (it != kept.end()) return it->second;
+        }
+        auto pos = [&](int64_t f) { return (f / P * PR + f % P / W - rlo) * PC + f % W + left; };
+        int64_t most = 0;
+        for (int64_t t = 0; t < tiles; t++) most = std::max(most, pos(t * tile + tile - 1) + rhi * PC + chi + 1 - (pos(t * tile) + rlo * PC + clo) / unit * unit);
+        most = (most + unit - 1) / unit * unit;
+        std::lock_guard<std::mutex> lock(mu);
+        if (kept.size() >= 1024) kept.clear();
+        kept.emplace(key, most);
+        return most;
+    }
+};
+
 // Convolutions of 16-bit operands with horizontal stride 2 from windows in LDS (kernels/conv_strided.h), for shapes that the row kernel takes too.  False: not
 // covered, or the row kernel is the faster one: more than one tap on maps of less than 100 pixels, whose tiles hold mostly margins, or on more tiles than
 // compute units.  us, row kernel / this: 32 x 256 x 14 x 14 3x3 -> 256 20.7 / 22.3, 32 x 128 x 14 x 14 5x5 -> 128 17.9 / 21.4, 64 x 512 x 14 x 14 3x3 -> 512 45.0 / 56.4, 64 x 128 x
@@ -258,14 +287,10 @@ static bool conv_strided(const mjt_tensor* x, const mjt_tensor* w, const mjt_ten
     }
     const int64_t PR = OH + rhi - rlo, PC = OW + chi - clo, P = OH * OW, total = N * P, nrp = phase[0] && phase[1] ? 2 : 1;
     if (N * PR * PC >= (int64_t(1) << 30)) return false;
-    auto pos = [&](int64_t f) { return (f / P * PR + f % P / OW - rlo) * PC + f % OW - clo; };
-    auto span_of = [&](int64_t tile) {
-        int64_t most = 0;
-        for (int64_t t = 0; t < (total + tile - 1) / tile && t < P; t++)       // (tiles begin at the same places of an image again after that)
-            most = std::max(most, pos(t * tile + tile - 1) + rhi * PC + chi + 1 - (pos(t * tile) + rlo * PC + clo));
-        return most;
-    };
     const int64_t cus = ctx().dry_run || ctx().prop.multiProcessorCount <= 0 ? 256 : ctx().prop.multiProcessorCount;
+    if (taps > 1 && (total + 127) / 128 * (K / (K % 128 == 0 ? 128 : K % 64 == 0 ? 64 : 32)) > cus) return false;      // (the fewest tiles there are)
+    const MarginPlanes planes{total, P, OW, PR, PC, rlo, rhi, clo, chi, -clo, 1};
+    const int64_t spans[2] = {planes.span(64), planes.span(128)};
     const int64_t KU = taps >= 6 ? 1 : taps >= 3 || C % 64 ? 2 : 4, stages = C / (16 * KU);      // (C is a multiple of 32)
     // Channels and positions of a workgroup by what a stage is estimated to take: its operands' way out of LDS and the next stage's way in, at 128
     // bytes a cycle, and 400 cycles for its barrier and what nothing hides.
@@ -273,7 +298,7 @@ static bool conv_strided(const mjt_tensor* x, const mjt_tensor* w, const mjt_ten
     double best = 1e300;
     for (int64_t wk = K % 64 ? 1 : 2; wk <= 4 && K % (32 * wk) == 0; wk *= 2)
         for (int64_t pt = 1; pt <= 2; pt++) {
-            const int64_t sp = span_of(64 * pt), stage_bytes = KU * (taps * wk * 1024 + nrp * 2 * sp * 32);
+            const int64_t sp = spans[pt - 1], stage_bytes = KU * (taps * wk * 1024 + nrp * 2 * sp * 32);
             if (2 * stage_bytes > 160 * 1024 || (sp * nrp * 2 * KU + 128 * wk - 1) / (128 * wk) > 6) continue;
             const int64_t wgs = (total + 64 * pt - 1) / (64 * pt) * (K / (32 * wk));
             const double t = std::ceil((double)wgs / cus) * ((double)(2 * wk * KU * taps * (1 + pt) * 1024 + stage_bytes) / 128 + 400.0);
@@ -1277,15 +1302,8 @@ static bool conv_dgrad_all_phases(const mjt_tensor* dy, const mjt_tensor* w, con
     const int64_t unit = OW % 2 == 0 ? 2 : 1, HB = (H + SH - 1) / SH, WB = (W + SW - 1) / SW, lpc = (-clo + unit - 1) / unit * unit;
     const int64_t PR = HB + rhi - rlo, PC = (lpc + WB + chi + unit - 1) / unit * unit, total = N * HB * WB, CT = (C + 63) / 64;
     if (N * PR * PC >= (int64_t(1) << 30)) return false;
-    auto pos = [&](int64_t f) { return (f / (HB * WB) * PR + f % (HB * WB) / WB - rlo) * PC + f % WB + lpc; };
-    auto span_of = [&](int64_t tile) {
-        int64_t most = 0;
-        for (int64_t t = 0; t < (total + tile - 1) / tile && t < HB * WB; t++)       // (tiles begin at the same places of an image again after that)
-            most = std::max(most, pos(t * tile + tile - 1) + rhi * PC + chi + 1 - (pos(t * tile) + rlo * PC + clo) / unit * unit);
-        return (most + unit - 1) / unit * unit;
-    };
     const int64_t cus = ctx().dry_run || ctx().prop.multiProcessorCount <= 0 ? 256 : ctx().prop.multiProcessorCount;
-    const int64_t PT = (total + 127) / 128 * CT >= cus ? 2 : 1, span = span_of(64 * PT), tiles = (total + 64 * PT - 1) / (64 * PT) * CT;
+    const int64_t PT = (total + 127) / 128 * CT >= cus ? 2 : 1, span = MarginPlanes{total, HB * WB, WB, PR, PC, rlo, rhi, clo, chi, lpc, unit}.span(64 * PT), tiles = (total + 64 * PT - 1) / (64 * PT) * CT;
     // A stage of 6 to 9 taps is 16 channels of dy, of fewer taps more, so that its MFMAs take longer than its barrier.  Where every workgroup has
     // a compute unit to itself nothing hides a stage's latency: twice as many (us, 16 / 32 channels: 1 x 512 x 7 x 7 -> 512 29.0 / 26.4, 8 x 256 x 28 x 28 -> 256 17.8 / 16.7).
     auto fits = [&](int64_t ku) { return 2 * ku * (taps * 2048 + span * 32) <= 160 * 1024 && span / unit * 2 * ku <= 4 * 256; };

@@ -6,6 +6,7 @@ import ctypes
 import json
 import os
 import re
+import time
 
 import numpy as np
 import pytest
@@ -580,6 +581,33 @@ def test_conv_builds_that_ran_out_of_registers_are_not_run(compile_only):
     x, dy = L.tensor(P, "bfloat16", (4, 64, 16, 16)), L.tensor(P, "bfloat16", (4, 64, 16, 16))
     assert lib.mjt_conv2d_meta_wgrad(ctypes.byref(x), ctypes.byref(dy), ctypes.byref(dw), ctypes.byref(p)) == 0
     assert L.last_kernel().startswith("mjt_conv_wgrad_mfma_bf16")
+
+
+def test_plans_of_strided_convolutions_are_not_worked_out_anew(compile_only):
+    """Host time of a call on large maps: no walk over their tiles after the first, whether the kernel of windows takes the call or not.  (It was
+    19 to 50 times that of a small map; the bound leaves room for a busy machine.)"""
+    L, lib = compile_only, compile_only.load()
+
+    def least(call, n, c, size, k, r):
+        o = (size - 1) // 2 + 1
+        x, w, y = L.tensor(P, "bfloat16", [n, c, size, size]), L.tensor(P, "bfloat16", [k, c, r, r]), L.tensor(P, "bfloat16", [n, k, o, o])
+        p = L.ConvParams(2, 2, r // 2, r // 2, 1, 1)
+        a = [ctypes.byref(q) for q in ((x, w, y, p) if call == "mjt_conv2d_meta" else (y, w, x, p))]
+        times = []
+        for _ in range(30):
+            t = time.perf_counter()
+            L.check(getattr(lib, call)(*a))
+            times.append(time.perf_counter() - t)
+        return min(times), L.last_kernel()
+    small, kern = least("mjt_conv2d_meta", 4, 64, 28, 64, 3)
+    assert "_strided_" in kern
+    for shape, strided in (((64, 32, 224, 64, 3), False), ((64, 64, 112, 64, 3), False), ((64, 256, 112, 512, 1), True)):
+        took, kern = least("mjt_conv2d_meta", *shape)
+        assert ("_strided_" in kern) == strided and took < 6 * small + 10e-6, (shape, kern, took, small)
+    small, kern = least("mjt_conv2d_meta_dgrad", 4, 64, 28, 64, 3)
+    assert "_dgrad_" in kern
+    took, kern = least("mjt_conv2d_meta_dgrad", 64, 32, 224, 64, 3)
+    assert "_dgrad_" in kern and took < 6 * small + 10e-6, (took, small)
 
 
 def test_scatter_and_gather_entries_pick_their_kernels(compile_only, monkeypatch):
