@@ -392,7 +392,10 @@ PyObject* binary(PyObject* x0, PyObject* y0, PyObject* op) {
     if (!xp) return nullptr;
     Ref yp(broadcast_plain(y.p, xs));
     if (!yp) return nullptr;
-    return binary(xp.p, yp.p, op);
+    if (Py_EnterRecursiveCall(" while shapes are matched")) return nullptr;
+    PyObject* z = binary(xp.p, yp.p, op);
+    Py_LeaveRecursiveCall();
+    return z;
 }
 PyObject* ternary(PyObject* c0, PyObject* x0, PyObject* y0) {
     Ref v[3] = {Ref(as_var(c0)), Ref(), Ref()};
@@ -420,7 +423,10 @@ PyObject* ternary(PyObject* c0, PyObject* x0, PyObject* y0) {
             const bool bx = larger(0, 1), by = larger(0, 2);
             if (bx && !spread(1, 0)) return nullptr;
             if (by && !spread(2, 0)) return nullptr;
-            return ternary(v[0].p, v[1].p, v[2].p);
+            if (Py_EnterRecursiveCall(" while shapes are matched")) return nullptr;      // (no elements and one do not meet)
+            PyObject* z = ternary(v[0].p, v[1].p, v[2].p);
+            Py_LeaveRecursiveCall();
+            return z;
         }
         if (!(s[0].n == s[1].n && s[0].n == s[2].n)) return PyErr_Format(PyExc_ValueError, "Number of dims should be the same.");
         Ref a(shape_list(s[1])), b(shape_list(s[2])), c(shape_list(s[0]));

@@ -6,6 +6,8 @@ import ctypes
 import json
 import os
 import re
+import subprocess
+import sys
 import time
 
 import numpy as np
@@ -1474,6 +1476,24 @@ def test_native_constructors_take_what_they_took():
     assert ref() is None                                       # no cycle keeps a graph alive
     with jt.flag_scope(compile_options={"k": 3}):
         assert (x + 1.0).compile_options == {"k": 3}
+
+
+def test_native_constructors_that_find_no_common_shape_raise():
+    """A select between no elements and one: an error, as in byte code, where the native one ran out of stack.  (In a process of its own.)"""
+    code = """if 1:
+        import numpy as np
+        import jittor_amd as jt
+        none, one = jt.array(np.ones([0], np.float32)), jt.array(np.ones([1], np.float32))
+        for a in ((none, one, none), (one, none, none), (none, none, one), (none > 0, one, one)):
+            try:
+                jt.ternary(*a)
+            except RecursionError:
+                print("refused")
+            else:
+                print("made")
+        """
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and r.stdout.split() == ["refused"] * 4, (r.returncode, r.stdout, r.stderr[-500:])
 
 
 def test_graph_keys_tell_graphs_apart():
