@@ -107,6 +107,24 @@ bool read_shape(PyObject* seq, Shape* s) {
     }
     return true;
 }
+// named axes: an integer or integers
+bool read_dims(PyObject* dims, Shape* s) {
+    if (PyIndex_Check(dims) && !PySequence_Check(dims)) {
+        s->n = 1;
+        s->e[0] = PyNumber_AsSsize_t(dims, PyExc_OverflowError);
+        return s->e[0] != -1 || !PyErr_Occurred();
+    }
+    Ref f(PySequence_Fast(dims, "dims are an integer or a sequence of integers"));
+    if (!f) return false;
+    const Py_ssize_t n = PySequence_Fast_GET_SIZE(f.p);
+    if (n > MOST) { PyErr_Format(PyExc_ValueError, "at most %lld dims are supported", g_max_dim); return false; }
+    s->n = (int)n;
+    for (Py_ssize_t i = 0; i < n; i++) {
+        s->e[i] = PyNumber_AsSsize_t(PySequence_Fast_GET_ITEM(f.p, i), PyExc_OverflowError);
+        if (s->e[i] == -1 && PyErr_Occurred()) return false;
+    }
+    return true;
+}
 bool var_shape(PyObject* v, Shape* s) {
     Ref a = attr(v, s_shape);
     return a && read_shape(a.p, s);
@@ -529,14 +547,7 @@ FUNCTION(broadcast) {
     if (!x) return nullptr;
     Shape shape, xs, dims;
     if (is_var(a[1]) ? !var_shape(a[1], &shape) : !read_shape(a[1], &shape)) return nullptr;
-    if (a[2]) {
-        if (PyIndex_Check(a[2]) && !PySequence_Check(a[2])) {
-            dims.n = 1;
-            dims.e[0] = PyNumber_AsSsize_t(a[2], PyExc_OverflowError);
-            if (dims.e[0] == -1 && PyErr_Occurred()) return nullptr;
-        } else if (!read_shape(a[2], &dims))
-            return nullptr;
-    }
+    if (a[2] && !read_dims(a[2], &dims)) return nullptr;
     if (!dims.n) return broadcast_plain(x.p, shape);
     if (!var_shape(x.p, &xs)) return nullptr;
     if (shape.n == 0) return PyErr_Format(PyExc_ValueError, "Number of shape should greater than 0.");
@@ -580,14 +591,7 @@ FUNCTION(reduce) {
     if (!is) return PyErr_Format(PyExc_ValueError, "reduce op %R is not associative; not supported on the device", a[1]);
     Shape xs, dims;
     if (!var_shape(x.p, &xs)) return nullptr;
-    if (a[2]) {
-        if (PyIndex_Check(a[2]) && !PySequence_Check(a[2])) {
-            dims.n = 1;
-            dims.e[0] = PyNumber_AsSsize_t(a[2], PyExc_OverflowError);
-            if (dims.e[0] == -1 && PyErr_Occurred()) return nullptr;
-        } else if (!read_shape(a[2], &dims))
-            return nullptr;
-    }
+    if (a[2] && !read_dims(a[2], &dims)) return nullptr;
     long long rmask = dims.n ? 0 : (1ll << xs.n) - 1;
     for (int i = 0; i < dims.n; i++) {
         const long long d = dims.e[i] < 0 ? dims.e[i] + xs.n : dims.e[i];

@@ -1496,6 +1496,15 @@ def test_native_constructors_that_find_no_common_shape_raise():
     assert r.returncode == 0 and r.stdout.split() == ["refused"] * 4, (r.returncode, r.stdout, r.stderr[-500:])
 
 
+@pytest.mark.parametrize("dims", ["0", ["0"], [1.0], 1.0, np.float32(1), None, [[1]], [None], np.array(1)])
+def test_named_axes_are_integers(dims):
+    x = jt.array(np.ones((2, 3), np.float32))
+    for call in (lambda: jt.reduce(x, "add", dims), lambda: jt.broadcast(x, [4, 2, 3], dims)):
+        with pytest.raises(TypeError):
+            call()
+    assert jt.reduce(x, "add", [np.int64(1), True]).shape == [2] and jt.reduce(x, "add", np.array([0, -1])).shape == [1] and jt.broadcast(x, [4, 2, 3], range(1)).shape == [4, 2, 3]
+
+
 def test_graph_keys_tell_graphs_apart():
     """What a key depends on: ops, attributes, shapes, types, wiring, which results are asked for, what is computed already, flags, the
     register; the same graph built again has the same key."""
