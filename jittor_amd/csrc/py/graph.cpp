@@ -107,6 +107,16 @@ bool read_shape(PyObject* seq, Shape* s) {
     }
     return true;
 }
+bool count_elements(const Shape& s, long long* num) {
+    *num = 1;
+    bool over = false;
+    for (int i = 0; i < s.n; i++) {
+        if (s.e[i] == 0) { *num = 0; return true; }
+        over = over || __builtin_mul_overflow(*num, s.e[i], num);
+    }
+    if (over) PyErr_SetString(PyExc_OverflowError, "a shape of 2^63 elements or more");
+    return !over;
+}
 // named axes: an integer or integers
 bool read_dims(PyObject* dims, Shape* s) {
     if (PyIndex_Check(dims) && !PySequence_Check(dims)) {
@@ -337,16 +347,13 @@ bool broadcast_rule(const Shape& x, const Shape& y, long long* bmask, long long*
         yi--;
     }
     if (zdim > g_max_dim) { PyErr_Format(PyExc_ValueError, "at most %lld dims are supported", g_max_dim); return false; }
-    *num = 1;
-    for (int i = 0; i < zdim; i++) {
+    for (int i = 0; i < zdim; i++)
         if (z->e[i] < 0) {
             Ref a(shape_list(*z));
             if (a) PyErr_Format(PyExc_ValueError, "Shape should greater than 0: %R", a.p);
             return false;
         }
-        *num *= z->e[i];
-    }
-    return true;
+    return count_elements(*z, num);
 }
 PyObject* broadcast_to(PyObject* x, const Shape& xs, const Shape& shape, long long bmask, long long kmask) {
     Shape z;
@@ -441,7 +448,7 @@ PyObject* ternary(PyObject* c0, PyObject* x0, PyObject* y0) {
             const bool bx = larger(0, 1), by = larger(0, 2);
             if (bx && !spread(1, 0)) return nullptr;
             if (by && !spread(2, 0)) return nullptr;
-            if (Py_EnterRecursiveCall(" while shapes are matched")) return nullptr;      // (no elements and one do not meet)
+            if (Py_EnterRecursiveCall(" while shapes are matched")) return nullptr;      // (no extents and one do not meet)
             PyObject* z = ternary(v[0].p, v[1].p, v[2].p);
             Py_LeaveRecursiveCall();
             return z;
@@ -481,7 +488,7 @@ PyObject* reduce_mask(PyObject* x, PyObject* op, long long rmask, long long kmas
     }
     Shape xs, z;
     if (!var_shape(x, &xs)) return nullptr;
-    long long num = 1;
+    long long num;
     for (int i = 0; i < xs.n; i++) {
         if (rmask >> i & 1) {
             if (kmask >> i & 1) z.e[z.n++] = 1;
@@ -492,7 +499,7 @@ PyObject* reduce_mask(PyObject* x, PyObject* op, long long rmask, long long kmas
         z.e[z.n++] = 1;
         kmask |= 1;
     }
-    for (int i = 0; i < z.n; i++) num *= z.e[i];
+    if (!count_elements(z, &num)) return nullptr;
     Ref dtype(typed_rule('r', op, have.p, s_reduce_dtype_infer));
     if (!dtype) return nullptr;
     PyObject* d;

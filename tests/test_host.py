@@ -1505,6 +1505,15 @@ def test_named_axes_are_integers(dims):
     assert jt.reduce(x, "add", [np.int64(1), True]).shape == [2] and jt.reduce(x, "add", np.array([0, -1])).shape == [1] and jt.broadcast(x, [4, 2, 3], range(1)).shape == [4, 2, 3]
 
 
+def test_element_counts_do_not_wrap_round():
+    """Extents whose product passes 2^63 are refused; with an extent of 0 there are no elements whatever the others are."""
+    x = jt.array(np.ones([1], np.float32))
+    for shape in ([2 ** 40, 2 ** 40], [2 ** 32, 2 ** 31], [2 ** 21] * 3):
+        with pytest.raises(OverflowError):
+            jt.broadcast(x, shape)
+    assert jt.broadcast(x, [2 ** 31, 2 ** 31]).num == 2 ** 62 and jt.broadcast(x, [2 ** 40, 2 ** 40, 0]).num == 0
+
+
 def test_graph_keys_tell_graphs_apart():
     """What a key depends on: ops, attributes, shapes, types, wiring, which results are asked for, what is computed already, flags, the
     register; the same graph built again has the same key."""
