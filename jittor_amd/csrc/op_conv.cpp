@@ -1457,8 +1457,8 @@ void conv_dgrad_impl(const mjt_tensor* dy, const mjt_tensor* w, const mjt_tensor
             for (int64_t b = 0; b < sw; b++) {
                 const Phase &qr = rows[a], &qc = cols[b];
                 mjt_tensor ty = view(part + (a * sw + b) * plane * dsz, dx->dtype, {N, C, Hs, Ws});
-                if (qr.taps == 0 || qc.taps == 0) {                 // no tap reaches these positions: zeros
-                    reindex(*dy, ty, {"0", "0", "0", "0"}, {"1"});
+                if (qr.taps == 0 || qc.taps == 0) {                 // no tap reaches these positions: zeros (the source, of the same type, is not read)
+                    reindex(ty, ty, {"0", "0", "0", "0"}, {"1"});
                     continue;
                 }
                 mjt_tensor tw = view((char*)wbuf + woff[(size_t)(a * sw + b)] * esz, w->dtype, {C, K, qr.taps, qc.taps});

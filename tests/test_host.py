@@ -530,13 +530,13 @@ def test_conv_input_gradient_entry_validates_and_picks_its_path(compile_only):
     lib = L.load()
     P = 0x100000
 
-    def call(xs, ws, params, dys=None, dtype="bfloat16"):
+    def call(xs, ws, params, dys=None, dtype="bfloat16", out=None):
         N, C, H, W = xs
         K, _, R, S = ws
         sh, sw, ph, pw, dh, dw = params
         oh, ow = (H + 2 * ph - dh * (R - 1) - 1) // sh + 1, (W + 2 * pw - dw * (S - 1) - 1) // sw + 1
         dy, w = L.tensor(P, dtype, dys or (N, K, oh, ow)), L.tensor(P, dtype, ws)
-        dx, p = L.tensor(P, dtype, xs), L.ConvParams(*params)
+        dx, p = L.tensor(P, out or dtype, xs), L.ConvParams(*params)
         return lib.mjt_conv2d_meta_dgrad(ctypes.byref(dy), ctypes.byref(w), ctypes.byref(dx), ctypes.byref(p))
 
     assert call((2, 64, 28, 28), (64, 64, 3, 3), (2, 2, 1, 1, 1, 1)) == 0
@@ -550,6 +550,7 @@ def test_conv_input_gradient_entry_validates_and_picks_its_path(compile_only):
     assert call((2, 64, 28, 28), (64, 32, 3, 3), (2, 2, 1, 1, 1, 1)) == -1         # weight channels != dx channels
     assert call((2, 64, 28, 28), (64, 64, 1, 1), (1, 1, 1, 1, 1, 1)) == -1         # padding no tap reaches
     assert b"padding" in lib.mjt_last_error()
+    assert call((2, 8, 12, 12), (6, 8, 1, 1), (3, 3, 0, 0, 1, 1), out="float32") == 0      # phases that no tap reaches, in the result's type
 
 
 def test_conv_builds_that_ran_out_of_registers_are_not_run(compile_only):
