@@ -1341,7 +1341,7 @@ static bool conv_dgrad_all_phases(const mjt_tensor* dy, const mjt_tensor* w, con
     if (mjt_reindex(w, &tw, 4, idx, 0.0, 2, over, 0, nullptr) != MJT_OK) MJT_FAIL(MJT_ERR_DEVICE, "conv dgrad: a rearrangement failed: " << mjt_last_error());
     std::vector<uint64_t> a{bits_of_ptr(wbuf), bits_of_ptr(dy->ptr), bits_of_ptr(dx->ptr), (uint64_t)N, (uint64_t)(numel(dy) * 2), (uint64_t)packed};
     jit_launch(k, (unsigned)((tiles + 7) / 8 * 8), 1, 256, 0, a);
-    set_last_kernel(((H % SH == 0 && W % SW == 0 && DH == 1 && DW == 1 ? "conv_dgrad_phases:" : "") + k->name).c_str());
+    set_last_kernel(k->name.c_str());
     return true;
 }
 

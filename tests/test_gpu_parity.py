@@ -906,8 +906,10 @@ def _dgrad_reference(dy, w, H, W, params):
     ((1, 4, 12, 12), (5, 4, 3, 2), (3, 2, 1, 1, 1, 1), "float32", "float32", False),     # a phase that starts past dy's first row
     ((1, 4, 13, 12), (5, 4, 3, 3), (2, 2, 1, 1, 1, 1), "float32", "float32", False),     # 13 rows: dy spread out with zeros
     ((1, 4, 12, 12), (5, 4, 3, 3), (2, 2, 2, 2, 2, 2), "float32", "float32", False),     # dilation: likewise
-    ((2, 64, 28, 28), (64, 64, 3, 3), (2, 2, 1, 1, 1, 1), "bfloat16", "bfloat16", True), # each phase on the MFMA kernel
-    ((2, 64, 28, 28), (128, 64, 3, 3), (2, 2, 1, 1, 1, 1), "float16", "float32", True),
+    ((2, 64, 28, 28), (64, 64, 3, 3), (2, 2, 1, 1, 1, 1), "bfloat16", "bfloat16", "all"), # all phases in one kernel
+    ((2, 64, 28, 28), (128, 64, 3, 3), (2, 2, 1, 1, 1, 1), "float16", "float32", "all"),
+    ((2, 64, 27, 30), (64, 64, 3, 3), (3, 3, 0, 0, 1, 1), "bfloat16", "bfloat16", True), # each phase on the MFMA kernel
+    ((2, 64, 28, 28), (64, 64, 3, 3), (3, 3, 1, 1, 1, 1), "float16", "float32", False),  # no whole phases: dy spread out with zeros
     ((2, 64, 28, 28), (64, 64, 3, 3), (1, 1, 1, 1, 1, 1), "bfloat16", "float32", False),
     ((2, 8, 12, 12), (6, 8, 1, 1), (3, 3, 0, 0, 1, 1), "bfloat16", "float32", True),      # stride 3, phases no tap reaches: zeros of the result's type
 ], ids=lambda c: "x%s_w%s_p%s_%s" % ("x".join(map(str, c[0])), "x".join(map(str, c[1])), "".join(map(str, c[2])), c[3]))
@@ -937,8 +939,8 @@ def test_conv_input_gradient_entry(gpu, case):
     p = L.ConvParams(*params)
     L.check(L.load().mjt_conv2d_meta_dgrad(ctypes.byref(td), ctypes.byref(tw), ctypes.byref(tx), ctypes.byref(p)))
     kern = L.last_kernel()
-    assert kern.startswith("conv_dgrad_phases:") == phased, kern
-    if dtype != "float32" and phased and sh == 2:
+    assert kern.startswith("conv_dgrad_phases:") == (phased is True) and ("_dgrad_c" in kern) == (phased == "all"), kern
+    if dtype != "float32" and C == 64:
         assert "mjt_conv_mfma" in kern, kern
     raw = L.d2h(dx.raw_ptr(), dx.shape, L.NP_STORAGE[out_dtype])
     got = (O.BF16(raw).to_f32() if out_dtype == "bfloat16" else raw).astype(np.float64)

@@ -525,8 +525,8 @@ def test_shutdown_forgets_kernels_and_rebinding_compiles_again(compile_only, mon
 
 
 def test_conv_input_gradient_entry_validates_and_picks_its_path(compile_only):
-    """mjt_conv2d_meta_dgrad without a device: argument checks, and which of its three forms a geometry takes (one
-    convolution per stride phase, transposed flipped weights for stride 1, dy spread out with zeros otherwise)."""
+    """mjt_conv2d_meta_dgrad without a device: argument checks, and which of its four forms a geometry takes (16 bits at strides 1 and 2 one kernel for
+    all stride phases, transposed flipped weights for stride 1, one convolution per stride phase, dy spread out with zeros otherwise)."""
     lib = L.load()
     P = 0x100000
 
@@ -540,11 +540,16 @@ def test_conv_input_gradient_entry_validates_and_picks_its_path(compile_only):
         return lib.mjt_conv2d_meta_dgrad(ctypes.byref(dy), ctypes.byref(w), ctypes.byref(dx), ctypes.byref(p))
 
     assert call((2, 64, 28, 28), (64, 64, 3, 3), (2, 2, 1, 1, 1, 1)) == 0
-    assert L.last_kernel().startswith("conv_dgrad_phases:mjt_conv_mfma_bf16"), L.last_kernel()
+    assert L.last_kernel().startswith("mjt_conv_mfma_bf16_dgrad_c"), L.last_kernel()
     assert call((2, 64, 28, 28), (64, 64, 3, 3), (1, 1, 1, 1, 1, 1)) == 0
-    assert L.last_kernel().startswith("mjt_conv_mfma_bf16"), L.last_kernel()
-    assert call((2, 64, 27, 28), (64, 64, 3, 3), (2, 2, 1, 1, 1, 1)) == 0          # 27 rows: no whole phases
-    assert not L.last_kernel().startswith("conv_dgrad_phases"), L.last_kernel()
+    assert L.last_kernel().startswith("mjt_conv_mfma_bf16") and "_dgrad_c" not in L.last_kernel(), L.last_kernel()
+    assert call((2, 64, 27, 28), (64, 64, 3, 3), (2, 2, 1, 1, 1, 1)) == 0          # 27 rows: phases of unequal height
+    assert L.last_kernel().startswith("mjt_conv_mfma_bf16_dgrad_c"), L.last_kernel()
+    for rows, dtype, params in ((28, "float32", (2, 2, 1, 1, 1, 1)), (27, "bfloat16", (3, 3, 0, 0, 1, 1))):
+        assert call((2, 64, rows, rows), (64, 64, 3, 3), params, dtype=dtype) == 0
+        assert L.last_kernel().startswith("conv_dgrad_phases:"), L.last_kernel()
+        assert call((2, 64, rows + 1, rows), (64, 64, 3, 3), params, dtype=dtype) == 0     # no whole phases
+        assert not L.last_kernel().startswith("conv_dgrad_phases:") and "_dgrad_c" not in L.last_kernel(), L.last_kernel()
     assert call((2, 64, 28, 28), (64, 64, 3, 3), (2, 2, 1, 1, 1, 1), dys=(2, 64, 15, 14)) == -1
     assert b"dy shape" in lib.mjt_last_error()
     assert call((2, 64, 28, 28), (64, 32, 3, 3), (2, 2, 1, 1, 1, 1)) == -1         # weight channels != dx channels
