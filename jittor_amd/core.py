@@ -17,7 +17,10 @@ import numpy as np
 
 from . import _lib
 _lib.load()              # says what to build where nothing is
-from . import _graph
+try:
+    from . import _graph
+except ImportError as e:
+    raise ImportError("jittor_amd._graph is not built for this interpreter (%s); run `make -C jittor_amd/csrc` or __graft_entry__.build() with it" % e) from e
 from . import dtypes as dt
 from ._lib import MjtError
 from .flags import flags as _flags
@@ -213,7 +216,8 @@ class Op:
         self._out_ref = _ref(v) if v is not None else None
 
     def sig(self):
-        """What the execution depends on besides the operands and the result (None: not known)."""
+        """What the execution depends on besides the operands and the result (None: not known).  The classes below are described by
+        csrc/py/graph.cpp; theirs is for classes derived from them."""
         return None
 
     def __repr__(self):

@@ -1484,6 +1484,16 @@ def test_native_constructors_take_what_they_took():
         assert (x + 1.0).compile_options == {"k": 3}
 
 
+def test_native_front_end_is_this_interpreters():
+    """The extension carries the interpreter's tag, so that another one does not load it; where it is missing the import says what to do."""
+    import sysconfig
+    from jittor_amd import _graph
+    assert os.path.basename(_graph.__file__) == "_graph" + sysconfig.get_config_var("EXT_SUFFIX") != "_graph.so"
+    code = "import sys; sys.modules['jittor_amd._graph'] = None; import jittor_amd"
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=120)
+    assert r.returncode != 0 and "make -C jittor_amd/csrc" in r.stderr, r.stderr[-300:]
+
+
 def test_native_constructors_that_find_no_common_shape_raise():
     """A select between no elements and one: an error, as in byte code, where the native one ran out of stack.  (In a process of its own.)"""
     code = """if 1:
