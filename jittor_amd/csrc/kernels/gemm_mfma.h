@@ -732,11 +732,7 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
 
     // D of a 32x32 tile: lane holds column lane % 32, rows 8 * (e / 4) + 4 * (lane / 32) + e % 4
 #if OUT == 2
-#if CONV == 2 || SLICED
     float* __restrict__ C = (float*)p.a[2] + (long long)outer * (long long)p.a[11];
-#else
-    float* __restrict__ C = (float*)p.a[2] + (long long)outer * (long long)p.a[11];
-#endif
 #else
     unsigned short* __restrict__ C = (unsigned short*)p.a[2] + (long long)outer * (long long)p.a[11];
 #endif
