@@ -9,8 +9,8 @@
 // 4-byte aligned place: neighbouring lanes read neighbouring dwords.  A wave keeps the weights of 32 channels in registers for all its
 // pixels.  Four waves; a workgroup walks `per` tiles of TR output rows and loads the next tile's rows of x behind the MFMAs of the current.
 //
-// us, product that gathers / this: 32 x 3 x 224 x 224 7x7 -> 64 float32 107.9 / 64.7, bfloat16 57.4 / 27.2; -> 16 float32
-// 102 / 37; 32 x 3 x 190 x 190 -> 51 float32 80.9 / 50.2; 32 x 3 x 125 x 125 -> 64 bfloat16 24.2 / 16.5.  What bounds it: float32 the MFMAs, 54 GFLOP of parts and padding (43 at
+// us, product that gathers / this: 32 x 3 x 224 x 224 7x7 -> 64 float32 105.8 / 58.7, bfloat16 57.4 / 27.2; -> 16 float32
+// 102 / 31; 32 x 3 x 190 x 190 -> 51 float32 78.3 / 45; 32 x 3 x 125 x 125 -> 64 bfloat16 24.2 / 16.5.  What bounds it: float32 the MFMAs, 54 GFLOP of parts and padding (43 at
 // the rate of a large bfloat16 product); bfloat16 the stores, 51 MB.
 //
 // float32: sums that are not finite are thrown away, and the wave's 32 x 32 results come from float32 MFMAs over memory.

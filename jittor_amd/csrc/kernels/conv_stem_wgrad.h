@@ -10,7 +10,7 @@
 // Four waves: KH halves of the channels times groups that take every (4 / KH)-th step of 16 pixels of a row; the groups' sums meet in LDS.
 // A workgroup walks `per` tiles and leaves a slice of the sum, which a reduce launch adds up.
 //
-// us with the fold, product that gathers / this: 32 x 3 x 224 x 224 7x7 -> 64 107.5 / 68.0, -> 16 103 / 41.4, 32 x 3 x 190 x 190 -> 51 100.8 / 70.8; relative error against 64 bits
+// us with the fold, product that gathers / this: 32 x 3 x 224 x 224 7x7 -> 64 107 / 59.6, -> 16 103.5 / 36, 32 x 3 x 190 x 190 -> 51 99.6 / 65.5; relative error against 64 bits
 // 2.4e-7 / 1.8e-7 at 1 x 3 x 224 x 224.  What bounds it: 49 GFLOP of parts and padding on the MFMAs (39 at the rate of a large bfloat16 product) beside 5 dwords of LDS
 // and 4 shifts for every operand of 8 pixels; the fold takes 10.
 //

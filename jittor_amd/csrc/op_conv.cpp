@@ -1012,7 +1012,7 @@ static bool conv_wgrad_stem(const mjt_tensor* x, const mjt_tensor* dy, const mjt
     const int64_t KH = K > 32 ? 2 : 1, kblocks = (K + 32 * KH - 1) / (32 * KH), groups = 4 / KH, unit = W % 4 == 0 ? 4 : W % 2 == 0 ? 2 : 1, steps = (OW + 15) / 16;
     const int64_t lp = (PW + 3) / 4 * 4, halfw = std::max((lp + W + 1) / 2, steps * 16 + (S - 1 - PW + lp) / 2 + 2), dwords = (halfw + 1) / 2 | 1;
     // Rows of a tile and tiles of a workgroup by what they are estimated to take, in us: terms as for the forward kernel, the slices' fold as for the
-    // gathering product, whose estimate `other` is.  us, gather / this: 32 x 3 x 224 x 224 7x7 -> 64 107.5 / 68.0, -> 16 103 / 41; 8 x 3 x 224 x 224 -> 64 38.0 / 31.4;
+    // gathering product, whose estimate `other` is.  us, gather / this: 32 x 3 x 224 x 224 7x7 -> 64 107 / 59.6, -> 16 103.5 / 36; 8 x 3 x 224 x 224 -> 64 35.8 / 25.3;
     // 32 x 3 x 125 x 125 -> 64 53.7 / 43.1; on the other side 1 x 3 x 224 x 224 -> 64 14.8 / 19.9, 4 x 3 x 96 x 96 -> 48 13.8 / 18.3.  (Up to 64 columns, such as 3 x 3 taps
     // of 3 channels, the waves have few MFMAs to a step: 16 x 3 x 128 x 128 3x3 -> 64 16.6 / 16.6, 64 x 3 x 32 x 32 -> 16 11.1 / 13.6.)
     int64_t TR = 0, per = 1;

@@ -185,9 +185,9 @@ void gemm_launch(int in_dtype, int out_dtype, const void* A, const void* B, void
         // on 128 x 128, a little more where an operand is transposed on the way; a round of workgroups adds a first load and a
         // store that nothing overlaps.  64 x 64 tiles stay with the float32 MFMAs: their stage is bound by the splitting (46 to
         // 56 us / 52 to 57 for a^T b 1024 x 1024 x 2048, 17.1 / 15.7 for a b^T 8192 x 64 x 1024).
-        // us, float32 MFMAs on the tiles chosen before / so: a b^T 2048 x 1024 x 1024 42 / 32.7 (128 x 64), a b 45.6 / 35.7, a^T b 1024 x
-        // 1024 x 2048 54 / 40.5 (128 x 128, 4 slices), a b^T 2048^3 127 / 94 (128 x 128), 4096^3 966 / 709, 512 x 512 x 8192 a^T b
-        // 55 / 39, 64 x 512 x 512 x 256 143 / 65.5, 12 x 384 x 384 x 384 35.5 / 17.2.
+        // us, float32 MFMAs on the tiles chosen before / so: a b^T 2048 x 1024 x 1024 38.4 / 31.5 (128 x 64), a b 40.0 / 31.7, a^T b 1024 x
+        // 1024 x 2048 50.3 / 36.7 (128 x 128, 4 slices), a b^T 2048^3 126 / 92.5 (128 x 128), 4096^3 966 / 703, 512 x 512 x 8192 a^T b
+        // 51 / 35.4, 64 x 512 x 512 x 256 143 / 65.5, 12 x 384 x 384 x 384 35.5 / 17.2.
         const bool parts = in_dtype == MJT_FLOAT32 && stages >= 4;
         for (int t = 0; t < (parts ? 4 : 1); t++) {
             const int mi = t == 1 || t == 3 ? 2 : 1, ni = t >= 2 ? 2 : 1;
