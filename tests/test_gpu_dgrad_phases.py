@@ -38,7 +38,7 @@ def _want(df, wf, hw, p):
     a = np.ascontiguousarray(df.transpose(0, 2, 3, 1)).reshape(-1, k)
     for i in range(r):
         for j in range(s):
-            g = (a @ wf[:, :, i, j]).reshape(n, oh, ow, c).transpose(0, 3, 1, 2)
+            g = (a @ np.ascontiguousarray(wf[:, :, i, j])).reshape(n, oh, ow, c).transpose(0, 3, 1, 2)
             dx[:, :, i * dh:i * dh + (oh - 1) * sh + 1:sh, j * dw:j * dw + (ow - 1) * sw + 1:sw] += g
     return dx[:, :, ph:ph + hw[0], pw:pw + hw[1]]
 

@@ -43,7 +43,7 @@ def _want(xf, wf, ys, p):
     for i in range(r):
         for j in range(s):
             patch = xp[:, :, i * dh:i * dh + (oh - 1) * sh + 1:sh, j * dw:j * dw + (ow - 1) * sw + 1:sw]
-            y += wf[:, :, i, j] @ np.ascontiguousarray(patch.transpose(1, 0, 2, 3)).reshape(xf.shape[1], -1)
+            y += np.ascontiguousarray(wf[:, :, i, j]) @ np.ascontiguousarray(patch.transpose(1, 0, 2, 3)).reshape(xf.shape[1], -1)
     return y.reshape(k, n, oh, ow).transpose(1, 0, 2, 3)
 
 
