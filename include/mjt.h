@@ -194,7 +194,9 @@ typedef enum {
     MJT_VAR_SCALAR = 3,
     /* mjt_fused_reindex_reduce only: a tensor of the scatter target's shape read through the scatter's own index
      * program (the reindex of the forward pass, recomputed instead of stored) */
-    MJT_VAR_GATHERED = 4
+    MJT_VAR_GATHERED = 4,
+    /* the entry points that end in `_then` only: what the product computes, of its dtype, never written to memory */
+    MJT_VAR_PRODUCT = 5
 } mjt_var_role;
 
 typedef struct {
@@ -401,6 +403,23 @@ int mjt_conv2d_meta_wgrad_grouped(const mjt_tensor* x, const mjt_tensor* dy, con
  * against an earlier build that relayed to a vendor library: it returns 1. */
 int mjt_matmul(const mjt_tensor* a, const mjt_tensor* b, const mjt_tensor* c, int trans_a, int trans_b);
 int mjt_matmul_available(void);
+
+/* ---- products with an element-wise group behind them --------------------
+ * A convolution, its input gradient or a matrix product whose result only one
+ * element-wise group reads (bias, relu, residual sum, the mask of a relu's
+ * gradient; the reference's fuser keeps such ops in one group with the product
+ * where no library op takes it, executor.cc:555): the group runs on the product's values where
+ * the kernel would store them.  `desc` is that group over the shape of the
+ * product, with one MJT_VAR_PRODUCT var of the result's dtype; y, dx and c give
+ * the result's shape and dtype, their pointers are not used.  The values are
+ * what the plain call would have written.  MJT_ERR_UNSUPPORTED, with nothing
+ * written, where the product's route has no kernel that takes a group: call the
+ * product and mjt_fused_elementwise instead. */
+int mjt_conv2d_meta_then(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, const mjt_conv_params* p, int groups,
+                         const mjt_fused_desc* desc);
+int mjt_conv2d_meta_dgrad_then(const mjt_tensor* dy, const mjt_tensor* w, const mjt_tensor* dx, const mjt_conv_params* p,
+                               const mjt_fused_desc* desc);
+int mjt_matmul_then(const mjt_tensor* a, const mjt_tensor* b, const mjt_tensor* c, int trans_a, int trans_b, const mjt_fused_desc* desc);
 
 /* ---- index-expression helper ------------------------------------------
  * Parses one index expression (the language of opt/expr.h:38-143 restricted

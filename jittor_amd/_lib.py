@@ -37,7 +37,7 @@ OP_CODE = {n: i for i, n in enumerate(OPS)}
 BINARY_OPS = OPS[:24]
 UNARY_OPS = OPS[24:53]
 
-VAR_INPUT, VAR_INTERMEDIATE, VAR_OUTPUT, VAR_SCALAR, VAR_GATHERED = 0, 1, 2, 3, 4
+VAR_INPUT, VAR_INTERMEDIATE, VAR_OUTPUT, VAR_SCALAR, VAR_GATHERED, VAR_PRODUCT = 0, 1, 2, 3, 4, 5
 FOP_UNARY, FOP_BINARY, FOP_TERNARY, FOP_BROADCAST, FOP_ROW_REDUCE, FOP_COLUMN_SUM = 0, 1, 2, 3, 4, 5
 ERR_INVALID, ERR_UNSUPPORTED, ERR_COMPILE, ERR_DEVICE, ERR_NOT_INIT = -1, -2, -3, -4, -5     # mjt_status
 
@@ -93,6 +93,7 @@ EXPORTS = ["mjt_init", "mjt_shutdown", "mjt_last_error", "mjt_get_device_info",
            "mjt_event_destroy", "mjt_reduce", "mjt_reduce_static", "mjt_reindex", "mjt_reindex_reduce",
            "mjt_fused_elementwise", "mjt_fused_reduce", "mjt_fused_rows", "mjt_conv2d_meta", "mjt_conv2d_meta_pack", "mjt_conv2d_meta_packed", "mjt_conv2d_meta_grouped", "mjt_conv2d_meta_dgrad", "mjt_conv2d_meta_dgrad_depthwise", "mjt_conv2d_meta_wgrad", "mjt_conv2d_meta_wgrad_grouped",
            "mjt_reindex_then_reduce", "mjt_fused_reindex_reduce", "mjt_matmul", "mjt_matmul_available",
+           "mjt_conv2d_meta_then", "mjt_conv2d_meta_dgrad_then", "mjt_matmul_then",
            "mjt_expr_affine", "mjt_where_count", "mjt_where",
            "mjt_record_begin", "mjt_record_end", "mjt_record_relocate", "mjt_record_launch", "mjt_record_free",
            "mjt_jit_stats", "mjt_last_kernel"]
@@ -158,6 +159,9 @@ def load():
                                                   ctypes.POINTER(ConvParams), ctypes.c_int]
     lib.mjt_matmul.argtypes = [ctypes.POINTER(Tensor), ctypes.POINTER(Tensor), ctypes.POINTER(Tensor), ctypes.c_int, ctypes.c_int]
     lib.mjt_matmul_available.argtypes = []
+    lib.mjt_conv2d_meta_then.argtypes = lib.mjt_conv2d_meta_grouped.argtypes + [ctypes.POINTER(FusedDesc)]
+    lib.mjt_conv2d_meta_dgrad_then.argtypes = lib.mjt_conv2d_meta_dgrad.argtypes + [ctypes.POINTER(FusedDesc)]
+    lib.mjt_matmul_then.argtypes = lib.mjt_matmul.argtypes + [ctypes.POINTER(FusedDesc)]
     lib.mjt_where_count.argtypes = [ctypes.POINTER(Tensor), ctypes.POINTER(ctypes.c_int64)]
     lib.mjt_where.argtypes = [ctypes.POINTER(Tensor), ctypes.c_int64, ctypes.POINTER(Tensor)]
     lib.mjt_expr_affine.argtypes = [ctypes.c_char_p, ctypes.POINTER(Tensor), ctypes.POINTER(Tensor),

@@ -38,6 +38,7 @@ __global__ __launch_bounds__(256) void mjt_fill_pattern_kernel(T* __restrict__ d
 // Fills n elements of elem_size bytes with the low bytes of `pattern`
 // (identity values of the scatter op).
 void launch_fill_pattern(void* dst, uint64_t pattern, int elem_size, size_t n) {
+    check_no_epilogue();
     Context& c = ctx();
     if (n == 0) return;
     refuse_recording("a fill");
@@ -56,6 +57,7 @@ void launch_fill_pattern(void* dst, uint64_t pattern, int elem_size, size_t n) {
 }
 
 void launch_copy(void* dst, const void* src, size_t bytes) {
+    check_no_epilogue();
     Context& c = ctx();
     refuse_recording("a copy");
     if (c.dry_run) return;
@@ -78,6 +80,7 @@ void launch_copy(void* dst, const void* src, size_t bytes) {
 }
 
 void launch_fill_u32(void* dst, uint32_t pattern, size_t n_words) {
+    check_no_epilogue();
     Context& c = ctx();
     refuse_recording("a fill");
     if (c.dry_run) return;

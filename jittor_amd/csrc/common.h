@@ -130,7 +130,54 @@ const char* embedded_source(const char* name);
 
 // shared by the fused element-wise group and the reduce with an element-wise prologue (op_fused.cpp)
 int64_t fused_validate(const mjt_fused_desc* d, std::vector<int>* inputs, bool outputs_need_data,
-                       bool allow_gathered = false);   // returns the element count
+                       int also = -1);   // returns the element count; `also`: one more role that a var may have
+// The code of an element-wise group over vectors of `vec` adjacent elements: defines of the fragments that kernels/fused.h and
+// kernels/epilogue.h paste, and the parameter words that they read, from word `first` of the kernel's block on.
+struct FusedCode {
+    struct Dim {
+        int64_t size;
+        std::vector<int> bcast;   // per input tensor: 1 when broadcast along this axis
+    };
+    FusedCode(const mjt_fused_desc* d, const std::vector<int>& inputs, const std::vector<Dim>& dims, int vec, bool use64, int first);
+    std::string key() const;      // all that text() depends on
+    std::string text(const std::string& prefix, const char* load, const char* store) const;
+    std::vector<uint64_t> words;
+
+private:
+    const mjt_fused_desc* d;
+    const std::vector<int>& inputs;
+    const std::vector<Dim>& dims;
+    int vec;
+    bool use64, need_decode = false;
+    std::vector<int> p_dim, p_var;
+    std::vector<std::vector<int>> p_stride;
+};
+std::vector<FusedCode::Dim> fused_dims(const mjt_fused_desc* d, const std::vector<int>& inputs);
+// whether every access of `vec` elements is one of whole, aligned vectors
+bool fused_aligned(const mjt_fused_desc* d, const std::vector<int>& inputs, const std::vector<FusedCode::Dim>& dims, int vec);
+
+// ---- an element-wise group behind a product (op_epilogue.cpp, kernels/epilogue.h) ----
+// While an entry point with a group runs, the kernel that would write the product hands its values to the group instead.  A route
+// asks for the group's code where it builds that kernel and says so (epilogue_taken) where it launches it; any other launch is
+// refused, so that a route which knows nothing of groups ends the call with MJT_ERR_UNSUPPORTED and nothing written.
+struct EpilogueCode {
+    bool on = false;
+    int ops = 0;
+    std::string key, defs;                 // behind the kernel's own key; in front of its source
+    std::vector<uint64_t> words;           // behind the kernel's own parameter words
+    std::string suffix() const { return on ? "_then" + std::to_string(ops) : std::string(); }
+};
+// vec: adjacent elements that the kernel hands over at a time; first: its own parameter words; covered: elements of its result, which
+// lie in the order of the whole result.  Off where no group waits or the group cannot take them so.
+EpilogueCode epilogue_code(int vec, int first, int dtype, int64_t covered);
+void epilogue_taken(const EpilogueCode& code);
+bool epilogue_waits();
+void check_no_epilogue();                  // called by every launch
+// launches that prepare operands (rearranged weights, padded rows)
+struct Preparing {
+    Preparing();
+    ~Preparing();
+};
 std::string fused_emit_ops(const mjt_fused_desc* d, bool store_outputs);
 std::string fused_op_expr(const mjt_fused_desc* d, const mjt_fused_op& o);
 

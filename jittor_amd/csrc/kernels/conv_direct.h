@@ -7,7 +7,11 @@
 // Supplied by the host: TIN (element type of x and w), TOUT, G_, IDX (int when every element index fits 31 bits,
 // else long long: 64-bit index arithmetic costs a third of this kernel's time) and the geometry (C_ = channels per group).
 
-struct Params { void* a[4]; };   // 8-byte words; typed as pointers so loads/stores use the global address space   // x, w, y, number of outputs
+#ifndef EPI
+#define EPI 0
+#define EPI_WORDS 0
+#endif
+struct Params { void* a[4 + EPI_WORDS]; };   // 8-byte words; typed as pointers so loads/stores use the global address space   // x, w, y, number of outputs
 
 extern "C" __global__ __launch_bounds__(256) void ENTRY(Params p) {
     const TIN* __restrict__ xp = (const TIN*)p.a[0];
@@ -31,5 +35,11 @@ extern "C" __global__ __launch_bounds__(256) void ENTRY(Params p) {
                 const float wv = (float)wp[(((IDX)ko * C_ + c) * R_ + kh) * S_ + kw];
                 acc = acc + xv * wv;
             }
+#if EPI
+    mjt_epi_in<1> read;
+    mjt_epi_load(p, read, (MJT_EPI_INDEX)o);
+    mjt_epi_finish(p, read, (MJT_EPI_INDEX)o, {acc});
+#else
     yp[o] = (TOUT)acc;
+#endif
 }

@@ -71,7 +71,11 @@ typedef float mjt_f32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned mjt_u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned mjt_u32x4v __attribute__((ext_vector_type(4)));
 
-struct Params { void* a[4]; };   // x, packed w, y, number of images (typed as pointers: global address space)
+#ifndef EPI
+#define EPI 0
+#define EPI_WORDS 0
+#endif
+struct Params { void* a[4 + EPI_WORDS]; };   // x, packed w, y, number of images (typed as pointers: global address space)
 
 // ABL (0 in production): timing-only ablations, results are wrong with any bit set.  1 no output stores, 2 no input
 // rows (neither loaded nor written to LDS), 4 (only together with 1 and 2) no weight slabs copied, no fragment reads
@@ -582,6 +586,22 @@ extern "C" __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu
         int lane_e = lane;
         asm volatile("" : "+v"(lane_e));
         const int l16_e = lane_e & 15, lg_e = lane_e >> 4;
+#if EPI
+        // the group behind the convolution on V pixels of MT channels: what it reads of all of them is asked for first
+        auto group_behind = [&](auto vc, auto&& place, int t, int i) {
+            constexpr int V = decltype(vc)::v;
+            mjt_epi_in<V> read[MT];
+#pragma unroll
+            for (int m = 0; m < MT; m++) mjt_epi_load(p, read[m], (MJT_EPI_INDEX)place(m));
+#pragma unroll
+            for (int m = 0; m < MT; m++) {
+                float v[V];
+#pragma unroll
+                for (int k = 0; k < V; k++) v[k] = acc[m][t][i + k];
+                mjt_epi_finish(p, read[m], (MJT_EPI_INDEX)place(m), v);
+            }
+        };
+#endif
 #pragma unroll
         for (int t = 0; t < NT_; t++) {
 #if OW_ % 4 == 0
@@ -593,6 +613,9 @@ extern "C" __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu
             const int r = q0 / OW_, col = q0 - r * OW_;
             const int orow = r0 + wpx * TRW_ + r;
             if (q0 < TRW_ * OW_ && orow < row_lim && !(ABL & 1)) {
+#if EPI
+                group_behind(mjt_ic<4>(), [&](int m) { return (((size_t)n * YK_ + y_k0 + ko_base + m * 16 + l16_e) * OH_ + orow) * OW_ + col; }, t, 0);
+#else
 #pragma unroll
                 for (int m = 0; m < MT; m++) {
                     const mjt_f32x4 v = acc[m][t];
@@ -606,6 +629,7 @@ extern "C" __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu
                     *(mjt_f32x4*)((float*)p.a[2] + o) = v;
 #endif
                 }
+#endif
             }
 #elif OW_ % 2 == 0
             // an even width: pairs of pixels never straddle an output row (widths of 14: half the stores of single pixels)
@@ -615,6 +639,9 @@ extern "C" __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu
                 const int r = q / OW_, col = q - r * OW_;
                 const int orow = r0 + wpx * TRW_ + r;
                 if (q < TRW_ * OW_ && orow < row_lim && !(ABL & 1)) {
+#if EPI
+                    group_behind(mjt_ic<2>(), [&](int m) { return (((size_t)n * YK_ + y_k0 + ko_base + m * 16 + l16_e) * OH_ + orow) * OW_ + col; }, t, i);
+#else
 #pragma unroll
                     for (int m = 0; m < MT; m++) {
                         const size_t o = (((size_t)n * YK_ + y_k0 + ko_base + m * 16 + l16_e) * OH_ + orow) * OW_ + col;
@@ -627,6 +654,7 @@ extern "C" __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu
                         *(mjt_f32x2*)((float*)p.a[2] + o) = pr;
 #endif
                     }
+#endif
                 }
             }
 #else
@@ -636,6 +664,9 @@ extern "C" __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu
                 const int r = q / OW_, col = q - r * OW_;
                 const int orow = r0 + wpx * TRW_ + r;
                 if (q < TRW_ * OW_ && orow < row_lim && !(ABL & 1)) {
+#if EPI
+                    group_behind(mjt_ic<1>(), [&](int m) { return (((size_t)n * YK_ + y_k0 + ko_base + m * 16 + l16_e) * OH_ + orow) * OW_ + col; }, t, i);
+#else
 #pragma unroll
                     for (int m = 0; m < MT; m++) {
                         const size_t o = (((size_t)n * YK_ + y_k0 + ko_base + m * 16 + l16_e) * OH_ + orow) * OW_ + col;
@@ -645,6 +676,7 @@ extern "C" __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu
                         ((float*)p.a[2])[o] = acc[m][t][i];
 #endif
                     }
+#endif
                 }
             }
 #endif

@@ -38,7 +38,11 @@ template <int I, int N, class F> __device__ __forceinline__ void mjt_static_for(
     }
 }
 
-struct Params { void* a[6]; };       // x, w, y, images, tiles a workgroup, bytes of x
+#ifndef EPI
+#define EPI 0
+#define EPI_WORDS 0
+#endif
+struct Params { void* a[6 + EPI_WORDS]; };       // x, w, y, images, tiles a workgroup, bytes of x
 
 constexpr int ESZ = IN == 2 ? 4 : 2, PARTS = IN == 2 ? 3 : 1;
 constexpr int CRS = C_ * R_ * S_, ROWS = C_ * R_, STEPS = (ROWS + 1) / 2;
@@ -229,6 +233,20 @@ extern "C" __global__ __launch_bounds__(256, 2) void ENTRY(Params p) {
             // D: lane holds column (pixel) lane % 32, rows (k) 8 * (e / 4) + 4 * (lane / 32) + e % 4
             if (pt * 32 + l32 < NPX && oh < OH_) {
                 const long long base = ((long long)(n * K_ + k0 + 4 * half) * OH_ + oh) * OW_ + col;
+#if EPI
+                mjt_static_for<0, 4>([&](auto qc) {    // (what the group reads, four places at a time: sixteen would push the weights out)
+                    constexpr int q = decltype(qc)::v;
+                    mjt_epi_in<1> read[4];
+                    mjt_static_for<0, 4>([&](auto ec) {
+                        constexpr int e = decltype(ec)::v, k = 8 * q + e;
+                        mjt_epi_load(p, read[e], (MJT_EPI_INDEX)(K_ % 32 == 0 || k0 + 4 * half + k < K_ ? base + k * (OH_ * OW_) : 0));
+                    });
+                    mjt_static_for<0, 4>([&](auto ec) {
+                        constexpr int e = decltype(ec)::v, k = 8 * q + e;
+                        if (K_ % 32 == 0 || k0 + 4 * half + k < K_) mjt_epi_finish(p, read[e], (MJT_EPI_INDEX)(base + k * (OH_ * OW_)), {acc[4 * q + e]});
+                    });
+                });
+#else
                 mjt_static_for<0, 16>([&](auto ec) {
                     constexpr int e = decltype(ec)::v, k = 8 * (e / 4) + e % 4;
                     if (K_ % 32 == 0 || k0 + 4 * half + k < K_) {
@@ -241,6 +259,7 @@ extern "C" __global__ __launch_bounds__(256, 2) void ENTRY(Params p) {
 #endif
                     }
                 });
+#endif
             }
         }
     }

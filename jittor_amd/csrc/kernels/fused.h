@@ -5,12 +5,14 @@
 // registers as the reference's remove_intermediate pass arranges,
 // opt/pass/remove_intermediate_pass.cc:26-47).
 //
-// The host generates four code fragments and the constants below:
-//   VEC, UNROLL, BLOCK, index_t, NPARAM, MJT_LD / MJT_ST (plain or non-temporal access)
+// The host generates code fragments and the constants below:
+//   MJT_FUSED_VEC, MJT_FUSED_INDEX, UNROLL, BLOCK, NPARAM
 //   MJT_FUSED_DECODE   coordinates c0..c{n-1} of element e (only when a
 //                      broadcast input needs them)
-//   MJT_FUSED_LOADS    one vector (or scalar, when broadcast along the
-//                      innermost axis) load per input tensor
+//   MJT_FUSED_DECL     a vector (or scalar, when broadcast along the
+//                      innermost axis) per input tensor
+//   MJT_FUSED_LOADS    the loads of these, members of `t`
+//   MJT_FUSED_OUTS     a vector per output tensor
 //   MJT_FUSED_BODY     the op chain for lane element k, in topological order
 //   MJT_FUSED_STORES   one vector store per output tensor
 //
@@ -18,6 +20,9 @@
 // tensors move as 16-byte vectors; a workgroup covers UNROLL contiguous
 // BLOCK*VEC-element runs, which keeps UNROLL independent loads in flight per
 // lane.
+
+#define VEC MJT_FUSED_VEC
+typedef MJT_FUSED_INDEX index_t;
 
 struct Params { void* a[NPARAM]; };   // 8-byte words; typed as pointers so loads/stores use the global address space
 
@@ -30,7 +35,9 @@ extern "C" __global__ __launch_bounds__(BLOCK) void ENTRY(Params p) {
         if (j < nvec) {
             const index_t e = j * VEC;
             MJT_FUSED_DECODE
+            struct { MJT_FUSED_DECL } t;
             MJT_FUSED_LOADS
+            MJT_FUSED_OUTS
 #pragma unroll
             for (int k = 0; k < VEC; k++) {
                 MJT_FUSED_BODY

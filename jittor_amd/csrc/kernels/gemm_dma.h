@@ -7,7 +7,7 @@
 // [K][M]); B' is b, or b transposed when B_KCONT == 1 (memory [N][K]).  bfloat16 / float16 operands with exact
 // products and float32 accumulation.
 //
-// Supplied by the host: IN (0 bfloat16, 1 float16), OUT (0 bfloat16 by truncation, 1 float16 rounded to
+// Supplied by the host: VS (adjacent results a lane stores: 4, 2 or 1), IN (0 bfloat16, 1 float16), OUT (0 bfloat16 by truncation, 1 float16 rounded to
 // nearest even, 2 float32), A_KCONT, B_KCONT (the operand's memory has k innermost).  K is a multiple of 64, leading
 // dimensions are multiples of 16 bytes and the operand pointers 16-byte aligned (the host sends everything else to the
 // general kernel).
@@ -101,7 +101,11 @@ __device__ __forceinline__ void mjt_mfma2(mjt_f32x16& c, const mjt_u32x2& alo, c
 __device__ __forceinline__ void mjt_keep2(const mjt_u32x2& x) { asm volatile("" : : "v"(x)); }     // x is in its registers up to here
 __device__ __forceinline__ void mjt_pin(mjt_f32x16& x) { asm volatile("" : "+a"(x)); }            // what reads x later comes after this point
 
-struct Params { void* a[12]; };
+#ifndef EPI
+#define EPI 0
+#define EPI_WORDS 0
+#endif
+struct Params { void* a[12 + EPI_WORDS]; };
 
 #ifndef WPE
 #define WPE 1                   // workgroups (of one wave per SIMD) a compute unit is meant to hold
@@ -311,19 +315,78 @@ extern "C" __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu
         });
     }
     // The last MFMAs need time to read their operands and write their results; tie the registers to a point behind that.
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15\n\ts_nop 15" : : : "memory");
+    // (behind the barrier no copy into LDS is under way any more and nobody reads an operand there.)
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15\n\ts_nop 15\n\ts_barrier" : : : "memory");
     mjt_static_for<0, NSETS * FR>([&](auto ic) {
         constexpr int st = decltype(ic)::v / FR, f = decltype(ic)::v % FR;
         mjt_keep2(falo[st][f]); mjt_keep2(fahi[st][f]); mjt_keep2(fblo[st][f]); mjt_keep2(fbhi[st][f]);
     });
     mjt_static_for<0, NM>([&](auto ic) { mjt_pin(acc[decltype(ic)::v / FR][decltype(ic)::v % FR]); });
 
-    // D of a 32x32 tile: lane holds column lane % 32, rows 8 * (e / 4) + 4 * (lane / 32) + e % 4
-#if OUT == 2
-    float* __restrict__ C = (float*)p.a[2] + (long long)blockIdx.y * (long long)p.a[11];
+    // D of a 32x32 tile: lane holds column lane % 32, rows 8 * (e / 4) + 4 * (lane / 32) + e % 4.
+    const long long c0 = (long long)blockIdx.y * (long long)p.a[11];
+#if EPI || VS == 4
+    // A wave's results go through LDS, 32 rows at a time, so that a lane has VS adjacent columns and an instruction whole 128-byte
+    // pieces of rows: as they lie in the accumulators an instruction stores 64 bytes of two rows, and a group behind the product would
+    // read and write by the element.  (The pitch puts the two rows that one instruction writes into different halves of the banks.)
+    // Without a group only for vectors of four: 64 x 256 x 14 x 14 -> 1024 21.7 -> 20.3 us, 8192 x 512 x 2048 28.1 -> 27.1; rows of 3002 or
+    // 3001 (3000 x 1024) 32.4 -> 33.5 and 37.1.
+    constexpr int PITCH = WT + 8, LPR = WT / VS, IT = 32 * LPR / 64, BATCH = IT < 8 ? IT : 8;      // lanes a row; vectors a lane has of 32 rows
+    static_assert(4 * 32 * PITCH * 4 <= NBUF * STAGE_BYTES, "a wave's 32 rows in LDS");
+    float* const mine = (float*)lds + wave * (32 * PITCH);
+    // item of a lane: VS columns from column `lcol` of row `lrow` of the 32
+    auto lrow = [&](int item) { return (item * 64 + lane) / LPR; };
+    auto lcol = [&](int item) { return (item * 64 + lane) % LPR * VS; };
+#pragma unroll
+    for (int i = 0; i < FR; i++) {
+#pragma unroll
+        for (int j = 0; j < FR; j++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) mine[(8 * (e / 4) + 4 * (lane >> 5) + (e & 3)) * PITCH + j * 32 + (lane & 31)] = acc[i][j][e];
+#pragma unroll
+        for (int b = 0; b < IT; b += BATCH) {
+            long long at[BATCH];
+            bool in[BATCH];
+#pragma unroll
+            for (int q = 0; q < BATCH; q++) {
+                const int row = m0 + wm * WT + i * 32 + lrow(b + q), col = n0 + wn * WT + lcol(b + q);
+#if IMG
+                const int img = col / (PIECES * 8), px = col - img * (PIECES * 8);      // (VS divides a plane: the vector lies inside it or behind it)
+                in[q] = row < M && col < N && px < IMG;
+                at[q] = in[q] ? c0 + (long long)img * ldc + (long long)row * IMG + px : 0;
 #else
-    unsigned short* __restrict__ C = (unsigned short*)p.a[2] + (long long)blockIdx.y * (long long)p.a[11];
+                in[q] = row < M && col < N;                                          // (VS divides N)
+                at[q] = in[q] ? c0 + (long long)row * ldc + col : 0;
 #endif
+            }
+#if EPI
+            mjt_epi_in<VS> read[BATCH];
+#pragma unroll
+            for (int q = 0; q < BATCH; q++) mjt_epi_load(p, read[q], (MJT_EPI_INDEX)at[q]);
+#endif
+#pragma unroll
+            for (int q = 0; q < BATCH; q++) {
+                struct alignas(VS * 4) { float v[VS]; } r = *(decltype(r)*)&mine[lrow(b + q) * PITCH + lcol(b + q)];
+                if (!in[q]) continue;
+#if EPI
+                mjt_epi_finish(p, read[q], (MJT_EPI_INDEX)at[q], r.v);
+#elif OUT == 2
+                *(decltype(r)*)((float*)p.a[2] + at[q]) = r;
+#else
+                struct alignas(VS * 2) { unsigned short v[VS]; } o;
+#pragma unroll
+                for (int k = 0; k < VS; k++)
+#if OUT == 0
+                    o.v[k] = (unsigned short)(__float_as_uint(r.v[k]) >> 16);     // truncation (type/fp16_compute.h:238-241)
+#else
+                    o.v[k] = __builtin_bit_cast(unsigned short, (_Float16)r.v[k]);                // nearest even (type/fp16_compute.h:147-198)
+#endif
+                *(decltype(o)*)((unsigned short*)p.a[2] + at[q]) = o;
+#endif
+            }
+        }
+    }
+#else
 #pragma unroll
     for (int i = 0; i < FR; i++)
 #pragma unroll
@@ -332,10 +395,10 @@ extern "C" __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu
 #if IMG
             const int img = col / (PIECES * 8), px = col - img * (PIECES * 8);
             const bool col_in = col < N && px < IMG;
-            const long long col_at = (long long)img * ldc + px;
+            const long long col_at = c0 + (long long)img * ldc + px;
 #else
             const bool col_in = col < N;
-            const long long col_at = col;
+            const long long col_at = c0 + col;
 #endif
 #pragma unroll
             for (int e = 0; e < 16; e++) {
@@ -344,14 +407,14 @@ extern "C" __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu
                     const float v = acc[i][j][e];
                     const long long at = (long long)row * (IMG ? IMG : ldc) + col_at;
 #if OUT == 2
-                    C[at] = v;
+                    ((float*)p.a[2])[at] = v;
 #elif OUT == 0
-                    C[at] = (unsigned short)(__float_as_uint(v) >> 16);     // truncation (type/fp16_compute.h:238-241)
+                    ((unsigned short*)p.a[2])[at] = (unsigned short)(__float_as_uint(v) >> 16);     // truncation (type/fp16_compute.h:238-241)
 #else
-                    const _Float16 h = (_Float16)v;                                                  // nearest even (type/fp16_compute.h:147-198)
-                    C[at] = __builtin_bit_cast(unsigned short, h);
+                    ((unsigned short*)p.a[2])[at] = __builtin_bit_cast(unsigned short, (_Float16)v);     // nearest even (type/fp16_compute.h:147-198)
 #endif
                 }
             }
         }
+#endif
 }

@@ -121,7 +121,11 @@ typedef _Float16 mjt_h8 __attribute__((ext_vector_type(8)));
 #endif
 
 template <int V> struct mjt_ic { static constexpr int v = V; };
-struct Params { void* a[12]; };
+#ifndef EPI
+#define EPI 0
+#define EPI_WORDS 0
+#endif
+struct Params { void* a[12 + EPI_WORDS]; };
 // a[0] A  a[1] B  a[2] C  a[3] M (upper half: matrices of the batch)  a[4] N  a[5] K  a[6] lda  a[7] ldb  a[8] ldc (elements)
 // a[9] batch stride of A  a[10] of B  a[11] of C (elements)
 
@@ -731,11 +735,7 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
 #endif
 
     // D of a 32x32 tile: lane holds column lane % 32, rows 8 * (e / 4) + 4 * (lane / 32) + e % 4
-#if OUT == 2
-    float* __restrict__ C = (float*)p.a[2] + (long long)outer * (long long)p.a[11];
-#else
-    unsigned short* __restrict__ C = (unsigned short*)p.a[2] + (long long)outer * (long long)p.a[11];
-#endif
+    const long long c0 = (long long)outer * (long long)p.a[11];
 #pragma unroll
     for (int i = 0; i < FI; i++)
 #pragma unroll
@@ -744,23 +744,35 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
 #if CONV == 1
             const int img = col / (OH_ * OW_), px = col - img * (OH_ * OW_);      // y[img][row][px]
 #endif
+            auto row_of = [&](int e) { return m0 + wm * 32 * FI + i * 32 + 8 * (e / 4) + 4 * (lane >> 5) + (e & 3); };
+            auto place_of = [&](int row) {
+#if CONV == 1
+                return ((long long)img * K_ + row) * (OH_ * OW_) + px;
+#else
+                return c0 + (long long)row * ldc + col;
+#endif
+            };
+#if EPI
+            // what the group reads of all sixteen places is asked for before the first is finished
+            mjt_epi_in<1> read[16];
+#pragma unroll
+            for (int e = 0; e < 16; e++) mjt_epi_load(p, read[e], (MJT_EPI_INDEX)(row_of(e) < M && col < N ? place_of(row_of(e)) : 0));
+#endif
 #pragma unroll
             for (int e = 0; e < 16; e++) {
-                const int row = m0 + wm * 32 * FI + i * 32 + 8 * (e / 4) + 4 * (lane >> 5) + (e & 3);
+                const int row = row_of(e);
                 if (row < M && col < N) {
                     const float v = acc[i][j][e];
-#if CONV == 1
-                    const long long at = ((long long)img * K_ + row) * (OH_ * OW_) + px;
-#else
-                    const long long at = (long long)row * ldc + col;
-#endif
-#if OUT == 2
-                    C[at] = v;
+                    const long long at = place_of(row);
+#if EPI
+                    mjt_epi_finish(p, read[e], (MJT_EPI_INDEX)at, {v});
+#elif OUT == 2
+                    ((float*)p.a[2])[at] = v;
 #elif OUT == 0
-                    C[at] = (unsigned short)(__float_as_uint(v) >> 16);     // truncation (type/fp16_compute.h:238-241)
+                    ((unsigned short*)p.a[2])[at] = (unsigned short)(__float_as_uint(v) >> 16);     // truncation (type/fp16_compute.h:238-241)
 #else
                     const _Float16 h = (_Float16)v;                        // nearest even (type/fp16_compute.h:147-198)
-                    C[at] = __builtin_bit_cast(unsigned short, h);
+                    ((unsigned short*)p.a[2])[at] = __builtin_bit_cast(unsigned short, h);
 #endif
                 }
             }

@@ -206,23 +206,29 @@ static bool conv_stem(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor
     if (TR == 0) return false;
     const int64_t tiles = N * ((OH + TR - 1) / TR), grid = (tiles + per - 1) / per * kblocks;
     if (tiles >= (1 << 28) || grid >= (1 << 28)) return false;
+    const EpilogueCode ep = epilogue_code(1, 6, y->dtype, numel(y));
     std::ostringstream key;
-    key << "stem|" << C << "|" << H << "|" << W << "|" << K << "|" << R << "|" << S << "|" << OH << "|" << OW << "|" << SH << "|" << PH << "|" << PW << "|" << DH << "|" << in << narrow << "|" << TR;
+    key << "stem|" << C << "|" << H << "|" << W << "|" << K << "|" << R << "|" << S << "|" << OH << "|" << OW << "|" << SH << "|" << PH << "|" << PW << "|" << DH << "|" << in << narrow << "|" << TR << ep.key;
     JitKernel* k = cached(key.str());
     if (!k) {
         std::ostringstream name;
         name << "mjt_conv_igemm_" << mjt_dtype_name(x->dtype) << (y->dtype != x->dtype ? "_of32" : "") << "_stem_c" << C << "_k" << K << "_r" << R << "x" << S << "_s" << SH << "x2_p" << PH << "x" << PW << "_d"
-             << DH << "x1_rows" << TR << "_" << H << "x" << W;
+             << DH << "x1_rows" << TR << "_" << H << "x" << W << ep.suffix();
         std::ostringstream src;
-        src << "#define ENTRY " << name.str() << "\n#define IN " << in << "\n#define Y_16 " << narrow << "\n#define TR " << TR << "\n#define C_ " << C << "\n#define H_ " << H << "\n#define W_ " << W
+        src << ep.defs << "#define ENTRY " << name.str() << "\n#define IN " << in << "\n#define Y_16 " << narrow << "\n#define TR " << TR << "\n#define C_ " << C << "\n#define H_ " << H << "\n#define W_ " << W
             << "\n#define K_ " << K << "\n#define R_ " << R << "\n#define S_ " << S << "\n#define OH_ " << OH << "\n#define OW_ " << OW << "\n#define SH " << SH << "\n#define PH " << PH
             << "\n#define PW " << PW << "\n#define DH " << DH << "\n";
         src << embedded_source("split.h") << "\n" << embedded_source("conv_stem.h") << "\n";
         k = jit_get(src.str(), name.str());
         remember(key.str(), k);
     }
-    if (k->spilled != 0) return false;
+    if (k->spilled != 0) {
+        if (ep.on) check_no_epilogue();                     // (the convolution without the group is the better one)
+        return false;
+    }
     std::vector<uint64_t> a{bits_of_ptr(x->ptr), bits_of_ptr(w->ptr), bits_of_ptr(y->ptr), (uint64_t)N, (uint64_t)per, (uint64_t)(numel(x) * esz)};
+    a.insert(a.end(), ep.words.begin(), ep.words.end());
+    epilogue_taken(ep);
     jit_launch(k, (unsigned)grid, 1, 256, 0, a);
     set_last_kernel(k->name.c_str());
     return true;
@@ -541,15 +547,17 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
         geo_g << geo.str() << "#undef K_\n#define K_ " << Kg << "\n#define XC_ " << C * G << "\n#define YK_ " << K << "\n";
         key << "mfma|" << half << "|" << geo_g.str() << TRW << "|" << (y->dtype != MJT_FLOAT32) << "|" << WKO << "|" << WPX << "|" << RPW << "|" << MT << "|" << WPS
             << "|" << stage_depth << "|" << CBLK << "|" << NSLAB << "|" << abl;
+        const EpilogueCode ep = epilogue_code(OW % 4 == 0 ? 4 : OW % 2 == 0 ? 2 : 1, 4, y->dtype, numel(y));
+        key << ep.key;
         JitKernel* k = cached(key.str());
         JitKernel* kp = cached(key.str() + "|pack");
         if (!k || !kp) {
             std::ostringstream name;
             name << "mjt_conv_mfma_" << (half ? "f16" : "bf16") << "_c" << C << "_k" << Kg << (G > 1 ? "_g" + std::to_string(G) : std::string()) << "_" << H << "x" << W << "_r" << R << "x" << S << "_s"
                  << p->stride_h << "x" << p->stride_w << "_p" << p->pad_h << "x" << p->pad_w << "_d" << p->dil_h << "x"
-                 << p->dil_w << "_rows" << RPW << (y->dtype == MJT_FLOAT32 ? "_of32" : half ? "_of16" : "_obf16");
+                 << p->dil_w << "_rows" << RPW << (y->dtype == MJT_FLOAT32 ? "_of32" : half ? "_of16" : "_obf16") << ep.suffix();
             std::ostringstream src;
-            src << "#define ENTRY " << name.str() << "\n#define ENTRY_PACK " << name.str() << "_pack\n" << geo_g.str()
+            src << ep.defs << "#define ENTRY " << name.str() << "\n#define ENTRY_PACK " << name.str() << "_pack\n" << geo_g.str()
                 << "#define MT " << MT << "\n#define WKO " << WKO << "\n#define WPX " << WPX << "\n#define TRW " << TRW << "\n#define NT " << NT << "\n#define LROWS " << LROWS << "\n#define LCOLS " << LCOLS
                 << "\n#define RPW " << RPW << "\n#define NFULL " << NFULL << "\n#define TAIL_TRW " << TAIL_TRW << "\n#define TAIL_NT "
                 << TAIL_NT << "\n#define TAIL_LROWS " << TAIL_LROWS << "\n#define Y_BF16 " << (y->dtype != MJT_FLOAT32 ? 1 : 0) << "\n#define IN_F16 " << (half ? 1 : 0)
@@ -568,6 +576,7 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
         // registers than a wave has (accumulation registers beyond the accumulators, scratch memory) may have moved one
         // whose load had not landed, so such a build is not run: the convolution takes the routes below.
         const bool regs_ok = k->spilled == 0 && k->agprs >= 0 && k->agprs <= MT * NT * 4;
+        if (!regs_ok && ep.on) check_no_epilogue();           // (the convolution without the group is the better one)
         if (regs_ok) {
             size_t wbytes = (size_t)numel(w) * 2;
             if (pack_mode) MJT_CHECK(packed && (uintptr_t)packed % 16 == 0, "conv: packed weights must be a 16-byte aligned device buffer");
@@ -591,10 +600,14 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
             char* wdst = (char*)(pack_mode ? packed : g_wpack);
             if (pack_mode != 2) {
                 std::vector<uint64_t> pa{bits_of_ptr(w->ptr), bits_of_ptr(wdst), 0, 0};
+                pa.resize(4 + ep.words.size());
+                Preparing preparing;
                 jit_launch(kp, (unsigned)pblocks, (unsigned)G, 256, 0, pa);
             }
             if (pack_mode != 1) {
                 std::vector<uint64_t> a{bits_of_ptr(x->ptr), bits_of_ptr(wdst), bits_of_ptr(y->ptr), (uint64_t)N};
+                a.insert(a.end(), ep.words.begin(), ep.words.end());
+                epilogue_taken(ep);
                 jit_launch(k, (unsigned)blocks, (unsigned)G, (unsigned)(64 * WPX * WKO), 0, a);
             }
             return;
@@ -632,6 +645,7 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
             lda = (CRS * esz + 15) / 16 * 16 / esz;
             void* wpad = conv_scratch(4, (size_t)(K * lda * esz));
             mjt_tensor tw = view(w->ptr, w->dtype, {K, CRS}), tp = view(wpad, w->dtype, {K, lda});
+            Preparing preparing;
             const char* widx[2] = {"i0", "i1"};                 // columns past CRS lie outside w: overflow value 0
             if (mjt_reindex(&tw, &tp, 2, widx, 0.0, 0, nullptr, 0, nullptr) != MJT_OK)
                 MJT_FAIL(MJT_ERR_DEVICE, "conv: padding the weight rows failed: " << mjt_last_error());
@@ -700,14 +714,15 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
             const int out = y->dtype == MJT_BFLOAT16 ? 0 : y->dtype == MJT_FLOAT16 ? 1 : 2;
             std::ostringstream key;
             const bool xbuf = (64 * NI / P + 2) * C * H * W * esz < (int64_t(1) << 31);      // a tile's images through one buffer descriptor
-            key << "igemm|" << geo.str() << MI << NI << in << out << xbuf << split;
+            const EpilogueCode ep = epilogue_code(1, 12, y->dtype, numel(y));
+            key << "igemm|" << geo.str() << MI << NI << in << out << xbuf << split << ep.key;
             JitKernel* k = cached(key.str());
             if (!k) {
                 std::ostringstream name;
                 name << "mjt_conv_igemm_" << mjt_dtype_name(x->dtype) << (y->dtype != x->dtype ? "_of32" : "") << "_c" << C << "_k" << K << "_" << H << "x" << W << "_r" << R << "x" << S << "_s" << p->stride_h << "x"
-                     << p->stride_w << "_p" << p->pad_h << "x" << p->pad_w << "_d" << p->dil_h << "x" << p->dil_w << (split ? "_parts_" : "_") << 64 * MI << "x" << 64 * NI;
+                     << p->stride_w << "_p" << p->pad_h << "x" << p->pad_w << "_d" << p->dil_h << "x" << p->dil_w << (split ? "_parts_" : "_") << 64 * MI << "x" << 64 * NI << ep.suffix();
                 std::ostringstream src;
-                src << "#define ENTRY " << name.str() << "\n#define SPLIT " << (split ? 1 : 0) << "\n#define CONV 1\n#define IN " << in << "\n#define OUT " << out << "\n#define MI " << MI << "\n#define NI " << NI
+                src << ep.defs << "#define ENTRY " << name.str() << "\n#define SPLIT " << (split ? 1 : 0) << "\n#define CONV 1\n#define IN " << in << "\n#define OUT " << out << "\n#define MI " << MI << "\n#define NI " << NI
                     << "\n#define A_KCONT 1\n#define B_KCONT 0\n#define XBUF " << (xbuf ? 1 : 0) << "\n" << geo.str();
                 if (split) src << embedded_source("split.h") << "\n";
                 src << embedded_source("gemm_mfma.h") << "\n";
@@ -719,6 +734,8 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
             MJT_CHECK(grid < (int64_t(1) << 31), "conv: launch too large");
             std::vector<uint64_t> a{bits_of_ptr(wmat), bits_of_ptr(x->ptr), bits_of_ptr(y->ptr), (uint64_t)K, (uint64_t)NP, (uint64_t)CRS,
                                     (uint64_t)lda, 0, 0, 0, 0, 0};
+            a.insert(a.end(), ep.words.begin(), ep.words.end());
+            epilogue_taken(ep);
             jit_launch(k, (unsigned)grid, 1, product_threads(split), 0, a);
             return;
         }
@@ -784,7 +801,8 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
     // ---- direct path ----------------------------------------------------------------
     const bool idx32 = numel(x) < (int64_t(1) << 31) && numel(y) < (int64_t(1) << 31) - 256 && numel(w) < (int64_t(1) << 31);
     std::ostringstream key;
-    key << "direct|" << geo.str() << x->dtype << "|" << y->dtype << "|" << G << "|" << idx32;
+    const EpilogueCode ep = epilogue_code(1, 4, y->dtype, numel(y));
+    key << "direct|" << geo.str() << x->dtype << "|" << y->dtype << "|" << G << "|" << idx32 << ep.key;
     JitKernel* k = cached(key.str());
     if (!k) {
         std::ostringstream name;
@@ -793,11 +811,13 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
              << "x" << p->pad_w << "_d" << p->dil_h << "x" << p->dil_w;
         if (G > 1) name << "_g" << G;
         if (!idx32) name << "_i64";
+        name << ep.suffix();
         std::ostringstream src;
-        src << "#define ENTRY " << name.str() << "\n#define TIN " << dtype_cname(x->dtype) << "\n#define TOUT "
+        src << ep.defs << "#define ENTRY " << name.str() << "\n#define TIN " << dtype_cname(x->dtype) << "\n#define TOUT "
             << dtype_cname(y->dtype) << "\n#define G_ " << G << "\n#define IDX " << (idx32 ? "int" : "long long")
             << "\n" << geo.str();
-        src << embedded_source("prelude.h") << "\n" << embedded_source("conv_direct.h") << "\n";
+        if (!ep.on) src << embedded_source("prelude.h") << "\n";
+        src << embedded_source("conv_direct.h") << "\n";
         k = jit_get(src.str(), name.str());
         remember(key.str(), k);
     }
@@ -805,6 +825,8 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
     const int64_t blocks = (total + 255) / 256;
     MJT_CHECK(blocks < (int64_t(1) << 31), "conv: launch too large");
     std::vector<uint64_t> a{bits_of_ptr(x->ptr), bits_of_ptr(w->ptr), bits_of_ptr(y->ptr), (uint64_t)total};
+    a.insert(a.end(), ep.words.begin(), ep.words.end());
+    epilogue_taken(ep);
     jit_launch(k, (unsigned)blocks, 1, 256, 0, a);
 }
 
@@ -1480,7 +1502,10 @@ void conv_dgrad_impl(const mjt_tensor* dy, const mjt_tensor* w, const mjt_tensor
         return;
     }
     mjt_tensor tw = view(wbuf, w->dtype, {C, K, R, S});
-    reindex(*w, tw, {"i1", "i0", str(R - 1) + "-i2", str(S - 1) + "-i3"}, {});
+    {
+        Preparing preparing;
+        reindex(*w, tw, {"i1", "i0", str(R - 1) + "-i2", str(S - 1) + "-i3"}, {});
+    }
     const mjt_conv_params q = {1, 1, (int32_t)(dh * (R - 1) - ph), (int32_t)(dw * (S - 1) - pw), (int32_t)dh, (int32_t)dw};
     if (sh == 1 && sw == 1) {
         conv_impl(dy, &tw, dx, &q, 1);
@@ -1488,7 +1513,10 @@ void conv_dgrad_impl(const mjt_tensor* dy, const mjt_tensor* w, const mjt_tensor
     }
     const int64_t ZH = H + 2 * ph - dh * (R - 1), ZW = W + 2 * pw - dw * (S - 1);
     mjt_tensor tz = view(conv_scratch(3, (size_t)(N * K * ZH * ZW * esz)), dy->dtype, {N, K, ZH, ZW});
-    reindex(*dy, tz, {"i0", "i1", "i2/" + str(sh), "i3/" + str(sw)}, {"i2%" + str(sh) + "!=0", "i3%" + str(sw) + "!=0"});
+    {
+        Preparing preparing;
+        reindex(*dy, tz, {"i0", "i1", "i2/" + str(sh), "i3/" + str(sw)}, {"i2%" + str(sh) + "!=0", "i3%" + str(sw) + "!=0"});
+    }
     conv_impl(&tz, &tw, dx, &q, 1);
 }
 }  // namespace mjt

@@ -20,16 +20,11 @@ const bool g_registered = (at_shutdown(&forget), true);
 bool is_unary_op(int op) { return op >= MJT_OP_ABS && op <= MJT_OP_SIGMOID; }
 bool is_binary_op(int op) { return op >= MJT_OP_POW && op <= MJT_OP_MEAN; }
 
-struct MergedDim {
-    int64_t size;
-    std::vector<int> bcast;   // per input tensor: 1 when broadcast along this axis
-};
-
 std::string vname(int i) { return "v" + std::to_string(i); }
 
 }  // namespace
 
-int64_t fused_validate(const mjt_fused_desc* d, std::vector<int>* inputs_out, bool outputs_need_data, bool allow_gathered) {
+int64_t fused_validate(const mjt_fused_desc* d, std::vector<int>* inputs_out, bool outputs_need_data, int also) {
     MJT_CHECK(d, "fused: null descriptor");
     MJT_CHECK(d->ndim >= 1 && d->ndim <= MJT_MAX_DIM, "fused: rank " << d->ndim);
     MJT_CHECK(d->n_vars > 0 && d->n_ops > 0 && d->vars && d->ops, "fused: empty group");
@@ -45,12 +40,12 @@ int64_t fused_validate(const mjt_fused_desc* d, std::vector<int>* inputs_out, bo
     for (int i = 0; i < nv; i++) {
         const mjt_fused_var& v = d->vars[i];
         dtype_size(v.dtype);
-        MJT_CHECK(v.role >= MJT_VAR_INPUT && v.role <= (allow_gathered ? MJT_VAR_GATHERED : MJT_VAR_SCALAR),
-                  "fused: var " << i << " has role " << v.role);
+        MJT_CHECK((v.role >= MJT_VAR_INPUT && v.role <= MJT_VAR_SCALAR) || v.role == also, "fused: var " << i << " has role " << v.role);
         if (v.role == MJT_VAR_GATHERED) {
             MJT_CHECK(total == 0 || v.ptr, "fused: gathered var " << i << " has no data");
             defined[i] = 1;
         }
+        if (v.role == MJT_VAR_PRODUCT) defined[i] = 1;
         if (v.role == MJT_VAR_INPUT) {
             MJT_CHECK(total == 0 || v.ptr, "fused: input var " << i << " has no data");
             MJT_CHECK((v.bcast_mask >> d->ndim) == 0, "fused: bcast_mask of var " << i << " exceeds the rank");
@@ -124,18 +119,12 @@ std::string fused_emit_ops(const mjt_fused_desc* d, bool store_outputs) {
     return body.str();
 }
 
-void fused_impl(const mjt_fused_desc* d) {
-    require_init();
-    std::vector<int> inputs;          // var ids of tensor inputs
-    const int64_t total = fused_validate(d, &inputs, true);
-    const int nv = d->n_vars;
-    if (total == 0) return;
-
-    // ---- merge axes: drop extent-1 axes, fuse neighbours on which every input agrees -------
-    std::vector<MergedDim> dims;
+// ---- merge axes: drop extent-1 axes, fuse neighbours on which every input agrees -------
+std::vector<FusedCode::Dim> fused_dims(const mjt_fused_desc* d, const std::vector<int>& inputs) {
+    std::vector<FusedCode::Dim> dims;
     for (int a = 0; a < d->ndim; a++) {
         if (d->shape[a] == 1) continue;
-        MergedDim m;
+        FusedCode::Dim m;
         m.size = d->shape[a];
         for (int id : inputs) m.bcast.push_back((d->vars[id].bcast_mask >> a) & 1);
         if (!dims.empty() && dims.back().bcast == m.bcast)
@@ -144,11 +133,160 @@ void fused_impl(const mjt_fused_desc* d) {
             dims.push_back(m);
     }
     if (dims.empty()) {
-        MergedDim m;
+        FusedCode::Dim m;
         m.size = 1;
         m.bcast.assign(inputs.size(), 0);
         dims.push_back(m);
     }
+    return dims;
+}
+
+bool fused_aligned(const mjt_fused_desc* d, const std::vector<int>& inputs, const std::vector<FusedCode::Dim>& dims, int vec) {
+    if (dims.back().size % vec) return false;
+    for (int i = 0; i < d->n_vars; i++) {
+        const mjt_fused_var& fv = d->vars[i];
+        if (fv.role == MJT_VAR_OUTPUT && (uintptr_t)fv.ptr % (size_t)(vec * dtype_size(fv.dtype))) return false;
+    }
+    for (size_t k = 0; k < inputs.size(); k++) {
+        const mjt_fused_var& fv = d->vars[inputs[k]];
+        if (dims.back().bcast[k]) continue;   // scalar load per lane
+        if ((uintptr_t)fv.ptr % (size_t)(vec * dtype_size(fv.dtype))) return false;
+    }
+    return true;
+}
+
+// ---- parameter block layout ---------------------------------------------------
+// from word `first` on: per merged axis: extent, divider | per var: pointer or scalar bits
+// | per (input with broadcast, merged axis): stride in elements
+FusedCode::FusedCode(const mjt_fused_desc* desc, const std::vector<int>& ins, const std::vector<Dim>& axes, int v, bool i64, int first)
+    : d(desc), inputs(ins), dims(axes), vec(v), use64(i64), p_dim(axes.size()), p_var(desc->n_vars, -1), p_stride(ins.size()) {
+    const int nd = (int)dims.size();
+    auto next = [&]() { return first + (int)words.size(); };
+    for (int a = 0; a < nd; a++) {
+        p_dim[a] = next();
+        words.push_back((uint64_t)dims[a].size);
+        words.push_back(pack_divmod((uint64_t)dims[a].size));
+    }
+    for (int i = 0; i < d->n_vars; i++) {
+        const mjt_fused_var& fv = d->vars[i];
+        if (fv.role == MJT_VAR_INTERMEDIATE || fv.role == MJT_VAR_PRODUCT) continue;
+        p_var[i] = next();
+        if (fv.role == MJT_VAR_SCALAR) {
+            if (dtype_is_float(fv.dtype)) words.push_back(bits_of(fv.fvalue));
+            else words.push_back((uint64_t)fv.ivalue);
+        } else
+            words.push_back(bits_of_ptr(fv.ptr));
+    }
+    for (size_t k = 0; k < inputs.size(); k++) {
+        bool any = false;
+        for (int a = 0; a < nd; a++) any |= dims[a].bcast[k] != 0;
+        if (!any) continue;
+        need_decode = true;
+        int64_t stride = 1;
+        std::vector<int64_t> st(nd, 0);
+        for (int a = nd - 1; a >= 0; a--) {
+            if (!dims[a].bcast[k]) {
+                st[a] = stride;
+                stride *= dims[a].size;
+            }
+        }
+        for (int a = 0; a < nd; a++) {
+            p_stride[k].push_back(next());
+            words.push_back((uint64_t)st[a]);
+        }
+    }
+}
+
+std::string FusedCode::key() const {
+    std::ostringstream key;
+    key << dims.size() << "|" << vec << "|" << use64 << "|";
+    for (const Dim& a : dims) {
+        for (int b : a.bcast) key << b;
+        key << ",";
+    }
+    for (int i = 0; i < d->n_vars; i++) key << d->vars[i].role << ":" << d->vars[i].dtype << ";";
+    for (int k = 0; k < d->n_ops; k++) {
+        const mjt_fused_op& o = d->ops[k];
+        key << o.kind << ":" << o.op << ":" << o.in[0] << ":" << (o.kind >= MJT_FOP_BINARY ? o.in[1] : -1) << ":"
+            << (o.kind == MJT_FOP_TERNARY ? o.in[2] : -1) << ">" << o.out << ";";
+    }
+    return key.str();
+}
+
+std::string FusedCode::text(const std::string& prefix, const char* ld, const char* st) const {
+    const int nd = (int)dims.size(), nv = d->n_vars;
+    const char* IT = use64 ? "long long" : "int";
+    std::ostringstream scal, dec, decl, outs, loads, body, stores;
+    for (int i = 0; i < nv; i++) {
+        const mjt_fused_var& fv = d->vars[i];
+        if (fv.role != MJT_VAR_SCALAR) continue;
+        const char* T = dtype_cname(fv.dtype);
+        if (dtype_is_float(fv.dtype))
+            scal << "const " << T << " " << vname(i) << " = (" << T << ")__longlong_as_double((long long)(unsigned long long)p.a["
+                 << p_var[i] << "]); ";
+        else
+            scal << "const " << T << " " << vname(i) << " = (" << T << ")(long long)(unsigned long long)p.a[" << p_var[i] << "]; ";
+    }
+    if (need_decode) {
+        dec << IT << " rem_ = e; ";
+        for (int a = nd - 1; a >= 0; a--) {
+            if (a == 0) {
+                dec << "const " << IT << " c0 = rem_; ";
+            } else if (use64) {
+                dec << "const " << IT << " q" << a << " = rem_ / (" << IT << ")(unsigned long long)p.a[" << p_dim[a] << "]; const " << IT
+                    << " c" << a << " = rem_ - q" << a << " * (" << IT << ")(unsigned long long)p.a[" << p_dim[a] << "]; rem_ = q" << a
+                    << "; ";
+            } else {
+                dec << "const int q" << a << " = (int)mjt_div((unsigned)rem_, mjt_unpack_divmod((unsigned long long)p.a[" << p_dim[a] + 1
+                    << "], 0)); const int c" << a << " = rem_ - q" << a << " * (int)(unsigned long long)p.a[" << p_dim[a] << "]; rem_ = q"
+                    << a << "; ";
+            }
+        }
+    }
+    for (size_t k = 0; k < inputs.size(); k++) {
+        int id = inputs[k];
+        const char* T = dtype_cname(d->vars[id].dtype);
+        std::string off = "e";
+        if (!p_stride[k].empty()) {
+            off = "(";
+            for (int a = 0; a < nd; a++) {
+                if (dims[a].bcast[k]) continue;
+                off += "c" + std::to_string(a) + " * (" + IT + ")(unsigned long long)p.a[" + std::to_string(p_stride[k][a]) + "] + ";
+            }
+            off += "0)";
+        }
+        const bool one = dims.back().bcast[k] && vec > 1;      // one value for the lane's vector
+        decl << "mjt_pack<" << T << ", " << (one ? 1 : vec) << "> in" << id << "; ";
+        if (one) loads << "t.in" << id << ".v[0] = ((const " << T << "*)p.a[" << p_var[id] << "])[" << off << "]; ";
+        else loads << ld << "(t.in" << id << ", (const " << T << "*)p.a[" << p_var[id] << "] + " << off << "); ";
+        body << "const " << T << " " << vname(id) << " = t.in" << id << ".v[" << (one ? "0" : "k") << "]; ";
+    }
+    body << fused_emit_ops(d, true);
+    for (int i = 0; i < nv; i++)
+        if (d->vars[i].role == MJT_VAR_OUTPUT) {
+            outs << "mjt_pack<" << dtype_cname(d->vars[i].dtype) << ", " << vec << "> out" << i << "; ";
+            stores << st << "((" << dtype_cname(d->vars[i].dtype) << "*)p.a[" << p_var[i] << "] + e, out" << i << "); ";
+        }
+    std::ostringstream frag;
+    frag << "#define " << prefix << "_VEC " << vec << "\n#define " << prefix << "_INDEX " << IT << "\n";
+    frag << "#define " << prefix << "_SCALARS " << scal.str() << "\n";
+    frag << "#define " << prefix << "_DECODE " << dec.str() << "\n";
+    frag << "#define " << prefix << "_DECL " << decl.str() << "\n";
+    frag << "#define " << prefix << "_LOADS " << loads.str() << "\n";
+    frag << "#define " << prefix << "_OUTS " << outs.str() << "\n";
+    frag << "#define " << prefix << "_BODY " << body.str() << "\n";
+    frag << "#define " << prefix << "_STORES " << stores.str() << "\n";
+    return frag.str();
+}
+
+void fused_impl(const mjt_fused_desc* d) {
+    require_init();
+    std::vector<int> inputs;          // var ids of tensor inputs
+    const int64_t total = fused_validate(d, &inputs, true);
+    const int nv = d->n_vars;
+    if (total == 0) return;
+
+    const std::vector<FusedCode::Dim> dims = fused_dims(d, inputs);
     const int nd = (int)dims.size();
     bool use64 = total >= (int64_t(1) << 31);
 
@@ -158,20 +296,7 @@ void fused_impl(const mjt_fused_desc* d) {
         if (d->vars[i].role == MJT_VAR_INPUT || d->vars[i].role == MJT_VAR_OUTPUT)
             maxsize = std::max(maxsize, dtype_size(d->vars[i].dtype));
     int vec = std::min(8, 16 / maxsize);
-    auto aligned = [&](int v) {
-        if (dims.back().size % v) return false;
-        for (int i = 0; i < nv; i++) {
-            const mjt_fused_var& fv = d->vars[i];
-            if (fv.role == MJT_VAR_OUTPUT && (uintptr_t)fv.ptr % (size_t)(v * dtype_size(fv.dtype))) return false;
-        }
-        for (size_t k = 0; k < inputs.size(); k++) {
-            const mjt_fused_var& fv = d->vars[inputs[k]];
-            if (dims.back().bcast[k]) continue;   // scalar load per lane
-            if ((uintptr_t)fv.ptr % (size_t)(v * dtype_size(fv.dtype))) return false;
-        }
-        return true;
-    };
-    while (vec > 1 && !aligned(vec)) vec /= 2;
+    while (vec > 1 && !fused_aligned(d, inputs, dims, vec)) vec /= 2;
     int64_t nvec = total / vec;
     // measured on MI355X: one vector per lane is fastest for the chain workloads (more vectors per
     // lane cost registers and occupancy); outputs too large to be re-read from cache are stored
@@ -192,61 +317,12 @@ void fused_impl(const mjt_fused_desc* d) {
     int unroll = 1;
     int nt = streams ? 2 : 0;   // bit 0: non-temporal loads, bit 1: non-temporal stores
 
-    // ---- parameter block layout ---------------------------------------------------
-    // a[0] nvec | per merged axis: extent, divider | per var: pointer or scalar bits
-    // | per (input with broadcast, merged axis): stride in elements
-    std::vector<uint64_t> args;
-    args.push_back((uint64_t)nvec);
-    std::vector<int> p_dim(nd), p_var(nv, -1);
-    for (int a = 0; a < nd; a++) {
-        p_dim[a] = (int)args.size();
-        args.push_back((uint64_t)dims[a].size);
-        args.push_back(pack_divmod((uint64_t)dims[a].size));
-    }
-    for (int i = 0; i < nv; i++) {
-        const mjt_fused_var& fv = d->vars[i];
-        if (fv.role == MJT_VAR_INTERMEDIATE) continue;
-        p_var[i] = (int)args.size();
-        if (fv.role == MJT_VAR_SCALAR) {
-            if (dtype_is_float(fv.dtype)) args.push_back(bits_of(fv.fvalue));
-            else args.push_back((uint64_t)fv.ivalue);
-        } else
-            args.push_back(bits_of_ptr(fv.ptr));
-    }
-    std::vector<std::vector<int>> p_stride(inputs.size());
-    bool need_decode = false;
-    for (size_t k = 0; k < inputs.size(); k++) {
-        bool any = false;
-        for (int a = 0; a < nd; a++) any |= dims[a].bcast[k] != 0;
-        if (!any) continue;
-        need_decode = true;
-        int64_t stride = 1;
-        std::vector<int64_t> st(nd, 0);
-        for (int a = nd - 1; a >= 0; a--) {
-            if (!dims[a].bcast[k]) {
-                st[a] = stride;
-                stride *= dims[a].size;
-            }
-        }
-        for (int a = 0; a < nd; a++) {
-            p_stride[k].push_back((int)args.size());
-            args.push_back((uint64_t)st[a]);
-        }
-    }
+    const FusedCode code(d, inputs, dims, vec, use64, 1);
+    std::vector<uint64_t> args{(uint64_t)nvec};
+    args.insert(args.end(), code.words.begin(), code.words.end());
 
-    // ---- static key -----------------------------------------------------------------
     std::ostringstream key;
-    key << nd << "|" << vec << "|" << unroll << "|" << use64 << "|" << block << "|" << nt << "|";
-    for (int a = 0; a < nd; a++) {
-        for (int b : dims[a].bcast) key << b;
-        key << ",";
-    }
-    for (int i = 0; i < nv; i++) key << d->vars[i].role << ":" << d->vars[i].dtype << ";";
-    for (int k = 0; k < d->n_ops; k++) {
-        const mjt_fused_op& o = d->ops[k];
-        key << o.kind << ":" << o.op << ":" << o.in[0] << ":" << (o.kind >= MJT_FOP_BINARY ? o.in[1] : -1) << ":"
-            << (o.kind == MJT_FOP_TERNARY ? o.in[2] : -1) << ">" << o.out << ";";
-    }
+    key << unroll << "|" << block << "|" << nt << "|" << code.key();
     JitKernel* kern = nullptr;
     {
         std::lock_guard<std::mutex> lock(g_mu);
@@ -254,78 +330,9 @@ void fused_impl(const mjt_fused_desc* d) {
         if (it != g_kernels.end()) kern = it->second;
     }
     if (!kern) {
-        const char* IT = use64 ? "long long" : "int";
-        std::ostringstream scal, dec, loads, body, stores;
-        for (int i = 0; i < nv; i++) {
-            const mjt_fused_var& fv = d->vars[i];
-            if (fv.role != MJT_VAR_SCALAR) continue;
-            const char* T = dtype_cname(fv.dtype);
-            if (dtype_is_float(fv.dtype))
-                scal << "const " << T << " " << vname(i) << " = (" << T << ")__longlong_as_double((long long)(unsigned long long)p.a["
-                     << p_var[i] << "]); ";
-            else
-                scal << "const " << T << " " << vname(i) << " = (" << T << ")(long long)(unsigned long long)p.a[" << p_var[i] << "]; ";
-        }
-        if (need_decode) {
-            dec << IT << " rem_ = e; ";
-            for (int a = nd - 1; a >= 0; a--) {
-                if (a == 0) {
-                    dec << "const " << IT << " c0 = rem_; ";
-                } else if (use64) {
-                    dec << "const " << IT << " q" << a << " = rem_ / (" << IT << ")(unsigned long long)p.a[" << p_dim[a] << "]; const " << IT
-                        << " c" << a << " = rem_ - q" << a << " * (" << IT << ")(unsigned long long)p.a[" << p_dim[a] << "]; rem_ = q" << a
-                        << "; ";
-                } else {
-                    dec << "const int q" << a << " = (int)mjt_div((unsigned)rem_, mjt_unpack_divmod((unsigned long long)p.a[" << p_dim[a] + 1
-                        << "], 0)); const int c" << a << " = rem_ - q" << a << " * (int)(unsigned long long)p.a[" << p_dim[a] << "]; rem_ = q"
-                        << a << "; ";
-                }
-            }
-        }
-        for (size_t k = 0; k < inputs.size(); k++) {
-            int id = inputs[k];
-            const char* T = dtype_cname(d->vars[id].dtype);
-            std::string off = "e";
-            if (!p_stride[k].empty()) {
-                off = "(";
-                for (int a = 0; a < nd; a++) {
-                    if (dims[a].bcast[k]) continue;
-                    off += "c" + std::to_string(a) + " * (" + IT + ")(unsigned long long)p.a[" + std::to_string(p_stride[k][a]) + "] + ";
-                }
-                off += "0)";
-            }
-            if (dims.back().bcast[k] && vec > 1) {
-                loads << "const " << T << " s" << id << " = ((const " << T << "*)p.a[" << p_var[id] << "])[" << off << "]; ";
-            } else {
-                loads << "mjt_pack<" << T << ", VEC> in" << id << "; MJT_LD(in" << id << ", (const " << T << "*)p.a["
-                      << p_var[id] << "] + " << off << "); ";
-            }
-        }
-        for (int i = 0; i < nv; i++)
-            if (d->vars[i].role == MJT_VAR_OUTPUT)
-                loads << "mjt_pack<" << dtype_cname(d->vars[i].dtype) << ", VEC> out" << i << "; ";
-        for (size_t k = 0; k < inputs.size(); k++) {
-            int id = inputs[k];
-            const char* T = dtype_cname(d->vars[id].dtype);
-            if (dims.back().bcast[k] && vec > 1)
-                body << "const " << T << " " << vname(id) << " = s" << id << "; ";
-            else
-                body << "const " << T << " " << vname(id) << " = in" << id << ".v[k]; ";
-        }
-        body << fused_emit_ops(d, true);
-        for (int i = 0; i < nv; i++)
-            if (d->vars[i].role == MJT_VAR_OUTPUT)
-                stores << "MJT_ST((" << dtype_cname(d->vars[i].dtype) << "*)p.a[" << p_var[i] << "] + e, out" << i << "); ";
-
         std::ostringstream frag;
-        frag << "#define VEC " << vec << "\n#define UNROLL " << unroll << "\n#define index_t " << IT << "\n#define NPARAM "
-             << args.size() << "\n#define BLOCK " << block << "\n#define MJT_LD " << ((nt & 1) ? "mjt_load_nt" : "mjt_load")
-             << "\n#define MJT_ST " << ((nt & 2) ? "mjt_store_nt" : "mjt_store") << "\n";
-        frag << "#define MJT_FUSED_SCALARS " << scal.str() << "\n";
-        frag << "#define MJT_FUSED_DECODE " << dec.str() << "\n";
-        frag << "#define MJT_FUSED_LOADS " << loads.str() << "\n";
-        frag << "#define MJT_FUSED_BODY " << body.str() << "\n";
-        frag << "#define MJT_FUSED_STORES " << stores.str() << "\n";
+        frag << code.text("MJT_FUSED", (nt & 1) ? "mjt_load_nt" : "mjt_load", (nt & 2) ? "mjt_store_nt" : "mjt_store") << "#define UNROLL " << unroll
+             << "\n#define NPARAM " << args.size() << "\n#define BLOCK " << block << "\n";
         uint64_t h = 1469598103934665603ull;
         for (unsigned char c : frag.str()) {
             h ^= c;

@@ -63,6 +63,7 @@ const void* padded_rows(int which, const void* src, int dtype, int64_t rows, int
     t.shape[0] = d.shape[0] = rows;
     t.shape[1] = ld;
     d.shape[1] = ldp;
+    Preparing preparing;
     const char* idx[2] = {"i0", "i1"};                          // columns past ld lie outside the source: overflow value 0
     if (mjt_reindex(&t, &d, 2, idx, 0.0, 0, nullptr, 0, nullptr) != MJT_OK) MJT_FAIL(MJT_ERR_DEVICE, "matmul: padding the rows failed: " << mjt_last_error());
     return d.ptr;
@@ -121,15 +122,20 @@ void gemm_launch(int in_dtype, int out_dtype, const void* A, const void* B, void
             // workgroups: 3072 x 3072 x 1024 35.4 / 31.7; 8192 x 1024 x 1024 26.8 / 22.1; 64 x 512 x 28 x 28 -> 512 as a
             // product 82.3 / 63.7); with at most one tile each a ring of four (2048^3 21.7 / 24.8; 1536^3 15.3 / 20.5)
             const int nbuf = tile == 256 ? 2 : (double)tm * tn * batch > (double)cus ? 2 : 4, wpe = tile == 128 && nbuf == 2 ? 2 : 1;
+            // adjacent results that a lane stores: rows of C have to be such vectors, wherever a tile ends
+            const int osz = dtype_size(out_dtype);
+            auto whole = [&](int v) { return N % v == 0 && ldc % v == 0 && sc % v == 0 && (uintptr_t)C % (size_t)(v * osz) == 0; };
+            const int vs = whole(4) ? 4 : whole(2) ? 2 : 1;
+            const EpilogueCode ep = epilogue_code(vs, 12, out_dtype, ldc == N && (batch == 1 || sc == M * N) ? M * N * batch : -1);
             std::ostringstream key;
-            key << "gemmd|" << in << out << a_kcont << b_kcont << tile << nbuf;
+            key << "gemmd|" << in << out << a_kcont << b_kcont << tile << nbuf << vs << ep.key;
             JitKernel* k = cached(key.str());
             if (!k) {
                 std::ostringstream name;
                 name << "mjt_gemm_mfma_" << mjt_dtype_name(in_dtype) << "_" << mjt_dtype_name(out_dtype) << "_" << tile << "x" << tile << (a_kcont ? "_n" : "_t")
-                     << (b_kcont ? "t" : "n") << "_direct" << (wpe == 2 ? "2" : "");
+                     << (b_kcont ? "t" : "n") << "_direct" << (wpe == 2 ? "2" : "") << ep.suffix();
                 std::ostringstream src;
-                src << "#define ENTRY " << name.str() << "\n#define IN " << in << "\n#define OUT " << out << "\n#define A_KCONT " << (a_kcont ? 1 : 0)
+                src << ep.defs << "#define VS " << vs << "\n#define ENTRY " << name.str() << "\n#define IN " << in << "\n#define OUT " << out << "\n#define A_KCONT " << (a_kcont ? 1 : 0)
                     << "\n#define B_KCONT " << (b_kcont ? 1 : 0) << "\n#define TILE " << tile << "\n#define NBUF " << nbuf << "\n#define WPE " << wpe << "\n";
                 src << embedded_source("gemm_dma.h") << "\n";
                 k = jit_get(src.str(), name.str());
@@ -141,9 +147,12 @@ void gemm_launch(int in_dtype, int out_dtype, const void* A, const void* B, void
             if (k->spilled == 0 && k->agprs >= 0 && k->agprs <= tile * tile / 256) {
                 const int64_t grid = (tm * tn + 7) / 8 * 8;
                 MJT_CHECK(grid < (int64_t(1) << 31), "matmul: launch too large");
+                args.insert(args.end(), ep.words.begin(), ep.words.end());
+                epilogue_taken(ep);
                 jit_launch(k, (unsigned)grid, (unsigned)batch, 256, 0, args);
                 return;
             }
+            if (ep.on) check_no_epilogue();                      // (the product without the group is the better one)
         }
     }
     if (fast) {
@@ -210,15 +219,16 @@ void gemm_launch(int in_dtype, int out_dtype, const void* A, const void* B, void
         const int in = in_dtype == MJT_BFLOAT16 ? 0 : in_dtype == MJT_FLOAT16 ? 1 : 2;
         const int out = slices > 1 || out_dtype == MJT_FLOAT32 ? 2 : out_dtype == MJT_BFLOAT16 ? 0 : 1;
         const bool one_stage = stages == 1 && !getenv("MJT_GEMM_TWO_BUFFERS");       // a single stage of the kernel's k loop
+        const EpilogueCode ep = epilogue_code(1, 12, out_dtype, slices == 1 && ldc == N && (batch == 1 || sc == M * N) ? M * N * batch : -1);
         std::ostringstream key;
-        key << "gemm|" << in << out << MI << NI << a_kcont << b_kcont << one_stage << (slices > 1) << split;
+        key << "gemm|" << in << out << MI << NI << a_kcont << b_kcont << one_stage << (slices > 1) << split << ep.key;
         JitKernel* k = cached(key.str());
         if (!k) {
             std::ostringstream name;
             name << "mjt_gemm_mfma_" << mjt_dtype_name(in_dtype) << "_" << (out == 2 ? "float32" : mjt_dtype_name(out_dtype)) << "_" << 64 * MI << "x" << 64 * NI
-                 << (a_kcont ? "_n" : "_t") << (b_kcont ? "t" : "n") << (one_stage ? "_k1" : "") << (split ? "_parts" : "") << (slices > 1 ? "_slices" : "");
+                 << (a_kcont ? "_n" : "_t") << (b_kcont ? "t" : "n") << (one_stage ? "_k1" : "") << (split ? "_parts" : "") << (slices > 1 ? "_slices" : "") << ep.suffix();
             std::ostringstream src;
-            src << "#define NBUF " << (one_stage ? 1 : 2) << "\n#define SLICED " << (slices > 1 ? 1 : 0) << "\n#define SPLIT " << (split ? 1 : 0) << "\n";
+            src << ep.defs << "#define NBUF " << (one_stage ? 1 : 2) << "\n#define SLICED " << (slices > 1 ? 1 : 0) << "\n#define SPLIT " << (split ? 1 : 0) << "\n";
             src << "#define ENTRY " << name.str() << "\n#define IN " << in << "\n#define OUT " << out << "\n#define MI " << MI
                 << "\n#define NI " << NI << "\n#define A_KCONT " << (a_kcont ? 1 : 0) << "\n#define B_KCONT " << (b_kcont ? 1 : 0) << "\n";
             if (split) src << embedded_source("split.h") << "\n";
@@ -231,6 +241,8 @@ void gemm_launch(int in_dtype, int out_dtype, const void* A, const void* B, void
         MJT_CHECK(grid < (int64_t(1) << 31), "matmul: launch too large");
         if (slices == 1) {
             args[3] |= (uint64_t)batch << 32;
+            args.insert(args.end(), ep.words.begin(), ep.words.end());
+            epilogue_taken(ep);
             jit_launch(k, (unsigned)grid, 1, product_threads(split), 0, args);
             return;
         }
@@ -297,22 +309,29 @@ bool gemm_pixels(int in_dtype, int out_dtype, const void* A, const void* x, void
     if (P % 8 == 0 && a_kcont && (K < 128 || (K < 512 && tm * tn <= cus / 2))) return false;
     const int in = in_dtype == MJT_BFLOAT16 ? 0 : 1, out = out_dtype == MJT_BFLOAT16 ? 0 : out_dtype == MJT_FLOAT16 ? 1 : 2;
     const int nbuf = tm * tn > cus ? 2 : 4, wpe = nbuf == 2 ? 2 : 1;      // as for the plain product: two workgroups a unit, or a deeper ring
+    const int osz = dtype_size(out_dtype), vs = P % 4 == 0 && (uintptr_t)y % (size_t)(4 * osz) == 0 ? 4 : (uintptr_t)y % (size_t)(2 * osz) == 0 ? 2 : 1;
+    const EpilogueCode ep = epilogue_code(vs, 12, out_dtype, M * P * images);
     std::ostringstream key;
-    key << "gemmpx|" << in << out << a_kcont << tile << nbuf << "|" << P;
+    key << "gemmpx|" << in << out << a_kcont << tile << nbuf << vs << "|" << P << ep.key;
     JitKernel* k = cached(key.str());
     if (!k) {
         std::ostringstream name;
-        name << "mjt_gemm_mfma_" << mjt_dtype_name(in_dtype) << "_" << mjt_dtype_name(out_dtype) << "_" << tile << "x" << tile << (a_kcont ? "_n" : "_t") << "_pixels" << P << (wpe == 2 ? "_direct2" : "_direct");
+        name << "mjt_gemm_mfma_" << mjt_dtype_name(in_dtype) << "_" << mjt_dtype_name(out_dtype) << "_" << tile << "x" << tile << (a_kcont ? "_n" : "_t") << "_pixels" << P << (wpe == 2 ? "_direct2" : "_direct") << ep.suffix();
         std::ostringstream src;
-        src << "#define ENTRY " << name.str() << "\n#define IN " << in << "\n#define OUT " << out << "\n#define A_KCONT " << (a_kcont ? 1 : 0) << "\n#define B_KCONT 0\n#define IMG " << P
+        src << ep.defs << "#define VS " << vs << "\n#define ENTRY " << name.str() << "\n#define IN " << in << "\n#define OUT " << out << "\n#define A_KCONT " << (a_kcont ? 1 : 0) << "\n#define B_KCONT 0\n#define IMG " << P
             << "\n#define TILE " << tile << "\n#define NBUF " << nbuf << "\n#define WPE " << wpe << "\n";
         src << embedded_source("gemm_dma.h") << "\n";
         k = jit_get(src.str(), name.str());
         remember(key.str(), k);
     }
-    if (k->spilled != 0 || k->agprs < 0 || k->agprs > tile * tile / 256) return false;     // (see gemm_launch)
+    if (k->spilled != 0 || k->agprs < 0 || k->agprs > tile * tile / 256) {                 // (see gemm_launch)
+        if (ep.on) check_no_epilogue();
+        return false;
+    }
     std::vector<uint64_t> args{bits_of_ptr(A), bits_of_ptr(x), bits_of_ptr(y), (uint64_t)M, (uint64_t)N, (uint64_t)K, (uint64_t)lda, (uint64_t)(K * P), (uint64_t)(M * P), 0,
                                (uint64_t)(images * K * P * 2), 0};
+    args.insert(args.end(), ep.words.begin(), ep.words.end());
+    epilogue_taken(ep);
     jit_launch(k, (unsigned)((tm * tn + 7) / 8 * 8), 1, 256, 0, args);
     return true;
 }

@@ -538,7 +538,7 @@ void fused_reindex_reduce_impl(const mjt_fused_desc* d, const mjt_tensor* x, int
     check_tensor(x, "fused reindex_reduce x");
     check_extras(n_ex, ex);
     std::vector<int> inputs;
-    fused_validate(d, &inputs, false, true);
+    fused_validate(d, &inputs, false, MJT_VAR_GATHERED);
     int out = -1;
     for (int i = 0; i < d->n_vars; i++)
         if (d->vars[i].role == MJT_VAR_OUTPUT) {

@@ -348,6 +348,7 @@ JitKernel* jit_lookup(const std::string& source) {
 
 void jit_launch(JitKernel* k, unsigned grid_x, unsigned grid_y, unsigned block, unsigned shmem,
                 const std::vector<uint64_t>& args, unsigned grid_z) {
+    check_no_epilogue();
     if (t_recording) {
         t_recording->launches.push_back(Launch{k, grid_x, grid_y, grid_z, block, shmem, args});
         return;

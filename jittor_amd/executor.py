@@ -24,7 +24,7 @@ from . import profiler as _profiler
 from .flags import flags
 
 stats = {"launches": 0, "fused_groups": 0, "fused_reduces": 0, "conv_matches": 0, "syncs": 0, "sunk_ops": 0, "matmul_matches": 0,
-         "wgrad_kernel": 0, "wgrad_chunked": 0, "gather_reduces": 0, "fused_scatters": 0, "fused_rows": 0, "plans": 0, "replays": 0, "recorded_launches": 0}
+         "wgrad_kernel": 0, "wgrad_chunked": 0, "gather_reduces": 0, "fused_scatters": 0, "fused_rows": 0, "fused_products": 0, "plans": 0, "replays": 0, "recorded_launches": 0}
 
 
 class ConvUnit:
@@ -1037,10 +1037,12 @@ def _execute(ops, target_ids):
             elif members:
                 reads = reads_of(members)
             plain = isinstance(op, ReduceOp)
-            tasks.append(rowfuse.Task(lambda op=op: run_node(op), reads, {op.out.id}, members if plain else (), op if plain else None))
+            tasks.append(rowfuse.Task(lambda op=op: run_node(op), reads, {op.out.id}, members if plain else (), op if plain else None, op))
     # chains of groups and row reduces over one shape run as one kernel each (while a profile is taken the parts are timed as they are)
     if flags["enable_row_fusion"] and _profiler.active() is None:
         tasks = rowfuse.merge(tasks, ins, pre, consumers, target_ids, sys.modules[__name__]) or tasks
+    if flags["enable_product_fusion"] and _profiler.active() is None:
+        tasks = _behind_products(tasks, ins, consumers, target_ids, pre)
     for t in tasks:
         t.run()
     # materialised vars become leaves: the graph behind them can be dropped
@@ -1048,6 +1050,50 @@ def _execute(ops, target_ids):
         if op.out._buf is not None:
             op.out._op = None
             op.inputs = []
+
+
+def _behind_products(tasks, ins, consumers, target_ids, pre):
+    """A product whose result only one element group reads runs with the group behind it, at the group's place: the values go
+    through the group where the product's kernel would store them (mjt_*_then).  With several such products the group goes with
+    the last; the others' results are in memory by then."""
+    made_by = {t.node.out.id: t for t in tasks if isinstance(t.node, (ConvUnit, ConvBwdDataUnit, MatmulUnit))
+               and (t.node.kind != "conv_bwd_x" or t.node.groups == 1)}
+    place = {id(t): i for i, t in enumerate(tasks)}
+    gone = set()
+    for t in tasks:
+        if not t.members or t.reduce is not None or t.node is not None:
+            continue
+        ids = {op.id for op in t.members}
+        shape = list(t.members[-1].out.shape)
+        best = None
+        for op in t.members:
+            reads = ins(op) if isinstance(op, BroadcastOp) else op.inputs
+            for u in reads:
+                p = made_by.get(u.id)
+                if p is None or id(p) in gone or list(u.shape) != shape or u.id in target_ids or u._buf is not None or getattr(u, "_stop_fuse", False) \
+                        or any(c.id not in ids for c in consumers.get(u.id, ())):
+                    continue
+                # every reader takes the result as it is, no broadcast of it
+                if any(isinstance(c, BroadcastOp) for c in consumers.get(u.id, ())):
+                    continue
+                if best is None or place[id(p)] > place[id(best)]:
+                    best = p
+        if best is None:
+            continue
+        gone.add(id(best))
+        t.reads = (t.reads - best.writes) | best.reads
+        t.run = _product_runner(best, t, consumers, target_ids, pre)
+    return [t for t in tasks if id(t) not in gone]
+
+
+def _product_runner(product, group, consumers, target_ids, pre):
+    alone, behind, members, unit = product.run, group.run, group.members, product.node
+
+    def run():
+        if not _run_group(members, consumers, target_ids, pre=pre, product=unit):
+            alone()
+            behind()
+    return run
 
 
 def _alloc_out(v):
@@ -1326,9 +1372,10 @@ def _run_single(op):
         raise MjtError(-2, "no kernel for op %r" % (op,))
 
 
-def _run_group(members, consumers, target_ids, reduce=None, pre=None, scatter=None, gathered=None):
+def _run_group(members, consumers, target_ids, reduce=None, pre=None, scatter=None, gathered=None, product=None):
     """One launch for a group of element / broadcast ops.  With `reduce` (the ReduceOp that consumes the
-    group's only result) the group runs as that reduce's prologue; returns False when the library does
+    group's only result) the group runs as that reduce's prologue, with `product` (a unit whose result only
+    the group reads) behind that product; returns False when the library does
     not take the group in that form (a tensor broadcast inside it), True otherwise."""
     lib = _libh()
     member_ids = {op.id for op in members}
@@ -1353,6 +1400,9 @@ def _run_group(members, consumers, target_ids, reduce=None, pre=None, scatter=No
         if gathered and u.id in gathered:
             i = add_var(_lib.VAR_GATHERED, u.dtype, ptr=_ptr_of(gathered[u.id].inputs[0]))
             index[key] = i
+            return i
+        if product is not None and u.id == product.out.id:
+            i = index[key] = add_var(_lib.VAR_PRODUCT, u.dtype)
             return i
         if u._op is None and u._host is not None and u.num == 1:
             # one-element host array: by-value kernel argument (ops/array_op.cc:56-60)
@@ -1427,6 +1477,29 @@ def _run_group(members, consumers, target_ids, reduce=None, pre=None, scatter=No
                 _cap.ptrs.append((varr, pv[0], pv[1], pv[2]))
             elif pv is not None:
                 _cap.scalars.append((varr, pv[0], pv[1]))
+    if product is not None:
+        a, b = product.inputs
+        rc = None
+        if isinstance(product, MatmulUnit):
+            ta, tb = _tensor_of(a), _tensor_of(b)
+            n = a.shape[-1] if product.trans[0] else a.shape[-2]
+            k = b.shape[-2] if product.trans[1] else b.shape[-1]
+            tc = _tensor(0, product.out.dtype, list(a.shape[:-2]) + [n, k])
+            rc = lib.mjt_matmul_then(ctypes.byref(ta), ctypes.byref(tb), ctypes.byref(tc), int(product.trans[0]), int(product.trans[1]), ctypes.byref(desc))
+        else:
+            ta, tb = _tensor_of(a), _tensor_of(b)
+            ty = _tensor(0, product.out.dtype, product.out.shape)
+            p = _lib.ConvParams(*product.params)
+            if isinstance(product, ConvUnit):
+                rc = lib.mjt_conv2d_meta_then(ctypes.byref(ta), ctypes.byref(tb), ctypes.byref(ty), ctypes.byref(p), product.groups, ctypes.byref(desc))
+            else:
+                rc = lib.mjt_conv2d_meta_dgrad_then(ctypes.byref(ta), ctypes.byref(tb), ctypes.byref(ty), ctypes.byref(p), ctypes.byref(desc))
+        if rc == _lib.ERR_UNSUPPORTED:
+            return False
+        _lib.check(rc)
+        stats["launches"] += 1
+        stats["fused_products"] += 1
+        return True
     if scatter is not None:
         rout, extras = scatter.out, scatter.inputs[1:]
         had_buf = rout._buf is not None

@@ -23,10 +23,10 @@ _SUMMED = ("float32", "float16", "bfloat16")
 
 class Task:
     """One step of an execution: an element group, a reduce (with its prologue group), or anything else."""
-    __slots__ = ("run", "members", "reduce", "reads", "writes", "place", "narrowed")
+    __slots__ = ("run", "members", "reduce", "reads", "writes", "place", "narrowed", "node")
 
-    def __init__(self, run, reads, writes, members=(), reduce=None):
-        self.run, self.members, self.reduce = run, list(members), reduce
+    def __init__(self, run, reads, writes, members=(), reduce=None, node=None):
+        self.run, self.members, self.reduce, self.node = run, list(members), reduce, node
         self.reads, self.writes = reads, writes                # ids of the vars in memory that it needs and leaves
         self.place, self.narrowed = None, None                 # narrowed: the var a column sum is cast to, instead of its own
 
