@@ -420,6 +420,10 @@ int mjt_conv2d_meta_then(const mjt_tensor* x, const mjt_tensor* w, const mjt_ten
 int mjt_conv2d_meta_dgrad_then(const mjt_tensor* dy, const mjt_tensor* w, const mjt_tensor* dx, const mjt_conv_params* p,
                                const mjt_fused_desc* desc);
 int mjt_matmul_then(const mjt_tensor* a, const mjt_tensor* b, const mjt_tensor* c, int trans_a, int trans_b, const mjt_fused_desc* desc);
+/* mjt_fused_reindex_reduce with a group behind it as well: the gradient of a pooling and the mask of the relu in front of it. */
+int mjt_fused_reindex_reduce_then(const mjt_fused_desc* desc, const mjt_tensor* x, int op, int n_indexes, const char* const* indexes,
+                                  int n_overflow_conditions, const char* const* overflow_conditions, int n_extras, const mjt_tensor* extras,
+                                  const mjt_fused_desc* behind);
 
 /* ---- index-expression helper ------------------------------------------
  * Parses one index expression (the language of opt/expr.h:38-143 restricted

@@ -1,4 +1,5 @@
-// Products with an element-wise group behind them: mjt_conv2d_meta_then, mjt_conv2d_meta_dgrad_then, mjt_matmul_then.
+// Products and scatters with an element-wise group behind them: mjt_conv2d_meta_then, mjt_conv2d_meta_dgrad_then, mjt_matmul_then,
+// mjt_fused_reindex_reduce_then.
 #include "common.h"
 
 namespace mjt {
@@ -7,6 +8,8 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
                void* packed);
 void conv_dgrad_impl(const mjt_tensor* dy, const mjt_tensor* w, const mjt_tensor* dx, const mjt_conv_params* p);
 void matmul_impl(const mjt_tensor* a, const mjt_tensor* b, const mjt_tensor* c, int trans_a, int trans_b, bool share_a);
+void fused_reindex_reduce_impl(const mjt_fused_desc* d, const mjt_tensor* x, int op, int n_idx, const char* const* idx, int n_ofc,
+                               const char* const* ofc, int n_ex, const mjt_tensor* ex);
 
 namespace {
 
@@ -63,6 +66,7 @@ EpilogueCode epilogue_code(int vec, int first, int dtype, int64_t covered) {
     EpilogueCode e;
     Waiting* w = t_waiting;
     if (!w || w->taken || t_preparing || dtype != w->dtype || covered != w->total) return e;
+    if (dtype != MJT_FLOAT32 && dtype != MJT_BFLOAT16 && dtype != MJT_FLOAT16) return e;          // (handed over as float32)
     while (vec > 1 && !fused_aligned(w->d, w->inputs, w->dims, vec)) vec /= 2;
     if (!fused_aligned(w->d, w->inputs, w->dims, vec)) return e;
     const FusedCode code(w->d, w->inputs, w->dims, vec, w->total >= (int64_t(1) << 31), first);
@@ -103,6 +107,15 @@ extern "C" int mjt_conv2d_meta_then(const mjt_tensor* x, const mjt_tensor* w, co
 extern "C" int mjt_conv2d_meta_dgrad_then(const mjt_tensor* dy, const mjt_tensor* w, const mjt_tensor* dx, const mjt_conv_params* p,
                                           const mjt_fused_desc* desc) {
     return mjt::guarded([&] { mjt::then(dx, desc, [&](const mjt_tensor* r) { mjt::conv_dgrad_impl(dy, w, r, p); }); });
+}
+extern "C" int mjt_fused_reindex_reduce_then(const mjt_fused_desc* desc, const mjt_tensor* x, int op, int n_indexes, const char* const* indexes,
+                                             int n_overflow_conditions, const char* const* overflow_conditions, int n_extras, const mjt_tensor* extras,
+                                             const mjt_fused_desc* behind) {
+    return mjt::guarded([&] {
+        mjt::then(x, behind, [&](const mjt_tensor* r) {
+            mjt::fused_reindex_reduce_impl(desc, r, op, n_indexes, indexes, n_overflow_conditions, overflow_conditions, n_extras, extras);
+        });
+    });
 }
 extern "C" int mjt_matmul_then(const mjt_tensor* a, const mjt_tensor* b, const mjt_tensor* c, int trans_a, int trans_b, const mjt_fused_desc* desc) {
     return mjt::guarded([&] { mjt::then(c, desc, [&](const mjt_tensor* r) { mjt::matmul_impl(a, b, r, trans_a, trans_b, false); }); });

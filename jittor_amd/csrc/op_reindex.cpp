@@ -365,6 +365,8 @@ bool try_window_scatter(Plan* plan, int op, const mjt_tensor* x, const mjt_tenso
     for (int i = 0; i < XD; i++) vk << "," << x->shape[i];
     vk << "," << y->shape[a_oh] << "," << y->shape[a_ow];
     if (sp) vk << "|P" << sp->key;
+    const EpilogueCode ep = epilogue_code(wvec, (int)args.size(), x->dtype, xn);
+    vk << ep.key;
     const std::string vkey = vk.str();
     JitKernel* kern = nullptr;
     {
@@ -396,7 +398,7 @@ bool try_window_scatter(Plan* plan, int op, const mjt_tensor* x, const mjt_tenso
         const int ta = x->dtype == MJT_FLOAT16 || x->dtype == MJT_BFLOAT16 ? MJT_FLOAT32 : x->dtype;
         std::ostringstream frag;
         frag << "#define TX " << dtype_cname(x->dtype) << "\n#define TACC " << dtype_cname(ta) << "\n#define index_t " << IT << "\n#define VEC " << wvec
-             << "\n#define NPARAM " << args.size() << "\n#define NB " << nb << "\n#define KH " << KH << "\n#define KW " << KW << "\n#define SH " << SH << "\n#define SW " << SW
+             << "\n#define NPARAM " << args.size() + ep.words.size() << "\n#define NB " << nb << "\n#define KH " << KH << "\n#define KW " << KW << "\n#define SH " << SH << "\n#define SW " << SW
              << "\n#define DH " << DH << "\n#define DW " << DW << "\n#define CH " << CH << "\n#define CW " << CW << "\n#define NCH " << NCH
              << "\n#define NCU " << columns(wvec) << "\n";
         // extents as literals: the lane's coordinates come from divisions by them
@@ -413,8 +415,8 @@ bool try_window_scatter(Plan* plan, int op, const mjt_tensor* x, const mjt_tenso
             h *= 1099511628211ull;
         }
         char name[96];
-        snprintf(name, sizeof(name), "mjt_window_scatter_%s_%016llx", mjt_op_name(op), (unsigned long long)h);
-        std::string src = std::string("#define ENTRY ") + name + "\n" + frag.str() + embedded_source("prelude.h") + "\n" +
+        snprintf(name, sizeof(name), "mjt_window_scatter_%s_%016llx%s", mjt_op_name(op), (unsigned long long)h, ep.suffix().c_str());
+        std::string src = ep.defs + "#define ENTRY " + name + "\n" + frag.str() + (ep.on ? "" : embedded_source("prelude.h")) + "\n" +
                           embedded_source("window_scatter.h") + "\n";
         kern = jit_get(src, name);
         std::lock_guard<std::mutex> lock(g_mu);
@@ -422,6 +424,8 @@ bool try_window_scatter(Plan* plan, int op, const mjt_tensor* x, const mjt_tenso
     }
     const int64_t blocks = (xn / wvec + 255) / 256;
     if (blocks >= (int64_t(1) << 31)) return false;
+    args.insert(args.end(), ep.words.begin(), ep.words.end());
+    epilogue_taken(ep);
     jit_launch(kern, (unsigned)blocks, 1, 256, 0, args);
     return true;
 }

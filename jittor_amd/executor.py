@@ -784,6 +784,13 @@ def _execute(ops, target_ids):
         for u in node.inputs:
             consumers.setdefault(u.id, []).append(node)
 
+    if flags["enable_product_fusion"]:
+        _masks_from_results(sched, consumers, target_ids)
+    consumers = {}
+    for node in sched:
+        for u in node.inputs:
+            consumers.setdefault(u.id, []).append(node)
+
     # ---- element ops whose result is only ever broadcast move behind the broadcast ------------
     # broadcast(f(a, b)) == f(broadcast(a), broadcast(b)): the small op then runs inside the kernel of the
     # broadcast's consumers (recomputed per element) instead of as a launch of its own, as the reference's
@@ -1042,7 +1049,7 @@ def _execute(ops, target_ids):
     if flags["enable_row_fusion"] and _profiler.active() is None:
         tasks = rowfuse.merge(tasks, ins, pre, consumers, target_ids, sys.modules[__name__]) or tasks
     if flags["enable_product_fusion"] and _profiler.active() is None:
-        tasks = _behind_products(tasks, ins, consumers, target_ids, pre)
+        tasks = _behind_products(tasks, ins, consumers, target_ids, pre, scatter_of)
     for t in tasks:
         t.run()
     # materialised vars become leaves: the graph behind them can be dropped
@@ -1052,12 +1059,53 @@ def _execute(ops, target_ids):
             op.inputs = []
 
 
-def _behind_products(tasks, ins, consumers, target_ids, pre):
-    """A product whose result only one element group reads runs with the group behind it, at the group's place: the values go
-    through the group where the product's kernel would store them (mjt_*_then).  With several such products the group goes with
+def _masks_from_results(sched, consumers, target_ids):
+    """relu's gradient reads its mask x > 0.  Where the relu's result y is in memory anyway, the mask is y > 0 there, and it need not be
+    stored beside y: y = x > 0 ? x : 0 is x or 0 exactly as x > 0 says, a NaN included.  Only for an x that a kernel of its own makes or
+    that is in memory: inside a group x may be wider than y, and a tiny x is 0 in y."""
+    producer = {node.out.id: node for node in sched}
+
+    def zero(v):
+        while isinstance(v._op, BroadcastOp) and v._buf is None:
+            v = v._op.inputs[0]
+        return v._op is None and v._host is not None and v.num == 1 and _scalar_value(v) in ((0.0, 0),)
+
+    place = {node.id: i for i, node in enumerate(sched)}
+    made = []                                                   # (behind which op, the new ones)
+    for t in sched:
+        if not isinstance(t, TernaryOp) or t.out._buf is not None:
+            continue
+        cond, x, other = t.inputs
+        c = producer.get(cond.id)
+        if not isinstance(c, BinaryOp) or c.op != "greater" or cond.id in target_ids or c.inputs[0] is not x or x.dtype != t.out.dtype \
+                or x.dtype not in _FLOAT_RANK or list(x.shape) != list(t.out.shape) or not zero(c.inputs[1]) or not zero(other):
+            continue
+        p = producer.get(x.id)
+        if p is not None and p.fusable:
+            continue
+        users = consumers.get(t.out.id, ())
+        if t.out.id not in target_ids and all(u.fusable or isinstance(u, ReduceOp) for u in users):
+            continue
+        later = [u for u in consumers.get(cond.id, ()) if u.fusable and place[u.id] > place[t.id]]
+        if not later:
+            continue
+        with core.no_grad():
+            mask = core.binary(t.out, 0.0, "greater")          # (with a zero of its own: the other's group need not hand its out)
+        spread = [u._op for u in mask._op.inputs if u is not t.out and u._op is not None]
+        made.append((t, spread + [mask._op]))
+        for u in later:
+            u.inputs = [mask if v is cond else v for v in u.inputs]
+    for t, ops in made:
+        at = sched.index(t) + 1
+        sched[at:at] = ops
+
+
+def _behind_products(tasks, ins, consumers, target_ids, pre, scatter_of):
+    """A product, or a scatter with a group in front of it, whose result only one element group reads runs with the group behind it, at the group's place: the values go
+    through the group where the kernel would store them (mjt_*_then).  With several such products the group goes with
     the last; the others' results are in memory by then."""
-    made_by = {t.node.out.id: t for t in tasks if isinstance(t.node, (ConvUnit, ConvBwdDataUnit, MatmulUnit))
-               and (t.node.kind != "conv_bwd_x" or t.node.groups == 1)}
+    made_by = {t.node.out.id: t for t in tasks if (isinstance(t.node, (ConvUnit, ConvBwdDataUnit, MatmulUnit))
+               and (t.node.kind != "conv_bwd_x" or t.node.groups == 1)) or (t.node is not None and t.node.id in scatter_of)}
     place = {id(t): i for i, t in enumerate(tasks)}
     gone = set()
     for t in tasks:
@@ -1082,15 +1130,19 @@ def _behind_products(tasks, ins, consumers, target_ids, pre):
             continue
         gone.add(id(best))
         t.reads = (t.reads - best.writes) | best.reads
-        t.run = _product_runner(best, t, consumers, target_ids, pre)
+        t.run = _product_runner(best, t, consumers, target_ids, pre, scatter_of.get(best.node.id))
     return [t for t in tasks if id(t) not in gone]
 
 
-def _product_runner(product, group, consumers, target_ids, pre):
+def _product_runner(product, group, consumers, target_ids, pre, scatter):
     alone, behind, members, unit = product.run, group.run, group.members, product.node
 
     def run():
-        if not _run_group(members, consumers, target_ids, pre=pre, product=unit):
+        if scatter is not None:
+            done = _run_group(scatter[0], consumers, target_ids, scatter=unit, gathered=scatter[1], pre=pre, behind=members)
+        else:
+            done = _run_group(members, consumers, target_ids, pre=pre, product=unit)
+        if not done:
             alone()
             behind()
     return run
@@ -1372,12 +1424,9 @@ def _run_single(op):
         raise MjtError(-2, "no kernel for op %r" % (op,))
 
 
-def _run_group(members, consumers, target_ids, reduce=None, pre=None, scatter=None, gathered=None, product=None):
-    """One launch for a group of element / broadcast ops.  With `reduce` (the ReduceOp that consumes the
-    group's only result) the group runs as that reduce's prologue, with `product` (a unit whose result only
-    the group reads) behind that product; returns False when the library does
-    not take the group in that form (a tensor broadcast inside it), True otherwise."""
-    lib = _libh()
+def _describe(members, consumers, target_ids, pre=None, gathered=None, product=None, virtual=False):
+    """The library's description of a group of element / broadcast ops, None where nobody reads a result of it.  `product`: the var
+    whose values a kernel hands to the group; `virtual`: the group's results are not written."""
     member_ids = {op.id for op in members}
     shape = members[-1].out.shape
     fvars, fops, prov = [], [], []
@@ -1401,7 +1450,7 @@ def _run_group(members, consumers, target_ids, reduce=None, pre=None, scatter=No
             i = add_var(_lib.VAR_GATHERED, u.dtype, ptr=_ptr_of(gathered[u.id].inputs[0]))
             index[key] = i
             return i
-        if product is not None and u.id == product.out.id:
+        if product is not None and u.id == product.id:
             i = index[key] = add_var(_lib.VAR_PRODUCT, u.dtype)
             return i
         if u._op is None and u._host is not None and u.num == 1:
@@ -1456,14 +1505,14 @@ def _run_group(members, consumers, target_ids, reduce=None, pre=None, scatter=No
         out = op.out
         used_outside = out.id in target_ids or any(c.id not in member_ids for c in consumers.get(out.id, ()))
         if used_outside:
-            oi = add_var(_lib.VAR_OUTPUT, out.dtype, ptr=None if reduce is not None or scatter is not None else _alloc_out(out))
+            oi = add_var(_lib.VAR_OUTPUT, out.dtype, ptr=None if virtual else _alloc_out(out))
             outputs.append(out)
         else:
             oi = add_var(_lib.VAR_INTERMEDIATE, out.dtype)
         index[(out.id, 0)] = oi
         add_op(op, ins, oi)
     if not outputs:
-        return True
+        return None
     desc = _lib.FusedDesc()
     desc.ndim = len(shape)
     for i, s in enumerate(shape):
@@ -1477,6 +1526,19 @@ def _run_group(members, consumers, target_ids, reduce=None, pre=None, scatter=No
                 _cap.ptrs.append((varr, pv[0], pv[1], pv[2]))
             elif pv is not None:
                 _cap.scalars.append((varr, pv[0], pv[1]))
+    return desc
+
+
+def _run_group(members, consumers, target_ids, reduce=None, pre=None, scatter=None, gathered=None, product=None,
+               behind=None):
+    """One launch for a group of element / broadcast ops.  With `reduce` (the ReduceOp that consumes the
+    group's only result) the group runs as that reduce's prologue, with `product` (a unit whose result only
+    the group reads) behind that product; `behind`: the group that runs behind the scatter; returns False when the library does
+    not take the group in that form (a tensor broadcast inside it), True otherwise."""
+    lib = _libh()
+    desc = _describe(members, consumers, target_ids, pre, gathered, product and product.out, reduce is not None or scatter is not None)
+    if desc is None:
+        return True
     if product is not None:
         a, b = product.inputs
         rc = None
@@ -1498,6 +1560,21 @@ def _run_group(members, consumers, target_ids, reduce=None, pre=None, scatter=No
             return False
         _lib.check(rc)
         stats["launches"] += 1
+        stats["fused_products"] += 1
+        return True
+    if behind is not None:
+        extras = scatter.inputs[1:]
+        after = _describe(behind, consumers, target_ids, pre, None, scatter.out)
+        tx = _tensor(0, scatter.out.dtype, scatter.out.shape)
+        ex = _tensor_array(extras)
+        rc = lib.mjt_fused_reindex_reduce_then(ctypes.byref(desc), ctypes.byref(tx), _lib.OP_CODE[scatter.op], len(scatter.indexes),
+                                               _lib.c_strings(scatter.indexes), len(scatter.overflow_conditions),
+                                               _lib.c_strings(scatter.overflow_conditions), len(extras), ex, ctypes.byref(after))
+        if rc == _lib.ERR_UNSUPPORTED:
+            return False
+        _lib.check(rc)
+        stats["launches"] += 1
+        stats["fused_scatters"] += 1
         stats["fused_products"] += 1
         return True
     if scatter is not None:

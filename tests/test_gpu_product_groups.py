@@ -27,7 +27,7 @@ def _both(build, fused=1):
                 got = [v.raw() for v in vs]
                 if on in out:
                     for a, b in zip(out[on], got):
-                        assert np.array_equal(a, b)
+                        assert np.array_equal(a.view(np.uint8), b.view(np.uint8))
                 out[on] = [a.copy() for a in got]
             assert (E.stats["fused_products"] - before == 3 * fused) if on else (E.stats["fused_products"] == before)
         finally:
@@ -35,6 +35,13 @@ def _both(build, fused=1):
     for i, (a, b) in enumerate(zip(out[True], out[False])):
         assert a.shape == b.shape and np.array_equal(a.view(np.uint8), b.view(np.uint8)), "result %d" % i
     return out[True]
+
+
+def _taken(build):
+    """How many groups the graph's kernels take along."""
+    before = E.stats["fused_products"]
+    jt.sync(build())
+    return E.stats["fused_products"] - before
 
 
 def _var(rng, shape, dt, scale=1.0):
@@ -93,14 +100,10 @@ def test_linear(gpu, m, k, n, dt):
     x, w, b = _var(rng, [m, k], dt), _var(rng, [n, k], dt, k ** -0.5), _var(rng, [n], dt)
     x2, w2, rows = _var(rng, [k, m], dt), _var(rng, [k, n], dt, k ** -0.5), _var(rng, [m, 1], dt)
 
-    def count(build):
-        """Whether the product's route takes a group: not where a sum is cut into slices, nor the kernel without MFMAs."""
-        before = E.stats["fused_products"]
-        jt.sync(build())
-        return E.stats["fused_products"] - before
+    # (not where a sum is cut into slices, nor on the kernel without MFMAs)
     for build in (lambda: [jt.nn.relu(jt.nn.linear(x, w, b))], lambda: [jt.nn.matmul(x, w2) * rows],
                   lambda: [jt.nn.linear(x, w, b).sigmoid() * jt.nn.matmul(x, w2)]):
-        _both(build, count(build))
+        _both(build, _taken(build))
 
 
 def test_batches_and_large_tiles(gpu):
@@ -131,6 +134,42 @@ def test_values_that_are_not_finite(gpu):
         a, b = vx.cast(dt), vw.cast(dt)
         jt.sync([a, b])
         _both(lambda: [jt.nn.relu(jt.nn.matmul(a, b)), ])
+
+
+# windows that overlap or not, vectors of 4, 2 and 1 elements of a row, a mean's and a maximum's gradient
+@pytest.mark.parametrize("shape,k,st,pad,op", [((2, 24, 33, 32), 3, 2, 1, "maximum"), ((3, 16, 18, 22), 2, 2, 0, "maximum"), ((2, 16, 25, 25), 3, 1, 1, "mean"), ((2, 9, 16, 20), 3, 3, 0, "mean")])
+@pytest.mark.parametrize("dt", ["float32", "bfloat16", "float16"])
+def test_pooling_gradients(gpu, shape, k, st, pad, op, dt):
+    """relu, pooling and their gradients: the mask behind the pooling's gradient, read from the relu's result."""
+    rng = np.random.default_rng(15)
+    x, w = _var(rng, [shape[0], 8] + list(shape[2:]), dt), _var(rng, [shape[1], 8, 3, 3], dt, 0.2)
+    o = [(d + 2 * pad - k) // st + 1 for d in shape[2:]]
+    g = _var(rng, [shape[0], shape[1]] + o, dt)
+
+    def step():
+        y = jt.nn.pool(jt.nn.relu(jt.nn.conv2d(x, w, padding=1)), k, op, pad, st)
+        return [y] + list(jt.grad((y * g).sum(), [w]))
+    fused = _taken(step)
+    assert fused == 2 or (op == "mean" and fused >= 1)
+    _both(step, fused)
+
+
+@pytest.mark.parametrize("dt", ["float32", "bfloat16", "float16"])
+def test_masks_of_tiny_and_undefined_values(gpu, dt):
+    """y > 0 is x > 0 where x is rounded to y's type already, the smallest numbers and NaN included."""
+    tiny = {"float32": [1e-45, -1e-45, 1e-38], "bfloat16": [1e-38, -1e-38, 9.2e-41], "float16": [6e-8, -6e-8, 3e-5]}[dt]
+    v = np.array(tiny + [0.0, -0.0, np.inf, -np.inf, np.nan, 1.0, -1.0] + [2.0] * 6, np.float32)
+    eye = np.eye(128, dtype=np.float32)
+    a = np.zeros((128, 128), np.float32)
+    a[:16, 0], a[16:32, 5] = v, v[::-1]
+    va, ve, g = jt.array(a).cast(dt), jt.array(eye).cast(dt), jt.array(eye * 3 + 1).cast(dt)
+    jt.sync([va, ve, g])
+
+    def step():
+        y = jt.nn.relu(jt.nn.matmul(va, ve))
+        z = jt.nn.matmul(y, ve)
+        return [z] + list(jt.grad((z * g).sum(), [ve, va]))
+    _both(step, _taken(step))
 
 
 def test_a_product_that_others_read_stays(gpu):
