@@ -359,6 +359,13 @@ int mjt_conv2d_meta_dgrad(const mjt_tensor* dy, const mjt_tensor* w, const mjt_t
 int mjt_conv2d_meta_dgrad_depthwise(const mjt_tensor* dy, const mjt_tensor* w, const mjt_tensor* dx,
                                     const mjt_conv_params* p, int groups);
 
+/* Both gradients of a depthwise convolution of stride 1 without dilation, with
+ * as many output as input channels: dx and dw as the two entry points around
+ * this one give them, in one kernel that reads dy and x once each.  Other
+ * convolutions return MJT_ERR_UNSUPPORTED. */
+int mjt_conv2d_meta_backward_depthwise(const mjt_tensor* x, const mjt_tensor* dy, const mjt_tensor* w, const mjt_tensor* dx,
+                                       const mjt_tensor* dw, const mjt_conv_params* p, int groups);
+
 /* Weight gradient of the same convolution (the pattern
  * reindex(x) * broadcast(dy) -> reduce.add over (n, oh, ow) that jt.grad builds;
  * opt/tuner/conv_tuner.cc:375-397 relays it to a backward-w library op,

@@ -93,7 +93,7 @@ EXPORTS = ["mjt_init", "mjt_shutdown", "mjt_last_error", "mjt_get_device_info",
            "mjt_event_destroy", "mjt_reduce", "mjt_reduce_static", "mjt_reindex", "mjt_reindex_reduce",
            "mjt_fused_elementwise", "mjt_fused_reduce", "mjt_fused_rows", "mjt_conv2d_meta", "mjt_conv2d_meta_pack", "mjt_conv2d_meta_packed", "mjt_conv2d_meta_grouped", "mjt_conv2d_meta_dgrad", "mjt_conv2d_meta_dgrad_depthwise", "mjt_conv2d_meta_wgrad", "mjt_conv2d_meta_wgrad_grouped",
            "mjt_reindex_then_reduce", "mjt_fused_reindex_reduce", "mjt_matmul", "mjt_matmul_available",
-           "mjt_conv2d_meta_then", "mjt_conv2d_meta_dgrad_then", "mjt_matmul_then", "mjt_fused_reindex_reduce_then",
+           "mjt_conv2d_meta_backward_depthwise", "mjt_conv2d_meta_then", "mjt_conv2d_meta_dgrad_then", "mjt_matmul_then", "mjt_fused_reindex_reduce_then",
            "mjt_expr_affine", "mjt_where_count", "mjt_where",
            "mjt_record_begin", "mjt_record_end", "mjt_record_relocate", "mjt_record_launch", "mjt_record_free",
            "mjt_jit_stats", "mjt_last_kernel"]
@@ -153,6 +153,7 @@ def load():
     lib.mjt_conv2d_meta_dgrad.argtypes = [ctypes.POINTER(Tensor), ctypes.POINTER(Tensor), ctypes.POINTER(Tensor),
                                           ctypes.POINTER(ConvParams)]
     lib.mjt_conv2d_meta_dgrad_depthwise.argtypes = lib.mjt_conv2d_meta_grouped.argtypes
+    lib.mjt_conv2d_meta_backward_depthwise.argtypes = [ctypes.POINTER(Tensor)] * 5 + [ctypes.POINTER(ConvParams), ctypes.c_int]
     lib.mjt_conv2d_meta_wgrad.argtypes = [ctypes.POINTER(Tensor), ctypes.POINTER(Tensor), ctypes.POINTER(Tensor),
                                           ctypes.POINTER(ConvParams)]
     lib.mjt_conv2d_meta_wgrad_grouped.argtypes = [ctypes.POINTER(Tensor), ctypes.POINTER(Tensor), ctypes.POINTER(Tensor),

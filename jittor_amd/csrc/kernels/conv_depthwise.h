@@ -12,12 +12,21 @@
 //         and, for a strided convolution, the rows and columns of dy UH and UW apart in LDS with zeros between them.
 // MODE 1: partial[slice][ko][tap] = sum over the slice's images and all positions of dy * x; the slices are added up by
 //         a reduce launch.
+// MODE 2: both gradients of a convolution of stride 1 without dilation at once.  dy is staged as for the input gradient; the lane that makes a
+//         strip of dx has the same strip of x in registers and multiplies the window's rows with it as well, which gives the weight
+//         gradient's terms: dy is read once, x once, dx written once.  Cells around dy are zeros that are no terms of the weight
+//         gradient, harmless unless x is infinite there; and a zero around x times an infinite dy is a term that this way does not
+//         see.  Either leaves some sum of the workgroup not finite, and then its sums are taken again, term by term.
+//         us with the fold, input and weight gradient / both: float32 3x3 32 x 128 x 56 x 56 49.8 / 37.0 (154 MB: 24.5 at the rate of a copy),
+//         64 x 256 x 14 x 14 21.6 / 19.2, 8 x 32 x 112 x 112 25.3 / 18.4, 4 x 512 x 7 x 7 7.9 / 5.2, 5x5 64 x 24 x 56 x 56 34.0 / 26.1; bfloat16 3x3
+//         32 x 128 x 56 x 56 35.1 / 26.3.  (x asked for ahead of the window, like dy: 148 registers instead of 126, three workgroups a
+//         unit instead of four, 39.9; held to 128 registers it spills, 46.6.)
 // Supplied by the host: TIN, TOUT, the geometry (H_, W_ of the staged planes, OH_, OW_ of the planes a lane's strips lie
 // in, R_, S_, SH, SW, PH, PW, DH, DW), UH, UW, MULT, K_ (planes per image of y / dy), TH (rows of a plane per
 // workgroup, NTILE such tiles per plane), PPW (planes, or images of one channel in MODE 1, staged together), VEC (elements
 // per staging load), CW, RS, STVEC (elements per access of y / dy).
 
-struct Params { void* a[6]; };   // MODE 0: x, w, y, planes of y;  MODE 1: x, dy, partial, images, images per slice
+struct Params { void* a[7]; };   // MODE 0: x, w, y, planes of y;  MODE 1: x, dy, partial, images, images per slice;  MODE 2: dy, x, partial, images, images per slice, w, dx
 
 constexpr int NV = ((CW - 1) * SW + (S_ - 1) * DW + 1 + 3) / 4;        // 16-byte pieces of a strip's row
 constexpr int NCG = (OW_ + CW - 1) / CW;                               // column groups of a row
@@ -160,6 +169,68 @@ extern "C" __global__ __launch_bounds__(256) void ENTRY(Params p) {
     float acc[R_ * S_];
 #pragma unroll
     for (int k = 0; k < R_ * S_; k++) acc[k] = 0.0f;
+#if MODE == 2
+    const TIN* __restrict__ wp = (const TIN*)p.a[5];
+    TOUT* __restrict__ dxp = (TOUT*)p.a[6];
+    float w[R_ * S_];
+#pragma unroll
+    for (int k = 0; k < R_ * S_; k++) w[k] = (float)wp[ko * (R_ * S_) + R_ * S_ - 1 - k];
+    auto both = [&](long long n, int count, int oh0) {
+        for (int t = threadIdx.x; t < TASKS; t += 256) {
+            const int pl = t / (NST * NCG), rest = t - pl * (NST * NCG), row = rest / NCG, cg = rest - row * NCG;
+            if (pl >= count) break;
+            const long long at = ((n + pl) * K_ + ko) * (OH_ * OW_);
+            float xv[RS][CW], dx[RS][CW];
+#pragma unroll
+            for (int ro = 0; ro < RS; ro++) {
+                const int oh = oh0 + row * RS + ro;
+                const bool row_in = row * RS + ro < TH && oh < OH_;
+#pragma unroll
+                for (int j = 0; j < CW; j += STVEC) {                   // out of range: the first element, replaced by zero
+                    const bool in = row_in && cg * CW + j < OW_;
+                    mjt_pack<TIN, STVEC> v;
+                    mjt_load(v, dyp + at + (in ? oh * OW_ + cg * CW + j : 0));
+#pragma unroll
+                    for (int k = 0; k < STVEC; k++) {
+                        xv[ro][j + k] = in ? (float)v.v[k] : 0.0f;
+                        dx[ro][j + k] = 0.0f;
+                    }
+                }
+            }
+            mjt_dw_rows(pl, row, cg, [&](int lr, const float* d) {
+#pragma unroll
+                for (int ro = 0; ro < RS; ro++)
+#pragma unroll
+                    for (int r = 0; r < R_; r++)
+                        if (ro + r == lr) {
+#pragma unroll
+                            for (int s = 0; s < S_; s++)
+#pragma unroll
+                                for (int j = 0; j < CW; j++) {
+                                    dx[ro][j] = dx[ro][j] + d[j + s] * w[r * S_ + s];
+                                    acc[(R_ - 1 - r) * S_ + S_ - 1 - s] = acc[(R_ - 1 - r) * S_ + S_ - 1 - s] + d[j + s] * xv[ro][j];
+                                }
+                        }
+            });
+            TOUT* const dst = dxp + at;
+#pragma unroll
+            for (int ro = 0; ro < RS; ro++) {
+                const int oh = oh0 + row * RS + ro;
+                if (row * RS + ro < TH && oh < OH_) {
+#pragma unroll
+                    for (int j = 0; j < CW; j += STVEC) {
+                        if (cg * CW + j < OW_) {
+                            mjt_pack<TOUT, STVEC> o;
+#pragma unroll
+                            for (int k = 0; k < STVEC; k++) o.v[k] = (TOUT)dx[ro][j + k];
+                            mjt_store(dst + oh * OW_ + cg * CW + j, o);
+                        }
+                    }
+                }
+            }
+        }
+    };
+#else
     auto sums = [&](long long n, int count, int oh0) {
         for (int t = threadIdx.x; t < TASKS; t += 256) {
             const int pl = t / (NST * NCG), rest = t - pl * (NST * NCG), strip = rest / NCG, cg = rest - strip * NCG;
@@ -202,6 +273,7 @@ extern "C" __global__ __launch_bounds__(256) void ENTRY(Params p) {
             });
         }
     };
+#endif
     auto images = [&](long long n) { return n1 - n < PPW ? (n1 > n ? (int)(n1 - n) : 0) : PPW; };
     const TIN* __restrict__ xc = xp + (ko / MULT) * (H_ * W_);
     const long long istride = (long long)C * (H_ * W_);
@@ -216,7 +288,11 @@ extern "C" __global__ __launch_bounds__(256) void ENTRY(Params p) {
             __syncthreads();
             const long long next = n + PPW < n1 ? n + PPW : n;
             mjt_dw_load(v, xc + next * istride, istride, images(next), 0, 0);
+#if MODE == 2
+            both(n, images(n), 0);
+#else
             sums(n, images(n), 0);
+#endif
         }
     } else {
         for (long long n = slice * ips; n < n1; n += PPW)
@@ -226,11 +302,44 @@ extern "C" __global__ __launch_bounds__(256) void ENTRY(Params p) {
                     mjt_dw_clear();
                     __syncthreads();
                 }
+#if MODE == 2
+                mjt_dw_stage(xc + n * istride, istride, images(n), tl * TH);
+                __syncthreads();
+                both(n, images(n), tl * TH);
+#else
                 mjt_dw_stage(xc + n * istride, istride, images(n), tl * TH);
                 __syncthreads();
                 sums(n, images(n), tl * TH);
+#endif
             }
     }
+#if MODE == 2
+    {
+        float z = 0.0f;                                                 // not zero if any sum is not finite
+#pragma unroll
+        for (int k = 0; k < R_ * S_; k++) z = z + acc[k] * 0.0f;
+        if (__syncthreads_or(!(z == 0.0f))) {
+            constexpr int PADH = R_ - 1 - PH, PADW = S_ - 1 - PW;       // the convolution's own padding
+#pragma unroll
+            for (int k = 0; k < R_ * S_; k++) acc[k] = 0.0f;
+            for (long long n = slice * ips; n < n1; n++) {
+                const TIN* const d = xp + (n * K_ + ko) * (H_ * W_);
+                const TIN* const x = dyp + (n * K_ + ko) * (OH_ * OW_);
+                for (int i = threadIdx.x; i < H_ * W_; i += 256) {
+                    const int oh = i / W_, ow = i - oh * W_;
+                    const float dv = (float)d[i];
+#pragma unroll
+                    for (int k = 0; k < R_ * S_; k++) {
+                        const int h = oh - PADH + k / S_, c = ow - PADW + k % S_;
+                        const bool in = h >= 0 && h < OH_ && c >= 0 && c < OW_;
+                        const float xv = (float)x[in ? h * OW_ + c : 0];
+                        acc[k] = acc[k] + dv * (in ? xv : 0.0f);
+                    }
+                }
+            }
+        }
+    }
+#endif
     __shared__ float fold[4][R_ * S_];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll

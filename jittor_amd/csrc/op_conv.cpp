@@ -137,8 +137,8 @@ JitKernel* depthwise_kernel(int mode, const DepthwiseShape& g, const DepthwisePl
     JitKernel* k = cached(key.str());
     if (k) return k;
     std::ostringstream name;
-    name << (mode ? "mjt_conv_wgrad_direct_" : "mjt_conv_direct_") << mjt_dtype_name(tin);
-    if (!mode) name << "_" << mjt_dtype_name(tout);
+    name << (mode == 2 ? "mjt_conv_backward_direct_" : mode ? "mjt_conv_wgrad_direct_" : "mjt_conv_direct_") << mjt_dtype_name(tin);
+    if (mode != 1) name << "_" << mjt_dtype_name(tout);
     name << "_depthwise_" << g.H << "x" << g.W << "_r" << g.R << "x" << g.S << "_s" << g.SH << "x" << g.SW << "_p" << g.PH << "x" << g.PW << "_d" << g.DH
          << "x" << g.DW << "_u" << g.UH << "x" << g.UW << (g.flip ? "_flip" : "") << (g.mult > 1 ? "_m" + std::to_string(g.mult) : std::string()) << "_g" << g.K / g.mult;
     std::ostringstream src;
@@ -164,7 +164,7 @@ bool depthwise_run(const DepthwiseShape& g, const mjt_tensor* x, const mjt_tenso
     const int64_t blocks = (planes + q.PPW - 1) / q.PPW * q.NTILE;
     if (blocks >= (int64_t(1) << 31)) return false;
     JitKernel* k = depthwise_kernel(0, g, q, x->dtype, y->dtype);
-    std::vector<uint64_t> a{bits_of_ptr(x->ptr), bits_of_ptr(w->ptr), bits_of_ptr(y->ptr), (uint64_t)planes, 0, 0};
+    std::vector<uint64_t> a{bits_of_ptr(x->ptr), bits_of_ptr(w->ptr), bits_of_ptr(y->ptr), (uint64_t)planes, 0, 0, 0};
     jit_launch(k, (unsigned)blocks, 1, 256, 0, a);
     return true;
 }
@@ -885,7 +885,7 @@ static void conv_wgrad_direct(const mjt_tensor* x, const mjt_tensor* dy, const m
             JitKernel* k = depthwise_kernel(1, g, q, x->dtype, x->dtype);
             const bool in_place = slices == 1 && dw->dtype == MJT_FLOAT32;
             void* part = in_place ? dw->ptr : wgrad_partials((size_t)slices * (size_t)numel(dw) * 4);
-            std::vector<uint64_t> a{bits_of_ptr(x->ptr), bits_of_ptr(dy->ptr), bits_of_ptr(part), (uint64_t)N, (uint64_t)ips, 0};
+            std::vector<uint64_t> a{bits_of_ptr(x->ptr), bits_of_ptr(dy->ptr), bits_of_ptr(part), (uint64_t)N, (uint64_t)ips, 0, 0};
             jit_launch(k, (unsigned)(slices * K), 1, 256, 0, a);
             if (!in_place) fold_wgrad_slices(part, slices, dw);
             set_last_kernel(k->name.c_str());
@@ -1546,7 +1546,60 @@ void conv_dgrad_depthwise(const mjt_tensor* dy, const mjt_tensor* w, const mjt_t
     const DepthwiseShape g{OH, OW, H, W, R, S, 1, 1, p->dil_h * (R - 1) - p->pad_h, p->dil_w * (S - 1) - p->pad_w, p->dil_h, p->dil_w, p->stride_h, p->stride_w, C, 1, true};
     if (numel(dy) == 0 || !depthwise_run(g, dy, w, dx)) MJT_FAIL(MJT_ERR_UNSUPPORTED, "conv dgrad: this shape takes another route");
 }
+
+// Both gradients of a depthwise convolution of stride 1 with as many output as input channels, in one kernel over dy and x.
+void conv_backward_depthwise(const mjt_tensor* x, const mjt_tensor* dy, const mjt_tensor* w, const mjt_tensor* dx, const mjt_tensor* dw, const mjt_conv_params* p,
+                             int64_t G) {
+    require_init();
+    check_tensor(x, "conv backward x");
+    check_tensor(dy, "conv backward dy");
+    check_tensor(w, "conv backward w");
+    check_tensor(dx, "conv backward dx");
+    check_tensor(dw, "conv backward dw");
+    MJT_CHECK(p, "conv backward: null parameters");
+    MJT_CHECK(x->ndim == 4 && dy->ndim == 4 && w->ndim == 4 && dx->ndim == 4 && dw->ndim == 4, "conv backward: every tensor must have rank 4");
+    MJT_CHECK(x->dtype == dy->dtype && x->dtype == w->dtype && (x->dtype == MJT_BFLOAT16 || x->dtype == MJT_FLOAT16 || x->dtype == MJT_FLOAT32),
+              "conv backward: x, dy and w must share one of float32 / bfloat16 / float16");
+    MJT_CHECK((dx->dtype == MJT_FLOAT32 || dx->dtype == x->dtype) && (dw->dtype == MJT_FLOAT32 || dw->dtype == x->dtype), "conv backward: dx and dw must be float32 or the operands' dtype");
+    const int64_t N = x->shape[0], C = x->shape[1], H = x->shape[2], W = x->shape[3], R = w->shape[2], S = w->shape[3], OH = dy->shape[2], OW = dy->shape[3];
+    for (int i = 0; i < 4; i++) MJT_CHECK(dx->shape[i] == x->shape[i] && dw->shape[i] == w->shape[i], "conv backward: dx and dw must have the shapes of x and w");
+    MJT_CHECK(dy->shape[0] == N && dy->shape[1] == w->shape[0], "conv backward: dy " << shape_str(dy) << " does not follow from x " << shape_str(x) << " and w " << shape_str(w));
+    if (G < 2 || C != G || w->shape[0] != G || w->shape[1] != 1 || p->stride_h != 1 || p->stride_w != 1 || p->dil_h != 1 || p->dil_w != 1)
+        MJT_FAIL(MJT_ERR_UNSUPPORTED, "conv backward: only depthwise convolutions of stride 1 without dilation, with as many output as input channels");
+    MJT_CHECK(OH == H + 2 * p->pad_h - R + 1 && OW == W + 2 * p->pad_w - S + 1, "conv backward: dy " << shape_str(dy) << " does not follow from x " << shape_str(x));
+    if (numel(x) == 0 || numel(dy) == 0 || p->pad_h < 0 || p->pad_w < 0 || p->pad_h > R - 1 || p->pad_w > S - 1 || getenv("MJT_NO_FASTPATH"))
+        MJT_FAIL(MJT_ERR_UNSUPPORTED, "conv backward: this shape takes another route");
+    const int64_t cus = ctx().dry_run || ctx().prop.multiProcessorCount <= 0 ? 256 : ctx().prop.multiProcessorCount;
+    // slices of images: as many workgroups as the compute units hold at once, four each, or two where more taps take more registers (us
+    // with 2 / 3 / 4 / 6 a unit: 32 x 128 x 56 x 56 3x3 float32 38.0 / 39.3 / 37.0 / 38.6, 32 x 96 x 31 x 29 19.1 / 17.6 / 18.5 / 21.2; 5x5 64 x 24 x 56 x 56
+    // 26.1 / 33.7 / 34.3 / 39.2, 64 x 512 x 14 x 14 30.7 / 30.2 / 39.8 / 49.0)
+    int64_t slices = (R * S <= 9 ? 4 : 2) * cus / C;
+    if (slices < 1) slices = 1;
+    if (slices > N) slices = N;
+    if (N * OH * OW < 2048) slices = 1;
+    const int64_t ips = (N + slices - 1) / slices;
+    slices = (N + ips - 1) / ips;
+    const DepthwiseShape g{OH, OW, H, W, R, S, 1, 1, R - 1 - p->pad_h, S - 1 - p->pad_w, 1, 1, 1, 1, C, 1, true};
+    DepthwisePlan q;
+    // (strips are read from x and written to dx: vectors that suit both)
+    const int wide = std::max(dtype_size(x->dtype), dtype_size(dx->dtype));
+    const void* strips = (const void*)((uintptr_t)x->ptr | (uintptr_t)dx->ptr);
+    if (slices * C >= (int64_t(1) << 31) || !depthwise_plan(g, dtype_size(dy->dtype), wide, dy->ptr, strips, int64_t(1) << 40, ips, &q))
+        MJT_FAIL(MJT_ERR_UNSUPPORTED, "conv backward: this shape takes another route");
+    JitKernel* k = depthwise_kernel(2, g, q, x->dtype, dx->dtype);
+    const bool in_place = slices == 1 && dw->dtype == MJT_FLOAT32;
+    void* part = in_place ? dw->ptr : wgrad_partials((size_t)slices * (size_t)numel(dw) * 4);
+    std::vector<uint64_t> a{bits_of_ptr(dy->ptr), bits_of_ptr(x->ptr), bits_of_ptr(part), (uint64_t)N, (uint64_t)ips, bits_of_ptr(w->ptr), bits_of_ptr(dx->ptr)};
+    jit_launch(k, (unsigned)(slices * C), 1, 256, 0, a);
+    if (!in_place) fold_wgrad_slices(part, slices, dw);
+    set_last_kernel(k->name.c_str());
+}
 }  // namespace mjt
+
+extern "C" int mjt_conv2d_meta_backward_depthwise(const mjt_tensor* x, const mjt_tensor* dy, const mjt_tensor* w, const mjt_tensor* dx, const mjt_tensor* dw,
+                                                  const mjt_conv_params* p, int groups) {
+    return mjt::guarded([&] { mjt::conv_backward_depthwise(x, dy, w, dx, dw, p, groups); });
+}
 
 extern "C" int mjt_conv2d_meta_dgrad_depthwise(const mjt_tensor* dy, const mjt_tensor* w, const mjt_tensor* dx, const mjt_conv_params* p, int groups) {
     return mjt::guarded([&] { mjt::conv_dgrad_depthwise(dy, w, dx, p, groups); });

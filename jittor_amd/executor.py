@@ -1050,6 +1050,8 @@ def _execute(ops, target_ids):
         tasks = rowfuse.merge(tasks, ins, pre, consumers, target_ids, sys.modules[__name__]) or tasks
     if flags["enable_product_fusion"] and _profiler.active() is None:
         tasks = _behind_products(tasks, ins, consumers, target_ids, pre, scatter_of)
+    if _profiler.active() is None:
+        tasks = _depthwise_gradients(tasks)
     for t in tasks:
         t.run()
     # materialised vars become leaves: the graph behind them can be dropped
@@ -1057,6 +1059,56 @@ def _execute(ops, target_ids):
         if op.out._buf is not None:
             op.out._op = None
             op.inputs = []
+
+
+def _depthwise_gradients(tasks):
+    """The two gradients of a depthwise convolution of stride 1 read the same dy: one call makes both, at the place of the first
+    of the two where the other's operands are there by then."""
+    writer = {v: i for i, t in enumerate(tasks) for v in t.writes}
+    weights = [(i, t) for i, t in enumerate(tasks) if isinstance(t.node, ConvBwdWeightUnit) and t.node.groups > 1]
+    gone = set()
+    for i, t in enumerate(tasks):
+        d = t.node
+        if not isinstance(d, ConvBwdDataUnit) or d.groups == 1 or d.params[:2] != (1, 1) or d.params[4:] != (1, 1):
+            continue
+        dy, w = d.inputs
+        if not (d.groups == w.shape[0] == d.out.shape[1] and w.shape[1] == 1):
+            continue
+        for j, u in weights:
+            g = u.node
+            if id(u) in gone or g.inputs[1] is not dy or g.params != d.params or g.groups != d.groups or list(g.out.shape) != list(w.shape) \
+                    or list(g.inputs[0].shape) != list(d.out.shape):
+                continue
+            first, other = (t, u) if i < j else (u, t)
+            if any(writer.get(v, -1) >= min(i, j) for v in other.reads):
+                continue
+            first.run = _both_gradients(d, g, t.run, u.run)
+            first.reads, first.writes = first.reads | other.reads, first.writes | other.writes
+            gone.add(id(other))
+            break
+    return [t for t in tasks if id(t) not in gone]
+
+
+def _both_gradients(data, weight, run_data, run_weight):
+    def run():
+        x, dy, w = weight.inputs[0], data.inputs[0], data.inputs[1]
+        had = [v._buf is not None for v in (data.out, weight.out)]
+        tx, td, tw = _tensor_of(x), _tensor_of(dy), _tensor_of(w)
+        tdx, tdw = (_tensor(_alloc_out(v), v.dtype, v.shape) for v in (data.out, weight.out))
+        p = _lib.ConvParams(*data.params)
+        rc = _libh().mjt_conv2d_meta_backward_depthwise(ctypes.byref(tx), ctypes.byref(td), ctypes.byref(tw), ctypes.byref(tdx), ctypes.byref(tdw),
+                                                        ctypes.byref(p), data.groups)
+        if rc == 0:
+            stats["launches"] += 1
+            return
+        if rc != _lib.ERR_UNSUPPORTED:
+            _lib.check(rc)
+        for v, h in zip((data.out, weight.out), had):
+            if not h:
+                v._buf = None
+        run_data()
+        run_weight()
+    return run
 
 
 def _masks_from_results(sched, consumers, target_ids):
