@@ -94,7 +94,7 @@ typedef unsigned short TIN;
 #define CONV 0
 #endif
 #ifndef SLICED
-#define SLICED 0                 // 1: workgroup (tile, slice) sums stages slice * a[9] .. of K into its own float32 C, a[11] apart
+#define SLICED 0                 // 1: workgroup (tile, slice) sums stages slice * a[9] .. of K into its own float32 C (or y), a[11] apart
 #endif
 // A convolution's sum is known here, and images have few channels: a single stage takes one buffer, so that eight workgroups share a
 // compute unit instead of four, two stages one register set, and the loop of whole stages is left out where it would not be entered.
@@ -747,7 +747,7 @@ extern "C" __global__ __launch_bounds__(NTHR) void ENTRY(Params p) {
             auto row_of = [&](int e) { return m0 + wm * 32 * FI + i * 32 + 8 * (e / 4) + 4 * (lane >> 5) + (e & 3); };
             auto place_of = [&](int row) {
 #if CONV == 1
-                return ((long long)img * K_ + row) * (OH_ * OW_) + px;
+                return (SLICED ? c0 : 0) + ((long long)img * K_ + row) * (OH_ * OW_) + px;
 #else
                 return c0 + (long long)row * ldc + col;
 #endif

@@ -622,8 +622,15 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
     // shifted input planes written by one reindex per chunk of images (a 1x1 convolution of stride 1 without padding
     // reads x itself), the product on kernels/gemm_mfma.h with the weights shared across the batch.  Rows of cols are
     // padded to a multiple of 16 bytes when the pixel count is not one (the GEMM kernel's fast path wants aligned rows).
+    // Small ones with long sums as well: the kernel of one lane a result below walks them in 0.05 (1x1) to 0.1 us a term, the product's
+    // kernel in 0.03 behind 3 us, and 3 more where the weights' rows are copied (us, one lane a result / this: float32 4 x 16 x 6 x 6 3x3
+    // stride 2 -> 16 10.4 / 7.0, 8 x 39 x 6 x 6 3x3 stride 2 -> 39 26.0 / 12.4, 2 x 256 x 7 x 7 1x1 -> 64 15.6 / 8.7, 1 x 16 x 8 x 8 3x3 -> 16
+    // 6.6 / 6.8; float16 2 x 18 x 10 x 10 3x3 -> 16 15.6 / 8.1; bfloat16 1 x 215 x 7 x 7 3x3 -> 17 167 / 15.8; on the other side float32
+    // 2 x 8 x 10 x 10 3x3 -> 8 4.6 / 5.7, 3 x 100 x 9 x 9 1x1 -> 100 6.7 / 7.4).
     const int64_t P = OH * OW, CRS = C * R * S;
-    if (G == 1 && !getenv("MJT_NO_FASTPATH") && !getenv("MJT_CONV_NO_GEMM") && (double)N * K * P * CRS >= (double)(1 << 22) &&
+    const bool long_sum = (x->dtype == MJT_FLOAT32 || x->dtype == MJT_BFLOAT16 || x->dtype == MJT_FLOAT16) &&
+                          CRS >= ((CRS * dtype_size(x->dtype)) % 16 || (uintptr_t)w->ptr % 16 ? 160 : 128);
+    if (G == 1 && !getenv("MJT_NO_FASTPATH") && !getenv("MJT_CONV_NO_GEMM") && ((double)N * K * P * CRS >= (double)(1 << 22) || long_sum) &&
         P < (int64_t(1) << 31) && CRS < (int64_t(1) << 31) && matmul_available()) {
         if (!flat_forced && conv_stem(x, w, y, p)) return;
         const int64_t esz = dtype_size(x->dtype);
@@ -678,8 +685,12 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
         const int64_t NP = N * P, tiles64 = ((K + 63) / 64) * ((NP + 63) / 64);
         // (16-bit operands with a long sum and fewer 64 x 64 tiles than compute units stay on the column matrices, whose
         // product picks its tiles for a part-filled chip: 32 x 512 x 7 x 7 3x3 -> 512, 200 tiles: 102 us here, 71 there)
-        const bool ig_fits = !ig16 || tiles64 >= cus || CRS <= 1024;
-        if (!plain && ((x->dtype == MJT_FLOAT32 && y->dtype == MJT_FLOAT32) || ig16) && ig_fits && !getenv("MJT_CONV_NO_IGEMM") &&
+        // (or on slices of the sum here, where these are few enough: the reduce reads their float32 results)
+        const bool ig_fits = !ig16 || tiles64 >= cus || CRS <= 1024 || tiles64 * 4 <= cus;
+        // (a 1x1 convolution whose product would leave most of the chip idle comes here for the slices: the product below takes the images
+        // as a batch, whose sums stay whole; float32 3 x 1024 x 14 x 14 -> 256 25.0 us there, 15.8 here; 10 x 512 x 16 x 16 -> 128 15.3, 13.8)
+        const bool few_long = CRS >= (ig16 ? 512 : 256) && tiles64 * 2 <= cus;
+        if ((!plain || few_long) && ((x->dtype == MJT_FLOAT32 && y->dtype == MJT_FLOAT32) || ig16) && ig_fits && !getenv("MJT_CONV_NO_IGEMM") &&
             numel(x) < (int64_t(1) << 31) && numel(y) < (int64_t(1) << 31) && H < 16384 && W < 16384 &&
             (R - 1) * p->dil_h < 16384 && (S - 1) * p->dil_w < 16384 && p->pad_h < 16384 && p->pad_w < 16384 &&
             OH * p->stride_h < 16384 && OW * p->stride_w < 16384) {
@@ -700,29 +711,59 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
             const bool tall = ig16 && K > 64 && ((K + 127) / 128) * ((NP + 63) / 64) >= cus;
             int MI = big || tall ? 2 : 1, NI = big ? 2 : 1;
             bool split = false;
-            if (!ig16 && CRS >= 128) {
-                const int64_t stages = (CRS + 31) / 32;
-                double least = 1e30;
+            // Few tiles and a long sum: the sum is cut into up to 16 slices, whose float32 results a reduce launch adds up (one launch
+            // up to 16, which leaves the scratch memory alone).  A stage (32 float32 or 64 16-bit elements of the sum) of a 64 x 64 tile
+            // takes as long as above, 1.1 us in 16 bits; the reduce 5 us and its traffic, a group behind the convolution that then has
+            // to run by itself 3 more.  (us, whole / in slices with the reduce: float32 3 x 272 x 7 x 7 3x3 -> 470 65 / 16.0, 1 x 512 x 7 x 7 3x3
+            // -> 512 122 / 17.9, 16 x 256 x 14 x 14 3x3 -> 256 69.5 / 45.9, 4 x 64 x 14 x 14 3x3 -> 64 19.4 / 10.0, 32 x 128 x 9 x 9 3x3 -> 128 35.3 /
+            // 19.0, 6 x 256 x 14 x 14 3x3 stride 2 -> 512 64.5 / 18.6; 16 bits, column matrices / so: 6 x 400 x 14 x 14 5x5 -> 51 77.9 / 24.4,
+            // 12 x 300 x 15 x 15 5x5 -> 20 76.2 / 29.9, 20 x 500 x 7 x 7 3x3 -> 256 45.9 / 36.1.)
+            const int64_t ks = ig16 ? 64 : 32, stages = (CRS + ks - 1) / ks;
+            int64_t slices = 1, per = stages;
+            auto estimate = [&](int t, int64_t n) {
+                const int mi = t ? 2 : 1, ni = t == 2 ? 2 : 1;
+                const double tiles = (double)(((K + 64 * mi - 1) / (64 * mi)) * ((NP + 64 * ni - 1) / (64 * ni)));
+                const double rounds = std::ceil(tiles * (double)n / cus), st = (double)((stages + n - 1) / n);
+                const double us = t == 0 ? ((ig16 ? 1.1 : 0.92) * st + 3.0) * (0.25 + 0.75 * rounds) : t == 1 ? (1.05 * st + 4.0) * rounds : (1.85 * st + 5.0) * rounds;
+                return us + (n == 1 ? 0.0 : 5.0 + (double)n * K * NP * 8 / 3e6 + (epilogue_waits() ? 3.0 : 0.0));
+            };
+            double least = 1e30;
+            if (!ig16 && CRS >= 128)
                 for (int t = big ? 1 : 0; t < 3; t++) {
-                    const int mi = t ? 2 : 1, ni = t == 2 ? 2 : 1;
-                    const double rounds = std::ceil((double)(((K + 64 * mi - 1) / (64 * mi)) * ((NP + 64 * ni - 1) / (64 * ni))) / cus);
-                    const double us = t == 0 ? (0.92 * stages + 3.0) * (0.25 + 0.75 * rounds) : t == 1 ? (1.05 * stages + 4.0) * rounds : (1.85 * stages + 5.0) * rounds;
-                    if (us < least) { least = us; MI = mi; NI = ni; split = t > 0; }
+                    const double us = estimate(t, 1);
+                    if (us < least) { least = us; MI = t ? 2 : 1; NI = t == 2 ? 2 : 1; split = t > 0; }
+                }
+            else if (!big && !tall)
+                least = estimate(0, 1);
+            for (int64_t n = 2; n <= 16 && n <= stages / 2 && least < 1e30; n++) {
+                const int64_t pn = (stages + n - 1) / n, nn = (stages + pn - 1) / pn;
+                for (int t = 0; t < (ig16 || CRS < 128 ? 1 : 3); t++) {
+                    const double us = estimate(t, nn);
+                    if (us < least && nn * K * NP * 4 <= (int64_t(256) << 20)) {
+                        least = us; slices = nn; per = pn; MI = t ? 2 : 1; NI = t == 2 ? 2 : 1; split = t > 0;
+                    }
                 }
             }
+            if (const char* e = getenv("MJT_CONV_SLICES")) {         // for tests: at most so many slices (1: none) of the tile chosen
+                const int64_t n = std::max(1, std::min(atoi(e), 16));
+                per = (stages + n - 1) / n;
+                slices = (stages + per - 1) / per;
+            }
+            void* part_mem = slices > 1 ? scratch_if_any((size_t)(slices * K * NP * 4)) : nullptr;
+            if (!part_mem) slices = 1;
             const int in = x->dtype == MJT_BFLOAT16 ? 0 : x->dtype == MJT_FLOAT16 ? 1 : 2;
-            const int out = y->dtype == MJT_BFLOAT16 ? 0 : y->dtype == MJT_FLOAT16 ? 1 : 2;
+            const int out = slices > 1 ? 2 : y->dtype == MJT_BFLOAT16 ? 0 : y->dtype == MJT_FLOAT16 ? 1 : 2;
             std::ostringstream key;
             const bool xbuf = (64 * NI / P + 2) * C * H * W * esz < (int64_t(1) << 31);      // a tile's images through one buffer descriptor
-            const EpilogueCode ep = epilogue_code(1, 12, y->dtype, numel(y));
-            key << "igemm|" << geo.str() << MI << NI << in << out << xbuf << split << ep.key;
+            const EpilogueCode ep = epilogue_code(1, 12, y->dtype, slices > 1 ? -1 : numel(y));
+            key << "igemm|" << geo.str() << MI << NI << in << out << xbuf << split << (slices > 1) << ep.key;
             JitKernel* k = cached(key.str());
             if (!k) {
                 std::ostringstream name;
                 name << "mjt_conv_igemm_" << mjt_dtype_name(x->dtype) << (y->dtype != x->dtype ? "_of32" : "") << "_c" << C << "_k" << K << "_" << H << "x" << W << "_r" << R << "x" << S << "_s" << p->stride_h << "x"
-                     << p->stride_w << "_p" << p->pad_h << "x" << p->pad_w << "_d" << p->dil_h << "x" << p->dil_w << (split ? "_parts_" : "_") << 64 * MI << "x" << 64 * NI << ep.suffix();
+                     << p->stride_w << "_p" << p->pad_h << "x" << p->pad_w << "_d" << p->dil_h << "x" << p->dil_w << (split ? "_parts_" : "_") << 64 * MI << "x" << 64 * NI << (slices > 1 ? "_slices" : "") << ep.suffix();
                 std::ostringstream src;
-                src << ep.defs << "#define ENTRY " << name.str() << "\n#define SPLIT " << (split ? 1 : 0) << "\n#define CONV 1\n#define IN " << in << "\n#define OUT " << out << "\n#define MI " << MI << "\n#define NI " << NI
+                src << ep.defs << "#define ENTRY " << name.str() << "\n#define SPLIT " << (split ? 1 : 0) << "\n#define SLICED " << (slices > 1 ? 1 : 0) << "\n#define CONV 1\n#define IN " << in << "\n#define OUT " << out << "\n#define MI " << MI << "\n#define NI " << NI
                     << "\n#define A_KCONT 1\n#define B_KCONT 0\n#define XBUF " << (xbuf ? 1 : 0) << "\n" << geo.str();
                 if (split) src << embedded_source("split.h") << "\n";
                 src << embedded_source("gemm_mfma.h") << "\n";
@@ -730,13 +771,18 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
                 remember(key.str(), k);
             }
             const int64_t tiles = ((K + 64 * MI - 1) / (64 * MI)) * ((NP + 64 * NI - 1) / (64 * NI));
-            const int64_t grid = (tiles + 7) / 8 * 8;
+            const int64_t grid = (tiles * slices + 7) / 8 * 8;
             MJT_CHECK(grid < (int64_t(1) << 31), "conv: launch too large");
-            std::vector<uint64_t> a{bits_of_ptr(wmat), bits_of_ptr(x->ptr), bits_of_ptr(y->ptr), (uint64_t)K, (uint64_t)NP, (uint64_t)CRS,
-                                    (uint64_t)lda, 0, 0, 0, 0, 0};
+            std::vector<uint64_t> a{bits_of_ptr(wmat), bits_of_ptr(x->ptr), bits_of_ptr(slices > 1 ? part_mem : y->ptr), (uint64_t)K, (uint64_t)NP, (uint64_t)CRS,
+                                    (uint64_t)lda, 0, 0, (uint64_t)(slices > 1 ? per : 0), 0, (uint64_t)(slices > 1 ? K * NP : 0)};
             a.insert(a.end(), ep.words.begin(), ep.words.end());
             epilogue_taken(ep);
             jit_launch(k, (unsigned)grid, 1, product_threads(split), 0, a);
+            if (slices > 1) {
+                mjt_tensor part = view(part_mem, MJT_FLOAT32, {slices, K * NP}), whole = view(y->ptr, y->dtype, {K * NP});
+                if (mjt_reduce(&part, &whole, MJT_OP_ADD, 0b01) != MJT_OK) MJT_FAIL(MJT_ERR_DEVICE, "conv: adding up the slices failed: " << mjt_last_error());
+                set_last_kernel(k->name.c_str());
+            }
             return;
         }
         int64_t chunk = (int64_t(1) << 30) / (CRS * Ppad * esz);
