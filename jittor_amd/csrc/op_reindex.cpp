@@ -302,18 +302,11 @@ void run_generic(Plan* plan, bool scatter, int op, const mjt_tensor* x, const mj
     jit_launch(kern, (unsigned)blocks, 1, 256, 0, args);
 }
 
-// A scatter through a window pattern (x[b.., oh*SH + kh*DH + CH, ow*SW + kw*DW + CW] op= y[b.., oh, ow, kh, kw], no
-// overflow conditions, no extras: the gradient of pooling) runs as a gather over x: every element of x folds the windows
-// that reach it (kernels/window_scatter.h) -- no atomic updates, no identity fill.  Measured on the gradient of a 3x3
-// stride-2 maximum pooling of [64,64,112,112] float32: 1042 us of queued atomic adds (plus 20 us of fill) against 139 us.  Returns false when the pattern is another one; the caller then fills and scatters.
-bool try_window_scatter(Plan* plan, int op, const mjt_tensor* x, const mjt_tensor* y, int n_ofc, int n_ex, const ScatterPrologue* sp) {
-    if (getenv("MJT_NO_FASTPATH") || getenv("MJT_NO_WINDOW_SCATTER")) return false;
-    if (n_ofc != 0 || n_ex != 0 || !plan->all_affine) return false;
-    if (op != MJT_OP_ADD && op != MJT_OP_MAXIMUM && op != MJT_OP_MINIMUM && op != MJT_OP_MULTIPLY) return false;
-    if (x->dtype == MJT_BOOL) return false;
+// The window pattern x[b.., oh*SH + kh*DH + CH, ow*SW + kw*DW + CW] of a loop y[b.., oh, ow, kh, kw], neither of them empty.
+struct Window { int64_t SH, SW, DH, DW, CH, CW; };
+bool window_of(Plan* plan, const mjt_tensor* x, const mjt_tensor* y, Window* g) {
     const int XD = x->ndim, YD = y->ndim, nb = XD - 2;
-    if (XD < 2 || YD != XD + 2) return false;
-    if (numel(x) == 0 || numel(y) == 0) return false;
+    if (XD < 2 || YD != XD + 2 || numel(x) == 0 || numel(y) == 0) return false;
     std::vector<int64_t> xs(x->shape, x->shape + XD), ys(y->shape, y->shape + YD);
     std::vector<Affine> aff(XD);
     for (int i = 0; i < XD; i++)
@@ -330,11 +323,90 @@ bool try_window_scatter(Plan* plan, int op, const mjt_tensor* x, const mjt_tenso
         if (k != a_oh && k != a_kh && ah.coef[k]) return false;
         if (k != a_ow && k != a_kw && aw.coef[k]) return false;
     }
-    const int64_t SH = ah.coef[a_oh], DH = ah.coef[a_kh], CH = ah.c0, SW = aw.coef[a_ow], DW = aw.coef[a_kw], CW = aw.c0;
-    if (SH < 1 || SW < 1 || DH < 1 || DW < 1 || SH > 8 || SW > 8 || DH > 8 || DW > 8) return false;
-    if (CH < -64 || CH > 64 || CW < -64 || CW > 64) return false;
-    const int64_t KH = y->shape[a_kh], KW = y->shape[a_kw];
-    if (KH < 1 || KW < 1 || KH * KW > 64) return false;
+    *g = Window{ah.coef[a_oh], aw.coef[a_ow], ah.coef[a_kh], aw.coef[a_kw], ah.c0, aw.c0};
+    if (g->SH < 1 || g->SW < 1 || g->DH < 1 || g->DW < 1 || g->SH > 8 || g->SW > 8 || g->DH > 8 || g->DW > 8) return false;
+    if (g->CH < -64 || g->CH > 64 || g->CW < -64 || g->CW > 64) return false;
+    return y->shape[a_kh] >= 1 && y->shape[a_kw] >= 1 && y->shape[a_kh] * y->shape[a_kw] <= 64;
+}
+
+// A gather through a window pattern that is folded over the windows (pooling): kernels/window_fold.h, where rows of x are whole 16-byte
+// pieces and a lane's pieces fit its registers.  False: not covered.
+bool try_window_fold(Plan* plan, int rop, const mjt_tensor* x, const mjt_tensor* y, const mjt_tensor* z, double overflow_value, int nred, int n_ofc, int n_ex) {
+    const char* env = getenv("MJT_WINDOW_FOLD");               // 0: never, 1: also where it is the slower one
+    if (getenv("MJT_NO_FASTPATH") || (env && !strcmp(env, "0"))) return false;
+    if (nred != 2 || n_ofc != 0 || n_ex != 0 || !plan->all_affine || x->dtype == MJT_BOOL) return false;
+    Window g;
+    if (!window_of(plan, x, y, &g)) return false;
+    const int XD = x->ndim, nb = XD - 2;
+    const int64_t H = x->shape[nb], W = x->shape[nb + 1], OH = y->shape[nb], OW = y->shape[nb + 1], KH = y->shape[nb + 2], KW = y->shape[nb + 3];
+    const int64_t esz = dtype_size(x->dtype), zsz = dtype_size(z->dtype), LV = 16 / esz, xn = numel(x), zn = numel(z);
+    if (W % LV || (uintptr_t)x->ptr % 16 || xn >= (int64_t(1) << 31) || zn >= (int64_t(1) << 31)) return false;
+    // neighbouring outputs of a lane: as many as begin at whole pieces, twice as many while they are less than 16 bytes on both sides
+    int64_t OV = LV;
+    while (OV > 1 && OV / 2 * g.SW % LV == 0) OV /= 2;
+    if (OV * g.SW * esz <= 16 && OV * zsz < 16) OV *= 2;
+    auto floor_div = [](int64_t a, int64_t b) { return a >= 0 ? a / b : -((-a + b - 1) / b); };
+    const int64_t pieces = floor_div((OV - 1) * g.SW + g.CW + (KW - 1) * g.DW, LV) - floor_div(g.CW, LV) + 1;
+    auto rows = [&](int64_t r) { return (r - 1) * g.SH + (KH - 1) * g.DH + 1; };
+    // two rows of outputs where their windows share rows of x; at most 96 registers of pieces
+    int64_t OR = g.SH < (KH - 1) * g.DH + 1 && OH > 1 ? 2 : 1;
+    if (rows(OR) * pieces > 24) OR = 1;
+    if (rows(OR) * pieces > 24) return false;
+    const int64_t planes = zn / (OH * OW), lanes = planes * ((OH + OR - 1) / OR) * ((OW + OV - 1) / OV);
+    // few outputs are better spread over more lanes (3x3 stride-2 maximum, us, one output a lane / so: 32 x 64 x 112 x 112 float32 35.9 /
+    // 28.4 (4.5 TB/s), bfloat16 38.2 / 13.0 (5.9); 18 x 23 x 80 x 80 float32 5.6 / 5.1; 9 x 16 x 88 x 88 bfloat16 4.3 / 4.3; on the other side
+    // 4 x 32 x 48 x 48 float32 3.3 / 4.0, 1 x 32 x 32 x 32 bfloat16 2.9 / 3.8)
+    if (zn < (1 << 18) && !env) return false;
+    int64_t ZV = OV;
+    while (ZV > 1 && (OW % ZV || (uintptr_t)z->ptr % (size_t)(ZV * zsz) || ZV * zsz > 16)) ZV /= 2;
+    std::ostringstream vk;
+    vk << "WF" << rop << "," << z->dtype << "|" << g.SH << "," << g.SW << "," << g.DH << "," << g.DW << "," << g.CH << "," << g.CW << "," << KH << "," << KW << "," << H << "," << W << "," << OH << ","
+       << OW << "," << OR << "," << OV << "," << ZV;
+    const std::string vkey = vk.str();
+    JitKernel* kern = nullptr;
+    {
+        std::lock_guard<std::mutex> lock(g_mu);
+        auto it = plan->kernels.find(vkey);
+        if (it != plan->kernels.end()) kern = it->second;
+    }
+    if (!kern) {
+        const int ta = z->dtype == MJT_FLOAT16 || z->dtype == MJT_BFLOAT16 ? MJT_FLOAT32 : z->dtype;       // accumulator as in the reduce kernels
+        const std::string opn = rop == MJT_OP_MEAN ? "add" : mjt_op_name(rop);
+        std::ostringstream name, src;
+        name << "mjt_window_fold_" << mjt_op_name(rop) << "_" << mjt_dtype_name(x->dtype) << "_" << mjt_dtype_name(z->dtype) << "_" << H << "x" << W << "_k" << KH << "x" << KW << "_s" << g.SH << "x"
+             << g.SW << "_d" << g.DH << "x" << g.DW << "_c" << (g.CH < 0 ? "m" : "") << std::abs(g.CH) << (g.CW < 0 ? "m" : "x") << std::abs(g.CW) << "_o" << OH << "x" << OW << "_l" << OR << "x" << OV << "v" << ZV;
+        src << "#define ENTRY " << name.str() << "\n#define TX " << dtype_cname(x->dtype) << "\n#define TZ " << dtype_cname(z->dtype) << "\n#define TACC " << dtype_cname(ta)
+            << "\n#define LV " << LV << "\n#define OR " << OR << "\n#define OV " << OV << "\n#define ZV " << ZV << "\n#define KH " << KH << "\n#define KW " << KW << "\n#define SH " << g.SH
+            << "\n#define SW " << g.SW << "\n#define DH " << g.DH << "\n#define DW " << g.DW << "\n#define CH " << g.CH << "\n#define CW " << g.CW << "\n#define H_ " << H << "\n#define W_ " << W
+            << "\n#define OH_ " << OH << "\n#define OW_ " << OW << "\n#define INIT mjt_init_" << opn << "<TACC>()\n";
+        // (a multiply-add for every window that an element is in, as the kernel of one output a lane has it: shared, the product would be
+        // rounded by itself)
+        if (rop == MJT_OP_MEAN) src << "#define COMBINE(a, x) " << (ta == MJT_FLOAT32 ? "__builtin_fmaf(TACC(x), rcount, (a))" : ta == MJT_FLOAT64 ? "__builtin_fma(TACC(x), rcount, (a))" : "((a) + TACC(x) * rcount)") << "\n";
+        else src << "#define COMBINE(a, x) mjt_" << opn << "<TACC>((a), (x))\n";
+        src << embedded_source("prelude.h") << "\n" << embedded_source("window_fold.h") << "\n";
+        kern = jit_get(src.str(), name.str());
+        std::lock_guard<std::mutex> lock(g_mu);
+        plan->kernels.emplace(vkey, kern);
+    }
+    jit_launch(kern, (unsigned)((lanes + 255) / 256), 1, 256, 0,
+               {bits_of_ptr(x->ptr), bits_of_ptr(z->ptr), (uint64_t)lanes, bits_of(overflow_value), bits_of(1.0 / (double)(KH * KW))});
+    return true;
+}
+
+// A scatter through a window pattern (x[b.., oh*SH + kh*DH + CH, ow*SW + kw*DW + CW] op= y[b.., oh, ow, kh, kw], no
+// overflow conditions, no extras: the gradient of pooling) runs as a gather over x: every element of x folds the windows
+// that reach it (kernels/window_scatter.h) -- no atomic updates, no identity fill.  Measured on the gradient of a 3x3
+// stride-2 maximum pooling of [64,64,112,112] float32: 1042 us of queued atomic adds (plus 20 us of fill) against 139 us.  Returns false when the pattern is another one; the caller then fills and scatters.
+bool try_window_scatter(Plan* plan, int op, const mjt_tensor* x, const mjt_tensor* y, int n_ofc, int n_ex, const ScatterPrologue* sp) {
+    if (getenv("MJT_NO_FASTPATH") || getenv("MJT_NO_WINDOW_SCATTER")) return false;
+    if (n_ofc != 0 || n_ex != 0 || !plan->all_affine) return false;
+    if (op != MJT_OP_ADD && op != MJT_OP_MAXIMUM && op != MJT_OP_MINIMUM && op != MJT_OP_MULTIPLY) return false;
+    if (x->dtype == MJT_BOOL) return false;
+    const int XD = x->ndim, YD = y->ndim, nb = XD - 2;
+    Window g;
+    if (!window_of(plan, x, y, &g)) return false;
+    const int a_oh = nb, a_ow = nb + 1, a_kh = nb + 2, a_kw = nb + 3;
+    const int64_t SH = g.SH, SW = g.SW, DH = g.DH, DW = g.DW, CH = g.CH, CW = g.CW, KH = y->shape[a_kh], KW = y->shape[a_kw];
     const int64_t NCH = (KH - 1) * DH / SH + 1, NCW = (KW - 1) * DW / SW + 1;
     if (NCH * NCW > 16) return false;
 
@@ -356,12 +428,27 @@ bool try_window_scatter(Plan* plan, int op, const mjt_tensor* x, const mjt_tenso
     // elements: 2x2 stride 2 of [64,128,64,64] 57.3 / 60.6, 17.9 / 22.6 (40 bodies at 8); 3x3 stride 2 of [32,64,112,112] 83.8 / 79.5,
     // 27.6 / 27.0 (80); 4x4 stride 2 of [16,64,64,64] 25.7 / 23.4, 7.9 / 7.7 (96); 2x2 stride 1 of the same 37.8 / 32.9, 10.7 / 8.5 (144))
     auto columns = [&](int v) { return (v - 1 + (KW - 1) * DW) / SW + 1; };      // of windows that reach v neighbouring elements
+    // Blocks of SH rows x a multiple of SW columns, where a lane's rows are long enough for them: bodies are then counted by the windows
+    // that do reach an element.  At most 40 again.  (Gradient of a 3x3 stride-2 maximum with the mask of a relu behind it, us, a row a lane /
+    // so: 32 x 64 x 112 x 112 float32 59.5 / 49.0 (5.3 TB/s), bfloat16 43.9 + 19.7 for the mask / 30.6; 18 x 23 x 80 x 80 float32 8.8 + 5.3 / 6.8;
+    // 4 x 32 x 48 x 48 float32 3.7 + 2.1 / 3.6; on the other side 1 x 32 x 32 x 32 bfloat16 2.8 / 3.7.)
+    const char* benv = getenv("MJT_WINDOW_BLOCKS");             // 0: never, 1: also where they are the slower ones
+    int bvec = sp && (benv ? strcmp(benv, "0") != 0 : xn >= (1 << 17)) ? wvec : 0;
+    auto reached = [&](int64_t first, int64_t n, int64_t stride, int64_t dil, int64_t taps, int64_t c0) {
+        int64_t count = 0;                                                       // (element, tap) pairs of n elements from a multiple of the stride on
+        for (int64_t e = first; e < first + n; e++)
+            for (int64_t t = 0; t < taps; t++) count += ((e - c0 - t * dil) % stride + stride) % stride == 0;
+        return count;
+    };
+    while (bvec > 0 && (bvec % SW != 0 || reached(0, SH, SH, DH, KH, CH) * reached(0, bvec, SW, DW, KW, CW) > 40)) bvec /= 2;
+    const bool blocks_of = bvec >= 2;
     while (wvec > 1 && NCH * columns(wvec) * wvec > 40) wvec /= 2;
+    if (blocks_of) wvec = bvec;
     // without a prologue the candidates are loads from y itself, far apart for neighbouring elements of x: more of them
     // per lane coalesce worse (3x3 stride-2 windows into [64,64,112,112]: 230 us with four elements per lane, 175 with one)
     if (!sp) wvec = 1;
     std::ostringstream vk;
-    vk << "WS" << op << (use64 ? "L" : "I") << wvec << "|" << SH << "," << SW << "," << DH << "," << DW << "," << CH << "," << CW << "," << KH << "," << KW;
+    vk << "WS" << op << (use64 ? "L" : "I") << wvec << (blocks_of ? "B" : "") << "|" << SH << "," << SW << "," << DH << "," << DW << "," << CH << "," << CW << "," << KH << "," << KW;
     for (int i = 0; i < XD; i++) vk << "," << x->shape[i];
     vk << "," << y->shape[a_oh] << "," << y->shape[a_ow];
     if (sp) vk << "|P" << sp->key;
@@ -400,7 +487,7 @@ bool try_window_scatter(Plan* plan, int op, const mjt_tensor* x, const mjt_tenso
         frag << "#define TX " << dtype_cname(x->dtype) << "\n#define TACC " << dtype_cname(ta) << "\n#define index_t " << IT << "\n#define VEC " << wvec
              << "\n#define NPARAM " << args.size() + ep.words.size() << "\n#define NB " << nb << "\n#define KH " << KH << "\n#define KW " << KW << "\n#define SH " << SH << "\n#define SW " << SW
              << "\n#define DH " << DH << "\n#define DW " << DW << "\n#define CH " << CH << "\n#define CW " << CW << "\n#define NCH " << NCH
-             << "\n#define NCU " << columns(wvec) << "\n";
+             << "\n#define NCU " << columns(wvec) << "\n#define BLOCKS " << (blocks_of ? 1 : 0) << "\n";
         // extents as literals: the lane's coordinates come from divisions by them
         frag << "#define xshape_h " << x->shape[nb] << "\n#define xshape_w " << x->shape[nb + 1] << "\n#define yshape_oh " << y->shape[a_oh]
              << "\n#define yshape_ow " << y->shape[a_ow] << "\n";
@@ -422,8 +509,10 @@ bool try_window_scatter(Plan* plan, int op, const mjt_tensor* x, const mjt_tenso
         std::lock_guard<std::mutex> lock(g_mu);
         plan->kernels.emplace(vkey, kern);
     }
-    const int64_t blocks = (xn / wvec + 255) / 256;
+    const int64_t lanes = blocks_of ? xn / (x->shape[XD - 2] * x->shape[XD - 1]) * ((x->shape[XD - 2] + SH - 1) / SH) * (x->shape[XD - 1] / wvec) : xn / wvec;
+    const int64_t blocks = (lanes + 255) / 256;
     if (blocks >= (int64_t(1) << 31)) return false;
+    if (blocks_of) args[2] = (uint64_t)lanes;
     args.insert(args.end(), ep.words.begin(), ep.words.end());
     epilogue_taken(ep);
     jit_launch(kern, (unsigned)blocks, 1, 256, 0, args);
@@ -532,6 +621,7 @@ void reindex_then_reduce_impl(const mjt_tensor* x, const mjt_tensor* yshape, con
     y.ptr = z->ptr;                                   // never dereferenced: only its shape is used
     std::string key = plan_key(false, 0, x, &y, n_idx, idx, n_ofc, ofc, n_ex, ex);
     Plan* plan = get_plan(key, x, &y, y.ndim, n_idx, idx, n_ofc, ofc, n_ex, ex);
+    if (try_window_fold(plan, rop, x, &y, z, overflow_value, nred, n_ofc, n_ex)) return;
     run_generic(plan, false, 0, x, &y, overflow_value, n_ex, ex, z, rop, nred);
 }
 
