@@ -178,6 +178,19 @@ struct Preparing {
     Preparing();
     ~Preparing();
 };
+// The sum of a product's slices (op_slices.cpp), at most 16 of n float32 results each, into y (n elements of a float type up to 32 bits) or
+// the group that waits behind the product.  Made before the slices are launched, under Preparing: a group that cannot be taken ends the call
+// there.  whole: the n elements are the product's whole result, in its order.
+struct SliceFold {
+    SliceFold(const void* part, void* y, int dtype, int64_t n, int64_t slices, bool whole);
+    void launch();
+
+private:
+    JitKernel* k;
+    EpilogueCode ep;
+    std::vector<uint64_t> args;
+    int64_t blocks;
+};
 std::string fused_emit_ops(const mjt_fused_desc* d, bool store_outputs);
 std::string fused_op_expr(const mjt_fused_desc* d, const mjt_fused_op& o);
 

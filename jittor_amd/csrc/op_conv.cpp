@@ -711,10 +711,9 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
             const bool tall = ig16 && K > 64 && ((K + 127) / 128) * ((NP + 63) / 64) >= cus;
             int MI = big || tall ? 2 : 1, NI = big ? 2 : 1;
             bool split = false;
-            // Few tiles and a long sum: the sum is cut into up to 16 slices, whose float32 results a reduce launch adds up (one launch
-            // up to 16, which leaves the scratch memory alone).  A stage (32 float32 or 64 16-bit elements of the sum) of a 64 x 64 tile
-            // takes as long as above, 1.1 us in 16 bits; the reduce 5 us and its traffic, a group behind the convolution that then has
-            // to run by itself 3 more.  (us, whole / in slices with the reduce: float32 3 x 272 x 7 x 7 3x3 -> 470 65 / 16.0, 1 x 512 x 7 x 7 3x3
+            // Few tiles and a long sum: the sum is cut into up to 16 slices, whose float32 results are added up by a launch behind them,
+            // which also takes a group behind the convolution along.  A stage (32 float32 or 64 16-bit elements of the sum) of a 64 x 64 tile
+            // takes as long as above, 1.1 us in 16 bits; that launch 5 us and its traffic.  (us, whole / in slices: float32 3 x 272 x 7 x 7 3x3 -> 470 65 / 16.0, 1 x 512 x 7 x 7 3x3
             // -> 512 122 / 17.9, 16 x 256 x 14 x 14 3x3 -> 256 69.5 / 45.9, 4 x 64 x 14 x 14 3x3 -> 64 19.4 / 10.0, 32 x 128 x 9 x 9 3x3 -> 128 35.3 /
             // 19.0, 6 x 256 x 14 x 14 3x3 stride 2 -> 512 64.5 / 18.6; 16 bits, column matrices / so: 6 x 400 x 14 x 14 5x5 -> 51 77.9 / 24.4,
             // 12 x 300 x 15 x 15 5x5 -> 20 76.2 / 29.9, 20 x 500 x 7 x 7 3x3 -> 256 45.9 / 36.1.)
@@ -725,7 +724,7 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
                 const double tiles = (double)(((K + 64 * mi - 1) / (64 * mi)) * ((NP + 64 * ni - 1) / (64 * ni)));
                 const double rounds = std::ceil(tiles * (double)n / cus), st = (double)((stages + n - 1) / n);
                 const double us = t == 0 ? ((ig16 ? 1.1 : 0.92) * st + 3.0) * (0.25 + 0.75 * rounds) : t == 1 ? (1.05 * st + 4.0) * rounds : (1.85 * st + 5.0) * rounds;
-                return us + (n == 1 ? 0.0 : 5.0 + (double)n * K * NP * 8 / 3e6 + (epilogue_waits() ? 3.0 : 0.0));
+                return us + (n == 1 ? 0.0 : 5.0 + (double)n * K * NP * 8 / 3e6);
             };
             double least = 1e30;
             if (!ig16 && CRS >= 128)
@@ -755,7 +754,7 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
             const int out = slices > 1 ? 2 : y->dtype == MJT_BFLOAT16 ? 0 : y->dtype == MJT_FLOAT16 ? 1 : 2;
             std::ostringstream key;
             const bool xbuf = (64 * NI / P + 2) * C * H * W * esz < (int64_t(1) << 31);      // a tile's images through one buffer descriptor
-            const EpilogueCode ep = epilogue_code(1, 12, y->dtype, slices > 1 ? -1 : numel(y));
+            const EpilogueCode ep = epilogue_code(1, 12, y->dtype, slices > 1 ? -1 : numel(y));      // (a group behind slices runs where they are added up)
             key << "igemm|" << geo.str() << MI << NI << in << out << xbuf << split << (slices > 1) << ep.key;
             JitKernel* k = cached(key.str());
             if (!k) {
@@ -776,13 +775,18 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
             std::vector<uint64_t> a{bits_of_ptr(wmat), bits_of_ptr(x->ptr), bits_of_ptr(slices > 1 ? part_mem : y->ptr), (uint64_t)K, (uint64_t)NP, (uint64_t)CRS,
                                     (uint64_t)lda, 0, 0, (uint64_t)(slices > 1 ? per : 0), 0, (uint64_t)(slices > 1 ? K * NP : 0)};
             a.insert(a.end(), ep.words.begin(), ep.words.end());
-            epilogue_taken(ep);
-            jit_launch(k, (unsigned)grid, 1, product_threads(split), 0, a);
-            if (slices > 1) {
-                mjt_tensor part = view(part_mem, MJT_FLOAT32, {slices, K * NP}), whole = view(y->ptr, y->dtype, {K * NP});
-                if (mjt_reduce(&part, &whole, MJT_OP_ADD, 0b01) != MJT_OK) MJT_FAIL(MJT_ERR_DEVICE, "conv: adding up the slices failed: " << mjt_last_error());
-                set_last_kernel(k->name.c_str());
+            if (slices == 1) {
+                epilogue_taken(ep);
+                jit_launch(k, (unsigned)grid, 1, product_threads(split), 0, a);
+                return;
             }
+            SliceFold fold(part_mem, y->ptr, y->dtype, K * NP, slices, true);
+            {
+                Preparing preparing;
+                jit_launch(k, (unsigned)grid, 1, product_threads(split), 0, a);
+            }
+            fold.launch();
+            set_last_kernel(k->name.c_str());
             return;
         }
         int64_t chunk = (int64_t(1) << 30) / (CRS * Ppad * esz);

@@ -246,21 +246,15 @@ void gemm_launch(int in_dtype, int out_dtype, const void* A, const void* B, void
             jit_launch(k, (unsigned)grid, 1, product_threads(split), 0, args);
             return;
         }
-        mjt_tensor part{}, whole{};
-        part.ptr = part_mem;
-        part.dtype = MJT_FLOAT32;
-        part.ndim = 2;
-        part.shape[0] = slices;
-        part.shape[1] = M * N;
-        whole.ptr = C;
-        whole.dtype = out_dtype;
-        whole.ndim = 1;
-        whole.shape[0] = M * N;
-        args[2] = bits_of_ptr(part.ptr);
+        args[2] = bits_of_ptr(part_mem);
         args[9] = (uint64_t)per;
         args[11] = (uint64_t)(M * N);
-        jit_launch(k, (unsigned)grid, 1, product_threads(split), 0, args);
-        if (mjt_reduce(&part, &whole, MJT_OP_ADD, 0b01) != MJT_OK) MJT_FAIL(MJT_ERR_DEVICE, "matmul: adding up the slices failed: " << mjt_last_error());
+        SliceFold fold(part_mem, C, out_dtype, M * N, slices, true);
+        {
+            Preparing preparing;
+            jit_launch(k, (unsigned)grid, 1, product_threads(split), 0, args);
+        }
+        fold.launch();
         set_last_kernel(k->name.c_str());
         return;
     }

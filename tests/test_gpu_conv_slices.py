@@ -71,16 +71,21 @@ def test_values_beyond_the_parts_range(gpu, value):
         assert "slices" in _check((3, 256, 14, 14), 256, 3, 1, "float32", values=v)
 
 
-def test_group_behind_runs_by_itself(gpu):
-    """A group behind a sliced convolution is refused by it and runs as a pass of its own, on the same values."""
+@pytest.mark.parametrize("dtype,shape,k", [("float32", (2, 256, 7, 7), 64), ("float32", (1, 130, 5, 3), 3), ("bfloat16", (3, 270, 9, 9), 70), ("float16", (1, 200, 7, 5), 18)])
+def test_group_behind(gpu, dtype, shape, k):
+    """A group behind a sliced convolution runs where the slices are added up, on the same values as by itself."""
     rng = np.random.default_rng(2)
-    x = jt.array(rng.standard_normal((2, 256, 7, 7)).astype(np.float32))
-    w = jt.array(rng.standard_normal((64, 256, 3, 3)).astype(np.float32))
-    b = jt.array(rng.standard_normal((1, 64, 1, 1)).astype(np.float32))
-    for _ in range(4):                                         # executed, replayed by its calls, recorded, by the recording
-        y = jt.nn.conv2d(x, w, padding=1)
-        z = jt.nn.relu(y + b)
-        only = jt.nn.relu(jt.nn.conv2d(x, w, padding=1) + b).numpy()
-        jt.sync([y, z])
-        assert np.array_equal(z.numpy(), np.maximum(y.numpy() + b.numpy(), 0))
-        assert np.array_equal(only, z.numpy())
+    x, _ = _var(rng.standard_normal(shape).astype(np.float32), dtype)
+    w, _ = _var(rng.standard_normal((k, shape[1], 3, 3)).astype(np.float32), dtype)
+    b, _ = _var(rng.standard_normal((1, k, 1, 1)).astype(np.float32), dtype)
+    out = {}
+    for fused in (1, 0):
+        with jt.flag_scope(enable_product_fusion=fused):
+            for _ in range(4):                                 # executed, replayed by its calls, recorded, by the recording
+                y = jt.nn.conv2d(x, w, padding=1)
+                z = jt.nn.relu(y + b)
+                only = jt.nn.relu(jt.nn.conv2d(x, w, padding=1) + b)
+                jt.sync([y, z])
+                got = [v.raw().copy() for v in (y, z, only)]
+                for a, c in zip(out.setdefault(0, got), got):
+                    assert np.array_equal(a.view(np.uint8), c.view(np.uint8))
