@@ -685,8 +685,9 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
         const int64_t NP = N * P, tiles64 = ((K + 63) / 64) * ((NP + 63) / 64);
         // (16-bit operands with a long sum and fewer 64 x 64 tiles than compute units stay on the column matrices, whose
         // product picks its tiles for a part-filled chip: 32 x 512 x 7 x 7 3x3 -> 512, 200 tiles: 102 us here, 71 there)
-        // (or on slices of the sum here, where these are few enough: the reduce reads their float32 results)
-        const bool ig_fits = !ig16 || tiles64 >= cus || CRS <= 1024 || tiles64 * 4 <= cus;
+        // (from 20 stages on a quarter of the chip's tiles take slices of the sum here: 6 x 160 x 9 x 9 3x3 -> 100 16.8 on column matrices, 11.4
+        // so; 2 x 200 x 9 x 9 3x3 -> 64 17.3, 10.5; 18 stages, 2 x 128 x 7 x 7 3x3 -> 128 13.5, 9.4, are left there)
+        const bool ig_fits = !ig16 || tiles64 >= cus || CRS <= 1024 || (CRS > 19 * 64 && tiles64 * 4 <= cus);
         // (a 1x1 convolution whose product would leave most of the chip idle comes here for the slices: the product below takes the images
         // as a batch, whose sums stay whole; float32 3 x 1024 x 14 x 14 -> 256 25.0 us there, 15.8 here; 10 x 512 x 16 x 16 -> 128 15.3, 13.8)
         const bool few_long = CRS >= (ig16 ? 512 : 256) && tiles64 * 2 <= cus;
@@ -760,7 +761,7 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
             if (!k) {
                 std::ostringstream name;
                 name << "mjt_conv_igemm_" << mjt_dtype_name(x->dtype) << (y->dtype != x->dtype ? "_of32" : "") << "_c" << C << "_k" << K << "_" << H << "x" << W << "_r" << R << "x" << S << "_s" << p->stride_h << "x"
-                     << p->stride_w << "_p" << p->pad_h << "x" << p->pad_w << "_d" << p->dil_h << "x" << p->dil_w << (split ? "_parts_" : "_") << 64 * MI << "x" << 64 * NI << (slices > 1 ? "_slices" : "") << ep.suffix();
+                     << p->stride_w << "_p" << p->pad_h << "x" << p->pad_w << "_d" << p->dil_h << "x" << p->dil_w << (slices > 1 ? "_slices" : "") << (split ? "_parts_" : "_") << 64 * MI << "x" << 64 * NI << ep.suffix();
                 std::ostringstream src;
                 src << ep.defs << "#define ENTRY " << name.str() << "\n#define SPLIT " << (split ? 1 : 0) << "\n#define SLICED " << (slices > 1 ? 1 : 0) << "\n#define CONV 1\n#define IN " << in << "\n#define OUT " << out << "\n#define MI " << MI << "\n#define NI " << NI
                     << "\n#define A_KCONT 1\n#define B_KCONT 0\n#define XBUF " << (xbuf ? 1 : 0) << "\n" << geo.str();

@@ -15,7 +15,11 @@ from .core import UnaryOp, BinaryOp, TernaryOp, BroadcastOp, ReduceOp
 
 MOST_COLUMNS = 16384             # a row has to fit the registers of a workgroup (csrc/op_rows.cpp)
 MOST_OPS = 128
-LEAST_ELEMENTS = 1 << 15         # below, the parts' kernels, which many graphs share, take 3 us each and stay
+# A small space is bound by its launches, 3 us each, not by its memory: a training step's chain of many is worth a kernel of its own, the
+# three of a normalisation, whose kernels many graphs share, are not (us a pass, apart / as one: softmax 307 x 69 with its gradient, seven
+# launches, 79 / 46; layer normalisation with its gradients float32 40 x 500 126 / 80, bfloat16 27 x 1092 161 / 106; a small CNN step with a
+# cross entropy over 4 x 5 310 / 277).
+SMALL, SMALL_PARTS = 1 << 15, 6
 FULL, ROW, COLUMN, ROUNDED = 0, 1, 2, 256
 SINGLE, OTHER = 3, 4
 _SUMMED = ("float32", "float16", "bfloat16")
@@ -120,7 +124,7 @@ class _Chooser:
             for k in shape[first:]:
                 cols *= k
             num = red.inputs[0].num
-            if 0 < cols <= MOST_COLUMNS and num >= LEAST_ELEMENTS:
+            if 0 < cols <= MOST_COLUMNS and num > 0:
                 found[(tuple(shape), first)] = num
         return sorted(found, key=lambda k: -found[k])
 
@@ -179,7 +183,7 @@ class _Chooser:
             n_rows = sum(1 for i in part if self.tasks[i].reduce is not None and place[i] == FULL)
             n_ops = sum(len(self.tasks[i].members) + 1 for i in part)
             passes = sum(1 for i in part if place[i] != ROW)   # over the full size, which become one
-            if n_rows and passes >= 2 and n_ops <= MOST_OPS:
+            if n_rows and (passes >= 2 if num >= SMALL else len(part) >= SMALL_PARTS) and n_ops <= MOST_OPS:
                 for i in part:
                     self.tasks[i].place = place[i]
                 return part
