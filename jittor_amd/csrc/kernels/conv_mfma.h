@@ -726,6 +726,7 @@ extern "C" __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu
 }
 
 // Weight re-pack: w[ko][c][kh][kw] -> Wp[tap][c/CB][k-step][ko/16][lg][l16][8 c] (c = CB block + 32 k-step + 8 lg + ..)
+// a[2] != 0 (one group): w is laid out [c][ko][kh][kw] and its taps are read from the last to the first.
 extern "C" __global__ __launch_bounds__(256) void ENTRY_PACK(Params p) {
     const int total = K_ * C_ * R_ * S_;                      // of one group: blockIdx.y
     const unsigned short* __restrict__ w = (const unsigned short*)p.a[0] + (size_t)blockIdx.y * total;
@@ -739,6 +740,6 @@ extern "C" __global__ __launch_bounds__(256) void ENTRY_PACK(Params p) {
         int cb = rest % NCB;
         int tap = rest / NCB;
         int c = cb * CB + ks * 32 + c32;
-        wp[o] = w[((size_t)ko * C_ + c) * (R_ * S_) + tap];
+        wp[o] = p.a[2] ? w[((size_t)c * K_ + ko) * (R_ * S_) + (R_ * S_ - 1 - tap)] : w[((size_t)ko * C_ + c) * (R_ * S_) + tap];
     }
 }

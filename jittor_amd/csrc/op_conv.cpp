@@ -5,6 +5,7 @@
 #include <array>
 #include <cmath>
 #include <map>
+#include <functional>
 #include <mutex>
 #include <unordered_map>
 
@@ -358,8 +359,19 @@ static bool conv_strided(const mjt_tensor* x, const mjt_tensor* w, const mjt_ten
 // packed / pack_mode: 0 the call packs the weights itself (into the library's buffer) and runs; 1 it only packs them
 // into `packed`; 2 it runs on weights packed by an earlier call of mode 1 for the same shapes and parameters.  Modes 1
 // and 2 exist for the MFMA kernel only and fail with MJT_ERR_UNSUPPORTED for a convolution that takes another route.
-void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, const mjt_conv_params* p, int64_t G, bool free_extent = false,
-               int pack_mode = 0, void* packed = nullptr) {
+// flipped: w [K,C,R,S] is still to be written, by fill(): it is the transpose of forward [C,K,R,S] with the taps from the last to the first
+// (an input gradient).  The MFMA kernel packs it from there in one pass (256 x 256 x 3 x 3 bfloat16, us: transposed 5.0 and packed 4.8, 4.8 so);
+// the other routes have it filled in first.
+struct FlippedWeights {
+    const mjt_tensor* forward;
+    std::function<void()> fill;
+};
+static void conv_run(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, const mjt_conv_params* p, int64_t G, bool free_extent,
+                     int pack_mode, void* packed, const FlippedWeights* flipped) {
+    auto need_weights = [&] {
+        if (flipped) flipped->fill();
+        flipped = nullptr;
+    };
     require_init();
     check_tensor(x, "conv x");
     check_tensor(w, "conv w");
@@ -386,6 +398,7 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
     MJT_CHECK(numel(x) < (int64_t(1) << 40) && numel(y) < (int64_t(1) << 40), "conv: too large");
     Context& c = ctx();
 
+    if (R * S == 1 || G > 1 || p->stride_h > 1 || p->stride_w > 1) need_weights();
     // a 1x1 convolution on large enough planes of an even number of pixels: one product for the batch, x read as it lies
     if (G == 1 && R == 1 && S == 1 && p->stride_h == 1 && p->stride_w == 1 && p->pad_h == 0 && p->pad_w == 0 && OH == H && OW == W && pack_mode == 0 &&
         !getenv("MJT_NO_FASTPATH") && !getenv("MJT_CONV_NO_GEMM") && !getenv("MJT_CONV_FLAT") && (double)N * K * C * H * W >= (double)(1 << 22) &&
@@ -599,7 +612,7 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
             // one launch for all groups (the group is the grid's second axis)
             char* wdst = (char*)(pack_mode ? packed : g_wpack);
             if (pack_mode != 2) {
-                std::vector<uint64_t> pa{bits_of_ptr(w->ptr), bits_of_ptr(wdst), 0, 0};
+                std::vector<uint64_t> pa{bits_of_ptr(flipped ? flipped->forward->ptr : w->ptr), bits_of_ptr(wdst), (uint64_t)(flipped ? 1 : 0), 0};
                 pa.resize(4 + ep.words.size());
                 Preparing preparing;
                 jit_launch(kp, (unsigned)pblocks, (unsigned)G, 256, 0, pa);
@@ -614,6 +627,7 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
         }
     }
 
+    need_weights();
     if (pack_mode) MJT_FAIL(MJT_ERR_UNSUPPORTED, "conv: this convolution does not run on packed weights (mjt_conv2d_meta takes it)");
 
     // ---- column matrices x weights on the GEMM kernel -----------------------------------
@@ -879,6 +893,11 @@ void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, co
     a.insert(a.end(), ep.words.begin(), ep.words.end());
     epilogue_taken(ep);
     jit_launch(k, (unsigned)blocks, 1, 256, 0, a);
+}
+
+void conv_impl(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor* y, const mjt_conv_params* p, int64_t G, bool free_extent = false,
+               int pack_mode = 0, void* packed = nullptr) {
+    conv_run(x, w, y, p, G, free_extent, pack_mode, packed, nullptr);
 }
 
 // The buffer of per-slice partial weight gradients, grown to `bytes`.
@@ -1553,15 +1572,16 @@ void conv_dgrad_impl(const mjt_tensor* dy, const mjt_tensor* w, const mjt_tensor
         return;
     }
     mjt_tensor tw = view(wbuf, w->dtype, {C, K, R, S});
-    {
+    const FlippedWeights flipped{w, [&] {
         Preparing preparing;
         reindex(*w, tw, {"i1", "i0", str(R - 1) + "-i2", str(S - 1) + "-i3"}, {});
-    }
+    }};
     const mjt_conv_params q = {1, 1, (int32_t)(dh * (R - 1) - ph), (int32_t)(dw * (S - 1) - pw), (int32_t)dh, (int32_t)dw};
     if (sh == 1 && sw == 1) {
-        conv_impl(dy, &tw, dx, &q, 1);
+        conv_run(dy, &tw, dx, &q, 1, false, 0, nullptr, &flipped);
         return;
     }
+    flipped.fill();
     const int64_t ZH = H + 2 * ph - dh * (R - 1), ZW = W + 2 * pw - dw * (S - 1);
     mjt_tensor tz = view(conv_scratch(3, (size_t)(N * K * ZH * ZW * esz)), dy->dtype, {N, K, ZH, ZW});
     {
