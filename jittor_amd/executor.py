@@ -1361,12 +1361,16 @@ def _run_single(op):
         # which chooses between it and the MFMA kernel for the others) otherwise.  us, chunks / gathering: 64 x 512 x 7 x 7 3x3 61 / 88,
         # 64 x 256 x 15 x 15 3x3 97 / 114, 64 x 256 x 13 x 13 77 / 85, but 64 x 64 x 13 x 13 57 / 22; 64 x 256 x 14 x 14 3x3 63 / 61,
         # 1x1 60 / 22.  The line at 2^27 keeps small layers on the route they had, 13 to 30 us where the gathering product takes
-        # 10 to 18 (8 x 32 x 14 x 14 3x3 -> 64 17.8 / 11.0, 8 x 128 x 7 x 7 3x3 13.7 / 16.3).
+        # 10 to 18 (8 x 32 x 14 x 14 3x3 -> 64 17.8 / 11.0, 8 x 128 x 7 x 7 3x3 13.7 / 16.3).  Not of fewer than six images, or of a number that
+        # makes no chunk, which would run image by image with their rows copied, six launches for two or three (us of kernels, forward and
+        # gradients, that / gathering: bottleneck block of 1 x 1024 x 14 x 14 173 / 131, of 2 147 / 142; 51 x 16 x 11 x 11 3x3 -> 133 72.1 / 64.1,
+        # 6 x 144 x 7 x 7 1x1 -> 172 41.8 / 34.5, 4 x 64 x 14 x 14 3x3 -> 128 47.0 / 43.8).
         half = x.dtype in ("bfloat16", "float16")
         narrow = OW % 8 != 0 and OW < 0.6 * 32 * -(-OW // 32)
         # Rows of at most 8 pixels with 2 to 9 taps stay with the library: 64 x 512 x 7 x 7 3x3 43 from windows in LDS.
         windows = OW <= 8 and 2 <= R * S <= 9 and sw <= 2
-        chunked = half and narrow and (OH * OW % 2 == 1 and N % 8 == 0 and not windows or N * OH * OW * K * C * R * S < 1 << 27)
+        together = next((a // math.gcd(OH * OW, a) for a in (64, 8) if N % (a // math.gcd(OH * OW, a)) == 0), 0)      # images that make a chunk
+        chunked = half and narrow and together and N >= 6 and (OH * OW % 2 == 1 and N % 8 == 0 and not windows or N * OH * OW * K * C * R * S < 1 << 27)
         if (half or x.dtype == "float32") and not chunked and flags["enable_conv_wgrad_kernel"]:
             # the MFMA kernel (16 bits) or the product that gathers its operands; shapes they do not cover come back as
             # unsupported and take the paths below
