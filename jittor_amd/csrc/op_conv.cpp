@@ -699,9 +699,11 @@ static void conv_run(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor*
         const int64_t NP = N * P, tiles64 = ((K + 63) / 64) * ((NP + 63) / 64);
         // (16-bit operands with a long sum and fewer 64 x 64 tiles than compute units stay on the column matrices, whose
         // product picks its tiles for a part-filled chip: 32 x 512 x 7 x 7 3x3 -> 512, 200 tiles: 102 us here, 71 there)
-        // (from 20 stages on a quarter of the chip's tiles take slices of the sum here: 6 x 160 x 9 x 9 3x3 -> 100 16.8 on column matrices, 11.4
-        // so; 2 x 200 x 9 x 9 3x3 -> 64 17.3, 10.5; 18 stages, 2 x 128 x 7 x 7 3x3 -> 128 13.5, 9.4, are left there)
-        const bool ig_fits = !ig16 || tiles64 >= cus || CRS <= 1024 || (CRS > 19 * 64 && tiles64 * 4 <= cus);
+        // (above 18 stages, tiles for at most a quarter of the chip, or half of it where one row of tiles has all output channels and the gather
+        // is not repeated, take slices of the sum here; us, column matrices / so: 6 x 160 x 9 x 9 3x3 -> 100 16.8 / 11.4, 51 x 133 x 11 x 11 3x3 -> 16
+        // 33.7 / 19.5, 64 x 200 x 11 x 11 5x5 -> 64 76.0 / 41.8; on the other side 20 x 256 x 9 x 9 3x3 -> 256 28.6 / 30.8, 12 x 130 x 13 x 13 3x3 -> 250 22.1 /
+        // 25.5; 18 stages, 2 x 128 x 7 x 7 3x3 -> 128 13.5 / 9.4, are left there)
+        const bool ig_fits = !ig16 || tiles64 >= cus || CRS <= 1024 || (CRS > 18 * 64 && tiles64 * (K <= 64 ? 2 : 4) <= cus);
         // (a 1x1 convolution whose product would leave most of the chip idle comes here for the slices: the product below takes the images
         // as a batch, whose sums stay whole; float32 3 x 1024 x 14 x 14 -> 256 25.0 us there, 15.8 here; 10 x 512 x 16 x 16 -> 128 15.3, 13.8)
         const bool few_long = CRS >= (ig16 ? 512 : 256) && tiles64 * 2 <= cus;
@@ -1437,6 +1439,30 @@ static bool conv_dgrad_all_phases(const mjt_tensor* dy, const mjt_tensor* w, con
     return true;
 }
 
+// The same for a few thousand results of any of the types, from dy and w as they lie (kernels/conv_dgrad_direct.h).
+static void conv_dgrad_direct(const mjt_tensor* dy, const mjt_tensor* w, const mjt_tensor* dx, const mjt_conv_params* p) {
+    const int64_t C = dx->shape[1], H = dx->shape[2], W = dx->shape[3], K = dy->shape[1], OH = dy->shape[2], OW = dy->shape[3], R = w->shape[2], S = w->shape[3];
+    const int64_t total = numel(dx), lpo = K >= 32 ? 16 : K >= 8 ? 8 : K >= 4 ? 4 : 1;
+    std::ostringstream geo, name;
+    geo << "#define C_ " << C << "\n#define H_ " << H << "\n#define W_ " << W << "\n#define K_ " << K << "\n#define R_ " << R << "\n#define S_ " << S << "\n#define OH_ " << OH << "\n#define OW_ " << OW
+        << "\n#define SH " << p->stride_h << "\n#define SW " << p->stride_w << "\n#define PH " << p->pad_h << "\n#define PW " << p->pad_w << "\n#define DH " << p->dil_h << "\n#define DW " << p->dil_w
+        << "\n#define LPO " << lpo << "\n#define TIN " << dtype_cname(dy->dtype) << "\n#define TOUT " << dtype_cname(dx->dtype) << "\n";
+    const EpilogueCode ep = epilogue_code(1, 4, dx->dtype, total);
+    const std::string key = "dgdirect|" + geo.str() + ep.key;
+    JitKernel* k = cached(key);
+    if (!k) {
+        name << "mjt_conv_direct_dgrad_" << mjt_dtype_name(dy->dtype) << "_" << mjt_dtype_name(dx->dtype) << "_c" << C << "_k" << K << "_" << H << "x" << W << "_r" << R << "x" << S << "_s" << p->stride_h << "x"
+             << p->stride_w << "_p" << p->pad_h << "x" << p->pad_w << "_d" << p->dil_h << "x" << p->dil_w << ep.suffix();
+        k = jit_get(ep.defs + "#define ENTRY " + name.str() + "\n" + geo.str() + (ep.on ? "" : embedded_source("prelude.h")) + "\n" + embedded_source("conv_dgrad_direct.h") + "\n", name.str());
+        remember(key, k);
+    }
+    std::vector<uint64_t> a{bits_of_ptr(dy->ptr), bits_of_ptr(w->ptr), bits_of_ptr(dx->ptr), (uint64_t)total};
+    a.insert(a.end(), ep.words.begin(), ep.words.end());
+    epilogue_taken(ep);
+    jit_launch(k, (unsigned)((total * lpo + 255) / 256), 1, 256, 0, a);
+    set_last_kernel(k->name.c_str());
+}
+
 // Input gradient of the convolution y = conv(x, w): dx[n,c,h,w] = sum over (k, r, s) of dy[n,k,oh,ow] * w[k,c,r,s] with
 // h = oh*sh - ph + r*dh, w = ow*sw - pw + s*dw.  It is itself a convolution of dy, run on the forward kernels:
 //   * 16-bit operands at strides 1 and 2 other than 1 x 1: one launch for all phases (above);
@@ -1507,6 +1533,14 @@ void conv_dgrad_impl(const mjt_tensor* dy, const mjt_tensor* w, const mjt_tensor
         cols = phases(sw, pw, S);
         for (const Phase& q : rows) by_phase = by_phase && q.pad >= 0;
         for (const Phase& q : cols) by_phase = by_phase && q.pad >= 0;
+    }
+    // Few multiply-adds: all phases in one launch, a result at a time.  It looks at every tap of every channel, 1.2 us a million (float32, us,
+    // phase by phase in five or six launches / so: 4 x 16 x 6 x 6 3x3 -> 16 22.8 / 3.6, 4 x 16 x 16 x 16 -> 16 17.8 / 5.3, 2 x 8 x 8 x 8 -> 8 10.6 / 2.9; on the
+    // other side, 47 and 58 million, 13 x 48 x 18 x 18 3x3 -> 26 28.8 / 53.9, 8 x 64 x 14 x 14 3x3 -> 64 34.0 / 77.2).
+    if ((sh > 1 || sw > 1) && K > 0 && !getenv("MJT_NO_FASTPATH") && !getenv("MJT_CONV_DGRAD_NO_PHASES") && R * S <= 49 && numel(dy) < (int64_t(1) << 30) && (double)numel(dx) * K * R * S < (double)(1 << 23)) {
+        conv_dgrad_direct(dy, w, dx, p);
+        if (by_phase) set_last_kernel(("conv_dgrad_phases:" + std::string(mjt_last_kernel())).c_str());
+        return;
     }
     if (by_phase) {
         const int64_t Hs = H / sh, Ws = W / sw, dsz = dtype_size(dx->dtype);
