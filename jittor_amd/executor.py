@@ -1068,7 +1068,7 @@ def _depthwise_gradients(tasks):
     of the two where the other's operands are there by then."""
     writer = {v: i for i, t in enumerate(tasks) for v in t.writes}
     weights = [(i, t) for i, t in enumerate(tasks) if isinstance(t.node, ConvBwdWeightUnit) and t.node.groups > 1]
-    gone = set()
+    gone, paired = set(), set()                                # paired: weight gradients; branches that are summed share their dy
     for i, t in enumerate(tasks):
         d = t.node
         if not isinstance(d, ConvBwdDataUnit) or d.groups == 1 or d.params[:2] != (1, 1) or d.params[4:] != (1, 1):
@@ -1078,7 +1078,7 @@ def _depthwise_gradients(tasks):
             continue
         for j, u in weights:
             g = u.node
-            if id(u) in gone or g.inputs[1] is not dy or g.params != d.params or g.groups != d.groups or list(g.out.shape) != list(w.shape) \
+            if id(u) in paired or g.inputs[1] is not dy or g.params != d.params or g.groups != d.groups or list(g.out.shape) != list(w.shape) \
                     or list(g.inputs[0].shape) != list(d.out.shape):
                 continue
             first, other = (t, u) if i < j else (u, t)
@@ -1087,6 +1087,7 @@ def _depthwise_gradients(tasks):
             first.run = _both_gradients(d, g, t.run, u.run)
             first.reads, first.writes = first.reads | other.reads, first.writes | other.writes
             gone.add(id(other))
+            paired.add(id(u))
             break
     return [t for t in tasks if id(t) not in gone]
 

@@ -1340,6 +1340,35 @@ def test_replayed_result_is_the_memory_of_its_own_input(fake_buffers, shared_fir
     assert fake_buffers.stats["replays"] > replays + 1
 
 
+@pytest.mark.parametrize("targets", ["x1 x2 w1 w2", "w1 w2 x1 x2", "w2 x1 x2 w1", "x2 w1 x1 w2", "x1 w2 x2", "w1 x2 w2"])
+@pytest.mark.parametrize("shared,branches", [(False, 2), (True, 2), (False, 3)])
+def test_depthwise_branches_that_are_summed(fake_buffers, monkeypatch, targets, shared, branches):
+    """Branches that are summed send one dy to several input and weight gradients: each is computed, by one call, and no more calls
+    make two at once than there are of either."""
+    monkeypatch.setitem(fake_buffers.flags, "enable_replay", True)
+    v = {}
+    for i in range(1, branches + 1):
+        v["x%d" % i] = v["x1"] if shared and i > 1 else jt.array(np.ones((8, 32, 14, 14), np.float32)) * float(i)
+        v["w%d" % i] = jt.array(np.ones((32, 1, 3, 3), np.float32)) * float(i)
+    jt.sync(list(v.values()))
+    fake_buffers._plans.clear()
+    y = sum((jt.nn.conv2d(v["x%d" % i], v["w%d" % i], padding=1, groups=32) for i in range(2, branches + 1)), jt.nn.conv2d(v["x1"], v["w1"], padding=1, groups=32))
+    names = [n for n in targets.split() if not (shared and n == "x2")] + (["x3", "w3"] if branches == 3 else [])
+    grads = jt.grad((y * y).sum(), [v[n] for n in names])
+    jt.sync(grads)
+    assert all(g._buf is not None for g in grads)
+    plan, = fake_buffers._plans.values()
+    made, both = [], 0
+    for fn, args in plan.calls:
+        outs = {"mjt_conv2d_meta_backward_depthwise": (3, 4), "mjt_conv2d_meta_dgrad_depthwise": (2,), "mjt_conv2d_meta_wgrad_grouped": (2,)}.get(fn.__name__, ())
+        made += [args[k]._obj.ptr for k in outs]
+        both += len(outs) == 2
+    n_x, n_w = sum(n[0] == "x" for n in names) * (branches if shared else 1), sum(n[0] == "w" for n in names)
+    assert len(made) == len(set(made)) == n_x + n_w and both == min(n_x, n_w)
+    if not shared:
+        assert set(made) == {g._buf.ptr for g in grads}
+
+
 def test_fused_rows_descriptor_is_checked(compile_only):
     """mjt_fused_rows: what it hands back runs part by part, what makes no sense is an error; nothing is launched."""
     L, lib = compile_only, compile_only.load()
