@@ -958,6 +958,20 @@ struct Key {
         return text(t.p);
     }
 };
+// A one-element host array whose bytes are all zero.  Values are data and no part of a graph's key, but this the executor looks at (a
+// select against zero is a relu, executor.py:_masks_from_results): it asks here, and the key of a graph with a select says it of every number.
+bool zero_number(PyObject* u) {
+    PyObject* h = absent(u, s__op) ? own(u, s__host) : nullptr;
+    Py_buffer view;
+    if (!h || h == Py_None) return false;
+    if (PyObject_GetBuffer(h, &view, PyBUF_SIMPLE)) { PyErr_Clear(); return false; }
+    bool zero = view.len == view.itemsize;
+    for (Py_ssize_t i = 0; zero && i < view.len; i++) zero = ((const char*)view.buf)[i] == 0;
+    PyBuffer_Release(&view);
+    return zero;
+}
+PyObject* py_zero_number(PyObject*, PyObject* u) { return PyBool_FromLong(zero_number(u)); }
+
 // signature(ops, targets, flags): everything the execution of `ops` depends on besides the data, as bytes (with what ops of other classes
 // say of themselves beside them), or None where an op does not know or its result is gone.
 PyObject* py_signature(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
@@ -965,6 +979,8 @@ PyObject* py_signature(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     std::unordered_map<PyObject*, int> made, leaf;
     std::unordered_set<PyObject*> targets;
     for (Py_ssize_t i = 0; i < PyList_GET_SIZE(args[1]); i++) targets.insert(PyList_GET_ITEM(args[1], i));
+    std::vector<PyObject*> leaves;
+    bool selects = false;
     Key k;
     k.b.reserve(4096);
     Ref others;
@@ -980,7 +996,7 @@ PyObject* py_signature(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         auto get = [&](PyObject* name) { return own(op, name); };
         if (t == t_unary) { k.b.push_back('u'); ok = k.text(get(s_op)); }
         else if (t == t_binary) { k.b.push_back('b'); ok = k.text(get(s_op)); }
-        else if (t == t_ternary) k.b.push_back('t');
+        else if (t == t_ternary) { k.b.push_back('t'); selects = true; }
         else if (t == t_broadcast) { k.b.push_back('c'); ok = k.integer(get(s_bcast_mask)) && k.integer(get(s_keepdims_mask)); }
         else if (t == t_reduce) { k.b.push_back('r'); ok = k.text(get(s_op)) && k.integer(get(s_reduce_mask)) && k.integer(get(s_keepdims_mask)); }
         else if (t == t_reindex) {
@@ -1014,12 +1030,15 @@ PyObject* py_signature(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
             auto [l, first] = leaf.emplace(u, (int)leaf.size());
             k.num(-1 - l->second);
             if (first) {
+                leaves.push_back(u);
                 if (!k.var(u)) return nullptr;
                 k.b.push_back((char)((absent(u, s__op) ? 1 : 0) | (absent(u, s__buf) ? 2 : 0) | (absent(u, s__host) ? 4 : 0) | (flag(u, s__stop_fuse) ? 8 : 0)));
             }
         }
         made[out] = (int)i;
     }
+    if (selects)
+        for (PyObject* u : leaves) k.b.push_back(zero_number(u) ? 1 : 0);
     // the flags are entered once and keep their order
     PyObject *name, *value;
     Py_ssize_t at = 0;
@@ -1075,6 +1094,7 @@ PyMethodDef methods[] = {
     {"as_var", py_as_var, METH_O, "a Var, or the Var of a number or array"},
     {"new_id", py_new_id, METH_NOARGS, "the next id of a Var or op"},
     {"pending_ops", py_pending_ops, METH_O, "pending producers behind the targets, in topological order"},
+    {"zero_number", py_zero_number, METH_O, "zero_number(var): whether it is one element in host memory whose bytes are all zero"},
     {"signature", (PyCFunction)(void (*)(void))py_signature, METH_FASTCALL, "signature(ops, targets, flags): hashable description of a graph, or None"},
     {"gradients", (PyCFunction)(void (*)(void))py_gradients, METH_FASTCALL, "gradients(loss, targets, others): a gradient per target"},
     {"setup", py_setup, METH_O, "takes the classes and tables of core.py"},

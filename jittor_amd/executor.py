@@ -1123,7 +1123,7 @@ def _masks_from_results(sched, consumers, target_ids):
     def zero(v):
         while isinstance(v._op, BroadcastOp) and v._buf is None:
             v = v._op.inputs[0]
-        return v._op is None and v._host is not None and v.num == 1 and _scalar_value(v) in ((0.0, 0),)
+        return _graph.zero_number(v)                           # (which the graph's key tells, so that a plan is one for zeros only)
 
     place = {node.id: i for i, node in enumerate(sched)}
     made = []                                                   # (behind which op, the new ones)

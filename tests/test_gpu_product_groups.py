@@ -172,6 +172,29 @@ def test_masks_of_tiny_and_undefined_values(gpu, dt):
     _both(step, _taken(step))
 
 
+@pytest.mark.parametrize("what", ["other", "threshold", "both"])
+def test_masks_of_selects_against_other_numbers(gpu, what):
+    """One graph with zeros, then with other numbers, captured, replayed and from recorded launches: the mask is that of x > t."""
+    rng = np.random.default_rng(16)
+    X = rng.integers(-2, 3, (2, 8, 12, 12)).astype(np.float32)
+    x, w, g = jt.array(X), _var(rng, [16, 8, 3, 3], "float32"), _var(rng, [2, 16, 12, 12], "float32")
+    jt.sync([x, w, g])
+
+    def step(t, b):
+        y = jt.ternary(x > jt.array(np.float32([t])), x, jt.array(np.float32([b])))
+        gx = jt.grad((jt.nn.conv2d(y, w, padding=1) * g).sum(), x)
+        jt.sync([y, gx])
+        return y.numpy(), gx.numpy()
+
+    whole = step(-3.0, 0.0)[1]                                   # nothing masked
+    assert (whole != 0).all()
+    for v in (0.0, 5.0, 0.0, -1.0, 0.0):
+        t, b = v if what != "other" else 0.0, v if what != "threshold" else 0.0
+        for _ in range(3):
+            y, gx = step(t, b)
+            assert np.array_equal(y, np.where(X > t, X, np.float32(b))) and np.array_equal(gx, np.where(X > t, whole, 0)), (t, b)
+
+
 def test_a_product_that_others_read_stays(gpu):
     """A result that is asked for, that a reduce reads too, or that is broadcast, is written as before."""
     rng = np.random.default_rng(12)

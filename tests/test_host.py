@@ -1590,3 +1590,33 @@ def test_graph_keys_tell_graphs_apart():
         assert _graph.signature(_graph.pending_ops([vs[4]]), [vs[4]], executor.flags) != k0
     vs[2].stop_fuse()
     assert _graph.signature(_graph.pending_ops([vs[4]]), [vs[4]], executor.flags) != k0
+
+
+def test_graph_keys_tell_a_select_against_zero(fake_buffers):
+    """What a relu's mask is read from depends on whether the threshold and the other operand are zero: the key of a graph with a select
+    tells zeros from other numbers, other numbers are data."""
+    from jittor_amd import _graph
+    w = jt.array(np.ones((8, 4, 3, 3), np.float32))
+    jt.sync([w])
+
+    def step(threshold, other):
+        x = jt.array(np.ones((2, 4, 9, 9), np.float32)) * 2.0
+        jt.sync([x])
+        y = jt.ternary(x > (0.0 if threshold == 0 else jt.array(np.float32([threshold]))), x, jt.array(np.float32([other])))
+        z = jt.nn.conv2d(y, w, padding=1)
+        gx = jt.grad((z * z).sum(), x)
+        key = _graph.signature(_graph.pending_ops([z, gx]), [z, gx], fake_buffers.flags)
+        replays = fake_buffers.stats["replays"]
+        jt.sync([z, gx])
+        return key, fake_buffers.stats["replays"] - replays
+
+    keys = {}
+    for threshold, other, known in ((0, 0, 0), (0, 5, 0), (3, 0, 0), (2, 7, 0), (0, 0, 1), (0, 6, 1), (-1, 0, 1), (5, 5, 1)):
+        key, replays = step(threshold, other)
+        assert replays == known, (threshold, other)
+        assert keys.setdefault((threshold == 0, other == 0), key) == key
+    assert len(set(keys.values())) == len(keys) == 4
+    number = lambda v, dtype: _graph.zero_number(jt.array(np.asarray(v, dtype)))
+    assert number([0], np.float32) and number([0], np.int64) and number([False], np.bool_) and number([0], np.float16)
+    assert not number([1e-45], np.float32) and not number([-0.0], np.float32) and not number([0, 0], np.float32) and not number([1], np.int8)
+    assert not _graph.zero_number(jt.array(np.zeros([1], np.float32)) + 0.0)
