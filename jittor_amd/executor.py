@@ -1120,10 +1120,10 @@ def _masks_from_results(sched, consumers, target_ids):
     that is in memory: inside a group x may be wider than y, and a tiny x is 0 in y."""
     producer = {node.out.id: node for node in sched}
 
-    def zero(v):
+    def zero(v):                                                # the zero that v spreads, or None
         while isinstance(v._op, BroadcastOp) and v._buf is None:
             v = v._op.inputs[0]
-        return _graph.zero_number(v)                           # (which the graph's key tells, so that a plan is one for zeros only)
+        return v if _graph.zero_number(v) else None            # (which the graph's key tells, so that a plan is one for zeros only)
 
     place = {node.id: i for i, node in enumerate(sched)}
     made = []                                                   # (behind which op, the new ones)
@@ -1133,7 +1133,7 @@ def _masks_from_results(sched, consumers, target_ids):
         cond, x, other = t.inputs
         c = producer.get(cond.id)
         if not isinstance(c, BinaryOp) or c.op != "greater" or cond.id in target_ids or c.inputs[0] is not x or x.dtype != t.out.dtype \
-                or x.dtype not in _FLOAT_RANK or list(x.shape) != list(t.out.shape) or not zero(c.inputs[1]) or not zero(other):
+                or x.dtype not in _FLOAT_RANK or list(x.shape) != list(t.out.shape) or zero(c.inputs[1]) is None or zero(other) is None:
             continue
         p = producer.get(x.id)
         if p is not None and p.fusable:
@@ -1145,7 +1145,8 @@ def _masks_from_results(sched, consumers, target_ids):
         if not later:
             continue
         with core.no_grad():
-            mask = core.binary(t.out, 0.0, "greater")          # (with a zero of its own: the other's group need not hand its out)
+            # the graph's own zero, which a replay finds, spread once more: the other's group need not hand its out
+            mask = core.binary(t.out, zero(c.inputs[1]), "greater")
         spread = [u._op for u in mask._op.inputs if u is not t.out and u._op is not None]
         made.append((t, spread + [mask._op]))
         for u in later:

@@ -1369,6 +1369,29 @@ def test_depthwise_branches_that_are_summed(fake_buffers, monkeypatch, targets, 
         assert set(made) == {g._buf.ptr for g in grads}
 
 
+@pytest.mark.parametrize("zeros", [(0.0, 0.0), (0, 0), (False, 0.0), "arrays", "arrays of halves"])
+def test_masks_read_from_results_are_replayed(fake_buffers, zeros):
+    """convolution, select against zero, convolution, with gradients: whatever the zeros are, the mask is read from the select's result and
+    the graph is replayed and recorded."""
+    stats = fake_buffers.stats
+    w1, w2 = jt.array(np.ones((8, 4, 3, 3), np.float32)), jt.array(np.ones((8, 8, 3, 3), np.float32))
+    x = jt.array(np.ones((2, 4, 9, 9), np.float32))
+    jt.sync([x, w1, w2])
+    fake_buffers._plans.clear()
+
+    def step():
+        zero = [jt.array(np.zeros([1], np.float16 if "halves" in zeros else np.float32)) for _ in range(2)] if isinstance(zeros, str) else zeros
+        v = jt.nn.conv2d(x, w1, padding=1)
+        z = jt.nn.conv2d(jt.ternary(v > zero[0], v, zero[1]), w2, padding=1)
+        jt.sync([z] + list(jt.grad((z * z).sum(), [w1, w2])))
+    before = dict(stats)
+    for _ in range(4):
+        step()
+    assert stats["plans"] == before["plans"] + 1 and stats["replays"] == before["replays"] + 3
+    assert stats["recorded_launches"] > before["recorded_launches"]
+    assert stats["fused_products"] == before["fused_products"] + 8          # the select behind one product, the mask behind another
+
+
 def test_fused_rows_descriptor_is_checked(compile_only):
     """mjt_fused_rows: what it hands back runs part by part, what makes no sense is an error; nothing is launched."""
     L, lib = compile_only, compile_only.load()
