@@ -1466,6 +1466,7 @@ static void conv_dgrad_direct(const mjt_tensor* dy, const mjt_tensor* w, const m
 // Input gradient of the convolution y = conv(x, w): dx[n,c,h,w] = sum over (k, r, s) of dy[n,k,oh,ow] * w[k,c,r,s] with
 // h = oh*sh - ph + r*dh, w = ow*sw - pw + s*dw.  It is itself a convolution of dy, run on the forward kernels:
 //   * 16-bit operands at strides 1 and 2 other than 1 x 1: one launch for all phases (above);
+//   * any other stride above 1 with few multiply-adds: one launch, a result at a time (conv_dgrad_direct);
 //   * stride 1: with the weights transposed and their taps flipped, padding d*(R-1) - p;
 //   * a stride without dilation, H and W multiples of it: one stride-1 convolution per stride phase.  The rows
 //     h = sh*i + a of dx see only the taps r = r_a + sh*u (r_a = (a + ph) % sh, u = 0 .. U_a - 1) and
@@ -1537,9 +1538,9 @@ void conv_dgrad_impl(const mjt_tensor* dy, const mjt_tensor* w, const mjt_tensor
     // Few multiply-adds: all phases in one launch, a result at a time.  It looks at every tap of every channel, 1.2 us a million (float32, us,
     // phase by phase in five or six launches / so: 4 x 16 x 6 x 6 3x3 -> 16 22.8 / 3.6, 4 x 16 x 16 x 16 -> 16 17.8 / 5.3, 2 x 8 x 8 x 8 -> 8 10.6 / 2.9; on the
     // other side, 47 and 58 million, 13 x 48 x 18 x 18 3x3 -> 26 28.8 / 53.9, 8 x 64 x 14 x 14 3x3 -> 64 34.0 / 77.2).
-    if ((sh > 1 || sw > 1) && K > 0 && !getenv("MJT_NO_FASTPATH") && !getenv("MJT_CONV_DGRAD_NO_PHASES") && R * S <= 49 && numel(dy) >= 1 && numel(dy) < (int64_t(1) << 30) && (double)numel(dx) * K * R * S < (double)(1 << 23)) {
+    if ((sh > 1 || sw > 1) && K > 0 && !getenv("MJT_NO_FASTPATH") && !getenv("MJT_CONV_DGRAD_NO_DIRECT") && !getenv("MJT_CONV_DGRAD_NO_PHASES") && R * S <= 49 && numel(dy) >= 1 &&
+        numel(dy) < (int64_t(1) << 30) && (double)numel(dx) * K * R * S < (double)(1 << 23)) {
         conv_dgrad_direct(dy, w, dx, p);
-        if (by_phase) set_last_kernel(("conv_dgrad_phases:" + std::string(mjt_last_kernel())).c_str());
         return;
     }
     if (by_phase) {

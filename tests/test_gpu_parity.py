@@ -5,6 +5,7 @@ for atomic scatter-add.  Full-size benchmark shapes are checked through
 closed forms and size-independent properties."""
 import ctypes
 import json
+import math
 import os
 
 import numpy as np
@@ -913,10 +914,19 @@ def _dgrad_reference(dy, w, H, W, params):
     ((2, 64, 28, 28), (64, 64, 3, 3), (1, 1, 1, 1, 1, 1), "bfloat16", "float32", False),
     ((2, 8, 12, 12), (6, 8, 1, 1), (3, 3, 0, 0, 1, 1), "bfloat16", "float32", True),      # stride 3, phases no tap reaches: zeros of the result's type
 ], ids=lambda c: "x%s_w%s_p%s_%s" % ("x".join(map(str, c[0])), "x".join(map(str, c[1])), "".join(map(str, c[2])), c[3]))
-def test_conv_input_gradient_entry(gpu, case):
+@pytest.mark.parametrize("without", ["", "DIRECT", "PHASES"])
+def test_conv_input_gradient_entry(gpu, case, without, monkeypatch):
     """mjt_conv2d_meta_dgrad against the definition of the gradient in float64 (per element within 1e-4 of the sum of
-    its terms' magnitudes, plus the result type's rounding), and for float32 against the oracle's gradient graph."""
+    its terms' magnitudes, plus the result type's rounding), and for float32 against the oracle's gradient graph: as it chooses (few
+    multiply-adds at a stride above 1 in one launch), without that launch (phase by phase), and without phases (dy spread out with zeros)."""
     xshape, wshape, params, dtype, out_dtype, phased = case
+    if without:
+        if params[:2] == (1, 1):
+            pytest.skip("stride 1 has neither")
+        monkeypatch.setenv("MJT_CONV_DGRAD_NO_" + without, "1")
+    direct = not without and params[:2] != (1, 1) and phased != "all" and math.prod(xshape) * math.prod(wshape) // xshape[1] < 1 << 23
+    if direct or without == "PHASES":
+        phased = False
     sh, sw, ph, pw, dh, dw_ = params
     N, C, H, W = xshape
     K, _, R, S = wshape
@@ -939,7 +949,7 @@ def test_conv_input_gradient_entry(gpu, case):
     p = L.ConvParams(*params)
     L.check(L.load().mjt_conv2d_meta_dgrad(ctypes.byref(td), ctypes.byref(tw), ctypes.byref(tx), ctypes.byref(p)))
     kern = L.last_kernel()
-    assert kern.startswith("conv_dgrad_phases:") == (phased is True) and ("_dgrad_c" in kern) == (phased == "all"), kern
+    assert kern.startswith("conv_dgrad_phases:") == (phased is True) and ("_dgrad_c" in kern) == (phased == "all") and kern.startswith("mjt_conv_direct_dgrad_") == direct, kern
     if dtype != "float32" and C == 64:
         assert "mjt_conv_mfma" in kern, kern
     raw = L.d2h(dx.raw_ptr(), dx.shape, L.NP_STORAGE[out_dtype])

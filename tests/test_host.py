@@ -524,9 +524,10 @@ def test_shutdown_forgets_kernels_and_rebinding_compiles_again(compile_only, mon
     assert calls()[0] >= first + 3                           # compiled again, not taken from a stale table
 
 
-def test_conv_input_gradient_entry_validates_and_picks_its_path(compile_only):
-    """mjt_conv2d_meta_dgrad without a device: argument checks, and which of its four forms a geometry takes (16 bits at strides 1 and 2 one kernel for
-    all stride phases, transposed flipped weights for stride 1, one convolution per stride phase, dy spread out with zeros otherwise)."""
+def test_conv_input_gradient_entry_validates_and_picks_its_path(compile_only, monkeypatch):
+    """mjt_conv2d_meta_dgrad without a device: argument checks, and which of its five forms a geometry takes (16 bits at strides 1 and 2 one kernel for
+    all stride phases, transposed flipped weights for stride 1, few multiply-adds a result at a time, one convolution per stride phase, dy spread out with
+    zeros otherwise), by the name of the kernel that runs."""
     lib = L.load()
     P = 0x100000
 
@@ -550,6 +551,13 @@ def test_conv_input_gradient_entry_validates_and_picks_its_path(compile_only):
         assert L.last_kernel().startswith("conv_dgrad_phases:"), L.last_kernel()
         assert call((2, 64, rows + 1, rows), (64, 64, 3, 3), params, dtype=dtype) == 0     # no whole phases
         assert not L.last_kernel().startswith("conv_dgrad_phases:") and "_dgrad_c" not in L.last_kernel(), L.last_kernel()
+    for rows in (10, 11):                                      # few multiply-adds, with and without whole phases
+        assert call((2, 8, rows, 12), (6, 8, 3, 3), (2, 2, 1, 1, 1, 1), dtype="float32") == 0
+        assert L.last_kernel().startswith("mjt_conv_direct_dgrad_float32"), L.last_kernel()
+        with monkeypatch.context() as m:
+            m.setenv("MJT_CONV_DGRAD_NO_DIRECT", "1")
+            assert call((2, 8, rows, 12), (6, 8, 3, 3), (2, 2, 1, 1, 1, 1), dtype="float32") == 0
+            assert L.last_kernel().startswith("conv_dgrad_phases:" if rows == 10 else "mjt_conv_direct_float32"), L.last_kernel()
     assert call((2, 64, 28, 28), (64, 64, 3, 3), (2, 2, 1, 1, 1, 1), dys=(2, 64, 15, 14)) == -1
     assert b"dy shape" in lib.mjt_last_error()
     assert call((2, 64, 28, 28), (64, 32, 3, 3), (2, 2, 1, 1, 1, 1)) == -1         # weight channels != dx channels
