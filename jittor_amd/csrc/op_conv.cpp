@@ -1538,7 +1538,7 @@ void conv_dgrad_impl(const mjt_tensor* dy, const mjt_tensor* w, const mjt_tensor
     // Few multiply-adds: all phases in one launch, a result at a time.  It looks at every tap of every channel, 1.2 us a million (float32, us,
     // phase by phase in five or six launches / so: 4 x 16 x 6 x 6 3x3 -> 16 22.8 / 3.6, 4 x 16 x 16 x 16 -> 16 17.8 / 5.3, 2 x 8 x 8 x 8 -> 8 10.6 / 2.9; on the
     // other side, 47 and 58 million, 13 x 48 x 18 x 18 3x3 -> 26 28.8 / 53.9, 8 x 64 x 14 x 14 3x3 -> 64 34.0 / 77.2).
-    if ((sh > 1 || sw > 1) && K > 0 && !getenv("MJT_NO_FASTPATH") && !getenv("MJT_CONV_DGRAD_NO_DIRECT") && !getenv("MJT_CONV_DGRAD_NO_PHASES") && R * S <= 49 && numel(dy) >= 1 &&
+    if ((sh > 1 || sw > 1) && K > 0 && !getenv("MJT_NO_FASTPATH") && !getenv("MJT_CONV_DGRAD_NO_DIRECT") && !getenv("MJT_CONV_DGRAD_NO_PHASES") && R * S <= 49 && numel(dx) >= 1 && numel(dy) >= 1 &&
         numel(dy) < (int64_t(1) << 30) && (double)numel(dx) * K * R * S < (double)(1 << 23)) {
         conv_dgrad_direct(dy, w, dx, p);
         return;

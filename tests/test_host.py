@@ -564,6 +564,9 @@ def test_conv_input_gradient_entry_validates_and_picks_its_path(compile_only, mo
     assert call((2, 64, 28, 28), (64, 64, 1, 1), (1, 1, 1, 1, 1, 1)) == -1         # padding no tap reaches
     assert b"padding" in lib.mjt_last_error()
     assert call((2, 8, 12, 12), (6, 8, 1, 1), (3, 3, 0, 0, 1, 1), out="float32") == 0      # phases that no tap reaches, in the result's type
+    for rows, cols, dys in ((0, 9, (2, 6, 1, 6)), (4, 0, (2, 6, 3, 1))):         # a dx of no elements whose dy has some: refused, nothing is launched
+        assert call((2, 8, rows, cols), (6, 8, 3, 3), (2, 2, 2, 2, 1, 1), dys=dys, dtype="float32") == -1
+        assert b"empty output" in lib.mjt_last_error()
 
 
 def test_conv_builds_that_ran_out_of_registers_are_not_run(compile_only):
