@@ -99,6 +99,12 @@ __device__ __forceinline__ void mjt_mfma2(mjt_f32x16& c, const mjt_u32x2& alo, c
     asm volatile(MJT_MFMA_ASM " %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
 }
 __device__ __forceinline__ void mjt_keep2(const mjt_u32x2& x) { asm volatile("" : : "v"(x)); }     // x is in its registers up to here
+// What lanes of the wave wrote to LDS before is there for all its lanes after: the hardware keeps a wave's LDS accesses in order, this keeps the compiler from another one.
+__device__ __forceinline__ void mjt_wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 __device__ __forceinline__ void mjt_pin(mjt_f32x16& x) { asm volatile("" : "+a"(x)); }            // what reads x later comes after this point
 
 #ifndef EPI
@@ -343,6 +349,7 @@ extern "C" __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu
         for (int j = 0; j < FR; j++)
 #pragma unroll
             for (int e = 0; e < 16; e++) mine[(8 * (e / 4) + 4 * (lane >> 5) + (e & 3)) * PITCH + j * 32 + (lane & 31)] = acc[i][j][e];
+        mjt_wave_fence();
 #pragma unroll
         for (int b = 0; b < IT; b += BATCH) {
             long long at[BATCH];
@@ -385,6 +392,7 @@ extern "C" __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu
 #endif
             }
         }
+        mjt_wave_fence();                                                                // (before the next 32 rows overwrite these)
     }
 #else
 #pragma unroll
