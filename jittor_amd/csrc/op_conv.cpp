@@ -627,7 +627,6 @@ static void conv_run(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor*
         }
     }
 
-    need_weights();
     if (pack_mode) MJT_FAIL(MJT_ERR_UNSUPPORTED, "conv: this convolution does not run on packed weights (mjt_conv2d_meta takes it)");
 
     // ---- column matrices x weights on the GEMM kernel -----------------------------------
@@ -646,7 +645,7 @@ static void conv_run(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor*
                           CRS >= ((CRS * dtype_size(x->dtype)) % 16 || (uintptr_t)w->ptr % 16 ? 160 : 128);
     if (G == 1 && !getenv("MJT_NO_FASTPATH") && !getenv("MJT_CONV_NO_GEMM") && ((double)N * K * P * CRS >= (double)(1 << 22) || long_sum) &&
         P < (int64_t(1) << 31) && CRS < (int64_t(1) << 31) && matmul_available()) {
-        if (!flat_forced && conv_stem(x, w, y, p)) return;
+        if (!flat_forced && !flipped && conv_stem(x, w, y, p)) return;       // (of stride 2)
         const int64_t esz = dtype_size(x->dtype);
         const int64_t Ppad = (P * esz + 15) / 16 * 16 / esz;
         const bool plain = R == 1 && S == 1 && p->stride_h == 1 && p->stride_w == 1 && p->pad_h == 0 && p->pad_w == 0 && Ppad == P && OH == H && OW == W;
@@ -662,7 +661,9 @@ static void conv_run(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor*
         // rows that are not (3 x 7 x 7 float32 taps: 588 bytes) are copied into rows padded with zeros once per call.
         const void* wmat = w->ptr;
         int64_t lda = CRS;
-        if ((CRS * esz) % 16 || (uintptr_t)w->ptr % 16) {
+        auto weight_rows = [&] {                                // (each route below, once it is sure to run)
+            need_weights();
+            if ((CRS * esz) % 16 == 0 && (uintptr_t)w->ptr % 16 == 0) return;
             lda = (CRS * esz + 15) / 16 * 16 / esz;
             void* wpad = conv_scratch(4, (size_t)(K * lda * esz));
             mjt_tensor tw = view(w->ptr, w->dtype, {K, CRS}), tp = view(wpad, w->dtype, {K, lda});
@@ -671,8 +672,10 @@ static void conv_run(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor*
             if (mjt_reindex(&tw, &tp, 2, widx, 0.0, 0, nullptr, 0, nullptr) != MJT_OK)
                 MJT_FAIL(MJT_ERR_DEVICE, "conv: padding the weight rows failed: " << mjt_last_error());
             wmat = wpad;
-        }
+        };
         if (flat && !plain) {
+            check_no_epilogue();                                // (column matrices take no group: refused before the weights are touched)
+            weight_rows();
             const int64_t osz = dtype_size(y->dtype);
             void* cols = conv_scratch(0, (size_t)(CRS * NP0 * esz));
             void* yt = conv_scratch(5, (size_t)(K * NP0 * osz));
@@ -789,15 +792,22 @@ static void conv_run(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor*
             const int64_t tiles = ((K + 64 * MI - 1) / (64 * MI)) * ((NP + 64 * NI - 1) / (64 * NI));
             const int64_t grid = (tiles * slices + 7) / 8 * 8;
             MJT_CHECK(grid < (int64_t(1) << 31), "conv: launch too large");
-            std::vector<uint64_t> a{bits_of_ptr(wmat), bits_of_ptr(x->ptr), bits_of_ptr(slices > 1 ? part_mem : y->ptr), (uint64_t)K, (uint64_t)NP, (uint64_t)CRS,
-                                    (uint64_t)lda, 0, 0, (uint64_t)(slices > 1 ? per : 0), 0, (uint64_t)(slices > 1 ? K * NP : 0)};
-            a.insert(a.end(), ep.words.begin(), ep.words.end());
+            auto args = [&] {
+                weight_rows();
+                std::vector<uint64_t> a{bits_of_ptr(wmat), bits_of_ptr(x->ptr), bits_of_ptr(slices > 1 ? part_mem : y->ptr), (uint64_t)K, (uint64_t)NP, (uint64_t)CRS,
+                                        (uint64_t)lda, 0, 0, (uint64_t)(slices > 1 ? per : 0), 0, (uint64_t)(slices > 1 ? K * NP : 0)};
+                a.insert(a.end(), ep.words.begin(), ep.words.end());
+                return a;
+            };
             if (slices == 1) {
+                if (!ep.on) check_no_epilogue();
+                const std::vector<uint64_t> a = args();
                 epilogue_taken(ep);
                 jit_launch(k, (unsigned)grid, 1, product_threads(split), 0, a);
                 return;
             }
             SliceFold fold(part_mem, y->ptr, y->dtype, K * NP, slices, true);
+            const std::vector<uint64_t> a = args();
             {
                 Preparing preparing;
                 jit_launch(k, (unsigned)grid, 1, product_threads(split), 0, a);
@@ -806,6 +816,8 @@ static void conv_run(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor*
             set_last_kernel(k->name.c_str());
             return;
         }
+        if (!plain) check_no_epilogue();
+        weight_rows();
         int64_t chunk = (int64_t(1) << 30) / (CRS * Ppad * esz);
         if (const char* e = getenv("MJT_CONV_GEMM_CHUNK"))      // images per chunk, for tests of the chunk loop
             if (atoi(e) >= 1) chunk = atoi(e);
@@ -859,6 +871,7 @@ static void conv_run(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor*
         return;
     }
 
+    need_weights();
     // ---- depthwise: one input channel per group -----------------------------------------
     if (G > 1 && C == 1 && !free_extent) {
         const DepthwiseShape g{H, W, OH, OW, R, S, p->stride_h, p->stride_w, p->pad_h, p->pad_w, p->dil_h, p->dil_w, 1, 1, K, K / G, false};

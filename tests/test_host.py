@@ -1151,6 +1151,34 @@ def test_routes_that_want_workspace_have_one_without(compile_only, monkeypatch):
     assert product(301, 203, 129, "bfloat16", 0, 0).startswith("mjt_gemm_mfma_")
 
 
+@pytest.mark.parametrize("what", ["conv", "dgrad"])
+@pytest.mark.parametrize("flat", ["0", "1"])
+def test_routes_without_a_group_refuse_before_they_prepare(compile_only, monkeypatch, what, flat):
+    """A convolution through column matrices takes no group behind it, and says so before it launches anything: neither the copy of its
+    weight rows to whole 16 bytes nor, for an input gradient, the transposed weights."""
+    lib = compile_only.load()
+    monkeypatch.setenv("MJT_CONV_NO_IGEMM", "1")
+    monkeypatch.setenv("MJT_CONV_FLAT", flat)
+    dt = "float32" if flat == "0" else "bfloat16"              # (the whole-batch product is one of 16 bits)
+    code = L.DTYPE_CODE[dt]
+    x, w, y = L.tensor(P, dt, [2, 15, 30, 30]), L.tensor(P, dt, [33, 15, 3, 3]), L.tensor(P, dt, [2, 33, 30, 30])
+    out = y if what == "conv" else x
+    fv = (L.FusedVar * 2)(L.FusedVar(L.VAR_PRODUCT, code, None), L.FusedVar(L.VAR_OUTPUT, code, P))
+    fo = (L.FusedOp * 1)(L.FusedOp(L.FOP_UNARY, L.OP_CODE["negative"], (0, 0, 0), 1))
+    d = L.FusedDesc(4, tuple(out.shape[:4]), 2, fv, 1, fo)
+    p = L.ConvParams(1, 1, 1, 1, 1, 1)
+    probe = L.tensor(P, "float32", [64])
+    L.check(lib.mjt_reduce(ctypes.byref(probe), ctypes.byref(L.tensor(P, "float32", [1])), L.OP_CODE["add"], 1))
+    last = L.last_kernel()
+    if what == "conv":
+        rc = lib.mjt_conv2d_meta_then(ctypes.byref(x), ctypes.byref(w), ctypes.byref(y), ctypes.byref(p), 1, ctypes.byref(d))
+    else:
+        rc = lib.mjt_conv2d_meta_dgrad_then(ctypes.byref(y), ctypes.byref(w), ctypes.byref(x), ctypes.byref(p), ctypes.byref(d))
+    assert rc == L.ERR_UNSUPPORTED and L.last_kernel() == last
+    L.check(lib.mjt_conv2d_meta(ctypes.byref(x), ctypes.byref(w), ctypes.byref(y), ctypes.byref(p)))
+    assert L.last_kernel() == ("conv_as_batch_gemm" if flat == "1" else "conv_as_reindex_gemm")
+
+
 def test_float32_weight_gradient_of_a_few_tiles_is_cut_into_slices(compile_only, monkeypatch):
     """One to thirty tiles and a sum of ten to a hundred stages: small tiles, and as many slices as there are compute units to run
     them (they need workspace, so that a limit on it hands the call back), not one workgroup for the whole sum."""
