@@ -180,9 +180,9 @@ struct Preparing {
 };
 // The sum of a product's slices (op_slices.cpp), at most 16 of n float32 results each, into y (n elements of a float type up to 32 bits) or
 // the group that waits behind the product.  Made before the slices are launched, under Preparing: a group that cannot be taken ends the call
-// there.  whole: the n elements are the product's whole result, in its order.
+// there.  The n elements are the product's whole result, in its order.
 struct SliceFold {
-    SliceFold(const void* part, void* y, int dtype, int64_t n, int64_t slices, bool whole);
+    SliceFold(const void* part, void* y, int dtype, int64_t n, int64_t slices);
     void launch();
 
 private:

@@ -806,7 +806,7 @@ static void conv_run(const mjt_tensor* x, const mjt_tensor* w, const mjt_tensor*
                 jit_launch(k, (unsigned)grid, 1, product_threads(split), 0, a);
                 return;
             }
-            SliceFold fold(part_mem, y->ptr, y->dtype, K * NP, slices, true);
+            SliceFold fold(part_mem, y->ptr, y->dtype, K * NP, slices);
             const std::vector<uint64_t> a = args();
             {
                 Preparing preparing;

@@ -249,7 +249,7 @@ void gemm_launch(int in_dtype, int out_dtype, const void* A, const void* B, void
         args[2] = bits_of_ptr(part_mem);
         args[9] = (uint64_t)per;
         args[11] = (uint64_t)(M * N);
-        SliceFold fold(part_mem, C, out_dtype, M * N, slices, true);
+        SliceFold fold(part_mem, C, out_dtype, M * N, slices);
         {
             Preparing preparing;
             jit_launch(k, (unsigned)grid, 1, product_threads(split), 0, args);

@@ -16,12 +16,12 @@ void forget() {   // the kernels belong to the run-time compiler's cache, which 
 const bool g_registered = (at_shutdown(&forget), true);
 }  // namespace
 
-SliceFold::SliceFold(const void* part, void* y, int dtype, int64_t n, int64_t slices, bool whole) {
+SliceFold::SliceFold(const void* part, void* y, int dtype, int64_t n, int64_t slices) {
     MJT_CHECK(slices >= 1 && slices <= 16 && (dtype == MJT_FLOAT32 || dtype == MJT_BFLOAT16 || dtype == MJT_FLOAT16), "slices of a sum: not covered");
     const int osz = dtype_size(dtype);
     int vs = 4;
     while (vs > 1 && (n % vs || (uintptr_t)y % (size_t)(vs * osz))) vs /= 2;
-    ep = epilogue_code(vs, 3, dtype, whole ? n : -1);
+    ep = epilogue_code(vs, 3, dtype, n);
     if (!ep.on) check_no_epilogue();                              // (before anything is launched)
     const int out = dtype == MJT_BFLOAT16 ? 0 : dtype == MJT_FLOAT16 ? 1 : 2;
     std::ostringstream key;

@@ -1052,7 +1052,7 @@ def _execute(ops, target_ids):
         tasks = rowfuse.merge(tasks, ins, pre, consumers, target_ids, sys.modules[__name__]) or tasks
     if flags["enable_product_fusion"] and _profiler.active() is None:
         tasks = _behind_products(tasks, ins, consumers, target_ids, pre, scatter_of)
-    if _profiler.active() is None:
+    if flags["enable_gradient_pairs"] and _profiler.active() is None:
         tasks = _depthwise_gradients(tasks)
     for t in tasks:
         t.run()

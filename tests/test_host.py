@@ -1381,10 +1381,11 @@ def test_replayed_result_is_the_memory_of_its_own_input(fake_buffers, shared_fir
 
 @pytest.mark.parametrize("targets", ["x1 x2 w1 w2", "w1 w2 x1 x2", "w2 x1 x2 w1", "x2 w1 x1 w2", "x1 w2 x2", "w1 x2 w2"])
 @pytest.mark.parametrize("shared,branches", [(False, 2), (True, 2), (False, 3)])
-def test_depthwise_branches_that_are_summed(fake_buffers, monkeypatch, targets, shared, branches):
+@pytest.mark.parametrize("pairs", [True, False])
+def test_depthwise_branches_that_are_summed(fake_buffers, monkeypatch, targets, shared, branches, pairs):
     """Branches that are summed send one dy to several input and weight gradients: each is computed, by one call, and no more calls
-    make two at once than there are of either."""
-    monkeypatch.setitem(fake_buffers.flags, "enable_replay", True)
+    make two at once than there are of either (none without the flag)."""
+    monkeypatch.setitem(fake_buffers.flags, "enable_gradient_pairs", pairs)
     v = {}
     for i in range(1, branches + 1):
         v["x%d" % i] = v["x1"] if shared and i > 1 else jt.array(np.ones((8, 32, 14, 14), np.float32)) * float(i)
@@ -1403,7 +1404,7 @@ def test_depthwise_branches_that_are_summed(fake_buffers, monkeypatch, targets, 
         made += [args[k]._obj.ptr for k in outs]
         both += len(outs) == 2
     n_x, n_w = sum(n[0] == "x" for n in names) * (branches if shared else 1), sum(n[0] == "w" for n in names)
-    assert len(made) == len(set(made)) == n_x + n_w and both == min(n_x, n_w)
+    assert len(made) == len(set(made)) == n_x + n_w and both == (min(n_x, n_w) if pairs else 0)
     if not shared:
         assert set(made) == {g._buf.ptr for g in grads}
 
