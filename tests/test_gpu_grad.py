@@ -168,7 +168,7 @@ def _conv_grads_ref(x, w, r, stride, pad, dil):
     return dX[:, :, pad:pad + H, pad:pad + W], dW
 
 
-@pytest.mark.parametrize("case", [
+META_CONVS = [
     dict(x=(2, 3, 6, 6), w=(4, 3, 3, 3), stride=1, pad=1, dil=1, units=3),
     dict(x=(3, 8, 12, 10), w=(6, 8, 3, 3), stride=1, pad=2, dil=2, units=3),
     dict(x=(2, 4, 9, 9), w=(5, 4, 3, 3), stride=1, pad=0, dil=1, units=3),
@@ -176,16 +176,16 @@ def _conv_grads_ref(x, w, r, stride, pad, dil):
     dict(x=(2, 4, 12, 10), w=(5, 4, 3, 3), stride=2, pad=1, dil=1, units=3),     # ... rows and columns the stride never reaches
     dict(x=(1, 3, 13, 13), w=(2, 3, 3, 3), stride=3, pad=0, dil=2, units=3),     # stride 3, dilation 2
     dict(x=(2, 6, 8, 8), w=(4, 6, 1, 1), stride=1, pad=0, dil=1, units=3),
-])
-@pytest.mark.parametrize("direct", [True, False], ids=["", "no_direct"])
+]
+
+
+@pytest.mark.parametrize("case,direct", [(c, d) for c in META_CONVS for d in (True, False) if d or c["stride"] > 1])
 def test_grad_meta_conv(gpu, case, direct, monkeypatch):
     """Gradients of the meta-op convolution (nn.py:1245-1262) with respect to input and weight against a
     direct float64 evaluation (test_conv_tuner.py:105-133 checks the same pair).  Forward, input gradient
     (stride 1) and weight gradient are each recognised and run as one convolution call, so the
     7-dimensional intermediates are never computed (the invariant of test_longest_dis_fuse.py:51-66)."""
     if not direct:                                             # small strided input gradients by phases or over zero-spaced dy
-        if case["stride"] == 1:
-            pytest.skip("stride 1 has one route")
         monkeypatch.setenv("MJT_CONV_DGRAD_NO_DIRECT", "1")
     rng = np.random.default_rng(6)
     x = rng.standard_normal(case["x"]).astype(np.float32)

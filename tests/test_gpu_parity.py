@@ -896,7 +896,7 @@ def _dgrad_reference(dy, w, H, W, params):
     return dx[:, :, ph:ph + H, pw:pw + W], mag[:, :, ph:ph + H, pw:pw + W]
 
 
-@pytest.mark.parametrize("case", [
+DGRAD = [
     # x shape,         w shape,          (sh, sw, ph, pw, dh, dw), dtype,     result,    by phases
     ((2, 8, 10, 12), (6, 8, 3, 3), (1, 1, 1, 1, 1, 1), "float32", "float32", False),
     ((2, 8, 10, 12), (6, 8, 3, 3), (2, 2, 1, 1, 1, 1), "float32", "float32", True),
@@ -913,16 +913,17 @@ def _dgrad_reference(dy, w, H, W, params):
     ((2, 64, 28, 28), (64, 64, 3, 3), (3, 3, 1, 1, 1, 1), "float16", "float32", False),  # no whole phases: dy spread out with zeros
     ((2, 64, 28, 28), (64, 64, 3, 3), (1, 1, 1, 1, 1, 1), "bfloat16", "float32", False),
     ((2, 8, 12, 12), (6, 8, 1, 1), (3, 3, 0, 0, 1, 1), "bfloat16", "float32", True),      # stride 3, phases no tap reaches: zeros of the result's type
-], ids=lambda c: "x%s_w%s_p%s_%s" % ("x".join(map(str, c[0])), "x".join(map(str, c[1])), "".join(map(str, c[2])), c[3]))
-@pytest.mark.parametrize("without", ["", "DIRECT", "PHASES"])
+]
+
+
+@pytest.mark.parametrize("case,without", [(c, w) for c in DGRAD for w in ("", "DIRECT", "PHASES") if not w or (c[2][:2] != (1, 1) and (w == "PHASES" or c[5] != "all"))],
+                         ids=lambda c: c or "any" if isinstance(c, str) else "x%s_w%s_p%s_%s" % ("x".join(map(str, c[0])), "x".join(map(str, c[1])), "".join(map(str, c[2])), c[3]))
 def test_conv_input_gradient_entry(gpu, case, without, monkeypatch):
     """mjt_conv2d_meta_dgrad against the definition of the gradient in float64 (per element within 1e-4 of the sum of
     its terms' magnitudes, plus the result type's rounding), and for float32 against the oracle's gradient graph: as it chooses (few
     multiply-adds at a stride above 1 in one launch), without that launch (phase by phase), and without phases (dy spread out with zeros)."""
     xshape, wshape, params, dtype, out_dtype, phased = case
     if without:
-        if params[:2] == (1, 1):
-            pytest.skip("stride 1 has neither")
         monkeypatch.setenv("MJT_CONV_DGRAD_NO_" + without, "1")
     direct = not without and params[:2] != (1, 1) and phased != "all" and math.prod(xshape) * math.prod(wshape) // xshape[1] < 1 << 23
     if direct or without == "PHASES":

@@ -1,6 +1,7 @@
 """Pooling on blocks: windows folded from whole 16-byte pieces (kernels/window_fold.h) and their gradients on blocks of rows and columns
 (kernels/window_scatter.h with BLOCKS), against the kernels of one output and one row a lane, which are held to the oracle elsewhere: every
-result meets its window in the same order, so they agree bit for bit."""
+result meets its window in the same order, so folds and a maximum's gradient agree bit for bit; the terms of a mean's gradient are products, which one
+kernel may round before it adds them and the other not, so it agrees within that rounding."""
 import numpy as np
 import pytest
 
