@@ -916,7 +916,13 @@ DGRAD = [
 ]
 
 
-@pytest.mark.parametrize("case,without", [(c, w) for c in DGRAD for w in ("", "DIRECT", "PHASES") if not w or (c[2][:2] != (1, 1) and (w == "PHASES" or c[5] != "all"))],
+def _in_one_launch(case):
+    """Few multiply-adds at a stride above 1, where no kernel of all phases is."""
+    x, w, params, phased = case[0], case[1], case[2], case[5]
+    return params[:2] != (1, 1) and phased != "all" and math.prod(x) * math.prod(w) // x[1] < 1 << 23
+
+
+@pytest.mark.parametrize("case,without", [(c, w) for c in DGRAD for w in ("", "DIRECT", "PHASES") if not w or (_in_one_launch(c) if w == "DIRECT" else c[5])],
                          ids=lambda c: c or "any" if isinstance(c, str) else "x%s_w%s_p%s_%s" % ("x".join(map(str, c[0])), "x".join(map(str, c[1])), "".join(map(str, c[2])), c[3]))
 def test_conv_input_gradient_entry(gpu, case, without, monkeypatch):
     """mjt_conv2d_meta_dgrad against the definition of the gradient in float64 (per element within 1e-4 of the sum of
@@ -925,7 +931,7 @@ def test_conv_input_gradient_entry(gpu, case, without, monkeypatch):
     xshape, wshape, params, dtype, out_dtype, phased = case
     if without:
         monkeypatch.setenv("MJT_CONV_DGRAD_NO_" + without, "1")
-    direct = not without and params[:2] != (1, 1) and phased != "all" and math.prod(xshape) * math.prod(wshape) // xshape[1] < 1 << 23
+    direct = not without and _in_one_launch(case)
     if direct or without == "PHASES":
         phased = False
     sh, sw, ph, pw, dh, dw_ = params
