@@ -961,7 +961,7 @@ struct Key {
 // A one-element host array whose bytes are all zero.  Values are data and no part of a graph's key, but this the executor looks at (a
 // select against zero is a relu, executor.py:_masks_from_results): it asks here, and the key of a graph with a select says it of every number.
 bool zero_number(PyObject* u) {
-    PyObject* h = absent(u, s__op) ? own(u, s__host) : nullptr;
+    PyObject *n = own(u, s_num), *h = n && PyLong_CheckExact(n) && PyLong_AsLongLong(n) == 1 && absent(u, s__op) ? own(u, s__host) : nullptr;
     Py_buffer view;
     if (!h || h == Py_None) return false;
     if (PyObject_GetBuffer(h, &view, PyBUF_SIMPLE)) { PyErr_Clear(); return false; }
